@@ -53,25 +53,25 @@ MODELS = {
 def listed() -> List[dict]:
     return [
         # one user's chat: every token waits for a whole step
-        _decode("llama decode, one sequence", "llama-3-8b", 1, 1023),
+        _decode("llama decode one sequence", "llama-3-8b", 1, 1023),
         # a busy server: 64 conversations of 2048 tokens
-        _decode("llama decode, 64 sequences", "llama-3-8b", 64, 2048),
+        _decode("llama decode 64 sequences", "llama-3-8b", 64, 2048),
         # a few long conversations, past the sliding window of half the layers
-        _decode("gemma decode, long", "gemma-2-9b", 5, 5003),
+        _decode("gemma decode long", "gemma-2-9b", 5, 5003),
         # the serving benchmark: 4-bit weights, 64 sequences behind prompts of 512
-        _decode("deepseek 4-bit decode, 64", "deepseek-v2-lite", 64, 512, 4),
+        _decode("deepseek 4-bit decode 64", "deepseek-v2-lite", 64, 512, 4),
         # the same model for one user in a long conversation
-        _decode("deepseek 4-bit decode, one", "deepseek-v2-lite", 1, 3001, 4),
+        _decode("deepseek 4-bit decode one", "deepseek-v2-lite", 1, 3001, 4),
         # a question of a few words
-        _prompt("tinyllama, short prompt", "tinyllama-1.1b", 1, 57),
+        _prompt("tinyllama short prompt", "tinyllama-1.1b", 1, 57),
         # a document that fills the context
-        _prompt("llama, long prompt", "llama-3-8b", 1, 8192),
+        _prompt("llama long prompt", "llama-3-8b", 1, 8192),
         # a long document in chunks, past the sliding window
-        _prompt("gemma, chunked prompt", "gemma-2-9b", 1, 6001, chunk=4096),
+        _prompt("gemma chunked prompt", "gemma-2-9b", 1, 6001, chunk=4096),
         # the serving benchmark's prompts
-        _prompt("deepseek 4-bit, 64 prompts", "deepseek-v2-lite", 64, 512, 4),
+        _prompt("deepseek 4-bit 64 prompts", "deepseek-v2-lite", 64, 512, 4),
         # recurrent and latent-attention layers over long documents
-        _prompt("tuvutar, long prompts", "tuvutar-2b", 2, 4001),
+        _prompt("tuvutar long prompts", "tuvutar-2b", 2, 4001),
         # services under mixed load
         _batches("tuvutar service", "tuvutar-2b", 12, 17, 1300, 6),
         _batches("dufinex service", "dufinex-7b", 16, 9, 900, 6),
