@@ -31,8 +31,8 @@ void launch_attn_decode(const void*, const void*, const void*, void*, float*,
                         int, int, long, float, float, int, hipStream_t);
 bool attn_decode_supported_shape(int, int);
 void launch_attn_prefill(const void*, const void*, const void*, void*, int,
-                         int, int, int, int, long, long, int, int, float,
-                         float, int, int, hipStream_t);
+                         int, int, int, int, long, long, long, long, long, int,
+                         int, float, float, int, int, hipStream_t);
 bool attn_prefill_supported(int, int);
 void launch_mfma_probe(const void*, const void*, float*, hipStream_t);
 void launch_w4a16_gemv(const void*, const void*, const void*, const void*,
@@ -343,7 +343,16 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                            double scale, double softcap, int64_t window,
                            int64_t causal_offset) {
   check_bf16(q, "q");
-  auto qc = q.contiguous();
+  // rows of queries are read where they lie, in 16-byte pieces
+  auto whole = [](const torch::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  const bool in_place = whole(q) && q.stride(3) == 1 && q.stride(0) % 8 == 0 &&
+                        q.stride(1) % 8 == 0 && q.stride(2) % 8 == 0;
+  auto qc = in_place ? q : q.contiguous();
+  if (!whole(qc)) qc = qc.clone();
+  if (!whole(k)) k = k.clone(at::MemoryFormat::Contiguous);
+  if (!whole(v)) v = v.clone(at::MemoryFormat::Contiguous);
   const int B = qc.size(0), Hq = qc.size(1), T = qc.size(2), Dk = qc.size(3);
   const int Hkv = k.size(1), S = k.size(2), Dv = v.size(3);
   TORCH_CHECK(k.stride(3) == 1 && v.stride(3) == 1, "K/V rows must be contiguous");
@@ -357,12 +366,14 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k, torch::Tensor v,
               " Dv=", Dv);
   long kScap = k.stride(1) / Dk;
   long vScap = v.stride(1) / Dv;
-  auto out = torch::empty({B, Hq, T, Dv}, qc.options());
+  // heads of a token side by side, as the output projection reads them
+  auto out = torch::empty({B, T, Hq, Dv}, qc.options());
   launch_attn_prefill(qc.data_ptr(), k.data_ptr(), v.data_ptr(),
-                      out.data_ptr(), B, Hq, Hkv, T, S, kScap, vScap, Dk, Dv,
+                      out.data_ptr(), B, Hq, Hkv, T, S, qc.stride(0),
+                      qc.stride(1), qc.stride(2), kScap, vScap, Dk, Dv,
                       (float)scale, (float)softcap, (int)window,
                       (int)causal_offset, cur_stream());
-  return out;
+  return out.transpose(1, 2);
 }
 
 torch::Tensor mfma_probe(torch::Tensor A, torch::Tensor Bm) {

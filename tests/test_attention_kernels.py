@@ -1,0 +1,86 @@
+"""Attention kernels at the edges of their tiles, against 64-bit attention."""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def ext():
+    from mlx_sharding_amd import ops
+    e = ops.hip_ext()
+    assert e is not None, "HIP extension must be built on a GPU box"
+    return e
+
+
+def attention(q, k, v, scale, cap, window, offset):
+    """(output, what the weights' absolute values make of |v|) in 64 bits."""
+    q, k, v = q.double(), k.double(), v.double()
+    rep = q.shape[1] // k.shape[1]
+    k, v = k.repeat_interleave(rep, 1), v.repeat_interleave(rep, 1)
+    s = (q @ k.transpose(-1, -2).contiguous()) * scale
+    if cap:
+        s = torch.tanh(s / cap) * cap
+    at = torch.arange(q.shape[2], device=q.device)[:, None] + offset
+    key = torch.arange(k.shape[2], device=q.device)[None, :]
+    hidden = key > at
+    if window:
+        hidden = hidden | (key <= at - window)
+    p = torch.softmax(s.masked_fill(hidden, -math.inf), -1)
+    return p @ v, p @ v.abs()
+
+
+def cached(B, H, S, D, room):
+    """Rows [B, H, S, D] of a cache whose other rows are NaN."""
+    buf = torch.full((B, H, S + room, D), math.nan, dtype=torch.bfloat16,
+                     device="cuda")
+    buf[:, :, :S] = torch.randn(B, H, S, D, device="cuda")
+    return buf[:, :, :S]
+
+
+PREFILL = [(32, 16), (32, 32), (32, 64), (64, 32), (64, 64), (64, 128), (128, 32),
+           (128, 64), (128, 128), (192, 64), (192, 128), (256, 256)]
+
+
+@pytest.mark.parametrize("Dk,Dv", PREFILL)
+def test_prefill_edges(Dk, Dv):
+    """Tiles of 128 queries and 64 (32) keys: one query, one more and one less
+    than a tile, windows that begin inside tiles, fewer heads than XCDs, a
+    negative scale (and none), queries as slices of wider rows."""
+    torch.manual_seed(Dk + Dv)
+    for B, Hq, Hkv, T, offset, cap, window, scale in (
+            (1, 8, 4, 1, 77, 0.0, 0, 0.1), (1, 4, 2, 57, 0, 0.0, 0, 0.1),
+            (2, 8, 2, 129, 0, 0.0, 0, 0.1), (1, 2, 1, 127, 64, 20.0, 65, 0.1),
+            (1, 3, 1, 300, 31, 30.0, 0, 0.2), (1, 8, 8, 130, 75, 0.0, 50, -0.1),
+            (1, 2, 2, 33, 0, 0.0, 1, 0.1), (1, 2, 2, 128, 0, 0.0, 0, 0.0)):
+        S = T + offset
+        rows = torch.randn(B, T, Hq, Dk + 8, dtype=torch.bfloat16, device="cuda")
+        q = rows[..., 8:].transpose(1, 2)
+        k, v = cached(B, Hkv, S, Dk, 37), cached(B, Hkv, S, Dv, 37)
+        out = ext().attn_prefill(q, k, v, scale, cap, window, offset).double()
+        expect, size = attention(q, k, v, scale, cap, window, offset)
+        # weights and result are rounded to bf16 (2^-8 each); exponents of up
+        # to 2^8 in 32-bit steps come to less than 2^-13 of a weight
+        bound = 2.0 ** -8 * (size + expect.abs()) + 2.0 ** -13 * size + 1e-6
+        assert (out.shape == expect.shape
+                and bool(((out - expect).abs() <= bound).all())), (T, offset, window)
+
+
+def test_prefill_large_scores():
+    """The reference of the exponents moves late and far: scores that grow
+    with the key by hundreds, and one key that stands out."""
+    torch.manual_seed(0)
+    T, D = 200, 128
+    q = torch.full((1, 8, T, D), 1.0, dtype=torch.bfloat16, device="cuda")
+    k = (torch.arange(T, device="cuda") / D * 4).bfloat16()[None, None, :, None]
+    k = k.expand(1, 8, T, D).contiguous()
+    k[:, 1, 70] = 9.0
+    v = torch.randn(1, 8, T, D, device="cuda").bfloat16()
+    for scale in (1.0, 0.01, -1.0):
+        out = ext().attn_prefill(q, k, v, scale, 0.0, 0, 0).double()
+        expect, size = attention(q, k, v, scale, 0.0, 0, 0)
+        # scores of up to 1200 are off by 2^-24 of themselves each way
+        bound = 2.0 ** -8 * (size + expect.abs()) + 2.0 ** -12 * size + 1e-6
+        assert bool(((out - expect).abs() <= bound).all()), scale
