@@ -355,3 +355,306 @@ extern "C" bool attn_decode_supported_shape(int G, int Dv) {
   return G == 1 || G == 2 || G == 4 || G == 6 || G == 7 || G == 8 ||
          G == 16;
 }
+
+// ---------------------------------------------------------------------------
+// The same on matrix cores, for the head sizes that models have.
+//
+// A block serves all (up to 16) query heads of one key/value head over a slice
+// of its keys.  Tiles of keys and values go to LDS without passing registers, the
+// next one while this one is worked on; what it reads from memory is all that
+// bounds it, and two blocks a CU keep 64 KB and more in flight.  S^T = K Q^T on
+// 16x16x32 products: a wave takes 16 keys (with tiles of 32 keys also half of the
+// contraction), leaves its scores in LDS, and after a barrier every wave has the
+// weights of the whole tile in the layout of the next product's operand and makes
+// a quarter of the output's columns, O^T = V^T P^T.  So waves share no outputs.
+// V^T is read by ds_read_b64_tr_b16 out of rows as they lie in memory; values that
+// lie in the keys' rows (a cached latent) are staged once for both.
+// Weights stay 32-bit: they enter as a high and a low bf16 part (16 bits and
+// more, at twice the products, which have time to spare).
+// Slices come from the length on the device, so they are even under capture.
+// Measured (before: dot products and sums on the vector units, up to 8 slices of
+// the capacity): 64 sequences of 2049 keys, 32 heads of 128 over 8: 179 -> 109 us
+// (4.9 TB/s, what a copy reaches); one of 1024: 24 -> 8.4; 5 of 5004, 16 heads of
+// 256 over 8, capped: 91 -> 45; 16 heads over a latent of 576/512, 64 x 513 keys:
+// 66 -> 22, 1 x 3002: 75 -> 14.
+// ---------------------------------------------------------------------------
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+#define DT_MAXSPLIT 64
+
+struct DecodeArgs {
+  const char *q, *k, *v;   // rows: q [B, Hq, DK], k, v [B, Hkv, cap, *]
+  char* out;
+  float *part_o, *part_ml; // [B * Hq, nsplit, DV], [B * Hq, nsplit, 2]
+  const int* s_ptr;
+  int Hq, Hkv, S, nsplit, window;
+  long cap;
+  float c;                 // score -> power of two; behind a cap: 1
+  float cap_in, cap_out;   // e^(2 score / cap) as 2^(cap_in s); cap in base 2
+};
+
+__device__ __forceinline__ void dt_to_lds(const char* src, char* dst) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) void*)src,
+      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+// Place of a 16-byte piece within its row in LDS: keys are read a row a lane,
+// values four rows by 32 bytes a quarter wave.
+template <int N, bool KEYS>
+__device__ __forceinline__ int dt_place(int row, int piece) {
+  if (KEYS) return piece ^ (row & 7);
+  return N >= 16 ? piece ^ ((row & 7) << 1) : piece ^ ((row & 3) << 1);
+}
+
+// largest of the four lanes that share a column
+__device__ __forceinline__ float column_max(float x) {
+  x = fmaxf(x, __shfl_xor(x, 16, WAVE));
+  return fmaxf(x, __shfl_xor(x, 32, WAVE));
+}
+
+template <int DK, int DV, int KT, bool INROW>
+__global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
+    const DecodeArgs a) {
+  constexpr int KP = DK / 8, VP = INROW ? KP : DV / 8;  // pieces of a row
+  constexpr int NK = DK / 32, ND = DV / 64;
+  constexpr int KB = KT * DK * 2, VB = INROW ? 0 : KT * DV * 2;
+  constexpr int HALVES = 64 / KT;
+  static_assert(KT == 64 || KT == 32, "four waves make the scores of a tile");
+  static_assert(NK % HALVES == 0 && KB % 4096 == 0 && VB % 4096 == 0, "sizes");
+  __shared__ __attribute__((aligned(16))) char smem[2 * (KB + VB)];
+  __shared__ float sc[2][HALVES][KT][16];
+
+  const int S = (int)min(a.s_ptr ? (long)*a.s_ptr + 1 : (long)a.S, a.cap);
+  const int b = blockIdx.x / a.Hkv, hk = blockIdx.x % a.Hkv;
+  const int G = a.Hq / a.Hkv;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int l16 = lane & 15, lg = lane >> 4;
+
+  const int lo = a.window > 0 && S > a.window ? S - a.window : 0;
+  const int per = ((S - lo + a.nsplit - 1) / a.nsplit + KT - 1) / KT * KT;
+  const int from = min(S, lo + per * (int)blockIdx.y);
+  const int to = min(S, from + per);
+
+  const char* kbase = a.k + (long)blockIdx.x * a.cap * (DK * 2);
+  const char* vbase = a.v + (long)blockIdx.x * a.cap * (DV * 2);
+  // rows behind the slice repeat its last one; their weights are zero
+  auto stage = [&](int t, int buf) {
+    char* dst = smem + buf * (KB + VB);
+    const char* ks = kbase + (long)t * (DK * 2);
+    const char* vs = vbase + (long)t * (DV * 2);
+    const int last = to - 1 - t;
+#pragma unroll
+    for (int i = 0; i < KB / 4096; ++i) {
+      const int part = i * 4 + wid, s = part * 64 + lane, row = s / KP;
+      dt_to_lds(ks + min(row, last) * (DK * 2) +
+                    dt_place<KP, true>(row, s % KP) * 16, dst + part * 1024);
+    }
+#pragma unroll
+    for (int i = 0; i < VB / 4096; ++i) {
+      const int part = i * 4 + wid, s = part * 64 + lane, row = s / VP;
+      dt_to_lds(vs + min(row, last) * (DV * 2) +
+                    dt_place<VP, false>(row, s % VP) * 16,
+                dst + KB + part * 1024);
+    }
+  };
+  if (from < to) stage(from, 0);
+
+  const long row0 = (long)b * a.Hq + hk * G;  // first query head
+  const int kb = KT == 64 ? wid : wid & 1, half = KT == 64 ? 0 : wid >> 1;
+  bf16x8_t qf[NK / HALVES];
+  {
+    const char* src = a.q + (row0 + min(l16, G - 1)) * (DK * 2) +
+                      half * (NK / HALVES) * 64 + lg * 16;
+#pragma unroll
+    for (int i = 0; i < NK / HALVES; ++i)
+      qf[i] = *reinterpret_cast<const bf16x8_t*>(src + i * 64);
+  }
+  float m = -1e30f, l = 0.0f;  // reference of the exponents (base 2), sum
+  f32x4 o[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) o[d] = f32x4{0, 0, 0, 0};
+
+  int buf = 0;
+  for (int t = from; t < to; t += KT, buf ^= 1) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (t + KT < to) stage(t + KT, buf ^ 1);
+    const char* kt = smem + buf * (KB + VB);
+    const char* vt = kt + KB;
+
+    f32x4 s4 = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < NK / HALVES; ++i) {
+      const int piece = (half * (NK / HALVES) + i) * 4 + lg;
+      const bf16x8_t f = *reinterpret_cast<const bf16x8_t*>(
+          kt + (kb * 16 + l16) * KP * 16 + dt_place<KP, true>(l16, piece) * 16);
+      s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f, qf[i], s4, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sc[buf][half][kb * 16 + lg * 4 + r][l16] = s4[r];
+    __syncthreads();
+
+    float p[KT / 32][8], top = -INFINITY;
+#pragma unroll
+    for (int x = 0; x < KT / 32; ++x)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = x * 32 + (j >> 2) * 16 + lg * 4 + (j & 3);
+        float v = sc[buf][0][key][l16];
+        if (HALVES == 2) v += sc[buf][HALVES - 1][key][l16];
+        if (a.cap_out > 0.0f) {
+          const float e = __builtin_amdgcn_exp2f(v * a.cap_in);
+          v = a.cap_out - 2.0f * a.cap_out * __builtin_amdgcn_rcpf(e + 1.0f);
+        } else {
+          v *= a.c;
+        }
+        p[x][j] = t + key < to ? v : -INFINITY;
+        top = fmaxf(top, p[x][j]);
+      }
+    top = column_max(top);
+    const float m_new = fmaxf(m, top);
+    if (__any(m_new > m)) {
+      const float f = __builtin_amdgcn_exp2f(m - m_new);
+      m = m_new;
+      l *= f;
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[d][r] *= f;
+    }
+#pragma unroll
+    for (int x = 0; x < KT / 32; ++x) {
+      bf16x8_t high, low;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float w = __builtin_amdgcn_exp2f(p[x][j] - m);
+        l += w;
+        high[j] = (__bf16)w;
+        low[j] = (__bf16)(w - (float)high[j]);
+      }
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        const int row = lg * 4 + (l16 >> 2);  // of this half of 16 keys
+        const int piece = (wid * ND + d) * 2 + (l16 >> 1 & 1);
+        const char* src = vt + (x * 32 + row) * VP * 16 +
+                          dt_place<VP, INROW>(row, piece) * 16 + (l16 & 1) * 8;
+        const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(INROW ? src - KB : src));
+        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(
+                (INROW ? src - KB : src) + 16 * VP * 16));
+        const bf16x8_t v = __builtin_bit_cast(
+            bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, high, o[d], 0, 0, 0);
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, low, o[d], 0, 0, 0);
+      }
+    }
+  }
+
+  l += __shfl_xor(l, 16, WAVE);
+  l += __shfl_xor(l, 32, WAVE);
+  if (l16 >= G) return;
+  const long row = row0 + l16;
+  const int col = wid * ND * 16 + lg * 4;
+  if (a.nsplit == 1) {
+    const float f = 1.0f / l;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      bf16 w[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) w[r] = f2bf(o[d][r] * f);
+      *reinterpret_cast<short4v*>(a.out + (row * DV + col + d * 16) * 2) =
+          *reinterpret_cast<short4v*>(w);
+    }
+    return;
+  }
+  const long part = row * a.nsplit + blockIdx.y;
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+    *reinterpret_cast<f32x4*>(a.part_o + part * DV + col + d * 16) = o[d];
+  if (wid == 0 && lg == 0) {
+    a.part_ml[part * 2] = m;
+    a.part_ml[part * 2 + 1] = l;
+  }
+}
+
+// One block per query head: weighs the slices (an empty one has sum zero) and
+// adds them up, four columns a thread.
+__global__ __launch_bounds__(128) void attn_decode_merge_kernel(
+    const float* __restrict__ part_o, const float* __restrict__ part_ml,
+    short* __restrict__ out, int n, int Dv) {
+  __shared__ float w[DT_MAXSPLIT];
+  const long row = blockIdx.x;
+  if (threadIdx.x < WAVE) {
+    const int s = threadIdx.x;
+    const float ms = s < n ? part_ml[(row * n + s) * 2] : -1e30f;
+    const float ls = s < n ? part_ml[(row * n + s) * 2 + 1] : 0.0f;
+    const float e = __builtin_amdgcn_exp2f(ms - wave_max(ms));
+    w[s] = e / wave_sum(ls * e);
+  }
+  __syncthreads();
+  for (int d = threadIdx.x * 4; d < Dv; d += 512) {
+    const float* p = part_o + row * n * Dv + d;
+    f32x4 o = {0, 0, 0, 0};
+#pragma unroll 8
+    for (int s = 0; s < n; ++s) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(p + (long)s * Dv);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] += v[j] * w[s];
+    }
+    bf16 r[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[j] = f2bf(o[j]);
+    *reinterpret_cast<short4v*>(out + row * Dv + d) =
+        *reinterpret_cast<short4v*>(r);
+  }
+}
+
+// head sizes (keys, values), keys of a tile, values within the keys' rows
+#define DT_SIZES(DO)                                                         \
+  DO(64, 64, 64, false) DO(128, 128, 64, false) DO(192, 128, 32, false)      \
+  DO(256, 256, 32, false) DO(576, 512, 32, true)
+
+extern "C" int attn_decode_tile(int G, int Dk, int Dv, bool inrow) {
+  if (G > 16) return 0;
+#define DT_HAS(K, V, T, R) if (Dk == K && Dv == V && inrow == R) return T;
+  DT_SIZES(DT_HAS)
+#undef DT_HAS
+  return 0;
+}
+
+template <int DK, int DV, int KT, bool INROW>
+static void attn_decode_tile_go(const DecodeArgs& a, int B, hipStream_t stream) {
+  attn_decode_tile_kernel<DK, DV, KT, INROW>
+      <<<dim3((unsigned)(B * a.Hkv), (unsigned)a.nsplit), dim3(AD_BLOCK), 0,
+         stream>>>(a);
+  if (a.nsplit > 1)
+    attn_decode_merge_kernel<<<dim3((unsigned)(B * a.Hq)), dim3(128), 0,
+                               stream>>>(a.part_o, a.part_ml, (short*)a.out,
+                                         a.nsplit, DV);
+}
+
+// q [B, Hq, Dk]; all bases are multiples of 16 bytes
+extern "C" void launch_attn_decode_tile(
+    const void* q, const void* k, const void* v, void* out, float* part_o,
+    float* part_ml, int nsplit, const int* s_ptr, int B, int Hq, int Hkv, int S,
+    long Scap, int Dk, int Dv, bool inrow, float scale, float softcap,
+    int window, hipStream_t stream) {
+  constexpr float LOG2E = 1.44269504088896340736f;
+  DecodeArgs a{(const char*)q, (const char*)k, (const char*)v, (char*)out,
+               part_o, part_ml, s_ptr, Hq, Hkv, S, nsplit, window, Scap,
+               scale * LOG2E, 0.0f, 0.0f};
+  if (softcap > 0.0f) {
+    a.cap_in = 2.0f * a.c / softcap;
+    a.cap_out = softcap * LOG2E;
+  }
+#define DT_GO(K, V, T, R)                         \
+  if (Dk == K && Dv == V && inrow == R)           \
+    attn_decode_tile_go<K, V, T, R>(a, B, stream);
+  DT_SIZES(DT_GO)
+#undef DT_GO
+}

@@ -30,6 +30,11 @@ void launch_attn_decode(const void*, const void*, const void*, void*, float*,
                         float*, int, const int*, int, int, int, int, long,
                         int, int, long, float, float, int, hipStream_t);
 bool attn_decode_supported_shape(int, int);
+int attn_decode_tile(int, int, int, bool);
+void launch_attn_decode_tile(const void*, const void*, const void*, void*,
+                             float*, float*, int, const int*, int, int, int,
+                             int, long, int, int, bool, float, float, int,
+                             hipStream_t);
 void launch_attn_prefill(const void*, const void*, const void*, void*, int,
                          int, int, int, int, long, long, long, long, long, int,
                          int, float, float, int, int, hipStream_t);
@@ -284,6 +289,17 @@ void mla_append_kv(torch::Tensor kvh, torch::Tensor kpe, torch::Tensor kcache,
 
 // q [B, Hq, 1, Dk]; k/v: cache views [B, Hkv, S, D] with row-contiguous
 // last dim over a [B, Hkv, Scap, D] buffer.
+// Slices of the keys for the tile kernel: up to 512 blocks, two a CU, which are
+// all at work at once, and no slice under one tile.  256 blocks leave half of the
+// loads in flight unused (5 sequences of 5004 keys, 8 heads of 256: 68 us, 45 with
+// 512), 1024 come in two rounds and double what the merge reads (48 us; 64 cached
+// latents of 2048 tokens: 49 us, 40 with 512).
+static int decode_slices(long pairs, long span, int tile) {
+  return (int)std::max<long>(
+      1, std::min<long>({64, 512 / std::max<long>(pairs, 1),
+                         (span + tile - 1) / tile}));
+}
+
 torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                           double scale, double softcap, int64_t window,
                           c10::optional<torch::Tensor> pos) {
@@ -313,6 +329,29 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
     TORCH_CHECK(pos->scalar_type() == torch::kInt32, "pos must be int32");
     s_ptr = pos->data_ptr<int>();
   }
+  auto fopts = qc.options().dtype(torch::kFloat32);
+  const auto at16 = [](const torch::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  const bool inrow = v.data_ptr() == k.data_ptr() && vstride == Dk && Dv < Dk;
+  const int tile = at16(qc) && at16(k) && at16(v) && (inrow || vstride == Dv)
+                       ? attn_decode_tile(Hq / Hkv, Dk, Dv, inrow)
+                       : 0;
+  if (tile) {
+    const int nsplit = decode_slices((long)B * Hkv, s_ptr ? kScap : (long)S, tile);
+    torch::Tensor po, pml;
+    if (nsplit > 1) {
+      po = torch::empty({(long)B * Hq * nsplit * Dv}, fopts);
+      pml = torch::empty({(long)B * Hq * nsplit * 2}, fopts);
+    }
+    launch_attn_decode_tile(
+        qc.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+        nsplit > 1 ? po.data_ptr<float>() : nullptr,
+        nsplit > 1 ? pml.data_ptr<float>() : nullptr, nsplit, s_ptr, B, Hq, Hkv,
+        S, kScap, Dk, Dv, inrow, (float)scale, (float)softcap, (int)window,
+        cur_stream());
+    return out;
+  }
   // split-S for parallelism: target ~1024 blocks, slices of >= 512 keys
   // (>= 256 keys when B*Hkv alone leaves the chip block-starved, e.g.
   // absorbed MLA with Hkv = 1)
@@ -325,7 +364,6 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   float* part_ml = nullptr;
   torch::Tensor po, pml;
   if (nsplit > 1) {
-    auto fopts = qc.options().dtype(torch::kFloat32);
     po = torch::empty({(long)B * Hq * nsplit * Dv}, fopts);
     pml = torch::empty({(long)B * Hq * nsplit * 2}, fopts);
     part_o = po.data_ptr<float>();

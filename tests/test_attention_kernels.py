@@ -84,3 +84,33 @@ def test_prefill_large_scores():
         # scores of up to 1200 are off by 2^-24 of themselves each way
         bound = 2.0 ** -8 * (size + expect.abs()) + 2.0 ** -12 * size + 1e-6
         assert bool(((out - expect).abs() <= bound).all()), scale
+
+
+DECODE = [(4, 4, 64, 64), (8, 1, 64, 64), (8, 2, 128, 128), (14, 2, 128, 128),
+          (12, 2, 128, 128), (16, 1, 128, 128), (3, 3, 192, 128),
+          (16, 8, 256, 256), (16, 1, 576, 512), (4, 1, 576, 512)]
+
+
+@pytest.mark.parametrize("captured", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,Dk,Dv", DECODE)
+def test_decode_edges(Hq, Hkv, Dk, Dv, captured):
+    """Tiles of 64 or 32 keys and slices of them: one key, one more and one less
+    than a tile, slices that are empty, windows that begin inside a tile; values
+    within the keys' rows; the length on the device."""
+    torch.manual_seed(Hq + Dk)
+    for S in (1, 2, 31, 33, 64, 65, 500, 3001):
+        for cap, window, scale in ((0.0, 0, 0.08), (30.0, 0, 0.1),
+                                   (0.0, 100, -0.08), (50.0, 64, 0.2)):
+            q = torch.randn(2, Hq, 1, Dk, dtype=torch.bfloat16, device="cuda") * 2
+            k = cached(2, Hkv, S, Dk, 70)
+            v = k[..., :Dv] if Dk == 576 else cached(2, Hkv, S, Dv, 70)
+            given, pos = (k, v), None
+            if captured:  # whole buffers and the last key's place
+                given = [t.as_strided((2, Hkv, S + 70, t.shape[3]), t.stride())
+                         for t in (k, v)]
+                pos = torch.tensor([S - 1], dtype=torch.int32, device="cuda")
+            out = ext().attn_decode(q, *given, scale, cap, window, pos).double()
+            expect, size = attention(q, k, v, scale, cap, window, S - 1)
+            # the result is rounded to bf16; 32-bit weights in two bf16 parts
+            bound = 2.0 ** -8 * expect.abs() + 2.0 ** -13 * size + 1e-6
+            assert bool(((out - expect).abs() <= bound).all()), (S, cap, window)
