@@ -71,6 +71,27 @@ class Linear(nn.Module):
         return y
 
 
+def project(m, x: torch.Tensor, *, norm: Optional[nn.Module] = None,
+            act: Optional[str] = None,
+            residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """ops.project with the weights of a Linear or FusedColumns, packed ones
+    through their bf16 copy."""
+    w, q = m.weight, m.quant
+    if q is not None:
+        w = ops.resident_weight(m.weight, m.scales, m.biases, x.shape[-1],
+                                q.group_size, q.bits)
+    if w is not None:
+        return ops.project(x, w, m.bias, norm=norm, act=act, residual=residual)
+    # no room for the copy
+    if norm is not None:
+        x = norm(x)
+    y = ops.quantized_linear(x, m.weight, m.scales, m.biases, q.group_size,
+                             q.bits)
+    if m.bias is not None:
+        y = y + m.bias
+    return ops.finish(y, act, residual)
+
+
 class RMSNorm(nn.Module):
     def __init__(self, dim: int, eps: float = 1e-5, weight_offset: float = 0.0,
                  dtype: torch.dtype = torch.bfloat16):

@@ -17,7 +17,7 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, QuantConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import Linear, RMSNorm, StageModel, owned_layer_indices
+from .base import Linear, RMSNorm, StageModel, owned_layer_indices, project
 from .llama import LlamaMLP, _Inner
 
 
@@ -193,12 +193,31 @@ class MLAAttention(nn.Module):
         self._w_uk = w[:, : self.qk_nope, :].contiguous()
         self._w_uv = w[:, self.qk_nope:, :].transpose(1, 2).contiguous()
 
-    def forward(self, x, cos, sin, cache: Optional[KVCache]):
+    def forward(self, x, cos, sin, cache: Optional[KVCache],
+                norm: Optional[RMSNorm] = None,
+                residual: Optional[torch.Tensor] = None):
+        """norm: for x's rows first; residual: added to what is returned.  For
+        few tokens, where both go with the projections."""
+        if norm is not None and self._fused_qkv is None:
+            x, norm = norm(x), None
         if cache is not None and cache.n_kv_heads == 1 and self.n_heads > 1:
-            return self._forward_absorbed(x, cos, sin, cache)
-        return self._forward_naive(x, cos, sin, cache)
+            return self._forward_absorbed(x, cos, sin, cache, norm, residual)
+        return self._forward_naive(x, cos, sin, cache, norm, residual)
 
-    def _forward_absorbed(self, x, cos, sin, cache: KVCache):
+    def _queries_and_latent(self, x, norm):
+        """(queries, cached row before norm and rotation) where one projection
+        makes both."""
+        if norm is None:
+            return self._fused_qkv(x)
+        return project(self._fused_qkv, x, norm=norm).split(
+            self._fused_qkv.splits, -1)
+
+    def _output(self, out, residual):
+        if residual is None:
+            return self.o_proj(out)
+        return project(self.o_proj, out, residual=residual)
+
+    def _forward_absorbed(self, x, cos, sin, cache: KVCache, norm, residual):
         """Compressed-cache path: cache rows are [c_kv | k_pe] (rank +
         rope).  Decode = MQA over the compressed rows with q/out
         absorbed through W_UK/W_UV; prefill expands K/V from the
@@ -209,7 +228,7 @@ class MLAAttention(nn.Module):
         nh, rank, rope = self.n_heads, self.kv_lora_rank, self.qk_rope
         ckv = None
         if self._fused_qkv is not None:
-            qh, ckv = self._fused_qkv(x)
+            qh, ckv = self._queries_and_latent(x, norm)
         elif self.q_lora_rank:
             qh = self.q_b_proj(self.q_a_layernorm(self.q_a_proj(x)))
         else:
@@ -250,7 +269,7 @@ class MLAAttention(nn.Module):
             ov = torch.bmm(o.permute(1, 0, 2, 3).reshape(nh, B * T, rank),
                            self._w_uv)
             out = ov.view(nh, B, T, self.v_head_dim).permute(1, 2, 0, 3)
-            return self.o_proj(out.reshape(B, T, -1))
+            return self._output(out.reshape(B, T, -1), residual)
 
         # prefill: expand the WHOLE compressed prefix (covers chunked
         # prefill, where earlier chunks live only in the cache)
@@ -275,13 +294,14 @@ class MLAAttention(nn.Module):
             v = kvh[..., self.qk_nope:].transpose(1, 2).contiguous()
         qf = torch.cat([q_nope, q_pe], dim=-1).transpose(1, 2)
         out = ops.attention(qf, k, v, self.scale, causal_offset=offset)
-        return self.o_proj(out.transpose(1, 2).reshape(B, T, -1))
+        return self._output(out.transpose(1, 2).reshape(B, T, -1), residual)
 
-    def _forward_naive(self, x, cos, sin, cache: Optional[KVCache]):
+    def _forward_naive(self, x, cos, sin, cache: Optional[KVCache], norm,
+                       residual):
         B, T, _ = x.shape
         ckv = None
         if self._fused_qkv is not None:
-            qh, ckv = self._fused_qkv(x)
+            qh, ckv = self._queries_and_latent(x, norm)
         elif self.q_lora_rank:
             qh = self.q_b_proj(self.q_a_layernorm(self.q_a_proj(x)))
         else:
@@ -326,7 +346,7 @@ class MLAAttention(nn.Module):
                 k, v = cache.update(k, v)
         out = ops.attention(qf, k, v, self.scale, causal_offset=offset,
                             pos_dev=gp)
-        return self.o_proj(out.transpose(1, 2).reshape(B, T, -1))
+        return self._output(out.transpose(1, 2).reshape(B, T, -1), residual)
 
 
 class DeepseekV2MoE(nn.Module):
@@ -403,6 +423,11 @@ class DeepseekV2DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
     def forward(self, x, cos, sin, cache):
+        if ops.few_tokens(x):
+            h = self.self_attn(x, cos, sin, cache, self.input_layernorm, x)
+            if isinstance(self.mlp, LlamaMLP):
+                return self.mlp(h, self.post_attention_layernorm, h)
+            return h + self.mlp(self.post_attention_layernorm(h))
         attn = self.self_attn(self.input_layernorm(x), cos, sin, cache)
         # fused: h = x + attn; y = rms_norm(h) in one kernel
         pn = self.post_attention_layernorm

@@ -18,7 +18,7 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import Linear, RMSNorm, StageModel, owned_layer_indices
+from .base import Linear, RMSNorm, StageModel, owned_layer_indices, project
 from .llama import _Inner
 
 
@@ -40,9 +40,17 @@ class Gemma2Attention(nn.Module):
         self.o_proj = Linear(self.n_heads * self.head_dim, H, q("o_proj"))
         self._fused_qkv = None  # set by fuse_model()
 
-    def forward(self, x, cos, sin, cache: Optional[KVCache]):
+    def forward(self, x, cos, sin, cache: Optional[KVCache],
+                norm: Optional[RMSNorm] = None):
+        """norm: for x's rows first (few tokens, where it goes with the
+        projection)."""
         B, T, _ = x.shape
-        if self._fused_qkv is not None:
+        if norm is not None and self._fused_qkv is None:
+            x, norm = norm(x), None
+        if norm is not None:
+            q, k, v = project(self._fused_qkv, x, norm=norm).split(
+                self._fused_qkv.splits, -1)
+        elif self._fused_qkv is not None:
             q, k, v = self._fused_qkv(x)
         else:
             q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
@@ -83,7 +91,13 @@ class Gemma2MLP(nn.Module):
         self.down_proj = Linear(I, H, q("down_proj"))
         self._fused_gu = None  # set by fuse_model()
 
-    def forward(self, x):
+    def forward(self, x, norm: Optional[RMSNorm] = None):
+        """norm: as in Gemma2Attention."""
+        if self._fused_gu is not None and ops.few_tokens(x):
+            return self.down_proj(project(self._fused_gu, x, norm=norm,
+                                          act="gelu_tanh"))
+        if norm is not None:
+            x = norm(x)
         if self._fused_gu is not None:
             g, u = self._fused_gu(x)
         else:
@@ -104,6 +118,11 @@ class Gemma2DecoderLayer(nn.Module):
         self.post_feedforward_layernorm = RMSNorm(H, eps, weight_offset=1.0)
 
     def forward(self, x, cos, sin, cache):
+        if ops.few_tokens(x):
+            h = x + self.post_attention_layernorm(
+                self.self_attn(x, cos, sin, cache, self.input_layernorm))
+            return h + self.post_feedforward_layernorm(
+                self.mlp(h, self.pre_feedforward_layernorm))
         h = x + self.post_attention_layernorm(
             self.self_attn(self.input_layernorm(x), cos, sin, cache))
         return h + self.post_feedforward_layernorm(

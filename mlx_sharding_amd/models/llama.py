@@ -16,7 +16,7 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import Linear, RMSNorm, StageModel, owned_layer_indices
+from .base import Linear, RMSNorm, StageModel, owned_layer_indices, project
 
 
 class LlamaAttention(nn.Module):
@@ -40,10 +40,19 @@ class LlamaAttention(nn.Module):
         self._fused_qkv = None  # set by fuse_model()
 
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
-                cache: Optional[KVCache]) -> torch.Tensor:
+                cache: Optional[KVCache], norm: Optional[RMSNorm] = None,
+                residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """norm: for x's rows first; residual: added to what is returned.  For
+        few tokens, where both go with the projections."""
         B, T, _ = x.shape
-        if self._fused_qkv is not None:
+        if self._fused_qkv is not None and norm is not None:
+            q, k, v = project(self._fused_qkv, x, norm=norm).split(
+                self._fused_qkv.splits, -1)
+        elif self._fused_qkv is not None:
             q, k, v = self._fused_qkv(x)
+        elif norm is not None:
+            q, k, v = (project(m, x, norm=norm)
+                       for m in (self.q_proj, self.k_proj, self.v_proj))
         else:
             q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
         q = q.view(B, T, self.n_heads, self.head_dim)
@@ -70,6 +79,8 @@ class LlamaAttention(nn.Module):
         out = ops.attention(q, k, v, self.scale, causal_offset=offset,
                             pos_dev=gp)
         out = out.transpose(1, 2).reshape(B, T, -1)
+        if residual is not None:
+            return project(self.o_proj, out, residual=residual)
         return self.o_proj(out)
 
 
@@ -84,7 +95,16 @@ class LlamaMLP(nn.Module):
         self.down_proj = Linear(I, H, q("down_proj"))
         self._fused_gu = None  # set by fuse_model()
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, norm: Optional[RMSNorm] = None,
+                residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """norm, residual: as in LlamaAttention."""
+        if self._fused_gu is not None and ops.few_tokens(x):
+            y = project(self._fused_gu, x, norm=norm, act="silu")
+            return project(self.down_proj, y, residual=residual)
+        if norm is not None:
+            x = norm(x)
+        if residual is not None:
+            return residual + self(x)
         if self._fused_gu is not None:
             g, u = self._fused_gu(x)
         else:
@@ -102,6 +122,9 @@ class LlamaDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
     def forward(self, x, cos, sin, cache):
+        if ops.few_tokens(x):
+            h = self.self_attn(x, cos, sin, cache, self.input_layernorm, x)
+            return self.mlp(h, self.post_attention_layernorm, h)
         attn = self.self_attn(self.input_layernorm(x), cos, sin, cache)
         # fused: h = x + attn; y = rms_norm(h) in one kernel
         pn = self.post_attention_layernorm

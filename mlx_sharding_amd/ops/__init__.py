@@ -208,8 +208,87 @@ def _dq_cache_ok(nbytes: int) -> bool:
     return True
 
 
+_FEW_ROWS = 16  # tokens of a batch that linear_few takes
+_ACTS = {None: 0, "silu": 1, "gelu_tanh": 2}
+
+
+def _plain(t: torch.Tensor) -> bool:
+    """An ordinary tensor that nothing differentiates, maps or traces."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter)
+            and not (t.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and torch.autograd.forward_ad._current_level < 0)
+
+
+def few_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether x W^T runs on linear_few.hip: up to 16 bf16 rows that begin, as
+    W's, at whole 16-byte vectors.  A contraction above 8192 only for 8 rows: 16
+    rows of 14336 into 4096 take 29 us there and 26 in the library, 8 take 24.6
+    and 26.6."""
+    K = weight.shape[-1]
+    rows = x.numel() // K if K else 0
+    return (0 < rows <= (_FEW_ROWS if K <= 8192 else 8) and _use_hip(x)
+            and weight.dim() == 2 and K % 32 == 0 and weight.shape[0] > 0
+            and x.dtype == weight.dtype == torch.bfloat16 and weight.is_cuda
+            and _plain(x) and _plain(weight) and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
+            and x.stride(-1) == 1 and weight.data_ptr() % 16 == 0
+            and x.data_ptr() % 16 == 0
+            and all(s % 8 == 0 for s in x.stride()[:-1])
+            and _few_ext() is not None)
+
+
+def _few_ext():
+    if _load_ext() is not None:
+        return _EXT
+    from .ragged import hip_ragged
+    return hip_ragged()
+
+
+def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None):
+    x2 = x.reshape(-1, x.shape[-1])
+    if x2.data_ptr() % 16 or x2.stride(0) % 8:
+        x2 = x2.clone()
+    if residual is not None:
+        residual = residual.reshape(x2.shape[0], -1)
+    y = _few_ext().linear_few(
+        x2, weight, bias, residual, None if norm is None else norm.weight,
+        0.0 if norm is None else norm.eps,
+        0.0 if norm is None else norm.weight_offset, _ACTS[act])
+    return y.view(*x.shape[:-1], y.shape[-1])
+
+
+def project(x, weight, bias=None, *, norm=None, act=None, residual=None):
+    """x W^T + bias, of x's rows as ``norm`` (an RMSNorm) makes them; ``act``:
+    the gated unit act(gate) * up of the result's halves; plus ``residual``.
+    One kernel for few rows, else one for each of these."""
+    if (few_rows(x, weight) and (bias is None or _plain(bias))
+            and (norm is None or norm.weight.data_ptr() % 16 == 0
+                 and norm.weight.dtype == torch.bfloat16)
+            and (residual is None or residual.dtype == torch.bfloat16
+                 and residual.stride(-1) == 1)):
+        return _linear_few(x, weight, bias, residual, norm, act)
+    if norm is not None:
+        x = norm(x)
+    return finish(linear(x, weight, bias), act, residual)
+
+
+def finish(y, act=None, residual=None):
+    """The gated unit of y's halves, plus a residual; either may be left out."""
+    if act is not None:
+        half = y.shape[-1] // 2
+        y = (swiglu if act == "silu" else geglu)(y[..., :half], y[..., half:])
+    return y if residual is None else residual + y
+
+
+def few_tokens(x: torch.Tensor) -> bool:
+    """Whether a layer's projections on x take what lies between them along
+    (``project``)."""
+    return (x.dtype == torch.bfloat16 and use_native(x) and _plain(x)
+            and 0 < x.numel() <= _FEW_ROWS * x.shape[-1])
+
+
 def linear(x, weight, bias=None):
-    """Dense linear.  The MFMA decode GEMV (MLXS_AMD_DENSE_GEMV=1) was
+    """Dense linear; up to 16 rows run on linear_few.hip.  The MFMA decode GEMV (MLXS_AMD_DENSE_GEMV=1) was
     a NEGATIVE result at batch-64 decode shapes: hipBLASLt's small-GEMM
     kernels run ~13 us in-graph and the split-K fp32-atomic traffic
     (M*O*4*nk bytes) rivals the weight bytes on small-O projections
@@ -258,7 +337,21 @@ def linear(x, weight, bias=None):
             if bias is not None:
                 y = y + bias
             return y.reshape(*lead, y.shape[-1])
+    if few_rows(x, weight) and (bias is None or _plain(bias)):
+        return _linear_few(x, weight, bias)
     return torch.nn.functional.linear(x, weight, bias)
+
+
+def resident_weight(w_q, scales, biases, in_features: int, group_size: int,
+                    bits: int):
+    """The bf16 copy of a quantized projection on the GPU that is kept beside it,
+    or None where the budget has no room for it."""
+    w = getattr(w_q, "_mlxs_dqw", None)
+    if w is None and _dq_cache_ok(w_q.shape[0] * in_features * 2):
+        w = _require_ext("quantized_linear").dequant(
+            w_q, scales, biases, in_features, group_size, bits)
+        w_q._mlxs_dqw = w
+    return w
 
 
 def quantized_linear(x, w_q, scales, biases, group_size: int, bits: int):
@@ -275,11 +368,7 @@ def quantized_linear(x, w_q, scales, biases, group_size: int, bits: int):
         # memory is tight (MLXS_AMD_NO_DQ_CACHE=1 disables the cache;
         # routed EXPERT weights — the bulk of an MoE checkpoint — stay
         # packed and use the w4 MFMA kernels).
-        w = getattr(w_q, "_mlxs_dqw", None)
-        O = w_q.shape[0]
-        if w is None and _dq_cache_ok(O * H * 2):
-            w = ext.dequant(w_q, scales, biases, H, group_size, bits)
-            w_q._mlxs_dqw = w
+        w = resident_weight(w_q, scales, biases, H, group_size, bits)
         if w is not None:
             y = linear(x2, w)
         elif (M <= _GEMV_MAX_M and group_size in (32, 64, 128)

@@ -6,6 +6,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include "hip_common.h"
+#include "linear_few.h"
 
 extern "C" {
 void launch_rms_norm(const void*, void*, const void*, long, int, float, float,
@@ -748,6 +749,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill_shape_ok", [](int64_t dk, int64_t dv) {
     return attn_prefill_supported((int)dk, (int)dv);
   });
+  m.def("linear_few", &linear_few);
+  m.def("linear_few", &linear_few);
   m.def("mfma_probe", &mfma_probe);
   m.def("w4a16_gemv", &w4a16_gemv);
   m.def("w4f16_gemv", &w4f16_gemv);

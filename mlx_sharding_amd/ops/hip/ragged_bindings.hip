@@ -2,6 +2,7 @@
 // Every operand's device, type, shape and alignment is checked here, before
 // anything is launched.
 
+#include "linear_few.h"
 #include "ragged_bindings.h"
 #include "ragged_grouped.h"
 #include "ragged_prefill.h"
@@ -816,6 +817,7 @@ Tensor cap_logits(Tensor z, double scale, double limit) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("glu", &glu);
+  m.def("linear_few", &linear_few);
   m.def("clamped_glu", &clamped_glu, py::arg("gate"), py::arg("up"),
         py::arg("limit"), py::arg("alpha"), py::arg("gate_bias") = py::none(),
         py::arg("up_bias") = py::none());

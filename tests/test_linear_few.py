@@ -1,0 +1,104 @@
+"""The product for few rows and what goes with it, against 64 bits."""
+
+import types
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from mlx_sharding_amd import ops
+
+
+def make(M, O, K, act, wide):
+    g = torch.Generator().manual_seed(M + O + K)
+    new = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()  # noqa: E731
+    x = new(M, K + 8 * wide)[:, 8 * wide:]      # rows as slices of wider ones
+    w = (torch.randn(O, K + 16 * wide, generator=g) * 0.05).bfloat16().cuda()[:, :K]
+    norm = types.SimpleNamespace(weight=new(K), eps=1e-5, weight_offset=1.0)
+    return x, w, norm, new(O), new(M, O // 2 if act else O)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,O,K", [
+    (1, 2, 32), (3, 18, 96), (16, 34, 2080), (5, 4098, 64), (16, 8194, 160),
+    (4, 8210, 32), (9, 4100, 256), (2, 16386, 96), (16, 16400, 1056),
+    (8, 96, 14336), (7, 8200, 2016)])
+def test_edges(M, O, K):
+    """Tiles of 16, 32 and 64 columns with remainders, contractions that are not
+    whole chunks, fewer steps than waves; norm, bias, unit, residual."""
+    for act in (None, "silu", "gelu_tanh"):
+        x, w, norm, bias, res = make(M, O, K, act, wide=K % 64 == 0)
+        assert ops.few_rows(x, w)
+        for normed in (False, True):
+            for rest in (False, True):
+                b, r = (bias, res) if rest else (None, None)
+                y = ops.project(x, w, b, norm=norm if normed else None, act=act,
+                                residual=r).double()
+                h, size = x.double(), x.double().abs()
+                if normed:
+                    f = torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + 1e-5)
+                    h, size = ((t * f * (norm.weight.double() + 1.0)) for t in (h, size))
+                z = h @ w.double().T
+                # 32-bit sums, and rows rounded to bf16 behind the norm
+                off = (size.abs() @ w.double().abs().T) * (
+                    K * 2.0 ** -24 + (2.0 ** -8 if normed else 0.0))
+                if rest:
+                    z = z + bias.double()
+                if act:
+                    gate, up = z.chunk(2, -1)
+                    og, ou = off.chunk(2, -1)
+                    unit = F.silu if act == "silu" else lambda t: F.gelu(
+                        t, approximate="tanh")
+                    z = unit(gate) * up
+                    # both units grow by at most 1.13 of their argument
+                    off = 1.13 * og * (up.abs() + ou) + unit(gate).abs() * ou + 1e-6
+                if rest:
+                    z = z + res.double()
+                bound = 2.0 ** -8 * z.abs() + off + 1e-6
+                assert bool(((y - z).abs() <= bound).all()), (act, normed, rest)
+
+
+@pytest.mark.gpu
+def test_same_as_separate_kernels():
+    """What the projection takes along, beside the kernels it stands for."""
+    x, w, norm, bias, _ = make(16, 512, 256, None, wide=True)
+    several = torch.cat([x, x])                   # too many rows: separate
+    assert not ops.few_rows(several, w)
+    norm = types.SimpleNamespace(
+        weight=norm.weight, eps=1e-5, weight_offset=1.0)
+    one = ops.project(x, w, bias, act="silu")
+    two = ops.project(several, w, bias, act="silu")[:16]
+    assert (one.double() - two.double()).norm() < 0.01 * two.double().norm()
+
+
+@pytest.mark.gpu
+def test_other_forms_keep_the_library():
+    """Calls that the kernel does not take run as before."""
+    w = torch.randn(24, 64, device="cuda").bfloat16()
+    x = torch.randn(2, 3, 64, device="cuda").bfloat16()
+    expect = x.double() @ w.double().T
+    close = lambda y: (y.double() - expect).norm() < 0.01 * expect.norm()  # noqa: E731
+    assert close(ops.linear(x, w))
+    at = torch.randn(6 * 64 + 1, device="cuda").bfloat16()  # rows off 16 bytes
+    odd = at[1:].view(2, 3, 64)
+    odd.copy_(x)
+    assert not ops.few_rows(odd, w) and close(ops.linear(odd, w))
+    turned = w.t().contiguous().t()                 # columns side by side
+    assert not ops.few_rows(x, turned) and close(ops.linear(x, turned))
+    assert ops.linear(x.float(), w.float()).dtype == torch.float32
+    assert ops.linear(x[:, :0], w).shape == (2, 0, 24)
+    # what is differentiated or mapped
+    p = torch.nn.Parameter(w)
+    ops.linear(x, p).float().sum().backward()
+    assert p.grad is not None
+    assert close(torch.vmap(lambda r: ops.linear(r, w))(x))
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        tangent = torch.autograd.forward_ad.unpack_dual(ops.linear(dual, w)).tangent
+    assert tangent is not None
+
+
+def test_cpu_tensors_keep_torch():
+    x, w = torch.randn(2, 64).bfloat16(), torch.randn(24, 64).bfloat16()
+    assert not ops.few_rows(x, w) and not ops.few_tokens(x)
+    assert torch.equal(ops.linear(x, w), F.linear(x, w))
