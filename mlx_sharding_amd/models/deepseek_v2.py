@@ -378,6 +378,36 @@ class DeepseekV2MoE(nn.Module):
                 and n_tokens <= 128 and self.n_experts <= 64
                 and self.top_k <= 8)
 
+    def _packing(self):
+        """(bits, group size) of the routed experts; 16 bits: not packed."""
+        q = self.switch_mlp.quant
+        return (16, 128) if q is None else (q.bits, q.group_size)
+
+    def decodes(self, x) -> bool:
+        """Whether ``decode`` takes these tokens."""
+        m = self.switch_mlp
+        return (x.numel() <= 128 * x.shape[-1] and self.gate.bias is None
+                and self._fused_gate_ok(x.numel() // x.shape[-1])
+                and ops.expert_rows_ok(x, self.gate.weight, m.up_proj.weight,
+                                       m.down_proj.weight, self.top_k,
+                                       *self._packing()))
+
+    def decode(self, x, residual, norm):
+        """The residual x (+ residual) after this feed-forward of it, normed:
+        three kernels for the routed experts, with norm, router and choice in a
+        fourth."""
+        shape, H = x.shape, x.shape[-1]
+        y, h, choice, weight = ops.expert_route(
+            x.reshape(-1, H), None if residual is None else residual.reshape(-1, H),
+            norm, self.gate.weight, self.top_k, self.routed_scaling_factor,
+            self.norm_topk_prob)
+        m = self.switch_mlp
+        stacks = [[p.weight] if m.quant is None else [p.weight, p.scales, p.biases]
+                  for p in (m.gate_proj, m.up_proj, m.down_proj)]
+        rows = ops.expert_rows(y, choice, weight, *stacks, *self._packing())
+        shared = None if self.shared_experts is None else self.shared_experts(y)
+        return ops.expert_sum(rows, h, shared, y.shape[0]).view(shape)
+
     def forward(self, x):
         B, T, H = x.shape
         flat = x.reshape(-1, H)
@@ -423,11 +453,18 @@ class DeepseekV2DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
     def forward(self, x, cos, sin, cache):
+        experts = isinstance(self.mlp, DeepseekV2MoE)
+        decode = experts and self.mlp.decodes(x)
         if ops.few_tokens(x):
             h = self.self_attn(x, cos, sin, cache, self.input_layernorm, x)
-            if isinstance(self.mlp, LlamaMLP):
+            if decode:
+                return self.mlp.decode(h, None, self.post_attention_layernorm)
+            if not experts:
                 return self.mlp(h, self.post_attention_layernorm, h)
             return h + self.mlp(self.post_attention_layernorm(h))
+        if decode:
+            attn = self.self_attn(self.input_layernorm(x), cos, sin, cache)
+            return self.mlp.decode(attn, x, self.post_attention_layernorm)
         attn = self.self_attn(self.input_layernorm(x), cos, sin, cache)
         # fused: h = x + attn; y = rms_norm(h) in one kernel
         pn = self.post_attention_layernorm

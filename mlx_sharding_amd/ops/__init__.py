@@ -539,6 +539,62 @@ def moe_gate_subranges(router_logits_bf16, top_k: int,
                                         norm_topk_prob))
 
 
+_ROWS_PAIRS = 1024  # (token, expert) pairs that moe_rows.hip takes
+
+
+def expert_rows_ok(x, gate_w, up, down, top: int, bits: int, group_size: int
+                   ) -> bool:
+    """Whether a decoding step's routed experts run on moe_rows.hip.  gate_w: the
+    router's; up, down: stacked matrices of an expert kind (packed, or bf16 with
+    ``bits`` 16)."""
+    if not (x.dtype == torch.bfloat16 and use_native(x) and _plain(x)):
+        return False
+    per = 1 if bits == 16 else 32 // bits
+    E, I, H = up.shape[0], up.shape[1], up.shape[2] * per
+    longest = hip_ext().moe_rows_longest(bits)
+    return (E <= 64 and top <= E and 0 < x.numel() // H * top <= _ROWS_PAIRS
+            and H % 128 == 0 and I % 128 == 0 and max(H, I) <= longest
+            and tuple(down.shape) == (E, H, I // per)
+            and (bits == 16 or group_size in (32, 64, 128))
+            and gate_w.dtype == torch.bfloat16 and tuple(gate_w.shape) == (E, H))
+
+
+def expert_route(x, residual, norm, gate_w, top: int, scaling: float,
+                 normalize: bool):
+    """(rows of x + residual as ``norm`` makes them, x + residual, experts and
+    weights of every token), one kernel; rows [N, H]."""
+    return _require_ext("moe_route").moe_route(
+        x, residual, norm.weight, norm.eps, norm.weight_offset, gate_w, top,
+        scaling, normalize)
+
+
+def expert_rows(y, choice, weight, gate, up, down, bits: int, group_size: int):
+    """The chosen experts' weighted outputs, fp32 [N * top, H]; gate, up, down:
+    [matrix] in bf16 or [packed, scales, biases]."""
+    return _require_ext("moe_rows").moe_rows(
+        y, choice, weight, *(_expert_stack(m, bits, group_size)
+                             for m in (gate, up, down)), bits, group_size)
+
+
+def _expert_stack(m, bits: int, group_size: int) -> torch.Tensor:
+    """An expert kind's matrices as moe_rows.hip reads them; packed ones are laid
+    out at their first use and kept beside the checkpoint's."""
+    if bits == 16:
+        return m[0]
+    w = m[0]
+    packed = getattr(w, "_mlxs_rows", None)
+    if packed is None:
+        packed = _require_ext("moe_pack").moe_pack(*m, bits, group_size)
+        if not w.requires_grad and w.is_leaf:
+            w._mlxs_rows = packed
+    return packed
+
+
+def expert_sum(rows, h, shared, n_tokens: int):
+    """h + shared + a token's rows, bf16 [N, H]."""
+    return _require_ext("moe_combine").moe_combine(rows, h, shared, n_tokens)
+
+
 def grouped_expert_mlp_subs(x, gate_w, up_w, down_w, subs, max_tok: int = 4):
     """Run the grouped expert MLP from prebuilt sub-range arrays.
 

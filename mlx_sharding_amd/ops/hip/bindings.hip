@@ -7,6 +7,7 @@
 
 #include "hip_common.h"
 #include "linear_few.h"
+#include "moe_rows.h"
 
 extern "C" {
 void launch_rms_norm(const void*, void*, const void*, long, int, float, float,
@@ -625,6 +626,157 @@ torch::Tensor moe_w4_mfma(torch::Tensor x, torch::Tensor wq,
 
 // Fused fp16-dequant gate+up+SiLU over repacked quant words.
 // x [N, H] fp16; gq/uq [E, I, H*bits/32] repacked; scales/biases bf16.
+// -- routed experts of a decoding step (moe_rows.hip) -----------------------
+
+static void check_rows(const torch::Tensor& t, const char* name, long n, long w) {
+  check_bf16(t, name);
+  TORCH_CHECK(t.dim() == 2 && t.size(0) == n && t.size(1) == w &&
+                  t.is_contiguous() &&
+                  reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+              name, ": contiguous rows of ", w, " at 16 bytes");
+}
+
+// x [N, H] (+ residual) -> normed rows, x + residual (or x), experts and weights
+// of every token [N, top]
+std::vector<torch::Tensor> moe_route(torch::Tensor x,
+                                     c10::optional<torch::Tensor> residual,
+                                     torch::Tensor norm, double eps,
+                                     double offset, torch::Tensor gate,
+                                     int64_t top, double scaling,
+                                     bool normalize) {
+  TORCH_CHECK(x.dim() == 2 && gate.dim() == 2 && norm.dim() == 1, "shapes");
+  const long N = x.size(0), H = x.size(1), E = gate.size(0);
+  TORCH_CHECK(N >= 1 && H % 128 == 0 && H <= 8192,
+              "rows of a multiple of 128, up to 8192");
+  TORCH_CHECK(E >= 1 && E <= 64 && top >= 1 && top <= E, "up to 64 experts");
+  check_rows(x, "x", N, H);
+  check_rows(gate, "gate", E, H);
+  check_rows(norm.unsqueeze(0), "norm", 1, H);
+  if (residual.has_value()) check_rows(*residual, "residual", N, H);
+  auto y = torch::empty_like(x);
+  auto h = residual.has_value() ? torch::empty_like(x) : x;
+  auto choice = torch::empty({N, top}, x.options().dtype(torch::kInt32));
+  auto weight = torch::empty({N, top}, x.options().dtype(torch::kFloat32));
+  const MoeRouteArgs a{
+      (const __bf16*)x.data_ptr(),
+      residual.has_value() ? (const __bf16*)residual->data_ptr() : nullptr,
+      (const __bf16*)norm.data_ptr(), (const __bf16*)gate.data_ptr(),
+      (__bf16*)h.data_ptr(), (__bf16*)y.data_ptr(), choice.data_ptr<int>(),
+      weight.data_ptr<float>(), (int)H, (int)E, (int)top, (float)eps,
+      (float)offset, (float)scaling, normalize};
+  launch_moe_route(&a, (int)N, cur_stream());
+  return {y, h, choice, weight};
+}
+
+// Packed words [E, O, K * bits / 32] with scales and offsets [E, O, K / gs] in the
+// order of moe_rows.hip: [E, O / 16, K / 128, words of a tile]
+torch::Tensor moe_pack(torch::Tensor w, torch::Tensor scales,
+                       torch::Tensor offsets, int64_t bits, int64_t gs) {
+  TORCH_CHECK(bits == 4 || bits == 8, "4 or 8 bits");
+  TORCH_CHECK(gs == 32 || gs == 64 || gs == 128, "group size");
+  TORCH_CHECK(w.is_cuda() && w.dim() == 3 && w.element_size() == 4 &&
+                  w.is_contiguous() &&
+                  reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
+              "packed words, contiguous, at 16 bytes");
+  const long E = w.size(0), O = w.size(1), K = w.size(2) * 32 / bits;
+  TORCH_CHECK(K % 128 == 0 && O % 16 == 0, "whole tiles");
+  for (const auto& t : {scales, offsets}) {
+    check_bf16(t, "scales and offsets");
+    TORCH_CHECK(t.dim() == 3 && t.is_contiguous() && t.size(0) == E &&
+                    t.size(1) == O && t.size(2) == K / gs, "one per group");
+  }
+  auto out = torch::empty({E, O / 16, K / 128, moe_pack_words(bits, gs)},
+                          w.options().dtype(torch::kInt32));
+  if (out.numel())
+    launch_moe_pack(w.data_ptr(), scales.data_ptr(), offsets.data_ptr(),
+                    out.data_ptr(), (int)(E * O), (int)K, (int)bits, (int)gs,
+                    cur_stream());
+  return out;
+}
+
+// One stack of experts' matrices: from moe_pack, or bf16 [E, O, K]
+struct ExpertStack {
+  const void* w;
+  long E, O, K;
+};
+
+static ExpertStack expert_stack(const torch::Tensor& t, int bits, int gs) {
+  TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
+                  reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+              "stacks are contiguous, at 16 bytes");
+  ExpertStack s{t.data_ptr(), t.size(0), 0, 0};
+  if (bits == 16) {
+    check_bf16(t, "weights");
+    TORCH_CHECK(t.dim() == 3, "a stack");
+    s.O = t.size(1);
+    s.K = t.size(2);
+  } else {
+    TORCH_CHECK(t.dim() == 4 && t.scalar_type() == torch::kInt32 &&
+                    t.size(3) == moe_pack_words(bits, gs), "a packed stack");
+    s.O = t.size(1) * 16;
+    s.K = t.size(2) * 128;
+  }
+  TORCH_CHECK(s.K % 128 == 0 && s.O % 16 == 0 && s.K >= 128 && s.O >= 16 &&
+                  s.K <= moe_rows_longest(bits), "sizes of an expert");
+  return s;
+}
+
+// Every pair's expert output, weighted, fp32 [N * top, H]; bits 16: bf16 stacks
+torch::Tensor moe_rows(torch::Tensor x, torch::Tensor choice,
+                       torch::Tensor weight, torch::Tensor gate,
+                       torch::Tensor up, torch::Tensor down, int64_t bits,
+                       int64_t gs) {
+  TORCH_CHECK(bits == 4 || bits == 8 || bits == 16, "4, 8 or 16 bits");
+  TORCH_CHECK(bits == 16 || gs == 32 || gs == 64 || gs == 128, "group size");
+  const auto g = expert_stack(gate, bits, gs), u = expert_stack(up, bits, gs),
+             d = expert_stack(down, bits, gs);
+  TORCH_CHECK(g.E == u.E && g.O == u.O && g.K == u.K && d.E == g.E &&
+                  d.O == g.K && d.K == g.O, "stacks of one shape");
+  TORCH_CHECK(choice.dim() == 2 && choice.is_contiguous() &&
+                  choice.scalar_type() == torch::kInt32 && choice.is_cuda() &&
+                  weight.sizes() == choice.sizes() && weight.is_contiguous() &&
+                  weight.scalar_type() == torch::kFloat32 && weight.is_cuda(),
+              "choice int32, weight fp32 [N, top]");
+  const long N = choice.size(0), P = choice.numel();
+  TORCH_CHECK(P >= 1 && P <= MR_PAIRS, "up to ", MR_PAIRS, " pairs");
+  check_rows(x, "x", N, g.K);
+  auto h = torch::empty({P, g.O}, x.options().dtype(bits == 16 ? torch::kBFloat16
+                                                                : torch::kHalf));
+  auto y = torch::empty({P, d.O}, x.options().dtype(torch::kFloat32));
+  // Rows of weights per block: as many as leave 512 blocks, two a CU, all at work
+  // at once (64 tokens, 64 experts, 4 bits: 89 us; 116 with 256 blocks, 103 with
+  // 1024).
+  auto tiles = [&](long O) {
+    return (int)std::max<long>(1, O / 16 * std::min(g.E, P) / 512);
+  };
+  MoeRowsArgs a{x.data_ptr(), g.w, u.w, h.data_ptr(),
+                choice.data_ptr<int>(), weight.data_ptr<float>(), (int)P,
+                (int)choice.size(1), (int)g.E, (int)g.O, (int)g.K, tiles(g.O)};
+  launch_moe_rows(&a, (int)bits, (int)gs, true, cur_stream());
+  a = MoeRowsArgs{h.data_ptr(), d.w, nullptr, y.data_ptr(), choice.data_ptr<int>(), weight.data_ptr<float>(),
+                  (int)P, (int)choice.size(1), (int)d.E, (int)d.O, (int)d.K,
+                  tiles(d.O)};
+  launch_moe_rows(&a, (int)bits, (int)gs, false, cur_stream());
+  return y;
+}
+
+// A token's pairs, and the rows h and shared where given, added up in 32 bits
+torch::Tensor moe_combine(torch::Tensor rows, c10::optional<torch::Tensor> h,
+                          c10::optional<torch::Tensor> shared, int64_t N) {
+  TORCH_CHECK(rows.is_cuda() && rows.scalar_type() == torch::kFloat32 &&
+                  rows.dim() == 2 && rows.is_contiguous() && N >= 1 &&
+                  rows.size(0) % N == 0 && rows.size(1) % 4 == 0, "rows");
+  const long H = rows.size(1);
+  if (h.has_value()) check_rows(*h, "h", N, H);
+  if (shared.has_value()) check_rows(*shared, "shared", N, H);
+  auto out = torch::empty({N, H}, rows.options().dtype(torch::kBFloat16));
+  launch_moe_combine(rows.data_ptr<float>(), h.has_value() ? h->data_ptr() : nullptr,
+                     shared.has_value() ? shared->data_ptr() : nullptr,
+                     out.data_ptr(), (int)N, (int)H, (int)(rows.size(0) / N),
+                     cur_stream());
+  return out;
+}
+
 torch::Tensor moe_w4f16_gateup(torch::Tensor x, torch::Tensor gq,
                                torch::Tensor uq, torch::Tensor gsc,
                                torch::Tensor gbi, torch::Tensor usc,
@@ -750,6 +902,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return attn_prefill_supported((int)dk, (int)dv);
   });
   m.def("linear_few", &linear_few);
+  m.def("moe_route", &moe_route);
+  m.def("moe_pack", &moe_pack);
+  m.def("moe_rows", &moe_rows);
+  m.def("moe_rows_longest", [](int64_t bits) { return moe_rows_longest((int)bits); });
+  m.def("moe_combine", &moe_combine);
   m.def("linear_few", &linear_few);
   m.def("mfma_probe", &mfma_probe);
   m.def("w4a16_gemv", &w4a16_gemv);

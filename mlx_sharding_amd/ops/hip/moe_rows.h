@@ -1,0 +1,40 @@
+// Arguments of the routed experts' kernels of a decoding step (moe_rows.hip).
+#pragma once
+
+#include "hip_common.h"
+
+#define MR_PAIRS 1024  // (token, expert) pairs of a batch
+
+struct MoeRowsArgs {
+  const void* x;             // bf16 rows [N, K] (up), h rows [pairs, K] (down)
+  const void *w, *w2;        // packed (moe_pack) or bf16 [E, O, K]; up: gate's, up's
+  void* y;                   // up: h [pairs, O]; down: fp32 [pairs, O]
+  const int* choice;         // [pairs] expert
+  const float* weight;       // [pairs]
+  int pairs, top, experts, O, K;
+  int tiles;                 // of 16 rows of w, per block
+};
+
+struct MoeRouteArgs {
+  const __bf16 *x, *residual, *norm, *gate;  // rows [N, H], [H], [E, H]
+  __bf16 *h, *y;       // x + residual (if given), normed rows
+  int* choice;
+  float* weight;
+  int H, E, top;
+  float eps, offset, scaling;
+  int normalize;
+};
+
+extern "C" {
+// words of a packed tile of 16 rows by 128 of the contraction
+inline int moe_pack_words(int bits, int gs) {
+  return 16 * 128 * bits / 32 + 16 * (128 / gs);
+}
+void launch_moe_pack(const void*, const void*, const void*, void*, int, int, int,
+                     int, hipStream_t);
+void launch_moe_rows(const MoeRowsArgs*, int, int, bool, hipStream_t);
+int moe_rows_longest(int);
+void launch_moe_route(const MoeRouteArgs*, int, hipStream_t);
+void launch_moe_combine(const float*, const void*, const void*, void*, int, int,
+                        int, hipStream_t);
+}

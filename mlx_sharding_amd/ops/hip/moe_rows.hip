@@ -1,0 +1,494 @@
+// Routed experts of a decoding step, up to 128 tokens and 64 experts.
+//
+//   moe_route    residual update, RMS norm, router product, softmax and choice of
+//                a token, a block each
+//   moe_up       act(gate) * up of every chosen (token, expert) pair
+//   moe_down     the pairs' outputs, weighted, in 32 bits
+//   moe_combine  a token's pairs, shared experts and residual added up
+//
+// No sort: a block of an expert looks through the choices (at most 1024) for its
+// pairs.  Rows of pairs lie at token * top + place.
+//
+// The products are bound by reading the experts' packed weights.  Read naively,
+// rows of x out of L2 are twice those bytes and more (16 rows of 16 bits for 16
+// rows of 4), which held the kernel before this at 2.7 TB/s.  So rows of x stay
+// in registers: a wave of eight takes every eighth unit of 128 of the contraction
+// and keeps those parts of 16 tokens while the block walks over its rows of
+// weights, the next 16 rows asked for before these are used.  The waves add up
+// through LDS.
+//
+// Within a unit a lane has 32 consecutive values of a row: k = unit * 128 +
+// (lane >> 4) * 32 + step * 8 + j, which is 16 bytes at 4 bits and one scale; A
+// and B agree on that order.  moe_pack lays packed weights out in it once, a
+// tile's scales behind its words: a wave's load is 1 KB in one piece, where rows
+// as they come are 64 bytes each and scales 2 (64 tokens, 64 experts of 1408 x
+// 2048 at 4 bits: 113 us so, 89 packed).
+// 4 and 8 bits become fp16 numbers 1024 + q by an OR, exactly, and one fma rounds
+// them to s q + b; values of a word are laid out in pairs for it.
+// Measured, norm, router, choice, experts and sum of 64 experts of 1408 x 2048 (6 a
+// token) beside the kernels before (norm and residual apart): 1 token at 4 bits
+// 33 us, 48 and norms; 64 tokens 104, 166 (experts alone 3.5 TB/s); 8 bits 147,
+// 247; bf16, experts alone, 64 tokens 234 us (4.7 TB/s).
+
+#include "moe_rows.h"
+
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+#define MR_WAVES 8
+#define MR_BLOCK (MR_WAVES * WAVE)
+#define MR_UNIT 128
+
+// -- operands ---------------------------------------------------------------
+
+template <int BITS>
+struct Operand {
+  typedef f16x8 V;
+  typedef f16x4 H;
+  typedef _Float16 E;
+  static __device__ __forceinline__ f32x4 mma(V a, V b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct Operand<16> {
+  typedef bf16x8_t V;
+  typedef bf16x4_t H;
+  typedef __bf16 E;
+  static __device__ __forceinline__ f32x4 mma(V a, V b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+
+// a lane's 32 values of one unit, as they come from memory
+template <int BITS>
+struct Packed {
+  uint4 q[BITS / 4];
+  unsigned scale;  // scale and offset, bf16
+  // w: this lane's first 16 bytes; sc: its scale (packed only)
+  __device__ __forceinline__ void load(const char* w, const char* sc) {
+#pragma unroll
+    for (int i = 0; i < BITS / 4; ++i)
+      q[i] = *reinterpret_cast<const uint4*>(w + i * (BITS == 16 ? 16 : 1024));
+    if (BITS < 16) scale = *reinterpret_cast<const unsigned*>(sc);
+  }
+  // values 8 i .. 8 i + 7
+  __device__ __forceinline__ typename Operand<BITS>::V operand(int i) const {
+    const unsigned* u = reinterpret_cast<const unsigned*>(q);
+    if constexpr (BITS == 16) {
+      return __builtin_bit_cast(bf16x8_t, q[i]);
+    } else {
+      constexpr float MID = BITS == 4 ? 8.0f : 128.0f;
+      const float sf = __uint_as_float(scale << 16);
+      const _Float16 sh = (_Float16)sf;
+      const _Float16 bh = (_Float16)(__uint_as_float(scale & 0xFFFF0000u) + MID * sf);
+      const f16x2 s2 = {sh, sh}, b2 = {bh, bh};
+      const _Float16 c = (_Float16)(-1024.0f - MID);
+      f16x8 out;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const unsigned word = BITS == 4 ? u[i] >> (4 * j)
+                                        : u[2 * i + j / 2] >> (8 * (j & 1));
+        const unsigned v =
+            (word & (BITS == 4 ? 0x000F000Fu : 0x00FF00FFu)) | 0x64006400u;
+        const f16x2 f =
+            (__builtin_bit_cast(f16x2, v) + f16x2{c, c}) * s2 + b2;
+        out[2 * j] = f[0];
+        out[2 * j + 1] = f[1];
+      }
+      return out;
+    }
+  }
+};
+
+// -- products ---------------------------------------------------------------
+
+template <int BITS, int GS, int UPW, bool UP>
+__global__ __launch_bounds__(
+    MR_BLOCK, UPW <= (BITS == 16 && UP ? 1 : 2) ? 4 : 2) void moe_rows_kernel(
+    const MoeRowsArgs a) {
+  typedef Operand<BITS> Op;
+  typedef typename Op::V V;
+  constexpr int MATS = UP ? 2 : 1;
+  __shared__ short list[MR_PAIRS];
+  __shared__ int found;
+  __shared__ __attribute__((aligned(16))) f32x4 red[2][MR_WAVES][MATS][WAVE];
+
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int l16 = lane & 15, lg = lane >> 4;
+  // a block per expert, or where there are fewer pairs per pair: of its expert, if
+  // it is the first of it
+  const bool by_pair = gridDim.y < (unsigned)a.experts;
+  const int e = by_pair ? a.choice[blockIdx.y] : blockIdx.y;
+  if (wid == 0) {
+    int n = 0;
+    for (int i = 0; i < a.pairs; i += WAVE) {
+      const bool mine = i + lane < a.pairs && a.choice[i + lane] == e;
+      const unsigned long long all = __ballot(mine);
+      if (mine) list[n + __popcll(all & ((1ull << lane) - 1))] = (short)(i + lane);
+      n += __popcll(all);
+    }
+    if (lane == 0) found = n;
+  }
+  __syncthreads();
+  const int n = by_pair && list[0] != (int)blockIdx.y ? 0 : found;
+  if (n == 0) return;
+  const int t0 = blockIdx.x * a.tiles, t1 = min(t0 + a.tiles, a.O / 16);
+
+  const int units = a.K / MR_UNIT;
+  // this lane's place in its first unit of the block's first rows
+  const int k0 = wid * MR_UNIT + lg * 32;
+  constexpr int UNIT = (16 * MR_UNIT * BITS / 32 + 16 * (MR_UNIT / GS)) * 4;
+  const long step = BITS == 16 ? (long)16 * a.K * 2 : (long)units * UNIT;
+  const long begin = ((long)e * (a.O / 16) + t0) * step +
+                     (BITS == 16 ? ((long)l16 * a.K + k0) * 2
+                                 : (long)wid * UNIT + lane * 16);
+  const int scales = 16 * MR_UNIT * BITS / 8 - lane * 16 +
+                     (l16 * (MR_UNIT / GS) + lg * 32 / GS) * 4;
+  const char* wp[2] = {(const char*)a.w + begin, (const char*)a.w2 + begin};
+  auto fetch = [&](Packed<BITS>& r, int m, int u, int t) {
+    constexpr int far = MR_WAVES * (BITS == 16 ? MR_UNIT * 2 : UNIT);
+    const char* p = wp[m] + t * step + (long)u * far;  // between a wave's units
+    r.load(p, p + scales);
+  };
+
+  int buf = 0;
+  for (int first = 0; first < n; first += 16) {
+    const int pair = list[min(first + l16, n - 1)];
+    V x[UPW][4];
+    Packed<BITS> next[MATS][UPW];
+#pragma unroll
+    for (int u = 0; u < UPW; ++u) {
+      if (wid + u * MR_WAVES >= units) continue;
+#pragma unroll
+      for (int m = 0; m < MATS; ++m) fetch(next[m][u], m, u, 0);
+      const short* src = (const short*)a.x +
+                         (long)(UP ? pair / a.top : pair) * a.K + k0 +
+                         u * MR_WAVES * MR_UNIT;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (UP && BITS != 16) {
+          const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(src + i * 8);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x[u][i][j] = (_Float16)(float)v[j];
+        } else {
+          x[u][i] = *reinterpret_cast<const V*>(src + i * 8);
+        }
+      }
+    }
+    for (int t = t0; t < t1; ++t, buf ^= 1) {
+      f32x4 acc[MATS];
+#pragma unroll
+      for (int m = 0; m < MATS; ++m) acc[m] = f32x4{0, 0, 0, 0};
+      const int ahead = min(t + 1, t1 - 1) - t0;
+#pragma unroll
+      for (int u = 0; u < UPW; ++u) {
+        if (wid + u * MR_WAVES >= units) continue;
+#pragma unroll
+        for (int m = 0; m < MATS; ++m) {
+          const Packed<BITS> r = next[m][u];
+          fetch(next[m][u], m, u, ahead);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            acc[m] = Op::mma(r.operand(i), x[u][i], acc[m]);
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < MATS; ++m) red[buf][wid][m][lane] = acc[m];
+      __syncthreads();
+      // one wave finishes these rows, the others go on
+      if (wid != t % MR_WAVES) continue;
+      f32x4 v[MATS];
+#pragma unroll
+      for (int m = 0; m < MATS; ++m) {
+        v[m] = red[buf][0][m][lane];
+#pragma unroll
+        for (int w = 1; w < MR_WAVES; ++w) {
+          const f32x4 p = red[buf][w][m][lane];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[m][j] += p[j];
+        }
+      }
+      if (first + l16 >= n) continue;
+      const long at = (long)pair * a.O + t * 16 + lg * 4;
+      if constexpr (UP) {
+        typedef typename Op::H H4;
+        H4 h;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float g = v[0][j];
+          h[j] = (typename Op::E)(g / (1.0f + __expf(-g)) * v[MATS - 1][j]);
+        }
+        *reinterpret_cast<H4*>((typename Op::E*)a.y + at) = h;
+      } else {
+        const float w = a.weight[pair];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[0][j] *= w;
+        *reinterpret_cast<f32x4*>((float*)a.y + at) = v[0];
+      }
+    }
+  }
+}
+
+// A wave per tile of 16 rows by one unit: words in operand order, pairs of values
+// 16 bits apart, then (scale, offset) of every row and group.
+template <int BITS>
+__global__ __launch_bounds__(WAVE) void moe_pack_kernel(
+    const unsigned* __restrict__ w, const unsigned short* __restrict__ scale,
+    const unsigned short* __restrict__ offset, unsigned* __restrict__ out, int K,
+    int gs, int words) {
+  const int units = K / MR_UNIT;
+  const long tile = blockIdx.x / units;
+  const int unit = blockIdx.x % units;
+  const int lane = threadIdx.x, l16 = lane & 15, lg = lane >> 4;
+  const long row = tile * 16 + l16;
+  unsigned* dst = out + (long)blockIdx.x * words;
+  const unsigned* src = w + row * (K * BITS / 32) +
+                        (unit * MR_UNIT + lg * 32) * BITS / 32;
+#pragma unroll
+  for (int i = 0; i < BITS / 4; ++i) {
+    const uint4 q = *reinterpret_cast<const uint4*>(src + i * 4);
+    uint4 r;
+    const unsigned* a = reinterpret_cast<const unsigned*>(&q);
+    unsigned* b = reinterpret_cast<unsigned*>(&r);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const unsigned v = a[j];
+      if (BITS == 4) {
+        const unsigned even = (v & 0xF) | (v >> 4 & 0xF0) | (v >> 8 & 0xF00) |
+                              (v >> 12 & 0xF000);
+        const unsigned u = v >> 4;
+        const unsigned odd = (u & 0xF) | (u >> 4 & 0xF0) | (u >> 8 & 0xF00) |
+                             (u >> 12 & 0xF000);
+        b[j] = even | odd << 16;
+      } else {
+        b[j] = (v & 0xFF0000FFu) | (v >> 8 & 0xFF00) | (v << 8 & 0xFF0000);
+      }
+    }
+    *reinterpret_cast<uint4*>(dst + i * 256 + lane * 4) = r;
+  }
+  const int groups = MR_UNIT / gs;
+  for (int i = lane; i < 16 * groups; i += WAVE) {
+    const long at = (tile * 16 + i / groups) * (K / gs) + unit * groups + i % groups;
+    dst[16 * MR_UNIT * BITS / 32 + i] = scale[at] | (unsigned)offset[at] << 16;
+  }
+}
+
+// rows: of all experts
+extern "C" void launch_moe_pack(const void* w, const void* scale,
+                                const void* offset, void* out, int rows, int K,
+                                int bits, int gs, hipStream_t stream) {
+  const dim3 grid((unsigned)(rows / 16 * (K / MR_UNIT))), block(WAVE);
+  const int words = moe_pack_words(bits, gs);
+  if (bits == 4) {
+    moe_pack_kernel<4><<<grid, block, 0, stream>>>(
+        (const unsigned*)w, (const unsigned short*)scale,
+        (const unsigned short*)offset, (unsigned*)out, K, gs, words);
+  } else {
+    moe_pack_kernel<8><<<grid, block, 0, stream>>>(
+        (const unsigned*)w, (const unsigned short*)scale,
+        (const unsigned short*)offset, (unsigned*)out, K, gs, words);
+  }
+}
+
+template <int BITS, int GS, bool UP>
+static void moe_rows_go(const MoeRowsArgs& a, hipStream_t stream) {
+  const dim3 grid((unsigned)((a.O / 16 + a.tiles - 1) / a.tiles),
+                  (unsigned)min(a.experts, a.pairs));
+  const dim3 block(MR_BLOCK);
+  const int upw = (a.K / MR_UNIT + MR_WAVES - 1) / MR_WAVES;
+  if (upw <= 1) {
+    moe_rows_kernel<BITS, GS, 1, UP><<<grid, block, 0, stream>>>(a);
+  } else if (upw <= 2) {
+    moe_rows_kernel<BITS, GS, 2, UP><<<grid, block, 0, stream>>>(a);
+  } else if (upw <= 3) {
+    moe_rows_kernel<BITS, GS, 3, UP><<<grid, block, 0, stream>>>(a);
+  } else if constexpr (BITS < 16) {
+    moe_rows_kernel<BITS, GS, 5, UP><<<grid, block, 0, stream>>>(a);
+  }
+}
+
+// the longest contraction
+extern "C" int moe_rows_longest(int bits) {
+  return MR_UNIT * MR_WAVES * (bits < 16 ? 5 : 3);
+}
+
+template <bool UP>
+static void moe_rows_pick(const MoeRowsArgs& a, int bits, int gs,
+                          hipStream_t stream) {
+  if (bits == 16) {
+    moe_rows_go<16, MR_UNIT, UP>(a, stream);
+  } else if (bits == 4) {
+    if (gs == 32) moe_rows_go<4, 32, UP>(a, stream);
+    else if (gs == 64) moe_rows_go<4, 64, UP>(a, stream);
+    else moe_rows_go<4, 128, UP>(a, stream);
+  } else {
+    if (gs == 32) moe_rows_go<8, 32, UP>(a, stream);
+    else if (gs == 64) moe_rows_go<8, 64, UP>(a, stream);
+    else moe_rows_go<8, 128, UP>(a, stream);
+  }
+}
+
+// K: whole units, as many as registers hold (moe_rows_longest); O: whole tiles of
+// 16 rows; at most MR_PAIRS pairs.
+extern "C" void launch_moe_rows(const MoeRowsArgs* a, int bits, int gs,
+                                bool up, hipStream_t stream) {
+  if (up) moe_rows_pick<true>(*a, bits, gs, stream);
+  else moe_rows_pick<false>(*a, bits, gs, stream);
+}
+
+// -- router -----------------------------------------------------------------
+
+// A block per token.  The router's product runs on the matrix cores with the
+// token in every column: a wave has 16 experts and a quarter of the contraction,
+// and asks for its weights (64 x H, out of L2) before the norm, which waits for
+// rows and sums meanwhile: all of this is latency.
+__global__ __launch_bounds__(1024) void moe_route_kernel(const MoeRouteArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __bf16* row = reinterpret_cast<__bf16*>(smem);     // [H]
+  __shared__ float scratch[16];
+  __shared__ float part[4][64];
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lg = lane >> 4, eg = wid & 3, quarter = wid >> 2;
+  const long t = blockIdx.x;
+
+  // This thread's columns of the row, up to 8192 of which rows have; they are
+  // asked for ahead of the router's weights, as loads come back in order.
+  const int col = threadIdx.x * 8;
+  bf16x8_t v, r, n;
+  if (col < a.H) {
+    v = *reinterpret_cast<const bf16x8_t*>(a.x + t * a.H + col);
+    if (a.residual)
+      r = *reinterpret_cast<const bf16x8_t*>(a.residual + t * a.H + col);
+    n = *reinterpret_cast<const bf16x8_t*>(a.norm + col);
+  }
+  const int steps = a.H / 128;  // of 32, of this quarter
+  const bool works = eg * 16 < a.E;
+  const __bf16* g = a.gate + (long)min(eg * 16 + (lane & 15), a.E - 1) * a.H +
+                    quarter * steps * 32 + lg * 8;
+  bf16x8_t w[16];
+  if (works) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      w[i] = *reinterpret_cast<const bf16x8_t*>(g + min(i, steps - 1) * 32);
+  }
+
+  float ss = 0.0f;
+  if (col < a.H) {
+    if (a.residual) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = (__bf16)((float)v[j] + (float)r[j]);
+      *reinterpret_cast<bf16x8_t*>(a.h + t * a.H + col) = v;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss = fmaf((float)v[j], (float)v[j], ss);
+  }
+  ss = block_sum<1024>(ss, scratch);
+  const float f = rsqrtf(ss / a.H + a.eps);
+  if (col < a.H) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      v[j] = (__bf16)((float)v[j] * f * ((float)n[j] + a.offset));
+    *reinterpret_cast<bf16x8_t*>(row + col) = v;
+    *reinterpret_cast<bf16x8_t*>(a.y + t * a.H + col) = v;
+  }
+  __syncthreads();
+
+  if (works) {
+    const __bf16* x = row + quarter * steps * 32 + lg * 8;
+    f32x4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+    for (int s = 0; s < steps; s += 16) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (s + i < steps)
+          acc[i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              w[i], *reinterpret_cast<const bf16x8_t*>(x + (s + i) * 32),
+              acc[i & 1], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (s + 16 + i < steps)
+          w[i] = *reinterpret_cast<const bf16x8_t*>(g + (s + 16 + i) * 32);
+    }
+    if ((lane & 15) == 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        part[quarter][eg * 16 + lg * 4 + r] = acc[0][r] + acc[1][r];
+    }
+  }
+  __syncthreads();
+  if (wid != 0) return;
+  // softmax over experts, a lane each; a lane's place is the number of experts
+  // before it, by weight and then by number (as bits, so also where a row is not
+  // a number)
+  const float z = lane < a.E ? (part[0][lane] + part[1][lane]) +
+                                   (part[2][lane] + part[3][lane])
+                             : -INFINITY;
+  const float top = wave_max(z);
+  const float p = lane < a.E ? __expf(z - top) : 0.0f;
+  const float share = p / wave_sum(p);
+  const int key = __float_as_int(share) & 0x7FFFFFFF;
+  int place = 0;
+#pragma unroll
+  for (int i = 0; i < 64; ++i) {
+    const int k = __builtin_amdgcn_readlane(key, i);
+    place += k > key || (k == key && i < lane);
+  }
+  const bool chosen = place < a.top && lane < a.E;
+  float mine = share;
+  if (a.normalize) mine /= wave_sum(chosen ? share : 0.0f) + 1e-20f;
+  if (chosen) {
+    a.choice[t * a.top + place] = lane;
+    a.weight[t * a.top + place] = mine * a.scaling;
+  }
+}
+
+extern "C" void launch_moe_route(const MoeRouteArgs* a, int N,
+                                 hipStream_t stream) {
+  moe_route_kernel<<<dim3((unsigned)N), dim3(1024), (size_t)a->H * 2, stream>>>(*a);
+}
+
+// -- sum --------------------------------------------------------------------
+
+__global__ __launch_bounds__(256) void moe_combine_kernel(
+    const float* __restrict__ rows, const __bf16* __restrict__ h,
+    const __bf16* __restrict__ shared, __bf16* __restrict__ out, int H, int top) {
+  const long t = blockIdx.x;
+  for (int i = (blockIdx.y * 256 + threadIdx.x) * 4; i < H;
+       i += 256 * 4 * gridDim.y) {
+    f32x4 v = {0, 0, 0, 0};
+#pragma unroll 8
+    for (int k = 0; k < top; ++k) {
+      const f32x4 r =
+          *reinterpret_cast<const f32x4*>(rows + (t * top + k) * H + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] += r[j];
+    }
+    bf16x4_t o;
+    if (shared) {
+      const bf16x4_t s = *reinterpret_cast<const bf16x4_t*>(shared + t * H + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] += (float)s[j];
+    }
+    if (h) {
+      const bf16x4_t r = *reinterpret_cast<const bf16x4_t*>(h + t * H + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] += (float)r[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = (__bf16)v[j];
+    *reinterpret_cast<bf16x4_t*>(out + t * H + i) = o;
+  }
+}
+
+extern "C" void launch_moe_combine(const float* rows, const void* h,
+                                   const void* shared, void* out, int N, int H,
+                                   int top, hipStream_t stream) {
+  const unsigned parts = (unsigned)((H + 1023) / 1024);
+  moe_combine_kernel<<<dim3((unsigned)N, parts), dim3(256), 0, stream>>>(
+      rows, (const __bf16*)h, (const __bf16*)shared, (__bf16*)out, H, top);
+}

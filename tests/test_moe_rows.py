@@ -1,0 +1,142 @@
+"""Routed experts of a decoding step, against 64 bits."""
+
+import types
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from mlx_sharding_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def stack(E, O, K, bits, gs, gen):
+    """(matrices as ops.expert_rows takes them, their values in 64 bits)"""
+    if bits == 16:
+        w = (torch.randn(E, O, K, generator=gen, device="cuda") * 0.03).bfloat16()
+        return [w], w.double()
+    words = torch.randint(0, 2 ** 32, (E, O, K * bits // 32), generator=gen,
+                          device="cuda").to(torch.uint32)
+    new = lambda std: (torch.randn(E, O, K // gs, generator=gen,  # noqa: E731
+                                   device="cuda") * std).bfloat16()
+    s, b = new(0.0025 if bits == 4 else 0.00016), new(0.005)
+    shifts = torch.arange(0, 32, bits, device="cuda")
+    q = (words.view(torch.int32).to(torch.int64)[..., None] >> shifts) & (2 ** bits - 1)
+    q = q.reshape(E, O, K // gs, gs).double()
+    return [words, s, b], (q * s.double()[..., None] + b.double()[..., None]).flatten(-2)
+
+
+@pytest.mark.parametrize("N,E,top,I,H,bits,gs", [
+    (1, 8, 2, 128, 256, 4, 64),        # fewer units than waves, pairs than experts
+    (3, 5, 5, 384, 1152, 16, 128),     # all experts, nine units
+    (33, 3, 2, 128, 128, 4, 128),      # one unit; groups of 16 tokens and a rest
+    (128, 64, 6, 256, 512, 8, 32),     # most tokens
+    (100, 4, 1, 256, 384, 4, 32), (16, 64, 8, 1408, 2048, 8, 64),
+    (64, 64, 6, 1408, 2048, 4, 64), (17, 16, 4, 1536, 5120, 4, 128),
+    (9, 16, 4, 1536, 3072, 16, 128), (128, 1, 1, 128, 640, 8, 128)])
+def test_experts(N, E, top, I, H, bits, gs):
+    gen = torch.Generator("cuda").manual_seed(N + H)
+    randn = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    gate, gd = stack(E, I, H, bits, gs, gen)
+    up, ud = stack(E, I, H, bits, gs, gen)
+    down, dd = stack(E, H, I, bits, gs, gen)
+    x, res, shared = (randn(N, H).bfloat16() for _ in range(3))
+    norm = types.SimpleNamespace(weight=(1 + 0.1 * randn(H)).bfloat16(), eps=1e-6,
+                                 weight_offset=0.5)
+    router = (randn(E, H) * 0.05).bfloat16()
+    assert ops.expert_rows_ok(x, router, up[0], down[0], top, bits, gs)
+    y, h, choice, weight = ops.expert_route(x, res, norm, router, top, 1.5, True)
+    hd = (x.double() + res.double()).bfloat16()
+    assert torch.equal(h, hd)
+    yd = hd.double()
+    yd = yd * torch.rsqrt(yd.pow(2).mean(-1, keepdim=True) + 1e-6)
+    yd = yd * (norm.weight.double() + 0.5)
+    assert bool(((y.double() - yd).abs() <= 2.0 ** -8 * yd.abs() + 1e-6).all())
+
+    # chosen experts are the largest, up to 32-bit sums over H products
+    p = torch.softmax(y.double() @ router.double().T, -1)
+    own, best = p.gather(1, choice.long()), p.topk(top, -1).values
+    assert bool((choice.sort(-1).values.diff(dim=-1) > 0).all())
+    assert bool(((own - best).abs() <= 1e-5).all())
+    share = 1.5 * own / own.sum(-1, keepdim=True)
+    assert bool(((weight.double() - share).abs() <= 1e-5).all())
+
+    rows = ops.expert_rows(y, choice, weight, gate, up, down, bits, gs).double()
+    e, a = choice.long().flatten(), y.double().repeat_interleave(top, 0)
+    # weights and units are rounded to fp16 (2^-11 each) or units to bf16 (2^-8)
+    wide = bits == 16
+    uw, uh = (0.0, 2.0 ** -8) if wide else (2.0 ** -11, 2.0 ** -11)
+    tiny = H * 2.0 ** -24
+    for i in range(0, N * top, 64):
+        j = slice(i, i + 64)
+        dot = lambda m, v: torch.bmm(m[e[j]], v[..., None])[..., 0]  # noqa: E731
+        g, u = dot(gd, a[j]), dot(ud, a[j])
+        size = lambda m: dot(m.abs(), a[j].abs()) * (2 * uw + tiny)  # noqa: E731
+        unit = F.silu(g) * u
+        off = 1.1 * size(gd) * (u.abs() + size(ud)) + F.silu(g).abs() * size(ud)
+        off = off + uh * unit.abs() + 6e-8
+        w = weight.double().flatten()[j, None]
+        expect = w * dot(dd, unit)
+        bound = w * (dot(dd.abs(), off) + dot(dd.abs(), unit.abs()) * (2 * uw + tiny))
+        assert bool(((rows[j] - expect).abs() <= bound + 1e-6).all())
+
+    out = ops.expert_sum(rows.float(), h, shared, N).double()
+    total = h.double() + shared.double() + rows.view(N, top, H).sum(1)
+    assert bool(((out - total).abs() <= 2.0 ** -8 * total.abs() + 1e-5).all())
+    assert torch.equal(ops.expert_sum(rows.float(), None, None, N),
+                       rows.float().view(N, top, H).sum(1).bfloat16()) or top > 2
+
+
+def test_ties_and_rows_that_are_no_numbers():
+    """Equal scores: the first experts.  NaN: some experts, each once."""
+    H, E, top = 256, 12, 4
+    norm = types.SimpleNamespace(weight=torch.ones(H, device="cuda").bfloat16(),
+                                 eps=1e-6, weight_offset=0.0)
+    x = torch.ones(3, H, device="cuda").bfloat16()
+    x[1] = float("nan")
+    router = torch.zeros(E, H, device="cuda").bfloat16()
+    router[7] = 1.0
+    _, _, choice, weight = ops.expert_route(x, None, norm, router, top, 1.0, False)
+    assert choice[0].tolist() == [7, 0, 1, 2] == choice[2].tolist()
+    assert choice[1].sort().values.tolist() == [0, 1, 2, 3]
+    assert bool(weight[1].isnan().all())
+
+
+def test_layer_as_before():
+    """A decoder layer's step on these kernels beside the general path."""
+    from mlx_sharding_amd.config import ModelConfig
+    from mlx_sharding_amd.models.deepseek_v2 import DeepseekV2MoE
+    for bits in (4, 8, 0):
+        raw = {"model_type": "deepseek_v2", "hidden_size": 512,
+               "moe_intermediate_size": 256, "n_routed_experts": 16,
+               "num_experts_per_tok": 3, "n_shared_experts": 1,
+               "intermediate_size": 256}
+        if bits:
+            raw["quantization"] = {"group_size": 64, "bits": bits}
+        cfg = ModelConfig.from_dict(raw)
+        q = cfg.quantization
+        torch.manual_seed(bits)
+        with torch.device("cuda"):
+            moe = DeepseekV2MoE(cfg, lambda p: q, "m")
+        for name, p in moe.named_parameters():
+            if p.is_floating_point():
+                std = {"scales": 0.0025 / 16 ** (bits == 8), "biases": 0.005}
+                p.data.normal_(0, std.get(name.rsplit(".", 1)[-1], 0.05))
+            else:
+                p.data.random_(0, 2 ** 31 - 1)
+            p.requires_grad_(False)
+        norm = types.SimpleNamespace(weight=torch.ones(512, device="cuda").bfloat16(),
+                                     eps=1e-6, weight_offset=0.0)
+        for B, T in ((1, 1), (40, 1), (2, 9)):
+            x = torch.randn(B, T, 512, device="cuda").bfloat16()
+            assert moe.decodes(x)
+            got = moe.decode(x, None, norm).double()
+            # the same choice: where two experts are nearly tied, the general
+            # path's bf16 scores may fall the other way
+            y, _, choice, weight = ops.expert_route(
+                x.view(-1, 512), None, norm, moe.gate.weight, 3, 1.0, False)
+            rest = moe.switch_mlp(y, weight, choice.long()) + moe.shared_experts(y)
+            expect = x.double() + rest.double().view_as(x)
+            assert got.shape == x.shape
+            assert (got - expect).norm() < 0.01 * expect.norm()
