@@ -168,6 +168,7 @@ class MLAAttention(nn.Module):
         # nh*(nope+rope) + nh*vd — 8.9x less KV traffic for V2-Lite).
         self._w_uk = None
         self._w_uv = None
+        self._w_rows = None
 
     def absorbed_supported(self) -> bool:
         """True when the HIP decode kernel handles the absorbed shape
@@ -179,17 +180,51 @@ class MLAAttention(nn.Module):
         return (dk % 8 == 0 and self.kv_lora_rank % 8 == 0
                 and ext.attn_decode_shape_ok(self.n_heads, self.kv_lora_rank))
 
-    def _ensure_absorb(self, device, dtype):
-        if self._w_uk is not None:
-            return
+    def _up_weights(self, device, dtype):
+        """[heads, nope + v, rank]"""
         w = self.kv_b_proj.weight
         if self.kv_b_proj.quant is not None:
             qc = self.kv_b_proj.quant
             w = ops.dequantize(w, self.kv_b_proj.scales, self.kv_b_proj.biases,
                                qc.group_size, qc.bits)
         w = w.to(device=device, dtype=dtype)
-        w = w.view(self.n_heads, self.qk_nope + self.v_head_dim,
-                   self.kv_lora_rank)
+        return w.view(self.n_heads, self.qk_nope + self.v_head_dim,
+                      self.kv_lora_rank)
+
+    def _one_token_ok(self, x, latent, cache) -> bool:
+        """Whether mla_decode.hip takes this step."""
+        dk = self.kv_lora_rank + self.qk_rope
+        return (ops.use_native(x) and x.dtype == cache.dtype == torch.bfloat16
+                and latent.dtype == x.dtype and self.qk_nope % 32 == 0
+                and self.v_head_dim % 16 == 0 and self.qk_head_dim % 8 == 0
+                and self.kv_b_proj.bias is None
+                and bool(ops.hip_ext().attn_decode_tile(
+                    self.n_heads, dk, self.kv_lora_rank, True)))
+
+    def _one_token(self, qh, latent, cos, sin, cache: KVCache):
+        """Attention of one token per sequence over the compressed rows: [B, 1,
+        heads * v].  qh, latent: as projected."""
+        B = qh.shape[0]
+        if self._w_rows is None:
+            # the contraction last, as the kernels read
+            w = self._up_weights(qh.device, qh.dtype)
+            self._w_rows = (w[:, : self.qk_nope].transpose(1, 2).contiguous(),
+                            w[:, self.qk_nope:].contiguous())
+        ext, norm = ops.hip_ext(), self.kv_a_layernorm
+        pos, at = cache.claim(B, 1)
+        rows = cache.keys_buffer()
+        q, latent = qh.reshape(B, -1), latent.reshape(B, -1)
+        if q.data_ptr() % 16 or q.stride(0) % 8:
+            q = q.clone()
+        q = ext.mla_prepare(q, latent, self._w_rows[0], norm.weight, norm.eps,
+                            norm.weight_offset, cos, sin, rows, pos, at)
+        return ext.mla_attend(q, rows, self._w_rows[1], self.scale, pos,
+                              at + 1).view(B, 1, -1)
+
+    def _ensure_absorb(self, device, dtype):
+        if self._w_uk is not None:
+            return
+        w = self._up_weights(device, dtype)
         self._w_uk = w[:, : self.qk_nope, :].contiguous()
         self._w_uv = w[:, self.qk_nope:, :].transpose(1, 2).contiguous()
 
@@ -233,13 +268,15 @@ class MLAAttention(nn.Module):
             qh = self.q_b_proj(self.q_a_layernorm(self.q_a_proj(x)))
         else:
             qh = self.q_proj(x)
+        if ckv is None:
+            ckv = self.kv_a_proj_with_mqa(x)
+        if T == 1 and self._one_token_ok(qh, ckv, cache):
+            return self._output(self._one_token(qh, ckv, cos, sin, cache), residual)
         qh = qh.view(B, T, nh, self.qk_head_dim)
         q_nope = qh[..., : self.qk_nope]
         q_pe = ops.apply_rope(qh[..., self.qk_nope:], cos, sin,
                               interleaved=True)
 
-        if ckv is None:
-            ckv = self.kv_a_proj_with_mqa(x)
         c_kv, k_pe = ckv.split([rank, rope], dim=-1)
         c_kv = self.kv_a_layernorm(c_kv)
         k_pe = ops.apply_rope(k_pe.view(B, T, 1, rope), cos, sin,

@@ -386,7 +386,7 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 struct DecodeArgs {
   const char *q, *k, *v;   // rows: q [B, Hq, DK], k, v [B, Hkv, cap, *]
-  char* out;
+  char* out;               // null: one slice is left as a partial result, too
   float *part_o, *part_ml; // [B * Hq, nsplit, DV], [B * Hq, nsplit, 2]
   const int* s_ptr;
   int Hq, Hkv, S, nsplit, window;
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
   if (l16 >= G) return;
   const long row = row0 + l16;
   const int col = wid * ND * 16 + lg * 4;
-  if (a.nsplit == 1) {
+  if (a.nsplit == 1 && a.out) {
     const float f = 1.0f / l;
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
@@ -632,7 +632,7 @@ static void attn_decode_tile_go(const DecodeArgs& a, int B, hipStream_t stream) 
   attn_decode_tile_kernel<DK, DV, KT, INROW>
       <<<dim3((unsigned)(B * a.Hkv), (unsigned)a.nsplit), dim3(AD_BLOCK), 0,
          stream>>>(a);
-  if (a.nsplit > 1)
+  if (a.nsplit > 1 && a.out)
     attn_decode_merge_kernel<<<dim3((unsigned)(B * a.Hq)), dim3(128), 0,
                                stream>>>(a.part_o, a.part_ml, (short*)a.out,
                                          a.nsplit, DV);

@@ -7,6 +7,7 @@
 
 #include "hip_common.h"
 #include "linear_few.h"
+#include "mla_decode.h"
 #include "moe_rows.h"
 
 extern "C" {
@@ -375,6 +376,97 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                      out.data_ptr(), part_o, part_ml, nsplit, s_ptr, B, Hq,
                      Hkv, S, kScap, Dk, Dv, vstride, (float)scale,
                      (float)softcap, (int)window, cur_stream());
+  return out;
+}
+
+// -- latent attention of one token per sequence (mla_decode.hip) -------------
+
+// q [N, heads * (nope + rope)], latent [N, rank + rope] before norm and rotation;
+// w [heads, rank, nope]; cos, sin [1, rope / 2] of the token's position; cache
+// [N, 1, cap, rank + rope] gets the row at pos (on the device) or pos0.  Returns
+// queries over cached rows, [N, heads, 1, rank + rope].
+torch::Tensor mla_prepare(torch::Tensor q, torch::Tensor latent, torch::Tensor w,
+                          torch::Tensor norm, double eps, double offset,
+                          torch::Tensor cos, torch::Tensor sin,
+                          torch::Tensor cache, c10::optional<torch::Tensor> pos,
+                          int64_t pos0) {
+  for (const auto& t : {q, latent, w, norm, cache}) check_bf16(t, "operand");
+  TORCH_CHECK(q.dim() == 2 && latent.dim() == 2 && w.dim() == 3 &&
+                  norm.dim() == 1 && cache.dim() == 4 && cache.size(1) == 1,
+              "shapes");
+  const long N = q.size(0), heads = w.size(0), rank = w.size(1), nope = w.size(2);
+  const long rope = latent.size(1) - rank;
+  TORCH_CHECK(N >= 1 && latent.size(0) == N && cache.size(0) == N &&
+                  q.size(1) == heads * (nope + rope) && norm.size(0) == rank &&
+                  cache.size(3) == rank + rope, "sizes");
+  TORCH_CHECK(rank % 32 == 0 && nope % 32 == 0 && nope >= 32 && rope >= 2 &&
+                  rope % 2 == 0 && (nope + rope) % 8 == 0 && (rank + rope) % 4 == 0,
+              "sizes of parts");
+  auto whole = [](const torch::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  TORCH_CHECK(q.stride(1) == 1 && q.stride(0) % 8 == 0 && latent.stride(1) == 1 &&
+                  w.is_contiguous() && norm.is_contiguous() &&
+                  cache.is_contiguous() && whole(q) && whole(w) && whole(cache),
+              "layout");
+  TORCH_CHECK(cos.is_cuda() && sin.is_cuda() &&
+                  cos.scalar_type() == torch::kFloat32 &&
+                  sin.scalar_type() == torch::kFloat32 && cos.is_contiguous() &&
+                  sin.is_contiguous() && cos.numel() == rope / 2 &&
+                  sin.numel() == rope / 2, "one position's rotations");
+  if (pos.has_value()) {
+    TORCH_CHECK(pos->is_cuda() && pos->scalar_type() == torch::kInt32, "pos int32");
+  } else {
+    TORCH_CHECK(pos0 >= 0 && pos0 < cache.size(2), "no room in the cache");
+  }
+  auto out = torch::empty({N, heads, 1, rank + rope}, q.options());
+  const MlaPrepareArgs a{
+      (const __bf16*)q.data_ptr(), (const __bf16*)latent.data_ptr(),
+      (const __bf16*)w.data_ptr(), (const __bf16*)norm.data_ptr(),
+      cos.data_ptr<float>(), sin.data_ptr<float>(), (__bf16*)out.data_ptr(),
+      (__bf16*)cache.data_ptr(), pos.has_value() ? pos->data_ptr<int>() : nullptr,
+      q.stride(0), latent.stride(0), cache.size(2), pos0, (int)N, (int)heads,
+      (int)nope, (int)rope, (int)rank, (float)eps, (float)offset};
+  launch_mla_prepare(&a, cur_stream());
+  return out;
+}
+
+// q from mla_prepare over the first S rows (captured: pos + 1) of the cache; w
+// [heads, vdim, rank].  Returns [N, heads * vdim].
+torch::Tensor mla_attend(torch::Tensor q, torch::Tensor cache, torch::Tensor w,
+                         double scale, c10::optional<torch::Tensor> pos,
+                         int64_t S) {
+  for (const auto& t : {q, cache, w}) check_bf16(t, "operand");
+  TORCH_CHECK(q.dim() == 4 && cache.dim() == 4 && w.dim() == 3, "shapes");
+  const long N = q.size(0), heads = q.size(1), D = q.size(3);
+  const long vdim = w.size(1), rank = w.size(2);
+  const int tile = attn_decode_tile(heads, D, rank, true);
+  TORCH_CHECK(tile, "no kernel for these heads");
+  TORCH_CHECK(cache.size(0) == N && cache.size(1) == 1 && cache.size(3) == D &&
+                  w.size(0) == heads && vdim % 16 == 0 && rank % 32 == 0, "sizes");
+  for (const auto& t : {q, cache, w})
+    TORCH_CHECK(t.is_contiguous() &&
+                    reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "layout");
+  const int* s_ptr = nullptr;
+  if (pos.has_value()) {
+    TORCH_CHECK(pos->is_cuda() && pos->scalar_type() == torch::kInt32, "pos int32");
+    s_ptr = pos->data_ptr<int>();
+  } else {
+    TORCH_CHECK(S >= 1 && S <= cache.size(2), "rows of the cache");
+  }
+  const int n = decode_slices(N, s_ptr ? cache.size(2) : S, tile);
+  auto fopts = q.options().dtype(torch::kFloat32);
+  auto po = torch::empty({N * heads * n, rank}, fopts);
+  auto pml = torch::empty({N * heads * n, 2}, fopts);
+  launch_attn_decode_tile(q.data_ptr(), cache.data_ptr(), cache.data_ptr(), nullptr,
+                          po.data_ptr<float>(), pml.data_ptr<float>(), n, s_ptr,
+                          (int)N, (int)heads, 1, (int)S, cache.size(2), (int)D,
+                          (int)rank, true, (float)scale, 0.0f, 0, cur_stream());
+  auto out = torch::empty({N, heads * vdim}, q.options());
+  const MlaFinishArgs a{po.data_ptr<float>(), pml.data_ptr<float>(),
+                        (const __bf16*)w.data_ptr(), (__bf16*)out.data_ptr(), (int)N,
+                        (int)heads, (int)rank, (int)vdim, n};
+  launch_mla_finish(&a, cur_stream());
   return out;
 }
 
@@ -902,6 +994,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return attn_prefill_supported((int)dk, (int)dv);
   });
   m.def("linear_few", &linear_few);
+  m.def("mla_prepare", &mla_prepare);
+  m.def("mla_attend", &mla_attend);
+  m.def("attn_decode_tile", [](int64_t g, int64_t dk, int64_t dv, bool inrow) {
+    return attn_decode_tile((int)g, (int)dk, (int)dv, inrow);
+  });
   m.def("moe_route", &moe_route);
   m.def("moe_pack", &moe_pack);
   m.def("moe_rows", &moe_rows);

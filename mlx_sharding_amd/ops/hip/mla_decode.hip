@@ -1,0 +1,190 @@
+// Latent attention of one token per sequence, before and after the attention over
+// cached rows [latent | rotated key part] (attn_decode.hip).
+//
+//   mla_prepare  queries into the space of the cached rows, [W_uk^T q | rotated
+//                part], and the token's own row, normed and rotated, into the cache
+//   mla_finish   slices of the keys merged, and W_uv of every head's latent
+//
+// Both are latency: each head's matrix is 128 KB and all of them pass in under a
+// microsecond; as separate products, copies, rotations and norms they were twelve
+// kernels of 4 to 13 us.  A block takes 16 tokens of one head, a wave 16 rows of
+// its matrix, read with the contraction contiguous ([head, row, contraction]).
+// MEASURED
+
+#include "mla_decode.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+
+#define MD_WAVES 4
+#define MD_BLOCK (MD_WAVES * WAVE)
+
+__device__ __forceinline__ void turn_pair(float& a, float& b, float c, float s) {
+  const float x = a * c - b * s;
+  b = b * c + a * s;
+  a = x;
+}
+
+// grid: (heads x blocks of 64 latent columns, tiles of 16 tokens), then N blocks
+// for the cached rows
+__global__ __launch_bounds__(MD_BLOCK) void mla_prepare_kernel(
+    const MlaPrepareArgs a) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int row_w = a.rank + a.rope;
+  const int cols = (a.rank + 63) / 64, tiles = (a.N + 15) / 16;
+  const int products = a.heads * cols * tiles;
+  if ((int)blockIdx.x >= products) {
+    // one token's row: waves share the columns
+    __shared__ float scratch[MD_WAVES];
+    const int t = blockIdx.x - products;
+    const __bf16* c = a.latent + (long)t * a.ld_latent;
+    float ss = 0.0f;
+    for (int i = threadIdx.x; i < a.rank; i += MD_BLOCK) {
+      const float f = (float)c[i];
+      ss = fmaf(f, f, ss);
+    }
+    ss = block_sum<MD_BLOCK>(ss, scratch);
+    const float f = rsqrtf(ss / a.rank + a.eps);
+    const long pos = a.pos ? *a.pos : a.pos0;
+    if (pos >= a.cap) return;
+    __bf16* row = a.cache + ((long)t * a.cap + pos) * row_w;
+    for (int i = threadIdx.x; i < a.rank; i += MD_BLOCK)
+      row[i] = (__bf16)((float)c[i] * f * ((float)a.norm[i] + a.offset));
+    for (int i = threadIdx.x; i < a.rope / 2; i += MD_BLOCK) {
+      float u = (float)c[a.rank + 2 * i], v = (float)c[a.rank + 2 * i + 1];
+      turn_pair(u, v, a.cos[i], a.sin[i]);
+      row[a.rank + 2 * i] = (__bf16)u;
+      row[a.rank + 2 * i + 1] = (__bf16)v;
+    }
+    return;
+  }
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int h = blockIdx.x % a.heads;
+  const int cb = blockIdx.x / a.heads % cols, tile = blockIdx.x / a.heads / cols;
+  const int tok = min(tile * 16 + l16, a.N - 1);
+  const long q_head = (long)h * (a.nope + a.rope);
+  const int r0 = cb * 64 + wid * 16;
+  if (r0 < a.rank) {
+    const __bf16* w = a.w + ((long)h * a.rank + min(r0 + l16, a.rank - 1)) * a.nope +
+                      lg * 8;
+    const __bf16* q = a.q + (long)tok * a.ld_q + q_head + lg * 8;
+    f32x4 acc = {0, 0, 0, 0};
+    for (int k = 0; k < a.nope; k += 128) {
+      bf16x8_t wf[4], qf[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (k + i * 32 < a.nope) {
+          wf[i] = *reinterpret_cast<const bf16x8_t*>(w + k + i * 32);
+          qf[i] = *reinterpret_cast<const bf16x8_t*>(q + k + i * 32);
+        }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (k + i * 32 < a.nope)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], qf[i], acc, 0, 0, 0);
+    }
+    if (tile * 16 + l16 < a.N) {
+      bf16x4_t o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = (__bf16)acc[j];
+      *reinterpret_cast<bf16x4_t*>(a.out + ((long)tok * a.heads + h) * row_w + r0 +
+                                   lg * 4) = o;
+    }
+  }
+  if (cb != 0) return;
+  // the rotated part of these 16 queries
+  for (int i = threadIdx.x; i < 16 * a.rope / 2; i += MD_BLOCK) {
+    const int t = tile * 16 + i / (a.rope / 2), p = i % (a.rope / 2);
+    if (t >= a.N) break;
+    const __bf16* q = a.q + (long)t * a.ld_q + q_head + a.nope + 2 * p;
+    float u = (float)q[0], v = (float)q[1];
+    turn_pair(u, v, a.cos[p], a.sin[p]);
+    __bf16* o = a.out + ((long)t * a.heads + h) * row_w + a.rank + 2 * p;
+    o[0] = (__bf16)u;
+    o[1] = (__bf16)v;
+  }
+}
+
+// grid: (heads, tiles of 16 tokens); all of a head's output columns
+__global__ __launch_bounds__(512) void mla_finish_kernel(const MlaFinishArgs a) {
+  // a token's latent [16][rank + 8] in bf16: the odd stride keeps the 16 rows that
+  // a read meets in different banks
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __bf16* lat = reinterpret_cast<__bf16*>(smem);
+  __shared__ float weight[16][64];
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int h = blockIdx.x, t0 = blockIdx.y * 16, n = a.slices;
+  const int stride = a.rank + 8;
+  // the first rows of the matrix are asked for before the slices
+  const int l16 = lane & 15, lg = lane >> 4;
+  auto rows = [&](int r0) {
+    return a.w + ((long)h * a.vdim + r0 + l16) * a.rank + lg * 8;
+  };
+  bf16x8_t wf[16];
+  auto fetch = [&](const __bf16* w, int k) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (k + i * 32 < a.rank)
+        wf[i] = *reinterpret_cast<const bf16x8_t*>(w + k + i * 32);
+  };
+  if (wid * 16 < a.vdim) fetch(rows(wid * 16), 0);
+  for (int i = wid; i < 16; i += 8) {
+    const long row = (long)min(t0 + i, a.N - 1) * a.heads + h;
+    const float m = lane < n ? a.part_ml[(row * n + lane) * 2] : -1e30f;
+    const float l = lane < n ? a.part_ml[(row * n + lane) * 2 + 1] : 0.0f;
+    const float top = wave_max(m);
+    const float e = __builtin_amdgcn_exp2f(m - top);
+    const float sum = wave_sum(l * e);
+    weight[i][lane] = e / sum;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 16 * (a.rank / 4); i += 512) {
+    const int t = i / (a.rank / 4), d = i % (a.rank / 4) * 4;
+    if (t0 + t >= a.N) break;
+    const float* p = a.part_o + ((long)(t0 + t) * a.heads + h) * n * a.rank + d;
+    f32x4 o = {0, 0, 0, 0};
+#pragma unroll 8
+    for (int s = 0; s < n; ++s) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(p + (long)s * a.rank);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] += v[j] * weight[t][s];
+    }
+    bf16x4_t r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[j] = (__bf16)o[j];
+    *reinterpret_cast<bf16x4_t*>(lat + t * stride + d) = r;
+  }
+  __syncthreads();
+  const int tok = min(l16, a.N - 1 - t0);
+  const __bf16* x = lat + tok * stride + lg * 8;
+  for (int r0 = wid * 16; r0 < a.vdim; r0 += 128) {
+    f32x4 acc = {0, 0, 0, 0};
+    for (int k = 0; k < a.rank; k += 512) {
+      if (r0 + k != wid * 16) fetch(rows(r0), k);
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (k + i * 32 < a.rank)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              wf[i], *reinterpret_cast<const bf16x8_t*>(x + k + i * 32), acc, 0,
+              0, 0);
+    }
+    if (t0 + l16 >= a.N) continue;
+    bf16x4_t o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = (__bf16)acc[j];
+    *reinterpret_cast<bf16x4_t*>(a.out + ((long)(t0 + l16) * a.heads + h) * a.vdim +
+                                 r0 + lg * 4) = o;
+  }
+}
+
+extern "C" void launch_mla_prepare(const MlaPrepareArgs* a, hipStream_t stream) {
+  const int products = a->heads * ((a->rank + 63) / 64) * ((a->N + 15) / 16);
+  mla_prepare_kernel<<<dim3((unsigned)(products + a->N)), dim3(MD_BLOCK), 0,
+                       stream>>>(*a);
+}
+
+extern "C" void launch_mla_finish(const MlaFinishArgs* a, hipStream_t stream) {
+  mla_finish_kernel<<<dim3((unsigned)a->heads, (unsigned)((a->N + 15) / 16)),
+                      dim3(512), (size_t)16 * (a->rank + 8) * 2, stream>>>(*a);
+}

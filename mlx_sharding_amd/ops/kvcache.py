@@ -92,6 +92,15 @@ class KVCache:
         self.offset += T
         return (self._k[:, :, : self.offset], self._v[:, :, : self.offset])
 
+    def claim(self, batch: int, T: int):
+        """Places for T more rows, for a kernel that writes them itself:
+        (position on the device or None, first place)."""
+        if self.graph_pos is not None:
+            return self.graph_pos, 0
+        self._ensure(batch, self.offset + T)
+        self.offset += T
+        return None, self.offset - T
+
     def append_rope_kv(self, k: torch.Tensor, v: torch.Tensor,
                        cos: torch.Tensor, sin: torch.Tensor,
                        interleaved: bool = False):

@@ -114,3 +114,65 @@ def test_decode_edges(Hq, Hkv, Dk, Dv, captured):
             # the result is rounded to bf16; 32-bit weights in two bf16 parts
             bound = 2.0 ** -8 * expect.abs() + 2.0 ** -13 * size + 1e-6
             assert bool(((out - expect).abs() <= bound).all()), (S, cap, window)
+
+
+@pytest.mark.parametrize("captured", [False, True])
+@pytest.mark.parametrize("N,S,nope,vdim", [(1, 1, 128, 128), (1, 3002, 128, 128),
+                                           (3, 33, 32, 16), (17, 64, 160, 208),
+                                           (64, 513, 128, 128), (129, 40, 64, 64)])
+def test_latent_one_token(N, S, nope, vdim, captured):
+    """One token per sequence over a cached latent, from projected rows to heads'
+    outputs: remainders of 16 tokens, matrices of other sizes, one and many
+    slices of the keys."""
+    H, rank, rope, room = 16, 512, 64, 5
+    torch.manual_seed(N + S)
+    bf = lambda *s: torch.randn(*s, device="cuda").bfloat16()  # noqa: E731
+    y = bf(N, H * (nope + rope) + rank + rope)
+    q, latent = y.split([H * (nope + rope), rank + rope], -1)
+    wk, wv = bf(H, rank, nope) * 0.1, bf(H, vdim, rank) * 0.05
+    norm = (1 + 0.1 * torch.randn(rank, device="cuda")).bfloat16()
+    angle = torch.rand(1, rope // 2, device="cuda") * 6
+    cos, sin = torch.cos(angle), torch.sin(angle)
+    cache = cached(N, 1, S - 1, rank + rope, room + 1).as_strided(
+        (N, 1, S + room, rank + rope),
+        ((S + room) * (rank + rope), (S + room) * (rank + rope), rank + rope, 1))
+    before = cache.clone()
+    pos = torch.tensor([S - 1], dtype=torch.int32, device="cuda")
+    qf = ext().mla_prepare(q, latent, wk, norm, 1e-6, 0.0, cos, sin, cache,
+                           pos if captured else None, 0 if captured else S - 1)
+    out = ext().mla_attend(qf, cache, wv, 0.05, pos if captured else None,
+                           1 if captured else S).double()
+
+    def turned(t):
+        a, b = t.double()[..., 0::2], t.double()[..., 1::2]
+        c, s = cos.double(), sin.double()
+        return torch.stack([a * c - b * s, b * c + a * s], -1).flatten(-2)
+
+    close = lambda got, expect, off=0.0: bool(  # noqa: E731
+        ((got.double() - expect).abs() <= 2.0 ** -8 * expect.abs() + off + 1e-5).all())
+    # the token's row, and only that
+    c = latent[:, :rank].double()
+    row = torch.cat([c * torch.rsqrt(c.pow(2).mean(-1, keepdim=True) + 1e-6)
+                     * norm.double(), turned(latent[:, rank:])], -1)
+    assert close(cache[:, 0, S - 1], row)
+    cache_but = cache.clone()
+    cache_but[:, 0, S - 1] = before[:, 0, S - 1]
+    assert torch.equal(cache_but.view(torch.int16), before.view(torch.int16))
+    # queries
+    qh = q.reshape(N, H, nope + rope)
+    heads_first = qh[..., :nope].double().transpose(0, 1).contiguous()
+    space = torch.bmm(heads_first, wk.double().transpose(1, 2).contiguous())
+    expect = torch.cat([space.transpose(0, 1), turned(qh[..., nope:])], -1)
+    sums = torch.bmm(heads_first.abs(), wk.double().abs().transpose(1, 2).contiguous())
+    assert close(qf[:, :, 0, :rank], expect[..., :rank],
+                 sums.transpose(0, 1) * nope * 2.0 ** -24)
+    assert close(qf[:, :, 0, rank:], expect[..., rank:])
+    # outputs, from the queries and rows as they were rounded
+    rows = cache[:, :, :S]
+    o, size = attention(qf, rows, rows[..., :rank], 0.05, 0.0, 0, S - 1)
+    o, size = (t[:, :, 0].transpose(0, 1).contiguous() for t in (o, size))
+    w = wv.double().transpose(1, 2).contiguous()
+    expect = torch.bmm(o, w).transpose(0, 1).reshape(N, -1)
+    # the latents between the two products are rounded to bf16
+    off = torch.bmm(2.0 ** -8 * o.abs() + 2.0 ** -13 * size, w.abs())
+    assert close(out, expect, off.transpose(0, 1).reshape(N, -1))
