@@ -17,7 +17,7 @@
 //    outputs O = diag(exp G) Q S0 + A U, and the next state
 //    exp(G_last) S0 + K^T diag(exp(G_last - G)) U.  One kernel makes
 //    (I + L)^-1 diag(beta) and A of all chunks at once, a second walks the
-//    chunks of a (request, head, 16 value columns).  All products run on the
+//    chunks of a (request, head, 16 or 32 value columns).  All products run on the
 //    fp32 matrix cores.
 //  * decays per channel: exp(G) is a vector then, and L and A sum
 //    k_i[d] k_j[d] exp(G_i[d] - G_j[d]) over channels.  Between the tokens of two
@@ -28,6 +28,7 @@
 //    chunk lies in two such blocks of 1, 2, 4, 8, 16 or more tokens.
 //
 // A request at position 0 starts from a zero state whatever its slot holds.
+#include <type_traits>
 #include "ragged_common.h"
 
 #define DR_CHUNK 64
@@ -957,194 +958,410 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(
   }
 }
 
-// The same walk with the state depth fixed at 16 * ND: every global operand
-// of the next chunk is fetched into registers right after the current chunk
-// used it, so its latency passes behind the products that remain.  Rows past
-// the end of a chunk repeat its last one: their beta is 0, so they write
+// The same walk with the state depth fixed at 16 * ND, CT column tiles a block, and
+// eight waves: four for the state (K S, then U, then the next S), four for the
+// outputs (Q S, A U), a SIMD has one of each.  Chunks follow one another, so what
+// counts is the way from one state to the next: three products with a barrier
+// behind each.  The matrix cores are at work for most of it, as the output waves
+// fill what the state waves leave.
+//   * K lies in LDS, once for its rows (K S) and its columns (the next S), and is
+//     loaded there a chunk ahead without registers; 16-byte pieces of a row are
+//     swapped by the row, so that neither way of reading meets banks twice.  All
+//     other operands are asked for a chunk ahead, too.
+//   * S, U and what leads to U lie transposed in LDS, [column][row]: one 16-byte
+//     access has what four products take or make.
+//   * column blocks of one (request, head) read the same operands and run on one
+//     XCD; two column tiles a block halve what comes out of its L2, where there are
+//     blocks enough.
+// CH: decays per channel; then K for the state (kt) is another array.
+// Rows past the end of a chunk repeat its last one: their beta is 0, so they write
 // nothing, and their outputs are not stored.
-template <typename T, int ND, bool CH>
-__global__ __launch_bounds__(256, 1) void delta_walk_fixed_kernel(
+// Bound by fp32 matrix products: 128 of a SIMD per chunk and tile, 1.7 us, of 3.4
+// (5.8 for two tiles); the rest is latency at the three barriers, and loads, which
+// take a third more of the first phase when they are all asked for at its start.
+// Depth 128, 16 heads, one block per column tile and four waves before: 2 x 4001
+// tokens 343 -> 229 us, 1 x 8192 641 -> 398, 8 x 1024 354 -> 184, 11 requests of 17
+// to 1160 212 -> 143; decays per channel, 2 x 4001 350 -> 285, 6 of 30 to 900 117 -> 92.
+template <typename T, int ND, int CT, bool CH>
+__global__ __launch_bounds__(512, 2) void delta_walk_fixed_kernel(
     const float* __restrict__ qn, const float* __restrict__ kn,
     const float* __restrict__ ktn, const T* __restrict__ vn, const float* __restrict__ tm,
     const float* __restrict__ am, const float* __restrict__ ge,
     float* __restrict__ state, float* __restrict__ o,
     const int* __restrict__ chunks, const int* __restrict__ chunk_cu,
     const int* __restrict__ pos0, const int* __restrict__ slots, int n_short,
-    int tok_base, int KH, int H, int D, int V, int Vp) {
+    int tok_base, int n_long, int KH, int H, int D, int V, int Vp) {
   constexpr int Dp = ND * 16;
-  constexpr int NT = (ND + 3) / 4;  // state row tiles per wave
-  const int v0 = blockIdx.x * 16;
-  const int h = blockIdx.y;
-  const int e = blockIdx.z;
+  constexpr int NT = (ND + 3) / 4;       // state row tiles per wave
+  constexpr int KP = Dp / 4;             // 16-byte pieces of a row of K
+  constexpr int KW = DR_CHUNK * Dp;      // one chunk of K
+  constexpr int SS = Dp + 4, US = DR_CHUNK + 4;
+  const int cols = Vp / (16 * CT), pairs = H * n_long;
+  int pair = blockIdx.x / cols, vt = blockIdx.x % cols;
+  if (pairs % 8 == 0) {  // blocks go round the XCDs
+    const int slot = blockIdx.x >> 3;
+    pair = slot / cols * 8 + (blockIdx.x & 7);
+    vt = slot % cols;
+  }
+  const int e = pair / H, h = pair % H;
+  const int v0 = vt * 16 * CT;
   const int kh = h / (H / KH);
-  const int tid = threadIdx.x;
-  const int lane = tid & (WAVE - 1);
-  const int wid = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int w = wid & 3;
   const int lr = lane & 15, g4 = lane >> 4;
 
-  __shared__ float ss[Dp * 17];  // state columns
-  __shared__ float xs[64 * 17];  // V - exp(G) K S
-  __shared__ float us[64 * 17];  // U
-  __shared__ float uw[64 * 17];  // exp(G_last - G) U
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  float* kl = reinterpret_cast<float*>(smem);    // [2][64][Dp] K
+  float* kc = kl + 2 * KW;                       // [64][Dp] kt (CH)
+  float* st = kl + (CH ? 3 : 2) * KW;            // [CT][16][SS] state
+  float* xt = st + CT * 16 * SS;                 // [CT][16][US] V - exp(G) K S
+  float* ut = xt + CT * 16 * US;                 // [CT][16][US] U
+  float* wt = ut + CT * 16 * US;                 // ... exp(G_last - G) U
 
-  const bool fresh = pos0[n_short + e] == 0;
-  float* sg = state + ((long)slots[n_short + e] * H + h) * (long)D * V;
-  for (int i = tid; i < Dp * 16; i += 256) {
-    const int d = i >> 4, v = v0 + (i & 15);
-    ss[d * 17 + (i & 15)] =
-        (!fresh && d < D && v < V) ? sg[(long)d * V + v] : 0.0f;
-  }
+  // place of a piece in a row's LDS
+  auto place = [](int row, int piece) { return piece ^ (row & (KP < 16 ? KP - 1 : 15)); };
+  // one of PARTS pieces that this wave brings of a chunk of K.  Offsets in a chunk are
+  // 32 bits wide.
+  constexpr int PARTS = (KW / 256 + 7) / 8;
+  const unsigned krow = KH * Dp * 4;
+  auto stage = [&](const float* src, float* dst, int i0, int len, int i) {
+    const char* from = reinterpret_cast<const char*>(src + ((long)i0 * KH + kh) * Dp);
+    const int part = i * 8 + wid;
+    if (KW / 256 % 8 && part >= KW / 256) return;
+    const int at = part * 64 + lane, row = at / KP;
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) void*)(
+            from + (unsigned)min(row, len - 1) * krow +
+            (unsigned)place(row, at % KP) * 16),
+        (__attribute__((address_space(3))) void*)(dst + part * 256), 16, 0, 0);
+  };
 
-  const long rstride = (long)KH * Dp;
-  const f32x4 zero = {0, 0, 0, 0};
-  const int row = wid * 16 + lr;            // A-operand row
-  const int row_c = wid * 16 + g4 * 4;      // first C row
-
-  f32x4 kf[ND], qf[ND], tf[4], af[4], kt[NT][4];
-  float vf[4], gr[4], gl[4], g_all;
-  f32x4 gd[NT];  // decays of this lane's state rows
-
-  auto load_rows = [&](int i0, int len) {
-    const long at = ((long)(i0 + min(row, len - 1)) * KH + kh) * Dp + g4 * 4;
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-      kf[d] = load4(kn + at + d * 16);
-      qf[d] = load4(qn + at + d * 16);
-    }
-  };
-  auto load_misc = [&](int c, int i0, int len) {
-    const float* gc = ge + ((long)c * H + h) * (CH ? Dp : 128);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = row_c + r;
-      vf[r] = (float)vn[((long)(i0 + min(i, len - 1)) * H + h) * Vp + v0 + lr];
-      gr[r] = CH ? 1.0f : gc[i];
-      gl[r] = CH ? 1.0f : gc[64 + i];
-    }
-    if (!CH) g_all = gc[63];
-  };
-  auto load_decay = [&](int c) {
-    if constexpr (CH) {
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const int d0 = wid * 16 + n * 64;
-        if (d0 < Dp) gd[n] = load4(ge + ((long)c * H + h) * Dp + d0 + g4 * 4);
-      }
-    }
-  };
-  auto load_mat = [&](const float* m, int c, f32x4 (&f)[4]) {
-    const float* p = m + ((long)c * H + h) * 4096 + row * 64 + g4 * 4;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) f[j] = load4(p + j * 16);
-  };
-  auto load_kt = [&](int i0, int len) {
+  // the two kinds of waves have loops of their own, with the same barriers
+  auto walk = [&](auto kind) {
+    constexpr bool keeps = decltype(kind)::value;  // a state wave
+    const bool fresh = pos0[n_short + e] == 0;
+    float* sg = state + ((long)slots[n_short + e] * H + h) * (long)D * V;
+    const f32x4 zero = {0, 0, 0, 0};
+    f32x4 own[NT][CT];                     // this wave's rows of the state
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
-      const int d0 = wid * 16 + n * 64;
-      if (d0 >= Dp) continue;
-      const float* ka = ktn + ((long)i0 * KH + kh) * Dp + d0 + lr;
+      const int d0 = w * 16 + n * 64 + g4 * 4;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int t = 0; t < CT; ++t) {
+        const int v = v0 + t * 16 + lr;
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const int i = min(j * 16 + g4 * 4 + s, len - 1);
-          kt[n][j][s] = ka[i * rstride];
+        for (int r = 0; r < 4; ++r)
+          own[n][t][r] = keeps && !fresh && d0 + r < D && v < V
+                             ? sg[(long)(d0 + r) * V + v] : 0.0f;
+        if (keeps && d0 < Dp) store4(st + (t * 16 + lr) * SS + d0, own[n][t]);
+      }
+    }
+
+    const long rstride = (long)KH * Dp;
+    const int row = w * 16 + lr;              // A-operand row
+    const int row_c = w * 16 + g4 * 4;        // first C row
+
+    const unsigned vrow = H * Vp;
+    // 0, unknown to the compiler: scalar loads come in any order, and a wait for LDS
+    // would be one for all of them
+    unsigned nought = 0;
+    asm volatile("" : "+v"(nought));
+    // what comes a chunk ahead: T or A, rows of Q (output waves), V and decays
+    struct Ahead {
+      f32x4 m[4], q[ND], gr, gl, gd[NT];
+      T v[CT][4];
+      float all;
+    };
+    // in pieces, to go between the products: asked for at once they stand in the way
+    constexpr int PIECES = PARTS + 5 + (keeps ? CT : ND);
+    auto fetch = [&](Ahead& f, float* kd, int c, int i0, int len, int i) {
+      const long ch = (long)c * H + h;
+      const float* gc = ge + ch * (CH ? Dp : 128);
+      if (i < PARTS) {
+        stage(kn, kd, i0, len, i);
+      } else if (i < PARTS + 4) {
+        const int j = i - PARTS;
+        const float* mp = (keeps ? tm : am) + ch * 4096;
+        if (j <= w) f.m[j] = load4(mp + (unsigned)(row * 64 + g4 * 4 + j * 16));
+      } else if (i == PARTS + 4) {
+        if (!CH) f.gr = load4(gc + (unsigned)row_c);
+        if constexpr (keeps) {
+          if (!CH) {
+            f.gl = load4(gc + (unsigned)(64 + row_c));
+            f.all = gc[63 + nought];
+          } else {
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+              const int d0 = w * 16 + n * 64;
+              if (d0 < Dp) f.gd[n] = load4(gc + (unsigned)(d0 + g4 * 4));
+            }
+          }
         }
-    }
-  };
-
-  const int c_end = chunk_cu[e + 1];
-  int c = chunk_cu[e];
-  int i0 = chunks[2 * c] - tok_base, len = chunks[2 * c + 1];
-  load_rows(i0, len);
-  load_misc(c, i0, len);
-  load_mat(tm, c, tf);
-  load_mat(am, c, af);
-  load_kt(i0, len);
-  load_decay(c);
-  __syncthreads();
-
-  for (; c < c_end; ++c) {
-    const int cn = min(c + 1, c_end - 1);  // the last one is fetched twice
-    const int j0 = chunks[2 * cn] - tok_base;
-    const int jl = chunks[2 * cn + 1];
-
-    f32x4 ks = zero, qs = zero;
+      } else if constexpr (keeps) {
+        const int t = i - PARTS - 5;
+        const T* vp = vn + ((long)i0 * H + h) * Vp + v0;
 #pragma unroll
-    for (int d = 0; d < ND; ++d)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const float sv = ss[(d * 16 + g4 * 4 + s) * 17 + lr];
-        ks = mma4(kf[d][s], sv, ks);
-        qs = mma4(qf[d][s], sv, qs);
+        for (int r = 0; r < 4; ++r)
+          f.v[t][r] = vp[(unsigned)min(row_c + r, len - 1) * vrow + (unsigned)(t * 16 + lr)];
+      } else {
+        const int d = i - PARTS - 5;
+        const float* qp = qn + ((long)i0 * KH + kh) * Dp;
+        f.q[d] = load4(qp + (unsigned)min(row, len - 1) * (krow / 4) +
+                       (unsigned)(d * 16 + g4 * 4));
       }
-    load_rows(j0, jl);
-    f32x4 oc;
-    float glk[4];
-    const float g_now = g_all;
+    };
+    // a barrier for what waves wrote into LDS; loads on their way there for the next
+    // chunk, which __syncthreads would wait for, go on
+    auto sync_lds = [] {
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // loads above stay above: what follows finds its operands under way
+    auto issued = [] { __builtin_amdgcn_sched_barrier(0); };
+
+    const int c_end = chunk_cu[e + 1];
+    int c = chunk_cu[e];
+    int i0 = chunks[2 * c] - tok_base, len = chunks[2 * c + 1];
+    int cn = min(c + 1, c_end - 1);  // the last one is fetched twice
+    int j0 = chunks[2 * cn] - tok_base, jl = chunks[2 * cn + 1];
+    Ahead now = {}, next = {};
+    float vf[CT][4];
+    auto arrived = [&] {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      now = next;
+      // made here, so that no later use waits for the loads behind these
+      auto here = [](auto& x) { asm volatile("" : "+v"(x)); };
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      xs[(row_c + r) * 17 + lr] = vf[r] - gr[r] * ks[r];
-      oc[r] = gr[r] * qs[r];
-      glk[r] = gl[r];
-    }
-    load_misc(cn, j0, jl);
+      for (int j = 0; j < 4; ++j) here(now.m[j]);
+      if (!CH) here(now.gr);
+      if constexpr (keeps) {
+        if (!CH) here(now.gl);
+        if (!CH) here(now.all);
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+          if (CH) here(now.gd[n]);
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            vf[t][r] = (float)now.v[t][r];
+            here(vf[t][r]);
+          }
+      } else {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) here(now.q[d]);
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) fetch(next, kl, c, i0, len, i);
+    auto stage_kt = [&](int i0, int len) {
+#pragma unroll
+      for (int i = 0; i < PARTS; ++i) stage(ktn, kc, i0, len, i);
+    };
+    if (CH) stage_kt(i0, len);
+    arrived();
     __syncthreads();
 
-    f32x4 u = zero;
+    for (int buf = 0; c < c_end; ++c, buf ^= 1) {
+      const int ahead = min(cn + 1, c_end - 1);
+      const int2 then = reinterpret_cast<const int2*>(chunks)[ahead + nought];
+      const float* k = kl + buf * KW;
+
+      f32x4 acc[CT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j <= wid) {
+      for (int t = 0; t < CT; ++t) acc[t] = zero;
+      // rows of K or Q times the state for pieces FROM to TO of the depth, GR of
+      // them under way while others are in the matrix cores
+      auto rows_of = [&](auto from, auto to) {
+        constexpr int F = decltype(from)::value, E = decltype(to)::value;
+        constexpr int GR = CT == 1 ? 4 : 2;
+        f32x4 a[E - F], b[E - F][CT];
+        auto read = [&](int d) {
+          if constexpr (keeps)
+            a[d - F] = load4(k + row * Dp + place(row, d * 4 + g4) * 4);
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
-          u = mma4(tf[j][s], xs[(j * 16 + g4 * 4 + s) * 17 + lr], u);
+          for (int t = 0; t < CT; ++t)
+            b[d - F][t] = load4(st + (t * 16 + lr) * SS + d * 16 + g4 * 4);
+        };
+#pragma unroll
+        for (int d = F; d < E && d < F + GR; ++d) read(d);
+        issued();
+#pragma unroll
+        for (int d0 = F; d0 < E; d0 += GR) {
+#pragma unroll
+          for (int d = d0 + GR; d < d0 + 2 * GR && d < E; ++d) read(d);
+          issued();
+#pragma unroll
+          for (int d = d0; d < d0 + GR && d < E; ++d) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+              for (int t = 0; t < CT; ++t)
+                acc[t] = mma4(keeps ? a[d - F][s] : now.q[d][s], b[d - F][t][s], acc[t]);
+            issued();
+            constexpr int per = (PIECES + ND - 1) / ND;
+#pragma unroll
+            for (int i = d * per; i < (d + 1) * per && i < PIECES; ++i)
+              fetch(next, kl + (buf ^ 1) * KW, cn, j0, jl, i);
+            issued();
+          }
+        }
+      };
+      // the matrix of this wave times columns of `x`
+      auto lower = [&](const float* x, f32x4 (&to)[CT]) {
+        f32x4 b[4][CT];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < CT; ++t)
+            b[j][t] = load4(x + (t * 16 + lr) * US + j * 16 + g4 * 4);
+        issued();
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (j <= w) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+              for (int t = 0; t < CT; ++t) to[t] = mma4(now.m[j][s], b[j][t][s], to[t]);
+          }
+      };
+      using std::integral_constant;
+      if constexpr (keeps) {
+        rows_of(integral_constant<int, 0>{}, integral_constant<int, ND>{});
+#pragma unroll
+        for (int t = 0; t < CT; ++t) {
+          f32x4 x;
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            x[r] = vf[t][r] - (CH ? acc[t][r] : now.gr[r] * acc[t][r]);
+          store4(xt + (t * 16 + lr) * US + row_c, x);
+        }
+      } else {
+        rows_of(integral_constant<int, 0>{}, integral_constant<int, (ND + 1) / 2>{});
       }
-    load_mat(tm, cn, tf);
+      sync_lds();
+
+      float ka[NT][4][4];  // columns of kt
+      if constexpr (keeps) {
+        f32x4 u[CT];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      us[(row_c + r) * 17 + lr] = u[r];
-      uw[(row_c + r) * 17 + lr] = u[r] * glk[r];
+        for (int t = 0; t < CT; ++t) u[t] = zero;
+        if (!CH) {
+#pragma unroll
+          for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+              for (int s = 0; s < 4; ++s) {
+                const int i = j * 16 + g4 * 4 + s, d = min(w * 16 + n * 64, Dp - 16) + lr;
+                ka[n][j][s] = k[i * Dp + place(i, d >> 2) * 4 + (lr & 3)];
+              }
+        }
+        lower(xt, u);
+#pragma unroll
+        for (int t = 0; t < CT; ++t) {
+          store4(ut + (t * 16 + lr) * US + row_c, u[t]);
+          if (!CH) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u[t][r] *= now.gl[r];
+            store4(wt + (t * 16 + lr) * US + row_c, u[t]);
+          }
+        }
+      } else {
+        if constexpr (ND > 1)
+          rows_of(integral_constant<int, (ND + 1) / 2>{}, integral_constant<int, ND>{});
+        if (!CH) {
+#pragma unroll
+          for (int t = 0; t < CT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][r] *= now.gr[r];
+        }
+      }
+      if (CH) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // kt of this chunk
+      sync_lds();
+
+      if constexpr (keeps) {
+        const float* uw = CH ? ut : wt;
+        f32x4 b[4][CT];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < CT; ++t)
+            b[j][t] = load4(uw + (t * 16 + lr) * US + j * 16 + g4 * 4);
+        if (CH) {
+#pragma unroll
+          for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+              for (int s = 0; s < 4; ++s) {
+                const int i = j * 16 + g4 * 4 + s, d = min(w * 16 + n * 64, Dp - 16) + lr;
+                ka[n][j][s] = kc[i * Dp + place(i, d >> 2) * 4 + (lr & 3)];
+              }
+        }
+        issued();
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int t = 0; t < CT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) own[n][t][r] *= CH ? now.gd[n][r] : now.all;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+              for (int t = 0; t < CT; ++t)
+                own[n][t] = mma4(ka[n][j][s], b[j][t][s], own[n][t]);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          const int d0 = w * 16 + n * 64;
+          if (d0 >= Dp) continue;
+#pragma unroll
+          for (int t = 0; t < CT; ++t)
+            store4(st + (t * 16 + lr) * SS + d0 + g4 * 4, own[n][t]);
+        }
+      } else {
+        lower(ut, acc);
+        float* op = o + ((long)i0 * H + h) * Vp + v0;
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (row_c + r < len) op[(unsigned)(row_c + r) * vrow + t * 16 + lr] = acc[t][r];
+      }
+      arrived();
+      __syncthreads();
+      // all have read this chunk's kt
+      if (CH && c + 1 < c_end) stage_kt(j0, jl);
+      i0 = j0;
+      len = jl;
+      cn = ahead;
+      j0 = __builtin_amdgcn_readfirstlane(then.x) - tok_base;
+      jl = __builtin_amdgcn_readfirstlane(then.y);
     }
-    __syncthreads();
-
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j <= wid) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-          oc = mma4(af[j][s], us[(j * 16 + g4 * 4 + s) * 17 + lr], oc);
-      }
-    load_mat(am, cn, af);
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (row_c + r < len)
-        o[((long)(i0 + row_c + r) * H + h) * Vp + v0 + lr] = oc[r];
-
+    if (!keeps) return;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
-      const int d0 = wid * 16 + n * 64;
-      if (d0 >= Dp) continue;
-      f32x4 sn;
+      const int d0 = w * 16 + n * 64 + g4 * 4;
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        sn[r] = (CH ? gd[n][r] : g_now) * ss[(d0 + g4 * 4 + r) * 17 + lr];
+      for (int t = 0; t < CT; ++t) {
+        const int v = v0 + t * 16 + lr;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-          sn = mma4(kt[n][j][s], uw[(j * 16 + g4 * 4 + s) * 17 + lr], sn);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ss[(d0 + g4 * 4 + r) * 17 + lr] = sn[r];
+        for (int r = 0; r < 4; ++r)
+          if (d0 + r < D && v < V) sg[(long)(d0 + r) * V + v] = own[n][t][r];
+      }
     }
-    load_kt(j0, jl);
-    load_decay(cn);
-    __syncthreads();
-    i0 = j0;
-    len = jl;
-  }
-  for (int i = tid; i < Dp * 16; i += 256) {
-    const int d = i >> 4, v = v0 + (i & 15);
-    if (d < D && v < V) sg[(long)d * V + v] = ss[d * 17 + (i & 15)];
+  };
+  if (wid < 4) {
+    walk(std::true_type{});
+  } else {
+    walk(std::false_type{});
   }
 }
 
@@ -1223,17 +1440,45 @@ struct DeltaLongArgs {
   float eps;
 };
 
+template <typename T, int ND, int CT, bool CH>
+static void delta_walk_tiles(const DeltaLongArgs& a, const DeltaDims& dm,
+                             const float* q, const float* k, const float* kt,
+                             int KH, hipStream_t stream) {
+  const size_t smem =
+      ((CH ? 3 : 2) * DR_CHUNK * ND * 16 +
+       CT * 16 * (ND * 16 + 4 + 3 * (DR_CHUNK + 4))) * sizeof(float);
+  if (smem > 65536)
+    (void)hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&delta_walk_fixed_kernel<T, ND, CT, CH>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+  const dim3 grid((unsigned)(a.Vp / (16 * CT) * dm.H * a.n_long));
+  delta_walk_fixed_kernel<T, ND, CT, CH><<<grid, dim3(512), smem, stream>>>(
+      q, k, kt, (const T*)a.vn, a.tm, a.am, a.ge, a.state, a.o, a.chunks,
+      a.chunk_cu, a.pos0, a.slots, a.n_short, a.tok_base, a.n_long, KH, dm.H, dm.D,
+      dm.V, a.Vp);
+}
+
+template <typename T, int ND, bool CH>
+static void delta_walk_go(const DeltaLongArgs& a, const DeltaDims& dm,
+                          const float* q, const float* k, const float* kt, int KH,
+                          hipStream_t stream) {
+  // A CU has one block, so with more than 256 column tiles two of them a block: 32
+  // chunks of 4 requests, 16 heads, 231 us with one, 186 with two; at 256 (2 requests
+  // of 63 chunks) 228 and 344.
+  if (a.Vp % 32 == 0 && (long)a.Vp / 16 * dm.H * a.n_long > 256) {
+    delta_walk_tiles<T, ND, 2, CH>(a, dm, q, k, kt, KH, stream);
+  } else {
+    delta_walk_tiles<T, ND, 1, CH>(a, dm, q, k, kt, KH, stream);
+  }
+}
+
 // KH: heads that q, k and kt have
 template <typename T, bool CH>
 static void delta_walk_t(const DeltaLongArgs& a, const DeltaDims& dm,
                          const float* q, const float* k, const float* kt, int KH,
                          dim3 grid, hipStream_t stream) {
   const dim3 block(256);
-#define DW_GO(N)                                                              \
-  delta_walk_fixed_kernel<T, N, CH><<<grid, block, 0, stream>>>(              \
-      q, k, kt, (const T*)a.vn, a.tm, a.am, a.ge, a.state, a.o, a.chunks,     \
-      a.chunk_cu, a.pos0, a.slots, a.n_short, a.tok_base, KH, dm.H, dm.D,     \
-      dm.V, a.Vp)
+#define DW_GO(N) delta_walk_go<T, N, CH>(a, dm, q, k, kt, KH, stream)
   if (a.Dp == 16) DW_GO(1);
   else if (a.Dp == 32) DW_GO(2);
   else if (a.Dp == 64) DW_GO(4);

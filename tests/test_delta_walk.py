@@ -1,0 +1,58 @@
+"""The walk over chunks of the gated delta rule: a block takes one column tile of a
+(request, head) where there are few of them and two where there are many.  The tests
+of single requests against the oracle cover the first; here many requests at once
+have to give what each gives alone."""
+
+import pytest
+import torch
+
+from mlx_sharding_amd.models.mixers import GatedDelta
+from mlx_sharding_amd.ops.paged import PagedState, RaggedBatch
+
+pytestmark = pytest.mark.gpu
+
+LENS = (34, 80, 81, 82, 145, 146, 217, 50, 338)
+
+
+def _run(m, rows, dtype):
+    """Each request in two portions, so that the states of the first are read back."""
+    lens = [len(r) for r in rows]
+    dev = rows[0].device
+    state = PagedState([m.store_spec()], sum(-(-n // 64) * 64 for n in lens), len(lens),
+                       dtype, dev)
+    held = [state.admit(i) for i in range(len(lens))]
+    out = []
+    for part in (0, 1):
+        take = [r[-17:] if part else r[:-17] for r in rows]
+        for i, h in enumerate(held):
+            state.reserve(i, h.length + len(take[i]))
+        b = RaggedBatch([(h, len(t)) for h, t in zip(held, take)], dev)
+        y = m(torch.cat(take), b, state.layers[0])
+        out.append(y.split([len(t) for t in take]))
+        for h, t in zip(held, take):
+            h.length += len(t)
+    return [torch.cat(x) for x in zip(*out)]
+
+
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("heads", [4, 8])   # 36 and 72 (request, head): by eights or not
+@pytest.mark.parametrize("D", [16, 32, 64, 96, 128])
+def test_many_as_alone(D, heads, channel):
+    dev = torch.device("cuda")
+    torch.manual_seed(D + heads)
+    with dev:
+        m = GatedDelta(64, heads, heads // 2, D, 128, 4, 1e-6, dtype=torch.float32,
+                       ranks=(32, 32) if channel else None,
+                       gate="sigmoid" if channel else "silu")
+    for name, p in m.named_parameters():
+        p.data.normal_(0, 0.5 if "conv" in name else 0.1)
+    m.A_log.data.normal_(0.5, 0.7)
+    m.dt_bias.data.normal_(-3, 1)
+    m.prepare()
+    rows = [torch.randn(n, 64, device=dev) for n in LENS]
+    many = _run(m, rows, torch.float32)
+    for r, got in zip(rows, many):
+        want, = _run(m, [r], torch.float32)
+        # the projections may sum in another order: a few roundings of 2^-24 over 64
+        # terms, carried through a state that forgets
+        assert (got - want).abs().max() <= 1e-4 * want.abs().max()
