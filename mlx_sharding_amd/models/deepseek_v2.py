@@ -221,6 +221,38 @@ class MLAAttention(nn.Module):
         return ext.mla_attend(q, rows, self._w_rows[1], self.scale, pos,
                               at + 1).view(B, 1, -1)
 
+    def _prompt_ok(self, qh, latent, cos, cache) -> bool:
+        """Whether mla_rows and mla_prompt take this prompt."""
+        norm = self.kv_a_layernorm.weight
+        return (cache.graph_pos is None and ops.use_native(qh)
+                and (self.qk_nope, self.qk_rope, self.v_head_dim) == (128, 64, 128)
+                and qh.dtype == latent.dtype == cache.dtype == norm.dtype
+                == torch.bfloat16 and cos.dtype == torch.float32
+                and self.kv_lora_rank % 8 == 0
+                and latent.data_ptr() % 16 == 0 and latent.stride(1) % 8 == 0
+                and (latent.shape[0] == 1
+                     or latent.stride(0) == latent.shape[1] * latent.stride(1))
+                and qh.data_ptr() % 16 == 0 and qh.stride(1) % 8 == 0
+                and norm.data_ptr() % 16 == 0)
+
+    def _prompt(self, qh, latent, cos, sin, cache: KVCache):
+        """Attention of a prompt: [B, T, heads * v].  Keys are never put together:
+        the kernel takes their parts where the projection and the cache have them,
+        and turns the queries."""
+        B, T, _ = latent.shape
+        ext, norm = ops.hip_ext(), self.kv_a_layernorm
+        _, at = cache.claim(B, T)
+        rows = cache.keys_buffer()
+        cos, sin = cos.contiguous(), sin.contiguous()
+        c = ext.mla_rows(latent, norm.weight, norm.eps, norm.weight_offset, cos,
+                         sin, rows, at, at == 0)
+        S = at + T
+        if at:  # earlier rows are in the cache alone
+            c = rows[:, 0, :S, : self.kv_lora_rank].contiguous()
+        kv = self.kv_b_proj(c).view(B, S, self.n_heads, -1)
+        q = qh.view(B, T, self.n_heads, self.qk_head_dim)
+        return ext.mla_prompt(q, kv, rows, cos, sin, self.scale, at)
+
     def _ensure_absorb(self, device, dtype):
         if self._w_uk is not None:
             return
@@ -272,6 +304,8 @@ class MLAAttention(nn.Module):
             ckv = self.kv_a_proj_with_mqa(x)
         if T == 1 and self._one_token_ok(qh, ckv, cache):
             return self._output(self._one_token(qh, ckv, cos, sin, cache), residual)
+        if T > 1 and self._prompt_ok(qh, ckv, cos, cache):
+            return self._output(self._prompt(qh, ckv, cos, sin, cache), residual)
         qh = qh.view(B, T, nh, self.qk_head_dim)
         q_nope = qh[..., : self.qk_nope]
         q_pe = ops.apply_rope(qh[..., self.qk_nope:], cos, sin,

@@ -42,6 +42,9 @@ void launch_attn_prefill(const void*, const void*, const void*, void*, int,
                          int, int, int, int, long, long, long, long, long, int,
                          int, float, float, int, int, hipStream_t);
 bool attn_prefill_supported(int, int);
+void launch_mla_prompt(const void*, const void*, const void*, const float*,
+                       const float*, void*, int, int, int, int, long, long, long, long,
+                       int, float, int, hipStream_t);
 void launch_mfma_probe(const void*, const void*, float*, hipStream_t);
 void launch_w4a16_gemv(const void*, const void*, const void*, const void*,
                        void*, int, int, int, int, int, hipStream_t);
@@ -467,6 +470,77 @@ torch::Tensor mla_attend(torch::Tensor q, torch::Tensor cache, torch::Tensor w,
                         (const __bf16*)w.data_ptr(), (__bf16*)out.data_ptr(), (int)N,
                         (int)heads, (int)rank, (int)vdim, n};
   launch_mla_finish(&a, cur_stream());
+  return out;
+}
+
+static void check_turns(const torch::Tensor& cos, const torch::Tensor& sin, long n) {
+  for (const auto& t : {cos, sin})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kFloat32 &&
+                    t.is_contiguous() && t.numel() == n &&
+                    reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0,
+                "rotations of the prompt's positions");
+}
+
+// Rows [B, T, rank + rope] of a prompt, as projected, into the cache from row pos0 on;
+// with `rows` also returned, normed, [B, T, rank].
+torch::Tensor mla_rows(torch::Tensor latent, torch::Tensor norm, double eps,
+                       double offset, torch::Tensor cos, torch::Tensor sin,
+                       torch::Tensor cache, int64_t pos0, bool rows) {
+  for (const auto& t : {latent, norm, cache}) check_bf16(t, "operand");
+  TORCH_CHECK(latent.dim() == 3 && norm.dim() == 1 && cache.dim() == 4 &&
+                  cache.size(1) == 1, "shapes");
+  const long B = latent.size(0), T = latent.size(1), rank = norm.size(0);
+  const long rope = latent.size(2) - rank;
+  TORCH_CHECK(B >= 1 && T >= 1 && cache.size(0) == B &&
+                  cache.size(3) == rank + rope && rank >= 8 && rank % 8 == 0 &&
+                  rope >= 8 && rope % 8 == 0, "sizes");
+  TORCH_CHECK(pos0 >= 0 && pos0 + T <= cache.size(2), "no room in the cache");
+  auto whole = [](const torch::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  TORCH_CHECK(latent.stride(2) == 1 && latent.stride(1) % 8 == 0 &&
+                  (B == 1 || latent.stride(0) == T * latent.stride(1)) &&
+                  norm.is_contiguous() && cache.is_contiguous() && whole(latent) &&
+                  whole(norm) && whole(cache), "layout");
+  check_turns(cos, sin, T * rope / 2);
+  torch::Tensor out;
+  if (rows) out = torch::empty({B, T, rank}, latent.options());
+  const MlaRowsArgs a{
+      (const __bf16*)latent.data_ptr(), (const __bf16*)norm.data_ptr(),
+      cos.data_ptr<float>(), sin.data_ptr<float>(), (__bf16*)cache.data_ptr(),
+      rows ? (__bf16*)out.data_ptr() : nullptr, latent.stride(1), cache.size(2),
+      pos0, B * T, (int)T, (int)rank, (int)rope, (float)eps, (float)offset};
+  launch_mla_rows(&a, cur_stream());
+  return out;
+}
+
+// q [B, T, H, 192], unrotated; kv [B, S, H, 256]; cache [B, 1, cap, width] with S
+// rows.  Returns [B, T, H * 128].
+torch::Tensor mla_prompt(torch::Tensor q, torch::Tensor kv, torch::Tensor cache,
+                         torch::Tensor cos, torch::Tensor sin, double scale,
+                         int64_t causal_offset) {
+  for (const auto& t : {q, kv, cache}) check_bf16(t, "operand");
+  TORCH_CHECK(q.dim() == 4 && kv.dim() == 4 && cache.dim() == 4, "shapes");
+  const long B = q.size(0), T = q.size(1), H = q.size(2), S = kv.size(1);
+  TORCH_CHECK(B >= 1 && T >= 1 && H >= 1 && q.size(3) == 192 && kv.size(0) == B &&
+                  kv.size(2) == H && kv.size(3) == 256 && cache.size(0) == B &&
+                  cache.size(1) == 1 && cache.size(3) >= 64 &&
+                  cache.size(3) % 8 == 0, "sizes");
+  TORCH_CHECK(causal_offset >= 0 && causal_offset + T == S && S <= cache.size(2),
+              "rows of the cache");
+  for (const auto& t : {q, kv, cache})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "alignment");
+  TORCH_CHECK(q.stride(3) == 1 && q.stride(0) % 8 == 0 && q.stride(1) % 8 == 0 &&
+                  q.stride(2) % 8 == 0 && kv.is_contiguous() &&
+                  cache.is_contiguous(), "layout");
+  TORCH_CHECK(H <= 65536 / 8, "row offsets of a tile in 32 bits");
+  check_turns(cos, sin, T * 32);
+  auto out = torch::empty({B, T, H * 128}, q.options());
+  launch_mla_prompt(q.data_ptr(), kv.data_ptr(), cache.data_ptr(),
+                    cos.data_ptr<float>(), sin.data_ptr<float>(), out.data_ptr(),
+                    (int)B, (int)H, (int)T, (int)S, q.stride(0), q.stride(2),
+                    q.stride(1), cache.size(2), (int)cache.size(3), (float)scale,
+                    (int)causal_offset, cur_stream());
   return out;
 }
 
@@ -994,6 +1068,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return attn_prefill_supported((int)dk, (int)dv);
   });
   m.def("linear_few", &linear_few);
+  m.def("mla_rows", &mla_rows);
+  m.def("mla_prompt", &mla_prompt);
   m.def("mla_prepare", &mla_prepare);
   m.def("mla_attend", &mla_attend);
   m.def("attn_decode_tile", [](int64_t g, int64_t dk, int64_t dv, bool inrow) {

@@ -23,7 +23,18 @@ struct MlaFinishArgs {
   int N, heads, rank, vdim, slices;
 };
 
+// Rows of a prompt.  rank and rope are multiples of 8, all rows begin at 16 bytes.
+struct MlaRowsArgs {
+  const __bf16 *latent, *norm;  // [B * T, rank + rope], [rank]
+  const float *cos, *sin;       // [T, rope / 2]
+  __bf16 *cache, *rows;         // [B, cap, rank + rope], [B * T, rank] or null
+  long ld_latent, cap, pos0, N;
+  int T, rank, rope;
+  float eps, offset;
+};
+
 extern "C" {
+void launch_mla_rows(const MlaRowsArgs*, hipStream_t);
 void launch_mla_prepare(const MlaPrepareArgs*, hipStream_t);
 void launch_mla_finish(const MlaFinishArgs*, hipStream_t);
 }

@@ -176,3 +176,53 @@ def test_latent_one_token(N, S, nope, vdim, captured):
     # the latents between the two products are rounded to bf16
     off = torch.bmm(2.0 ** -8 * o.abs() + 2.0 ** -13 * size, w.abs())
     assert close(out, expect, off.transpose(0, 1).reshape(N, -1))
+
+
+@pytest.mark.parametrize("B,T,at,H", [(1, 2, 0, 2), (2, 33, 0, 3), (3, 130, 70, 16),
+                                      (1, 300, 129, 8), (8, 128, 0, 16)])
+def test_latent_prompt(B, T, at, H):
+    """A prompt, or the next part of one, over keys in two parts: rows into the
+    cache, then attention with queries that the kernel turns; tiles of 128 queries
+    and 64 keys with remainders, operands as slices of wider rows."""
+    rank, rope, room = 64, 64, 3
+    S = at + T
+    torch.manual_seed(S + H)
+    bf = lambda *s: torch.randn(*s, device="cuda").bfloat16()  # noqa: E731
+    q, latent = bf(B, T, H * 192 + rank + rope).split([H * 192, rank + rope], -1)
+    norm = (1 + 0.1 * torch.randn(rank, device="cuda")).bfloat16()
+    angle = torch.rand(T, rope // 2, device="cuda") * 6
+    cos, sin = torch.cos(angle), torch.sin(angle)
+    cache = cached(B, 1, at, rank + rope, room + T).as_strided(
+        (B, 1, S + room, rank + rope),
+        ((S + room) * (rank + rope), (S + room) * (rank + rope), rank + rope, 1))
+    before = cache.clone()
+    rows = ext().mla_rows(latent, norm, 1e-6, 0.0, cos, sin, cache, at, True)
+
+    def turned(t, c, s):
+        a, b = t.double()[..., 0::2], t.double()[..., 1::2]
+        return torch.stack([a * c - b * s, b * c + a * s], -1).flatten(-2)
+
+    close = lambda got, expect: bool(  # noqa: E731
+        ((got.double() - expect).abs() <= 2.0 ** -8 * expect.abs() + 1e-5).all())
+    c = latent[..., :rank].double()
+    normed = c * torch.rsqrt(c.pow(2).mean(-1, keepdim=True) + 1e-6) * norm.double()
+    assert close(rows, normed)
+    new = cache[:, 0, at: S]
+    assert torch.equal(new[..., :rank], rows)
+    assert close(new[..., rank:], turned(latent[..., rank:], cos.double(), sin.double()))
+    others = torch.cat([cache[:, :, :at], cache[:, :, S:]], 2)
+    assert torch.equal(others.view(torch.int16),
+                       torch.cat([before[:, :, :at], before[:, :, S:]], 2).view(torch.int16))
+    kv = bf(B, S, H, 256)
+    qh = q.view(B, T, H, 192)
+    out = ext().mla_prompt(qh, kv, cache, cos, sin, 0.1, at).view(B, T, H, 128)
+    k = torch.cat([kv[..., :128], cache[:, 0, :S, None, rank:].expand(B, S, H, 64)], -1)
+    # queries are rounded behind their rotation
+    qt = torch.cat([qh[..., :128].double(), turned(
+        qh[..., 128:], cos.double()[:, None], sin.double()[:, None]).bfloat16().double()], -1)
+    expect, size = attention(qt.transpose(1, 2), k.transpose(1, 2),
+                             kv[..., 128:].transpose(1, 2), 0.1, 0.0, 0, at)
+    # a query that rounds the other way than in 64 bits moves scores: 64 terms of
+    # 2^-8 times |q k| near 1, few of them; weights are rounded to bf16
+    bound = 2.0 ** -8 * expect.abs() + 2.0 ** -7 * size + 1e-5
+    assert bool(((out.transpose(1, 2) - expect).abs() <= bound).all())
