@@ -9,6 +9,7 @@
 #include "linear_few.h"
 #include "mla_decode.h"
 #include "moe_rows.h"
+#include "moe_tiles.h"
 
 extern "C" {
 void launch_rms_norm(const void*, void*, const void*, long, int, float, float,
@@ -582,6 +583,54 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   return out.transpose(1, 2);
 }
 
+// Routed experts of a prompt: silu(x gate^T) * (x up^T), down of that, for the pairs
+// of choice [N, top] (int64).  Returns (rows [N * top, H], place of each pair).
+std::vector<torch::Tensor> moe_tiles(torch::Tensor x, torch::Tensor choice,
+                                     torch::Tensor gate, torch::Tensor up,
+                                     torch::Tensor down, int64_t tile) {
+  for (const auto& t : {x, gate, up, down}) check_bf16(t, "operand");
+  TORCH_CHECK(x.dim() == 2 && choice.dim() == 2 && gate.dim() == 3 &&
+                  down.dim() == 3 && gate.sizes() == up.sizes(), "shapes");
+  const long N = x.size(0), H = x.size(1), top = choice.size(1);
+  const long E = gate.size(0), I = gate.size(1), P = N * top;
+  TORCH_CHECK(choice.size(0) == N && gate.size(2) == H && down.size(0) == E &&
+                  down.size(1) == H && down.size(2) == I, "sizes");
+  TORCH_CHECK(choice.is_cuda() && choice.scalar_type() == torch::kInt64 &&
+                  choice.is_contiguous(), "choice: int64");
+  TORCH_CHECK(H % 64 == 0 && I % 64 == 0 && H >= 128 && I >= 128 &&
+                  E >= 1 && E <= MT_EXPERTS && P >= 1 && P < (1L << 30) &&
+                  (tile == 128 || tile == 256), "sizes that there is no kernel for");
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.stride(0) >= H &&
+                  N * x.stride(0) < (1L << 31) && H * I < (1L << 31) &&
+                  gate.is_contiguous() && up.is_contiguous() &&
+                  down.is_contiguous(), "layout");
+  for (const auto& t : {x, gate, up, down})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "alignment");
+  const int blocks = (int)((P + MT_BLOCK_PAIRS - 1) / MT_BLOCK_PAIRS);
+  const long most = P / tile + E;  // tiles
+  auto ints = torch::empty({blocks * E + 3 * most + 1 + P}, x.options().dtype(torch::kInt32));
+  auto where = torch::empty({N, top}, ints.options());
+  int* hist = ints.data_ptr<int>();
+  int* tiles = hist + blocks * E;
+  int* n_tiles = tiles + 3 * most;
+  int* tokens = n_tiles + 1;
+  const MoePlaceArgs place{choice.data_ptr<int64_t>(), hist, tiles, n_tiles,
+                           where.data_ptr<int>(), tokens, (int)P, (int)top, (int)E,
+                           blocks, (int)tile};
+  launch_moe_place(&place, cur_stream());
+  auto h = torch::empty({P, I}, x.options());
+  auto y = torch::empty({P, H}, x.options());
+  MoeTilesArgs a{(const char*)x.data_ptr(), (const char*)gate.data_ptr(),
+                 (const char*)up.data_ptr(), (__bf16*)h.data_ptr(), tokens, tiles,
+                 n_tiles, x.stride(0) * 2, (int)I, (int)H, 0};
+  launch_moe_tiles(&a, (int)tile, true, cur_stream());
+  MoeTilesArgs b{(const char*)h.data_ptr(), (const char*)down.data_ptr(), nullptr,
+                 (__bf16*)y.data_ptr(), nullptr, tiles, n_tiles, I * 2, (int)H,
+                 (int)I, 0};
+  launch_moe_tiles(&b, (int)tile, false, cur_stream());
+  return {y, where};
+}
+
 torch::Tensor mfma_probe(torch::Tensor A, torch::Tensor Bm) {
   check_bf16(A, "A");
   auto D = torch::empty({16, 16}, A.options().dtype(torch::kFloat32));
@@ -1080,6 +1129,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_rows", &moe_rows);
   m.def("moe_rows_longest", [](int64_t bits) { return moe_rows_longest((int)bits); });
   m.def("moe_combine", &moe_combine);
+  m.def("moe_tiles", &moe_tiles);
   m.def("linear_few", &linear_few);
   m.def("mfma_probe", &mfma_probe);
   m.def("w4a16_gemv", &w4a16_gemv);

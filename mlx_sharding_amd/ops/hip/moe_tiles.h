@@ -1,0 +1,34 @@
+// Arguments of the routed experts' kernels of a prompt (moe_tiles.hip).
+#pragma once
+
+#include "hip_common.h"
+
+#define MT_BLOCK_PAIRS 2048  // (token, expert) pairs of a placing block
+#define MT_EXPERTS 1024
+
+struct MoePlaceArgs {
+  const long* choice;  // [pairs] expert
+  int* hist;           // [blocks, experts]; from moe_plan on the first place of each
+  int* tiles;          // [count, 3]: expert, first pair, pairs
+  int* n_tiles;
+  int *where, *tokens;  // [pairs]: place of a pair, token of a place
+  int pairs, top, experts, blocks, tile;
+};
+
+// y[p, o] = x[token of p] . w[expert of p, o], of a gated unit silu(that) times the
+// same with w2.  K and O are multiples of 64, K at least 128; rows of w begin at 16
+// bytes; offsets within x (tokens given) and within an expert's matrix below 2^32.
+struct MoeTilesArgs {
+  const char *x, *w, *w2;  // [rows, K], [experts, O, K]; w2: up's
+  __bf16* y;               // [pairs, O]
+  const int* tokens;       // gated: row of x of a pair; else the pair is
+  const int *tiles, *n_tiles;
+  long xstride;            // bytes
+  int O, K, cols;          // cols: blocks across O
+};
+
+extern "C" {
+void launch_moe_place(const MoePlaceArgs*, hipStream_t);
+// pairs of a tile: 256 or 128
+void launch_moe_tiles(MoeTilesArgs*, int tile, bool gated, hipStream_t);
+}
