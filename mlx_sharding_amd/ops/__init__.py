@@ -208,7 +208,7 @@ def _dq_cache_ok(nbytes: int) -> bool:
     return True
 
 
-_FEW_ROWS = 16  # tokens of a batch that linear_few takes
+_FEW_ROWS = 64  # tokens of a batch that linear_few takes
 _ACTS = {None: 0, "silu": 1, "gelu_tanh": 2}
 
 
@@ -220,15 +220,19 @@ def _plain(t: torch.Tensor) -> bool:
             and torch.autograd.forward_ad._current_level < 0)
 
 
-def few_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Whether x W^T runs on linear_few.hip: up to 16 bf16 rows that begin, as
-    W's, at whole 16-byte vectors.  A contraction above 8192 only for 8 rows: 16
-    rows of 14336 into 4096 take 29 us there and 26 in the library, 8 take 24.6
-    and 26.6."""
+def few_rows(x: torch.Tensor, weight: torch.Tensor, alone: bool = False) -> bool:
+    """Whether x W^T runs on linear_few.hip: up to 64 bf16 rows that begin, as
+    W's, at whole 16-byte vectors.  A contraction above 8192 for 8 rows, or into
+    4096: 8 rows of 14336 into 4096 take 24.6 us there and 26.6 in the library, 32
+    rows 30.4 and 30.5, 64 rows 40.1 and 38.9.  ``alone``: with nothing taken along;
+    then the library is the better one for many rows of large weights (64 rows of
+    4096 into 28672: 54 us there, 51 in the library)."""
     K = weight.shape[-1]
     rows = x.numel() // K if K else 0
-    return (0 < rows <= (_FEW_ROWS if K <= 8192 else 8) and _use_hip(x)
-            and weight.dim() == 2 and K % 32 == 0 and weight.shape[0] > 0
+    return (0 < rows <= _FEW_ROWS and _use_hip(x) and weight.dim() == 2
+            and (K <= 8192 or rows <= 8 or weight.shape[0] <= 4096)
+            and not (alone and rows > 32 and weight.shape[0] * K > 1 << 25)
+            and K % 32 == 0 and weight.shape[0] > 0
             and x.dtype == weight.dtype == torch.bfloat16 and weight.is_cuda
             and _plain(x) and _plain(weight) and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
             and x.stride(-1) == 1 and weight.data_ptr() % 16 == 0
@@ -288,7 +292,7 @@ def few_tokens(x: torch.Tensor) -> bool:
 
 
 def linear(x, weight, bias=None):
-    """Dense linear; up to 16 rows run on linear_few.hip.  The MFMA decode GEMV (MLXS_AMD_DENSE_GEMV=1) was
+    """Dense linear; up to 64 rows run on linear_few.hip.  The MFMA decode GEMV (MLXS_AMD_DENSE_GEMV=1) was
     a NEGATIVE result at batch-64 decode shapes: hipBLASLt's small-GEMM
     kernels run ~13 us in-graph and the split-K fp32-atomic traffic
     (M*O*4*nk bytes) rivals the weight bytes on small-O projections
@@ -337,7 +341,7 @@ def linear(x, weight, bias=None):
             if bias is not None:
                 y = y + bias
             return y.reshape(*lead, y.shape[-1])
-    if few_rows(x, weight) and (bias is None or _plain(bias)):
+    if few_rows(x, weight, alone=True) and (bias is None or _plain(bias)):
         return _linear_few(x, weight, bias)
     return torch.nn.functional.linear(x, weight, bias)
 

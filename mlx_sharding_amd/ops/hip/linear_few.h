@@ -1,4 +1,4 @@
-// y = x W^T for up to 16 rows, with what goes with it (linear_few.hip); part of
+// y = x W^T for up to 64 rows, with what goes with it (linear_few.hip); part of
 // both extensions.
 #pragma once
 
@@ -29,8 +29,8 @@ static torch::Tensor linear_few(torch::Tensor x, torch::Tensor w,
   TORCH_CHECK(act >= 0 && act <= 2, "unknown unit");
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "shapes");
   const int M = x.size(0), K = x.size(1), O = w.size(0) / (act ? 2 : 1);
-  TORCH_CHECK(M >= 1 && M <= 16 && K >= 32 && K % 32 == 0 && O >= 1,
-              "1 to 16 rows of a multiple of 32");
+  TORCH_CHECK(M >= 1 && M <= 64 && K >= 32 && K % 32 == 0 && O >= 1,
+              "1 to 64 rows of a multiple of 32");
   TORCH_CHECK(!act || w.size(0) % 2 == 0, "a gated unit has two halves");
   for (const auto& t : {x, w})
     TORCH_CHECK(t.stride(1) == 1 && t.stride(0) % 8 == 0 && whole(t),

@@ -1,4 +1,4 @@
-// y = x W^T for few rows of x (decoding): what lies between two such products of
+// y = x W^T for few rows of x (decoding, short prompts): what lies between two such products of
 // a layer goes with them.
 //
 //   before:  RMS norm of x's rows with a weight per column
@@ -32,6 +32,45 @@ struct LinearFewArgs {
 };
 
 enum { LF_PLAIN = 0, LF_SILU = 1, LF_GELU = 2 };
+
+// sums of four columns of y from `col` on, and of an up projection's, to memory
+template <int ACT>
+__device__ __forceinline__ void finish_columns(const LinearFewArgs& a, int row,
+                                               int col, const f32x4* v) {
+      float o[4];
+  #pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int at = min(col + j, a.O - 1);
+        float f = v[0][j];
+        if (ACT) {
+          float up = v[1][j];
+          if (a.bias) {
+            f += (float)a.bias[at];
+            up += (float)a.bias[a.O + at];
+          }
+          if (ACT == LF_SILU) {
+            f = f / (1.0f + __expf(-f)) * up;
+          } else {
+            const float z = 0.7978845608028654f * (f + 0.044715f * f * f * f);
+            f = 0.5f * f * (1.0f + tanhf(z)) * up;
+          }
+        } else if (a.bias) {
+          f += (float)a.bias[at];
+        }
+        if (a.res) f += (float)a.res[(long)row * a.ldr + at];
+        o[j] = f;
+      }
+      __bf16* y = a.y + (long)row * a.ldy + col;
+      if (col + 3 < a.O && a.ldy % 4 == 0) {
+        typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<bf16x4_t*>(y) =
+            bf16x4_t{(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
+      } else {
+  #pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (col + j < a.O) y[j] = (__bf16)o[j];
+      }
+}
 
 // RT tiles of 16 rows of W; with a gated unit half of them are the gate's, the
 // others the up projection's
@@ -147,41 +186,7 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[h][j] *= f;
     }
-    const int row = l16, col = row0 + r * 16 + lg * 4;
-    if (row >= a.M) continue;
-    float o[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int at = min(col + j, a.O - 1);
-      float f = v[0][j];
-      if (ACT) {
-        float up = v[1][j];
-        if (a.bias) {
-          f += (float)a.bias[at];
-          up += (float)a.bias[a.O + at];
-        }
-        if (ACT == LF_SILU) {
-          f = f / (1.0f + __expf(-f)) * up;
-        } else {
-          const float z = 0.7978845608028654f * (f + 0.044715f * f * f * f);
-          f = 0.5f * f * (1.0f + tanhf(z)) * up;
-        }
-      } else if (a.bias) {
-        f += (float)a.bias[at];
-      }
-      if (a.res) f += (float)a.res[(long)row * a.ldr + at];
-      o[j] = f;
-    }
-    __bf16* y = a.y + (long)row * a.ldy + col;
-    if (col + 3 < a.O && a.ldy % 4 == 0) {
-      typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-      *reinterpret_cast<bf16x4_t*>(y) =
-          bf16x4_t{(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (col + j < a.O) y[j] = (__bf16)o[j];
-    }
+    if (l16 < a.M) finish_columns<ACT>(a, l16, row0 + r * 16 + lg * 4, v);
   }
 }
 
@@ -219,8 +224,227 @@ static void linear_few_tiles(const LinearFewArgs& a, int act, hipStream_t stream
   }
 }
 
+// The same for 17 to 64 rows of x.  Read by each wave from L2 as above, rows of x
+// would be the larger part of what is read, and 64 bytes of each of 16 rows take a
+// load four times as long as whole lines; here x and W come to LDS in whole lines, KS
+// steps of 32 columns at a time, into a ring of stages.  A wave takes one of the steps,
+// for all rows of W and of x or for half of x's.
+// Measured, beside the library's product (us; M x K x O): 17 x 2048 x 2048: 6.2, 11.0;
+// 64 of these: 8.4, 11.7; 64 x 2816 x 2048: 10.0, 14.7; 64 x 2048 x 11264: 15.4, 16.0;
+// 64 x 4096 x 4096: 13.7, 15.1; 64 x 4096 x 28672: 54, 51, with norm and unit 59,
+// beside 60 for three kernels; 64 x 14336 x 4096: 40, 39.  W to registers by rows of 64
+// bytes: 10.6 us for 64 x 2048 x 2048, 70 for 64 x 4096 x 28672.
+#define LS_WAVES 8
+
+// RT, TT: tiles of 16 rows of W and of x
+template <int RT, int TT, int KS, int ACT, bool NORM>
+__global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
+    const LinearFewArgs a) {
+  constexpr int YT = ACT ? RT / 2 : RT;
+  constexpr int PARTS = (RT + TT) * KS / LS_WAVES;  // loads to LDS, wave and stage
+  constexpr int STAGE = (RT + TT) * KS * 1024;
+  constexpr int RING = 4 * STAGE > 140 * 1024 ? 3 : 4;
+  // loads of a wave that may be under way when it comes to a stage
+  constexpr int BEHIND = (RING - 2) * (PARTS + (NORM ? 1 : 0));
+  constexpr int TW = TT * KS / LS_WAVES;            // tiles of x of a wave
+  constexpr int RP = KS * 4;                        // pieces of 16 bytes of a row
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ float squares[NORM ? LS_WAVES : 1][TW][WAVE];
+
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int step = wid % KS, tile0 = wid / KS * TW;
+  const int row0 = blockIdx.x * 16 * YT;
+
+  // A load to LDS is 1 KB of rows of W, then of x.  Pieces of a row are swapped by the
+  // row: those that a read meets lie in different banks.
+  auto place = [](int row, int piece) { return piece ^ (row & 15); };
+  const char* from[PARTS];
+  int col[PARTS];
+#pragma unroll
+  for (int i = 0; i < PARTS; ++i) {
+    const int at = (i * LS_WAVES + wid) * WAVE + lane, row = at / RP;
+    col[i] = place(row, at % RP) * 8;
+    if (row < RT * 16) {
+      const int r = row / 16 / YT * a.O + min(row0 + row / 16 % YT * 16 + row % 16, a.O - 1);
+      from[i] = (const char*)(a.w + (long)r * a.ldw);
+    } else {
+      from[i] = (const char*)(a.x + (long)min(row - RT * 16, a.M - 1) * a.ldx);
+    }
+  }
+  bf16x8_t g[NORM ? RING : 1];
+  const int stages = (a.K + KS * 32 - 1) / (KS * 32);
+  // columns behind the last one repeat others of its row; nobody takes them
+  auto issue = [&](int t, int slot) {
+    const int k0 = min(t, stages - 1) * (KS * 32);
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(
+              from[i] + (unsigned)min(k0 + col[i], a.K - 8) * 2),
+          (__attribute__((address_space(3))) void*)(
+              smem + slot * STAGE + (i * LS_WAVES + wid) * 1024), 16, 0, 0);
+    if (NORM)
+      g[slot] = *reinterpret_cast<const bf16x8_t*>(
+          a.norm + min(k0 + step * 32, a.K - 32) + lg * 8);
+  };
+  f32x4 acc[RT][TW];
+  float sq[TW];
+#pragma unroll
+  for (int i = 0; i < TW; ++i) {
+    sq[i] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[r][i] = f32x4{0, 0, 0, 0};
+  }
+  auto use = [&](int t, int s) {
+    if ((t * KS + step) * 32 >= a.K) return;
+    const char* at = smem + s * STAGE + l16 * RP * 16 + place(l16, step * 4 + lg) * 16;
+    bf16x8_t w[RT], v[TW];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+      w[r] = *reinterpret_cast<const bf16x8_t*>(at + r * RP * 256);
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+      v[i] = *reinterpret_cast<const bf16x8_t*>(at + (RT + tile0 + i) * RP * 256);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < TW; ++i) {
+      if (NORM) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float f = (float)v[i][j];
+          sq[i] = fmaf(f, f, sq[i]);
+          v[i][j] = (__bf16)(f * ((float)g[s][j] + a.offset));
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+        acc[r][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[r], v[i], acc[r][i],
+                                                            0, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < RING - 1; ++t) issue(t, t);
+  int t0 = 0;
+  for (; t0 + RING <= stages; t0 += RING) {
+#pragma unroll
+    for (int s = 0; s < RING; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      // vmcnt, in a form that the compiler takes into account
+      __builtin_amdgcn_s_waitcnt((BEHIND & 15) | (BEHIND >> 4) << 14 | 0xf70);
+      asm volatile("s_barrier" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      issue(t0 + s + RING - 1, (s + RING - 1) % RING);
+      use(t0 + s, s);
+    }
+  }
+  // the remainder is on its way
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0xf70 & ~0xc00f);
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int s = 0; s < RING - 1; ++s)
+    if (t0 + s < stages) use(t0 + s, s);
+  __syncthreads();
+  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [steps][RT][TT][lanes]
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+      red[((step * RT + r) * TT + tile0 + i) * WAVE + lane] = acc[r][i];
+  if (NORM) {
+#pragma unroll
+    for (int i = 0; i < TW; ++i) squares[wid][i][lane] = sq[i];
+  }
+  __syncthreads();
+
+  for (int n = wid; n < YT * TT; n += LS_WAVES) {
+    const int r = n / TT, i = n % TT;
+    f32x4 v[ACT ? 2 : 1];
+#pragma unroll
+    for (int h = 0; h < (ACT ? 2 : 1); ++h) {
+      v[h] = f32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int q = 0; q < KS; ++q) {
+        const f32x4 p = red[((q * RT + r + h * YT) * TT + i) * WAVE + lane];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[h][j] += p[j];
+      }
+    }
+    if (NORM) {
+      float s = 0.0f;
+#pragma unroll
+      for (int q = 0; q < KS; ++q) s += squares[i / TW * KS + q][i % TW][lane];
+      s += __shfl_xor(s, 16, WAVE);
+      s += __shfl_xor(s, 32, WAVE);
+      const float f = rsqrtf(s / a.K + a.eps);
+#pragma unroll
+      for (int h = 0; h < (ACT ? 2 : 1); ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[h][j] *= f;
+    }
+    if (i * 16 + l16 < a.M)
+      finish_columns<ACT>(a, i * 16 + l16, row0 + r * 16 + lg * 4, v);
+  }
+}
+
+template <int RT, int TT, int ACT, bool NORM>
+static void linear_some_go(const LinearFewArgs& a, hipStream_t stream) {
+  constexpr int KS = RT == 1 ? 8 : 4;
+  constexpr int cols = 16 * (ACT ? RT / 2 : RT);
+  constexpr int stage = (RT + TT) * KS * 1024;
+  constexpr int ring = (4 * stage > 140 * 1024 ? 3 : 4) * stage;
+  constexpr int smem = ring > KS * RT * TT * 1024 ? ring : KS * RT * TT * 1024;
+  if (smem > 56 * 1024)  // with the sums of squares above the default limit
+    (void)hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&linear_some_kernel<RT, TT, KS, ACT, NORM>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  linear_some_kernel<RT, TT, KS, ACT, NORM>
+      <<<dim3((unsigned)((a.O + cols - 1) / cols)), dim3(LS_WAVES * WAVE), smem,
+         stream>>>(a);
+}
+
+template <int RT, int ACT>
+static void linear_some_tiles(const LinearFewArgs& a, hipStream_t stream) {
+  if (a.M <= 32) {
+    if (a.norm) {
+      linear_some_go<RT, 2, ACT, true>(a, stream);
+    } else {
+      linear_some_go<RT, 2, ACT, false>(a, stream);
+    }
+  } else {
+    if (a.norm) {
+      linear_some_go<RT, 4, ACT, true>(a, stream);
+    } else {
+      linear_some_go<RT, 4, ACT, false>(a, stream);
+    }
+  }
+}
+
+// Tiles of W's rows per block: one up to 4096 rows, which are 256 blocks, two up to
+// 8192, then four (64 of x; one, two, four: 4096 rows of 4096 13.7, 17.0, 21.7 us;
+// 5632 of 2048 15.0, 10.8, 13.6; 11264 of 2048 23.3, 19.8, 15.4).
+static void linear_some(const LinearFewArgs& a, int act, hipStream_t stream) {
+  const bool many = (act ? 2 : 1) * a.O > 8192;
+  if (act == LF_SILU) {
+    if (many) linear_some_tiles<4, LF_SILU>(a, stream);
+    else linear_some_tiles<2, LF_SILU>(a, stream);
+  } else if (act == LF_GELU) {
+    if (many) linear_some_tiles<4, LF_GELU>(a, stream);
+    else linear_some_tiles<2, LF_GELU>(a, stream);
+  } else if (a.O <= 4096) {
+    linear_some_tiles<1, LF_PLAIN>(a, stream);
+  } else if (many) {
+    linear_some_tiles<4, LF_PLAIN>(a, stream);
+  } else {
+    linear_some_tiles<2, LF_PLAIN>(a, stream);
+  }
+}
+
 // Strides in elements; 16-byte loads: x, w, norm and the strides of x and w are
-// multiples of 8 elements, K of 32.  M up to 16.
+// multiples of 8 elements, K of 32.  M up to 64.
 extern "C" void launch_linear_few(const void* x, const void* w, const void* bias,
                                   const void* res, const void* norm, void* y,
                                   int M, int O, int K, long ldx, long ldw,
@@ -229,5 +453,10 @@ extern "C" void launch_linear_few(const void* x, const void* w, const void* bias
   const LinearFewArgs a{(const __bf16*)x, (const __bf16*)w, (const __bf16*)bias,
                         (const __bf16*)res, (const __bf16*)norm, (__bf16*)y,
                         M, O, K, ldx, ldw, ldr, ldy, eps, offset};
-  linear_few_tiles(a, act, stream);
+  // long rows: 16 of 14336 into 4096 take 29 us above, 27 below
+  if (M > 16 || (M > 8 && K > 8192)) {
+    linear_some(a, act, stream);
+  } else {
+    linear_few_tiles(a, act, stream);
+  }
 }

@@ -22,10 +22,13 @@ def make(M, O, K, act, wide):
 @pytest.mark.parametrize("M,O,K", [
     (1, 2, 32), (3, 18, 96), (16, 34, 2080), (5, 4098, 64), (16, 8194, 160),
     (4, 8210, 32), (9, 4100, 256), (2, 16386, 96), (16, 16400, 1056),
-    (8, 96, 14336), (7, 8200, 2016)])
+    (8, 96, 14336), (7, 8200, 2016), (17, 2, 32), (33, 18, 96), (64, 34, 2080),
+    (20, 4098, 64), (48, 8194, 160), (64, 8210, 288), (31, 16400, 1056),
+    (12, 96, 8224), (40, 100, 9216)])
 def test_edges(M, O, K):
     """Tiles of 16, 32 and 64 columns with remainders, contractions that are not
-    whole chunks, fewer steps than waves; norm, bias, unit, residual."""
+    whole chunks or stages, fewer steps than waves, 16 rows and more, 32 and more;
+    norm, bias, unit, residual."""
     for act in (None, "silu", "gelu_tanh"):
         x, w, norm, bias, res = make(M, O, K, act, wide=K % 64 == 0)
         assert ops.few_rows(x, w)
@@ -62,7 +65,7 @@ def test_edges(M, O, K):
 def test_same_as_separate_kernels():
     """What the projection takes along, beside the kernels it stands for."""
     x, w, norm, bias, _ = make(16, 512, 256, None, wide=True)
-    several = torch.cat([x, x])                   # too many rows: separate
+    several = torch.cat([x] * 5)                  # too many rows: separate
     assert not ops.few_rows(several, w)
     norm = types.SimpleNamespace(
         weight=norm.weight, eps=1e-5, weight_offset=1.0)
