@@ -212,33 +212,22 @@ _FEW_ROWS = 64  # tokens of a batch that linear_few takes
 _ACTS = {None: 0, "silu": 1, "gelu_tanh": 2}
 
 
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
 def _plain(t: torch.Tensor) -> bool:
     """An ordinary tensor that nothing differentiates, maps or traces."""
-    return (type(t) in (torch.Tensor, torch.nn.Parameter)
+    return (type(t) in _TENSORS
             and not (t.requires_grad and torch.is_grad_enabled())
             and not torch._C._functorch.is_functorch_wrapped_tensor(t)
             and torch.autograd.forward_ad._current_level < 0)
 
 
 def few_rows(x: torch.Tensor, weight: torch.Tensor, alone: bool = False) -> bool:
-    """Whether x W^T runs on linear_few.hip: up to 64 bf16 rows that begin, as
-    W's, at whole 16-byte vectors.  A contraction above 8192 for 8 rows, or into
-    4096: 8 rows of 14336 into 4096 take 24.6 us there and 26.6 in the library, 32
-    rows 30.4 and 30.5, 64 rows 40.1 and 38.9.  ``alone``: with nothing taken along;
-    then the library is the better one for many rows of large weights (64 rows of
-    4096 into 28672: 54 us there, 51 in the library)."""
-    K = weight.shape[-1]
-    rows = x.numel() // K if K else 0
-    return (0 < rows <= _FEW_ROWS and _use_hip(x) and weight.dim() == 2
-            and (K <= 8192 or rows <= 8 or weight.shape[0] <= 4096)
-            and not (alone and rows > 32 and weight.shape[0] * K > 1 << 25)
-            and K % 32 == 0 and weight.shape[0] > 0
-            and x.dtype == weight.dtype == torch.bfloat16 and weight.is_cuda
-            and _plain(x) and _plain(weight) and weight.stride(1) == 1 and weight.stride(0) % 8 == 0
-            and x.stride(-1) == 1 and weight.data_ptr() % 16 == 0
-            and x.data_ptr() % 16 == 0
-            and all(s % 8 == 0 for s in x.stride()[:-1])
-            and _few_ext() is not None)
+    """Whether x W^T runs on linear_few.hip (linear_few_takes there says when);
+    ``alone``: with nothing taken along."""
+    ext = _few_ext() if _use_hip(x) and _plain(x) and _plain(weight) else None
+    return ext is not None and ext.linear_few_takes(x, weight, alone)
 
 
 def _few_ext():
@@ -249,28 +238,29 @@ def _few_ext():
 
 
 def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None):
-    x2 = x.reshape(-1, x.shape[-1])
-    if x2.data_ptr() % 16 or x2.stride(0) % 8:
-        x2 = x2.clone()
-    if residual is not None:
-        residual = residual.reshape(x2.shape[0], -1)
-    y = _few_ext().linear_few(
-        x2, weight, bias, residual, None if norm is None else norm.weight,
-        0.0 if norm is None else norm.eps,
-        0.0 if norm is None else norm.weight_offset, _ACTS[act])
-    return y.view(*x.shape[:-1], y.shape[-1])
+    """project on linear_few.hip, or None where that does not take it.  A decoding
+    step calls this for each of its products: what can be seen from the tensors is
+    looked at in native code (in Python that took longer than the launch)."""
+    if (_force_torch() or type(x) not in _TENSORS or type(weight) not in _TENSORS
+            or torch.autograd.forward_ad._current_level >= 0):
+        return None
+    ext = _few_ext()
+    if ext is None:
+        return None
+    if norm is None:
+        return ext.linear_few_try(x, weight, bias, residual, None, 0.0, 0.0, _ACTS[act])
+    return ext.linear_few_try(x, weight, bias, residual, norm.weight, norm.eps,
+                              norm.weight_offset, _ACTS[act])
 
 
 def project(x, weight, bias=None, *, norm=None, act=None, residual=None):
     """x W^T + bias, of x's rows as ``norm`` (an RMSNorm) makes them; ``act``:
     the gated unit act(gate) * up of the result's halves; plus ``residual``.
     One kernel for few rows, else one for each of these."""
-    if (few_rows(x, weight) and (bias is None or _plain(bias))
-            and (norm is None or norm.weight.data_ptr() % 16 == 0
-                 and norm.weight.dtype == torch.bfloat16)
-            and (residual is None or residual.dtype == torch.bfloat16
-                 and residual.stride(-1) == 1)):
-        return _linear_few(x, weight, bias, residual, norm, act)
+    if x.is_cuda:
+        y = _linear_few(x, weight, bias, residual, norm, act)
+        if y is not None:
+            return y
     if norm is not None:
         x = norm(x)
     return finish(linear(x, weight, bias), act, residual)
@@ -297,7 +287,12 @@ def linear(x, weight, bias=None):
     kernels run ~13 us in-graph and the split-K fp32-atomic traffic
     (M*O*4*nk bytes) rivals the weight bytes on small-O projections
     (docs/PERFORMANCE.md).  Kept for shape-specific re-tuning."""
-    if (os.environ.get("MLXS_AMD_DENSE_GEMV")
+    gemv = os.environ.get("MLXS_AMD_DENSE_GEMV")
+    if not gemv and x.is_cuda and weight.shape[-1] < 16384:
+        # neither of the two kernels for long rows below
+        y = _linear_few(x, weight, bias)
+        return torch.nn.functional.linear(x, weight, bias) if y is None else y
+    if (gemv
             and _use_hip(x) and weight.dtype == torch.bfloat16
             and x.dtype == torch.bfloat16 and weight.shape[-1] % 32 == 0
             and weight.is_contiguous()):
@@ -341,9 +336,8 @@ def linear(x, weight, bias=None):
             if bias is not None:
                 y = y + bias
             return y.reshape(*lead, y.shape[-1])
-    if few_rows(x, weight, alone=True) and (bias is None or _plain(bias)):
-        return _linear_few(x, weight, bias)
-    return torch.nn.functional.linear(x, weight, bias)
+    y = _linear_few(x, weight, bias) if x.is_cuda else None
+    return torch.nn.functional.linear(x, weight, bias) if y is None else y
 
 
 def resident_weight(w_q, scales, biases, in_features: int, group_size: int,

@@ -1117,6 +1117,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return attn_prefill_supported((int)dk, (int)dv);
   });
   m.def("linear_few", &linear_few);
+  m.def("linear_few_takes", &linear_few_takes);
+  m.def("linear_few_try", &linear_few_try);
   m.def("mla_rows", &mla_rows);
   m.def("mla_prompt", &mla_prompt);
   m.def("mla_prepare", &mla_prepare);
@@ -1130,7 +1132,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_rows_longest", [](int64_t bits) { return moe_rows_longest((int)bits); });
   m.def("moe_combine", &moe_combine);
   m.def("moe_tiles", &moe_tiles);
-  m.def("linear_few", &linear_few);
   m.def("mfma_probe", &mfma_probe);
   m.def("w4a16_gemv", &w4a16_gemv);
   m.def("w4f16_gemv", &w4f16_gemv);
