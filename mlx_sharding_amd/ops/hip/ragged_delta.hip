@@ -67,13 +67,21 @@ __device__ __forceinline__ float out_gate(float x, bool sigmoid) {
 
 // ---------------------------------------------------------------------------
 // Short portions.  Block = (request, q/k head); its r = H / KH value heads
-// follow one another.  Threads: VT along V (power of two), DG groups along D,
-// RPT state rows per thread.
+// follow one another, HP at a time.  Threads: VT along V (power of two), DG groups
+// along D, RPT state rows per thread.
+//
+// Bound by latency: the state of a head, 64 KB, passes in half a microsecond a
+// block.  So all that a first token needs is asked for at once, what the convolution
+// takes before the state (loads come back in order), heads share their barriers, and
+// every wave makes the norms of q and k for itself: three barriers a token.
+// Measured (before: heads one after the other, nine barriers and loads behind them):
+// 12 requests, 16 q/k heads with 2 value heads of 128 x 128 each, 34 -> 17 us; 16
+// requests, 16 heads with decays per channel, 19.4 -> 16.8 (10.8 for one token each).
 // ---------------------------------------------------------------------------
 
 // EXACT: the threads tile the state without a remainder.  CH: decays per channel.
-template <typename T, int RPT, int NT, bool EXACT, bool CH>
-__global__ __launch_bounds__(NT, RPT <= 32 ? 4 : 2) void delta_short_kernel(
+template <typename T, int RPT, int NT, bool EXACT, bool CH, int HP>
+__global__ __launch_bounds__(NT, EXACT && RPT * HP <= 32 ? 4 : 2) void delta_short_kernel(
     const T* __restrict__ y, const T* __restrict__ z,
     const T* __restrict__ conv_w,
     const T* __restrict__ A_log, const T* __restrict__ dt_bias,
@@ -87,7 +95,7 @@ __global__ __launch_bounds__(NT, RPT <= 32 ? 4 : 2) void delta_short_kernel(
   const int t0 = cu[e];
   const int n = min(cu[e + 1] - t0, DR_SHORT);
   const bool fresh = pos0[e] == 0;
-  const long slot = slots[e];
+  const long slot = __builtin_amdgcn_readfirstlane(slots[e]);
   const int D = dm.D, V = dm.V;
   const int DG = NT / VT;
   const int tid = threadIdx.x;
@@ -98,145 +106,230 @@ __global__ __launch_bounds__(NT, RPT <= 32 ? 4 : 2) void delta_short_kernel(
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* qk = reinterpret_cast<float*>(smem);  // [n][2][D]
-  float* kq = qk + (long)n * 2 * D;            // [n]
-  float* vb = kq + DR_SHORT;                   // [n][V]
-  float* red = vb + (long)n * V;               // [2][DG][VT]
-  float* scratch = red + 2 * NT;               // [NT / WAVE]
-  float* gd = scratch + NT / WAVE;             // [n][D], decays per channel
+  float* vb = qk + (long)n * 2 * D;            // [HP][n][V]
+  float* red = vb + (long)HP * n * V;          // [HP][2][DG][VT]
+  float* scratch = red + HP * 2 * NT;          // [HP][NT / WAVE]
+  float* gd = scratch + HP * (NT / WAVE);      // [HP][n][D], decays per channel
 
   const int v = tid & (VT - 1);
   const int dg = tid / VT;
   const int d0 = dg * RPT;
   const int rep = dm.H / dm.KH;
-  // this thread's part of a head's state; asked for as early as possible
-  float S[RPT];
-  auto load_state = [&](int h) {
+  // this thread's part of the heads' states
+  float S[HP][RPT];
+  auto load_state = [&](int p, int h) {
     // uniform row base + one lane offset: no address per row and lane
     const float* sp = state + ((slot * dm.H + h) * (long)D) * V;
-    const int vc = EXACT ? v : min(v, V - 1);
+    unsigned at = EXACT ? d0 * V + v : min(d0, D - 1) * V + min(v, V - 1);
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
-      const float x = EXACT ? sp[d0 * V + v] : sp[min(d0 + i, D - 1) * V + vc];
-      S[i] = fresh ? 0.0f : x;
+      // rows behind the last one repeat it
+      const float x = sp[at];
+      S[p][i] = fresh ? 0.0f : x;
       if (EXACT) sp += V;
+      else at += d0 + i + 1 < D ? V : 0;
     }
   };
-  load_state(kh * rep);
 
-  // convolution + silu of channel c (column col of y) for all n tokens
-  auto convolve = [&](int c, int col, float* dst, int dstep) {
-    float w[DR_MAXTAPS], x[DR_MAXTAPS];
-    T* cs = conv_state + (slot * C + c) * hist;
-    // taps sit at the end of w/x, so the index of the newest is fixed
-    const int pad = DR_MAXTAPS - dm.taps;
+  // convolution + silu of a channel for all n tokens: channels 2 D of q and k, then
+  // V of each of the heads from h0 on
+  struct Conv {
+    T w[DR_MAXTAPS], x[DR_MAXTAPS - 1], first;
+  };
+  // taps sit at the end of w/x, so the index of the newest is fixed
+  const int pad = DR_MAXTAPS - dm.taps;
+  auto channel = [&](int i, int h0, int& c, int& col) {
+    if (i < 2 * D) {
+      const int which = i / D, d = i - which * D;
+      c = which * dm.KH * D + kh * D + d;
+      col = (which ? dm.kc : dm.qc) + kh * D + d;
+    } else {
+      c = h0 * V + i - 2 * D;
+      col = dm.vc + c;
+      c += 2 * dm.KH * D;
+    }
+  };
+  auto fetch = [&](Conv& f, int i, int h0) {
+    int c, col;
+    channel(i, h0, c, col);
+    const T* cs = conv_state + (slot * C + c) * hist;
 #pragma unroll
     for (int j = 0; j < DR_MAXTAPS; ++j) {
-      w[j] = j >= pad ? (float)conv_w[(long)c * dm.taps + j - pad] : 0.0f;
-      x[j] = (j >= pad && j < DR_MAXTAPS - 1 && !fresh) ? (float)cs[j - pad]
-                                                        : 0.0f;
+      f.w[j] = j >= pad ? conv_w[(long)c * dm.taps + j - pad] : (T)0.0f;
+      if (j < DR_MAXTAPS - 1) f.x[j] = j >= pad ? cs[j - pad] : (T)0.0f;
     }
+    f.first = y[(long)t0 * dm.ystride + col];
+  };
+  auto convolve = [&](const Conv& f, int i, int h0) {
+    int c, col;
+    channel(i, h0, c, col);
+    float x[DR_MAXTAPS];
+#pragma unroll
+    for (int j = 0; j < DR_MAXTAPS - 1; ++j) x[j] = fresh ? 0.0f : (float)f.x[j];
+    float* dst = qk + i;
+    int step = 2 * D;
+    if (i >= 2 * D) {
+      dst = vb + (long)(i - 2 * D) / V * n * V + (i - 2 * D) % V;
+      step = V;
+    }
+#pragma unroll 1
     for (int t = 0; t < n; ++t) {
-      x[DR_MAXTAPS - 1] = (float)y[(long)(t0 + t) * dm.ystride + col];
+      x[DR_MAXTAPS - 1] =
+          t ? (float)y[(long)(t0 + t) * dm.ystride + col] : (float)f.first;
       float a = 0.0f;
 #pragma unroll
-      for (int j = 0; j < DR_MAXTAPS; ++j) a += w[j] * x[j];
-      dst[(long)t * dstep] = silu_f(a);
+      for (int j = 0; j < DR_MAXTAPS; ++j) a += (float)f.w[j] * x[j];
+      dst[(long)t * step] = silu_f(a);
 #pragma unroll
       for (int j = 0; j < DR_MAXTAPS - 1; ++j) x[j] = x[j + 1];
     }
     // x[j] now holds the input one step older than slot j + 1: the last
     // taps - 1 inputs are x[pad .. MAXTAPS - 2]
+    T* cs = conv_state + (slot * C + c) * hist;
 #pragma unroll
     for (int j = 0; j < DR_MAXTAPS - 1; ++j)
       if (j >= pad) cs[j - pad] = (T)x[j];
   };
 
-  for (int i = tid; i < 2 * D; i += NT) {
-    const int which = i / D, d = i - which * D;
-    const int c = which * dm.KH * D + kh * D + d;
-    convolve(c, (which ? dm.kc : dm.qc) + kh * D + d, qk + i, 2 * D);
-  }
-  __syncthreads();
-  for (int r = wid; r < 2 * n; r += NT / WAVE) {
-    float* row = qk + (long)r * D;
-    float ss = 0.0f;
-    for (int d = lane; d < D; d += WAVE) ss += row[d] * row[d];
-    ss = wave_sum(ss);
-    const float s = (r & 1 ? 1.0f : q_scale) / sqrtf(ss + 1e-6f);
-    for (int d = lane; d < D; d += WAVE) row[d] *= s;
-  }
-  __syncthreads();
-  for (int t = wid; t < n; t += NT / WAVE) {
-    float a = 0.0f;
-    for (int d = lane; d < D; d += WAVE)
-      a += qk[(long)t * 2 * D + d] * qk[(long)t * 2 * D + D + d];
-    a = wave_sum(a);
-    if (lane == 0) kq[t] = a;
-  }
-
-  for (int hh = 0; hh < rep; ++hh) {
-    const int h = kh * rep + hh;
-    __syncthreads();
-    for (int i = tid; i < V; i += NT)
-      convolve(2 * dm.KH * D + h * V + i, dm.vc + h * V + i, vb + i, V);
-    const float Al = (float)A_log[h], dt = CH ? 0.0f : (float)dt_bias[h];
+  const int vc = min(v, V - 1);
+  const float nw = (float)norm_w[vc];
+  for (int hh = 0; hh < rep; hh += HP) {
+    const int h0 = kh * rep + hh;
+    const int heads = HP == 1 ? 1 : min(HP, rep - hh);
+    const int begin = hh ? 2 * D : 0, end = 2 * D + heads * V;
+    Conv first;
+    if (begin + tid < end) fetch(first, begin + tid, h0);
+    // of the first token: decay, write strength, output gate
+    T a_in[HP], b_in[HP], g_in[HP], Al[HP], dt[HP];
+    auto inputs = [&](int t) {
+      const T* yt = y + (long)(t0 + t) * dm.ystride;
+      const T* zt = z + (long)(t0 + t) * dm.zstride;
+#pragma unroll
+      for (int p = 0; p < HP; ++p) {
+        const int h = h0 + min(p, heads - 1);
+        a_in[p] = CH ? (T)0.0f : zt[dm.ac + h];
+        b_in[p] = yt[dm.bc + h];
+        g_in[p] = zt[dm.gc + h * V + vc];
+      }
+    };
+    inputs(0);
+#pragma unroll
+    for (int p = 0; p < HP; ++p) {
+      const int h = h0 + min(p, heads - 1);
+      Al[p] = A_log[h];
+      dt[p] = CH ? (T)0.0f : dt_bias[h];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int p = 0; p < HP; ++p) load_state(p, h0 + min(p, heads - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    if (hh) __syncthreads();  // the previous heads' values have been read
+    if (begin + tid < end) convolve(first, begin + tid, h0);
+#pragma unroll 1
+    for (int i = begin + tid + NT; i < end; i += NT) {
+      Conv f;
+      fetch(f, i, h0);
+      convolve(f, i, h0);
+    }
     if constexpr (CH) {
-      const float rate = expf(Al);
-      for (int i = tid; i < n * D; i += NT) {
-        const int t = i / D, d = i - t * D;
+#pragma unroll 1
+      for (int i = tid; i < heads * n * D; i += NT) {
+        const int p = i / (n * D), t = i / D - p * n, d = i % D, h = h0 + p;
         gd[i] = decay_of<T>((float)z[(t0 + t) * dm.zstride + dm.ac + h * D + d],
-                            rate, (float)dt_bias[h * D + d]);
+                            expf((float)A_log[h]), (float)dt_bias[h * D + d]);
       }
     }
     __syncthreads();
     for (int t = 0; t < n; ++t) {
-      const T* yt = y + (long)(t0 + t) * dm.ystride;
-      const T* zt = z + (long)(t0 + t) * dm.zstride;
-      const float g =
-          CH ? 1.0f : expf(log_decay((float)zt[dm.ac + h], Al, dt));
-      const float beta = sigmoid_f((float)yt[dm.bc + h]);
+      if (t) inputs(t);
       const float* qr = qk + (long)t * 2 * D;
       const float* kr = qr + D;
-      float sk = 0.0f, sq = 0.0f;
-#pragma unroll
-      for (int i = 0; i < RPT; ++i)
-        if (EXACT || d0 + i < D) {
-          if (CH) S[i] *= gd[t * D + d0 + i];
-          sk += S[i] * kr[d0 + i];
-          sq += S[i] * qr[d0 + i];
-        }
-      red[dg * VT + v] = sk;
-      red[NT + dg * VT + v] = sq;
-      __syncthreads();
-      sk = 0.0f;
-      sq = 0.0f;
-      for (int i = 0; i < DG; ++i) {
-        sk += red[i * VT + v];
-        sq += red[NT + i * VT + v];
+      float qq = 0.0f, kk = 0.0f, qd = 0.0f;
+      for (int d = lane; d < D; d += WAVE) {
+        const float a = qr[d], b = kr[d];
+        qq += a * a;
+        kk += b * b;
+        qd += a * b;
       }
-      const float vv = v < V ? vb[(long)t * V + v] : 0.0f;
-      const float u = beta * (vv - g * sk);
-      const float o = g * sq + kq[t] * u;
+      const float fq = q_scale / sqrtf(wave_sum(qq) + 1e-6f);
+      const float fk = 1.0f / sqrtf(wave_sum(kk) + 1e-6f);
+      const float kq = wave_sum(qd) * fq * fk;
+      float sk[HP], sq[HP];
 #pragma unroll
-      for (int i = 0; i < RPT; ++i)
-        if (EXACT || d0 + i < D) S[i] = g * S[i] + kr[d0 + i] * u;
-      const bool mine = dg == 0 && v < V;
-      const float ss = block_sum<NT>(mine ? o * o : 0.0f, scratch);
-      if (mine) {
-        const float gate = out_gate((float)zt[dm.gc + h * V + v], dm.sigmoid);
-        out[(long)(t0 + t) * ((long)dm.H * V) + h * V + v] =
-            (T)(o / sqrtf(ss / (float)V + eps) * (float)norm_w[v] * gate);
-      }
-    }
-    float* sp = state + ((slot * dm.H + h) * (long)D) * V;
-    if (EXACT || v < V) {
+      for (int p = 0; p < HP; ++p) sk[p] = sq[p] = 0.0f;
 #pragma unroll
       for (int i = 0; i < RPT; ++i) {
-        if (EXACT || d0 + i < D) sp[d0 * V + v] = S[i];
-        sp += V;
+        if (EXACT || d0 + i < D) {
+          const float a = qr[d0 + i], b = kr[d0 + i];
+#pragma unroll
+          for (int p = 0; p < HP; ++p) {
+            if (CH) S[p][i] *= gd[(min(p, heads - 1) * n + t) * D + d0 + i];
+            sk[p] += S[p][i] * b;
+            sq[p] += S[p][i] * a;
+          }
+        }
+      }
+#pragma unroll
+      for (int p = 0; p < HP; ++p) {
+        red[p * 2 * NT + dg * VT + v] = sk[p];
+        red[p * 2 * NT + NT + dg * VT + v] = sq[p];
+      }
+      __syncthreads();
+      const bool mine = dg == 0 && v < V;
+      float g[HP], u[HP], o[HP];
+#pragma unroll
+      for (int p = 0; p < HP; ++p) {
+        float a = 0.0f, b = 0.0f;
+        for (int i = 0; i < DG; ++i) {
+          a += red[p * 2 * NT + i * VT + v];
+          b += red[p * 2 * NT + NT + i * VT + v];
+        }
+        g[p] = CH ? 1.0f : expf(log_decay((float)a_in[p], (float)Al[p], (float)dt[p]));
+        const float beta = sigmoid_f((float)b_in[p]);
+        const float vv =
+            v < V ? vb[((long)min(p, heads - 1) * n + t) * V + v] : 0.0f;
+        u[p] = beta * (vv - g[p] * a * fk);
+        o[p] = g[p] * b * fq + kq * u[p];
+        const float ss = wave_sum(mine ? o[p] * o[p] : 0.0f);
+        if (lane == 0) scratch[p * (NT / WAVE) + wid] = ss;
+      }
+#pragma unroll
+      for (int i = 0; i < RPT; ++i) {
+        if (EXACT || d0 + i < D) {
+          const float b = kr[d0 + i] * fk;
+#pragma unroll
+          for (int p = 0; p < HP; ++p) S[p][i] = g[p] * S[p][i] + b * u[p];
+        }
+      }
+      __syncthreads();
+      if (mine) {
+#pragma unroll
+        for (int p = 0; p < HP; ++p) {
+          if (p >= heads) break;
+          float ss = 0.0f;
+#pragma unroll
+          for (int w = 0; w < NT / WAVE; ++w) ss += scratch[p * (NT / WAVE) + w];
+          const float gate = out_gate((float)g_in[p], dm.sigmoid);
+          out[(long)(t0 + t) * ((long)dm.H * V) + (h0 + p) * V + v] =
+              (T)(o[p] / sqrtf(ss / (float)V + eps) * nw * gate);
+        }
       }
     }
-    if (hh + 1 < rep) load_state(h + 1);
+#pragma unroll
+    for (int p = 0; p < HP; ++p) {
+      if (p >= heads) break;
+      // a base of its own: the addresses of the loads are not kept till here
+      int head = (int)slot * dm.H + h0 + p;
+      asm volatile("" : "+v"(head));
+      float* sp = state + (long)__builtin_amdgcn_readfirstlane(head) * D * V;
+      if (EXACT || v < V) {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+          if (EXACT || d0 + i < D) sp[(unsigned)(d0 * V + v)] = S[p][i];
+          sp += V;
+        }
+      }
+    }
   }
 }
 
@@ -267,37 +360,52 @@ static void delta_short_t(const void* y, const void* z, const void* conv_w,
                           int max_len, float eps, hipStream_t stream) {
   const int vt = pow2_at_least(dm.V);
   const int rpt = delta_short_rows(dm.D, dm.V, DR_NT);
-  const size_t smem = ((size_t)max_len * ((CH ? 3 : 2) * dm.D + dm.V) +
-                       DR_SHORT + 2 * DR_NT + DR_NT / WAVE) * sizeof(float);
   const float q_scale = 1.0f / sqrtf((float)dm.D);
   dim3 grid((unsigned)n_req, (unsigned)dm.KH), block(DR_NT);
-#define DS_ONE(R, X)                                                         \
+  auto bytes = [&](int hp) {
+    return ((size_t)max_len * (2 * dm.D + hp * ((CH ? dm.D : 0) + dm.V)) +
+            hp * (2 * DR_NT + DR_NT / WAVE)) * sizeof(float);
+  };
+  // two heads at a time where there are two and what they need fits the registers
+  // and a quarter of LDS
+  const bool exact = dm.V == vt && dm.D == rpt * (DR_NT / vt);
+  const bool pairs = dm.H > dm.KH && exact && rpt <= 32 && bytes(2) <= 40960;
+  const size_t smem = bytes(pairs ? 2 : 1);
+#define DS_ONE(R, X, P)                                                      \
   do {                                                                       \
     if (smem > 65536)                                                        \
       (void)hipFuncSetAttribute(                                             \
           reinterpret_cast<const void*>(                                     \
-              &delta_short_kernel<T, R, DR_NT, X, CH>),                      \
+              &delta_short_kernel<T, R, DR_NT, X, CH, P>),                   \
           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);            \
-    delta_short_kernel<T, R, DR_NT, X, CH><<<grid, block, smem, stream>>>(   \
+    delta_short_kernel<T, R, DR_NT, X, CH, P><<<grid, block, smem, stream>>>(\
         (const T*)y, (const T*)z, (const T*)conv_w, (const T*)A_log,         \
         (const T*)dt_bias, (const T*)norm_w, state, (T*)conv_state, (T*)out, \
         cu, pos0, slots, dm, vt, q_scale, eps);                              \
   } while (0)
-#define DS_GO(R)                                                             \
+#define DS_GO(R, P)                                                          \
   do {                                                                       \
-    if (dm.V == vt && dm.D == R * (DR_NT / vt))                              \
-      DS_ONE(R, true);                                                       \
+    if (exact)                                                               \
+      DS_ONE(R, true, P);                                                    \
     else                                                                     \
-      DS_ONE(R, false);                                                      \
+      DS_ONE(R, false, P);                                                   \
+  } while (0)
+#define DS_PAIR(R)                                                           \
+  do {                                                                       \
+    if (pairs)                                                               \
+      DS_ONE(R, true, 2);                                                    \
+    else                                                                     \
+      DS_GO(R, 1);                                                           \
   } while (0)
   switch (rpt) {
-    case 4: DS_GO(4); break;
-    case 16: DS_GO(16); break;
-    case 32: DS_GO(32); break;
-    case 64: DS_GO(64); break;
-    case 128: DS_GO(128); break;
+    case 4: DS_PAIR(4); break;
+    case 16: DS_PAIR(16); break;
+    case 32: DS_PAIR(32); break;
+    case 64: DS_GO(64, 1); break;
+    case 128: DS_GO(128, 1); break;
     default: break;
   }
+#undef DS_PAIR
 #undef DS_GO
 #undef DS_ONE
 }
