@@ -22,9 +22,12 @@
 // (on their way from memory, the place in LDS is fixed), without which the rows
 // that a read meets share their banks.
 // Measured (before: 16 queries a wave, scores through LDS, V transposed element by
-// element): 8192 tokens, 32 heads of 128 over 8: 5310 -> 656 us (839 TFLOP/s);
-// 4096 tokens, 16 heads of 256 over 8, capped: 1600 -> 402 us (342); 64 prompts of
-// 512, 16 heads of 192/128: 1216 -> 174 us (496); 57 tokens: 8.4 -> 7.6 us.
+// element): 8192 tokens, 32 heads of 128 over 8: 5310 -> 601 us (914 TFLOP/s);
+// 4096 tokens, 16 heads of 256 over 8, capped: 1600 -> 242 us (567), 1905 behind 4096
+// with a window of 4096: 213 us (402 and 457 while places in LDS had a register each
+// and were spilled: each reload waited for the next tile's loads; 255 and 228 with all
+// of a query in registers); 64 prompts of 512, 16 heads of 192/128: 1216 -> 176 us
+// (490); 57 tokens: 8.4 -> 7.6 us.
 
 #include "hip_common.h"
 
@@ -94,7 +97,11 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
   constexpr int NK = DK / 16, NB = KT / 32, ND = (DV + 31) / 32;
   constexpr int KB = KT * DK * 2, VB = KT * DV * 2;
   // a lane of the columns behind DV = 16 reads past its row
+  // The last pieces of queries of 256 lie there, too: they and the sums leave too few
+  // registers to read keys and values ahead of their products.
+  constexpr int QL = DK == 256 ? 4 : 0;
   __shared__ __attribute__((aligned(16))) char smem[2 * (KB + VB) +
+                                                    AP_WAVES * QL * 1024 +
                                                     (DV < 32 ? 64 : 0)];
 
   // Blocks go round the XCDs.  Each XCD takes whole heads, `group` of them at a
@@ -164,6 +171,7 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
   const int qpos = min(a.offset + row, a.S - 1);       // last key seen
   const int qfrom = a.window > 0 ? a.offset + row - a.window + 1 : 0;
   bf16x8_t qf[NK];
+  char* ql = smem + 2 * (KB + VB) + (wid * QL * WAVE + lane) * 16;
   {
     const char* src =
         a.q + ((long)b * a.q_b + (long)h * a.q_h + (long)row * a.q_t) * 2 + hi * 16;
@@ -192,6 +200,9 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
         for (int j = 0; j < 8; ++j) qf[i][j] = -qf[i][j];
     }
   }
+#pragma unroll
+  for (int i = 0; i < QL; ++i)
+    *reinterpret_cast<bf16x8_t*>(ql + i * 1024) = qf[NK - QL + i];
   // keys that all of the wave's queries see, and those that any of them sees
   const int all_hi = min(a.offset + min(w0, a.T - 1), a.S - 1);
   const int any_hi = w0 < a.T ? min(a.offset + min(w0 + 31, a.T - 1), a.S - 1) : -1;
@@ -208,6 +219,16 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
   const int krow = l32 * KP * 16;
   const int i16 = lane & 15;
   const int vkey = hi * 4 + (i16 >> 2);
+  // Swapping moves a piece within 8 of keys, 16 of values: four places, the others lie
+  // behind them.
+  int kplace[NK < 4 ? NK : 4], vplace[ND < 4 ? ND : 4];
+#pragma unroll
+  for (int i = 0; i < (NK < 4 ? NK : 4); ++i)
+    kplace[i] = krow + key_place<KP>(l32, 2 * i + hi) * 16;
+#pragma unroll
+  for (int d = 0; d < (ND < 4 ? ND : 4); ++d)
+    vplace[d] = vkey * VP * 16 + (i16 & 1) * 8 +
+                value_place<VP>(vkey, d * 4 + (lane >> 4 & 1) * 2 + (i16 >> 1 & 1)) * 16;
   int buf = 0;
   for (int t = from; t < end; t += KT, buf ^= 1) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -227,8 +248,10 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
 #pragma unroll
       for (int n = 0; n < NB; ++n) {
         const bf16x8_t f = *reinterpret_cast<const bf16x8_t*>(
-            kt + n * 32 * KP * 16 + krow + key_place<KP>(l32, 2 * i + hi) * 16);
-        s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, qf[i], s[n], 0, 0, 0);
+            kt + n * 32 * KP * 16 + i / 4 * 128 + kplace[i % 4]);
+        const bf16x8_t q = i < NK - QL ? qf[i] : *reinterpret_cast<const bf16x8_t*>(
+                                                     ql + (i - NK + QL) * 1024);
+        s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, q, s[n], 0, 0, 0);
       }
     if (CAP) {
 #pragma unroll
@@ -282,9 +305,7 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
       for (int j = 0; j < 8; ++j) p[j] = (__bf16)s[x / 2][x % 2 * 8 + j];
 #pragma unroll
       for (int d = 0; d < ND; ++d) {
-        const int piece = value_place<VP>(
-            vkey, d * 4 + (lane >> 4 & 1) * 2 + (i16 >> 1 & 1));
-        const char* src = vt + (x * 16 + vkey) * VP * 16 + piece * 16 + (i16 & 1) * 8;
+        const char* src = vt + x * 16 * VP * 16 + d / 4 * 256 + vplace[d % 4];
         const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (__attribute__((address_space(3))) s16x4*)src);
         const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
