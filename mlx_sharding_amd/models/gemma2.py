@@ -118,15 +118,16 @@ class Gemma2DecoderLayer(nn.Module):
         self.post_feedforward_layernorm = RMSNorm(H, eps, weight_offset=1.0)
 
     def forward(self, x, cos, sin, cache):
+        post, pre = self.post_attention_layernorm, self.pre_feedforward_layernorm
         if ops.few_tokens(x):
-            h = x + self.post_attention_layernorm(
-                self.self_attn(x, cos, sin, cache, self.input_layernorm))
-            return h + self.post_feedforward_layernorm(
-                self.mlp(h, self.pre_feedforward_layernorm))
-        h = x + self.post_attention_layernorm(
-            self.self_attn(self.input_layernorm(x), cos, sin, cache))
-        return h + self.post_feedforward_layernorm(
-            self.mlp(self.pre_feedforward_layernorm(h)))
+            h = ops.norm_add(self.self_attn(x, cos, sin, cache, self.input_layernorm),
+                             post, x)
+            y = self.mlp(h, pre)
+        else:
+            h, y = ops.norm_add(
+                self.self_attn(self.input_layernorm(x), cos, sin, cache), post, x, pre)
+            y = self.mlp(y)
+        return ops.norm_add(y, self.post_feedforward_layernorm, h)
 
 
 class Gemma2StageModel(StageModel):

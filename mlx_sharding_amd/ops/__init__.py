@@ -94,6 +94,26 @@ def rms_norm_residual(x, residual, weight, eps: float = 1e-5, weight_offset: flo
     return ref.rms_norm(h, weight, eps, weight_offset), h
 
 
+def norm_add(x, norm, residual, then=None):
+    """h = residual + norm(x); with ``then``, another norm, (h, then(h)).  One kernel
+    on the GPU for bf16 rows of whole 16-byte vectors, up to 8192 columns."""
+    H = x.shape[-1]
+    norms = (norm,) if then is None else (norm, then)
+    if (x.dtype == residual.dtype == torch.bfloat16 and use_native(x)
+            and x.shape == residual.shape and x.numel() and H % 8 == 0 and H <= 8192
+            and all(_plain(t) and t.is_contiguous() and t.dtype == torch.bfloat16
+                    and t.data_ptr() % 16 == 0
+                    for t in (x, residual, *(n.weight for n in norms)))):
+        out = hip_ext().norm_add(
+            x, norm.weight, norm.eps, norm.weight_offset, residual,
+            None if then is None else then.weight,
+            0.0 if then is None else then.eps,
+            0.0 if then is None else then.weight_offset)
+        return out[0] if then is None else out
+    h = residual + norm(x)
+    return h if then is None else (h, then(h))
+
+
 def apply_rope(x, cos, sin, interleaved: bool = False):
     if _use_hip(x):
         return _require_ext("apply_rope").apply_rope(

@@ -17,6 +17,8 @@ void launch_rms_norm(const void*, void*, const void*, long, int, float, float,
 void launch_rms_norm_residual(const void*, const void*, void*, void*,
                               const void*, long, int, float, float,
                               hipStream_t);
+void launch_norm_add(const void*, const void*, const void*, const void*, void*, void*,
+                     long, int, float, float, float, float, hipStream_t);
 void launch_glu(const void*, const void*, void*, long, bool, hipStream_t);
 void launch_glu_strided(const void*, const void*, void*, long, int, long,
                         long, bool, hipStream_t);
@@ -168,6 +170,32 @@ std::vector<torch::Tensor> rms_norm_residual(torch::Tensor x,
                            h.data_ptr(), w.contiguous().data_ptr(), rows, H,
                            (float)eps, (float)w_off, cur_stream());
   return {y, h};
+}
+
+// (residual + norm(x), with a next norm's weight its rows of that)
+std::vector<torch::Tensor> norm_add(torch::Tensor x, torch::Tensor w, double eps,
+                                    double off, torch::Tensor resid,
+                                    c10::optional<torch::Tensor> w2, double eps2,
+                                    double off2) {
+  const long H = x.dim() ? x.size(-1) : 0;
+  TORCH_CHECK(H >= 8 && H <= 8192 && H % 8 == 0 && x.numel() >= H, "row size");
+  auto ok = [](const torch::Tensor& t, long n) {
+    check_bf16(t, "operand");
+    TORCH_CHECK(t.is_contiguous() && t.numel() == n &&
+                    reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "layout");
+  };
+  ok(x, x.numel());
+  ok(resid, x.numel());
+  ok(w, H);
+  if (w2.has_value()) ok(*w2, H);
+  auto h = torch::empty_like(x);
+  std::vector<torch::Tensor> out{h};
+  if (w2.has_value()) out.push_back(torch::empty_like(x));
+  launch_norm_add(x.data_ptr(), resid.data_ptr(), w.data_ptr(),
+                  w2.has_value() ? w2->data_ptr() : nullptr, h.data_ptr(),
+                  out.back().data_ptr(), x.numel() / H, (int)H, (float)eps,
+                  (float)off, (float)eps2, (float)off2, cur_stream());
+  return out;
 }
 
 torch::Tensor glu(torch::Tensor gate, torch::Tensor up, bool gelu) {
@@ -1093,6 +1121,7 @@ std::vector<torch::Tensor> moe_gate_subranges(torch::Tensor logits, int64_t K,
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "fused RMSNorm (gfx950)");
+  m.def("norm_add", &norm_add);
   m.def("rms_norm_residual", &rms_norm_residual);
   m.def("glu", &glu);
   m.def("softcap", &softcap_op);
