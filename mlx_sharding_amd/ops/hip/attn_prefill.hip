@@ -58,6 +58,11 @@ struct PrefillArgs {
   long pe_b;                 // bytes from one sequence to the next
   int kv_row, pe_row;        // bytes from one key to the next
   const float *cos, *sin;    // [T, (DK - NOPE) / 2]
+  // portions of a batch, rows of queries and of keys one behind the other; keys'
+  // first columns and values in rows of their own, queries have been turned
+  const int *portions;       // [tiles, 2]: request, first row
+  const int *cu, *pos0, *cuk;
+  int n_short, tok_base, v_row;
 };
 
 // 16 bytes a lane from memory to LDS, lane after lane from `dst` on
@@ -88,8 +93,10 @@ __device__ __forceinline__ int value_place(int row, int piece) {
   return piece;
 }
 
-// NOPE: columns of a key that lie with the values, 0: rows of keys and of values
-template <int DK, int DV, bool CAP, int NOPE = 0>
+// NOPE: columns of a key that lie with the values, 0: rows of keys and of values.
+// RAGGED: portions of a batch; weights enter the second product in two bf16 parts, as
+// they do in that cache's other kernels.
+template <int DK, int DV, bool CAP, int NOPE = 0, bool RAGGED = false>
 __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
     const PrefillArgs a) {
   constexpr int KT = DK + DV > 320 ? 32 : 64;  // keys of a tile
@@ -118,12 +125,26 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
   }
   const int b = head / a.Hq, h = head % a.Hq;
   const long kv = (long)b * a.Hkv + h / (a.Hq / a.Hkv);
-  const int q0 = tile * (AP_WAVES * 32);
+  int q0 = tile * (AP_WAVES * 32), T = a.T, S = a.S, offset = a.offset;
+  long t0 = 0, k0 = 0;
+  if (RAGGED) {
+    const int e = a.portions[2 * tile];
+    q0 = a.portions[2 * tile + 1];
+    t0 = a.cu[e];
+    T = a.cu[e + 1] - (int)t0;
+    offset = a.pos0[e];
+    S = offset + T;
+    k0 = a.cuk[e - a.n_short];
+  }
   const int lane = threadIdx.x & (WAVE - 1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l32 = lane & 31, hi = lane >> 5;
   const char *kbase, *vbase, *pbase = nullptr;
-  if (NOPE) {
+  if (RAGGED) {
+    kbase = a.k + k0 * a.kv_row + (long)h * NOPE * 2;
+    vbase = a.v + k0 * a.v_row + (long)h * DV * 2;
+    pbase = a.pe + k0 * a.pe_row;
+  } else if (NOPE) {
     kbase = a.k + (long)b * a.S * a.kv_row + (long)h * (NOPE + DV) * 2;
     vbase = kbase + NOPE * 2;
     pbase = a.pe + (long)b * a.pe_b;
@@ -131,7 +152,7 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
     kbase = a.k + kv * a.kcap * (DK * 2);
     vbase = a.v + kv * a.vcap * (DV * 2);
   }
-  const int krow_w = NOPE ? a.kv_row : DK * 2, vrow_w = NOPE ? a.kv_row : DV * 2;
+  const int krow_w = NOPE ? a.kv_row : DK * 2, vrow_w = RAGGED ? a.v_row : NOPE ? a.kv_row : DV * 2;
 
   // rows behind the last key repeat it; their weights are zero
   auto stage = [&](int t, int buf) {
@@ -139,7 +160,7 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
     const char* ks = kbase + (long)t * krow_w;
     const char* vs = vbase + (long)t * vrow_w;
     const char* ps = NOPE ? pbase + (long)t * a.pe_row : nullptr;
-    const int last = a.S - 1 - t;
+    const int last = S - 1 - t;
 #pragma unroll
     for (int i = 0; i < KB / 1024; i += AP_WAVES) {
       const int part = i + wid;
@@ -161,24 +182,24 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
     }
   };
 
-  const int end = min(a.S, a.offset + min(q0 + AP_WAVES * 32, a.T));
+  const int end = min(S, offset + min(q0 + AP_WAVES * 32, T));
   int from = 0;
-  if (a.window > 0) from = max(0, a.offset + q0 - a.window + 1) & ~(KT - 1);
+  if (a.window > 0) from = max(0, offset + q0 - a.window + 1) & ~(KT - 1);
   if (from < end) stage(from, 0);
 
   const int w0 = q0 + wid * 32;  // this wave's first query
-  const int row = min(w0 + l32, a.T - 1);
-  const int qpos = min(a.offset + row, a.S - 1);       // last key seen
-  const int qfrom = a.window > 0 ? a.offset + row - a.window + 1 : 0;
+  const int row = min(w0 + l32, T - 1);
+  const int qpos = min(offset + row, S - 1);       // last key seen
+  const int qfrom = a.window > 0 ? offset + row - a.window + 1 : 0;
   bf16x8_t qf[NK];
   char* ql = smem + 2 * (KB + VB) + (wid * QL * WAVE + lane) * 16;
   {
     const char* src =
-        a.q + ((long)b * a.q_b + (long)h * a.q_h + (long)row * a.q_t) * 2 + hi * 16;
+        a.q + ((long)b * a.q_b + (long)h * a.q_h + (t0 + row) * a.q_t) * 2 + hi * 16;
 #pragma unroll
     for (int i = 0; i < NK; ++i)
       qf[i] = *reinterpret_cast<const bf16x8_t*>(src + i * 32);
-    if (NOPE) {
+    if (NOPE && !RAGGED) {
       // as rounded rows of queries would be
 #pragma unroll
       for (int i = NOPE / 16; i < NK; ++i) {
@@ -204,10 +225,10 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
   for (int i = 0; i < QL; ++i)
     *reinterpret_cast<bf16x8_t*>(ql + i * 1024) = qf[NK - QL + i];
   // keys that all of the wave's queries see, and those that any of them sees
-  const int all_hi = min(a.offset + min(w0, a.T - 1), a.S - 1);
-  const int any_hi = w0 < a.T ? min(a.offset + min(w0 + 31, a.T - 1), a.S - 1) : -1;
-  const int all_lo = a.window > 0 ? a.offset + min(w0 + 31, a.T - 1) - a.window + 1 : 0;
-  const int any_lo = a.window > 0 ? a.offset + w0 - a.window + 1 : 0;
+  const int all_hi = min(offset + min(w0, T - 1), S - 1);
+  const int any_hi = w0 < T ? min(offset + min(w0 + 31, T - 1), S - 1) : -1;
+  const int all_lo = a.window > 0 ? offset + min(w0 + 31, T - 1) - a.window + 1 : 0;
+  const int any_lo = a.window > 0 ? offset + w0 - a.window + 1 : 0;
 
   float m = -1e30f, l = 0.0f;  // reference of the exponents (base 2), sum
   f32x16 o[ND];
@@ -300,9 +321,13 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
     l += sum;
 #pragma unroll
     for (int x = 0; x < KT / 16; ++x) {
-      bf16x8_t p;
+      bf16x8_t p, rest;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) p[j] = (__bf16)s[x / 2][x % 2 * 8 + j];
+      for (int j = 0; j < 8; ++j) {
+        const float w = s[x / 2][x % 2 * 8 + j];
+        p[j] = (__bf16)w;
+        if (RAGGED) rest[j] = (__bf16)(w - (float)p[j]);
+      }
 #pragma unroll
       for (int d = 0; d < ND; ++d) {
         const char* src = vt + x * 16 * VP * 16 + d / 4 * 256 + vplace[d % 4];
@@ -313,15 +338,19 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
         const short8v v = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
             __builtin_bit_cast(bf16x8_t, v), p, o[d], 0, 0, 0);
+        if (RAGGED)
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(bf16x8_t, v), rest, o[d], 0, 0, 0);
       }
     }
   }
 
   l += __shfl_xor(l, 32, WAVE);
-  if (w0 + l32 >= a.T) return;
+  if (w0 + l32 >= T) return;
   const float f = 1.0f / l;
   // out [B, T, Hq, DV]
-  char* dst = a.out + ((((long)b * a.T + w0 + l32) * a.Hq + h) * DV + hi * 4) * 2;
+  const long at = RAGGED ? t0 - a.tok_base : (long)b * T;
+  char* dst = a.out + (((at + w0 + l32) * a.Hq + h) * DV + hi * 4) * 2;
 #pragma unroll
   for (int d = 0; d < ND; ++d)
 #pragma unroll
@@ -419,6 +448,33 @@ extern "C" void launch_mla_prompt(const void* q, const void* kv, const void* cac
   a.sin = sin;
   prefill_setup(a, B, scale, 0.0f, 0, causal_offset);
   attn_prefill_kernel<192, 128, false, 128>
+      <<<dim3((unsigned)a.heads * a.tiles), dim3(AP_BLOCK), 0, stream>>>(a);
+}
+
+// The same for portions of a batch: q rows [dq = 192], turned; k [keys, H * 128], v
+// [keys, H * 128], rows [keys, width], whose last 64 columns are the rotated key part;
+// out [tokens, H * 128].  2 x 4001 tokens of 16 heads: 275 us, 604 in the general kernel
+// (16x16x32 products, tiles through registers, nothing on its way meanwhile).
+extern "C" void launch_latent_prompt(const void* q, const void* k, const void* v,
+                                     const void* rows, void* out,
+                                     const int* portions, const int* cu,
+                                     const int* pos0, const int* cuk, int n_short,
+                                     int tok_base, int n_tiles, int H, long q_t,
+                                     int width, float scale, hipStream_t stream) {
+  PrefillArgs a{(const char*)q, (const char*)k, (const char*)v, (char*)out,
+                H, H, 1, 1, 0, 192, q_t};
+  a.pe = (const char*)rows + (width - 64) * 2;
+  a.pe_row = width * 2;
+  a.kv_row = a.v_row = H * 128 * 2;
+  a.portions = portions;
+  a.cu = cu;
+  a.pos0 = pos0;
+  a.cuk = cuk;
+  a.n_short = n_short;
+  a.tok_base = tok_base;
+  prefill_setup(a, 1, scale, 0.0f, 0, 0);
+  a.tiles = n_tiles;
+  attn_prefill_kernel<192, 128, false, 128, true>
       <<<dim3((unsigned)a.heads * a.tiles), dim3(AP_BLOCK), 0, stream>>>(a);
 }
 

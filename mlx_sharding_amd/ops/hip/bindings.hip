@@ -45,6 +45,9 @@ void launch_attn_prefill(const void*, const void*, const void*, void*, int,
                          int, int, int, int, long, long, long, long, long, int,
                          int, float, float, int, int, hipStream_t);
 bool attn_prefill_supported(int, int);
+void launch_latent_prompt(const void*, const void*, const void*, const void*, void*,
+                          const int*, const int*, const int*, const int*, int, int, int,
+                          int, long, int, float, hipStream_t);
 void launch_mla_prompt(const void*, const void*, const void*, const float*,
                        const float*, void*, int, int, int, int, long, long, long, long,
                        int, float, int, hipStream_t);
@@ -570,6 +573,42 @@ torch::Tensor mla_prompt(torch::Tensor q, torch::Tensor kv, torch::Tensor cache,
                     (int)B, (int)H, (int)T, (int)S, q.stride(0), q.stride(2),
                     q.stride(1), cache.size(2), (int)cache.size(3), (float)scale,
                     (int)causal_offset, cur_stream());
+  return out;
+}
+
+// Attention of the long portions of a batch: q [tokens, >= H * 192], turned; k, v
+// [keys, H * 128]; rows [keys, width], whose last 64 columns are the rotated key part.
+// portions [n, 2] of 128 rows: request, first row.  Returns [tokens - tok_base, H * 128].
+torch::Tensor latent_prompt(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                            torch::Tensor rows, torch::Tensor portions,
+                            torch::Tensor cu, torch::Tensor pos0, torch::Tensor cuk,
+                            int64_t n_short, int64_t tok_base, int64_t H,
+                            double scale) {
+  for (const auto& t : {q, k, v, rows}) {
+    check_bf16(t, "operand");
+    TORCH_CHECK(t.dim() == 2 && t.stride(1) == 1 &&
+                    reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "layout");
+  }
+  const long keys = k.size(0);
+  TORCH_CHECK(H >= 1 && H <= 8192 && q.size(1) >= H * 192 && q.stride(0) % 8 == 0 &&
+                  tok_base >= 0 && tok_base < q.size(0), "queries");
+  TORCH_CHECK(k.size(1) == H * 128 && v.size(0) == keys && v.size(1) == H * 128 &&
+                  rows.size(0) == keys && rows.size(1) >= 64 &&
+                  rows.size(1) % 8 == 0 && k.is_contiguous() && v.is_contiguous() &&
+                  rows.is_contiguous(), "keys");
+  auto ints = [](const torch::Tensor& t, long n) {
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kInt32 && t.is_contiguous() &&
+                    t.numel() >= n, "int32 indices");
+    return t.data_ptr<int>();
+  };
+  TORCH_CHECK(portions.dim() == 2 && portions.size(1) == 2 && portions.size(0) >= 1,
+              "portions");
+  auto out = torch::empty({q.size(0) - tok_base, H * 128}, q.options());
+  launch_latent_prompt(q.data_ptr(), k.data_ptr(), v.data_ptr(), rows.data_ptr(),
+                       out.data_ptr(), ints(portions, 2), ints(cu, n_short + 2),
+                       ints(pos0, n_short + 1), ints(cuk, 2), (int)n_short,
+                       (int)tok_base, (int)portions.size(0), (int)H, q.stride(0),
+                       (int)rows.size(1), (float)scale, cur_stream());
   return out;
 }
 
@@ -1150,6 +1189,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_few_try", &linear_few_try);
   m.def("mla_rows", &mla_rows);
   m.def("mla_prompt", &mla_prompt);
+  m.def("latent_prompt", &latent_prompt);
   m.def("mla_prepare", &mla_prepare);
   m.def("mla_attend", &mla_attend);
   m.def("attn_decode_tile", [](int64_t g, int64_t dk, int64_t dv, bool inrow) {

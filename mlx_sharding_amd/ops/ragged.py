@@ -258,6 +258,15 @@ def _gather_rows(store: LayerStore, held, n: int) -> torch.Tensor:
     return store.rows[idx]
 
 
+def _prompt_ext(q, sh: LatentShape):
+    """The other extension where its attn_prefill.hip has a kernel for these heads."""
+    if (q.dtype == torch.bfloat16 and (sh.dimp, sh.rotp, sh.vdp) == (128, 64, 128)
+            and q.stride(0) % 8 == 0 and q.stride(1) == 1 and q.data_ptr() % 16 == 0):
+        from . import hip_ext
+        return hip_ext()
+    return None
+
+
 def latent_attention_expanded(q, store: LayerStore, w_uk, w_uv, sh: LatentShape,
                               scale: float, batch: RaggedBatch):
     """Attention of the long portions: keys and values of their whole prefix
@@ -268,6 +277,11 @@ def latent_attention_expanded(q, store: LayerStore, w_uk, w_uv, sh: LatentShape,
         lat = ext.latent_gather(store.rows, batch.blocks, batch.key_rows)
         c = lat[:, : sh.rankp]
         kx = F.linear(c, w_uk)
+        prompt = _prompt_ext(q, sh)
+        if prompt is not None:
+            return prompt.latent_prompt(
+                q, kx, F.linear(c, w_uv), lat, batch.tiles, batch.cu, batch.pos0,
+                batch.cuk, batch.n_short, batch.short_tokens, sh.heads, scale)
         vt = F.linear(w_uv, c)  # already transposed: [heads * vdp, keys]
         return ext.latent_attn_long(
             q, kx, lat, vt, batch.tiles, batch.cu, batch.pos0, batch.cuk,
