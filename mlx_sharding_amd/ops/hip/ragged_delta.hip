@@ -629,35 +629,70 @@ __global__ __launch_bounds__(DC_BLOCK) void delta_conv_state_kernel(
 
 // ---------------------------------------------------------------------------
 // Step 2, all chunks at once.  Block = (chunk, head), 4 waves; wave w makes
-// rows 16w..16w+15 of the two Gram matrices, wave 0 then inverts I + L, one
-// column per lane.
-//   tm [chunks, H, 64, 64]  (I + L)^-1 diag(beta)
+// rows 16w..16w+15 of the two Gram matrices and column tile w of the inverse.
+//   tm [chunks, H, 64, 64]  (I + L)^-1 diag(beta) (lower tiles only)
 //   am [chunks, H, 64, 64]  A (lower tiles only)
 //   ge [chunks, H, 2, 64]   exp(G), exp(G_last - G)
 // ---------------------------------------------------------------------------
 
 #define DR_LS 68
 
-// (I + L)^-1 times `by`, one column per lane; ls: L, rows of DR_LS
-__device__ __forceinline__ void invert_unit(const float* ls, float by, float* tm,
-                                            int lane) {
-  float x[DR_CHUNK];
+// Lower tiles of (I + L)^-1 diag(by), by four waves; ls: L, rows of DR_LS, whose
+// tiles on the diagonal are overwritten.  A wave inverts one of these by forward
+// substitution, a column per lane, and then makes the tiles below it from products,
+// X_ij = -X_ii sum_k L_ik X_kj: a product's result lies as the next one's operand.
+// One wave for all 64 rows left three idle through a chain four times as long: the
+// matrices of 126 chunks, 32 heads 167 -> 138 us, with decays per channel (a mixed
+// batch of 16 heads) 58 -> 46.
+__device__ __forceinline__ void invert_tiles(float* ls, const float* by, float* tm,
+                                             int wid, int lane) {
+  const int lr = lane & 15, g4 = lane >> 4;
+  float* own = ls + wid * 16 * DR_LS + wid * 16;
+  float x[16];
 #pragma unroll
-  for (int i = 0; i < DR_CHUNK; ++i) {
-    float a0 = i == lane ? 1.0f : 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
-    const float* row = ls + i * DR_LS;
+  for (int i = 0; i < 16; ++i) {
+    float a0 = i == lr ? 1.0f : 0.0f, a1 = 0.0f;
+    const float* row = own + i * DR_LS;
 #pragma unroll
-    for (int j = 0; j + 4 <= i; j += 4) {
-      const f32x4 l4 = load4(row + j);
-      a0 -= l4[0] * x[j];
-      a1 -= l4[1] * x[j + 1];
-      a2 -= l4[2] * x[j + 2];
-      a3 -= l4[3] * x[j + 3];
+    for (int j = 0; j + 2 <= i; j += 2) {
+      a0 -= row[j] * x[j];
+      a1 -= row[j + 1] * x[j + 1];
     }
+    if (i & 1) a0 -= row[i - 1] * x[i - 1];
+    x[i] = a0 + a1;
+  }
+  f32x4 d;
 #pragma unroll
-    for (int j = i & ~3; j < i; ++j) a0 -= row[j] * x[j];
-    x[i] = (a0 + a1) + (a2 + a3);
-    tm[i * 64 + lane] = x[i] * by;
+  for (int r = 0; r < 4; ++r)
+    d[r] = g4 < 2 ? (g4 ? x[4 + r] : x[r]) : (g4 == 2 ? x[8 + r] : x[12 + r]);
+  const float b = by[wid * 16 + lr];
+  auto put = [&](int i, const f32x4& v) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      tm[(i * 16 + g4 * 4 + r) * 64 + wid * 16 + lr] = v[r] * b;
+  };
+#pragma unroll
+  for (int r = 0; r < 4; ++r) own[(g4 * 4 + r) * DR_LS + lr] = d[r];
+  put(wid, d);
+  __syncthreads();
+  f32x4 col[4] = {d, d, d, d};  // tiles of this column, from the diagonal on
+#pragma unroll
+  for (int i = 1; i < 4; ++i) {
+    if (i <= wid) continue;
+    const float* row = ls + (i * 16 + lr) * DR_LS + g4 * 4;
+    f32x4 sum = {0, 0, 0, 0}, y = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < i; ++k) {
+      if (k < wid) continue;
+      const f32x4 l = load4(row + k * 16);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) sum = mma4(l[t], col[k][t], sum);
+    }
+    const f32x4 u = load4(row + i * 16);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) y = mma4(u[t], -sum[t], y);
+    col[i] = y;
+    put(i, y);
   }
 }
 
@@ -737,7 +772,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(
     }
   }
   __syncthreads();
-  if (wid == 0) invert_unit(ls, bs[lane], tm + ch * 4096, lane);
+  invert_tiles(ls, bs, tm + ch * 4096, wid, lane);
 }
 
 // The same for decays per channel, and what the walk multiplies the state with:
@@ -926,7 +961,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_channels_kernel(
     am[ch * 4096 + i * 64 + row] = qv;
   }
   __syncthreads();
-  if (wid == 0) invert_unit(ls, bs[lane], tm + ch * 4096, lane);
+  invert_tiles(ls, bs, tm + ch * 4096, wid, lane);
 }
 
 // ---------------------------------------------------------------------------
