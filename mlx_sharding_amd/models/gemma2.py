@@ -57,16 +57,16 @@ class Gemma2Attention(nn.Module):
         q = q.view(B, T, self.n_heads, self.head_dim)
         k = k.view(B, T, self.n_kv_heads, self.head_dim)
         v = v.view(B, T, self.n_kv_heads, self.head_dim)
-        q = ops.apply_rope(q, cos, sin).transpose(1, 2)
         offset = 0
         gp = None
         if cache is not None and ops.use_native(x):
-            # fused rope-k + cache scatter (see llama.py)
+            # rotations + cache scatter in one kernel (see llama.py)
             gp = cache.graph_pos
             if gp is None:
                 offset = cache.offset
-            k, v = cache.append_rope_kv(k, v, cos, sin)
+            q, k, v = cache.append_rope_qkv(q, k, v, cos, sin)
         else:
+            q = ops.apply_rope(q, cos, sin)
             k = ops.apply_rope(k, cos, sin).transpose(1, 2)
             v = v.transpose(1, 2)
             if cache is not None:
@@ -74,6 +74,7 @@ class Gemma2Attention(nn.Module):
                 if gp is None:
                     offset = cache.offset
                 k, v = cache.update(k, v)
+        q = q.transpose(1, 2)
         out = ops.attention(q, k, v, self.scale, causal_offset=offset,
                             softcap=self.softcap,
                             sliding_window=self.sliding_window, pos_dev=gp)

@@ -58,17 +58,16 @@ class LlamaAttention(nn.Module):
         q = q.view(B, T, self.n_heads, self.head_dim)
         k = k.view(B, T, self.n_kv_heads, self.head_dim)
         v = v.view(B, T, self.n_kv_heads, self.head_dim)
-        q = ops.apply_rope(q, cos, sin).transpose(1, 2)
         offset = 0
         gp = None
         if cache is not None and ops.use_native(x):
-            # fused rope-k + scatter into the caches (one kernel instead
-            # of rope + two index_copy launches)
+            # both rotations and the scatter into the caches in one kernel
             gp = cache.graph_pos
             if gp is None:
                 offset = cache.offset
-            k, v = cache.append_rope_kv(k, v, cos, sin)
+            q, k, v = cache.append_rope_qkv(q, k, v, cos, sin)
         else:
+            q = ops.apply_rope(q, cos, sin)
             k = ops.apply_rope(k, cos, sin).transpose(1, 2)
             v = v.transpose(1, 2)
             if cache is not None:
@@ -76,6 +75,7 @@ class LlamaAttention(nn.Module):
                 if gp is None:
                     offset = cache.offset
                 k, v = cache.update(k, v)
+        q = q.transpose(1, 2)
         out = ops.attention(q, k, v, self.scale, causal_offset=offset,
                             pos_dev=gp)
         out = out.transpose(1, 2).reshape(B, T, -1)

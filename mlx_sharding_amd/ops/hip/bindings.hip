@@ -28,6 +28,9 @@ void launch_rope(const void*, void*, const float*, const float*, long, int,
 void launch_mla_append_kv(const void*, const void*, void*, void*, const int*,
                           int, int, int, int, int, int, int, long, long,
                           hipStream_t);
+void launch_rope_qkv(const void*, const void*, const void*, const float*, const float*,
+                     void*, void*, void*, const int*, long, long, int, int, int, int,
+                     long, long, long, long, hipStream_t);
 void launch_rope_append_kv(const void*, const void*, const float*,
                            const float*, void*, void*, const int*, int, int,
                            int, int, int, long, bool, long, long,
@@ -263,6 +266,49 @@ torch::Tensor apply_rope(torch::Tensor x, torch::Tensor cos, torch::Tensor sin,
               sc.data_ptr<float>(), (long)B * T, T, nH, D, interleaved,
               rstride, hstride, cur_stream());
   return y;
+}
+
+// q, k, v [B, T, heads, D], heads side by side; caches [B, Hkv, cap, D].  Returns the
+// turned queries; keys (turned) and values go to the caches from row pos (pos0) on.
+torch::Tensor rope_qkv(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                       torch::Tensor cos, torch::Tensor sin, torch::Tensor kcache,
+                       torch::Tensor vcache, c10::optional<torch::Tensor> pos,
+                       int64_t pos0) {
+  const long B = q.size(0), T = q.size(1), D = q.size(3), Hkv = k.size(2);
+  auto whole = [](const torch::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  for (const auto& t : {q, k, v}) {
+    check_bf16(t, "operand");
+    TORCH_CHECK(t.dim() == 4 && t.size(0) == B && t.size(1) == T && t.size(3) == D &&
+                    t.stride(3) == 1 && t.stride(2) == D && t.stride(1) % 8 == 0 &&
+                    (B == 1 || t.stride(0) == T * t.stride(1)) && whole(t), "rows");
+  }
+  TORCH_CHECK(D >= 16 && D % 16 == 0 && B >= 1 && T >= 1 && v.size(2) == Hkv &&
+                  (q.size(2) + 3 * Hkv) * D < (1L << 30), "sizes");
+  for (const auto& t : {kcache, vcache}) {
+    check_bf16(t, "cache");
+    TORCH_CHECK(t.dim() == 4 && t.size(0) == B && t.size(1) == Hkv &&
+                    t.size(2) == kcache.size(2) && t.size(3) == D &&
+                    t.is_contiguous() && whole(t), "caches");
+  }
+  for (const auto& t : {cos, sin})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kFloat32 &&
+                    t.is_contiguous() && t.numel() == T * D / 2, "rotations");
+  const int* pp = nullptr;
+  if (pos.has_value()) {
+    TORCH_CHECK(pos->is_cuda() && pos->scalar_type() == torch::kInt32, "pos int32");
+    pp = pos->data_ptr<int>();
+  } else {
+    TORCH_CHECK(pos0 >= 0 && pos0 + T <= kcache.size(2), "no room in the cache");
+  }
+  auto out = torch::empty({B, T, q.size(2), D}, q.options());
+  launch_rope_qkv(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr<float>(),
+                  sin.data_ptr<float>(), out.data_ptr(), kcache.data_ptr(),
+                  vcache.data_ptr(), pp, pos0, B * T, (int)T, (int)q.size(2), (int)Hkv,
+                  (int)D, kcache.size(2), q.stride(1), k.stride(1), v.stride(1),
+                  cur_stream());
+  return out;
 }
 
 // k/v [B, T, Hkv, D]; caches full buffers [B, Hkv, Scap, D]
@@ -1161,6 +1207,9 @@ std::vector<torch::Tensor> moe_gate_subranges(torch::Tensor logits, int64_t K,
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "fused RMSNorm (gfx950)");
   m.def("norm_add", &norm_add);
+  m.def("rope_qkv", &rope_qkv, py::arg("q"), py::arg("k"), py::arg("v"),
+        py::arg("cos"), py::arg("sin"), py::arg("kcache"), py::arg("vcache"),
+        py::arg("pos") = py::none(), py::arg("pos0") = 0);
   m.def("rms_norm_residual", &rms_norm_residual);
   m.def("glu", &glu);
   m.def("softcap", &softcap_op);

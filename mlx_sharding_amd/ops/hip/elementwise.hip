@@ -514,6 +514,81 @@ extern "C" void launch_rope_append_kv(const void* k, const void* v,
         v_rstride);
 }
 
+// ---------------------------------------------------------------------------
+// Queries turned, keys turned into the cache, values into the cache: one kernel.  A
+// thread turns 8 dimensions and their partners, or copies 8 of a value.  Bound by launch
+// in a decoding step (two kernels before, 4.3 us each: one sequence through four layers
+// 484 -> 474 us, a prompt of 57 tokens through three 221 -> 210), by memory in a prompt
+// (the two took a block per row and head, 39 us for 4096 rows of 16 + 8 heads of 256).
+// ---------------------------------------------------------------------------
+
+struct RopeQkvArgs {
+  const __bf16 *q, *k, *v;
+  const float *cos, *sin;      // [T, D / 2]
+  __bf16 *out, *kcache, *vcache;  // [rows, Hq, D], [B, Hkv, cap, D]
+  const int* pos_ptr;          // the first row's place, or null: pos0
+  long qs, ks, vs, cap, pos0, total;
+  int T, Hq, Hkv, D, items;
+};
+
+__global__ __launch_bounds__(256) void rope_qkv_kernel(const RopeQkvArgs a) {
+  const long at = (long)blockIdx.x * 256 + threadIdx.x;
+  if (at >= a.total) return;
+  const long row = at / a.items;
+  int i = (int)(at - row * a.items);
+  const int t = (int)(row % a.T), D = a.D, half = D / 2;
+  const long b = row / a.T;
+  const long pos = (a.pos_ptr ? *a.pos_ptr : a.pos0) + t;
+  auto load = [](const __bf16* p) { return *reinterpret_cast<const bf16x8_t*>(p); };
+  const int turns = (a.Hq + a.Hkv) * (D / 16);
+  if (i >= turns) {  // a value
+    i -= turns;
+    const int h = i / (D / 8), d = i % (D / 8) * 8;
+    if (pos < a.cap)
+      *reinterpret_cast<bf16x8_t*>(a.vcache + ((b * a.Hkv + h) * a.cap + pos) * D + d) =
+          load(a.v + row * a.vs + h * D + d);
+    return;
+  }
+  int h = i / (D / 16);
+  const int d = i % (D / 16) * 8;
+  const bool query = h < a.Hq;
+  if (!query) h -= a.Hq;
+  const __bf16* x = (query ? a.q + row * a.qs : a.k + row * a.ks) + h * D + d;
+  const bf16x8_t u = load(x), v = load(x + half);
+  const float* c = a.cos + (long)t * half + d;
+  const float* s = a.sin + (long)t * half + d;
+  bf16x8_t y, z;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    y[j] = (__bf16)((float)u[j] * c[j] - (float)v[j] * s[j]);
+    z[j] = (__bf16)((float)v[j] * c[j] + (float)u[j] * s[j]);
+  }
+  __bf16* o;
+  if (query) {
+    o = a.out + (row * a.Hq + h) * D + d;
+  } else {
+    if (pos >= a.cap) return;
+    o = a.kcache + ((b * a.Hkv + h) * a.cap + pos) * D + d;
+  }
+  *reinterpret_cast<bf16x8_t*>(o) = y;
+  *reinterpret_cast<bf16x8_t*>(o + half) = z;
+}
+
+// strides of rows in elements; D a multiple of 16, all rows and bases of 8 elements
+extern "C" void launch_rope_qkv(const void* q, const void* k, const void* v,
+                                const float* cos, const float* sin, void* out,
+                                void* kcache, void* vcache, const int* pos_ptr,
+                                long pos0, long rows, int T, int Hq, int Hkv, int D,
+                                long cap, long qs, long ks, long vs,
+                                hipStream_t stream) {
+  RopeQkvArgs a{(const __bf16*)q, (const __bf16*)k, (const __bf16*)v, cos, sin,
+                (__bf16*)out, (__bf16*)kcache, (__bf16*)vcache, pos_ptr, qs, ks, vs,
+                cap, pos0, 0, T, Hq, Hkv, D};
+  a.items = (Hq + Hkv) * (D / 16) + Hkv * (D / 8);
+  a.total = rows * a.items;
+  rope_qkv_kernel<<<dim3((unsigned)((a.total + 255) / 256)), dim3(256), 0, stream>>>(a);
+}
+
 extern "C" void launch_mla_append_kv(const void* kvh, const void* kpe,
                                      void* kcache, void* vcache,
                                      const int* pos_ptr, int pos0, int B,

@@ -121,6 +121,27 @@ class KVCache:
         self.offset += T
         return (self._k[:, :, : self.offset], self._v[:, :, : self.offset])
 
+    def append_rope_qkv(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                        cos: torch.Tensor, sin: torch.Tensor):
+        """append_rope_kv with the queries turned as well: (q, k, v).  One kernel where
+        heads of a row lie side by side in whole 16-byte vectors."""
+        from .. import ops as _ops
+        B, T, _, D = k.shape
+        if not (D % 16 == 0 and self.k_head_dim == self.v_head_dim == D
+                and self.dtype == torch.bfloat16 and cos.dtype == torch.float32
+                and all(t.dtype == torch.bfloat16 and t.stride(3) == 1
+                        and t.stride(2) == D and t.stride(1) % 8 == 0
+                        and (B == 1 or t.stride(0) == T * t.stride(1))
+                        and t.data_ptr() % 16 == 0 for t in (q, k, v))):
+            q = _ops.apply_rope(q, cos, sin)
+            return (q, *self.append_rope_kv(k, v, cos, sin))
+        pos, at = self.claim(B, T)
+        q = _ops.hip_ext().rope_qkv(q, k, v, cos.contiguous(), sin.contiguous(),
+                                    self._k, self._v, pos, at)
+        if pos is not None:
+            return q, self._k, self._v
+        return q, self._k[:, :, : self.offset], self._v[:, :, : self.offset]
+
     @property
     def k(self) -> Optional[torch.Tensor]:
         return None if self._k is None else self._k[:, :, : self.offset]
