@@ -94,6 +94,7 @@ __global__ __launch_bounds__(NT, EXACT && RPT * HP <= 32 ? 4 : 2) void delta_sho
   const int kh = blockIdx.y;
   const int t0 = cu[e];
   const int n = min(cu[e + 1] - t0, DR_SHORT);
+  const int first_row = n > 0 ? t0 : 0;  // a portion without tokens may lie at the end
   const bool fresh = pos0[e] == 0;
   const long slot = __builtin_amdgcn_readfirstlane(slots[e]);
   const int D = dm.D, V = dm.V;
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(NT, EXACT && RPT * HP <= 32 ? 4 : 2) void delta_sho
       f.w[j] = j >= pad ? conv_w[(long)c * dm.taps + j - pad] : (T)0.0f;
       if (j < DR_MAXTAPS - 1) f.x[j] = j >= pad ? cs[j - pad] : (T)0.0f;
     }
-    f.first = y[(long)t0 * dm.ystride + col];
+    f.first = y[(long)first_row * dm.ystride + col];
   };
   auto convolve = [&](const Conv& f, int i, int h0) {
     int c, col;
@@ -201,9 +202,9 @@ __global__ __launch_bounds__(NT, EXACT && RPT * HP <= 32 ? 4 : 2) void delta_sho
     if (begin + tid < end) fetch(first, begin + tid, h0);
     // of the first token: decay, write strength, output gate
     T a_in[HP], b_in[HP], g_in[HP], Al[HP], dt[HP];
-    auto inputs = [&](int t) {
-      const T* yt = y + (long)(t0 + t) * dm.ystride;
-      const T* zt = z + (long)(t0 + t) * dm.zstride;
+    auto inputs = [&](int row) {
+      const T* yt = y + (long)row * dm.ystride;
+      const T* zt = z + (long)row * dm.zstride;
 #pragma unroll
       for (int p = 0; p < HP; ++p) {
         const int h = h0 + min(p, heads - 1);
@@ -212,7 +213,7 @@ __global__ __launch_bounds__(NT, EXACT && RPT * HP <= 32 ? 4 : 2) void delta_sho
         g_in[p] = zt[dm.gc + h * V + vc];
       }
     };
-    inputs(0);
+    inputs(first_row);
 #pragma unroll
     for (int p = 0; p < HP; ++p) {
       const int h = h0 + min(p, heads - 1);
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(NT, EXACT && RPT * HP <= 32 ? 4 : 2) void delta_sho
     }
     __syncthreads();
     for (int t = 0; t < n; ++t) {
-      if (t) inputs(t);
+      if (t) inputs(t0 + t);
       const float* qr = qk + (long)t * 2 * D;
       const float* kr = qr + D;
       float qq = 0.0f, kk = 0.0f, qd = 0.0f;
