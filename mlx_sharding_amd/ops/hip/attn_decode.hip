@@ -369,8 +369,9 @@ extern "C" bool attn_decode_supported_shape(int G, int Dv) {
 // a quarter of the output's columns, O^T = V^T P^T.  So waves share no outputs.
 // V^T is read by ds_read_b64_tr_b16 out of rows as they lie in memory; values that
 // lie in the keys' rows (a cached latent) are staged once for both.
-// Weights stay 32-bit: they enter as a high and a low bf16 part (16 bits and
-// more, at twice the products, which have time to spare).
+// Weights stay 32-bit: three bf16 parts hold all of their 24 bits, at three times the
+// products, which have time to spare (64 sequences of 2049 keys, as below: 101 us, 99
+// with two parts, which keep 16 bits; 104 where the parts are rounded, not cut off).
 // Slices come from the length on the device, so they are even under capture.
 // Measured (before: dot products and sums on the vector units, up to 8 slices of
 // the capacity): 64 sequences of 2049 keys, 32 heads of 128 over 8: 179 -> 109 us
@@ -381,6 +382,7 @@ extern "C" bool attn_decode_supported_shape(int G, int Dv) {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 #define DT_MAXSPLIT 64
 
@@ -528,13 +530,23 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
     }
 #pragma unroll
     for (int x = 0; x < KT / 32; ++x) {
-      bf16x8_t high, low;
+      bf16x8_t v[ND];
+      u32x4 w[3];  // pairs: the upper halves of what is left of each weight
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float w = __builtin_amdgcn_exp2f(p[x][j] - m);
-        l += w;
-        high[j] = (__bf16)w;
-        low[j] = (__bf16)(w - (float)high[j]);
+      for (int j = 0; j < 8; j += 2) {
+        float f[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          f[h] = __builtin_amdgcn_exp2f(p[x][j + h] - m);
+          l += f[h];
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const unsigned a = __float_as_uint(f[0]), b = __float_as_uint(f[1]);
+          w[i][j / 2] = __builtin_amdgcn_perm(b, a, 0x07060302);
+          f[0] -= __uint_as_float(a & 0xFFFF0000u);
+          f[1] -= __uint_as_float(b & 0xFFFF0000u);
+        }
       }
 #pragma unroll
       for (int d = 0; d < ND; ++d) {
@@ -547,11 +559,15 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
         const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (__attribute__((address_space(3))) s16x4*)(
                 (INROW ? src - KB : src) + 16 * VP * 16));
-        const bf16x8_t v = __builtin_bit_cast(
+        v[d] = __builtin_bit_cast(
             bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, high, o[d], 0, 0, 0);
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, low, o[d], 0, 0, 0);
       }
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              v[d], __builtin_bit_cast(bf16x8_t, w[i]), o[d], 0, 0, 0);
     }
   }
 

@@ -111,9 +111,39 @@ def test_decode_edges(Hq, Hkv, Dk, Dv, captured):
                 pos = torch.tensor([S - 1], dtype=torch.int32, device="cuda")
             out = ext().attn_decode(q, *given, scale, cap, window, pos).double()
             expect, size = attention(q, k, v, scale, cap, window, S - 1)
-            # the result is rounded to bf16; 32-bit weights in two bf16 parts
+            # the result is rounded to bf16, exponents come in 32-bit steps
             bound = 2.0 ** -8 * expect.abs() + 2.0 ** -13 * size + 1e-6
             assert bool(((out - expect).abs() <= bound).all()), (S, cap, window)
+
+
+def opposed(Hq, Hkv, Dk, Dv, S, step):
+    """q, k, v whose values come in pairs of opposite sign, with scores (at a scale of
+    1) that differ by twice ``step``: what is left of a pair's weights is their
+    difference.  Scores lie in 32 bits as they are."""
+    at = Dk - 2  # behind values that lie in the keys' rows
+    q = torch.zeros(2, Hq, 1, Dk, device="cuda")
+    q[..., at:] = 1.0
+    k, v = cached(2, Hkv, S, Dk, 70), cached(2, Hkv, S, Dv, 70)
+    base = torch.rand(2, Hkv, S // 2, device="cuda") - 1.0
+    k[..., at] = base.repeat_interleave(2, 2).bfloat16()
+    k[:, :, 0::2, at + 1], k[:, :, 1::2, at + 1] = step, -step
+    if Dk == 576:
+        v = k[..., :Dv]
+    v[:, :, 1::2] = -v[:, :, 0::2]
+    return q.bfloat16(), k, v
+
+
+@pytest.mark.parametrize("Hq,Hkv,Dk,Dv", DECODE)
+def test_decode_weights_are_whole(Hq, Hkv, Dk, Dv):
+    """All 24 bits of the weights count."""
+    torch.manual_seed(Hq + Dk)
+    q, k, v = opposed(Hq, Hkv, Dk, Dv, 512, 2.0 ** -15)
+    out = ext().attn_decode(q, k, v, 1.0, 0.0, 0, None).double()
+    expect, _ = attention(q, k, v, 1.0, 0.0, 0, 511)
+    # Of a difference of 2^-14: exponents in steps of 2^-24 and powers within 2^-23,
+    # twice, make 2^-8.2 at most and less than half on average; the result is rounded
+    # by 2^-9.  Weights of 16 bits would be off by 3%.
+    assert (out - expect).norm() < 0.008 * expect.norm()
 
 
 @pytest.mark.parametrize("captured", [False, True])
