@@ -20,6 +20,7 @@
 // indexed (guide §5.4 rule 20).
 
 #include "hip_common.h"
+#include "soft_cap.h"
 
 #define AD_BLOCK 256
 
@@ -370,14 +371,13 @@ extern "C" bool attn_decode_supported_shape(int G, int Dv) {
 // V^T is read by ds_read_b64_tr_b16 out of rows as they lie in memory; values that
 // lie in the keys' rows (a cached latent) are staged once for both.
 // Weights stay 32-bit: three bf16 parts hold all of their 24 bits, at three times the
-// products, which have time to spare (64 sequences of 2049 keys, as below: 101 us, 99
-// with two parts, which keep 16 bits; 104 where the parts are rounded, not cut off).
+// products, which have time to spare (the first size below: 2 us more than with two
+// parts, which keep 16 bits, and 3 less than with parts that are rounded, not cut off).
 // Slices come from the length on the device, so they are even under capture.
 // Measured (before: dot products and sums on the vector units, up to 8 slices of
-// the capacity): 64 sequences of 2049 keys, 32 heads of 128 over 8: 179 -> 109 us
-// (4.9 TB/s, what a copy reaches); one of 1024: 24 -> 8.4; 5 of 5004, 16 heads of
-// 256 over 8, capped: 91 -> 45; 16 heads over a latent of 576/512, 64 x 513 keys:
-// 66 -> 22, 1 x 3002: 75 -> 14.
+// the capacity): 64 sequences of 2049 keys, 32 heads of 128 over 8: 179 -> 98 us
+// (5.5 TB/s); one of 1024: 24 -> 7.2; 5 of 5004, 16 heads of 256 over 8, capped: 91 ->
+// 45; 16 heads over a latent of 576/512, 64 x 513 keys: 66 -> 22, 1 x 3002: 75 -> 13.
 // ---------------------------------------------------------------------------
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -393,8 +393,7 @@ struct DecodeArgs {
   const int* s_ptr;
   int Hq, Hkv, S, nsplit, window;
   long cap;
-  float c;                 // score -> power of two; behind a cap: 1
-  float cap_in, cap_out;   // e^(2 score / cap) as 2^(cap_in s); cap in base 2
+  SoftCap score;           // scale and cap
 };
 
 __device__ __forceinline__ void dt_to_lds(const char* src, char* dst) {
@@ -500,23 +499,24 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
     for (int r = 0; r < 4; ++r) sc[buf][half][kb * 16 + lg * 4 + r][l16] = s4[r];
     __syncthreads();
 
-    float p[KT / 32][8], top = -INFINITY;
+    float p[KT / 4], top = -INFINITY;  // 8 of every 32 keys
+    auto key_of = [&](int i) { return i / 4 * 16 + lg * 4 + (i & 3); };
 #pragma unroll
-    for (int x = 0; x < KT / 32; ++x)
+    for (int i = 0; i < KT / 4; ++i) {
+      p[i] = sc[buf][0][key_of(i)][l16];
+      if (HALVES == 2) p[i] += sc[buf][HALVES - 1][key_of(i)][l16];
+    }
+    if (a.score.out > 0.0f) {
+      soft_capped(a.score, p);
+    } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int key = x * 32 + (j >> 2) * 16 + lg * 4 + (j & 3);
-        float v = sc[buf][0][key][l16];
-        if (HALVES == 2) v += sc[buf][HALVES - 1][key][l16];
-        if (a.cap_out > 0.0f) {
-          const float e = __builtin_amdgcn_exp2f(v * a.cap_in);
-          v = a.cap_out - 2.0f * a.cap_out * __builtin_amdgcn_rcpf(e + 1.0f);
-        } else {
-          v *= a.c;
-        }
-        p[x][j] = t + key < to ? v : -INFINITY;
-        top = fmaxf(top, p[x][j]);
-      }
+      for (int i = 0; i < KT / 4; ++i) p[i] *= a.score.lin;
+    }
+#pragma unroll
+    for (int i = 0; i < KT / 4; ++i) {
+      if (t + key_of(i) >= to) p[i] = -INFINITY;
+      top = fmaxf(top, p[i]);
+    }
     top = column_max(top);
     const float m_new = fmaxf(m, top);
     if (__any(m_new > m)) {
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
         float f[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          f[h] = __builtin_amdgcn_exp2f(p[x][j + h] - m);
+          f[h] = __builtin_amdgcn_exp2f(p[x * 8 + j + h] - m);
           l += f[h];
         }
 #pragma unroll
@@ -660,14 +660,9 @@ extern "C" void launch_attn_decode_tile(
     float* part_ml, int nsplit, const int* s_ptr, int B, int Hq, int Hkv, int S,
     long Scap, int Dk, int Dv, bool inrow, float scale, float softcap,
     int window, hipStream_t stream) {
-  constexpr float LOG2E = 1.44269504088896340736f;
-  DecodeArgs a{(const char*)q, (const char*)k, (const char*)v, (char*)out,
-               part_o, part_ml, s_ptr, Hq, Hkv, S, nsplit, window, Scap,
-               scale * LOG2E, 0.0f, 0.0f};
-  if (softcap > 0.0f) {
-    a.cap_in = 2.0f * a.c / softcap;
-    a.cap_out = softcap * LOG2E;
-  }
+  const DecodeArgs a{(const char*)q, (const char*)k, (const char*)v, (char*)out,
+                     part_o, part_ml, s_ptr, Hq, Hkv, S, nsplit, window, Scap,
+                     soft_cap(scale, softcap)};
 #define DT_GO(K, V, T, R)                         \
   if (Dk == K && Dv == V && inrow == R)           \
     attn_decode_tile_go<K, V, T, R>(a, B, stream);

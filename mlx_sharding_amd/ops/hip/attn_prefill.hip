@@ -23,13 +23,14 @@
 // that a read meets share their banks.
 // Measured (before: 16 queries a wave, scores through LDS, V transposed element by
 // element): 8192 tokens, 32 heads of 128 over 8: 5310 -> 601 us (914 TFLOP/s);
-// 4096 tokens, 16 heads of 256 over 8, capped: 1600 -> 242 us (567), 1905 behind 4096
-// with a window of 4096: 213 us (402 and 457 while places in LDS had a register each
-// and were spilled: each reload waited for the next tile's loads; 255 and 228 with all
-// of a query in registers); 64 prompts of 512, 16 heads of 192/128: 1216 -> 176 us
+// 4096 tokens, 16 heads of 256 over 8, capped: 1600 -> 240 us (572), 1905 behind 4096
+// with a window of 4096: 210 us (400 and 450 while places in LDS had a register each
+// and were spilled: each reload waited for the next tile's loads; 13 and 15 us more with
+// all of a query in registers); 64 prompts of 512, 16 heads of 192/128: 1216 -> 176 us
 // (490); 57 tokens: 8.4 -> 7.6 us.
 
 #include "hip_common.h"
+#include "soft_cap.h"
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -47,7 +48,7 @@ struct PrefillArgs {
   long q_b, q_h, q_t;        // strides of q, elements
   long kcap, vcap;           // rows of a head's keys and values
   float c;                   // score -> power of two; behind a cap: 1
-  float cap_in, cap_out;     // e^(2 score / cap) as 2^(cap_in s); cap in base 2
+  SoftCap cap;
   int flip;                  // a negative scale: queries change their sign
   int window, offset;
   int heads, tiles, group;   // B * Hq, query tiles, heads that run together
@@ -276,12 +277,14 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
       }
     if (CAP) {
 #pragma unroll
-      for (int n = 0; n < NB; ++n)
+      for (int n = 0; n < NB; ++n) {
+        float v[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float e = __builtin_amdgcn_exp2f(s[n][r] * a.cap_in);
-          s[n][r] = a.cap_out - 2.0f * a.cap_out * __builtin_amdgcn_rcpf(e + 1.0f);
-        }
+        for (int r = 0; r < 16; ++r) v[r] = s[n][r];
+        soft_capped(a.cap, v);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[n][r] = v[r];
+      }
     }
     if (t + KT - 1 > all_hi || t < all_lo) {
 #pragma unroll
@@ -393,11 +396,8 @@ static void prefill_setup(PrefillArgs& a, int B, float scale, float softcap,
   a.flip = scale < 0.0f;
   // a scale of zero: hidden scores still have to vanish
   a.c = fmaxf(fabsf(scale) * LOG2E, 1e-30f);
-  if (softcap > 0.0f) {
-    a.cap_in = 2.0f * a.c / softcap;
-    a.cap_out = softcap * LOG2E;
-    a.c = 1.0f;
-  }
+  a.cap = soft_cap(fabsf(scale), softcap);
+  if (softcap > 0.0f) a.c = 1.0f;
   a.window = window;
   a.offset = offset;
   a.heads = B * a.Hq;

@@ -146,6 +146,40 @@ def test_decode_weights_are_whole(Hq, Hkv, Dk, Dv):
     assert (out - expect).norm() < 0.008 * expect.norm()
 
 
+@pytest.mark.parametrize("cap", [5.0, 50.0])
+def test_soft_cap_of_small_differences(cap):
+    """Capped scores keep the bits of their differences."""
+    torch.manual_seed(1)
+    q, k, v = opposed(8, 2, 128, 128, 512, 2.0 ** -15)
+    out = ext().attn_decode(q, k, v, 1.0, cap, 0, None).double()
+    expect, _ = attention(q, k, v, 1.0, cap, 0, 511)
+    # as above; the cap's own roundings are 2^-22 of scores of up to 1, twice.  Taken
+    # from cap * (1 - 2 / (e^2y + 1)), scores were off by 2^-24 of the cap and more
+    assert (out - expect).norm() < 0.012 * expect.norm()
+
+
+@pytest.mark.parametrize("cap,scale", [(20.0, 1.0), (30.0, -0.5), (50.0, 3.0)])
+def test_soft_cap_range(cap, scale):
+    """Scores from far below the cap to far above it, of both signs, in waves that
+    have only small ones and in mixed ones."""
+    torch.manual_seed(2)
+    D, S = 256, 300
+    size = torch.logspace(-3, 1.3, S, device="cuda")[:, None]
+    for top in (0.03, 1.0):
+        k = (torch.randn(1, 2, S, D, device="cuda") * size * top).bfloat16()
+        v = torch.randn(1, 2, S, D, device="cuda").bfloat16()
+        q = torch.randn(1, 8, S, D, device="cuda").bfloat16() * 0.25
+        for got, first in ((ext().attn_prefill(q, k, v, scale, cap, 0, 0), 0),
+                           (ext().attn_decode(q[:, :, -1:], k, v, scale, cap, 0, None),
+                            S - 1)):
+            expect, whole = attention(q[:, :, first:], k, v, scale, cap, 0, first)
+            # weights (of a prompt) and result are rounded to bf16; 32-bit scores
+            # below the cap are off by 2^-21 of it, each way
+            bound = (2.0 ** -8 * ((whole if first == 0 else 0) + expect.abs())
+                     + cap * 2.0 ** -20 * whole + 1e-6)
+            assert bool(((got.double() - expect).abs() <= bound).all()), (top, first)
+
+
 @pytest.mark.parametrize("captured", [False, True])
 @pytest.mark.parametrize("N,S,nope,vdim", [(1, 1, 128, 128), (1, 3002, 128, 128),
                                            (3, 33, 32, 16), (17, 64, 160, 208),
