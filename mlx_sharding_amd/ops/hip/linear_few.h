@@ -3,6 +3,7 @@
 #pragma once
 
 #include <torch/extension.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
 extern "C" void launch_linear_few(const void*, const void*, const void*,
@@ -17,9 +18,10 @@ static torch::Tensor linear_few(torch::Tensor x, torch::Tensor w,
                                 c10::optional<torch::Tensor> residual,
                                 c10::optional<torch::Tensor> norm, double eps,
                                 double offset, int64_t act) {
-  auto bf16 = [](const torch::Tensor& t) {
-    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16,
-                "linear_few takes bf16 tensors on the GPU");
+  auto bf16 = [&](const torch::Tensor& t) {
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
+                    t.device() == x.device(),
+                "linear_few takes bf16 tensors on one GPU");
   };
   auto whole = [](const torch::Tensor& t) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
@@ -54,6 +56,7 @@ static torch::Tensor linear_few(torch::Tensor x, torch::Tensor w,
     r = residual->data_ptr();
     ldr = residual->stride(0);
   }
+  const c10::DeviceGuard guard(x.device());  // and its current stream
   auto y = torch::empty({M, O}, x.options());
   launch_linear_few(x.data_ptr(), w.data_ptr(), b, r, n, y.data_ptr(), M, O, K,
                     x.stride(0), w.stride(0), ldr, O, (float)eps, (float)offset,
@@ -79,7 +82,7 @@ static bool linear_few_plain(const torch::Tensor& t) {
 // many rows of large weights (64 rows of 4096 into 28672: 54 us here, 51 there).
 static bool linear_few_takes(const torch::Tensor& x, const torch::Tensor& w,
                              bool alone) {
-  if (!x.is_cuda() || !w.is_cuda() || x.scalar_type() != torch::kBFloat16 ||
+  if (!x.is_cuda() || w.device() != x.device() || x.scalar_type() != torch::kBFloat16 ||
       w.scalar_type() != torch::kBFloat16 || w.dim() != 2 || x.dim() < 1 ||
       !linear_few_plain(x) || !linear_few_plain(w))
     return false;
@@ -103,7 +106,11 @@ static c10::optional<torch::Tensor> linear_few_try(
     torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
     c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> norm,
     double eps, double offset, int64_t act) {
+  auto elsewhere = [&](const c10::optional<torch::Tensor>& t) {
+    return t.has_value() && t->device() != x.device();
+  };
   if (!linear_few_takes(x, w, !residual.has_value() && !norm.has_value() && !act) ||
+      elsewhere(bias) || elsewhere(norm) || elsewhere(residual) ||
       (bias.has_value() && !linear_few_plain(*bias)) ||
       (norm.has_value() &&
        (norm->scalar_type() != torch::kBFloat16 ||
