@@ -94,7 +94,7 @@ class Gemma2MLP(nn.Module):
 
     def forward(self, x, norm: Optional[RMSNorm] = None):
         """norm: as in Gemma2Attention."""
-        if self._fused_gu is not None and ops.few_tokens(x):
+        if self._fused_gu is not None and (norm is not None or ops.few_tokens(x)):
             return self.down_proj(project(self._fused_gu, x, norm=norm,
                                           act="gelu_tanh"))
         if norm is not None:

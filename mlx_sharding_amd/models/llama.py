@@ -98,7 +98,7 @@ class LlamaMLP(nn.Module):
     def forward(self, x: torch.Tensor, norm: Optional[RMSNorm] = None,
                 residual: Optional[torch.Tensor] = None) -> torch.Tensor:
         """norm, residual: as in LlamaAttention."""
-        if self._fused_gu is not None and ops.few_tokens(x):
+        if self._fused_gu is not None and (norm is not None or ops.few_tokens(x)):
             y = project(self._fused_gu, x, norm=norm, act="silu")
             return project(self.down_proj, y, residual=residual)
         if norm is not None:

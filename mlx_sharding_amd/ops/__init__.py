@@ -19,6 +19,7 @@ import os
 from typing import Optional
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import reference as ref
 
@@ -235,12 +236,28 @@ _ACTS = {None: 0, "silu": 1, "gelu_tanh": 2}
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
+def _function_modes() -> bool:
+    """Whether function modes are at work, but that of a default device."""
+    n = torch._C._len_torch_function_stack()
+    return n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
+                         for i in range(n))
+
+
+def _watched() -> bool:
+    """Whether something around the call sees only torch's own operators: forward-mode
+    differentiation, torch.jit.trace, dispatch modes (make_fx, fake tensors), function
+    modes."""
+    return (torch.autograd.forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() > 0 or _function_modes())
+
+
 def _plain(t: torch.Tensor) -> bool:
     """An ordinary tensor that nothing differentiates, maps or traces."""
     return (type(t) in _TENSORS
             and not (t.requires_grad and torch.is_grad_enabled())
             and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-            and torch.autograd.forward_ad._current_level < 0)
+            and not _watched())
 
 
 def few_rows(x: torch.Tensor, weight: torch.Tensor, alone: bool = False) -> bool:
@@ -262,7 +279,7 @@ def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None):
     step calls this for each of its products: what can be seen from the tensors is
     looked at in native code (in Python that took longer than the launch)."""
     if (_force_torch() or type(x) not in _TENSORS or type(weight) not in _TENSORS
-            or torch.autograd.forward_ad._current_level >= 0):
+            or torch.autograd.forward_ad._current_level >= 0 or _function_modes()):
         return None
     ext = _few_ext()
     if ext is None:

@@ -4,6 +4,7 @@
 
 #include <torch/extension.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
 extern "C" void launch_linear_few(const void*, const void*, const void*,
@@ -75,6 +76,13 @@ static bool linear_few_plain(const torch::Tensor& t) {
          !(t.requires_grad() && at::GradMode::is_enabled());
 }
 
+// Whether torch.jit.trace or a dispatch mode records this thread's operators.
+static bool linear_few_recorded() {
+  static const c10::DispatchKeySet recorders(
+      {c10::DispatchKey::Python, c10::DispatchKey::Tracer});
+  return c10::impl::tls_local_dispatch_key_set().included_.has_any(recorders);
+}
+
 // Whether x w^T runs here: up to 64 bf16 rows that begin, as w's, at whole 16-byte
 // vectors.  A contraction above 8192 for 8 rows, or into 4096: 8 rows of 14336 into
 // 4096 take 24.6 us here and 26.6 in the library, 32 rows 30.4 and 30.5, 64 rows 40.1
@@ -84,7 +92,7 @@ static bool linear_few_takes(const torch::Tensor& x, const torch::Tensor& w,
                              bool alone) {
   if (!x.is_cuda() || w.device() != x.device() || x.scalar_type() != torch::kBFloat16 ||
       w.scalar_type() != torch::kBFloat16 || w.dim() != 2 || x.dim() < 1 ||
-      !linear_few_plain(x) || !linear_few_plain(w))
+      !linear_few_plain(x) || !linear_few_plain(w) || linear_few_recorded())
     return false;
   const long O = w.size(0), K = w.size(1);
   if (O < 1 || K < 32 || K % 32 || x.size(-1) != K) return false;

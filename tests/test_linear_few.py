@@ -101,6 +101,45 @@ def test_other_forms_keep_the_library():
     assert tangent is not None
 
 
+@pytest.mark.gpu
+def test_tracers_see_a_product():
+    """What records operators records torch's own, and what it made runs on other
+    rows."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from torch.utils.flop_counter import FlopCounterMode
+
+    class Names(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Calls(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func.__name__)
+            return func(*args, **(kwargs or {}))
+
+    w = torch.randn(24, 64, device="cuda").bfloat16()
+    x, other = (torch.randn(3, 64, device="cuda").bfloat16() for _ in range(2))
+    res = torch.randn(3, 24, device="cuda").bfloat16()
+    f = lambda t: ops.project(t, w, residual=res)  # noqa: E731
+    expect = other.double() @ w.double().T + res.double()
+    close = lambda y: (y.double() - expect).norm() < 0.01 * expect.norm()  # noqa: E731
+    assert close(torch.jit.trace(f, (x,), check_trace=False)(other))
+    assert close(make_fx(f)(x)(other))
+    for mode, name in ((Names, "mm"), (Calls, "linear")):
+        seen = []
+        with mode():
+            assert not ops.few_tokens(x)
+            y = f(other)
+        assert close(y) and any(name in s for s in seen), seen
+    with FlopCounterMode(display=False) as count:
+        f(x)
+    assert count.get_total_flops() == 2 * 3 * 64 * 24
+    with torch.device("cuda"):  # a mode, too, that records nothing
+        assert ops.few_tokens(x) and close(f(other))
+
+
 def test_cpu_tensors_keep_torch():
     x, w = torch.randn(2, 64).bfloat16(), torch.randn(24, 64).bfloat16()
     assert not ops.few_rows(x, w) and not ops.few_tokens(x)
