@@ -3,6 +3,7 @@
 #pragma once
 
 #include <torch/extension.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
@@ -94,6 +95,9 @@ static bool linear_few_takes(const torch::Tensor& x, const torch::Tensor& w,
       w.scalar_type() != torch::kBFloat16 || w.dim() != 2 || x.dim() < 1 ||
       !linear_few_plain(x) || !linear_few_plain(w) || linear_few_recorded())
     return false;
+  if (at::autocast::is_autocast_enabled(at::kCUDA) &&
+      at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16)
+    return false;  // a product of another type
   const long O = w.size(0), K = w.size(1);
   if (O < 1 || K < 32 || K % 32 || x.size(-1) != K) return false;
   const long rows = x.numel() / K;

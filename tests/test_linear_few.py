@@ -140,6 +140,19 @@ def test_tracers_see_a_product():
         assert ops.few_tokens(x) and close(f(other))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [3, 200])
+def test_autocast_names_the_type(rows):
+    """Few rows have the type that many have."""
+    w = torch.randn(24, 64, device="cuda").bfloat16()
+    x = torch.randn(rows, 64, device="cuda").bfloat16()
+    for kind in (torch.float16, torch.bfloat16):
+        with torch.autocast("cuda", dtype=kind):
+            y, expect = ops.linear(x, w), F.linear(x, w)
+        assert y.dtype == expect.dtype == kind
+        assert (y.double() - expect.double()).norm() < 0.01 * expect.double().norm()
+
+
 def test_cpu_tensors_keep_torch():
     x, w = torch.randn(2, 64).bfloat16(), torch.randn(24, 64).bfloat16()
     assert not ops.few_rows(x, w) and not ops.few_tokens(x)
