@@ -113,25 +113,38 @@ static bool linear_few_takes(const torch::Tensor& x, const torch::Tensor& w,
          whole(w);
 }
 
+// Whether a product here takes along what it is given: a bias per row of w and norm
+// weights per column, side by side, and a residual of the result's shape.  Other forms
+// (strides, broadcasts, other types and devices) are those of separate operators.
+static bool linear_few_along(const torch::Tensor& x, long O, long biases,
+                             const c10::optional<torch::Tensor>& bias,
+                             const c10::optional<torch::Tensor>& residual,
+                             const c10::optional<torch::Tensor>& norm) {
+  auto here = [&](const torch::Tensor& t) {
+    return t.device() == x.device() && t.scalar_type() == torch::kBFloat16 &&
+           linear_few_plain(t);
+  };
+  auto vec = [&](const c10::optional<torch::Tensor>& t, long n) {
+    return !t.has_value() || (here(*t) && t->is_contiguous() && t->numel() == n);
+  };
+  if (!vec(bias, biases) || !vec(norm, x.size(-1)) ||
+      (norm.has_value() && reinterpret_cast<uintptr_t>(norm->data_ptr()) % 16))
+    return false;
+  if (!residual.has_value()) return true;
+  return here(*residual) && residual->dim() == x.dim() && residual->size(-1) == O &&
+         residual->stride(-1) == 1 &&
+         residual->sizes().slice(0, x.dim() - 1) == x.sizes().slice(0, x.dim() - 1);
+}
+
 // linear_few for x of any number of dimensions, or nothing where it does not run here.
 static c10::optional<torch::Tensor> linear_few_try(
     torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
     c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> norm,
     double eps, double offset, int64_t act) {
-  auto elsewhere = [&](const c10::optional<torch::Tensor>& t) {
-    return t.has_value() && t->device() != x.device();
-  };
   if (!linear_few_takes(x, w, !residual.has_value() && !norm.has_value() && !act) ||
-      elsewhere(bias) || elsewhere(norm) || elsewhere(residual) ||
-      (bias.has_value() && !linear_few_plain(*bias)) ||
-      (norm.has_value() &&
-       (norm->scalar_type() != torch::kBFloat16 ||
-        reinterpret_cast<uintptr_t>(norm->data_ptr()) % 16)) ||
-      (residual.has_value() && (residual->scalar_type() != torch::kBFloat16 ||
-                                residual->stride(-1) != 1)))
+      !linear_few_along(x, w.size(0) / (act ? 2 : 1), w.size(0), bias, residual, norm))
     return {};
-  if (x.dim() == 2 && (!residual.has_value() || residual->dim() == 2))
-    return linear_few(x, w, bias, residual, norm, eps, offset, act);
+  if (x.dim() == 2) return linear_few(x, w, bias, residual, norm, eps, offset, act);
   auto rows = x.reshape({-1, x.size(-1)});
   if (rows.stride(0) % 8 || reinterpret_cast<uintptr_t>(rows.data_ptr()) % 16)
     rows = rows.clone();

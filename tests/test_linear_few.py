@@ -102,6 +102,42 @@ def test_other_forms_keep_the_library():
 
 
 @pytest.mark.gpu
+def test_other_forms_of_what_goes_along():
+    """Biases and residuals in the forms that separate operators take, on their own
+    and with a norm: strides, broadcasts, other types, gradients."""
+    x, w, norm, b, r = make(6, 24, 64, None, wide=False)
+    x, r = x.view(2, 3, 64), r.view(2, 3, 24)
+    wide = torch.randn(24, 2, device="cuda").bfloat16()
+    h = x.double()
+    normed = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + 1e-5) * (
+        norm.weight.double() + 1.0)
+
+    class Norm:
+        weight, eps, weight_offset = norm.weight, norm.eps, norm.weight_offset
+
+        def __call__(self, t):
+            return ops.rms_norm(t, self.weight, self.eps, self.weight_offset)
+
+    for bias in (None, wide[:, 1], b[:1].expand(24), b[:1], b[None]):
+        off = 0.0 if bias is None else bias.double()
+        expect = h @ w.double().T + off
+        y = ops.linear(x, w, bias)
+        assert y.shape == expect.shape
+        assert (y.double() - expect).norm() < 0.01 * expect.norm()
+        for res in (r, r[:1, :1], r[..., :1], r.float(), r[0], r.transpose(0, 1)
+                    .contiguous().transpose(0, 1), wide[:, 1]):
+            for n, rows in ((None, h), (Norm(), normed)):
+                expect = rows @ w.double().T + off + res.double()
+                y = ops.project(x, w, bias, norm=n, residual=res)
+                assert y.shape == expect.shape
+                assert y.dtype == torch.promote_types(x.dtype, res.dtype)
+                assert (y.double() - expect).norm() < 0.01 * expect.norm()
+    p = torch.nn.Parameter(r)
+    ops.project(x, w, residual=p).float().sum().backward()
+    assert bool((p.grad == 1).all())
+
+
+@pytest.mark.gpu
 def test_tracers_see_a_product():
     """What records operators records torch's own, and what it made runs on other
     rows."""
