@@ -607,7 +607,10 @@ def expert_rows_ok(x, gate_w, up, down, top: int, bits: int, group_size: int
     """Whether a decoding step's routed experts run on moe_rows.hip.  gate_w: the
     router's; up, down: stacked matrices of an expert kind (packed, or bf16 with
     ``bits`` 16)."""
-    if not (x.dtype == torch.bfloat16 and use_native(x) and _plain(x)):
+    if not (x.dtype == torch.bfloat16 and use_native(x) and _plain(x)
+            and bits in (4, 8, 16)
+            and all(t.device == x.device and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in (gate_w, up, down))):
         return False
     per = 1 if bits == 16 else 32 // bits
     E, I, H = up.shape[0], up.shape[1], up.shape[2] * per
@@ -624,8 +627,14 @@ def expert_route(x, residual, norm, gate_w, top: int, scaling: float,
     """(rows of x + residual as ``norm`` makes them, x + residual, experts and
     weights of every token), one kernel; rows [N, H]."""
     return _require_ext("moe_route").moe_route(
-        x, residual, norm.weight, norm.eps, norm.weight_offset, gate_w, top,
-        scaling, normalize)
+        _whole(x), None if residual is None else _whole(residual), norm.weight,
+        norm.eps, norm.weight_offset, gate_w, top, scaling, normalize)
+
+
+def _whole(t: torch.Tensor) -> torch.Tensor:
+    """t, side by side from a multiple of 16 bytes on."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
 
 
 def expert_rows(y, choice, weight, gate, up, down, bits: int, group_size: int):

@@ -140,3 +140,51 @@ def test_layer_as_before():
             expect = x.double() + rest.double().view_as(x)
             assert got.shape == x.shape
             assert (got - expect).norm() < 0.01 * expect.norm()
+
+
+def decoder_layer(bits=0, I=256, seed=0):
+    """A decoder layer with 16 routed experts and a shared one, of random weights."""
+    from mlx_sharding_amd.config import ModelConfig
+    from mlx_sharding_amd.models.deepseek_v2 import DeepseekV2DecoderLayer
+    raw = {"model_type": "deepseek_v2", "hidden_size": 512,
+           "moe_intermediate_size": I, "n_routed_experts": 16,
+           "num_experts_per_tok": 3, "n_shared_experts": 1, "intermediate_size": 256,
+           "num_attention_heads": 4, "kv_lora_rank": 64, "qk_nope_head_dim": 32,
+           "qk_rope_head_dim": 16, "v_head_dim": 32, "first_k_dense_replace": 0}
+    if bits:
+        raw["quantization"] = {"group_size": 64, "bits": bits}
+    cfg = ModelConfig.from_dict(raw)
+    torch.manual_seed(seed)
+    with torch.device("cuda"):
+        layer = DeepseekV2DecoderLayer(
+            cfg, lambda p: cfg.quantization if "switch" in p else None, "m", 0)
+    for name, p in layer.named_parameters():
+        kind = name.rsplit(".", 1)[-1]
+        if not p.is_floating_point():
+            p.data.random_(0, 2 ** 31 - 1)
+        elif "layernorm" in name:
+            p.data.normal_(1.0, 0.1)
+        else:
+            p.data.normal_(0, {"scales": 0.0025 / 16 ** (bits == 8),
+                               "biases": 0.005}.get(kind, 0.05))
+    return layer
+
+
+def one_position(rope=16):
+    angle = torch.rand(1, rope // 2, device="cuda")
+    return torch.cos(angle), torch.sin(angle)
+
+
+@pytest.mark.parametrize("B", [8, 100])
+def test_layer_takes_slices(B):
+    """Hidden states as the last token of longer ones, and off 16 bytes."""
+    layer = decoder_layer()
+    turn = one_position()
+    big = torch.randn(B, 3, 512, device="cuda").bfloat16()
+    x = big[:, -1:]
+    assert layer.mlp.decodes(x)
+    expect = layer(x.contiguous(), *turn, None)
+    assert torch.equal(layer(x, *turn, None), expect)
+    odd = torch.empty(B * 512 + 1, device="cuda").bfloat16()[1:].view(B, 1, 512)
+    odd.copy_(x)
+    assert torch.equal(layer(odd, *turn, None), expect)
