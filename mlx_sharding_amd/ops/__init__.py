@@ -646,16 +646,21 @@ def expert_rows(y, choice, weight, gate, up, down, bits: int, group_size: int):
 
 
 def _expert_stack(m, bits: int, group_size: int) -> torch.Tensor:
-    """An expert kind's matrices as moe_rows.hip reads them; packed ones are laid
-    out at their first use and kept beside the checkpoint's."""
+    """An expert kind's matrices as moe_rows.hip reads them.  Packed ones are laid
+    out at their first use, scales and biases with the words, and kept beside the
+    words, in place of the copy that the general kernels keep (repack_w4).  The copy
+    is made again where any of the three has been written or replaced since."""
     if bits == 16:
         return m[0]
     w = m[0]
-    packed = getattr(w, "_mlxs_rows", None)
-    if packed is None:
-        packed = _require_ext("moe_pack").moe_pack(*m, bits, group_size)
-        if not w.requires_grad and w.is_leaf:
-            w._mlxs_rows = packed
+    state = [(t.data_ptr(), 0 if t.is_inference() else t._version) for t in m]
+    kept = getattr(w, "_mlxs_rows", None)
+    if kept is not None and kept[0] == state:
+        return kept[1]
+    packed = _require_ext("moe_pack").moe_pack(*m, bits, group_size)
+    if not w.requires_grad and w.is_leaf and not torch.cuda.is_current_stream_capturing():
+        # what it was made of is held, so that no other tensor has its addresses
+        w._mlxs_rows = (state, packed, [t.detach() for t in m])
     return packed
 
 

@@ -188,3 +188,31 @@ def test_layer_takes_slices(B):
     odd = torch.empty(B * 512 + 1, device="cuda").bfloat16()[1:].view(B, 1, 512)
     odd.copy_(x)
     assert torch.equal(layer(odd, *turn, None), expect)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_experts_loaded_later(bits):
+    """Words, scales and biases that are loaded behind the first step, written where
+    they lie or put in place of the old ones, are what the next step takes."""
+    layer, other = decoder_layer(bits, seed=1), decoder_layer(bits, seed=2)
+    turn = one_position()
+    x = torch.randn(8, 1, 512, device="cuda").bfloat16()
+    assert layer.mlp.decodes(x)
+    before = layer(x, *turn, None)
+    theirs = dict(other.named_parameters())
+    for name, p in layer.named_parameters():
+        if "switch" not in name:
+            theirs[name].data.copy_(p)
+    for kind in ("scales", "biases", "weight"):
+        for name, p in layer.named_parameters():
+            if name.endswith("switch_mlp.down_proj." + kind):
+                p.copy_(theirs[name])
+            elif "switch" in name and name.endswith(kind):
+                p.data = theirs[name].detach().clone()
+        got = layer(x, *turn, None)
+        fresh = decoder_layer(bits, seed=3)
+        fresh.load_state_dict(layer.state_dict())
+        assert torch.equal(got, fresh(x, *turn, None))
+        assert not torch.equal(got, before)
+        before = got
+    assert torch.equal(got, other(x, *turn, None))
