@@ -218,6 +218,7 @@ class MLAAttention(nn.Module):
             q = q.clone()
         q = ext.mla_prepare(q, latent, self._w_rows[0], norm.weight, norm.eps,
                             norm.weight_offset, cos, sin, rows, pos, at)
+        cache.wrote(1)
         return ext.mla_attend(q, rows, self._w_rows[1], self.scale, pos,
                               at + 1).view(B, 1, -1)
 
@@ -246,6 +247,7 @@ class MLAAttention(nn.Module):
         cos, sin = cos.contiguous(), sin.contiguous()
         c = ext.mla_rows(latent, norm.weight, norm.eps, norm.weight_offset, cos,
                          sin, rows, at, at == 0)
+        cache.wrote(T)
         S = at + T
         if at:  # earlier rows are in the cache alone
             c = rows[:, 0, :S, : self.kv_lora_rank].contiguous()

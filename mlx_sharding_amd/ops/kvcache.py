@@ -94,12 +94,16 @@ class KVCache:
 
     def claim(self, batch: int, T: int):
         """Places for T more rows, for a kernel that writes them itself:
-        (position on the device or None, first place)."""
+        (position on the device or None, first place).  The rows count from
+        ``wrote`` on, when the kernel has been launched."""
         if self.graph_pos is not None:
             return self.graph_pos, 0
         self._ensure(batch, self.offset + T)
-        self.offset += T
-        return None, self.offset - T
+        return None, self.offset
+
+    def wrote(self, T: int):
+        if self.graph_pos is None:
+            self.offset += T
 
     def append_rope_kv(self, k: torch.Tensor, v: torch.Tensor,
                        cos: torch.Tensor, sin: torch.Tensor,
@@ -138,6 +142,7 @@ class KVCache:
         pos, at = self.claim(B, T)
         q = _ops.hip_ext().rope_qkv(q, k, v, cos.contiguous(), sin.contiguous(),
                                     self._k, self._v, pos, at)
+        self.wrote(T)
         if pos is not None:
             return q, self._k, self._v
         return q, self._k[:, :, : self.offset], self._v[:, :, : self.offset]
