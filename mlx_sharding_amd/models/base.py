@@ -22,7 +22,32 @@ from ..ops.kvcache import KVCache
 
 QuantPredicate = Callable[[str], bool]
 
+_READ = set()
 
+
+def read_in_place(cls):
+    """Marks modules whose weights a layer may read in place of a call, or which it may
+    call with more than their input."""
+    _READ.add(cls)
+    return cls
+
+
+def as_built(*modules) -> bool:
+    """Whether these are such modules and nothing depends on their calls: hooks, a
+    forward of their own.  (Subclasses are others.)"""
+    M = nn.modules.module
+    if M._global_forward_hooks or M._global_forward_pre_hooks:
+        return False
+    for m in modules:
+        if (type(m) not in _READ or m._forward_hooks or m._forward_pre_hooks
+                or "forward" in m.__dict__):
+            return False
+    return not torch.is_grad_enabled() or not (
+        M._global_backward_hooks or M._global_backward_pre_hooks
+        or any(m._backward_hooks or m._backward_pre_hooks for m in modules))
+
+
+@read_in_place
 class Linear(nn.Module):
     """Dense or MLX-affine-quantized linear, chosen per checkpoint key.
 
@@ -92,6 +117,7 @@ def project(m, x: torch.Tensor, *, norm: Optional[nn.Module] = None,
     return ops.finish(y, act, residual)
 
 
+@read_in_place
 class RMSNorm(nn.Module):
     def __init__(self, dim: int, eps: float = 1e-5, weight_offset: float = 0.0,
                  dtype: torch.dtype = torch.bfloat16):

@@ -17,10 +17,12 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, QuantConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import Linear, RMSNorm, StageModel, owned_layer_indices, project
+from .base import (Linear, RMSNorm, StageModel, as_built, owned_layer_indices, project,
+                   read_in_place)
 from .llama import LlamaMLP, _Inner
 
 
+@read_in_place
 class SwitchMLP(nn.Module):
     """Stacked routed experts: gate/up [E, I, H], down [E, H, I].
 
@@ -124,6 +126,7 @@ class _StackedLinear(nn.Module):
         return torch.stack(outs)
 
 
+@read_in_place
 class MLAAttention(nn.Module):
     def __init__(self, cfg: ModelConfig, quant_for, prefix: str):
         super().__init__()
@@ -195,6 +198,7 @@ class MLAAttention(nn.Module):
         """Whether mla_decode.hip takes this step."""
         dk = self.kv_lora_rank + self.qk_rope
         return (ops.use_native(x) and x.dtype == cache.dtype == torch.bfloat16
+                and as_built(self.kv_a_layernorm)
                 and latent.dtype == x.dtype and self.qk_nope % 32 == 0
                 and self.v_head_dim % 16 == 0 and self.qk_head_dim % 8 == 0
                 and self.kv_b_proj.bias is None
@@ -224,6 +228,8 @@ class MLAAttention(nn.Module):
 
     def _prompt_ok(self, qh, latent, cos, cache) -> bool:
         """Whether mla_rows and mla_prompt take this prompt."""
+        if not as_built(self.kv_a_layernorm):
+            return False
         norm = self.kv_a_layernorm.weight
         return (cache.graph_pos is None and ops.use_native(qh)
                 and (self.qk_nope, self.qk_rope, self.v_head_dim) == (128, 64, 128)
@@ -261,6 +267,10 @@ class MLAAttention(nn.Module):
         w = self._up_weights(device, dtype)
         self._w_uk = w[:, : self.qk_nope, :].contiguous()
         self._w_uv = w[:, self.qk_nope:, :].transpose(1, 2).contiguous()
+
+    def read(self):
+        """As in LlamaAttention."""
+        return (self.o_proj,)
 
     def forward(self, x, cos, sin, cache: Optional[KVCache],
                 norm: Optional[RMSNorm] = None,
@@ -422,6 +432,7 @@ class MLAAttention(nn.Module):
         return self._output(out.transpose(1, 2).reshape(B, T, -1), residual)
 
 
+@read_in_place
 class DeepseekV2MoE(nn.Module):
     def __init__(self, cfg: ModelConfig, quant_for, prefix: str):
         super().__init__()
@@ -459,7 +470,8 @@ class DeepseekV2MoE(nn.Module):
     def decodes(self, x) -> bool:
         """Whether ``decode`` takes these tokens."""
         m = self.switch_mlp
-        return (x.numel() <= 128 * x.shape[-1] and self.gate.bias is None
+        return (x.numel() <= 128 * x.shape[-1] and as_built(self, m, self.gate)
+                and self.gate.bias is None
                 and self._fused_gate_ok(x.numel() // x.shape[-1])
                 and ops.expert_rows_ok(x, self.gate.weight, m.up_proj.weight,
                                        m.down_proj.weight, self.top_k,
@@ -526,15 +538,19 @@ class DeepseekV2DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
     def forward(self, x, cos, sin, cache):
-        experts = isinstance(self.mlp, DeepseekV2MoE)
-        decode = experts and self.mlp.decodes(x)
-        if ops.few_tokens(x):
+        attn, mlp = self.self_attn, self.mlp
+        experts = isinstance(mlp, DeepseekV2MoE)
+        decode = experts and mlp.decodes(x)
+        if (ops.few_tokens(x) and as_built(attn, self.input_layernorm)
+                and as_built(*attn.read())
+                and (experts or (as_built(mlp) and as_built(*mlp.read())))):
             h = self.self_attn(x, cos, sin, cache, self.input_layernorm, x)
             if decode:
                 return self.mlp.decode(h, None, self.post_attention_layernorm)
             if not experts:
                 return self.mlp(h, self.post_attention_layernorm, h)
-            return h + self.mlp(self.post_attention_layernorm(h))
+            pn = self.post_attention_layernorm
+            return h + self.mlp(ops.rms_norm(h, pn.weight, pn.eps, pn.weight_offset))
         if decode:
             attn = self.self_attn(self.input_layernorm(x), cos, sin, cache)
             return self.mlp.decode(attn, x, self.post_attention_layernorm)

@@ -18,10 +18,12 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import Linear, RMSNorm, StageModel, owned_layer_indices, project
+from .base import (Linear, RMSNorm, StageModel, as_built, owned_layer_indices, project,
+                   read_in_place)
 from .llama import _Inner
 
 
+@read_in_place
 class Gemma2Attention(nn.Module):
     def __init__(self, cfg: ModelConfig, quant_for, prefix: str, layer_idx: int):
         super().__init__()
@@ -81,6 +83,7 @@ class Gemma2Attention(nn.Module):
         return self.o_proj(out.transpose(1, 2).reshape(B, T, -1))
 
 
+@read_in_place
 class Gemma2MLP(nn.Module):
     def __init__(self, cfg: ModelConfig, quant_for, prefix: str):
         super().__init__()
@@ -119,16 +122,18 @@ class Gemma2DecoderLayer(nn.Module):
         self.post_feedforward_layernorm = RMSNorm(H, eps, weight_offset=1.0)
 
     def forward(self, x, cos, sin, cache):
-        post, pre = self.post_attention_layernorm, self.pre_feedforward_layernorm
-        if ops.few_tokens(x):
-            h = ops.norm_add(self.self_attn(x, cos, sin, cache, self.input_layernorm),
-                             post, x)
+        first, post = self.input_layernorm, self.post_attention_layernorm
+        pre, last = self.pre_feedforward_layernorm, self.post_feedforward_layernorm
+        if not as_built(first, post, pre, last):
+            h = x + post(self.self_attn(first(x), cos, sin, cache))
+            return h + last(self.mlp(pre(h)))
+        if ops.few_tokens(x) and as_built(self.self_attn, self.mlp):
+            h = ops.norm_add(self.self_attn(x, cos, sin, cache, first), post, x)
             y = self.mlp(h, pre)
         else:
-            h, y = ops.norm_add(
-                self.self_attn(self.input_layernorm(x), cos, sin, cache), post, x, pre)
+            h, y = ops.norm_add(self.self_attn(first(x), cos, sin, cache), post, x, pre)
             y = self.mlp(y)
-        return ops.norm_add(y, self.post_feedforward_layernorm, h)
+        return ops.norm_add(y, last, h)
 
 
 class Gemma2StageModel(StageModel):

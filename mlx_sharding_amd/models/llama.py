@@ -16,9 +16,11 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import Linear, RMSNorm, StageModel, owned_layer_indices, project
+from .base import (Linear, RMSNorm, StageModel, as_built, owned_layer_indices, project,
+                   read_in_place)
 
 
+@read_in_place
 class LlamaAttention(nn.Module):
     def __init__(self, cfg: ModelConfig, quant_for, prefix: str):
         super().__init__()
@@ -38,6 +40,12 @@ class LlamaAttention(nn.Module):
         self.v_proj = Linear(H, self.n_kv_heads * self.head_dim, q("v_proj"), qkv_bias)
         self.o_proj = Linear(self.n_heads * self.head_dim, H, q("o_proj"), o_bias)
         self._fused_qkv = None  # set by fuse_model()
+
+    def read(self):
+        """Modules that are read in place of a call where few tokens come."""
+        if self._fused_qkv is not None:
+            return (self.o_proj,)
+        return self.q_proj, self.k_proj, self.v_proj, self.o_proj
 
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                 cache: Optional[KVCache], norm: Optional[RMSNorm] = None,
@@ -84,6 +92,7 @@ class LlamaAttention(nn.Module):
         return self.o_proj(out)
 
 
+@read_in_place
 class LlamaMLP(nn.Module):
     def __init__(self, cfg: ModelConfig, quant_for, prefix: str):
         super().__init__()
@@ -95,10 +104,15 @@ class LlamaMLP(nn.Module):
         self.down_proj = Linear(I, H, q("down_proj"))
         self._fused_gu = None  # set by fuse_model()
 
+    def read(self):
+        """As in LlamaAttention."""
+        return (self.down_proj,)
+
     def forward(self, x: torch.Tensor, norm: Optional[RMSNorm] = None,
                 residual: Optional[torch.Tensor] = None) -> torch.Tensor:
         """norm, residual: as in LlamaAttention."""
-        if self._fused_gu is not None and (norm is not None or ops.few_tokens(x)):
+        if self._fused_gu is not None and (
+                norm is not None or (ops.few_tokens(x) and as_built(self.down_proj))):
             y = project(self._fused_gu, x, norm=norm, act="silu")
             return project(self.down_proj, y, residual=residual)
         if norm is not None:
@@ -122,7 +136,9 @@ class LlamaDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
     def forward(self, x, cos, sin, cache):
-        if ops.few_tokens(x):
+        attn, mlp = self.self_attn, self.mlp
+        if (ops.few_tokens(x) and as_built(attn, mlp, self.input_layernorm)
+                and as_built(*attn.read(), *mlp.read())):
             h = self.self_attn(x, cos, sin, cache, self.input_layernorm, x)
             return self.mlp(h, self.post_attention_layernorm, h)
         attn = self.self_attn(self.input_layernorm(x), cos, sin, cache)
