@@ -9,6 +9,7 @@ RoPE on the qk_rope slice with mscale-adjusted softmax scale.
 
 from __future__ import annotations
 
+import os
 from typing import Dict, List, Optional, Tuple
 
 import torch
@@ -61,7 +62,6 @@ class SwitchMLP(nn.Module):
             # measured 5334 vs 5005 tok/s end to end) — packed is the
             # decode default; MLXS_AMD_MOE_RESIDENT=1 restores the old
             # resident-bf16 path for A/B
-            import os
             if os.environ.get("MLXS_AMD_MOE_RESIDENT"):
                 dense = self.resident_dense()
                 if dense is not None:
@@ -468,8 +468,11 @@ class DeepseekV2MoE(nn.Module):
         return (16, 128) if q is None else (q.bits, q.group_size)
 
     def decodes(self, x) -> bool:
-        """Whether ``decode`` takes these tokens."""
+        """Whether ``decode`` takes these tokens: not with MLXS_AMD_MOE_RESIDENT, which
+        asks for another kernel (SwitchMLP.forward_subs)."""
         m = self.switch_mlp
+        if m.quant is not None and os.environ.get("MLXS_AMD_MOE_RESIDENT"):
+            return False
         return (x.numel() <= 128 * x.shape[-1] and as_built(self, m, self.gate)
                 and self.gate.bias is None
                 and self._fused_gate_ok(x.numel() // x.shape[-1])
