@@ -1311,7 +1311,8 @@ __global__ __launch_bounds__(512, 2) void delta_walk_fixed_kernel(
 
     for (int buf = 0; c < c_end; ++c, buf ^= 1) {
       const int ahead = min(cn + 1, c_end - 1);
-      const int2 then = reinterpret_cast<const int2*>(chunks)[ahead + nought];
+      const int* then = chunks + 2 * (ahead + nought);  // at any multiple of 4 bytes
+      const int then_row = then[0], then_len = then[1];
       const float* k = kl + buf * KW;
 
       f32x4 acc[CT];
@@ -1486,8 +1487,8 @@ __global__ __launch_bounds__(512, 2) void delta_walk_fixed_kernel(
       i0 = j0;
       len = jl;
       cn = ahead;
-      j0 = __builtin_amdgcn_readfirstlane(then.x) - tok_base;
-      jl = __builtin_amdgcn_readfirstlane(then.y);
+      j0 = __builtin_amdgcn_readfirstlane(then_row) - tok_base;
+      jl = __builtin_amdgcn_readfirstlane(then_len);
     }
     if (!keeps) return;
 #pragma unroll

@@ -56,3 +56,31 @@ def test_many_as_alone(D, heads, channel):
         # the projections may sum in another order: a few roundings of 2^-24 over 64
         # terms, carried through a state that forgets
         assert (got - want).abs().max() <= 1e-4 * want.abs().max()
+
+
+@pytest.mark.parametrize("words", [0, 1])
+def test_chunks_at_any_word(words, monkeypatch):
+    """A batch's index arrays lie behind one another in one buffer: the list of chunks
+    begins at any multiple of four bytes."""
+    dev = torch.device("cuda")
+    torch.manual_seed(words)
+    with dev:
+        m = GatedDelta(64, 4, 2, 64, 128, 4, 1e-6, dtype=torch.float32, ranks=None,
+                       gate="silu")
+    for p in m.parameters():
+        p.data.normal_(0, 0.1)
+    m.prepare()
+    rows = [torch.randn(n, 64, device=dev) for n in LENS]
+    want = _run(m, rows, torch.float32)
+    init = RaggedBatch.__init__
+
+    def moved(self, *args):
+        init(self, *args)
+        n = self.chunks.numel()
+        room = torch.empty(n + 2, dtype=torch.int32, device=dev)[words: words + n]
+        self.chunks = room.view(-1, 2).copy_(self.chunks)
+        assert self.chunks.data_ptr() % 8 == 4 * words
+
+    monkeypatch.setattr(RaggedBatch, "__init__", moved)
+    for got, expect in zip(_run(m, rows, torch.float32), want):
+        assert torch.equal(got, expect)
