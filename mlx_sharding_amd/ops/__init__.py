@@ -260,13 +260,6 @@ def _plain(t: torch.Tensor) -> bool:
             and not _watched())
 
 
-def few_rows(x: torch.Tensor, weight: torch.Tensor, alone: bool = False) -> bool:
-    """Whether x W^T runs on linear_few.hip (linear_few_takes there says when);
-    ``alone``: with nothing taken along."""
-    ext = _few_ext() if _use_hip(x) and _plain(x) and _plain(weight) else None
-    return ext is not None and ext.linear_few_takes(x, weight, alone)
-
-
 def _few_ext():
     if _load_ext() is not None:
         return _EXT

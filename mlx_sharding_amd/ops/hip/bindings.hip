@@ -1233,8 +1233,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill_shape_ok", [](int64_t dk, int64_t dv) {
     return attn_prefill_supported((int)dk, (int)dv);
   });
-  m.def("linear_few", &linear_few);
-  m.def("linear_few_takes", &linear_few_takes);
   m.def("linear_few_try", &linear_few_try);
   m.def("mla_rows", &mla_rows);
   m.def("mla_prompt", &mla_prompt);

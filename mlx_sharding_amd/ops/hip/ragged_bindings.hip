@@ -817,8 +817,6 @@ Tensor cap_logits(Tensor z, double scale, double limit) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("glu", &glu);
-  m.def("linear_few", &linear_few);
-  m.def("linear_few_takes", &linear_few_takes);
   m.def("linear_few_try", &linear_few_try);
   m.def("clamped_glu", &clamped_glu, py::arg("gate"), py::arg("up"),
         py::arg("limit"), py::arg("alpha"), py::arg("gate_bias") = py::none(),

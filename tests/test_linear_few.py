@@ -9,6 +9,11 @@ import torch.nn.functional as F
 from mlx_sharding_amd import ops
 
 
+def taken(x, w):
+    """Whether ops.linear runs x W^T on the kernel."""
+    return ops._linear_few(x, w) is not None
+
+
 def make(M, O, K, act, wide):
     g = torch.Generator().manual_seed(M + O + K)
     new = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()  # noqa: E731
@@ -31,7 +36,7 @@ def test_edges(M, O, K):
     norm, bias, unit, residual."""
     for act in (None, "silu", "gelu_tanh"):
         x, w, norm, bias, res = make(M, O, K, act, wide=K % 64 == 0)
-        assert ops.few_rows(x, w)
+        assert taken(x, w)
         for normed in (False, True):
             for rest in (False, True):
                 b, r = (bias, res) if rest else (None, None)
@@ -66,7 +71,7 @@ def test_same_as_separate_kernels():
     """What the projection takes along, beside the kernels it stands for."""
     x, w, norm, bias, _ = make(16, 512, 256, None, wide=True)
     several = torch.cat([x] * 5)                  # too many rows: separate
-    assert not ops.few_rows(several, w)
+    assert not taken(several, w)
     norm = types.SimpleNamespace(
         weight=norm.weight, eps=1e-5, weight_offset=1.0)
     one = ops.project(x, w, bias, act="silu")
@@ -85,9 +90,9 @@ def test_other_forms_keep_the_library():
     at = torch.randn(6 * 64 + 1, device="cuda").bfloat16()  # rows off 16 bytes
     odd = at[1:].view(2, 3, 64)
     odd.copy_(x)
-    assert not ops.few_rows(odd, w) and close(ops.linear(odd, w))
+    assert not taken(odd, w) and close(ops.linear(odd, w))
     turned = w.t().contiguous().t()                 # columns side by side
-    assert not ops.few_rows(x, turned) and close(ops.linear(x, turned))
+    assert not taken(x, turned) and close(ops.linear(x, turned))
     assert ops.linear(x.float(), w.float()).dtype == torch.float32
     assert ops.linear(x[:, :0], w).shape == (2, 0, 24)
     # what is differentiated or mapped
@@ -191,5 +196,5 @@ def test_autocast_names_the_type(rows):
 
 def test_cpu_tensors_keep_torch():
     x, w = torch.randn(2, 64).bfloat16(), torch.randn(24, 64).bfloat16()
-    assert not ops.few_rows(x, w) and not ops.few_tokens(x)
+    assert not ops.few_tokens(x)
     assert torch.equal(ops.linear(x, w), F.linear(x, w))
