@@ -51,8 +51,8 @@ def as_built(*modules) -> bool:
 class Linear(nn.Module):
     """Dense or MLX-affine-quantized linear, chosen per checkpoint key.
 
-    Dense path → F.linear (hipBLASLt on ROCm).  Quantized path → the
-    w4a16/w8a16 dequant-GEMM op.  Parameter names (weight/scales/biases)
+    Dense path → ops.linear: linear_few.hip for up to 64 rows, else the
+    library.  Quantized path → the w4a16/w8a16 dequant-GEMM op.  Parameter names (weight/scales/biases)
     match the MLX checkpoint layout so pre-quantized checkpoints load
     directly (/root/reference/shard/utils.py:54-65 predicate: a
     `.scales` key exists for the module).

@@ -7,10 +7,11 @@ Policy (deliberate, per the MI355X-native design):
     native path.  Set ``MLXS_AMD_FORCE_TORCH=1`` only for debugging.
   * On CPU tensors the torch reference implementations run (the
     reference's CPU plumbing config needs no GPU code).
-  * Plain dense GEMMs (qkv/o projections, dense MLP matmuls, prefill
-    QK^T/PV batch matmuls) go through torch.matmul → hipBLASLt/rocBLAS,
-    which is the intended library path; everything fused/nonstandard
-    (norms, rope, decode attention, w4a16, MoE gather) is ours.
+  * Plain dense GEMMs of more than 64 rows (qkv/o projections, dense MLP
+    matmuls) go through torch.matmul → hipBLASLt/rocBLAS, which is the
+    intended library path.  Everything else is ours: products of up to 64
+    rows, with the norm, unit and residual around them (linear_few.hip),
+    norms, rope, attention, w4a16, routed experts.
 """
 
 from __future__ import annotations
@@ -315,10 +316,10 @@ def few_tokens(x: torch.Tensor) -> bool:
 
 
 def linear(x, weight, bias=None):
-    """Dense linear; up to 64 rows run on linear_few.hip.  The MFMA decode GEMV (MLXS_AMD_DENSE_GEMV=1) was
-    a NEGATIVE result at batch-64 decode shapes: hipBLASLt's small-GEMM
-    kernels run ~13 us in-graph and the split-K fp32-atomic traffic
-    (M*O*4*nk bytes) rivals the weight bytes on small-O projections
+    """Dense linear; up to 64 rows run on linear_few.hip where it takes them.  The MFMA
+    decode GEMV (MLXS_AMD_DENSE_GEMV=1) was a NEGATIVE result at batch-64 decode shapes:
+    hipBLASLt's small-GEMM kernels run ~13 us in-graph and the split-K fp32-atomic
+    traffic (M*O*4*nk bytes) rivals the weight bytes on small-O projections
     (docs/PERFORMANCE.md).  Kept for shape-specific re-tuning."""
     gemv = os.environ.get("MLXS_AMD_DENSE_GEMV")
     if not gemv and x.is_cuda and weight.shape[-1] < 16384:

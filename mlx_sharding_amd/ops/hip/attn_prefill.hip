@@ -104,10 +104,10 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
   constexpr int KP = DK / 8, VP = DV / 8;      // pieces of a row
   constexpr int NK = DK / 16, NB = KT / 32, ND = (DV + 31) / 32;
   constexpr int KB = KT * DK * 2, VB = KT * DV * 2;
-  // a lane of the columns behind DV = 16 reads past its row
-  // The last pieces of queries of 256 lie there, too: they and the sums leave too few
+  // The last pieces of queries of 256 lie in LDS: they and the sums leave too few
   // registers to read keys and values ahead of their products.
   constexpr int QL = DK == 256 ? 4 : 0;
+  // a lane of the columns behind DV = 16 reads past its row
   __shared__ __attribute__((aligned(16))) char smem[2 * (KB + VB) +
                                                     AP_WAVES * QL * 1024 +
                                                     (DV < 32 ? 64 : 0)];

@@ -371,8 +371,6 @@ void mla_append_kv(torch::Tensor kvh, torch::Tensor kpe, torch::Tensor kcache,
                        T, nh, nope, vd, rope, Scap, kpe_rs, cur_stream());
 }
 
-// q [B, Hq, 1, Dk]; k/v: cache views [B, Hkv, S, D] with row-contiguous
-// last dim over a [B, Hkv, Scap, D] buffer.
 // Slices of the keys for the tile kernel: up to 512 blocks, two a CU, which are
 // all at work at once, and no slice under one tile.  256 blocks leave half of the
 // loads in flight unused (5 sequences of 5004 keys, 8 heads of 256: 68 us, 45 with
@@ -384,6 +382,8 @@ static int decode_slices(long pairs, long span, int tile) {
                          (span + tile - 1) / tile}));
 }
 
+// q [B, Hq, 1, Dk]; k/v: cache views [B, Hkv, S, D] with row-contiguous
+// last dim over a [B, Hkv, Scap, D] buffer.
 torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                           double scale, double softcap, int64_t window,
                           c10::optional<torch::Tensor> pos) {
@@ -952,8 +952,6 @@ torch::Tensor moe_w4_mfma(torch::Tensor x, torch::Tensor wq,
   return y;
 }
 
-// Fused fp16-dequant gate+up+SiLU over repacked quant words.
-// x [N, H] fp16; gq/uq [E, I, H*bits/32] repacked; scales/biases bf16.
 // -- routed experts of a decoding step (moe_rows.hip) -----------------------
 
 static void check_rows(const torch::Tensor& t, const char* name, long n, long w) {
@@ -1081,9 +1079,9 @@ torch::Tensor moe_rows(torch::Tensor x, torch::Tensor choice,
                 choice.data_ptr<int>(), weight.data_ptr<float>(), (int)P,
                 (int)choice.size(1), (int)g.E, (int)g.O, (int)g.K, tiles(g.O)};
   launch_moe_rows(&a, (int)bits, (int)gs, true, cur_stream());
-  a = MoeRowsArgs{h.data_ptr(), d.w, nullptr, y.data_ptr(), choice.data_ptr<int>(), weight.data_ptr<float>(),
-                  (int)P, (int)choice.size(1), (int)d.E, (int)d.O, (int)d.K,
-                  tiles(d.O)};
+  a = MoeRowsArgs{h.data_ptr(), d.w, nullptr, y.data_ptr(), choice.data_ptr<int>(),
+                  weight.data_ptr<float>(), (int)P, (int)choice.size(1), (int)d.E,
+                  (int)d.O, (int)d.K, tiles(d.O)};
   launch_moe_rows(&a, (int)bits, (int)gs, false, cur_stream());
   return y;
 }
@@ -1105,6 +1103,8 @@ torch::Tensor moe_combine(torch::Tensor rows, c10::optional<torch::Tensor> h,
   return out;
 }
 
+// Fused fp16-dequant gate+up+SiLU over repacked quant words.
+// x [N, H] fp16; gq/uq [E, I, H*bits/32] repacked; scales/biases bf16.
 torch::Tensor moe_w4f16_gateup(torch::Tensor x, torch::Tensor gq,
                                torch::Tensor uq, torch::Tensor gsc,
                                torch::Tensor gbi, torch::Tensor usc,

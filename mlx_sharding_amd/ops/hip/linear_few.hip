@@ -22,7 +22,6 @@
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-
 struct LinearFewArgs {
   const __bf16 *x, *w, *bias, *res, *norm;
   __bf16* y;
@@ -37,39 +36,39 @@ enum { LF_PLAIN = 0, LF_SILU = 1, LF_GELU = 2 };
 template <int ACT>
 __device__ __forceinline__ void finish_columns(const LinearFewArgs& a, int row,
                                                int col, const f32x4* v) {
-      float o[4];
-  #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int at = min(col + j, a.O - 1);
-        float f = v[0][j];
-        if (ACT) {
-          float up = v[1][j];
-          if (a.bias) {
-            f += (float)a.bias[at];
-            up += (float)a.bias[a.O + at];
-          }
-          if (ACT == LF_SILU) {
-            f = f / (1.0f + __expf(-f)) * up;
-          } else {
-            const float z = 0.7978845608028654f * (f + 0.044715f * f * f * f);
-            f = 0.5f * f * (1.0f + tanhf(z)) * up;
-          }
-        } else if (a.bias) {
-          f += (float)a.bias[at];
-        }
-        if (a.res) f += (float)a.res[(long)row * a.ldr + at];
-        o[j] = f;
+  float o[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int at = min(col + j, a.O - 1);
+    float f = v[0][j];
+    if (ACT) {
+      float up = v[1][j];
+      if (a.bias) {
+        f += (float)a.bias[at];
+        up += (float)a.bias[a.O + at];
       }
-      __bf16* y = a.y + (long)row * a.ldy + col;
-      if (col + 3 < a.O && a.ldy % 4 == 0) {
-        typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-        *reinterpret_cast<bf16x4_t*>(y) =
-            bf16x4_t{(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
+      if (ACT == LF_SILU) {
+        f = f / (1.0f + __expf(-f)) * up;
       } else {
-  #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (col + j < a.O) y[j] = (__bf16)o[j];
+        const float z = 0.7978845608028654f * (f + 0.044715f * f * f * f);
+        f = 0.5f * f * (1.0f + tanhf(z)) * up;
       }
+    } else if (a.bias) {
+      f += (float)a.bias[at];
+    }
+    if (a.res) f += (float)a.res[(long)row * a.ldr + at];
+    o[j] = f;
+  }
+  __bf16* y = a.y + (long)row * a.ldy + col;
+  if (col + 3 < a.O && a.ldy % 4 == 0) {
+    typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<bf16x4_t*>(y) =
+        bf16x4_t{(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (col + j < a.O) y[j] = (__bf16)o[j];
+  }
 }
 
 // RT tiles of 16 rows of W; with a gated unit half of them are the gate's, the
@@ -77,7 +76,7 @@ __device__ __forceinline__ void finish_columns(const LinearFewArgs& a, int row,
 template <int RT, int ACT, bool NORM, int NW, int U>
 __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
     const LinearFewArgs a) {
-    __shared__ __attribute__((aligned(16))) f32x4 red[NW][RT][WAVE];
+  __shared__ __attribute__((aligned(16))) f32x4 red[NW][RT][WAVE];
   __shared__ float squares[NORM ? NW : 1][WAVE];
 
   const int lane = threadIdx.x & (WAVE - 1);

@@ -9,8 +9,8 @@
 // microsecond; as separate products, copies, rotations and norms they were twelve
 // kernels of 4 to 13 us.  A block takes 16 tokens of one head, a wave 16 rows of
 // its matrix, read with the contraction contiguous ([head, row, contraction]).
-// Measured: a step of one sequence through 24 layers of 16 heads 473 -> 385 us, of 64
-// sequences 943 -> 784.
+// Measured: a step of one sequence through four layers of 16 heads, experts and a
+// vocabulary of 12800 473 -> 385 us, of 64 sequences 943 -> 784.
 
 #include "mla_decode.h"
 
