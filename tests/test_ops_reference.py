@@ -274,3 +274,16 @@ def test_fp16_or_trick_dequant_exact():
         ref = s * q + b
         tol = max(abs(ref).max(), 8 * s) * 2 ** -9
         assert np.abs(got - ref).max() < max(tol, 2 * abs(b - float(np.float16(b))))
+
+
+def test_experts_by_library_products_on_cpu():
+    """The route of many tokens, with sizes that the GPU has a kernel for."""
+    from mlx_sharding_amd import ops
+    g = torch.Generator().manual_seed(3)
+    new = lambda *s: (torch.randn(*s, generator=g) * 0.05).bfloat16()  # noqa: E731
+    gate, up, down = new(4, 128, 128), new(4, 128, 128), new(4, 128, 128)
+    x, w = torch.randn(200, 128, generator=g).bfloat16(), torch.rand(200, 2, generator=g)
+    idx = torch.randint(0, 4, (200, 2), generator=g)
+    y = ops._moe_prefill_gemm(x, gate, up, down, w, idx).float()
+    expect = ref.grouped_expert_mlp(x, gate, up, down, w, idx).float()
+    assert (y - expect).norm() < 0.02 * expect.norm()
