@@ -428,7 +428,7 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
   __shared__ __attribute__((aligned(16))) char smem[2 * (KB + VB)];
   __shared__ float sc[2][HALVES][KT][16];
 
-  const int S = (int)min(a.s_ptr ? (long)*a.s_ptr + 1 : (long)a.S, a.cap);
+  const int S = a.s_ptr ? (int)min((long)*a.s_ptr + 1, a.cap) : a.S;
   const int b = blockIdx.x / a.Hkv, hk = blockIdx.x % a.Hkv;
   const int G = a.Hq / a.Hkv;
   const int lane = threadIdx.x & (WAVE - 1);

@@ -116,6 +116,18 @@ def test_decode_edges(Hq, Hkv, Dk, Dv, captured):
             assert bool(((out - expect).abs() <= bound).all()), (S, cap, window)
 
 
+@pytest.mark.parametrize("Hq,Hkv,Dk,Dv", [(8, 4, 128, 128), (8, 2, 64, 64)])
+def test_heads_of_one_memory(Hq, Hkv, Dk, Dv):
+    """Key and value heads that are one in memory, side by side in name only."""
+    torch.manual_seed(3)
+    q = torch.randn(1, Hq, 1, Dk, device="cuda").bfloat16()
+    k, v = (cached(1, 1, 300, D, 10).expand(1, Hkv, 300, D) for D in (Dk, Dv))
+    out = ext().attn_decode(q, k, v, 0.1, 0.0, 0, None).double()
+    expect, size = attention(q, k, v, 0.1, 0.0, 0, 299)
+    bound = 2.0 ** -8 * expect.abs() + 2.0 ** -13 * size + 1e-6
+    assert bool(((out - expect).abs() <= bound).all())
+
+
 def opposed(Hq, Hkv, Dk, Dv, S, step):
     """q, k, v whose values come in pairs of opposite sign, with scores (at a scale of
     1) that differ by twice ``step``: what is left of a pair's weights is their
