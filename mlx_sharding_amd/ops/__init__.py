@@ -509,7 +509,7 @@ def _tiles_ok(x, gate_w, up_w, down_w) -> bool:
     E, I, H = gate_w.shape
     return (x.dtype == torch.bfloat16 and use_native(x) and H % 64 == 0 and I % 64 == 0
             and min(H, I) >= 128 and E <= 1024 and H * I < 2 ** 31
-            and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= H
             and x.shape[0] * x.stride(0) < 2 ** 31 and x.data_ptr() % 16 == 0
             and all(w.device == x.device and w.dtype == torch.bfloat16
                     and w.is_contiguous() and _plain(w)

@@ -72,6 +72,10 @@ def test_other_sizes_take_the_general_path():
     # gate, up, unit and output are rounded to bf16 there
     scale = general.float().abs().max()
     assert (tiles.float() - general.detach().float()).abs().max() <= 2.0 ** -5 * scale
+    one = x[:1].expand(N, H)  # one row in memory
+    many = ops.grouped_expert_mlp(one, *stacks, w, choice)
+    expect = ops.grouped_expert_mlp(one.contiguous(), *stacks, w, choice).float()
+    assert (many.float() - expect).abs().max() <= 2.0 ** -5 * expect.abs().max()
     odd = [s[:, :100].contiguous() for s in stacks[:2]] + [stacks[2][..., :100].contiguous()]
     assert not ops._tiles_ok(x, *odd)
     assert ops.grouped_expert_mlp(x, *odd, w, choice).shape == (N, H)
