@@ -39,8 +39,10 @@ def as_built(*modules) -> bool:
     if M._global_forward_hooks or M._global_forward_pre_hooks:
         return False
     for m in modules:
-        if (type(m) not in _READ or m._forward_hooks or m._forward_pre_hooks
-                or "forward" in m.__dict__):
+        if type(m) not in _READ:
+            return False
+        own = m.__dict__
+        if own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own:
             return False
     return not torch.is_grad_enabled() or not (
         M._global_backward_hooks or M._global_backward_pre_hooks

@@ -270,7 +270,7 @@ class MLAAttention(nn.Module):
 
     def read(self):
         """As in LlamaAttention."""
-        return (self.o_proj,)
+        return (self._modules["o_proj"],)
 
     def forward(self, x, cos, sin, cache: Optional[KVCache],
                 norm: Optional[RMSNorm] = None,
@@ -541,28 +541,26 @@ class DeepseekV2DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
     def forward(self, x, cos, sin, cache):
-        attn, mlp = self.self_attn, self.mlp
+        attn, mlp, norm = self.self_attn, self.mlp, self.input_layernorm
         experts = isinstance(mlp, DeepseekV2MoE)
         decode = experts and mlp.decodes(x)
-        if (ops.few_tokens(x) and as_built(attn, self.input_layernorm)
+        if (ops.few_tokens(x) and as_built(attn, norm)
                 and as_built(*attn.read())
                 and (experts or (as_built(mlp) and as_built(*mlp.read())))):
-            h = self.self_attn(x, cos, sin, cache, self.input_layernorm, x)
+            h = attn(x, cos, sin, cache, norm, x)
             if decode:
-                return self.mlp.decode(h, None, self.post_attention_layernorm)
+                return mlp.decode(h, None, self.post_attention_layernorm)
             if not experts:
-                return self.mlp(h, self.post_attention_layernorm, h)
+                return mlp(h, self.post_attention_layernorm, h)
             pn = self.post_attention_layernorm
-            return h + self.mlp(ops.rms_norm(h, pn.weight, pn.eps, pn.weight_offset))
+            return h + mlp(ops.rms_norm(h, pn.weight, pn.eps, pn.weight_offset))
+        attn, pn = attn(norm(x), cos, sin, cache), self.post_attention_layernorm
         if decode:
-            attn = self.self_attn(self.input_layernorm(x), cos, sin, cache)
-            return self.mlp.decode(attn, x, self.post_attention_layernorm)
-        attn = self.self_attn(self.input_layernorm(x), cos, sin, cache)
+            return mlp.decode(attn, x, pn)
         # fused: h = x + attn; y = rms_norm(h) in one kernel
-        pn = self.post_attention_layernorm
         y, h = ops.rms_norm_residual(attn, x, pn.weight, pn.eps,
                                      pn.weight_offset)
-        return h + self.mlp(y)
+        return h + mlp(y)
 
 
 class DeepseekV2StageModel(StageModel):

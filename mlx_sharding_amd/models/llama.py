@@ -43,9 +43,10 @@ class LlamaAttention(nn.Module):
 
     def read(self):
         """Modules that are read in place of a call where few tokens come."""
+        m = self._modules
         if self._fused_qkv is not None:
-            return (self.o_proj,)
-        return self.q_proj, self.k_proj, self.v_proj, self.o_proj
+            return (m["o_proj"],)
+        return m["q_proj"], m["k_proj"], m["v_proj"], m["o_proj"]
 
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                 cache: Optional[KVCache], norm: Optional[RMSNorm] = None,
@@ -106,7 +107,7 @@ class LlamaMLP(nn.Module):
 
     def read(self):
         """As in LlamaAttention."""
-        return (self.down_proj,)
+        return (self._modules["down_proj"],)
 
     def forward(self, x: torch.Tensor, norm: Optional[RMSNorm] = None,
                 residual: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -136,17 +137,17 @@ class LlamaDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps)
 
     def forward(self, x, cos, sin, cache):
-        attn, mlp = self.self_attn, self.mlp
-        if (ops.few_tokens(x) and as_built(attn, mlp, self.input_layernorm)
+        attn, mlp, norm = self.self_attn, self.mlp, self.input_layernorm
+        if (ops.few_tokens(x) and as_built(attn, mlp, norm)
                 and as_built(*attn.read(), *mlp.read())):
-            h = self.self_attn(x, cos, sin, cache, self.input_layernorm, x)
-            return self.mlp(h, self.post_attention_layernorm, h)
-        attn = self.self_attn(self.input_layernorm(x), cos, sin, cache)
+            h = attn(x, cos, sin, cache, norm, x)
+            return mlp(h, self.post_attention_layernorm, h)
+        attn = attn(norm(x), cos, sin, cache)
         # fused: h = x + attn; y = rms_norm(h) in one kernel
         pn = self.post_attention_layernorm
         y, h = ops.rms_norm_residual(attn, x, pn.weight, pn.eps,
                                      pn.weight_offset)
-        return h + self.mlp(y)
+        return h + mlp(y)
 
 
 class _Inner(nn.Module):

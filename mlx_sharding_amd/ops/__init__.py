@@ -307,12 +307,9 @@ def finish(y, act=None, residual=None):
 
 def few_tokens(x: torch.Tensor) -> bool:
     """Whether a layer's projections on x take what lies between them along
-    (``project``).  Not where another kernel is asked for by MLXS_AMD_DENSE_GEMV or
-    MLXS_AMD_GEMM64 (``linear``)."""
+    (``project``)."""
     return (x.dtype == torch.bfloat16 and 0 < x.numel() <= _FEW_ROWS * x.shape[-1]
-            and use_native(x) and _plain(x)
-            and not (os.environ.get("MLXS_AMD_DENSE_GEMV")
-                     or os.environ.get("MLXS_AMD_GEMM64")))
+            and use_native(x) and _plain(x))
 
 
 def linear(x, weight, bias=None):

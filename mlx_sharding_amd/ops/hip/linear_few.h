@@ -6,7 +6,10 @@
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+
+#include <cstdlib>
 
 extern "C" void launch_linear_few(const void*, const void*, const void*,
                                   const void*, const void*, void*, int, int, int,
@@ -58,7 +61,8 @@ static torch::Tensor linear_few(torch::Tensor x, torch::Tensor w,
     r = residual->data_ptr();
     ldr = residual->stride(0);
   }
-  const c10::DeviceGuard guard(x.device());  // and its current stream
+  c10::OptionalDeviceGuard guard;  // and the device's current stream
+  if (x.get_device() != c10::hip::current_device()) guard.reset_device(x.device());
   auto y = torch::empty({M, O}, x.options());
   launch_linear_few(x.data_ptr(), w.data_ptr(), b, r, n, y.data_ptr(), M, O, K,
                     x.stride(0), w.stride(0), ldr, O, (float)eps, (float)offset,
@@ -84,6 +88,15 @@ static bool linear_few_recorded() {
   return c10::impl::tls_local_dispatch_key_set().included_.has_any(recorders);
 }
 
+// Whether the environment asks for another kernel for products of a contraction K.
+static bool linear_few_other(long K) {
+  auto set = [](const char* name) {
+    const char* v = std::getenv(name);
+    return v && *v;
+  };
+  return set("MLXS_AMD_DENSE_GEMV") || (K >= 16384 && set("MLXS_AMD_GEMM64"));
+}
+
 // Whether x w^T runs here: up to 64 bf16 rows that begin, as w's, at whole 16-byte
 // vectors.  A contraction above 8192 for 8 rows, or into 4096: 8 rows of 14336 into
 // 4096 take 24.6 us here and 26.6 in the library, 32 rows 30.4 and 30.5, 64 rows 40.1
@@ -99,7 +112,7 @@ static bool linear_few_takes(const torch::Tensor& x, const torch::Tensor& w,
       at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16)
     return false;  // a product of another type
   const long O = w.size(0), K = w.size(1);
-  if (O < 1 || K < 32 || K % 32 || x.size(-1) != K) return false;
+  if (O < 1 || K < 32 || K % 32 || x.size(-1) != K || linear_few_other(K)) return false;
   const long rows = x.numel() / K;
   if (rows < 1 || rows > 64 || (K > 8192 && rows > 8 && O > 4096) ||
       (alone && rows > 32 && O * K > 1 << 25))
