@@ -278,11 +278,13 @@ torch::Tensor rope_qkv(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   auto whole = [](const torch::Tensor& t) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
+  // from one token to the next
+  auto row = [&](const torch::Tensor& t) { return t.stride(T == 1 ? 0 : 1); };
   for (const auto& t : {q, k, v}) {
     check_bf16(t, "operand");
     TORCH_CHECK(t.dim() == 4 && t.size(0) == B && t.size(1) == T && t.size(3) == D &&
-                    t.stride(3) == 1 && t.stride(2) == D && t.stride(1) % 8 == 0 &&
-                    (B == 1 || t.stride(0) == T * t.stride(1)) && whole(t), "rows");
+                    t.stride(3) == 1 && t.stride(2) == D && row(t) % 8 == 0 &&
+                    (B == 1 || T == 1 || t.stride(0) == T * row(t)) && whole(t), "rows");
   }
   TORCH_CHECK(D >= 16 && D % 16 == 0 && B >= 1 && T >= 1 && v.size(2) == Hkv &&
                   (q.size(2) + 3 * Hkv) * D < (1L << 30), "sizes");
@@ -306,7 +308,7 @@ torch::Tensor rope_qkv(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   launch_rope_qkv(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr<float>(),
                   sin.data_ptr<float>(), out.data_ptr(), kcache.data_ptr(),
                   vcache.data_ptr(), pp, pos0, B * T, (int)T, (int)q.size(2), (int)Hkv,
-                  (int)D, kcache.size(2), q.stride(1), k.stride(1), v.stride(1),
+                  (int)D, kcache.size(2), row(q), row(k), row(v),
                   cur_stream());
   return out;
 }

@@ -134,9 +134,12 @@ class KVCache:
         if not (D % 16 == 0 and self.k_head_dim == self.v_head_dim == D
                 and self.dtype == torch.bfloat16 and cos.dtype == torch.float32
                 and all(t.dtype == torch.bfloat16 and t.stride(3) == 1
-                        and t.stride(2) == D and t.stride(1) % 8 == 0
-                        and (B == 1 or t.stride(0) == T * t.stride(1))
-                        and t.data_ptr() % 16 == 0 for t in (q, k, v))):
+                        and t.stride(2) == D and t.data_ptr() % 16 == 0
+                        # one token each: the stride between tokens says nothing
+                        and (t.stride(0) % 8 == 0 if T == 1 else
+                             t.stride(1) % 8 == 0
+                             and (B == 1 or t.stride(0) == T * t.stride(1)))
+                        for t in (q, k, v))):
             q = _ops.apply_rope(q, cos, sin)
             return (q, *self.append_rope_kv(k, v, cos, sin))
         pos, at = self.claim(B, T)

@@ -9,13 +9,14 @@ from mlx_sharding_amd import ops
 from mlx_sharding_amd.ops.kvcache import KVCache
 
 pytestmark = pytest.mark.gpu
+EXT = ops.hip_ext()
 
 
 @pytest.mark.parametrize("captured", [False, True])
 @pytest.mark.parametrize("B,T,Hq,Hkv,D", [(1, 1, 1, 1, 16), (3, 1, 8, 2, 64), (64, 1, 32, 8, 128),
                                           (1, 57, 32, 4, 64), (2, 300, 4, 2, 256),
                                           (1, 9, 3, 1, 24)])  # the last: apart
-def test_same_as_separate_kernels(B, T, Hq, Hkv, D, captured):
+def test_same_as_separate_kernels(B, T, Hq, Hkv, D, captured, monkeypatch):
     torch.manual_seed(D + T)
     rows = torch.randn(B, T, (Hq + 2 * Hkv) * D, device="cuda").bfloat16()
     q, k, v = (t.view(B, T, -1, D) for t in rows.split([Hq * D, Hkv * D, Hkv * D], -1))
@@ -32,7 +33,17 @@ def test_same_as_separate_kernels(B, T, Hq, Hkv, D, captured):
             c.graph_pos = torch.tensor([7], dtype=torch.int32, device="cuda")
         caches.append(c)
     one, two = caches
-    got = one.append_rope_qkv(q, k, v, cos, sin)
+    ran = []
+
+    class Spied:
+        def __getattr__(self, name):
+            ran.append(name)
+            return getattr(EXT, name)
+
+    with monkeypatch.context() as m:
+        m.setattr(ops, "hip_ext", Spied)
+        got = one.append_rope_qkv(q, k, v, cos, sin)
+    assert ran == (["rope_qkv"] if D % 16 == 0 else ["rope_append_kv"])
     want = (ops.apply_rope(q, cos, sin), *two.append_rope_kv(k, v, cos, sin))
     for a, b in zip((*got, one._k, one._v), (*want, two._k, two._v)):
         # a turn's two products may be contracted the other way round: one bf16 step
