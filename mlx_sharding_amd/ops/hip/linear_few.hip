@@ -13,7 +13,8 @@
 // there are enough of them and more than a few rows of x.  The norm's factor is
 // applied to the sums: x times the weight is rounded to bf16, as the normed row
 // was.
-// Measured, beside the library's product (us; M x K x O): 1 x 2048 x 2048: 5.0,
+// Measured with weights out of memory (sets of 1.5 GB and more by turns), beside the
+// library's product (us; M x K x O): 1 x 2048 x 2048: 5.0,
 // 11.0; 1 x 4096 x 4096: 8.4, 15.5; 1 x 4096 x 28672: 38 (6.2 TB/s), 62; 16 of
 // these: 48, 59; 1 x 14336 x 4096: 22.5, 26; 8 of these: 24.6, 26.6; 16: 29, 26.
 // With norm and unit, 1 x 4096 x 28672: 46, beside 72 for three kernels.
