@@ -245,10 +245,10 @@ def _function_modes() -> bool:
 
 
 def _watched() -> bool:
-    """Whether something around the call sees only torch's own operators: forward-mode
-    differentiation, torch.jit.trace, dispatch modes (make_fx, fake tensors), function
-    modes."""
-    return (torch.autograd.forward_ad._current_level >= 0
+    """Whether something around the call sees only torch's own operators: torch.compile,
+    forward-mode differentiation, torch.jit.trace, dispatch modes (make_fx, fake
+    tensors), function modes."""
+    return (torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0
             or torch._C._get_tracing_state() is not None
             or torch._C._len_torch_dispatch_stack() > 0 or _function_modes())
 
@@ -272,7 +272,8 @@ def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None):
     """project on linear_few.hip, or None where that does not take it.  A decoding
     step calls this for each of its products: what can be seen from the tensors is
     looked at in native code (in Python that took longer than the launch)."""
-    if (_force_torch() or type(x) not in _TENSORS or type(weight) not in _TENSORS
+    if (torch.compiler.is_compiling() or _force_torch()
+            or type(x) not in _TENSORS or type(weight) not in _TENSORS
             or torch.autograd.forward_ad._current_level >= 0 or _function_modes()):
         return None
     ext = _few_ext()

@@ -182,6 +182,23 @@ def test_tracers_see_a_product():
 
 
 @pytest.mark.gpu
+def test_compiled_in_one_graph():
+    """What torch.compile reads, it reads to the end."""
+    w = torch.randn(24, 64, device="cuda").bfloat16()
+    x = torch.randn(3, 64, device="cuda").bfloat16()
+    graphs = []
+
+    def backend(graph, inputs):
+        graphs.append([n.target for n in graph.graph.nodes if n.op == "call_function"])
+        return graph.forward
+
+    y = torch.compile(lambda t: ops.linear(t, w) * 2, backend=backend, fullgraph=True)(x)
+    expect = x.double() @ w.double().T * 2
+    assert len(graphs) == 1 and len(graphs[0]) == 2
+    assert (y.double() - expect).norm() < 0.01 * expect.norm()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [3, 200])
 def test_autocast_names_the_type(rows):
     """Few rows have the type that many have."""
