@@ -235,22 +235,25 @@ _ACTS = {None: 0, "silu": 1, "gelu_tanh": 2}
 
 
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
+_compiling = torch.compiler.is_compiling
+_forward_ad = torch.autograd.forward_ad
+_modes = torch._C._len_torch_function_stack
 
 
 def _function_modes() -> bool:
     """Whether function modes are at work, but that of a default device."""
-    n = torch._C._len_torch_function_stack()
-    return n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
-                         for i in range(n))
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
+               for i in range(_modes()))
 
 
 def _watched() -> bool:
     """Whether something around the call sees only torch's own operators: torch.compile,
     forward-mode differentiation, torch.jit.trace, dispatch modes (make_fx, fake
     tensors), function modes."""
-    return (torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0
+    return (_compiling() or _forward_ad._current_level >= 0
             or torch._C._get_tracing_state() is not None
-            or torch._C._len_torch_dispatch_stack() > 0 or _function_modes())
+            or torch._C._len_torch_dispatch_stack() > 0
+            or (_modes() > 0 and _function_modes()))
 
 
 def _plain(t: torch.Tensor) -> bool:
@@ -272,11 +275,10 @@ def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None):
     """project on linear_few.hip, or None where that does not take it.  A decoding
     step calls this for each of its products: what can be seen from the tensors is
     looked at in native code (in Python that took longer than the launch)."""
-    if (torch.compiler.is_compiling() or _force_torch()
-            or type(x) not in _TENSORS or type(weight) not in _TENSORS
-            or torch.autograd.forward_ad._current_level >= 0 or _function_modes()):
+    if (_compiling() or type(x) not in _TENSORS or type(weight) not in _TENSORS
+            or _forward_ad._current_level >= 0 or (_modes() and _function_modes())):
         return None
-    ext = _few_ext()
+    ext = _EXT if _EXT is not None else _few_ext()
     if ext is None:
         return None
     if norm is None:
@@ -319,11 +321,14 @@ def linear(x, weight, bias=None):
     hipBLASLt's small-GEMM kernels run ~13 us in-graph and the split-K fp32-atomic
     traffic (M*O*4*nk bytes) rivals the weight bytes on small-O projections
     (docs/PERFORMANCE.md).  Kept for shape-specific re-tuning."""
-    gemv = os.environ.get("MLXS_AMD_DENSE_GEMV")
-    if not gemv and x.is_cuda and weight.shape[-1] < 16384:
-        # neither of the two kernels for long rows below
+    longer = weight.shape[-1] >= 16384  # that two kernels below are for
+    if x.is_cuda and not longer:
         y = _linear_few(x, weight, bias)
-        return torch.nn.functional.linear(x, weight, bias) if y is None else y
+        if y is not None:
+            return y
+    gemv = os.environ.get("MLXS_AMD_DENSE_GEMV")
+    if not gemv and not longer:
+        return torch.nn.functional.linear(x, weight, bias)
     if (gemv
             and _use_hip(x) and weight.dtype == torch.bfloat16
             and x.dtype == torch.bfloat16 and weight.shape[-1] % 32 == 0
@@ -368,7 +373,7 @@ def linear(x, weight, bias=None):
             if bias is not None:
                 y = y + bias
             return y.reshape(*lead, y.shape[-1])
-    y = _linear_few(x, weight, bias) if x.is_cuda else None
+    y = _linear_few(x, weight, bias) if x.is_cuda and longer else None
     return torch.nn.functional.linear(x, weight, bias) if y is None else y
 
 

@@ -10,6 +10,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <cstdlib>
+#include <cstring>
 
 extern "C" void launch_linear_few(const void*, const void*, const void*,
                                   const void*, const void*, void*, int, int, int,
@@ -88,13 +89,14 @@ static bool linear_few_recorded() {
   return c10::impl::tls_local_dispatch_key_set().included_.has_any(recorders);
 }
 
-// Whether the environment asks for another kernel for products of a contraction K.
+// Whether the environment asks for other kernels, or for torch's own.
 static bool linear_few_other(long K) {
-  auto set = [](const char* name) {
+  auto is = [](const char* name, const char* value) {
     const char* v = std::getenv(name);
-    return v && *v;
+    return v && *v && (!value || !std::strcmp(v, value));
   };
-  return set("MLXS_AMD_DENSE_GEMV") || (K >= 16384 && set("MLXS_AMD_GEMM64"));
+  return is("MLXS_AMD_FORCE_TORCH", "1") || is("MLXS_AMD_DENSE_GEMV", nullptr) ||
+         (K >= 16384 && is("MLXS_AMD_GEMM64", nullptr));
 }
 
 // Whether x w^T runs here: up to 64 bf16 rows that begin, as w's, at whole 16-byte
