@@ -33,6 +33,20 @@ class CacheFull(RuntimeError):
     """No page or slot is free."""
 
 
+def upload(values: np.ndarray, device) -> torch.Tensor:
+    """The array on ``device``, in the order of the current stream.  A copy out of
+    pageable memory would wait for all that the stream has still to do, so that the
+    host could prepare no step while the last one runs; pinned memory goes back to
+    its pool once the copy is through."""
+    device = torch.device(device)
+    if device.type != "cuda":
+        return torch.from_numpy(values).to(device)
+    held = torch.empty(values.shape, dtype=torch.from_numpy(values).dtype,
+                       pin_memory=True)
+    held.numpy()[...] = values
+    return held.to(device, non_blocking=True)
+
+
 @dataclass
 class RowSpec:
     """A paged layer: ``width`` elements per token."""
@@ -183,8 +197,10 @@ class RaggedBatch:
     """
 
     def __init__(self, portions: Sequence[Tuple[Held, int]], device,
-                 max_keys: int = 0):
-        """portions: (what the request holds, number of new tokens)."""
+                 max_keys: int = 0, wait: bool = True):
+        """portions: (what the request holds, number of new tokens).  wait: the
+        arrays are there when this returns; otherwise they are on the current
+        stream, where the batch is then run."""
         lens = [n for _, n in portions]
         self.order = sorted(range(len(portions)),
                             key=lambda i: lens[i] > SHORT)
@@ -212,9 +228,9 @@ class RaggedBatch:
         tok_pos = (np.arange(self.n_tokens, dtype=np.int32)
                    - cu[tok_entry] + pos0[tok_entry]).astype(np.int32)
         parts = {
-            "cu": cu, "pos0": pos0,
-            "slots": np.array([h.slot for h in held], dtype=np.int32),
-            "tok_pos": tok_pos, "tok_entry": tok_entry, "pages": pages,
+            "cu": cu, "slots": np.array([h.slot for h in held], dtype=np.int32),
+            "pos0": pos0, "tok_pos": tok_pos,
+            "tok_entry": tok_entry, "pages": pages,
         }
         self.key_rows = 0
         if self.n_long:
@@ -256,7 +272,8 @@ class RaggedBatch:
                 span_cu=np.array(span_cu, dtype=np.int32))
         flat = np.concatenate([np.ascontiguousarray(a).reshape(-1)
                                for a in parts.values()])
-        dev = torch.from_numpy(flat).to(device)
+        dev = torch.from_numpy(flat).to(device) if wait else upload(flat, device)
+        self._places = dev[cu.size + E: cu.size + 2 * E + self.n_tokens]
         off = 0
         for name, a in parts.items():
             setattr(self, name, dev[off: off + a.size].view(a.shape))
@@ -267,8 +284,7 @@ class RaggedBatch:
     def advance(self):
         """Turn a batch of single tokens into the next one, on the device;
         pages must not have grown since."""
-        self.tok_pos.add_(1)
-        self.pos0.add_(1)
+        self._places.add_(1)  # pos0 and tok_pos
         self.max_pos += 1
         self.max_keys = max(self.max_keys, self.max_pos)
         self.host = [(s, n, p + 1, h) for s, n, p, h in self.host]
@@ -340,7 +356,8 @@ class RaggedCache:
         if T == 1 and d is not None and d.max_pos == self.offset:
             d.advance()
         else:
-            d = RaggedBatch([(h, T) for h in self.held], self.state.device)
+            d = RaggedBatch([(h, T) for h in self.held], self.state.device,
+                            wait=False)
         self._decode = d if T == 1 else None
         self.offset += T
         for h in self.held:

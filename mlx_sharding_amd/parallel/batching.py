@@ -20,10 +20,11 @@ from dataclasses import dataclass, field
 from typing import (Deque, Dict, Generator, Hashable, Iterator, List, Optional,
                     Sequence, Tuple)
 
+import numpy as np
 import torch
 
 from ..models.base import StageModel
-from ..ops.paged import PAGE, CacheFull, RaggedBatch
+from ..ops.paged import PAGE, CacheFull, RaggedBatch, upload
 from .engine import Sampler, SamplingParams
 
 __all__ = ["BatchEngine", "BatchScheduler", "BatchService", "CacheFull",
@@ -92,11 +93,10 @@ class BatchEngine:
                             any(len(h.pages) != pages.get(r)
                                 for r, h in zip(rids, held)))
         ids = [t for j in batch.order for t in portions[j].tokens]
-        x = torch.tensor(ids, dtype=torch.long, device=self.device)
         start = {batch.order[e]: batch.host[e][0] for e in range(len(portions))}
-        rows = torch.tensor([start[j] + int(w) for j, p in enumerate(portions)
-                             for w in p.want], dtype=torch.long,
-                            device=self.device)
+        ids += [start[j] + int(w) for j, p in enumerate(portions) for w in p.want]
+        x, rows = upload(np.array(ids, dtype=np.int64), self.device).split(
+            [batch.n_tokens, len(ids) - batch.n_tokens])
         logits = self.model.run(x, batch, state, rows=rows)
         for p, h in zip(portions, held):
             h.length += len(p.tokens)
@@ -111,7 +111,7 @@ class BatchEngine:
             batch = self._last
             batch.advance()
         else:
-            batch = RaggedBatch(list(zip(held, lens)), self.device)
+            batch = RaggedBatch(list(zip(held, lens)), self.device, wait=False)
         single = max(lens) == 1
         self._last = batch if single else None
         self._last_key = tuple((r, h.slot, h.length + 1)

@@ -1,0 +1,45 @@
+"""Arrays of a batch on their way to the device."""
+
+import numpy as np
+import pytest
+import torch
+
+from mlx_sharding_amd.ops.paged import RaggedBatch, PagedState, RowSpec, upload
+
+
+@pytest.mark.parametrize("n", [0, 1, 7, 4096])
+def test_upload_cpu(n):
+    a = np.arange(n, dtype=np.int64)
+    t = upload(a, "cpu")
+    assert t.dtype == torch.int64 and t.tolist() == a.tolist()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [0, 1, 1000])
+def test_upload_behind_work(n):
+    # many uploads while the stream is busy: none may find its memory taken
+    x = torch.randn(4096, 4096, device="cuda")
+    for _ in range(20):
+        x = x @ x / 64.0
+    out = [upload(np.full(n, i, dtype=np.int32), "cuda") for i in range(200)]
+    assert all(t.tolist() == [i] * n for i, t in enumerate(out))
+
+
+def _places(device):
+    state = PagedState([RowSpec(8)], 512, 3, torch.float32, torch.device(device))
+    for r, n in enumerate((5, 64, 130)):
+        state.admit(r)
+        state.reserve(r, n + 3)
+        state.live[r].length = n
+    batch = RaggedBatch([(state.live[r], 1) for r in range(3)], device, wait=False)
+    batch.advance()
+    batch.advance()
+    return batch
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_advance(device):
+    b = _places(device)
+    assert b.pos0.tolist() == b.tok_pos.tolist() == [7, 66, 132]
+    assert b.cu.tolist() == [0, 1, 2, 3] and b.tok_entry.tolist() == [0, 1, 2]
+    assert len(set(b.slots.tolist())) == 3 and b.max_pos == 133
