@@ -18,8 +18,8 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import (Linear, RMSNorm, StageModel, as_built, owned_layer_indices, project,
-                   read_in_place)
+from .base import (Linear, RMSNorm, StageModel, as_built, feed, owned_layer_indices,
+                   project, read_in_place)
 from .llama import _Inner
 
 
@@ -98,6 +98,8 @@ class Gemma2MLP(nn.Module):
     def forward(self, x, norm: Optional[RMSNorm] = None):
         """norm: as in Gemma2Attention."""
         if self._fused_gu is not None and (norm is not None or ops.few_tokens(x)):
+            if as_built(self.down_proj):
+                return feed(self._fused_gu, self.down_proj, x, "gelu_tanh", norm)
             return self.down_proj(project(self._fused_gu, x, norm=norm,
                                           act="gelu_tanh"))
         if norm is not None:

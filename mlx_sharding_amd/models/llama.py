@@ -16,8 +16,8 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import (Linear, RMSNorm, StageModel, as_built, owned_layer_indices, project,
-                   read_in_place)
+from .base import (Linear, RMSNorm, StageModel, as_built, feed, owned_layer_indices,
+                   project, read_in_place)
 
 
 @read_in_place
@@ -114,8 +114,7 @@ class LlamaMLP(nn.Module):
         """norm, residual: as in LlamaAttention."""
         if self._fused_gu is not None and (
                 norm is not None or (ops.few_tokens(x) and as_built(self.down_proj))):
-            y = project(self._fused_gu, x, norm=norm, act="silu")
-            return project(self.down_proj, y, residual=residual)
+            return feed(self._fused_gu, self.down_proj, x, "silu", norm, residual)
         if norm is not None:
             x = norm(x)
         if residual is not None:

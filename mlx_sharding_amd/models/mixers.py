@@ -23,7 +23,7 @@ from ..ops.paged import (HistorySpec, LayerSpec, LayerStore, RaggedBatch,
 from ..ops.ragged import (ClampedGLU, DeltaShape, GroupedShape, LatentShape,
                           Rotary, Turns)
 from ..ops.recurrent import ScanShape
-from .base import Linear, RMSNorm
+from .base import Linear, RMSNorm, as_built, feed
 
 
 def _param(*shape, dtype) -> nn.Parameter:
@@ -466,7 +466,7 @@ class GatedMLP(nn.Module):
     def __init__(self, width: int, ff: int, act: str,
                  dtype: torch.dtype = torch.bfloat16):
         super().__init__()
-        self.act = self.ACTS[act]
+        self.act, self.kind = self.ACTS[act], act
         self.gate = Linear(width, ff, dtype=dtype)
         self.up = Linear(width, ff, dtype=dtype)
         self.down = Linear(ff, width, dtype=dtype)
@@ -477,6 +477,8 @@ class GatedMLP(nn.Module):
         self.fused = FusedColumns([self.gate, self.up])
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
+        if self.fused is not None and ops.few_tokens(h) and as_built(self.down):
+            return feed(self.fused, self.down, h, self.kind)
         g, u = self.fused(h) if self.fused is not None else (self.gate(h), self.up(h))
         return self.down(self.act(g, u))
 

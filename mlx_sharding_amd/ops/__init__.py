@@ -271,20 +271,40 @@ def _few_ext():
     return hip_ragged()
 
 
-def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None):
-    """project on linear_few.hip, or None where that does not take it.  A decoding
-    step calls this for each of its products: what can be seen from the tensors is
-    looked at in native code (in Python that took longer than the launch)."""
-    if (_compiling() or type(x) not in _TENSORS or type(weight) not in _TENSORS
+def _few_for(x, *weights):
+    """The extension, if nothing around the call or about these tensors speaks against
+    linear_few.hip that is seen from Python only.  A decoding step asks for each of its
+    products: what can be seen from the tensors is looked at in native code (in Python
+    that took longer than the launch)."""
+    if (_compiling() or type(x) not in _TENSORS
+            or any(type(w) not in _TENSORS for w in weights)
             or _forward_ad._current_level >= 0 or (_modes() and _function_modes())):
         return None
-    ext = _EXT if _EXT is not None else _few_ext()
+    return _EXT if _EXT is not None else _few_ext()
+
+
+def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None):
+    """project on linear_few.hip, or None where that does not take it."""
+    ext = _few_for(x, weight)
     if ext is None:
         return None
     if norm is None:
         return ext.linear_few_try(x, weight, bias, residual, None, 0.0, 0.0, _ACTS[act])
     return ext.linear_few_try(x, weight, bias, residual, norm.weight, norm.eps,
                               norm.weight_offset, _ACTS[act])
+
+
+def feed_few(x, w_in, w_out, act, norm=None, residual=None):
+    """A feed-forward of few rows in one call: w_out of the gated unit of w_in's halves,
+    of x's rows as ``norm`` makes them, plus ``residual``; None where linear_few.hip does
+    not take both products."""
+    ext = _few_for(x, w_in, w_out) if x.is_cuda else None
+    if ext is None:
+        return None
+    if norm is None:
+        return ext.feed_few_try(x, w_in, w_out, residual, None, 0.0, 0.0, _ACTS[act])
+    return ext.feed_few_try(x, w_in, w_out, residual, norm.weight, norm.eps,
+                            norm.weight_offset, _ACTS[act])
 
 
 def project(x, weight, bias=None, *, norm=None, act=None, residual=None):

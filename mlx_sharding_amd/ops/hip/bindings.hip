@@ -1236,6 +1236,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return attn_prefill_supported((int)dk, (int)dv);
   });
   m.def("linear_few_try", &linear_few_try);
+  m.def("feed_few_try", &feed_few_try);
   m.def("mla_rows", &mla_rows);
   m.def("mla_prompt", &mla_prompt);
   m.def("latent_prompt", &latent_prompt);

@@ -15,15 +15,37 @@
 extern "C" void launch_linear_few(const void*, const void*, const void*,
                                   const void*, const void*, void*, int, int, int,
                                   long, long, long, long, float, float, int,
-                                  hipStream_t);
+                                  unsigned*, float*, unsigned*, int, hipStream_t);
+extern "C" long linear_few_room(int, int, int, int*);
+
+// Room for a product whose contraction blocks share; whatever runs before it clears the
+// numbers.
+struct LinearFewRoom {
+  torch::Tensor held;
+  unsigned* numbers = nullptr;
+  float* sums = nullptr;
+  int n = 0;
+
+  LinearFewRoom() = default;
+  LinearFewRoom(int M, int O, int K, const torch::Tensor& like) {
+    const long floats = linear_few_room(M, O, K, &n);
+    if (!n) return;
+    const long at = (n + 63) / 64 * 64;
+    held = torch::empty({at + floats}, like.options().dtype(torch::kFloat32));
+    numbers = reinterpret_cast<unsigned*>(held.data_ptr<float>());
+    sums = held.data_ptr<float>() + at;
+  }
+};
 
 // x [M, K], w [O, K] (act: [2 O, K]); bias per row of w, residual [M, O], norm
-// weights [K] for the rows of x; act 0: none, 1: silu, 2: gelu_tanh
-static torch::Tensor linear_few(torch::Tensor x, torch::Tensor w,
-                                c10::optional<torch::Tensor> bias,
-                                c10::optional<torch::Tensor> residual,
-                                c10::optional<torch::Tensor> norm, double eps,
-                                double offset, int64_t act) {
+// weights [K] for the rows of x; act 0: none, 1: silu, 2: gelu_tanh.  room: for a shared
+// contraction; clear: the numbers of another one's that runs behind this.
+static torch::Tensor linear_few_run(const torch::Tensor& x, const torch::Tensor& w,
+                                    const c10::optional<torch::Tensor>& bias,
+                                    const c10::optional<torch::Tensor>& residual,
+                                    const c10::optional<torch::Tensor>& norm, double eps,
+                                    double offset, int64_t act, const LinearFewRoom& room,
+                                    const LinearFewRoom& clear) {
   auto bf16 = [&](const torch::Tensor& t) {
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
                     t.device() == x.device(),
@@ -67,8 +89,17 @@ static torch::Tensor linear_few(torch::Tensor x, torch::Tensor w,
   auto y = torch::empty({M, O}, x.options());
   launch_linear_few(x.data_ptr(), w.data_ptr(), b, r, n, y.data_ptr(), M, O, K,
                     x.stride(0), w.stride(0), ldr, O, (float)eps, (float)offset,
-                    (int)act, c10::hip::getCurrentHIPStream().stream());
+                    (int)act, room.numbers, room.sums, clear.numbers, clear.n,
+                    c10::hip::getCurrentHIPStream().stream());
   return y;
+}
+
+static torch::Tensor linear_few(torch::Tensor x, torch::Tensor w,
+                                c10::optional<torch::Tensor> bias,
+                                c10::optional<torch::Tensor> residual,
+                                c10::optional<torch::Tensor> norm, double eps,
+                                double offset, int64_t act) {
+  return linear_few_run(x, w, bias, residual, norm, eps, offset, act, {}, {});
 }
 
 // An ordinary tensor that nothing differentiates, maps or traces.
@@ -99,33 +130,47 @@ static bool linear_few_other(long K) {
          (K >= 16384 && is("MLXS_AMD_GEMM64", nullptr));
 }
 
-// Whether x w^T runs here: up to 64 bf16 rows that begin, as w's, at whole 16-byte
-// vectors.  A contraction above 8192 for 8 rows, or into 4096: 8 rows of 14336 into
-// 4096 take 24.6 us here and 26.6 in the library, 32 rows 30.4 and 30.5, 64 rows 40.1
-// and 38.9.  alone: with nothing taken along; then the library is the better one for
-// many rows of large weights (64 rows of 4096 into 28672: 54 us here, 51 there).
-static bool linear_few_takes(const torch::Tensor& x, const torch::Tensor& w,
-                             bool alone) {
-  if (!x.is_cuda() || w.device() != x.device() || x.scalar_type() != torch::kBFloat16 ||
-      w.scalar_type() != torch::kBFloat16 || w.dim() != 2 || x.dim() < 1 ||
-      !linear_few_plain(x) || !linear_few_plain(w) || linear_few_recorded())
+static bool linear_few_whole(const torch::Tensor& t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
+// Whether x's rows can be read here: bf16, beginning at whole 16-byte vectors.
+static bool linear_few_input(const torch::Tensor& x) {
+  if (!x.is_cuda() || x.scalar_type() != torch::kBFloat16 || x.dim() < 1 ||
+      !linear_few_plain(x) || linear_few_recorded())
     return false;
   if (at::autocast::is_autocast_enabled(at::kCUDA) &&
       at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16)
     return false;  // a product of another type
-  const long O = w.size(0), K = w.size(1);
-  if (O < 1 || K < 32 || K % 32 || x.size(-1) != K || linear_few_other(K)) return false;
-  const long rows = x.numel() / K;
-  if (rows < 1 || rows > 64 || (K > 8192 && rows > 8 && O > 4096) ||
-      (alone && rows > 32 && O * K > 1 << 25))
-    return false;
-  auto whole = [](const torch::Tensor& t) {
-    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
-  };
   for (long d = 0; d + 1 < x.dim(); ++d)
     if (x.stride(d) % 8) return false;
-  return x.stride(-1) == 1 && w.stride(1) == 1 && w.stride(0) % 8 == 0 && whole(x) &&
-         whole(w);
+  return x.stride(-1) == 1 && linear_few_whole(x);
+}
+
+static bool linear_few_weight(const torch::Tensor& w, const torch::Tensor& x) {
+  return w.device() == x.device() && w.scalar_type() == torch::kBFloat16 &&
+         w.dim() == 2 && linear_few_plain(w) && w.stride(1) == 1 &&
+         w.stride(0) % 8 == 0 && linear_few_whole(w);
+}
+
+// Whether a product of this size runs here.  A contraction above 8192 for 8 rows, or
+// into 4096: 8 rows of 14336 into 4096 take 24.6 us here and 26.6 in the library, 32
+// rows 30.4 and 30.5, 64 rows 40.1 and 38.9.  alone: with nothing taken along; then the
+// library is the better one for many rows of large weights (64 rows of 4096 into 28672:
+// 54 us here, 51 there).
+static bool linear_few_sizes(long rows, long O, long K, bool alone) {
+  return O >= 1 && K >= 32 && K % 32 == 0 && rows >= 1 && rows <= 64 &&
+         !(K > 8192 && rows > 8 && O > 4096) &&
+         !(alone && rows > 32 && O * K > 1 << 25) && !linear_few_other(K);
+}
+
+// Whether x w^T runs here.
+static bool linear_few_takes(const torch::Tensor& x, const torch::Tensor& w,
+                             bool alone) {
+  if (!linear_few_input(x) || !linear_few_weight(w, x) || w.size(1) < 1 ||
+      x.size(-1) != w.size(1))
+    return false;
+  return linear_few_sizes(x.numel() / w.size(1), w.size(0), w.size(1), alone);
 }
 
 // Whether a product here takes along what it is given: a bias per row of w and norm
@@ -151,6 +196,22 @@ static bool linear_few_along(const torch::Tensor& x, long O, long biases,
          residual->sizes().slice(0, x.dim() - 1) == x.sizes().slice(0, x.dim() - 1);
 }
 
+// x's rows, as the kernels read them.
+static torch::Tensor linear_few_rows(const torch::Tensor& x) {
+  if (x.dim() == 2) return x;
+  auto rows = x.reshape({-1, x.size(-1)});
+  if (rows.stride(0) % 8 || reinterpret_cast<uintptr_t>(rows.data_ptr()) % 16)
+    rows = rows.clone();
+  return rows;
+}
+
+static torch::Tensor linear_few_shaped(const torch::Tensor& y, const torch::Tensor& x) {
+  if (x.dim() == 2) return y;
+  auto sizes = x.sizes().vec();
+  sizes.back() = y.size(1);
+  return y.view(sizes);
+}
+
 // linear_few for x of any number of dimensions, or nothing where it does not run here.
 static c10::optional<torch::Tensor> linear_few_try(
     torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
@@ -159,13 +220,38 @@ static c10::optional<torch::Tensor> linear_few_try(
   if (!linear_few_takes(x, w, !residual.has_value() && !norm.has_value() && !act) ||
       !linear_few_along(x, w.size(0) / (act ? 2 : 1), w.size(0), bias, residual, norm))
     return {};
-  if (x.dim() == 2) return linear_few(x, w, bias, residual, norm, eps, offset, act);
-  auto rows = x.reshape({-1, x.size(-1)});
-  if (rows.stride(0) % 8 || reinterpret_cast<uintptr_t>(rows.data_ptr()) % 16)
-    rows = rows.clone();
-  if (residual.has_value()) residual = residual->reshape({rows.size(0), -1});
-  auto y = linear_few(rows, w, bias, residual, norm, eps, offset, act);
-  auto sizes = x.sizes().vec();
-  sizes.back() = y.size(1);
-  return y.view(sizes);
+  const auto rows = linear_few_rows(x);
+  if (residual.has_value() && x.dim() != 2)
+    residual = residual->reshape({rows.size(0), -1});
+  return linear_few_shaped(
+      linear_few(rows, w, bias, residual, norm, eps, offset, act), x);
+}
+
+// A feed-forward: w_out of the gated unit of w_in's halves (act 1 or 2), of x's rows as
+// the norm makes them, plus the residual, or nothing where one of the products does not
+// run here.  The first clears the numbers that the blocks of the second count with.
+static c10::optional<torch::Tensor> feed_few_try(
+    torch::Tensor x, torch::Tensor w_in, torch::Tensor w_out,
+    c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> norm, double eps,
+    double offset, int64_t act) {
+  TORCH_CHECK(act == 1 || act == 2, "unknown unit");
+  if (!linear_few_takes(x, w_in, false) || !linear_few_weight(w_out, x) ||
+      w_in.size(0) != 2 * w_out.size(1))
+    return {};
+  const int M = x.numel() / x.size(-1), O = w_out.size(0), I = w_out.size(1);
+  // long contractions into many columns have a kernel of their own (gemm_kseg.hip)
+  if (I >= 16384 && O >= 8192 && !residual.has_value()) return {};
+  int shared = 0;
+  if (O >= 1 && I >= 32) linear_few_room(M, O, I, &shared);
+  if (!linear_few_sizes(M, O, I, !shared && !residual.has_value()) ||
+      !linear_few_along(x, I, 2 * I, {}, {}, norm) ||
+      !linear_few_along(x, O, O, {}, residual, {}))
+    return {};
+  const auto rows = linear_few_rows(x);
+  if (residual.has_value() && x.dim() != 2) residual = residual->reshape({M, -1});
+  const LinearFewRoom room(M, O, I, rows);
+  const auto units =
+      linear_few_run(rows, w_in, {}, {}, norm, eps, offset, act, {}, room);
+  return linear_few_shaped(
+      linear_few_run(units, w_out, {}, residual, {}, 0.0, 0.0, 0, room, {}), x);
 }

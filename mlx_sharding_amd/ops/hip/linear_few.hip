@@ -29,7 +29,59 @@ struct LinearFewArgs {
   int M, O, K;             // O: columns of y
   long ldx, ldw, ldr, ldy;
   float eps, offset;       // norm weights are norm + offset
+  // gridDim.y > 1: blocks share a tile's contraction, `share` steps (few) or stages
+  // (some) each.  part [tiles of y, gridDim.y,
+  // tiles of x, WAVE, 4], count: one number per tile of y and x, zero before.
+  float* part;
+  unsigned* count;
+  unsigned* zero;          // n_zero numbers that this launch clears for a later one
+  int n_zero, share;
 };
+
+// Where a block begins in the n chunks of a contraction; it goes round from there.
+// Rows of W and of x lie powers of two apart as a rule, and blocks in step at one column
+// ask few of the memory's channels: 16384 rows of 2048, 12 of x, 16.4 us from column 0 on,
+// 14.1 so (the blocks of an XCD, which are every eighth, three chunks apart; one apart
+// 14.2, seven 14.5); 28672 of 4096 with norm and unit 45.6, 43.5; 6144 of 4096 14.7, 13.2.
+__device__ __forceinline__ int first_of(int n) {
+  return (blockIdx.x >> 3) * 3 % (unsigned)max(n, 1);
+}
+
+// The sums of a tile that blocks share: leaves this one's, and true in the one that
+// comes last, which then has all, added in the blocks' order.  Sums pass the L2s, which
+// XCDs have of their own, by accesses of the device's scope.
+__device__ __forceinline__ bool sums_of_all(const LinearFewArgs& a, long tile,
+                                            int lane, f32x4& v) {
+  typedef unsigned long long u64;
+  typedef u64 u64x2 __attribute__((ext_vector_type(2)));
+  u64* to = reinterpret_cast<u64*>(a.part) + (tile * gridDim.y * WAVE + lane) * 2;
+  const u64x2 own = __builtin_bit_cast(u64x2, v);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    __hip_atomic_store(to + blockIdx.y * (WAVE * 2) + i, own[i], __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  unsigned before = 0;
+  if (lane == 0)
+    before = __hip_atomic_fetch_add(a.count + tile, 1u, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+  before = __builtin_amdgcn_readfirstlane(before);
+  if (before + 1 != gridDim.y) return false;
+  asm volatile("" ::: "memory");
+  v = f32x4{0, 0, 0, 0};
+#pragma unroll 4
+  for (unsigned s = 0; s < gridDim.y; ++s) {
+    u64x2 p;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      p[i] = __hip_atomic_load(to + s * (WAVE * 2) + i, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    const f32x4 f = __builtin_bit_cast(f32x4, p);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] += f[j];
+  }
+  return true;
+}
 
 enum { LF_PLAIN = 0, LF_SILU = 1, LF_GELU = 2 };
 
@@ -90,9 +142,9 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
 #pragma unroll
   for (int r = 0; r < RT; ++r) {
     const int row = r / YT * a.O + min(row0 + r % YT * 16 + l16, a.O - 1);
-    wp[r] = a.w + (long)row * a.ldw + lg * 8;
+    wp[r] = a.w + (long)row * a.ldw;
   }
-  const __bf16* xp = a.x + (long)min(l16, a.M - 1) * a.ldx + lg * 8;
+  const __bf16* xp = a.x + (long)min(l16, a.M - 1) * a.ldx;
 
   f32x4 acc[RT];
   float sq = 0.0f;
@@ -111,20 +163,29 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
     return *reinterpret_cast<const bf16x8_t*>(p);
   };
 
-  const int steps = a.K / 32, chunks = steps / U;
+  // this block's share of the contraction
+  const int s0 = blockIdx.y * a.share, steps = min(a.share, a.K / 32 - s0);
+  const int chunks = steps / U, first = first_of(chunks);
   // operands of one chunk; the next one's are asked for before this one is used,
   // rows of x among them, as loads come back in order
   struct Chunk {
     bf16x8_t w[RT][U], x[U], g[NORM ? U : 1];
   };
   auto fetch = [&](Chunk& f, int c) {
+    c += first;
+    if (c >= chunks) c -= chunks;
+    // the steps of a row one after the other: two are a line of 128 bytes, of which the
+    // second half is then on its way (28672 rows of 4096: by steps 51 us, by rows 45)
+    const int from = (s0 + c * U) * 32 + lg * 8;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int at = (c * U + u) * 32;
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
-      for (int r = 0; r < RT; ++r) f.w[r][u] = load(wp[r] + at);
-      f.x[u] = load(xp + at);
-      if (NORM) f.g[u] = load(a.norm + at + lg * 8);
+      for (int u = 0; u < U; ++u) f.w[r][u] = load(wp[r] + from + u * 32);
+#pragma unroll
+    for (int u = 0; u < U; ++u) f.x[u] = load(xp + from + u * 32);
+    if (NORM) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) f.g[u] = load(a.norm + from + u * 32);
     }
   };
   auto use = [&](const Chunk& f) {
@@ -147,12 +208,13 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
     if (c + NW < chunks) use(two);
   }
   // steps that make no whole chunk
-  for (int s = chunks * U + wid; s < steps; s += NW) {
-    bf16x8_t v = load(xp + s * 32);
-    if (NORM) v = normed(v, load(a.norm + s * 32 + lg * 8));
+  for (int s = s0 + chunks * U + wid; s < s0 + steps; s += NW) {
+    const int at = s * 32 + lg * 8;
+    bf16x8_t v = load(xp + at);
+    if (NORM) v = normed(v, load(a.norm + at));
 #pragma unroll
     for (int r = 0; r < RT; ++r)
-      acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load(wp[r] + s * 32), v,
+      acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load(wp[r] + at), v,
                                                        acc[r], 0, 0, 0);
   }
 
@@ -161,6 +223,8 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
   if (NORM) squares[wid][lane] = sq;
   __syncthreads();
 
+  if (a.zero && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < a.n_zero; i += NW * WAVE) a.zero[i] = 0;
   // a wave per tile of y: four columns of a row a lane
   for (int r = wid; r < YT; r += NW) {
     f32x4 v[ACT ? 2 : 1];
@@ -186,14 +250,24 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[h][j] *= f;
     }
+    if (!ACT && !NORM && gridDim.y > 1 &&
+        !sums_of_all(a, (long)blockIdx.x * YT + r, lane, v[0]))
+      continue;
     if (l16 < a.M) finish_columns<ACT>(a, l16, row0 + r * 16 + lg * 4, v);
   }
 }
 
+// Blocks that share a tile's contraction, as many as have something of it.
+static dim3 shared_grid(LinearFewArgs& a, int cols, int steps, int split) {
+  a.share = (steps + split - 1) / split;
+  return dim3((unsigned)((a.O + cols - 1) / cols),
+              (unsigned)((steps + a.share - 1) / a.share));
+}
+
 template <int RT, int ACT, int NW, int U>
-static void linear_few_go(const LinearFewArgs& a, hipStream_t stream) {
+static void linear_few_go(LinearFewArgs a, int split, hipStream_t stream) {
   constexpr int cols = 16 * (ACT ? RT / 2 : RT);
-  const dim3 grid((unsigned)((a.O + cols - 1) / cols)), block(NW * WAVE);
+  const dim3 grid = shared_grid(a, cols, a.K / 32, split), block(NW * WAVE);
   // the norm's weights and sums need registers: shorter chunks
   if (a.norm) {
     linear_few_kernel<RT, ACT, true, NW, 2><<<grid, block, 0, stream>>>(a);
@@ -207,20 +281,24 @@ static void linear_few_go(const LinearFewArgs& a, hipStream_t stream) {
 // rows of x are read once for 64 of W (28672 rows, 16 of x: 48 us, 51 with two, 56
 // with one), but one for few rows of x (one: 38 us, 45 with four).  A unit needs
 // both its halves; four from 16384 rows on (28672 rows, 16 of x, norm: 50 us, 53
-// with two; 12800, one of x: 14.0 with two, 15.8).
-static void linear_few_tiles(const LinearFewArgs& a, int act, hipStream_t stream) {
+// with two; 12800, one of x: 14.0 with two, 15.8).  One tile takes two steps at a time:
+// 4096 rows of 4096 8.3 us, of 14336 22.2, with four 9.2 and 23.3.
+static void linear_few_tiles(const LinearFewArgs& a, int act, int split,
+                             hipStream_t stream) {
   if (act == LF_SILU) {
-    if (a.O >= 8192) linear_few_go<4, LF_SILU, 4, 2>(a, stream);
-    else linear_few_go<2, LF_SILU, 8, 4>(a, stream);
+    if (a.O >= 8192) linear_few_go<4, LF_SILU, 4, 2>(a, 1, stream);
+    else linear_few_go<2, LF_SILU, 8, 4>(a, 1, stream);
   } else if (act == LF_GELU) {
-    if (a.O >= 8192) linear_few_go<4, LF_GELU, 4, 2>(a, stream);
-    else linear_few_go<2, LF_GELU, 8, 4>(a, stream);
-  } else if (a.O <= 4096 || (a.O > 8192 && a.M <= 4)) {
-    linear_few_go<1, LF_PLAIN, 8, 4>(a, stream);
+    if (a.O >= 8192) linear_few_go<4, LF_GELU, 4, 2>(a, 1, stream);
+    else linear_few_go<2, LF_GELU, 8, 4>(a, 1, stream);
+  } else if (a.O <= 4096) {
+    linear_few_go<1, LF_PLAIN, 8, 2>(a, split, stream);
+  } else if (a.O > 8192 && a.M <= 4) {
+    linear_few_go<1, LF_PLAIN, 8, 4>(a, 1, stream);
   } else if (a.O <= 8192) {
-    linear_few_go<2, LF_PLAIN, 8, 4>(a, stream);
+    linear_few_go<2, LF_PLAIN, 8, 4>(a, 1, stream);
   } else {
-    linear_few_go<4, LF_PLAIN, 4, 2>(a, stream);
+    linear_few_go<4, LF_PLAIN, 4, 2>(a, 1, stream);
   }
 }
 
@@ -274,10 +352,17 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
     }
   }
   bf16x8_t g[NORM ? RING : 1];
-  const int stages = (a.K + KS * 32 - 1) / (KS * 32);
+  // this block's share of the contraction
+  const int s0 = blockIdx.y * a.share;
+  const int stages = min(a.share, (a.K + KS * 32 - 1) / (KS * 32) - s0);
+  const int first = first_of(stages);
+  auto turned = [&](int t) {
+    t = min(t, stages - 1) + first;
+    return s0 + (t >= stages ? t - stages : t);
+  };
   // columns behind the last one repeat others of its row; nobody takes them
   auto issue = [&](int t, int slot) {
-    const int k0 = min(t, stages - 1) * (KS * 32);
+    const int k0 = turned(t) * (KS * 32);
 #pragma unroll
     for (int i = 0; i < PARTS; ++i)
       __builtin_amdgcn_global_load_lds(
@@ -298,7 +383,7 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
     for (int r = 0; r < RT; ++r) acc[r][i] = f32x4{0, 0, 0, 0};
   }
   auto use = [&](int t, int s) {
-    if ((t * KS + step) * 32 >= a.K) return;
+    if ((turned(t) * KS + step) * 32 >= a.K) return;
     const char* at = smem + s * STAGE + l16 * RP * 16 + place(l16, step * 4 + lg) * 16;
     bf16x8_t w[RT], v[TW];
 #pragma unroll
@@ -360,6 +445,8 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
   }
   __syncthreads();
 
+  if (a.zero && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < a.n_zero; i += LS_WAVES * WAVE) a.zero[i] = 0;
   for (int n = wid; n < YT * TT; n += LS_WAVES) {
     const int r = n / TT, i = n % TT;
     f32x4 v[ACT ? 2 : 1];
@@ -385,13 +472,16 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[h][j] *= f;
     }
+    if (!ACT && !NORM && gridDim.y > 1 &&
+        !sums_of_all(a, ((long)blockIdx.x * YT + r) * TT + i, lane, v[0]))
+      continue;
     if (i * 16 + l16 < a.M)
       finish_columns<ACT>(a, i * 16 + l16, row0 + r * 16 + lg * 4, v);
   }
 }
 
 template <int RT, int TT, int ACT, bool NORM>
-static void linear_some_go(const LinearFewArgs& a, hipStream_t stream) {
+static void linear_some_go(LinearFewArgs a, int split, hipStream_t stream) {
   constexpr int KS = RT == 1 ? 8 : 4;
   constexpr int cols = 16 * (ACT ? RT / 2 : RT);
   constexpr int stage = (RT + TT) * KS * 1024;
@@ -401,62 +491,99 @@ static void linear_some_go(const LinearFewArgs& a, hipStream_t stream) {
     (void)hipFuncSetAttribute(
         reinterpret_cast<const void*>(&linear_some_kernel<RT, TT, KS, ACT, NORM>),
         hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  const dim3 grid = shared_grid(a, cols, (a.K + KS * 32 - 1) / (KS * 32), split);
   linear_some_kernel<RT, TT, KS, ACT, NORM>
-      <<<dim3((unsigned)((a.O + cols - 1) / cols)), dim3(LS_WAVES * WAVE), smem,
-         stream>>>(a);
+      <<<grid, dim3(LS_WAVES * WAVE), smem, stream>>>(a);
 }
 
 template <int RT, int ACT>
-static void linear_some_tiles(const LinearFewArgs& a, hipStream_t stream) {
+static void linear_some_tiles(const LinearFewArgs& a, int split, hipStream_t stream) {
   if (a.M <= 32) {
     if (a.norm) {
-      linear_some_go<RT, 2, ACT, true>(a, stream);
+      linear_some_go<RT, 2, ACT, true>(a, split, stream);
     } else {
-      linear_some_go<RT, 2, ACT, false>(a, stream);
+      linear_some_go<RT, 2, ACT, false>(a, split, stream);
     }
   } else {
     if (a.norm) {
-      linear_some_go<RT, 4, ACT, true>(a, stream);
+      linear_some_go<RT, 4, ACT, true>(a, split, stream);
     } else {
-      linear_some_go<RT, 4, ACT, false>(a, stream);
+      linear_some_go<RT, 4, ACT, false>(a, split, stream);
     }
   }
 }
 
 // Tiles of W's rows per block: one up to 4096 rows, which are 256 blocks, two up to
 // 8192, then four (64 of x; one, two, four: 4096 rows of 4096 13.7, 17.0, 21.7 us;
-// 5632 of 2048 15.0, 10.8, 13.6; 11264 of 2048 23.3, 19.8, 15.4).
-static void linear_some(const LinearFewArgs& a, int act, hipStream_t stream) {
+// 5632 of 2048 15.0, 10.8, 13.6; 11264 of 2048 23.3, 19.8, 15.4).  Blocks that share
+// tiles have two, or four above 2816 rows.
+static void linear_some(const LinearFewArgs& a, int act, int split, hipStream_t stream) {
   const bool many = (act ? 2 : 1) * a.O > 8192;
   if (act == LF_SILU) {
-    if (many) linear_some_tiles<4, LF_SILU>(a, stream);
-    else linear_some_tiles<2, LF_SILU>(a, stream);
+    if (many) linear_some_tiles<4, LF_SILU>(a, 1, stream);
+    else linear_some_tiles<2, LF_SILU>(a, 1, stream);
   } else if (act == LF_GELU) {
-    if (many) linear_some_tiles<4, LF_GELU>(a, stream);
-    else linear_some_tiles<2, LF_GELU>(a, stream);
+    if (many) linear_some_tiles<4, LF_GELU>(a, 1, stream);
+    else linear_some_tiles<2, LF_GELU>(a, 1, stream);
+  } else if (split > 1) {
+    if (a.O <= 2816) linear_some_tiles<2, LF_PLAIN>(a, split, stream);
+    else linear_some_tiles<4, LF_PLAIN>(a, split, stream);
   } else if (a.O <= 4096) {
-    linear_some_tiles<1, LF_PLAIN>(a, stream);
+    linear_some_tiles<1, LF_PLAIN>(a, 1, stream);
   } else if (many) {
-    linear_some_tiles<4, LF_PLAIN>(a, stream);
+    linear_some_tiles<4, LF_PLAIN>(a, 1, stream);
   } else {
-    linear_some_tiles<2, LF_PLAIN>(a, stream);
+    linear_some_tiles<2, LF_PLAIN>(a, 1, stream);
   }
 }
 
+// Whether rows of x go through LDS: above 16, and above 8 where a block would read them
+// for many columns or from many blocks (12 of x; registers, LDS: 4096 rows of 4096 9.5,
+// 9.2 us; of 14336 26, 23.8; 2048 of 8192 15.7, 12.5; 8192 of 3584 15, 13.0; 2048 of
+// 2048 6.2, 6.4; 3648 of 2048 with norm 7.3, 8.3).
+static bool few_through_lds(int M, int O, int K, int act) {
+  return M > 16 || (M > 8 && ((act ? 2 : 1) * O > 4096 || K > 2048));
+}
+
+// Blocks that share a tile's contraction where the caller has room for their sums.  x is
+// read once per block, four times W with 16 rows of W and 64 of x: long rows then have
+// blocks of more rows and a part of the columns each (us, alone and shared; 64 of x: 4096
+// rows of 14336 39.6, 29.0; 3584 of 14336 39, 28.3; 2048 of 8192 20.7, 13.4, of 5632 17.6,
+// 11.5, of 2816 10.5, 8.9; 12 of x, 2048 of 8192 12.5, 10.5; 32 of x, 4096 of 14336 29.7,
+// 25.2, but 12 of these 23.8, 24.7).  Up to 2816 rows of W leave CUs idle without (one
+// of x, 2048 of 8192: 11.6, 9.7).
+static int few_split(int M, int O, int K, int act, bool norm) {
+  if (act || norm) return 1;
+  if (!few_through_lds(M, O, K, act)) return O <= 2816 && K >= 4096 ? 2 : 1;
+  if (O <= 2816) return K >= (M > 32 ? 2048 : 4096) ? 4 : 1;
+  return O <= 4608 && K >= 8192 && M > 16 ? 4 : 1;
+}
+
+// Room for a shared contraction: `numbers` to be cleared before, and sums behind them.
+extern "C" long linear_few_room(int M, int O, int K, int* numbers) {
+  const int split = few_split(M, O, K, 0, false);
+  const int tiles = (O + 63) / 64 * 4 * (M <= 16 ? 2 : (M + 31) / 32 * 2);
+  *numbers = split > 1 ? tiles : 0;
+  return (long)*numbers * split * WAVE * 4;
+}
+
 // Strides in elements; 16-byte loads: x, w, norm and the strides of x and w are
-// multiples of 8 elements, K of 32.  M up to 64.
+// multiples of 8 elements, K of 32.  M up to 64.  count, part: room for a shared
+// contraction, or null; zero: n_zero numbers to clear for one behind this.
 extern "C" void launch_linear_few(const void* x, const void* w, const void* bias,
                                   const void* res, const void* norm, void* y,
                                   int M, int O, int K, long ldx, long ldw,
                                   long ldr, long ldy, float eps, float offset,
-                                  int act, hipStream_t stream) {
+                                  int act, unsigned* count, float* part,
+                                  unsigned* zero, int n_zero, hipStream_t stream) {
   const LinearFewArgs a{(const __bf16*)x, (const __bf16*)w, (const __bf16*)bias,
                         (const __bf16*)res, (const __bf16*)norm, (__bf16*)y,
-                        M, O, K, ldx, ldw, ldr, ldy, eps, offset};
-  // long rows: 16 of 14336 into 4096 take 29 us above, 27 below
-  if (M > 16 || (M > 8 && K > 8192)) {
-    linear_some(a, act, stream);
+                        M, O, K, ldx, ldw, ldr, ldy, eps, offset, part, count, zero,
+                        n_zero, 0};
+  const int split = count ? few_split(M, O, K, act, norm != nullptr) : 1;
+  if (few_through_lds(M, O, K, act)) {
+    linear_some(a, act, split, stream);
   } else {
-    linear_few_tiles(a, act, stream);
+    linear_few_tiles(a, act, split, stream);
   }
 }

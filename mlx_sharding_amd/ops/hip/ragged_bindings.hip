@@ -818,6 +818,7 @@ Tensor cap_logits(Tensor z, double scale, double limit) {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("glu", &glu);
   m.def("linear_few_try", &linear_few_try);
+  m.def("feed_few_try", &feed_few_try);
   m.def("clamped_glu", &clamped_glu, py::arg("gate"), py::arg("up"),
         py::arg("limit"), py::arg("alpha"), py::arg("gate_bias") = py::none(),
         py::arg("up_bias") = py::none());
