@@ -98,7 +98,7 @@ class Linear(nn.Module):
         return y
 
 
-def _weight(m, in_features: int) -> Optional[torch.Tensor]:
+def dense_weight(m, in_features: int) -> Optional[torch.Tensor]:
     """The weights of a Linear or FusedColumns, packed ones through their bf16 copy;
     None where there is no room for it."""
     q = m.quant
@@ -113,7 +113,8 @@ def feed(into, out, x: torch.Tensor, act: str, norm: Optional[nn.Module] = None,
     """The gated unit of ``into``'s halves through ``out``, as ``project`` of each; one
     call for few rows."""
     if into.bias is None and out.bias is None and x.is_cuda:
-        w_in, w_out = _weight(into, x.shape[-1]), _weight(out, sum(into.splits) // 2)
+        w_in = dense_weight(into, x.shape[-1])
+        w_out = dense_weight(out, sum(into.splits) // 2)
         if w_in is not None and w_out is not None:
             y = ops.feed_few(x, w_in, w_out, act, norm, residual)
             if y is not None:
@@ -126,7 +127,7 @@ def project(m, x: torch.Tensor, *, norm: Optional[nn.Module] = None,
             residual: Optional[torch.Tensor] = None) -> torch.Tensor:
     """ops.project with the weights of a Linear or FusedColumns, packed ones
     through their bf16 copy."""
-    w, q = _weight(m, x.shape[-1]), m.quant
+    w, q = dense_weight(m, x.shape[-1]), m.quant
     if w is not None:
         return ops.project(x, w, m.bias, norm=norm, act=act, residual=residual)
     # no room for the copy

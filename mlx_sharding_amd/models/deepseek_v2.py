@@ -18,7 +18,8 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, QuantConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import (Linear, RMSNorm, StageModel, as_built, owned_layer_indices, project,
+from .base import (Linear, RMSNorm, StageModel, as_built, dense_weight,
+                   owned_layer_indices, project,
                    read_in_place)
 from .llama import LlamaMLP, _Inner
 
@@ -480,10 +481,21 @@ class DeepseekV2MoE(nn.Module):
                                        m.down_proj.weight, self.top_k,
                                        *self._packing()))
 
+    def _beside(self, y):
+        """The shared experts' matrices, where they go with the routed ones."""
+        m = self.shared_experts
+        if (m is None or m._fused_gu is None or not as_built(m, m.down_proj)
+                or m._fused_gu.bias is not None or m.down_proj.bias is not None
+                or not ops.few_tokens(y)):
+            return None
+        both = (dense_weight(m._fused_gu, y.shape[1]),
+                dense_weight(m.down_proj, m.down_proj.in_features))
+        return both if ops.expert_shared_ok(*y.shape, *both) else None
+
     def decode(self, x, residual, norm):
         """The residual x (+ residual) after this feed-forward of it, normed:
-        three kernels for the routed experts, with norm, router and choice in a
-        fourth."""
+        three kernels for the routed and the shared experts, with norm, router and
+        choice in a fourth."""
         shape, H = x.shape, x.shape[-1]
         y, h, choice, weight = ops.expert_route(
             x.reshape(-1, H), None if residual is None else residual.reshape(-1, H),
@@ -492,8 +504,12 @@ class DeepseekV2MoE(nn.Module):
         m = self.switch_mlp
         stacks = [[p.weight] if m.quant is None else [p.weight, p.scales, p.biases]
                   for p in (m.gate_proj, m.up_proj, m.down_proj)]
-        rows = ops.expert_rows(y, choice, weight, *stacks, *self._packing())
-        shared = None if self.shared_experts is None else self.shared_experts(y)
+        packed, beside = self._packing(), self._beside(y)
+        if beside is not None:
+            rows, shared = ops.expert_rows(y, choice, weight, *stacks, *packed, beside)
+        else:
+            rows = ops.expert_rows(y, choice, weight, *stacks, *packed)
+            shared = None if self.shared_experts is None else self.shared_experts(y)
         return ops.expert_sum(rows, h, shared, y.shape[0]).view(shape)
 
     def forward(self, x):

@@ -658,12 +658,25 @@ def _whole(t: torch.Tensor) -> torch.Tensor:
     return t.clone() if t.data_ptr() % 16 else t
 
 
-def expert_rows(y, choice, weight, gate, up, down, bits: int, group_size: int):
+def expert_rows(y, choice, weight, gate, up, down, bits: int, group_size: int,
+                shared=None):
     """The chosen experts' weighted outputs, fp32 [N * top, H]; gate, up, down:
-    [matrix] in bf16 or [packed, scales, biases]."""
-    return _require_ext("moe_rows").moe_rows(
+    [matrix] in bf16 or [packed, scales, biases].  shared: ([2 S, H], [H, S]) of a
+    feed-forward that all tokens pass (expert_shared_ok); then (those, its rows)."""
+    rows, other = _require_ext("moe_rows").moe_rows(
         y, choice, weight, *(_expert_stack(m, bits, group_size)
-                             for m in (gate, up, down)), bits, group_size)
+                             for m in (gate, up, down)), bits, group_size,
+        *(shared or (None, None)))
+    return rows if shared is None else (rows, other)
+
+
+def expert_shared_ok(n_tokens: int, H: int, w_in, w_out) -> bool:
+    """Whether expert_rows takes a shared feed-forward of these matrices along."""
+    return (n_tokens <= 8 and w_in is not None and w_out is not None
+            and w_out.shape[-1] % 64 == 0 and max(H, w_out.shape[-1]) <= 4096
+            and tuple(w_in.shape) == (2 * w_out.shape[-1], H) and w_out.shape[0] == H
+            and all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in (w_in, w_out)))
 
 
 def _expert_stack(m, bits: int, group_size: int) -> torch.Tensor:

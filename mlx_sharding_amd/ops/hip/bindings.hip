@@ -1049,17 +1049,20 @@ static ExpertStack expert_stack(const torch::Tensor& t, int bits, int gs) {
   return s;
 }
 
-// Every pair's expert output, weighted, fp32 [N * top, H]; bits 16: bf16 stacks
-torch::Tensor moe_rows(torch::Tensor x, torch::Tensor choice,
-                       torch::Tensor weight, torch::Tensor gate,
-                       torch::Tensor up, torch::Tensor down, int64_t bits,
-                       int64_t gs) {
+// Every pair's expert output, weighted, fp32 [N * top, H]; bits 16: bf16 stacks.
+// shared_in [2 S, H], shared_out [H, S]: a feed-forward that all tokens (up to 8) pass,
+// whose bf16 rows [N, H] come behind (no rows without).
+std::vector<torch::Tensor> moe_rows(torch::Tensor x, torch::Tensor choice,
+                                    torch::Tensor weight, torch::Tensor gate,
+                                    torch::Tensor up, torch::Tensor down, int64_t bits,
+                                    int64_t gs, c10::optional<torch::Tensor> shared_in,
+                                    c10::optional<torch::Tensor> shared_out) {
   TORCH_CHECK(bits == 4 || bits == 8 || bits == 16, "4, 8 or 16 bits");
   TORCH_CHECK(bits == 16 || gs == 32 || gs == 64 || gs == 128, "group size");
   const auto g = expert_stack(gate, bits, gs), u = expert_stack(up, bits, gs),
              d = expert_stack(down, bits, gs);
   TORCH_CHECK(g.E == u.E && g.O == u.O && g.K == u.K && d.E == g.E &&
-                  d.O == g.K && d.K == g.O, "stacks of one shape");
+                  d.O == g.K && d.K == g.O && g.E <= 64, "stacks of one shape");
   TORCH_CHECK(choice.dim() == 2 && choice.is_contiguous() &&
                   choice.scalar_type() == torch::kInt32 && choice.is_cuda() &&
                   weight.sizes() == choice.sizes() && weight.is_contiguous() &&
@@ -1068,24 +1071,46 @@ torch::Tensor moe_rows(torch::Tensor x, torch::Tensor choice,
   const long N = choice.size(0), P = choice.numel();
   TORCH_CHECK(P >= 1 && P <= MR_PAIRS, "up to ", MR_PAIRS, " pairs");
   check_rows(x, "x", N, g.K);
+  TORCH_CHECK(shared_in.has_value() == shared_out.has_value(), "both or none");
+  const long S = shared_in.has_value() ? shared_out->size(-1) : 0;
+  if (shared_in.has_value()) {
+    TORCH_CHECK(N <= 8 && S >= 64 && S % 64 == 0 && std::max(S, g.K) <= 16 * 256,
+                "sizes of the shared feed-forward");
+    check_rows(*shared_in, "shared_in", 2 * S, g.K);
+    check_rows(*shared_out, "shared_out", g.K, S);
+  }
   auto h = torch::empty({P, g.O}, x.options().dtype(bits == 16 ? torch::kBFloat16
                                                                 : torch::kHalf));
   auto y = torch::empty({P, d.O}, x.options().dtype(torch::kFloat32));
-  // Rows of weights per block: as many as leave 512 blocks, two a CU, all at work
-  // at once (64 tokens, 64 experts, 4 bits: 89 us; 116 with 256 blocks, 103 with
-  // 1024).
-  auto tiles = [&](long O) {
-    return (int)std::max<long>(1, O / 16 * std::min(g.E, P) / 512);
-  };
+  auto hs = torch::empty({N, S}, x.options());
+  auto ys = torch::empty({S ? N : 0, d.O}, x.options());
   MoeRowsArgs a{x.data_ptr(), g.w, u.w, h.data_ptr(),
                 choice.data_ptr<int>(), weight.data_ptr<float>(), (int)P,
-                (int)choice.size(1), (int)g.E, (int)g.O, (int)g.K, tiles(g.O)};
+                (int)choice.size(1), (int)g.E, (int)g.O, (int)g.K};
+  if (S) {
+    a.dx = (const __bf16*)x.data_ptr();
+    a.dw = (const __bf16*)shared_in->data_ptr();
+    a.dy = (__bf16*)hs.data_ptr();
+    a.dense = (int)S / 16;
+    a.N = (int)N;
+    a.DO = (int)S;
+    a.DK = (int)g.K;
+  }
   launch_moe_rows(&a, (int)bits, (int)gs, true, cur_stream());
-  a = MoeRowsArgs{h.data_ptr(), d.w, nullptr, y.data_ptr(), choice.data_ptr<int>(),
-                  weight.data_ptr<float>(), (int)P, (int)choice.size(1), (int)d.E,
-                  (int)d.O, (int)d.K, tiles(d.O)};
-  launch_moe_rows(&a, (int)bits, (int)gs, false, cur_stream());
-  return y;
+  MoeRowsArgs b{h.data_ptr(), d.w, nullptr, y.data_ptr(), choice.data_ptr<int>(),
+                weight.data_ptr<float>(), (int)P, (int)choice.size(1), (int)d.E,
+                (int)d.O, (int)d.K};
+  if (S) {
+    b.dx = (const __bf16*)hs.data_ptr();
+    b.dw = (const __bf16*)shared_out->data_ptr();
+    b.dy = (__bf16*)ys.data_ptr();
+    b.dense = (int)d.O / 16;
+    b.N = (int)N;
+    b.DO = (int)d.O;
+    b.DK = (int)S;
+  }
+  launch_moe_rows(&b, (int)bits, (int)gs, false, cur_stream());
+  return {y, ys};
 }
 
 // A token's pairs, and the rows h and shared where given, added up in 32 bits

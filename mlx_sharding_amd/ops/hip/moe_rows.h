@@ -12,7 +12,12 @@ struct MoeRowsArgs {
   const int* choice;         // [pairs] expert
   const float* weight;       // [pairs]
   int pairs, top, experts, O, K;
-  int tiles;                 // of 16 rows of w, per block
+  // the token's shared feed-forward in the same launch: its first `dense` = DO / 16
+  // blocks (or none).  dw: bf16 [2 DO, DK] (up: the gate's rows, the up projection's) or
+  // [DO, DK] (down); rows dx [N, DK] of it, results dy [N, DO]
+  const __bf16 *dx, *dw;
+  __bf16* dy;
+  int dense, N, DO, DK;
 };
 
 struct MoeRouteArgs {

@@ -6,8 +6,9 @@
 //   moe_down     the pairs' outputs, weighted, in 32 bits
 //   moe_combine  a token's pairs, shared experts and residual added up
 //
-// No sort: a block of an expert looks through the choices (at most 1024) for its
-// pairs.  Rows of pairs lie at token * top + place.
+// No sort: a block counts every expert's pairs, which tells its share of the work, and
+// looks through the choices (at most 1024) for those of an expert.  Rows of pairs lie at
+// token * top + place.
 //
 // The products are bound by reading the experts' packed weights.  Read naively,
 // rows of x out of L2 are twice those bytes and more (16 rows of 16 bits for 16
@@ -106,6 +107,87 @@ struct Packed {
 
 // -- products ---------------------------------------------------------------
 
+// A tile of the shared feed-forward for up to 8 tokens: the waves take the contraction by
+// turns in steps of 64 (two loads of a row, one line of 128 bytes).  Bound by what a CU
+// reads, about 30 bytes a nanosecond, so every tile has a block (one token, with 16, 32,
+// 64, 128, 176 blocks of 176 tiles beside the experts': 126, 70, 41, 32, 26 us; after
+// them 34, as two kernels).  More tokens need the blocks for experts: 16 alone 81 us, so 85.
+template <bool UP>
+__device__ __forceinline__ void dense_tiles(const MoeRowsArgs& a, f32x4* red) {
+  constexpr int MATS = UP ? 2 : 1;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int l16 = lane & 15, lg = lane >> 4;
+  auto load = [](const __bf16* p) { return *reinterpret_cast<const bf16x8_t*>(p); };
+  const __bf16* xp = a.dx + (long)min(l16, a.N - 1) * a.DK + lg * 8;
+  const int t = blockIdx.x;
+  const __bf16* wp[MATS];
+  f32x4 acc[MATS];
+#pragma unroll
+  for (int m = 0; m < MATS; ++m) {
+    wp[m] = a.dw + ((long)m * a.DO + t * 16 + l16) * a.DK + lg * 8;
+    acc[m] = f32x4{0, 0, 0, 0};
+  }
+  // three ahead: what a wave has of 2048 columns is four
+  constexpr int AHEAD = 4;
+  struct Part {
+    bf16x8_t w[MATS][2], x[2];
+  } part[AHEAD];
+  auto fetch = [&](Part& f, int k) {
+    if (k >= a.DK) return;
+#pragma unroll
+    for (int m = 0; m < MATS; ++m)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) f.w[m][i] = load(wp[m] + k + i * 32);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) f.x[i] = load(xp + k + i * 32);
+  };
+  constexpr int STEP = MR_WAVES * 64;
+#pragma unroll
+  for (int p = 0; p < AHEAD - 1; ++p) fetch(part[p], wid * 64 + p * STEP);
+  for (int k = wid * 64; k < a.DK; k += AHEAD * STEP) {
+#pragma unroll
+    for (int p = 0; p < AHEAD; ++p) {
+      if (k + p * STEP >= a.DK) break;
+      fetch(part[(p + AHEAD - 1) % AHEAD], k + (p + AHEAD - 1) * STEP);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int m = 0; m < MATS; ++m)
+          acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[p].w[m][i],
+                                                           part[p].x[i], acc[m], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < MATS; ++m) red[(wid * MATS + m) * WAVE + lane] = acc[m];
+  __syncthreads();
+  if (wid != 0 || l16 >= a.N) return;
+  f32x4 v[MATS];
+#pragma unroll
+  for (int m = 0; m < MATS; ++m) {
+    v[m] = red[m * WAVE + lane];
+#pragma unroll
+    for (int w = 1; w < MR_WAVES; ++w) {
+      const f32x4 p = red[(w * MATS + m) * WAVE + lane];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[m][j] += p[j];
+    }
+  }
+  bf16x4_t h;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float g = v[0][j];
+    h[j] = (__bf16)(UP ? g / (1.0f + __expf(-g)) * v[MATS - 1][j] : g);
+  }
+  *reinterpret_cast<bf16x4_t*>(a.dy + (long)l16 * a.DO + t * 16 + lg * 4) = h;
+}
+
+// Work is counted in tiles: 16 rows of an expert's matrices by up to 16 of its pairs.
+// Every block counts the pairs of all experts and takes an even share of all tiles, one
+// after the other.  With a block per expert and range of rows the longest one has the
+// expert with most pairs (64 experts of 1408 x 2048 at 4 bits, 64 tokens: an expert has 12
+// of them 91 us so, 90 shared; 52 179, 70; 128 tokens, 22 126, 112; one token 18.3, 20.2,
+// which is the counting).
 template <int BITS, int GS, int UPW, bool UP>
 __global__ __launch_bounds__(
     MR_BLOCK, UPW <= (BITS == 16 && UP ? 1 : 2) ? 4 : 2) void moe_rows_kernel(
@@ -113,59 +195,89 @@ __global__ __launch_bounds__(
   typedef Operand<BITS> Op;
   typedef typename Op::V V;
   constexpr int MATS = UP ? 2 : 1;
-  __shared__ short list[MR_PAIRS];
-  __shared__ int found;
+  __shared__ int count[64], ends[64];
+  __shared__ short list[16];
   __shared__ __attribute__((aligned(16))) f32x4 red[2][MR_WAVES][MATS][WAVE];
 
+  if ((int)blockIdx.x < a.dense) {
+    dense_tiles<UP>(a, &red[0][0][0][0]);
+    return;
+  }
   const int lane = threadIdx.x & (WAVE - 1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l16 = lane & 15, lg = lane >> 4;
-  // a block per expert, or where there are fewer pairs per pair: of its expert, if
-  // it is the first of it
-  const bool by_pair = gridDim.y < (unsigned)a.experts;
-  const int e = by_pair ? a.choice[blockIdx.y] : blockIdx.y;
-  if (wid == 0) {
-    int n = 0;
-    for (int i = 0; i < a.pairs; i += WAVE) {
-      const bool mine = i + lane < a.pairs && a.choice[i + lane] == e;
-      const unsigned long long all = __ballot(mine);
-      if (mine) list[n + __popcll(all & ((1ull << lane) - 1))] = (short)(i + lane);
-      n += __popcll(all);
-    }
-    if (lane == 0) found = n;
+  const int rows = a.O / 16;
+  if (threadIdx.x < 64) count[threadIdx.x] = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < a.pairs; i += MR_BLOCK) {
+    const unsigned e = a.choice[i];
+    if (e < (unsigned)a.experts) atomicAdd(&count[e], 1);
   }
   __syncthreads();
-  const int n = by_pair && list[0] != (int)blockIdx.y ? 0 : found;
-  if (n == 0) return;
-  const int t0 = blockIdx.x * a.tiles, t1 = min(t0 + a.tiles, a.O / 16);
+  if (wid == 0) {
+    int n = (count[lane] + 15) / 16;  // groups of pairs up to this expert
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) {
+      const int o = __shfl_up(n, off, WAVE);
+      if (lane >= off) n += o;
+    }
+    ends[lane] = n;
+  }
+  __syncthreads();
+  const unsigned all = ends[63] * rows, blocks = gridDim.x - a.dense;
+  const unsigned b = blockIdx.x - a.dense;
+  int at = b * all / blocks;
+  const int stop = (b + 1) * all / blocks;
 
   const int units = a.K / MR_UNIT;
-  // this lane's place in its first unit of the block's first rows
   const int k0 = wid * MR_UNIT + lg * 32;
   constexpr int UNIT = (16 * MR_UNIT * BITS / 32 + 16 * (MR_UNIT / GS)) * 4;
   const long step = BITS == 16 ? (long)16 * a.K * 2 : (long)units * UNIT;
-  const long begin = ((long)e * (a.O / 16) + t0) * step +
-                     (BITS == 16 ? ((long)l16 * a.K + k0) * 2
-                                 : (long)wid * UNIT + lane * 16);
   const int scales = 16 * MR_UNIT * BITS / 8 - lane * 16 +
                      (l16 * (MR_UNIT / GS) + lg * 32 / GS) * 4;
-  const char* wp[2] = {(const char*)a.w + begin, (const char*)a.w2 + begin};
-  auto fetch = [&](Packed<BITS>& r, int m, int u, int t) {
-    constexpr int far = MR_WAVES * (BITS == 16 ? MR_UNIT * 2 : UNIT);
-    const char* p = wp[m] + t * step + (long)u * far;  // between a wave's units
-    r.load(p, p + scales);
-  };
-
   int buf = 0;
-  for (int first = 0; first < n; first += 16) {
-    const int pair = list[min(first + l16, n - 1)];
-    V x[UPW][4];
+  while (at < stop) {
+    // one group of one expert's pairs, rows t0 to t1
+    const int group = at / rows, t0 = at - group * rows;
+    const int t1 = min(rows, t0 + stop - at);
+    at += t1 - t0;
+    const int e = __popcll(__ballot(ends[lane] <= group));
+    const int first = (group - (e ? ends[e - 1] : 0)) * 16;
+    const int n = min(16, count[e] - first);
+
+    // this lane's place in its first unit of the first rows
+    const long begin = ((long)e * rows + t0) * step +
+                       (BITS == 16 ? ((long)l16 * a.K + k0) * 2
+                                   : (long)wid * UNIT + lane * 16);
+    const char* wp[2] = {(const char*)a.w + begin, (const char*)a.w2 + begin};
+    auto fetch = [&](Packed<BITS>& r, int m, int u, int t) {
+      constexpr int far = MR_WAVES * (BITS == 16 ? MR_UNIT * 2 : UNIT);
+      const char* p = wp[m] + t * step + (long)u * far;  // between a wave's units
+      r.load(p, p + scales);
+    };
     Packed<BITS> next[MATS][UPW];
 #pragma unroll
     for (int u = 0; u < UPW; ++u) {
       if (wid + u * MR_WAVES >= units) continue;
 #pragma unroll
       for (int m = 0; m < MATS; ++m) fetch(next[m][u], m, u, 0);
+    }
+    if (wid == 0) {
+      int found = -first;
+      for (int i = 0; i < a.pairs && found < 16; i += WAVE) {
+        const bool mine = i + lane < a.pairs && a.choice[i + lane] == e;
+        const unsigned long long which = __ballot(mine);
+        const int place = found + __popcll(which & ((1ull << lane) - 1));
+        if (mine && place >= 0 && place < 16) list[place] = (short)(i + lane);
+        found += __popcll(which);
+      }
+    }
+    __syncthreads();
+    const int pair = list[min(l16, n - 1)];
+    V x[UPW][4];
+#pragma unroll
+    for (int u = 0; u < UPW; ++u) {
+      if (wid + u * MR_WAVES >= units) continue;
       const short* src = (const short*)a.x +
                          (long)(UP ? pair / a.top : pair) * a.K + k0 +
                          u * MR_WAVES * MR_UNIT;
@@ -213,8 +325,8 @@ __global__ __launch_bounds__(
           for (int j = 0; j < 4; ++j) v[m][j] += p[j];
         }
       }
-      if (first + l16 >= n) continue;
-      const long at = (long)pair * a.O + t * 16 + lg * 4;
+      if (l16 >= n) continue;
+      const long to = (long)pair * a.O + t * 16 + lg * 4;
       if constexpr (UP) {
         typedef typename Op::H H4;
         H4 h;
@@ -223,12 +335,12 @@ __global__ __launch_bounds__(
           const float g = v[0][j];
           h[j] = (typename Op::E)(g / (1.0f + __expf(-g)) * v[MATS - 1][j]);
         }
-        *reinterpret_cast<H4*>((typename Op::E*)a.y + at) = h;
+        *reinterpret_cast<H4*>((typename Op::E*)a.y + to) = h;
       } else {
         const float w = a.weight[pair];
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[0][j] *= w;
-        *reinterpret_cast<f32x4*>((float*)a.y + at) = v[0];
+        *reinterpret_cast<f32x4*>((float*)a.y + to) = v[0];
       }
     }
   }
@@ -297,8 +409,10 @@ extern "C" void launch_moe_pack(const void* w, const void* scale,
 
 template <int BITS, int GS, bool UP>
 static void moe_rows_go(const MoeRowsArgs& a, hipStream_t stream) {
-  const dim3 grid((unsigned)((a.O / 16 + a.tiles - 1) / a.tiles),
-                  (unsigned)min(a.experts, a.pairs));
+  // Two blocks a CU, all at work at once (64 tokens, 64 experts, 4 bits: 89 us; 116 with
+  // one, 103 with four), or a tile each where there are fewer.
+  const dim3 grid((unsigned)(
+      a.dense + min(512 - a.dense, a.O / 16 * min(a.experts, a.pairs))));
   const dim3 block(MR_BLOCK);
   const int upw = (a.K / MR_UNIT + MR_WAVES - 1) / MR_WAVES;
   if (upw <= 1) {
