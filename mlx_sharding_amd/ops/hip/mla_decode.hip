@@ -106,7 +106,7 @@ __global__ __launch_bounds__(MD_BLOCK) void mla_prepare_kernel(
   }
 }
 
-// grid: (heads, tiles of 16 tokens); all of a head's output columns
+// grid: (heads, tiles of 16 tokens, parts of a head's output columns)
 __global__ __launch_bounds__(512) void mla_finish_kernel(const MlaFinishArgs a) {
   // a token's latent [16][rank + 8] in bf16: the odd stride keeps the 16 rows that
   // a read meets in different banks
@@ -117,6 +117,9 @@ __global__ __launch_bounds__(512) void mla_finish_kernel(const MlaFinishArgs a) 
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int h = blockIdx.x, t0 = blockIdx.y * 16, n = a.slices;
   const int stride = a.rank + 8;
+  const int part = (a.vdim / 16 + gridDim.z - 1) / gridDim.z * 16;
+  const int first = blockIdx.z * part + wid * 16;
+  const int last = min(a.vdim, (int)(blockIdx.z + 1) * part);
   // the first rows of the matrix are asked for before the slices
   const int l16 = lane & 15, lg = lane >> 4;
   auto rows = [&](int r0) {
@@ -129,7 +132,7 @@ __global__ __launch_bounds__(512) void mla_finish_kernel(const MlaFinishArgs a) 
       if (k + i * 32 < a.rank)
         wf[i] = *reinterpret_cast<const bf16x8_t*>(w + k + i * 32);
   };
-  if (wid * 16 < a.vdim) fetch(rows(wid * 16), 0);
+  if (first < last) fetch(rows(first), 0);
   for (int i = wid; i < 16; i += 8) {
     const long row = (long)min(t0 + i, a.N - 1) * a.heads + h;
     const float m = lane < n ? a.part_ml[(row * n + lane) * 2] : -1e30f;
@@ -159,10 +162,10 @@ __global__ __launch_bounds__(512) void mla_finish_kernel(const MlaFinishArgs a) 
   __syncthreads();
   const int tok = min(l16, a.N - 1 - t0);
   const __bf16* x = lat + tok * stride + lg * 8;
-  for (int r0 = wid * 16; r0 < a.vdim; r0 += 128) {
+  for (int r0 = first; r0 < last; r0 += 128) {
     f32x4 acc = {0, 0, 0, 0};
     for (int k = 0; k < a.rank; k += 512) {
-      if (r0 + k != wid * 16) fetch(rows(r0), k);
+      if (r0 + k != first) fetch(rows(r0), k);
 #pragma unroll
       for (int i = 0; i < 16; ++i)
         if (k + i * 32 < a.rank)
@@ -232,6 +235,10 @@ extern "C" void launch_mla_prepare(const MlaPrepareArgs* a, hipStream_t stream) 
 }
 
 extern "C" void launch_mla_finish(const MlaFinishArgs* a, hipStream_t stream) {
-  mla_finish_kernel<<<dim3((unsigned)a->heads, (unsigned)((a->N + 15) / 16)),
+  // A CU reads about 30 bytes a nanosecond: 128 KB of a matrix and 128 KB or more of
+  // slices.  Parts share the slices, which then come from L2 (16 heads of 128 x 512, one
+  // token and 64; 1, 2, 4, 8 parts: 10.9, 9.0, 8.0, 7.6 us and 10.9, 8.9, 8.3, 12.8).
+  const unsigned parts = a->vdim % 64 ? 1 : 4;
+  mla_finish_kernel<<<dim3((unsigned)a->heads, (unsigned)((a->N + 15) / 16), parts),
                       dim3(512), (size_t)16 * (a->rank + 8) * 2, stream>>>(*a);
 }
