@@ -153,6 +153,25 @@ class RMSNorm(nn.Module):
         return ops.rms_norm(x, self.weight, self.eps, self.weight_offset)
 
 
+read_in_place(nn.Embedding)
+
+
+def head(norm: nn.Module, x: torch.Tensor, out: Optional[nn.Module] = None,
+         table: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``out``, or the product with an embedding's rows, of x's normed rows; one kernel
+    for few rows.  For 33 to 64 of them and more than 2^25 weights the library's product
+    is the faster one (linear_few.h), and the norm stays a kernel of its own."""
+    V, K = table.shape if out is None else (out.out_features, out.in_features)
+    if (ops.few_tokens(x) and (x.numel() <= 32 * K or V * K <= 1 << 25)
+            and as_built(norm)):
+        if out is None:
+            return ops.project(x, table, norm=norm)
+        if as_built(out):
+            return project(out, x, norm=norm)
+    x = norm(x)
+    return x @ table.t() if out is None else out(x)
+
+
 class StageModel(nn.Module):
     """Base class for one pipeline stage of a sharded model.
 
@@ -193,6 +212,27 @@ class StageModel(nn.Module):
             self._rt_sin = sin.contiguous()
             self._rt_len, self._rt_dev = n, device
         return self._rt_cos, self._rt_sin
+
+    def begin(self, x: torch.Tensor, cache, embed: Optional[nn.Module] = None,
+              scale: Optional[torch.Tensor] = None):
+        """(hidden states, cos, sin) of this forward: x, or its rows of ``embed``
+        (times ``scale``), and its positions' rotations."""
+        first = cache[0] if cache else None
+        if embed is None:
+            h = x
+        else:
+            pos = first.graph_pos if first is not None else None
+            if (pos is not None and x.shape[1] == 1 and type(embed) is nn.Embedding
+                    and as_built(embed) and embed.max_norm is None):
+                found = ops.step_begin(x, embed.weight, scale, pos,
+                                       *self._rope_tables(x.device, first.capacity))
+                if found is not None:
+                    return found
+            h = embed(x)
+            if scale is not None:
+                h = h * scale.to(h.dtype)
+        cos, sin, _ = self.rope_for(first, h.shape[1], h.device)
+        return h, cos, sin
 
     def rope_for(self, cache0, T: int, device):
         """(cos, sin, offset) for this forward; handles graph-pos mode

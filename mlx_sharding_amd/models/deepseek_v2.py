@@ -18,9 +18,8 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, QuantConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import (Linear, RMSNorm, StageModel, as_built, dense_weight,
-                   owned_layer_indices, project,
-                   read_in_place)
+from .base import (Linear, RMSNorm, StageModel, as_built, dense_weight, head,
+                   owned_layer_indices, project, read_in_place)
 from .llama import LlamaMLP, _Inner
 
 
@@ -661,13 +660,11 @@ class DeepseekV2StageModel(StageModel):
         return False
 
     def forward(self, x: torch.Tensor, cache: Optional[List[KVCache]] = None) -> torch.Tensor:
-        h = self.model.embed_tokens(x) if self.shard.is_first else x
-        T = h.shape[1]
-        cos, sin, _ = self.rope_for(cache[0] if cache else None, T, h.device)
+        h, cos, sin = self.begin(
+            x, cache, self.model.embed_tokens if self.shard.is_first else None)
         for j, i in enumerate(owned_layer_indices(self.shard)):
             c = cache[j] if cache is not None else None
             h = self.model.layers[str(i)](h, cos, sin, c)
         if self.shard.is_last:
-            h = self.model.norm(h)
-            h = self.lm_head(h)
+            h = head(self.model.norm, h, self.lm_head)
         return h

@@ -16,8 +16,8 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import (Linear, RMSNorm, StageModel, as_built, feed, owned_layer_indices,
-                   project, read_in_place)
+from .base import (Linear, RMSNorm, StageModel, as_built, feed, head,
+                   owned_layer_indices, project, read_in_place)
 
 
 @read_in_place
@@ -193,19 +193,14 @@ class LlamaStageModel(StageModel):
         return [(nkv, hd, hd) for _ in range(self.shard.n_layers)]
 
     def forward(self, x: torch.Tensor, cache: Optional[List[KVCache]] = None) -> torch.Tensor:
-        if self.shard.is_first:
-            h = self.model.embed_tokens(x)
-        else:
-            h = x
-        T = h.shape[1]
-        cos, sin, _ = self.rope_for(cache[0] if cache else None, T, h.device)
+        h, cos, sin = self.begin(
+            x, cache, self.model.embed_tokens if self.shard.is_first else None)
         for j, i in enumerate(owned_layer_indices(self.shard)):
             c = cache[j] if cache is not None else None
             h = self.model.layers[str(i)](h, cos, sin, c)
         if self.shard.is_last:
-            h = self.model.norm(h)
             if self.tie_word_embeddings:
-                h = h @ self.model.embed_tokens.weight.t()
+                h = head(self.model.norm, h, table=self.model.embed_tokens.weight)
             else:
-                h = self.lm_head(h)
+                h = head(self.model.norm, h, self.lm_head)
         return h

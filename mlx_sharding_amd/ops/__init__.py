@@ -116,6 +116,33 @@ def norm_add(x, norm, residual, then=None):
     return h if then is None else (h, then(h))
 
 
+def step_begin(tokens, table, scale, pos, cos, sin):
+    """What a captured decoding step begins with, in one kernel: the rows of an embedding
+    for tokens (times ``scale``) and the row of rotations of the position; None where
+    that kernel does not take them."""
+    if not (use_native(tokens) and tokens.dtype == torch.int64 and tokens.numel()
+            and tokens.is_contiguous()
+            and pos.dtype == torch.int32 and pos.numel() == 1
+            and all(_plain(t) and t.device == tokens.device
+                    for t in (tokens, table, pos, cos, sin))
+            and table.dtype == torch.bfloat16 and table.is_contiguous()
+            and table.shape[1] % 8 == 0 and table.data_ptr() % 16 == 0
+            and (scale is None or (_plain(scale) and scale.dtype == torch.bfloat16
+                                   and scale.device == tokens.device))):
+        return None
+    return hip_ext().step_begin(tokens, table, scale, pos, cos, sin)
+
+
+def step_end(logits, pos):
+    """Logits [rows, vocabulary] in fp32; the position moves on."""
+    if (use_native(logits) and logits.dtype == torch.bfloat16 and logits.numel()
+            and logits.stride(-1) == 1 and logits.shape[0] < 65536 and _plain(logits)):
+        return hip_ext().step_end(logits, pos)
+    out = logits.float()
+    pos.add_(1)
+    return out
+
+
 def apply_rope(x, cos, sin, interleaved: bool = False):
     if _use_hip(x):
         return _require_ext("apply_rope").apply_rope(

@@ -31,6 +31,10 @@ void launch_mla_append_kv(const void*, const void*, void*, void*, const int*,
 void launch_rope_qkv(const void*, const void*, const void*, const float*, const float*,
                      void*, void*, void*, const int*, long, long, int, int, int, int,
                      long, long, long, long, hipStream_t);
+void launch_step_begin(const long*, const void*, const void*, const int*, const float*,
+                       const float*, void*, float*, float*, long, long, int, long, int,
+                       hipStream_t);
+void launch_step_end(const void*, long, float*, int, int, int*, hipStream_t);
 void launch_rope_append_kv(const void*, const void*, const float*,
                            const float*, void*, void*, const int*, int, int,
                            int, int, int, long, bool, long, long,
@@ -311,6 +315,57 @@ torch::Tensor rope_qkv(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                   (int)D, kcache.size(2), row(q), row(k), row(v),
                   cur_stream());
   return out;
+}
+
+static void check_position(const torch::Tensor& pos) {
+  TORCH_CHECK(pos.is_cuda() && pos.scalar_type() == torch::kInt32 && pos.numel() == 1,
+              "one int32 position");
+}
+
+// The embedding rows of tokens [...] (times scale), and row pos of cos and sin.
+std::vector<torch::Tensor> step_begin(torch::Tensor tokens, torch::Tensor table,
+                                      c10::optional<torch::Tensor> scale,
+                                      torch::Tensor pos, torch::Tensor cos,
+                                      torch::Tensor sin) {
+  check_bf16(table, "embedding");
+  TORCH_CHECK(tokens.is_cuda() && tokens.scalar_type() == torch::kInt64 &&
+                  tokens.is_contiguous() && tokens.numel() >= 1, "tokens int64");
+  TORCH_CHECK(table.dim() == 2 && table.is_contiguous() && table.size(0) >= 1 &&
+                  table.size(1) >= 8 && table.size(1) % 8 == 0 &&
+                  reinterpret_cast<uintptr_t>(table.data_ptr()) % 16 == 0, "embedding");
+  if (scale.has_value()) {
+    check_bf16(*scale, "scale");
+    TORCH_CHECK(scale->numel() == 1, "one scale");
+  }
+  check_position(pos);
+  for (const auto& t : {cos, sin})
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kFloat32 && t.dim() == 2 &&
+                    t.is_contiguous() && t.sizes() == cos.sizes() && t.numel() >= 1,
+                "tables of rotations");
+  const long W = table.size(1), half = cos.size(1);
+  TORCH_CHECK(tokens.numel() * (W / 8) < (1L << 32), "sizes");
+  auto shape = tokens.sizes().vec();
+  shape.push_back(W);
+  auto h = torch::empty(shape, table.options());
+  auto c = torch::empty({1, half}, cos.options()), s = torch::empty({1, half}, cos.options());
+  launch_step_begin(tokens.data_ptr<long>(), table.data_ptr(),
+                    scale.has_value() ? scale->data_ptr() : nullptr, pos.data_ptr<int>(),
+                    cos.data_ptr<float>(), sin.data_ptr<float>(), h.data_ptr(),
+                    c.data_ptr<float>(), s.data_ptr<float>(), tokens.numel(),
+                    table.size(0), (int)W, cos.size(0), (int)half, cur_stream());
+  return {h, c, s};
+}
+
+// x [rows, n] in fp32; the position moves on.
+torch::Tensor step_end(torch::Tensor x, torch::Tensor pos) {
+  check_bf16(x, "logits");
+  check_position(pos);
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.size(0) >= 1 && x.size(0) < 65536 &&
+                  x.size(1) >= 1 && x.size(1) < (1L << 31) - 1024, "rows of logits");
+  auto y = torch::empty(x.sizes(), x.options().dtype(torch::kFloat32));
+  launch_step_end(x.data_ptr(), x.stride(0), y.data_ptr<float>(), (int)x.size(0),
+                  (int)x.size(1), pos.data_ptr<int>(), cur_stream());
+  return y;
 }
 
 // k/v [B, T, Hkv, D]; caches full buffers [B, Hkv, Scap, D]
@@ -1234,6 +1289,8 @@ std::vector<torch::Tensor> moe_gate_subranges(torch::Tensor logits, int64_t K,
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "fused RMSNorm (gfx950)");
   m.def("norm_add", &norm_add);
+  m.def("step_begin", &step_begin);
+  m.def("step_end", &step_end);
   m.def("rope_qkv", &rope_qkv, py::arg("q"), py::arg("k"), py::arg("v"),
         py::arg("cos"), py::arg("sin"), py::arg("kcache"), py::arg("vcache"),
         py::arg("pos") = py::none(), py::arg("pos0") = 0);

@@ -590,6 +590,81 @@ extern "C" void launch_rope_qkv(const void* q, const void* k, const void* v,
   rope_qkv_kernel<<<dim3((unsigned)((a.total + 255) / 256)), dim3(256), 0, stream>>>(a);
 }
 
+// ---------------------------------------------------------------------------
+// The two ends of a captured decoding step.  The first kernel takes the tokens' rows of
+// the embedding, scaled if asked for, and the rotations of the position; the last one
+// makes logits fp32 and moves the position on.  Bound by launch: each of the single
+// operations (one or two for the rows, a conversion and two selections for the
+// rotations; a conversion and an addition) takes 4 to 5 us within a captured step.
+// Tokens and positions outside their tables give NaN.
+// ---------------------------------------------------------------------------
+
+struct StepBeginArgs {
+  const long* tokens;      // [rows]
+  const __bf16 *table, *scale;  // [vocab, W]; scale: one value or null
+  const int* pos;
+  const float *cos, *sin;  // [places, half]
+  __bf16* h;               // [rows, W]
+  float *cos_at, *sin_at;  // [half]
+  long vocab, places, total;
+  int W, half;
+};
+
+__global__ __launch_bounds__(256) void step_begin_kernel(const StepBeginArgs a) {
+  const long at = (long)blockIdx.x * 256 + threadIdx.x;
+  if (at < a.half) {
+    const int p = *a.pos;
+    const bool in = p >= 0 && p < a.places;
+    a.cos_at[at] = in ? a.cos[(long)p * a.half + at] : __builtin_nanf("");
+    a.sin_at[at] = in ? a.sin[(long)p * a.half + at] : __builtin_nanf("");
+  }
+  if (at >= a.total) return;
+  const long row = at / (a.W / 8), d = at % (a.W / 8) * 8, token = a.tokens[row];
+  bf16x8_t v;
+  if (token >= 0 && token < a.vocab) {
+    v = *reinterpret_cast<const bf16x8_t*>(a.table + token * a.W + d);
+    if (a.scale) {
+      const float f = (float)*a.scale;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = (__bf16)((float)v[j] * f);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (__bf16)__builtin_nanf("");
+  }
+  *reinterpret_cast<bf16x8_t*>(a.h + row * a.W + d) = v;
+}
+
+// W a multiple of 8, table and h on whole 16-byte vectors
+extern "C" void launch_step_begin(const long* tokens, const void* table,
+                                  const void* scale, const int* pos, const float* cos,
+                                  const float* sin, void* h, float* cos_at,
+                                  float* sin_at, long rows, long vocab, int W,
+                                  long places, int half, hipStream_t stream) {
+  StepBeginArgs a{tokens, (const __bf16*)table, (const __bf16*)scale, pos, cos, sin,
+                  (__bf16*)h, cos_at, sin_at, vocab, places, rows * (W / 8), W, half};
+  const long n = a.total > half ? a.total : half;
+  step_begin_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream>>>(a);
+}
+
+__global__ __launch_bounds__(256) void step_end_kernel(
+    const __bf16* __restrict__ x, long stride, float* __restrict__ y, int n, int* pos) {
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) ++*pos;
+  const __bf16* row = x + blockIdx.y * stride;
+  float* to = y + (long)blockIdx.y * n;
+  const int i = blockIdx.x * 1024 + threadIdx.x;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (i + j * 256 < n) to[i + j * 256] = (float)row[i + j * 256];
+}
+
+// rows up to 65535
+extern "C" void launch_step_end(const void* x, long stride, float* y, int rows, int n,
+                                int* pos, hipStream_t stream) {
+  step_end_kernel<<<dim3((unsigned)((n + 1023) / 1024), rows), dim3(256), 0, stream>>>(
+      (const __bf16*)x, stride, y, n, pos);
+}
+
 extern "C" void launch_mla_append_kv(const void* kvh, const void* kpe,
                                      void* kcache, void* vcache,
                                      const int* pos_ptr, int pos0, int B,

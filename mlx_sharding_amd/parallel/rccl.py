@@ -24,6 +24,7 @@ from typing import List, Optional, Tuple
 import torch
 import torch.distributed as dist
 
+from .. import ops
 from ..config import ModelConfig
 from ..models import get_model_class
 from ..models.base import StageModel
@@ -409,17 +410,16 @@ class CapturedDecode:
                 out_h = None
                 out_t = None
                 if w.is_last:
-                    if return_logits:
-                        # serving: ship last-position logits; sampling
-                        # happens outside the graph
-                        out_t = h[:, -1, :].float()
-                    else:
-                        out_t = h[:, -1, :].float().argmax(-1)
+                    # serving: ship last-position logits; sampling happens
+                    # outside the graph
+                    out_t = ops.step_end(h[:, -1, :], pos)
+                    if not return_logits:
+                        out_t = out_t.argmax(-1)
                         if w.is_first:
                             x.copy_(out_t.reshape(micro, 1))  # self-feed
                 else:
                     out_h = h.to(w.dtype)
-                pos.add_(1)
+                    pos.add_(1)
                 return out_h, out_t
 
             # warmup on a side stream (hipblaslt workspaces etc.); the two
