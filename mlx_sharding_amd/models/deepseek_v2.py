@@ -79,7 +79,8 @@ class SwitchMLP(nn.Module):
             self.down_proj.weight, subs, max_tok)
 
     def forward(self, x_flat: torch.Tensor, weights: torch.Tensor,
-                indices: torch.Tensor) -> torch.Tensor:
+                indices: torch.Tensor, plus=()) -> torch.Tensor:
+        """plus: rows that are added."""
         if self.quant is not None:
             g, u, d = self.gate_proj, self.up_proj, self.down_proj
             return ops.grouped_expert_mlp_quant(
@@ -87,10 +88,10 @@ class SwitchMLP(nn.Module):
                 (g.weight, g.scales, g.biases),
                 (u.weight, u.scales, u.biases),
                 (d.weight, d.scales, d.biases),
-                weights, indices, self.quant.group_size, self.quant.bits)
+                weights, indices, self.quant.group_size, self.quant.bits, plus)
         return ops.grouped_expert_mlp(
             x_flat, self.gate_proj.weight, self.up_proj.weight,
-            self.down_proj.weight, weights, indices)
+            self.down_proj.weight, weights, indices, plus)
 
 
 class _StackedLinear(nn.Module):
@@ -511,14 +512,16 @@ class DeepseekV2MoE(nn.Module):
             shared = None if self.shared_experts is None else self.shared_experts(y)
         return ops.expert_sum(rows, h, shared, y.shape[0]).view(shape)
 
-    def forward(self, x):
+    def forward(self, x, residual=None):
+        """The routed and the shared experts' outputs, plus ``residual``."""
         B, T, H = x.shape
         flat = x.reshape(-1, H)
-        if (ops.use_native(flat)
-                and self._fused_gate_ok(flat.shape[0])):
+        shared, switch = self.shared_experts, self.switch_mlp
+        native = ops.use_native(flat)
+        logits = self.gate(flat.to(self.gate.weight.dtype))
+        if native and self._fused_gate_ok(flat.shape[0]):
             # fused gating: one kernel for softmax+topk+sort+subranges
             # (32-token sub-ranges for the MFMA w4 kernels, 4 for bf16)
-            logits = self.gate(flat.to(self.gate.weight.dtype))
             # 16-token sub-ranges for BOTH quant sub-paths: the bf16
             # MFMA kernels over resident copies, and the fp16-dequant
             # packed kernels (moe_w4f16.hip) in memory-tight mode
@@ -526,17 +529,21 @@ class DeepseekV2MoE(nn.Module):
             subs = ops.moe_gate_subranges(logits, self.top_k,
                                           self.routed_scaling_factor,
                                           self.norm_topk_prob, max_tok=mt)
-            y = self.switch_mlp.forward_subs(flat, subs, mt)
+            y = switch.forward_subs(flat, subs, mt)
         else:
-            logits = self.gate(flat.to(self.gate.weight.dtype)).float()
             n_group = self.n_group if self.topk_method == "group_limited_greedy" else 1
             w, idx = ops.moe_gate(logits, self.top_k, n_group, self.topk_group,
                                   self.routed_scaling_factor, self.norm_topk_prob)
-            w = w.to(x.dtype)
-            y = self.switch_mlp(flat, w, idx)
-        if self.shared_experts is not None:
-            y = y + self.shared_experts(flat)
-        return y.reshape(B, T, H)
+            if native and as_built(switch):
+                plus = [] if shared is None else [shared(flat)]
+                if residual is not None:
+                    plus.append(residual.reshape(-1, H))
+                return switch(flat, w, idx, plus).reshape(B, T, H)
+            y = switch(flat, w.to(x.dtype), idx)
+        if shared is not None:
+            y = y + shared(flat)
+        y = y.reshape(B, T, H)
+        return y if residual is None else residual + y
 
 
 class DeepseekV2DecoderLayer(nn.Module):
@@ -575,7 +582,7 @@ class DeepseekV2DecoderLayer(nn.Module):
         # fused: h = x + attn; y = rms_norm(h) in one kernel
         y, h = ops.rms_norm_residual(attn, x, pn.weight, pn.eps,
                                      pn.weight_offset)
-        return h + mlp(y)
+        return mlp(y, h) if experts and as_built(mlp) else h + mlp(y)
 
 
 class DeepseekV2StageModel(StageModel):

@@ -471,7 +471,13 @@ def quantized_linear(x, w_q, scales, biases, group_size: int, bits: int):
 
 def moe_gate(router_logits, top_k: int, n_group: int = 1, topk_group: int = 1,
              routed_scaling_factor: float = 1.0, norm_topk_prob: bool = False):
-    # Router is tiny ([N, E]); fp32 torch path is fine on both devices.
+    """(fp32 weights, experts) of every token.  One kernel on the GPU for bf16 logits of
+    up to 64 experts in one group, else torch's."""
+    if (use_native(router_logits) and n_group <= 1 and _plain(router_logits)
+            and router_logits.dtype == torch.bfloat16 and router_logits.is_contiguous()
+            and router_logits.shape[0] and top_k <= router_logits.shape[1] <= 64):
+        return tuple(hip_ext().moe_choose(router_logits, top_k, routed_scaling_factor,
+                                          norm_topk_prob))
     return ref.moe_gate(router_logits, top_k, n_group, topk_group,
                         routed_scaling_factor, norm_topk_prob)
 
@@ -567,8 +573,14 @@ def _tiles_ok(x, gate_w, up_w, down_w) -> bool:
             and _plain(x))
 
 
+def _plus(y, plus):
+    for t in plus:
+        y = y + t
+    return y
+
+
 def _moe_prefill_gemm(x, gate_w, up_w, down_w, weights, indices,
-                      dequant_all=None):
+                      dequant_all=None, plus=()):
     """Large-N path: moe_tiles.hip, or (sizes and dtypes that it does not take,
     weights that are differentiated) expert-padded batched GEMMs (hipBLASLt bmm).
 
@@ -585,7 +597,12 @@ def _moe_prefill_gemm(x, gate_w, up_w, down_w, weights, indices,
         ext = _require_ext("moe_tiles")
         tile = _tile_pairs(N * K // gate_w.shape[0])
         d, where = ext.moe_tiles(x, indices.long().contiguous(), gate_w, up_w, down_w, tile)
-        return ext.moe_gather_reduce(d, where, weights.reshape(N, K).float(), N)
+        along = [t for t in plus if t.shape == (N, H) and t.dtype == torch.bfloat16
+                 and t.is_contiguous() and t.data_ptr() % 8 == 0 and _plain(t)]
+        if len(along) < len(plus) or len(along) > 2:
+            along = []
+        y = ext.moe_gather_reduce(d, where, weights.reshape(N, K).float(), N, *along)
+        return y if along else _plus(y, plus)
     flat_e = indices.reshape(-1).long()
     order = torch.argsort(flat_e, stable=True)
     sorted_e = flat_e[order]
@@ -627,11 +644,11 @@ def _moe_prefill_gemm(x, gate_w, up_w, down_w, weights, indices,
         inv[order] = torch.arange(P, device=dev)
         pair_pos = dst[inv].view(N, K).to(torch.int32)
         pair_wts = weights.reshape(N, K).float()
-        return ext.moe_gather_reduce(d, pair_pos, pair_wts, N)
+        return _plus(ext.moe_gather_reduce(d, pair_pos, pair_wts, N), plus)
     y = d[dst].float() * wts[:, None]
     out = torch.zeros(N, H, device=dev, dtype=torch.float32)
     out.index_add_(0, tok, y)
-    return out.to(x.dtype)
+    return _plus(out.to(x.dtype), plus)
 
 
 def moe_gate_subranges(router_logits_bf16, top_k: int,
@@ -819,18 +836,20 @@ def grouped_expert_mlp_quant_subs(x, gate, up, down, subs,
     return out.to(x.dtype)
 
 
-def grouped_expert_mlp(x, gate_w, up_w, down_w, weights, indices):
+def grouped_expert_mlp(x, gate_w, up_w, down_w, weights, indices, plus=()):
+    """plus: rows [N, H] that are added."""
     if _use_hip(x):
         _require_ext("grouped_expert_mlp")
         if x.shape[0] * indices.shape[1] >= _MOE_GEMM_MIN_N:
-            return _moe_prefill_gemm(x, gate_w, up_w, down_w, weights, indices)
+            return _moe_prefill_gemm(x, gate_w, up_w, down_w, weights, indices,
+                                     plus=plus)
         E = gate_w.shape[0]
         sub_e, sub_off, sub_cnt, sorted_tok, sorted_wt, _ = \
             make_expert_subranges(indices, weights, E, max_tok=4)
-        return grouped_expert_mlp_subs(
+        return _plus(grouped_expert_mlp_subs(
             x, gate_w, up_w, down_w,
-            (sub_e, sub_off, sub_cnt, sorted_tok, sorted_wt))
-    return ref.grouped_expert_mlp(x, gate_w, up_w, down_w, weights, indices)
+            (sub_e, sub_off, sub_cnt, sorted_tok, sorted_wt)), plus)
+    return _plus(ref.grouped_expert_mlp(x, gate_w, up_w, down_w, weights, indices), plus)
 
 
 def expert_dequant(gate, up, down, group_size: int, bits: int):
@@ -880,9 +899,9 @@ def expert_dequant_resident(gate, up, down, group_size: int, bits: int):
 
 
 def grouped_expert_mlp_quant(x, gate, up, down, weights, indices,
-                             group_size: int, bits: int):
+                             group_size: int, bits: int, plus=()):
     """Quantized stacked experts: gate/up/down are (w_q, scales, biases)
-    triplets with stacked [E, ...] layout."""
+    triplets with stacked [E, ...] layout; plus: rows [N, H] that are added."""
     if _use_hip(x):
         ext = _require_ext("grouped_expert_mlp_quant")
         E = gate[0].shape[0]
@@ -895,13 +914,13 @@ def grouped_expert_mlp_quant(x, gate, up, down, weights, indices,
             return _moe_prefill_gemm(
                 x, None, None, None, weights, indices,
                 dequant_all=lambda: expert_dequant(gate, up, down,
-                                                   group_size, bits))
+                                                   group_size, bits), plus=plus)
         sub_e, sub_off, sub_cnt, sorted_tok, sorted_wt, _ = \
             make_expert_subranges(indices, weights, E, max_tok=16)
-        return grouped_expert_mlp_quant_subs(
+        return _plus(grouped_expert_mlp_quant_subs(
             x, gate, up, down,
             (sub_e, sub_off, sub_cnt, sorted_tok, sorted_wt),
-            group_size, bits)
+            group_size, bits), plus)
     # CPU reference: dequantize then dense grouped MLP
     E = gate[0].shape[0]
     gw = torch.stack([ref.dequantize(gate[0][e], gate[1][e], gate[2][e],
@@ -910,7 +929,7 @@ def grouped_expert_mlp_quant(x, gate, up, down, weights, indices,
                                      group_size, bits) for e in range(E)])
     dw = torch.stack([ref.dequantize(down[0][e], down[1][e], down[2][e],
                                      group_size, bits) for e in range(E)])
-    return ref.grouped_expert_mlp(x, gw, uw, dw, weights, indices)
+    return _plus(ref.grouped_expert_mlp(x, gw, uw, dw, weights, indices), plus)
 
 
 # Sampling runs on [B, V] once per token — torch argmax/multinomial are

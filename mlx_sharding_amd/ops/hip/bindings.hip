@@ -75,8 +75,8 @@ void launch_dequant(const void*, const void*, const void*, void*, long, int,
                     int, int, hipStream_t);
 void launch_moe_scatter_rows(const void*, void*, const int*, const int*, int,
                              int, hipStream_t);
-void launch_moe_gather_reduce(const void*, const int*, const float*, void*,
-                              int, int, int, hipStream_t);
+void launch_moe_gather_reduce(const void*, const int*, const float*, const void*,
+                              const void*, void*, int, int, int, hipStream_t);
 void launch_moe_gateup_mfma(const void*, const void*, const void*, void*,
                             const int*, const int*, const int*, const int*,
                             int, int, int, hipStream_t);
@@ -755,6 +755,22 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k, torch::Tensor v,
 
 // Routed experts of a prompt: silu(x gate^T) * (x up^T), down of that, for the pairs
 // of choice [N, top] (int64).  Returns (rows [N * top, H], place of each pair).
+// Softmax of rows of logits [N, E]: (weights fp32, experts) of the `top` largest.
+std::vector<torch::Tensor> moe_choose(torch::Tensor logits, int64_t top, double scaling,
+                                      bool normalize) {
+  check_bf16(logits, "logits");
+  TORCH_CHECK(logits.dim() == 2 && logits.is_contiguous() && logits.size(0) >= 1 &&
+                  logits.size(0) < (1L << 31) - 4 && logits.size(1) <= 64 && top >= 1 &&
+                  top <= logits.size(1), "logits");
+  const long N = logits.size(0);
+  auto choice = torch::empty({N, top}, logits.options().dtype(torch::kInt64));
+  auto weight = torch::empty({N, top}, logits.options().dtype(torch::kFloat32));
+  launch_moe_choose(logits.data_ptr(), choice.data_ptr<int64_t>(),
+                    weight.data_ptr<float>(), (int)N, (int)logits.size(1), (int)top,
+                    normalize, (float)scaling, cur_stream());
+  return {weight, choice};
+}
+
 std::vector<torch::Tensor> moe_tiles(torch::Tensor x, torch::Tensor choice,
                                      torch::Tensor gate, torch::Tensor up,
                                      torch::Tensor down, int64_t tile) {
@@ -1362,17 +1378,28 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                                   cur_stream());
         });
   m.def("moe_gather_reduce",
-        [](torch::Tensor d, torch::Tensor pos, torch::Tensor wts, int64_t N) {
+        [](torch::Tensor d, torch::Tensor pos, torch::Tensor wts, int64_t N,
+           c10::optional<torch::Tensor> plus, c10::optional<torch::Tensor> plus2) {
           check_bf16(d, "d");
           const int K = pos.size(1), H = d.size(-1);
           TORCH_CHECK(pos.scalar_type() == torch::kInt32, "pos int32");
           TORCH_CHECK(wts.scalar_type() == torch::kFloat32, "wts fp32");
+          auto rows = [&](const c10::optional<torch::Tensor>& t) -> const void* {
+            if (!t.has_value()) return nullptr;
+            check_bf16(*t, "rows to add");
+            TORCH_CHECK(t->is_contiguous() && t->numel() == N * H &&
+                            reinterpret_cast<uintptr_t>(t->data_ptr()) % 8 == 0,
+                        "rows to add");
+            return t->data_ptr();
+          };
           auto out = torch::empty({N, H}, d.options());
           launch_moe_gather_reduce(d.contiguous().data_ptr(),
                                    pos.contiguous().data_ptr<int>(),
-                                   wts.contiguous().data_ptr<float>(),
-                                   out.data_ptr(), (int)N, K, H,
+                                   wts.contiguous().data_ptr<float>(), rows(plus),
+                                   rows(plus2), out.data_ptr(), (int)N, K, H,
                                    cur_stream());
           return out;
-        });
+        }, py::arg("d"), py::arg("pos"), py::arg("wts"), py::arg("N"),
+        py::arg("plus") = py::none(), py::arg("plus2") = py::none());
+  m.def("moe_choose", &moe_choose);
 }

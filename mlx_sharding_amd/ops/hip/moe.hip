@@ -383,35 +383,53 @@ __global__ void moe_scatter_rows_kernel(const short* __restrict__ src,
   for (int i = threadIdx.x; i < H / 4; i += blockDim.x) d[i] = s[i];
 }
 
-// out[t] = sum_k wts[t,k] * d[pos[t,k]]  (bf16 rows, fp32 accumulate;
-// short4 vector loads — the scalar form measured 2.3 TB/s on ~1 GB of
-// traffic per prefill MoE layer)
-__global__ void moe_gather_reduce_kernel(const short* __restrict__ d,
-                                         const int* __restrict__ pos,    // [N,K]
-                                         const float* __restrict__ wts,  // [N,K]
-                                         short* __restrict__ out,        // [N,H]
-                                         int K, int H) {
-  const int t = blockIdx.x;
-  const int* prow = pos + (long)t * K;
-  const float* wrow = wts + (long)t * K;
-  short* orow = out + (long)t * H;
+// out[t] = sum_k wts[t,k] * d[pos[t,k]], plus row t of up to two others (bf16 rows, fp32
+// sums).  Bound by memory; a row's pairs are asked for four and two at a time.  For 32768
+// tokens of 2048, 6 pairs each, with both others: 234 us, 5.2 TB/s (one after the other, and two
+// additions behind: 201 + 2 x 65 us).
+__global__ __launch_bounds__(256) void moe_gather_reduce_kernel(
+    const short* __restrict__ d, const int* __restrict__ pos,  // [N,K]
+    const float* __restrict__ wts,                             // [N,K]
+    const short* __restrict__ plus, const short* __restrict__ plus2,  // [N,H] or null
+    short* __restrict__ out,                                   // [N,H]
+    int K, int H) {
+  const long t = blockIdx.x;
+  const int* prow = pos + t * K;
+  const float* wrow = wts + t * K;
   const int n4 = H / 4;
-  for (int i = threadIdx.x; i < n4; i += blockDim.x) {
-    float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
-    for (int k = 0; k < K; ++k) {
-      const float w = wrow[k];
-      short4v v = reinterpret_cast<const short4v*>(d + (long)prow[k] * H)[i];
-      a0 += w * bfbits2f(v.x);
-      a1 += w * bfbits2f(v.y);
-      a2 += w * bfbits2f(v.z);
-      a3 += w * bfbits2f(v.w);
+  for (int i = threadIdx.x; i < n4; i += 256) {
+    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto add = [&](short4v v, float w) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a[j] += w * bfbits2f(v[j]);
+    };
+    auto pair = [&](int k) {
+      return reinterpret_cast<const short4v*>(d + (long)prow[k] * H)[i];
+    };
+    short4v p, p2;
+    if (plus) p = reinterpret_cast<const short4v*>(plus + t * H)[i];
+    if (plus2) p2 = reinterpret_cast<const short4v*>(plus2 + t * H)[i];
+    int k = 0;
+    for (; k + 4 <= K; k += 4) {
+      const short4v v0 = pair(k), v1 = pair(k + 1), v2 = pair(k + 2), v3 = pair(k + 3);
+      add(v0, wrow[k]);
+      add(v1, wrow[k + 1]);
+      add(v2, wrow[k + 2]);
+      add(v3, wrow[k + 3]);
     }
+    if (k + 2 <= K) {
+      const short4v v0 = pair(k), v1 = pair(k + 1);
+      add(v0, wrow[k]);
+      add(v1, wrow[k + 1]);
+      k += 2;
+    }
+    if (k < K) add(pair(k), wrow[k]);
+    if (plus) add(p, 1.0f);
+    if (plus2) add(p2, 1.0f);
     short4v o;
-    o.x = (short)__bfloat16_as_ushort(f2bf(a0));
-    o.y = (short)__bfloat16_as_ushort(f2bf(a1));
-    o.z = (short)__bfloat16_as_ushort(f2bf(a2));
-    o.w = (short)__bfloat16_as_ushort(f2bf(a3));
-    reinterpret_cast<short4v*>(orow)[i] = o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = (short)__bfloat16_as_ushort(f2bf(a[j]));
+    reinterpret_cast<short4v*>(out + t * H)[i] = o;
   }
 }
 
@@ -423,10 +441,12 @@ extern "C" void launch_moe_scatter_rows(const void* src, void* dst,
 }
 
 extern "C" void launch_moe_gather_reduce(const void* d, const int* pos,
-                                         const float* wts, void* out, int N,
-                                         int K, int H, hipStream_t stream) {
+                                         const float* wts, const void* plus,
+                                         const void* plus2, void* out, int N, int K,
+                                         int H, hipStream_t stream) {
   moe_gather_reduce_kernel<<<dim3((unsigned)N), dim3(256), 0, stream>>>(
-      (const short*)d, pos, wts, (short*)out, K, H);
+      (const short*)d, pos, wts, (const short*)plus, (const short*)plus2, (short*)out, K,
+      H);
 }
 
 // ---------------------------------------------------------------------------

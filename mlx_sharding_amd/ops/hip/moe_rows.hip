@@ -32,6 +32,7 @@
 // 247; bf16, experts alone, 64 tokens 234 us (4.7 TB/s).
 
 #include "moe_rows.h"
+#include "moe_choice.h"
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -536,28 +537,14 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const MoeRouteArgs a) {
   }
   __syncthreads();
   if (wid != 0) return;
-  // softmax over experts, a lane each; a lane's place is the number of experts
-  // before it, by weight and then by number (as bits, so also where a row is not
-  // a number)
   const float z = lane < a.E ? (part[0][lane] + part[1][lane]) +
                                    (part[2][lane] + part[3][lane])
                              : -INFINITY;
-  const float top = wave_max(z);
-  const float p = lane < a.E ? __expf(z - top) : 0.0f;
-  const float share = p / wave_sum(p);
-  const int key = __float_as_int(share) & 0x7FFFFFFF;
-  int place = 0;
-#pragma unroll
-  for (int i = 0; i < 64; ++i) {
-    const int k = __builtin_amdgcn_readlane(key, i);
-    place += k > key || (k == key && i < lane);
-  }
-  const bool chosen = place < a.top && lane < a.E;
-  float mine = share;
-  if (a.normalize) mine /= wave_sum(chosen ? share : 0.0f) + 1e-20f;
-  if (chosen) {
+  int place;
+  float weight;
+  if (chosen_expert(z, lane, a.E, a.top, a.normalize, a.scaling, place, weight)) {
     a.choice[t * a.top + place] = lane;
-    a.weight[t * a.top + place] = mine * a.scaling;
+    a.weight[t * a.top + place] = weight;
   }
 }
 

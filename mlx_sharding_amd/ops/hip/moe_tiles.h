@@ -28,6 +28,7 @@ struct MoeTilesArgs {
 };
 
 extern "C" {
+void launch_moe_choose(const void*, long*, float*, int, int, int, int, float, hipStream_t);
 void launch_moe_place(const MoePlaceArgs*, hipStream_t);
 // pairs of a tile: 256 or 128
 void launch_moe_tiles(MoeTilesArgs*, int tile, bool gated, hipStream_t);
