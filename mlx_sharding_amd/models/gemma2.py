@@ -61,6 +61,12 @@ class Gemma2Attention(nn.Module):
         v = v.view(B, T, self.n_kv_heads, self.head_dim)
         offset = 0
         gp = None
+        out = None
+        if cache is not None and T == 1:
+            out = cache.attend_step(q, k, v, cos, sin, self.scale, self.softcap,
+                                    self.sliding_window)
+        if out is not None:
+            return self.o_proj(out)
         if cache is not None and ops.use_native(x):
             # rotations + cache scatter in one kernel (see llama.py)
             gp = cache.graph_pos

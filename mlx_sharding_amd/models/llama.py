@@ -69,7 +69,12 @@ class LlamaAttention(nn.Module):
         v = v.view(B, T, self.n_kv_heads, self.head_dim)
         offset = 0
         gp = None
-        if cache is not None and ops.use_native(x):
+        out = None
+        if cache is not None and T == 1:
+            out = cache.attend_step(q, k, v, cos, sin, self.scale)
+        if out is not None:
+            pass
+        elif cache is not None and ops.use_native(x):
             # both rotations and the scatter into the caches in one kernel
             gp = cache.graph_pos
             if gp is None:
@@ -84,10 +89,10 @@ class LlamaAttention(nn.Module):
                 if gp is None:
                     offset = cache.offset
                 k, v = cache.update(k, v)
-        q = q.transpose(1, 2)
-        out = ops.attention(q, k, v, self.scale, causal_offset=offset,
-                            pos_dev=gp)
-        out = out.transpose(1, 2).reshape(B, T, -1)
+        if out is None:
+            out = ops.attention(q.transpose(1, 2), k, v, self.scale,
+                                causal_offset=offset, pos_dev=gp)
+            out = out.transpose(1, 2).reshape(B, T, -1)
         if residual is not None:
             return project(self.o_proj, out, residual=residual)
         return self.o_proj(out)

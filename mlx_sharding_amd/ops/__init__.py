@@ -291,6 +291,9 @@ def _plain(t: torch.Tensor) -> bool:
             and not _watched())
 
 
+plain = _plain
+
+
 def _few_ext():
     if _load_ext() is not None:
         return _EXT

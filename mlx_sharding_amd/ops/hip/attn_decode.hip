@@ -394,6 +394,13 @@ struct DecodeArgs {
   int Hq, Hkv, S, nsplit, window;
   long cap;
   SoftCap score;           // scale and cap
+  // a whole step: q and the token's key and value as the projections left them, rows of
+  // qs, ks and vs elements from one sequence to the next; rotations; a number per
+  // (sequence, key/value head) that is 0 before and after
+  const char *knew, *vnew;
+  long qs, ks, vs;
+  const float *cos, *sin;  // [DK / 2]
+  unsigned* tickets;
 };
 
 __device__ __forceinline__ void dt_to_lds(const char* src, char* dst) {
@@ -416,7 +423,49 @@ __device__ __forceinline__ float column_max(float x) {
   return fmaxf(x, __shfl_xor(x, 32, WAVE));
 }
 
-template <int DK, int DV, int KT, bool INROW>
+// Partial results pass from the blocks of a (sequence, key/value head) to the one of them
+// that comes last by accesses of the device's scope, as XCDs have L2s of their own.
+typedef unsigned long long u64;
+typedef u64 u64x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void leave(float* to, f32x4 v) {
+  const u64x2 p = __builtin_bit_cast(u64x2, v);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    __hip_atomic_store(reinterpret_cast<u64*>(to) + i, p[i], __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 found(const float* at) {
+  return __hip_atomic_load(reinterpret_cast<const u64*>(at), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// 8 dimensions from d on of a head, turned: with those half a head away
+template <int D>
+__device__ __forceinline__ bf16x8_t turned(const char* head, int d, const DecodeArgs& a) {
+  constexpr int HALF = D / 2;
+  const int c0 = d & (HALF - 1);
+  const bf16x8_t u = *reinterpret_cast<const bf16x8_t*>(head + d * 2);
+  const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(head + (d ^ HALF) * 2);
+  const float by = d < HALF ? -1.0f : 1.0f;
+  bf16x8_t y;
+#pragma unroll
+  for (int i = 0; i < 8; i += 4) {
+    const f32x4 c = *reinterpret_cast<const f32x4*>(a.cos + c0 + i);
+    const f32x4 s = *reinterpret_cast<const f32x4*>(a.sin + c0 + i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      y[i + j] = (__bf16)((float)u[i + j] * c[j] + by * (float)v[i + j] * s[j]);
+  }
+  return y;
+}
+
+// STEP: queries and the token's key are turned here, its key and value go to the cache
+// and into the last tile, and the last block of a head merges the slices.  The chain
+// through memory to that block takes what the merging kernel took (5 us), the rotations
+// 2 to 3 instead of 4.6 in a kernel of their own: one sequence of 1024 keys, 32 heads of
+// 128 over 8, 14.1 -> 9.6 us for the three; 5 of 5004, 16 of 256 over 8, 51 -> 50; 64
+// of 2049 as before (one slice, 109).
+template <int DK, int DV, int KT, bool INROW, bool STEP>
 __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
     const DecodeArgs a) {
   constexpr int KP = DK / 8, VP = INROW ? KP : DV / 8;  // pieces of a row
@@ -425,6 +474,7 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
   constexpr int HALVES = 64 / KT;
   static_assert(KT == 64 || KT == 32, "four waves make the scores of a tile");
   static_assert(NK % HALVES == 0 && KB % 4096 == 0 && VB % 4096 == 0, "sizes");
+  static_assert(!STEP || (DK == DV && !INROW && (DK & (DK - 1)) == 0), "step");
   __shared__ __attribute__((aligned(16))) char smem[2 * (KB + VB)];
   __shared__ float sc[2][HALVES][KT][16];
 
@@ -439,6 +489,7 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
   const int per = ((S - lo + a.nsplit - 1) / a.nsplit + KT - 1) / KT * KT;
   const int from = min(S, lo + per * (int)blockIdx.y);
   const int to = min(S, from + per);
+  if (STEP && from >= to && from > lo) return;  // nothing of the keys, nor of the count
 
   const char* kbase = a.k + (long)blockIdx.x * a.cap * (DK * 2);
   const char* vbase = a.v + (long)blockIdx.x * a.cap * (DV * 2);
@@ -467,12 +518,34 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
   const long row0 = (long)b * a.Hq + hk * G;  // first query head
   const int kb = KT == 64 ? wid : wid & 1, half = KT == 64 ? 0 : wid >> 1;
   bf16x8_t qf[NK / HALVES];
-  {
+  if constexpr (STEP) {
+    const char* head = a.q + ((long)b * a.qs + (hk * G + min(l16, G - 1)) * DK) * 2;
+#pragma unroll
+    for (int i = 0; i < NK / HALVES; ++i)
+      qf[i] = turned<DK>(head, (half * (NK / HALVES) + i) * 32 + lg * 8, a);
+  } else {
     const char* src = a.q + (row0 + min(l16, G - 1)) * (DK * 2) +
                       half * (NK / HALVES) * 64 + lg * 16;
 #pragma unroll
     for (int i = 0; i < NK / HALVES; ++i)
       qf[i] = *reinterpret_cast<const bf16x8_t*>(src + i * 64);
+  }
+  // the token itself, at S - 1; it has no place where the cache is full
+  const bool newest = STEP && from < to && to == S && (!a.s_ptr || *a.s_ptr < a.cap);
+  constexpr int PIECES = DK / 8;
+  const int own = threadIdx.x % PIECES;  // piece of its rows
+  bf16x8_t fresh_k, fresh_v;
+  if (newest) {
+    const long at = (long)blockIdx.x * a.cap + S - 1;
+    fresh_v = *reinterpret_cast<const bf16x8_t*>(
+        a.vnew + ((long)b * a.vs + hk * DV + own * 8) * 2);
+    if (threadIdx.x < PIECES) {
+      fresh_k = turned<DK>(a.knew + ((long)b * a.ks + hk * DK) * 2, own * 8, a);
+      *reinterpret_cast<bf16x8_t*>(const_cast<char*>(a.k) + (at * DK + own * 8) * 2) =
+          fresh_k;
+      *reinterpret_cast<bf16x8_t*>(const_cast<char*>(a.v) + (at * DV + own * 8) * 2) =
+          fresh_v;
+    }
   }
   float m = -1e30f, l = 0.0f;  // reference of the exponents (base 2), sum
   f32x4 o[ND];
@@ -486,6 +559,18 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
     if (t + KT < to) stage(t + KT, buf ^ 1);
     const char* kt = smem + buf * (KB + VB);
     const char* vt = kt + KB;
+    if (newest && t + KT >= to) {
+      // what came from the token's place in the cache is not there yet, in its row and
+      // in those behind, which repeat it
+      const int row = S - 1 - t;
+      if (threadIdx.x < PIECES)
+        *reinterpret_cast<bf16x8_t*>(const_cast<char*>(kt) + row * KP * 16 +
+                                     dt_place<KP, true>(row, own) * 16) = fresh_k;
+      for (int r = row + threadIdx.x / PIECES; r < KT; r += AD_BLOCK / PIECES)
+        *reinterpret_cast<bf16x8_t*>(const_cast<char*>(vt) + r * VP * 16 +
+                                     dt_place<VP, INROW>(r, own) * 16) = fresh_v;
+      __syncthreads();
+    }
 
     f32x4 s4 = {0, 0, 0, 0};
 #pragma unroll
@@ -573,28 +658,92 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
 
   l += __shfl_xor(l, 16, WAVE);
   l += __shfl_xor(l, 32, WAVE);
-  if (l16 >= G) return;
   const long row = row0 + l16;
   const int col = wid * ND * 16 + lg * 4;
-  if (a.nsplit == 1 && a.out) {
+  auto write = [&](long r, int c, const f32x4& v, float f) {
+    bf16 w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = f2bf(v[i] * f);
+    *reinterpret_cast<short4v*>(a.out + (r * DV + c) * 2) = *reinterpret_cast<short4v*>(w);
+  };
+  // slices that have keys
+  const int slices = STEP ? max(1, (S - lo + per - 1) / max(per, 1)) : a.nsplit;
+  if (slices == 1 && a.out) {
+    if (l16 >= G) return;
     const float f = 1.0f / l;
 #pragma unroll
-    for (int d = 0; d < ND; ++d) {
-      bf16 w[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) w[r] = f2bf(o[d][r] * f);
-      *reinterpret_cast<short4v*>(a.out + (row * DV + col + d * 16) * 2) =
-          *reinterpret_cast<short4v*>(w);
-    }
+    for (int d = 0; d < ND; ++d) write(row, col + d * 16, o[d], f);
     return;
   }
   const long part = row * a.nsplit + blockIdx.y;
+  if constexpr (!STEP) {
+    if (l16 >= G) return;
 #pragma unroll
-  for (int d = 0; d < ND; ++d)
-    *reinterpret_cast<f32x4*>(a.part_o + part * DV + col + d * 16) = o[d];
-  if (wid == 0 && lg == 0) {
-    a.part_ml[part * 2] = m;
-    a.part_ml[part * 2 + 1] = l;
+    for (int d = 0; d < ND; ++d)
+      *reinterpret_cast<f32x4*>(a.part_o + part * DV + col + d * 16) = o[d];
+    if (wid == 0 && lg == 0) {
+      a.part_ml[part * 2] = m;
+      a.part_ml[part * 2 + 1] = l;
+    }
+  } else {
+    if (l16 < G) {
+#pragma unroll
+      for (int d = 0; d < ND; ++d) leave(a.part_o + part * DV + col + d * 16, o[d]);
+      if (wid == 0 && lg == 0) {
+        typedef float f32x2 __attribute__((ext_vector_type(2)));
+        __hip_atomic_store(reinterpret_cast<u64*>(a.part_ml) + part,
+                           __builtin_bit_cast(u64, f32x2{m, l}), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    __shared__ unsigned before;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+      before = __hip_atomic_fetch_add(a.tickets + blockIdx.x, 1u, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (before + 1 != (unsigned)slices) return;
+    if (threadIdx.x == 0)
+      __hip_atomic_store(a.tickets + blockIdx.x, 0u, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    for (int i = threadIdx.x; i < G * (DV / 4); i += AD_BLOCK) {
+      const int g = i / (DV / 4), c = i % (DV / 4) * 4;
+      const long p0 = (row0 + g) * a.nsplit;
+      float top = -1e30f, all = 0.0f;
+      f32x4 sum = {0, 0, 0, 0};
+      for (int n0 = 0; n0 < slices; n0 += 16) {  // many at once, with their weights
+        u64x2 v[16];
+        f32x2 ml[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const long n = p0 + min(n0 + j, slices - 1);
+          ml[j] = __builtin_bit_cast(f32x2, found(a.part_ml + n * 2));
+          const float* at = a.part_o + n * DV + c;
+          v[j] = u64x2{found(at), found(at + 2)};
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float most = top;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) most = fmaxf(most, ml[j][0]);
+        const float keep = __builtin_amdgcn_exp2f(top - most);
+        top = most;
+        all *= keep;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[r] *= keep;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          if (n0 + j >= slices) continue;
+          const f32x4 f = __builtin_bit_cast(f32x4, v[j]);
+          const float by = __builtin_amdgcn_exp2f(ml[j][0] - top);
+          all += ml[j][1] * by;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sum[r] += f[r] * by;
+        }
+      }
+      write(row0 + g, c, sum, 1.0f / all);
+    }
   }
 }
 
@@ -645,13 +794,27 @@ extern "C" int attn_decode_tile(int G, int Dk, int Dv, bool inrow) {
 
 template <int DK, int DV, int KT, bool INROW>
 static void attn_decode_tile_go(const DecodeArgs& a, int B, hipStream_t stream) {
-  attn_decode_tile_kernel<DK, DV, KT, INROW>
-      <<<dim3((unsigned)(B * a.Hkv), (unsigned)a.nsplit), dim3(AD_BLOCK), 0,
-         stream>>>(a);
+  const dim3 grid((unsigned)(B * a.Hkv), (unsigned)a.nsplit), block(AD_BLOCK);
+  if constexpr (DK == DV && !INROW) {
+    if (a.tickets) {
+      attn_decode_tile_kernel<DK, DV, KT, INROW, true><<<grid, block, 0, stream>>>(a);
+      return;
+    }
+  }
+  attn_decode_tile_kernel<DK, DV, KT, INROW, false><<<grid, block, 0, stream>>>(a);
   if (a.nsplit > 1 && a.out)
     attn_decode_merge_kernel<<<dim3((unsigned)(B * a.Hq)), dim3(128), 0,
                                stream>>>(a.part_o, a.part_ml, (short*)a.out,
                                          a.nsplit, DV);
+}
+
+static void attn_decode_tile_size(const DecodeArgs& a, int B, int Dk, int Dv, bool inrow,
+                                  hipStream_t stream) {
+#define DT_GO(K, V, T, R)                         \
+  if (Dk == K && Dv == V && inrow == R)           \
+    attn_decode_tile_go<K, V, T, R>(a, B, stream);
+  DT_SIZES(DT_GO)
+#undef DT_GO
 }
 
 // q [B, Hq, Dk]; all bases are multiples of 16 bytes
@@ -663,9 +826,23 @@ extern "C" void launch_attn_decode_tile(
   const DecodeArgs a{(const char*)q, (const char*)k, (const char*)v, (char*)out,
                      part_o, part_ml, s_ptr, Hq, Hkv, S, nsplit, window, Scap,
                      soft_cap(scale, softcap)};
-#define DT_GO(K, V, T, R)                         \
-  if (Dk == K && Dv == V && inrow == R)           \
-    attn_decode_tile_go<K, V, T, R>(a, B, stream);
-  DT_SIZES(DT_GO)
-#undef DT_GO
+  attn_decode_tile_size(a, B, Dk, Dv, inrow, stream);
+}
+
+// A step of one token per sequence: rows of q, k and v with strides of qs, ks and vs
+// elements; heads of D elements side by side; caches [B, Hkv, Scap, D].  All rows and
+// bases are multiples of 16 bytes; tickets [B * Hkv] are 0.  S: without s_ptr the
+// length with the token.
+extern "C" void launch_attn_step(const void* q, const void* k, const void* v, long qs,
+                                 long ks, long vs, const float* cos, const float* sin,
+                                 void* kcache, void* vcache, void* out, float* part_o,
+                                 float* part_ml, unsigned* tickets, int nsplit,
+                                 const int* s_ptr, int B, int Hq, int Hkv, int S,
+                                 long Scap, int D, float scale, float softcap, int window,
+                                 hipStream_t stream) {
+  const DecodeArgs a{(const char*)q, (const char*)kcache, (const char*)vcache, (char*)out,
+                     part_o, part_ml, s_ptr, Hq, Hkv, S, nsplit, window, Scap,
+                     soft_cap(scale, softcap), (const char*)k, (const char*)v, qs, ks, vs,
+                     cos, sin, tickets};
+  attn_decode_tile_size(a, B, D, D, false, stream);
 }

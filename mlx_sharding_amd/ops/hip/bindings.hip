@@ -48,6 +48,10 @@ void launch_attn_decode_tile(const void*, const void*, const void*, void*,
                              float*, float*, int, const int*, int, int, int,
                              int, long, int, int, bool, float, float, int,
                              hipStream_t);
+void launch_attn_step(const void*, const void*, const void*, long, long, long,
+                      const float*, const float*, void*, void*, void*, float*, float*,
+                      unsigned*, int, const int*, int, int, int, int, long, int, float,
+                      float, int, hipStream_t);
 void launch_attn_prefill(const void*, const void*, const void*, void*, int,
                          int, int, int, int, long, long, long, long, long, int,
                          int, float, float, int, int, hipStream_t);
@@ -514,6 +518,68 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                      out.data_ptr(), part_o, part_ml, nsplit, s_ptr, B, Hq,
                      Hkv, S, kScap, Dk, Dv, vstride, (float)scale,
                      (float)softcap, (int)window, cur_stream());
+  return out;
+}
+
+// Attention of one token per sequence from its projections on: q [B, 1, Hq, D], k and v
+// [B, 1, Hkv, D] before rotations, whose row goes to the caches at pos (on the device) or
+// pos0; tickets [B * Hkv] of zeros, which they are again afterwards.  [B, 1, Hq * D], or
+// nothing where these are operands of the separate kernels.
+c10::optional<torch::Tensor> attn_step(
+    torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor cos,
+    torch::Tensor sin, torch::Tensor kcache, torch::Tensor vcache,
+    c10::optional<torch::Tensor> pos, int64_t pos0, torch::Tensor tickets, double scale,
+    double softcap, int64_t window) {
+  if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || kcache.dim() != 4 ||
+      q.size(1) != 1)
+    return c10::nullopt;
+  const long B = q.size(0), Hq = q.size(2), D = q.size(3), Hkv = k.size(2);
+  auto whole = [](const torch::Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  auto on = [&](const torch::Tensor& t, at::ScalarType type) {
+    return t.device() == q.device() && t.scalar_type() == type;
+  };
+  if (!q.is_cuda() || B < 1 || Hkv < 1 || Hq % Hkv || Hq < 1 ||
+      !attn_decode_tile((int)(Hq / Hkv), (int)D, (int)D, false))
+    return c10::nullopt;
+  for (const auto& t : {q, k, v})
+    if (!on(t, torch::kBFloat16) || t.size(0) != B || t.size(1) != 1 || t.size(3) != D ||
+        t.stride(3) != 1 || t.stride(2) != D || t.stride(0) % 8 || !whole(t))
+      return c10::nullopt;
+  for (const auto& t : {kcache, vcache})
+    if (!on(t, torch::kBFloat16) || !t.is_contiguous() || !whole(t) ||
+        t.sizes() != kcache.sizes() || t.size(0) != B || t.size(1) != Hkv ||
+        t.size(3) != D)
+      return c10::nullopt;
+  for (const auto& t : {cos, sin})
+    if (!on(t, torch::kFloat32) || !t.is_contiguous() || t.numel() != D / 2 || !whole(t))
+      return c10::nullopt;
+  if (v.size(2) != Hkv || !on(tickets, torch::kInt32) || !tickets.is_contiguous() ||
+      tickets.numel() < B * Hkv)
+    return c10::nullopt;
+  const long cap = kcache.size(2);
+  const int* s_ptr = nullptr;
+  if (pos.has_value()) {
+    if (!on(*pos, torch::kInt32) || pos->numel() != 1) return c10::nullopt;
+    s_ptr = pos->data_ptr<int>();
+  } else {
+    TORCH_CHECK(pos0 >= 0 && pos0 < cap, "no room in the cache");
+  }
+  const int tile = attn_decode_tile((int)(Hq / Hkv), (int)D, (int)D, false);
+  const int nsplit = decode_slices(B * Hkv, s_ptr ? cap : pos0 + 1, tile);
+  auto out = torch::empty({B, 1, Hq * D}, q.options());
+  torch::Tensor part;
+  if (nsplit > 1)
+    part = torch::empty({B * Hq * nsplit * (D + 2)}, q.options().dtype(torch::kFloat32));
+  float* po = nsplit > 1 ? part.data_ptr<float>() : nullptr;
+  launch_attn_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0),
+                   v.stride(0), cos.data_ptr<float>(), sin.data_ptr<float>(),
+                   kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(), po,
+                   po ? po + B * Hq * nsplit * D : nullptr,
+                   reinterpret_cast<unsigned*>(tickets.data_ptr<int>()), nsplit, s_ptr,
+                   (int)B, (int)Hq, (int)Hkv, (int)pos0 + 1, cap, (int)D, (float)scale,
+                   (float)softcap, (int)window, cur_stream());
   return out;
 }
 
@@ -1305,6 +1371,7 @@ std::vector<torch::Tensor> moe_gate_subranges(torch::Tensor logits, int64_t K,
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "fused RMSNorm (gfx950)");
   m.def("norm_add", &norm_add);
+  m.def("attn_step", &attn_step);
   m.def("step_begin", &step_begin);
   m.def("step_end", &step_end);
   m.def("rope_qkv", &rope_qkv, py::arg("q"), py::arg("k"), py::arg("v"),

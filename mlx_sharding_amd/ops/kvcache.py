@@ -36,6 +36,8 @@ class KVCache:
         self.offset = 0
         self._k: Optional[torch.Tensor] = None
         self._v: Optional[torch.Tensor] = None
+        # zeros that a kernel counts its blocks with, and leaves as zeros
+        self._tickets: Optional[torch.Tensor] = None
         # hipGraph-captured decode: position lives on device (int32 [1]);
         # update() appends by index_copy_ and python offset is not advanced.
         self.graph_pos: Optional[torch.Tensor] = None
@@ -51,6 +53,9 @@ class KVCache:
                          dtype=self.dtype, device=self.device)
         nv = torch.empty(batch, self.n_kv_heads, new_cap, self.v_head_dim,
                          dtype=self.dtype, device=self.device)
+        if self._tickets is None and self.device.type == "cuda":
+            self._tickets = torch.zeros(batch * self.n_kv_heads, dtype=torch.int32,
+                                        device=self.device)
         if self._k is not None and self.offset > 0:
             nk[:, :, : self.offset] = self._k[:, :, : self.offset]
             nv[:, :, : self.offset] = self._v[:, :, : self.offset]
@@ -104,6 +109,25 @@ class KVCache:
     def wrote(self, T: int):
         if self.graph_pos is None:
             self.offset += T
+
+    def attend_step(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                    cos: torch.Tensor, sin: torch.Tensor, scale: float,
+                    softcap: float = 0.0, window: int = 0) -> Optional[torch.Tensor]:
+        """append_rope_qkv of one token per sequence and its attention in one kernel:
+        [B, 1, heads * D]; None (and nothing appended) where that does not take it."""
+        from .. import ops as _ops
+        if not (self.dtype == torch.bfloat16 and k.shape[1] == 1
+                and self.k_head_dim == self.v_head_dim == k.shape[3]
+                and _ops.use_native(q) and all(_ops.plain(t) for t in (q, k, v))):
+            return None
+        pos, at = self.claim(k.shape[0], 1)
+        if self._tickets is None:
+            return None
+        out = _ops.hip_ext().attn_step(q, k, v, cos, sin, self._k, self._v, pos, at,
+                                       self._tickets, scale, softcap, window)
+        if out is not None:
+            self.wrote(1)
+        return out
 
     def append_rope_kv(self, k: torch.Tensor, v: torch.Tensor,
                        cos: torch.Tensor, sin: torch.Tensor,
