@@ -25,10 +25,14 @@
 // as they come are 64 bytes each and scales 2 (64 tokens, 64 experts of 1408 x
 // 2048 at 4 bits: 113 us so, 89 packed).
 // 4 and 8 bits become fp16 numbers 1024 + q by an OR, exactly, and one fma rounds
-// them to s q + b; values of a word are laid out in pairs for it.
+// them to s q + b; values of a word are laid out in pairs for it.  The vector units are
+// at work for half of the time at 4 bits; with every second value left where it is, as
+// part of 64 + q, and both masks in one instruction a word of eight takes 13 of them
+// instead of 19 (64 tokens, both products: 92 -> 87 us).  Loads further ahead gain nothing
+// (two tiles 103 us), and cost tokens of which a block has one tile.
 // Measured, norm, router, choice, experts and sum of 64 experts of 1408 x 2048 (6 a
 // token) beside the kernels before (norm and residual apart): 1 token at 4 bits
-// 33 us, 48 and norms; 64 tokens 104, 166 (experts alone 3.5 TB/s); 8 bits 147,
+// 33 us, 48 and norms; 64 tokens 105, 166 (experts alone 3.5 TB/s); 8 bits 147,
 // 247; bf16, experts alone, 64 tokens 234 us (4.7 TB/s).
 
 #include "moe_rows.h"
@@ -65,6 +69,13 @@ struct Operand<16> {
   }
 };
 
+// (word & mask) | high in one instruction: with two literals the compiler takes two
+__device__ __forceinline__ unsigned masked(unsigned word, unsigned mask, unsigned high) {
+  unsigned v;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(v) : "v"(word), "s"(mask), "v"(high));
+  return v;
+}
+
 // a lane's 32 values of one unit, as they come from memory
 template <int BITS>
 struct Packed {
@@ -88,14 +99,17 @@ struct Packed {
       const _Float16 sh = (_Float16)sf;
       const _Float16 bh = (_Float16)(__uint_as_float(scale & 0xFFFF0000u) + MID * sf);
       const f16x2 s2 = {sh, sh}, b2 = {bh, bh};
-      const _Float16 c = (_Float16)(-1024.0f - MID);
+      // values as the last bits of 1024 + q, or, four bits up, of 64 + q; from there
+      // exactly to q - MID
+      constexpr unsigned LOW = BITS == 4 ? 0x000F000Fu : 0x00FF00FFu;
       f16x8 out;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const unsigned word = BITS == 4 ? u[i] >> (4 * j)
+        const bool up = BITS == 4 && (j & 1);
+        const unsigned word = BITS == 4 ? u[i] >> (8 * (j / 2))
                                         : u[2 * i + j / 2] >> (8 * (j & 1));
-        const unsigned v =
-            (word & (BITS == 4 ? 0x000F000Fu : 0x00FF00FFu)) | 0x64006400u;
+        const unsigned v = masked(word, up ? LOW << 4 : LOW, up ? 0x54005400u : 0x64006400u);
+        const _Float16 c = (_Float16)((up ? -64.0f : -1024.0f) - MID);
         const f16x2 f =
             (__builtin_bit_cast(f16x2, v) + f16x2{c, c}) * s2 + b2;
         out[2 * j] = f[0];
@@ -188,7 +202,9 @@ __device__ __forceinline__ void dense_tiles(const MoeRowsArgs& a, f32x4* red) {
 // after the other.  With a block per expert and range of rows the longest one has the
 // expert with most pairs (64 experts of 1408 x 2048 at 4 bits, 64 tokens: an expert has 12
 // of them 91 us so, 90 shared; 52 179, 70; 128 tokens, 22 126, 112; one token 18.3, 20.2,
-// which is the counting).
+// which is the counting).  Choices stay in LDS for the search of an expert's pairs, which
+// goes through them one load after the other otherwise (64 tokens, both products: 97 us
+// from memory, 92 so).
 template <int BITS, int GS, int UPW, bool UP>
 __global__ __launch_bounds__(
     MR_BLOCK, UPW <= (BITS == 16 && UP ? 1 : 2) ? 4 : 2) void moe_rows_kernel(
@@ -198,6 +214,7 @@ __global__ __launch_bounds__(
   constexpr int MATS = UP ? 2 : 1;
   __shared__ int count[64], ends[64];
   __shared__ short list[16];
+  __shared__ unsigned char chosen[MR_PAIRS];  // experts, 255: none
   __shared__ __attribute__((aligned(16))) f32x4 red[2][MR_WAVES][MATS][WAVE];
 
   if ((int)blockIdx.x < a.dense) {
@@ -212,6 +229,7 @@ __global__ __launch_bounds__(
   __syncthreads();
   for (int i = threadIdx.x; i < a.pairs; i += MR_BLOCK) {
     const unsigned e = a.choice[i];
+    chosen[i] = (unsigned char)min(e, 255u);
     if (e < (unsigned)a.experts) atomicAdd(&count[e], 1);
   }
   __syncthreads();
@@ -266,7 +284,7 @@ __global__ __launch_bounds__(
     if (wid == 0) {
       int found = -first;
       for (int i = 0; i < a.pairs && found < 16; i += WAVE) {
-        const bool mine = i + lane < a.pairs && a.choice[i + lane] == e;
+        const bool mine = i + lane < a.pairs && chosen[i + lane] == e;
         const unsigned long long which = __ballot(mine);
         const int place = found + __popcll(which & ((1ull << lane) - 1));
         if (mine && place >= 0 && place < 16) list[place] = (short)(i + lane);
