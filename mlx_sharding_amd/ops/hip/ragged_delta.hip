@@ -439,7 +439,13 @@ extern "C" void launch_delta_short(const void* y, const void* z,
 // beta -> fp32 [n, H].  One wave per (16 tokens of a chunk, piece): a piece is
 // a q or k head, 64 * CW value channels, or the gates.  A lane keeps its CW
 // neighbouring channels' inputs of all 16 tokens and their history in
-// registers.  NU: channel groups per lane and q/k head, D <= 64 * CW * NU.
+// registers.  NU: channel groups per lane and q/k head, D <= 64 * CW * NU.  TAPS: the
+// number of taps, or DR_MAXTAPS for any (taps that are not there are left out one by
+// one, as what they would meet need not be finite).
+// Bound by memory and by its instructions in like parts.  Blocks that follow one another
+// have neighbouring pieces of one row; one norm's root and quotient serve 16 tokens.
+// 8002 tokens of 16 q and k heads and 32 value heads of 128: 143 -> 93 us (3.5 TB/s); with
+// the taps chosen in the loop a third of the instructions were that.
 // ---------------------------------------------------------------------------
 
 // CW neighbouring elements at once (1 or 2)
@@ -467,7 +473,7 @@ __device__ __forceinline__ void store_lanes(T* p, const float (&o)[CW]) {
 #define DC_TT 16
 #define DC_SUB (DR_CHUNK / DC_TT)
 
-template <typename T, int NU, int CW>
+template <typename T, int NU, int CW, int TAPS>
 __global__ __launch_bounds__(DC_BLOCK) void delta_conv_kernel(
     const T* __restrict__ y, const T* __restrict__ conv_w,
     const T* __restrict__ A_log, const T* __restrict__ dt_bias,
@@ -476,13 +482,14 @@ __global__ __launch_bounds__(DC_BLOCK) void delta_conv_kernel(
     float* __restrict__ bt, const int* __restrict__ cu,
     const int* __restrict__ pos0, const int* __restrict__ slots,
     const int* __restrict__ tok_entry, const int* __restrict__ chunks,
-    int tok_base, DeltaDims dm, int Dp, int Vp, float q_scale) {
-  const int chunk = blockIdx.x / DC_SUB, sub = blockIdx.x % DC_SUB;
+    int tok_base, DeltaDims dm, int Dp, int Vp, float q_scale, int groups) {
+  const int part = blockIdx.x / groups, group = blockIdx.x - part * groups;
+  const int chunk = part / DC_SUB, sub = part % DC_SUB;
   const int t0 = chunks[2 * chunk] + sub * DC_TT;
   const int len = min(DC_TT, chunks[2 * chunk + 1] - sub * DC_TT);
   const int lane = threadIdx.x & (WAVE - 1);
   const int piece = __builtin_amdgcn_readfirstlane(
-      blockIdx.y * (DC_BLOCK / WAVE) + threadIdx.x / WAVE);
+      group * (DC_BLOCK / WAVE) + threadIdx.x / WAVE);
   const int D = dm.D, V = dm.V;
   const int n_qk = 2 * dm.KH;
   const int n_v = (dm.H * Vp + WAVE * CW - 1) / (WAVE * CW);
@@ -491,17 +498,17 @@ __global__ __launch_bounds__(DC_BLOCK) void delta_conv_kernel(
   const int e = tok_entry[t0];
   const int rel = t0 - cu[e];             // place within the portion
   const bool fresh = pos0[e] == 0;
-  const int hist = dm.taps - 1;
+  const int taps = TAPS < DR_MAXTAPS ? TAPS : dm.taps, hist = taps - 1;
   const int C = 2 * dm.KH * D + dm.H * V;
   const T* cs = conv_state + (long)slots[e] * C * hist;
   const T* yt = y + (long)t0 * dm.ystride;
 
   // channels c.. (columns col.. of y): convolved, silu'd values of 16 tokens
   auto convolve = [&](int c, int col, float (&o)[DC_TT][CW]) {
-    float x[DC_TT + DR_MAXTAPS - 1][CW], w[DR_MAXTAPS][CW];
+    float x[DC_TT + TAPS - 1][CW], w[TAPS][CW];
 #pragma unroll
-    for (int k = 0; k < DC_TT + DR_MAXTAPS - 1; ++k) {
-      const int t = k - (DR_MAXTAPS - 1);
+    for (int k = 0; k < DC_TT + TAPS - 1; ++k) {
+      const int t = k - (TAPS - 1);
 #pragma unroll
       for (int q = 0; q < CW; ++q) x[k][q] = 0.0f;
       if (t >= 0) {
@@ -516,12 +523,12 @@ __global__ __launch_bounds__(DC_BLOCK) void delta_conv_kernel(
             x[k][q] = (float)cs[(long)(c + q) * hist + hist + rel + t];
       }
     }
-    const int pad = DR_MAXTAPS - dm.taps;
+    const int pad = TAPS - taps;
 #pragma unroll
-    for (int j = 0; j < DR_MAXTAPS; ++j)
+    for (int j = 0; j < TAPS; ++j)
 #pragma unroll
       for (int q = 0; q < CW; ++q)
-        w[j][q] = j >= pad ? (float)conv_w[(long)(c + q) * dm.taps + j - pad]
+        w[j][q] = j >= pad ? (float)conv_w[(long)(c + q) * taps + j - pad]
                            : 0.0f;
 #pragma unroll
     for (int t = 0; t < DC_TT; ++t)
@@ -529,7 +536,7 @@ __global__ __launch_bounds__(DC_BLOCK) void delta_conv_kernel(
       for (int q = 0; q < CW; ++q) {
         float a = 0.0f;
 #pragma unroll
-        for (int j = 0; j < DR_MAXTAPS; ++j)
+        for (int j = 0; j < TAPS; ++j)
           if (j >= pad) a += w[j][q] * x[t + j][q];
         o[t][q] = silu_f(a);
       }
@@ -552,6 +559,7 @@ __global__ __launch_bounds__(DC_BLOCK) void delta_conv_kernel(
       }
     }
     float* dst = (which ? ko : qo) + (i0 * dm.KH + kh) * Dp;
+    float sq = 0.0f;  // lane t: of token t
 #pragma unroll
     for (int t = 0; t < DC_TT; ++t) {
       float ss = 0.0f;
@@ -560,7 +568,12 @@ __global__ __launch_bounds__(DC_BLOCK) void delta_conv_kernel(
 #pragma unroll
         for (int q = 0; q < CW; ++q) ss += o[u][t][q] * o[u][t][q];
       ss = wave_sum(ss);
-      const float s = (which ? 1.0f : q_scale) / sqrtf(ss + 1e-6f);
+      if (lane == t) sq = ss;
+    }
+    const float by = (which ? 1.0f : q_scale) / sqrtf(sq + 1e-6f);
+#pragma unroll
+    for (int t = 0; t < DC_TT; ++t) {
+      const float s = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(by), t));
       if (t < len) {
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
@@ -634,6 +647,8 @@ __global__ __launch_bounds__(DC_BLOCK) void delta_conv_state_kernel(
 //   tm [chunks, H, 64, 64]  (I + L)^-1 diag(beta) (lower tiles only)
 //   am [chunks, H, 64, 64]  A (lower tiles only)
 //   ge [chunks, H, 2, 64]   exp(G), exp(G_last - G)
+// Bound by latency, and by what is written.  Operands are on their way a step ahead, and
+// the value heads of a q/k head run on one XCD: 126 chunks of 32 heads 138 -> 110 us.
 // ---------------------------------------------------------------------------
 
 #define DR_LS 68
@@ -701,14 +716,18 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(
     const float* __restrict__ qn, const float* __restrict__ kn,
     const float* __restrict__ lg, const float* __restrict__ bt,
     float* __restrict__ tm, float* __restrict__ am, float* __restrict__ ge,
-    const int* __restrict__ chunks, int tok_base, int KH, int H, int Dp) {
-  const int c = blockIdx.x, h = blockIdx.y;
-  const int kh = h / (H / KH);
+    const int* __restrict__ chunks, int n_chunks, int tok_base, int KH, int H, int Dp) {
+  // blocks go round the XCDs: eight pairs of a chunk and a q/k head, then their next
+  // value head, which reads the same rows from the L2 they came to
+  const int r = H / KH, round = blockIdx.x / (8 * r), at = blockIdx.x - round * 8 * r;
+  const int pair = round * 8 + at % 8;
+  if (pair >= n_chunks * KH) return;
+  const int c = pair / KH, kh = pair - c * KH, h = kh * r + at / 8;
   const int i0 = chunks[2 * c] - tok_base;
   const int len = chunks[2 * c + 1];
   const int tid = threadIdx.x;
   const int lane = tid & (WAVE - 1);
-  const int wid = tid / WAVE;
+  const int wid = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int lr = lane & 15, g4 = lane >> 4;
 
   __shared__ double gs[DR_CHUNK];
@@ -744,20 +763,35 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(
   const float* kbase = kn + ((long)i0 * KH + kh) * Dp + g4 * 4;
   const float* qbase = qn + ((long)i0 * KH + kh) * Dp + g4 * 4;
   const long rstride = (long)KH * Dp;
-  for (int d = 0; d < Dp; d += 16) {
-    const f32x4 ka = load4(kbase + ra * rstride + d);
-    const f32x4 qa = load4(qbase + ra * rstride + d);
+  // one step's operands are on their way while another's are in the matrix cores
+  struct Step {
+    f32x4 q, k[4];
+  };
+  auto fetch = [&](Step& f, int d) {
+    f.q = load4(qbase + ra * rstride + d);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j <= wid) f.k[j] = load4(kbase + min(j * 16 + lr, len - 1) * rstride + d);
+  };
+  auto use = [&](const Step& f) {
+    const f32x4 ka = wid == 0 ? f.k[0] : wid == 1 ? f.k[1] : wid == 2 ? f.k[2] : f.k[3];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if (j > wid) continue;
-      const int rb = min(j * 16 + lr, len - 1);
-      const f32x4 kb = load4(kbase + rb * rstride + d);
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        kk[j] = mma4(ka[s], kb[s], kk[j]);
-        qk[j] = mma4(qa[s], kb[s], qk[j]);
+        kk[j] = mma4(ka[s], f.k[j][s], kk[j]);
+        qk[j] = mma4(f.q[s], f.k[j][s], qk[j]);
       }
     }
+  };
+  Step one, two;
+  fetch(one, 0);
+  for (int d = 0; d < Dp; d += 32) {
+    if (d + 16 < Dp) fetch(two, d + 16);
+    use(one);
+    if (d + 32 < Dp) fetch(one, d + 32);
+    if (d + 16 < Dp) use(two);
   }
   __syncthreads();
 #pragma unroll
@@ -1649,23 +1683,24 @@ static void delta_long_t(const DeltaLongArgs& a, const DeltaDims& dm,
   const int cw = pair ? 2 : 1;
   const int pieces =
       2 * dm.KH + (dm.H * a.Vp + WAVE * cw - 1) / (WAVE * cw) + 1;
-  dim3 g1((unsigned)(a.n_chunks * DC_SUB),
-          (unsigned)((pieces + DC_BLOCK / WAVE - 1) / (DC_BLOCK / WAVE)));
-#define DC_GO(N, W)                                                          \
-  delta_conv_kernel<T, N, W><<<g1, block, 0, stream>>>(                      \
+  const int groups = (pieces + DC_BLOCK / WAVE - 1) / (DC_BLOCK / WAVE);
+  const dim3 g1((unsigned)((long)a.n_chunks * DC_SUB * groups));
+#define DC_GO(N, W, TAPS)                                                    \
+  delta_conv_kernel<T, N, W, TAPS><<<g1, block, 0, stream>>>(                \
       (const T*)a.y, (const T*)a.conv_w, (const T*)a.A_log,                  \
       (const T*)a.dt_bias, (const T*)a.conv_state, a.qn, a.kn, (T*)a.vn,     \
       a.lg, a.bt, a.cu, a.pos0, a.slots, a.tok_entry, a.chunks, a.tok_base,  \
-      dm, a.Dp, a.Vp, q_scale)
+      dm, a.Dp, a.Vp, q_scale, groups)
   if (pair) {
-    if (a.Dp <= 128) DC_GO(1, 2);
-    else if (a.Dp <= 256) DC_GO(2, 2);
-    else DC_GO(4, 2);
+    if (a.Dp <= 128 && dm.taps == 4) DC_GO(1, 2, 4);
+    else if (a.Dp <= 128) DC_GO(1, 2, DR_MAXTAPS);
+    else if (a.Dp <= 256) DC_GO(2, 2, DR_MAXTAPS);
+    else DC_GO(4, 2, DR_MAXTAPS);
   } else {
-    if (a.Dp <= 64) DC_GO(1, 1);
-    else if (a.Dp <= 128) DC_GO(2, 1);
-    else if (a.Dp <= 256) DC_GO(4, 1);
-    else DC_GO(8, 1);
+    if (a.Dp <= 64) DC_GO(1, 1, DR_MAXTAPS);
+    else if (a.Dp <= 128) DC_GO(2, 1, DR_MAXTAPS);
+    else if (a.Dp <= 256) DC_GO(4, 1, DR_MAXTAPS);
+    else DC_GO(8, 1, DR_MAXTAPS);
   }
 #undef DC_GO
   dim3 g2((unsigned)a.n_long, (unsigned)((C + DC_BLOCK - 1) / DC_BLOCK));
@@ -1686,9 +1721,10 @@ static void delta_long_t(const DeltaLongArgs& a, const DeltaDims& dm,
 #undef DCH_GO
     delta_walk_t<T, true>(a, dm, a.qg, a.kg, a.kl, dm.H, g4, stream);
   } else {
-    delta_chunk_kernel<<<g3, block, 0, stream>>>(
-        a.qn, a.kn, a.lg, a.bt, a.tm, a.am, a.ge, a.chunks, a.tok_base, dm.KH,
-        dm.H, a.Dp);
+    const dim3 g((unsigned)(((long)a.n_chunks * dm.KH + 7) / 8 * 8 * (dm.H / dm.KH)));
+    delta_chunk_kernel<<<g, block, 0, stream>>>(
+        a.qn, a.kn, a.lg, a.bt, a.tm, a.am, a.ge, a.chunks, a.n_chunks, a.tok_base,
+        dm.KH, dm.H, a.Dp);
     delta_walk_t<T, false>(a, dm, a.qn, a.kn, a.kn, dm.KH, g4, stream);
   }
   dim3 g5((unsigned)((a.n_tok * dm.H + 4 * DG_ROWS - 1) / (4 * DG_ROWS)));
