@@ -57,6 +57,19 @@ class ExpertShape:
         few = tokens * self.top <= 48 * self.total
         return TILE_SHORT if few else TILE_LONG
 
+    def tiles(self, tokens: int) -> int:
+        """Pairs of a tile of the persistent kernel (moe_tiles.hip), 0: the others'.
+        Few pairs an expert are one tile of 16 for most, which reads weights as fast;
+        with few experts of few units there is not a tile for every second CU.  Measured
+        (us for both products, router and placement; as before, with 128, with 256):
+        64 experts of 2048 x 1024, a mean of 12 pairs: 182, 201, 219; of 24: 280, 206, 225;
+        of 48: 467, 216, 233; of 94: 305, 225, 240; of 140: 322, 309, 250; of 563: 681,
+        704, 587; 16 of 2048 x 1024, of 32: 102, 80, 91; 16 of 1024 x 512, of 64: 39, 42."""
+        mean = tokens * self.top / self.total
+        if mean <= 16 or self.experts * self.ff < 128 * 128:
+            return 0
+        return 128 if mean < 128 else 256
+
 
 def pack(w, width: int):
     """Weights [rows, columns], the columns padded to ``width``, as matrix-core
@@ -101,6 +114,14 @@ def route(h, router, correction, sh: ExpertShape, routing: Routing = Routing()):
     return idx, w
 
 
+def _tiled(h, up, down) -> bool:
+    """Whether moe_tiles.hip takes these operands."""
+    K, (_, O, F) = up.shape[2], down.shape
+    return (h.dtype == torch.bfloat16 and O % 64 == 0 and min(K, F, O) >= 128
+            and up.shape[1] == 2 * F and max(K, O) * F < 2 ** 31
+            and h.shape[0] * h.stride(0) < 2 ** 31)
+
+
 def expert_rows(h, router, correction, up, down, sh: ExpertShape,
                 routing: Routing = Routing(), glu: Optional[ClampedGLU] = None):
     """What the chosen experts make of rows h [N, width padded]: (rows, where
@@ -114,13 +135,18 @@ def expert_rows(h, router, correction, up, down, sh: ExpertShape,
     N = h.shape[0]
     if h.is_cuda:
         ext = _ext("experts")
-        tile = sh.tile(N)
+        tiled = sh.tiles(N) if (routing.on_input and glu is not None
+                                and _tiled(h, up, down)) else 0
+        tile = tiled or sh.tile(N)
         idx, weight, rank, hist = ext.expert_route(
             h, router, correction, sh.total, sh.experts, sh.top,
             routing.score == "sigmoid", routing.normalize)
         scale = weight if routing.on_input else None
-        where, tokens, tiles, scale = ext.expert_plan(idx, rank, hist, scale,
-                                                      sh.experts, tile)
+        where, tokens, tiles, used, scale = ext.expert_plan(idx, rank, hist, scale,
+                                                            sh.experts, tile)
+        if tiled:
+            return ext.expert_tiles(h, tokens, tiles, used, up, down, scale, tile,
+                                    glu.limit, glu.alpha), where, None
         form = (0.0, 0.0) if glu is None else (glu.limit, glu.alpha)
         u = ext.expert_gemm(h, tokens, tiles, up, scale, tile, N * sh.top,
                             1 if glu is None else 2, *form)

@@ -874,12 +874,12 @@ std::vector<torch::Tensor> moe_tiles(torch::Tensor x, torch::Tensor choice,
   auto y = torch::empty({P, H}, x.options());
   MoeTilesArgs a{(const char*)x.data_ptr(), (const char*)gate.data_ptr(),
                  (const char*)up.data_ptr(), (__bf16*)h.data_ptr(), tokens, tiles,
-                 n_tiles, x.stride(0) * 2, (int)I, (int)H, 0};
-  launch_moe_tiles(&a, (int)tile, true, cur_stream());
+                 n_tiles, x.stride(0) * 2, (int)I, (int)H, 0, I * H * 2};
+  launch_moe_tiles(&a, (int)tile, MT_SILU, cur_stream());
   MoeTilesArgs b{(const char*)h.data_ptr(), (const char*)down.data_ptr(), nullptr,
                  (__bf16*)y.data_ptr(), nullptr, tiles, n_tiles, I * 2, (int)H,
-                 (int)I, 0};
-  launch_moe_tiles(&b, (int)tile, false, cur_stream());
+                 (int)I, 0, I * H * 2};
+  launch_moe_tiles(&b, (int)tile, MT_SUMS, cur_stream());
   return {y, where};
 }
 

@@ -15,21 +15,28 @@ struct MoePlaceArgs {
   int pairs, top, experts, blocks, tile;
 };
 
-// y[p, o] = x[token of p] . w[expert of p, o], of a gated unit silu(that) times the
-// same with w2.  K and O are multiples of 64, K at least 128; rows of w begin at 16
-// bytes; offsets within x (tokens given) and within an expert's matrix below 2^32.
+// What is made of the sums: themselves, silu(those with w) * those with w2, or
+// g sigmoid(alpha g) (u + 1) of both times scale[p], g at most `limit`, u within +-limit.
+enum MoeUnit { MT_SUMS = 0, MT_SILU = 1, MT_CLAMPED = 2 };
+
+// y[p, o] of x[token of p] . w[expert of p, o] (and w2).  K and O are multiples of 64, K
+// at least 128; rows of w begin at 16 bytes; offsets within x (tokens given) and within
+// an expert's matrix below 2^32.
 struct MoeTilesArgs {
   const char *x, *w, *w2;  // [rows, K], [experts, O, K]; w2: up's
   __bf16* y;               // [pairs, O]
-  const int* tokens;       // gated: row of x of a pair; else the pair is
+  const int* tokens;       // of a unit: row of x of a pair; else the pair is
   const int *tiles, *n_tiles;
   long xstride;            // bytes
   int O, K, cols;          // cols: blocks across O
+  long wstride;            // bytes from one expert's matrix to the next
+  const float* scale;      // clamped: [pairs]
+  float limit, alpha;
 };
 
 extern "C" {
 void launch_moe_choose(const void*, long*, float*, int, int, int, int, float, hipStream_t);
 void launch_moe_place(const MoePlaceArgs*, hipStream_t);
 // pairs of a tile: 256 or 128
-void launch_moe_tiles(MoeTilesArgs*, int tile, bool gated, hipStream_t);
+void launch_moe_tiles(MoeTilesArgs*, int tile, MoeUnit, hipStream_t);
 }

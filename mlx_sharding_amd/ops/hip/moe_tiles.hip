@@ -17,6 +17,9 @@
 // us, 200 tokens 458 -> 246 (the weights alone take 225).  Before: pairs scattered to
 // experts padded to the fullest one (its count read back by the host), two batched
 // library products on transposed copies of the weights, the unit in between.
+// Clamped units (part of the ragged extension, which has places of its own) read their
+// pairs' weights out of LDS at the end of an item, where a load from memory would wait for
+// the stages under way.
 
 #include "moe_tiles.h"
 #include "moe_choice.h"
@@ -140,8 +143,9 @@ extern "C" void launch_moe_place(const MoePlaceArgs* a, hipStream_t stream) {
 
 #define MT_GROUP 4  // tiles whose blocks run together, with the same weights
 // MT: pairs of a tile
-template <int MT, bool GLU>
+template <int MT, MoeUnit UNIT>
 __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a) {
+  constexpr bool GLU = UNIT != MT_SUMS;
   constexpr int NP = MT / 64;          // 32-pair tiles of a wave
   constexpr int L = 4 + NP;            // loads per wave and stage
   constexpr int ST = (256 + MT) * 64;  // bytes of a stage
@@ -195,7 +199,7 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a)
     }
   };
   auto rows_of = [&](const Item& it, const int (&t)[NP], Rows& s) {
-    s.w = (GLU && wid >> 1 ? a.w2 : a.w) + (long)it.e * a.O * a.K * 2;
+    s.w = (GLU && wid >> 1 ? a.w2 : a.w) + it.e * a.wstride;
     s.x = a.x + (GLU ? 0 : it.p0 * a.xstride);
 #pragma unroll
     for (int i = 0; i < L; ++i) {
@@ -272,6 +276,7 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a)
   for (int i = 0; i < NP; ++i) f0.x[i] = rd(smem + xo[0] + i * 2048);
 
   int g = 0;  // stages so far
+  int flip = 0;
   for (bool more = true; more;) {
     more = at.tile >= 0;
     const Item nx = more ? item(ahead, at.n0) : it;
@@ -284,6 +289,17 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a)
       for (int j = 0; j < NP; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    // weights of this item's pairs go to LDS, and are there some steps later; those of
+    // the item before may still be read
+    if constexpr (UNIT == MT_CLAMPED) {
+      flip ^= 1;
+      if (wid * 64 < MT)
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)(
+                a.scale + it.p0 + min(wid * 64 + lane, it.np - 1)),
+            (__attribute__((address_space(3))) void*)(
+                smem + 4 * ST + (flip * MT + wid * 64) * 4), 4, 0, 0);
+    }
     auto step = [&](auto&& fetch) {
       half(f0, f1, g, 1, [&](int i) {
         if (L / 2 + i < L) fetch(2, L / 2 + i);
@@ -336,6 +352,14 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a)
       const int p = wm * (MT / 2) + j * 32 + l32;
       // all lanes take part in the exchange
       __bf16* row = a.y + (long)(it.p0 + min(p, it.np - 1)) * a.O;
+      // read here: the compiler would wait for all loads to LDS
+      float by = 1.0f;
+      if constexpr (UNIT == MT_CLAMPED) {
+        const auto* at = (__attribute__((address_space(3))) char*)(
+            smem + 4 * ST + (flip * MT + p) * 4);
+        asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(by) : "v"(at) : "memory");
+      }
 #pragma unroll
       for (int i = 0; i < (GLU ? 2 : 4); ++i)
 #pragma unroll
@@ -347,8 +371,14 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a)
             for (int r = 0; r < 4; ++r) {
               const int c = (2 * q + h) * 4 + r;
               if (GLU) {
-                const float z = sum(2 * i, j, c), u = sum(2 * i + 1, j, c);
-                v[h][r] = z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)) * u;
+                float z = sum(2 * i, j, c), u = sum(2 * i + 1, j, c);
+                if constexpr (UNIT == MT_CLAMPED) {
+                  z = fminf(z * by, a.limit);
+                  u = fminf(fmaxf(u * by, -a.limit), a.limit) + 1.0f;
+                  v[h][r] = z * __builtin_amdgcn_rcpf(1.0f + __expf(-a.alpha * z)) * u;
+                } else {
+                  v[h][r] = z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)) * u;
+                }
               } else v[h][r] = sum(i, j, c);
             }
           const int o = it.n0 + wn * (NC / 2) + i * 32 + q * 16;
@@ -363,28 +393,25 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <int MT, bool GLU>
+template <int MT, MoeUnit UNIT>
 static void moe_tiles_go(MoeTilesArgs& a, hipStream_t stream) {
-  const int smem = 4 * (256 + MT) * 64;
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_tiles_kernel<MT, GLU>),
+  const int smem = 4 * (256 + MT) * 64 + (UNIT == MT_CLAMPED ? 2 * MT * 4 : 0);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_tiles_kernel<MT, UNIT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-  a.cols = (a.O + (GLU ? 127 : 255)) / (GLU ? 128 : 256);
-  moe_tiles_kernel<MT, GLU><<<dim3(256), dim3(256), smem, stream>>>(a);
+  const int across = UNIT != MT_SUMS ? 128 : 256;
+  a.cols = (a.O + across - 1) / across;
+  moe_tiles_kernel<MT, UNIT><<<dim3(256), dim3(256), smem, stream>>>(a);
 }
 
-extern "C" void launch_moe_tiles(MoeTilesArgs* a, int tile, bool gated,
+template <int MT>
+static void moe_tiles_unit(MoeTilesArgs& a, MoeUnit unit, hipStream_t stream) {
+  if (unit == MT_SILU) moe_tiles_go<MT, MT_SILU>(a, stream);
+  else if (unit == MT_CLAMPED) moe_tiles_go<MT, MT_CLAMPED>(a, stream);
+  else moe_tiles_go<MT, MT_SUMS>(a, stream);
+}
+
+extern "C" void launch_moe_tiles(MoeTilesArgs* a, int tile, MoeUnit unit,
                                  hipStream_t stream) {
-  if (tile == 256) {
-    if (gated) {
-      moe_tiles_go<256, true>(*a, stream);
-    } else {
-      moe_tiles_go<256, false>(*a, stream);
-    }
-  } else {
-    if (gated) {
-      moe_tiles_go<128, true>(*a, stream);
-    } else {
-      moe_tiles_go<128, false>(*a, stream);
-    }
-  }
+  if (tile == 256) moe_tiles_unit<256>(*a, unit, stream);
+  else moe_tiles_unit<128>(*a, unit, stream);
 }

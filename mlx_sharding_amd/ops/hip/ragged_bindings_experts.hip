@@ -1,5 +1,6 @@
 // Python bindings of the routed experts.
 #include "ragged_bindings.h"
+#include "moe_tiles.h"
 #include "ragged_experts.h"
 
 extern "C" {
@@ -59,9 +60,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> expert_route(
   return {idx, weight, rank, hist};
 }
 
-// -> rows of the pairs [N, top], tokens of the rows [N * top], tiles [*, 3], and
-// the rows' weights [N * top] if weight is given
-std::tuple<Tensor, Tensor, Tensor, c10::optional<Tensor>> expert_plan(
+// -> rows of the pairs [N, top], tokens of the rows [N * top], tiles [*, 3], how many
+// of them there are, and the rows' weights [N * top] if weight is given
+std::tuple<Tensor, Tensor, Tensor, Tensor, c10::optional<Tensor>> expert_plan(
     Tensor idx, Tensor rank, Tensor hist, c10::optional<Tensor> weight,
     int64_t experts, int64_t tile) {
   PlanArgs a = {};
@@ -80,13 +81,14 @@ std::tuple<Tensor, Tensor, Tensor, c10::optional<Tensor>> expert_plan(
   a.n_tiles = (int)(pairs / tile + std::min<long>(experts, pairs));
   TORCH_CHECK(a.n_tiles <= 65535 * 16L);
   auto where = int_rows(idx, {a.n, a.top}), tokens = int_rows(idx, {pairs});
-  auto tiles = int_rows(idx, {a.n_tiles, 3});
+  auto tiles = int_rows(idx, {a.n_tiles, 3}), used = int_rows(idx, {1});
   a.idx = ints(idx, pairs, "idx");
   a.rank = ints(rank, pairs, "rank");
   a.hist = ints(hist, 0, "hist");
   a.where = where.data_ptr<int>();
   a.tokens = tokens.data_ptr<int>();
   a.tiles = tiles.data_ptr<int>();
+  a.used = used.data_ptr<int>();
   c10::optional<Tensor> scale;
   if (weight) {
     check_f32(*weight, "weight");
@@ -96,7 +98,7 @@ std::tuple<Tensor, Tensor, Tensor, c10::optional<Tensor>> expert_plan(
     a.scale = scale->data_ptr<float>();
   }
   if (a.n) launch_expert_plan(&a, stream());
-  return {where, tokens, tiles, scale};
+  return {where, tokens, tiles, used, scale};
 }
 
 // x rows (of `tokens`, or the pairs' own) times w [experts, O, K] and the rows'
@@ -143,6 +145,42 @@ Tensor expert_gemm(Tensor x, c10::optional<Tensor> tokens, Tensor tiles,
   a.tiles = ints(tiles, 0, "tiles");
   if (a.n_tiles) launch_expert_gemm(&a, (int)tile, f32, stream());
   return out;
+}
+
+// Both products of clamped units, by moe_tiles.hip: rows of x, which tokens of the pairs
+// are, times up [experts, 2 F, K] and the pairs' scale, and those times down [experts, O,
+// F] -> [pairs, O].  tiles of 128 or 256 pairs, of which `used` are there.
+Tensor expert_tiles(Tensor x, Tensor tokens, Tensor tiles, Tensor used, Tensor up,
+                    Tensor down, Tensor scale, int64_t tile, double limit,
+                    double alpha) {
+  for (const Tensor* t : {&x, &up, &down}) {
+    TORCH_CHECK(t->is_cuda() && t->scalar_type() == torch::kBFloat16, "bf16 operands");
+    aligned16(*t, "operand");
+  }
+  TORCH_CHECK(up.dim() == 3 && down.dim() == 3 && up.is_contiguous() &&
+              down.is_contiguous(), "stacked matrices");
+  const long stride = rows2(x, "x"), K = up.size(2), F = down.size(2), O = down.size(1);
+  TORCH_CHECK(x.size(1) == K && up.size(1) == 2 * F && up.size(0) == down.size(0));
+  TORCH_CHECK(K % 64 == 0 && F % 64 == 0 && O % 64 == 0 && K >= 128 && F >= 128 &&
+              stride % 8 == 0 && x.size(0) * stride < (1L << 31) &&
+              F * K < (1L << 31) && F * O < (1L << 31), "sizes that there is no kernel for");
+  TORCH_CHECK(tile == 128 || tile == 256, "tiles hold 128 or 256 pairs");
+  const long pairs = tokens.numel();
+  check_f32(scale, "scale");
+  TORCH_CHECK(scale.numel() == pairs && tiles.dim() == 2 && tiles.size(1) == 3);
+  auto h = torch::empty({pairs, F}, x.options()), y = torch::empty({pairs, O}, x.options());
+  if (!pairs) return y;
+  const char* w = (const char*)up.data_ptr();
+  MoeTilesArgs a{(const char*)x.data_ptr(), w, w + F * K * 2, (__bf16*)h.data_ptr(),
+                 ints(tokens, pairs, "tokens"), ints(tiles, 0, "tiles"),
+                 ints(used, 1, "used"), stride * 2, (int)F, (int)K, 0, 2 * F * K * 2,
+                 scale.data_ptr<float>(), (float)limit, (float)alpha};
+  launch_moe_tiles(&a, (int)tile, MT_CLAMPED, stream());
+  MoeTilesArgs b{(const char*)h.data_ptr(), (const char*)down.data_ptr(), nullptr,
+                 (__bf16*)y.data_ptr(), nullptr, a.tiles, a.n_tiles, F * 2, (int)O,
+                 (int)F, 0, O * F * 2};
+  launch_moe_tiles(&b, (int)tile, MT_SUMS, stream());
+  return y;
 }
 
 // x [N, W] += weighted rows of d (or of h where the pair has none)
@@ -209,6 +247,7 @@ void bind_experts(pybind11::module_& m) {
   m.def("expert_route", &expert_route);
   m.def("expert_plan", &expert_plan);
   m.def("expert_gemm", &expert_gemm);
+  m.def("expert_tiles", &expert_tiles);
   m.def("expert_combine", &expert_combine);
   m.def("token_gate", &token_gate);
 }

@@ -29,6 +29,7 @@ struct PlanArgs {
   int *where;      // [tokens, top]: row among the sorted pairs, or -1
   int *tokens;     // [pairs]: token of a sorted pair
   int *tiles;      // [n_tiles, 3]: expert, first pair, pairs (0: none)
+  int *used;       // tiles that have pairs, which come first
   long n;
   int experts, top, n_blocks, n_tiles, tile;
 };

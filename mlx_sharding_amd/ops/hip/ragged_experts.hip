@@ -234,6 +234,7 @@ __global__ __launch_bounds__(PB) void expert_plan_kernel(const PlanArgs a,
   __syncthreads();
 
   if (blockIdx.x == 0) {
+    if (tid == 0) *a.used = first[EX_MAXTOTAL];
     if (tid < a.experts) {
       for (int i = 0; i < cuts; ++i) {
         int* t = a.tiles + (long)(first[tid] + i) * 3;
