@@ -36,7 +36,8 @@ class KVCache:
         self.offset = 0
         self._k: Optional[torch.Tensor] = None
         self._v: Optional[torch.Tensor] = None
-        # zeros that a kernel counts its blocks with, and leaves as zeros
+        # zeros that attend_step's kernel counts its blocks with, and leaves as zeros;
+        # made for tokens, as a prompt has no need of them
         self._tickets: Optional[torch.Tensor] = None
         # hipGraph-captured decode: position lives on device (int32 [1]);
         # update() appends by index_copy_ and python offset is not advanced.
@@ -53,9 +54,6 @@ class KVCache:
                          dtype=self.dtype, device=self.device)
         nv = torch.empty(batch, self.n_kv_heads, new_cap, self.v_head_dim,
                          dtype=self.dtype, device=self.device)
-        if self._tickets is None and self.device.type == "cuda":
-            self._tickets = torch.zeros(batch * self.n_kv_heads, dtype=torch.int32,
-                                        device=self.device)
         if self._k is not None and self.offset > 0:
             nk[:, :, : self.offset] = self._k[:, :, : self.offset]
             nv[:, :, : self.offset] = self._v[:, :, : self.offset]
@@ -122,7 +120,9 @@ class KVCache:
             return None
         pos, at = self.claim(k.shape[0], 1)
         if self._tickets is None:
-            return None
+            if torch.cuda.is_current_stream_capturing():
+                return None  # the zeros would be written by replays only
+            self._make_tickets()
         out = _ops.hip_ext().attn_step(q, k, v, cos, sin, self._k, self._v, pos, at,
                                        self._tickets, scale, softcap, window)
         if out is not None:
@@ -197,6 +197,13 @@ class KVCache:
         b = batch if batch is not None else (
             self._k.shape[0] if self._k is not None else self.batch_size)
         self._ensure(b, cap)
+        # a capture's warm-up steps run on a stream of their own
+        self._make_tickets()
+
+    def _make_tickets(self):
+        if self._tickets is None and self._k is not None and self._k.is_cuda:
+            self._tickets = torch.zeros(self._k.shape[0] * self.n_kv_heads,
+                                        dtype=torch.int32, device=self._k.device)
 
     # a shorter prefix of what is cached can be returned to
     trimmable = True
