@@ -279,7 +279,9 @@ static void linear_few_go(LinearFewArgs a, int split, hipStream_t stream) {
 // Tiles of W's rows per block: one up to 4096 rows, which are 256 blocks; two up
 // to 8192 (6144 rows, 16 of x: 13.7 us, 17.0 with one); beyond that four, where
 // rows of x are read once for 64 of W (28672 rows, 16 of x: 48 us, 51 with two, 56
-// with one), but one for few rows of x (one: 38 us, 45 with four).  A unit needs
+// with one), but one for few rows of x without a norm (one: 38 us, 45 with four; the norm
+// is made in every block: one of x, 128256 rows of 4096 202 us so, 181 with four, of
+// 32000 rows of 3584 51 and 44).  A unit needs
 // both its halves; four from 16384 rows on (28672 rows, 16 of x, norm: 50 us, 53
 // with two; 12800, one of x: 14.0 with two, 15.8).  One tile takes two steps at a time:
 // 4096 rows of 4096 8.3 us, of 14336 22.2, with four 9.2 and 23.3.
@@ -293,7 +295,7 @@ static void linear_few_tiles(const LinearFewArgs& a, int act, int split,
     else linear_few_go<2, LF_GELU, 8, 4>(a, 1, stream);
   } else if (a.O <= 4096) {
     linear_few_go<1, LF_PLAIN, 8, 2>(a, split, stream);
-  } else if (a.O > 8192 && a.M <= 4) {
+  } else if (a.O > 8192 && a.M <= 4 && !a.norm) {
     linear_few_go<1, LF_PLAIN, 8, 4>(a, 1, stream);
   } else if (a.O <= 8192) {
     linear_few_go<2, LF_PLAIN, 8, 4>(a, 1, stream);
@@ -540,9 +542,20 @@ static void linear_some(const LinearFewArgs& a, int act, int split, hipStream_t 
 // Whether rows of x go through LDS: above 16, and above 8 where a block would read them
 // for many columns or from many blocks (12 of x; registers, LDS: 4096 rows of 4096 9.5,
 // 9.2 us; of 14336 26, 23.8; 2048 of 8192 15.7, 12.5; 8192 of 3584 15, 13.0; 2048 of
-// 2048 6.2, 6.4; 3648 of 2048 with norm 7.3, 8.3).
-static bool few_through_lds(int M, int O, int K, int act) {
-  return M > 16 || (M > 8 && ((act ? 2 : 1) * O > 4096 || K > 2048));
+// 2048 6.2, 6.4; 3648 of 2048 with norm 7.3, 8.3).  With norms or units few rows, too,
+// where a block has four tiles of W's rows (one of x; 16032 of 4096 with norm 30.8, 25.2
+// us; 12800 of 2048 15.9, 13.4; units of 12288 of 4096 27.8, 23.8).  Not where there are
+// blocks for all CUs and the contraction is short (12 of x; units of 16384 of 2048 14.6,
+// 16.6, of 21888 24.1, 25.3; 32000 of 2048 25.0, 27.2), nor where blocks come in many
+// rounds (12 of x; 128256 of 4096 with norm 182, 192; 18000 of 4096 43, 40; one of x,
+// units of 37888 of 3584 59, 61).
+static bool few_through_lds(int M, int O, int K, int act, bool norm) {
+  const int rows = (act ? 2 : 1) * O;
+  if (M > 16) return true;
+  if (rows >= 16384 && K <= 2048) return false;
+  if (rows > 24576 && (!act || M <= 8)) return false;
+  if (M > 8) return rows > 4096 || K > 2048;
+  return (act || norm) && rows > 8192;
 }
 
 // Blocks that share a tile's contraction where the caller has room for their sums.  x is
@@ -554,7 +567,7 @@ static bool few_through_lds(int M, int O, int K, int act) {
 // of x, 2048 of 8192: 11.6, 9.7).
 static int few_split(int M, int O, int K, int act, bool norm) {
   if (act || norm) return 1;
-  if (!few_through_lds(M, O, K, act)) return O <= 2816 && K >= 4096 ? 2 : 1;
+  if (!few_through_lds(M, O, K, act, norm)) return O <= 2816 && K >= 4096 ? 2 : 1;
   if (O <= 2816) return K >= (M > 32 ? 2048 : 4096) ? 4 : 1;
   return O <= 4608 && K >= 8192 && M > 16 ? 4 : 1;
 }
@@ -581,7 +594,7 @@ extern "C" void launch_linear_few(const void* x, const void* w, const void* bias
                         M, O, K, ldx, ldw, ldr, ldy, eps, offset, part, count, zero,
                         n_zero, 0};
   const int split = count ? few_split(M, O, K, act, norm != nullptr) : 1;
-  if (few_through_lds(M, O, K, act)) {
+  if (few_through_lds(M, O, K, act, norm != nullptr)) {
     linear_some(a, act, split, stream);
   } else {
     linear_few_tiles(a, act, split, stream);
