@@ -124,13 +124,17 @@ def feed(into, out, x: torch.Tensor, act: str, norm: Optional[nn.Module] = None,
 
 def project(m, x: torch.Tensor, *, norm: Optional[nn.Module] = None,
             act: Optional[str] = None,
-            residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+            residual: Optional[torch.Tensor] = None,
+            clear: Optional[torch.Tensor] = None) -> torch.Tensor:
     """ops.project with the weights of a Linear or FusedColumns, packed ones
     through their bf16 copy."""
     w, q = dense_weight(m, x.shape[-1]), m.quant
     if w is not None:
-        return ops.project(x, w, m.bias, norm=norm, act=act, residual=residual)
+        return ops.project(x, w, m.bias, norm=norm, act=act, residual=residual,
+                           clear=clear)
     # no room for the copy
+    if clear is not None:
+        clear.zero_()
     if norm is not None:
         x = norm(x)
     y = ops.quantized_linear(x, m.weight, m.scales, m.biases, q.group_size,

@@ -275,14 +275,16 @@ class MLAAttention(nn.Module):
 
     def forward(self, x, cos, sin, cache: Optional[KVCache],
                 norm: Optional[RMSNorm] = None,
-                residual: Optional[torch.Tensor] = None):
-        """norm: for x's rows first; residual: added to what is returned.  For
-        few tokens, where both go with the projections."""
+                residual: Optional[torch.Tensor] = None,
+                clear: Optional[torch.Tensor] = None):
+        """norm: for x's rows first; residual: added to what is returned; clear:
+        numbers that are zero afterwards.  For few tokens, where these go with the
+        projections."""
         if norm is not None and self._fused_qkv is None:
             x, norm = norm(x), None
         if cache is not None and cache.n_kv_heads == 1 and self.n_heads > 1:
-            return self._forward_absorbed(x, cos, sin, cache, norm, residual)
-        return self._forward_naive(x, cos, sin, cache, norm, residual)
+            return self._forward_absorbed(x, cos, sin, cache, norm, residual, clear)
+        return self._forward_naive(x, cos, sin, cache, norm, residual, clear)
 
     def _queries_and_latent(self, x, norm):
         """(queries, cached row before norm and rotation) where one projection
@@ -292,12 +294,12 @@ class MLAAttention(nn.Module):
         return project(self._fused_qkv, x, norm=norm).split(
             self._fused_qkv.splits, -1)
 
-    def _output(self, out, residual):
+    def _output(self, out, residual, clear):
         if residual is None:
             return self.o_proj(out)
-        return project(self.o_proj, out, residual=residual)
+        return project(self.o_proj, out, residual=residual, clear=clear)
 
-    def _forward_absorbed(self, x, cos, sin, cache: KVCache, norm, residual):
+    def _forward_absorbed(self, x, cos, sin, cache: KVCache, norm, residual, clear):
         """Compressed-cache path: cache rows are [c_kv | k_pe] (rank +
         rope).  Decode = MQA over the compressed rows with q/out
         absorbed through W_UK/W_UV; prefill expands K/V from the
@@ -316,9 +318,9 @@ class MLAAttention(nn.Module):
         if ckv is None:
             ckv = self.kv_a_proj_with_mqa(x)
         if T == 1 and self._one_token_ok(qh, ckv, cache):
-            return self._output(self._one_token(qh, ckv, cos, sin, cache), residual)
+            return self._output(self._one_token(qh, ckv, cos, sin, cache), residual, clear)
         if T > 1 and self._prompt_ok(qh, ckv, cos, cache):
-            return self._output(self._prompt(qh, ckv, cos, sin, cache), residual)
+            return self._output(self._prompt(qh, ckv, cos, sin, cache), residual, clear)
         qh = qh.view(B, T, nh, self.qk_head_dim)
         q_nope = qh[..., : self.qk_nope]
         q_pe = ops.apply_rope(qh[..., self.qk_nope:], cos, sin,
@@ -353,7 +355,7 @@ class MLAAttention(nn.Module):
             ov = torch.bmm(o.permute(1, 0, 2, 3).reshape(nh, B * T, rank),
                            self._w_uv)
             out = ov.view(nh, B, T, self.v_head_dim).permute(1, 2, 0, 3)
-            return self._output(out.reshape(B, T, -1), residual)
+            return self._output(out.reshape(B, T, -1), residual, clear)
 
         # prefill: expand the WHOLE compressed prefix (covers chunked
         # prefill, where earlier chunks live only in the cache)
@@ -378,10 +380,10 @@ class MLAAttention(nn.Module):
             v = kvh[..., self.qk_nope:].transpose(1, 2).contiguous()
         qf = torch.cat([q_nope, q_pe], dim=-1).transpose(1, 2)
         out = ops.attention(qf, k, v, self.scale, causal_offset=offset)
-        return self._output(out.transpose(1, 2).reshape(B, T, -1), residual)
+        return self._output(out.transpose(1, 2).reshape(B, T, -1), residual, clear)
 
     def _forward_naive(self, x, cos, sin, cache: Optional[KVCache], norm,
-                       residual):
+                       residual, clear):
         B, T, _ = x.shape
         ckv = None
         if self._fused_qkv is not None:
@@ -430,7 +432,7 @@ class MLAAttention(nn.Module):
                 k, v = cache.update(k, v)
         out = ops.attention(qf, k, v, self.scale, causal_offset=offset,
                             pos_dev=gp)
-        return self._output(out.transpose(1, 2).reshape(B, T, -1), residual)
+        return self._output(out.transpose(1, 2).reshape(B, T, -1), residual, clear)
 
 
 @read_in_place
@@ -492,15 +494,15 @@ class DeepseekV2MoE(nn.Module):
                 dense_weight(m.down_proj, m.down_proj.in_features))
         return both if ops.expert_shared_ok(*y.shape, *both) else None
 
-    def decode(self, x, residual, norm):
+    def decode(self, x, residual, norm, tickets=None):
         """The residual x (+ residual) after this feed-forward of it, normed:
         three kernels for the routed and the shared experts, with norm, router and
-        choice in a fourth."""
+        choice in a fourth.  tickets: a zero (int32) per token."""
         shape, H = x.shape, x.shape[-1]
         y, h, choice, weight = ops.expert_route(
             x.reshape(-1, H), None if residual is None else residual.reshape(-1, H),
             norm, self.gate.weight, self.top_k, self.routed_scaling_factor,
-            self.norm_topk_prob)
+            self.norm_topk_prob, tickets)
         m = self.switch_mlp
         stacks = [[p.weight] if m.quant is None else [p.weight, p.scales, p.biases]
                   for p in (m.gate_proj, m.up_proj, m.down_proj)]
@@ -569,9 +571,12 @@ class DeepseekV2DecoderLayer(nn.Module):
         if (ops.few_tokens(x) and as_built(attn, norm)
                 and as_built(*attn.read())
                 and (experts or (as_built(mlp) and as_built(*mlp.read())))):
-            h = attn(x, cos, sin, cache, norm, x)
+            # for the router's blocks, cleared on the way
+            tickets = x.new_empty(x.numel() // x.shape[-1],
+                                  dtype=torch.int32) if decode else None
+            h = attn(x, cos, sin, cache, norm, x, tickets)
             if decode:
-                return mlp.decode(h, None, self.post_attention_layernorm)
+                return mlp.decode(h, None, self.post_attention_layernorm, tickets)
             if not experts:
                 return mlp(h, self.post_attention_layernorm, h)
             pn = self.post_attention_layernorm

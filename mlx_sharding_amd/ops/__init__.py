@@ -313,15 +313,16 @@ def _few_for(x, *weights):
     return _EXT if _EXT is not None else _few_ext()
 
 
-def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None):
+def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None, clear=None):
     """project on linear_few.hip, or None where that does not take it."""
     ext = _few_for(x, weight)
     if ext is None:
         return None
     if norm is None:
-        return ext.linear_few_try(x, weight, bias, residual, None, 0.0, 0.0, _ACTS[act])
+        return ext.linear_few_try(x, weight, bias, residual, None, 0.0, 0.0, _ACTS[act],
+                                  clear)
     return ext.linear_few_try(x, weight, bias, residual, norm.weight, norm.eps,
-                              norm.weight_offset, _ACTS[act])
+                              norm.weight_offset, _ACTS[act], clear)
 
 
 def feed_few(x, w_in, w_out, act, norm=None, residual=None):
@@ -337,14 +338,17 @@ def feed_few(x, w_in, w_out, act, norm=None, residual=None):
                             norm.weight_offset, _ACTS[act])
 
 
-def project(x, weight, bias=None, *, norm=None, act=None, residual=None):
+def project(x, weight, bias=None, *, norm=None, act=None, residual=None, clear=None):
     """x W^T + bias, of x's rows as ``norm`` (an RMSNorm) makes them; ``act``:
-    the gated unit act(gate) * up of the result's halves; plus ``residual``.
-    One kernel for few rows, else one for each of these."""
+    the gated unit act(gate) * up of the result's halves; plus ``residual``;
+    ``clear``: numbers (int32) that are zero afterwards.  One kernel for few rows, else
+    one for each of these."""
     if x.is_cuda:
-        y = _linear_few(x, weight, bias, residual, norm, act)
+        y = _linear_few(x, weight, bias, residual, norm, act, clear)
         if y is not None:
             return y
+    if clear is not None:
+        clear.zero_()
     if norm is not None:
         x = norm(x)
     return finish(linear(x, weight, bias), act, residual)
@@ -691,12 +695,13 @@ def expert_rows_ok(x, gate_w, up, down, top: int, bits: int, group_size: int
 
 
 def expert_route(x, residual, norm, gate_w, top: int, scaling: float,
-                 normalize: bool):
+                 normalize: bool, tickets=None):
     """(rows of x + residual as ``norm`` makes them, x + residual, experts and
-    weights of every token), one kernel; rows [N, H]."""
+    weights of every token), one kernel; rows [N, H].  tickets: N zeros (int32), with
+    which a token has several blocks; they are used up."""
     return _require_ext("moe_route").moe_route(
         _whole(x), None if residual is None else _whole(residual), norm.weight,
-        norm.eps, norm.weight_offset, gate_w, top, scaling, normalize)
+        norm.eps, norm.weight_offset, gate_w, top, scaling, normalize, tickets)
 
 
 def _whole(t: torch.Tensor) -> torch.Tensor:

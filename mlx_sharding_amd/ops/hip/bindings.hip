@@ -1102,13 +1102,13 @@ static void check_rows(const torch::Tensor& t, const char* name, long n, long w)
 }
 
 // x [N, H] (+ residual) -> normed rows, x + residual (or x), experts and weights
-// of every token [N, top]
+// of every token [N, top].  tickets [N]: zeros that the blocks of a token count with
 std::vector<torch::Tensor> moe_route(torch::Tensor x,
                                      c10::optional<torch::Tensor> residual,
                                      torch::Tensor norm, double eps,
                                      double offset, torch::Tensor gate,
-                                     int64_t top, double scaling,
-                                     bool normalize) {
+                                     int64_t top, double scaling, bool normalize,
+                                     c10::optional<torch::Tensor> tickets) {
   TORCH_CHECK(x.dim() == 2 && gate.dim() == 2 && norm.dim() == 1, "shapes");
   const long N = x.size(0), H = x.size(1), E = gate.size(0);
   TORCH_CHECK(N >= 1 && H % 128 == 0 && H <= 8192,
@@ -1122,13 +1122,22 @@ std::vector<torch::Tensor> moe_route(torch::Tensor x,
   auto h = residual.has_value() ? torch::empty_like(x) : x;
   auto choice = torch::empty({N, top}, x.options().dtype(torch::kInt32));
   auto weight = torch::empty({N, top}, x.options().dtype(torch::kFloat32));
+  torch::Tensor logits;
+  if (tickets.has_value()) {
+    TORCH_CHECK(tickets->device() == x.device() && tickets->numel() == N &&
+                    tickets->scalar_type() == torch::kInt32 && tickets->is_contiguous(),
+                "a number per token");
+    logits = torch::empty({N, 64}, weight.options());
+  }
   const MoeRouteArgs a{
       (const __bf16*)x.data_ptr(),
       residual.has_value() ? (const __bf16*)residual->data_ptr() : nullptr,
       (const __bf16*)norm.data_ptr(), (const __bf16*)gate.data_ptr(),
       (__bf16*)h.data_ptr(), (__bf16*)y.data_ptr(), choice.data_ptr<int>(),
       weight.data_ptr<float>(), (int)H, (int)E, (int)top, (float)eps,
-      (float)offset, (float)scaling, normalize};
+      (float)offset, (float)scaling, normalize,
+      tickets.has_value() ? logits.data_ptr<float>() : nullptr,
+      tickets.has_value() ? reinterpret_cast<unsigned*>(tickets->data_ptr<int>()) : nullptr};
   launch_moe_route(&a, (int)N, cur_stream());
   return {y, h, choice, weight};
 }
@@ -1400,7 +1409,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill_shape_ok", [](int64_t dk, int64_t dv) {
     return attn_prefill_supported((int)dk, (int)dv);
   });
-  m.def("linear_few_try", &linear_few_try);
+  m.def("linear_few_try", &linear_few_try, py::arg("x"), py::arg("w"), py::arg("bias"),
+        py::arg("residual"), py::arg("norm"), py::arg("eps"), py::arg("offset"),
+        py::arg("act"), py::arg("clear") = py::none());
   m.def("feed_few_try", &feed_few_try);
   m.def("mla_rows", &mla_rows);
   m.def("mla_prompt", &mla_prompt);
@@ -1410,7 +1421,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_decode_tile", [](int64_t g, int64_t dk, int64_t dv, bool inrow) {
     return attn_decode_tile((int)g, (int)dk, (int)dv, inrow);
   });
-  m.def("moe_route", &moe_route);
+  m.def("moe_route", &moe_route, py::arg("x"), py::arg("residual"), py::arg("norm"),
+        py::arg("eps"), py::arg("offset"), py::arg("gate"), py::arg("top"),
+        py::arg("scaling"), py::arg("normalize"), py::arg("tickets") = py::none());
   m.def("moe_pack", &moe_pack);
   m.def("moe_rows", &moe_rows);
   m.def("moe_rows_longest", [](int64_t bits) { return moe_rows_longest((int)bits); });

@@ -213,18 +213,27 @@ static torch::Tensor linear_few_shaped(const torch::Tensor& y, const torch::Tens
 }
 
 // linear_few for x of any number of dimensions, or nothing where it does not run here.
+// clear: int32 numbers that are zero afterwards.
 static c10::optional<torch::Tensor> linear_few_try(
     torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
     c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> norm,
-    double eps, double offset, int64_t act) {
+    double eps, double offset, int64_t act, c10::optional<torch::Tensor> clear) {
   if (!linear_few_takes(x, w, !residual.has_value() && !norm.has_value() && !act) ||
       !linear_few_along(x, w.size(0) / (act ? 2 : 1), w.size(0), bias, residual, norm))
     return {};
   const auto rows = linear_few_rows(x);
   if (residual.has_value() && x.dim() != 2)
     residual = residual->reshape({rows.size(0), -1});
+  LinearFewRoom cleared;
+  if (clear.has_value()) {
+    TORCH_CHECK(clear->device() == x.device() && clear->is_contiguous() &&
+                    clear->scalar_type() == torch::kInt32 && clear->numel() < 1 << 20,
+                "numbers to clear");
+    cleared.numbers = reinterpret_cast<unsigned*>(clear->data_ptr<int>());
+    cleared.n = (int)clear->numel();
+  }
   return linear_few_shaped(
-      linear_few(rows, w, bias, residual, norm, eps, offset, act), x);
+      linear_few_run(rows, w, bias, residual, norm, eps, offset, act, {}, cleared), x);
 }
 
 // A feed-forward: w_out of the gated unit of w_in's halves (act 1 or 2), of x's rows as

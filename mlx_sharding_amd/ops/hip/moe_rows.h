@@ -28,6 +28,8 @@ struct MoeRouteArgs {
   int H, E, top;
   float eps, offset, scaling;
   int normalize;
+  float* logits;       // [N, 64], and a number per token that is 0 before: with these a
+  unsigned* tickets;   // token has a block for every 16 experts
 };
 
 extern "C" {

@@ -566,9 +566,114 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const MoeRouteArgs a) {
   }
 }
 
+// The same with a block for every 16 experts of a token: a CU reads about 30 bytes a
+// nanosecond, 8.5 us for all weights of 64 experts of 2048.  The last block of a token
+// has all logits, which pass the XCDs' L2s by accesses of the device's scope, and chooses.
+// One token: 13.0 -> 8.7 us, 64: 13.2 -> 9.1.
+__global__ __launch_bounds__(256) void moe_route_parts_kernel(const MoeRouteArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __bf16* row = reinterpret_cast<__bf16*>(smem);  // [H]
+  __shared__ float scratch[4];
+  __shared__ float part[4][16];
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lg = lane >> 4, first = blockIdx.y * 16;
+  const long t = blockIdx.x;
+
+  auto load = [](const __bf16* p) { return *reinterpret_cast<const bf16x8_t*>(p); };
+  bf16x8_t v[4], r[4], n[4];  // up to 8192 columns
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int col = (i * 256 + threadIdx.x) * 8;
+    if (col >= a.H) continue;
+    v[i] = load(a.x + t * a.H + col);
+    if (a.residual) r[i] = load(a.residual + t * a.H + col);
+    n[i] = load(a.norm + col);
+  }
+  const int steps = a.H / 128;  // of 32, of this quarter
+  const __bf16* g = a.gate + (long)min(first + (lane & 15), a.E - 1) * a.H +
+                    quarter * steps * 32 + lg * 8;
+  bf16x8_t w[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) w[i] = load(g + min(i, steps - 1) * 32);
+
+  float ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int col = (i * 256 + threadIdx.x) * 8;
+    if (col >= a.H) continue;
+    if (a.residual) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[i][j] = (__bf16)((float)v[i][j] + (float)r[i][j]);
+      if (blockIdx.y == 0) *reinterpret_cast<bf16x8_t*>(a.h + t * a.H + col) = v[i];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss = fmaf((float)v[i][j], (float)v[i][j], ss);
+  }
+  ss = block_sum<256>(ss, scratch);
+  const float f = rsqrtf(ss / a.H + a.eps);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int col = (i * 256 + threadIdx.x) * 8;
+    if (col >= a.H) continue;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      v[i][j] = (__bf16)((float)v[i][j] * f * ((float)n[i][j] + a.offset));
+    *reinterpret_cast<bf16x8_t*>(row + col) = v[i];
+    if (blockIdx.y == 0) *reinterpret_cast<bf16x8_t*>(a.y + t * a.H + col) = v[i];
+  }
+  __syncthreads();
+
+  const __bf16* x = row + quarter * steps * 32 + lg * 8;
+  f32x4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+  for (int s = 0; s < steps; s += 16) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (s + i < steps)
+        acc[i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], load(x + (s + i) * 32),
+                                                             acc[i & 1], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (s + 16 + i < steps) w[i] = load(g + (s + 16 + i) * 32);
+  }
+  if ((lane & 15) == 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) part[quarter][lg * 4 + j] = acc[0][j] + acc[1][j];
+  }
+  __syncthreads();
+  if (quarter != 0) return;
+  float* logits = a.logits + t * 64;
+  if (lane < 16)
+    __hip_atomic_store(logits + first + lane,
+                       (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  unsigned before = 0;
+  if (lane == 0)
+    before = __hip_atomic_fetch_add(a.tickets + t, 1u, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+  if (__builtin_amdgcn_readfirstlane(before) + 1 != gridDim.y) return;
+  asm volatile("" ::: "memory");
+  const float z = lane < a.E ? __hip_atomic_load(logits + lane, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT)
+                             : -INFINITY;
+  int place;
+  float weight;
+  if (chosen_expert(z, lane, a.E, a.top, a.normalize, a.scaling, place, weight)) {
+    a.choice[t * a.top + place] = lane;
+    a.weight[t * a.top + place] = weight;
+  }
+}
+
 extern "C" void launch_moe_route(const MoeRouteArgs* a, int N,
                                  hipStream_t stream) {
-  moe_route_kernel<<<dim3((unsigned)N), dim3(1024), (size_t)a->H * 2, stream>>>(*a);
+  const size_t smem = (size_t)a->H * 2;
+  if (a->tickets) {
+    moe_route_parts_kernel<<<dim3((unsigned)N, (unsigned)((a->E + 15) / 16)), dim3(256),
+                             smem, stream>>>(*a);
+  } else {
+    moe_route_kernel<<<dim3((unsigned)N), dim3(1024), smem, stream>>>(*a);
+  }
 }
 
 // -- sum --------------------------------------------------------------------

@@ -817,7 +817,9 @@ Tensor cap_logits(Tensor z, double scale, double limit) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("glu", &glu);
-  m.def("linear_few_try", &linear_few_try);
+  m.def("linear_few_try", &linear_few_try, py::arg("x"), py::arg("w"), py::arg("bias"),
+        py::arg("residual"), py::arg("norm"), py::arg("eps"), py::arg("offset"),
+        py::arg("act"), py::arg("clear") = py::none());
   m.def("feed_few_try", &feed_few_try);
   m.def("clamped_glu", &clamped_glu, py::arg("gate"), py::arg("up"),
         py::arg("limit"), py::arg("alpha"), py::arg("gate_bias") = py::none(),
