@@ -376,7 +376,7 @@ extern "C" bool attn_decode_supported_shape(int G, int Dv) {
 // Slices come from the length on the device, so they are even under capture.
 // Measured (before: dot products and sums on the vector units, up to 8 slices of
 // the capacity): 64 sequences of 2049 keys, 32 heads of 128 over 8: 179 -> 98 us
-// (5.5 TB/s); one of 1024: 24 -> 7.2; 5 of 5004, 16 heads of 256 over 8, capped: 91 ->
+// (now in the kernel for heads of 64 and 128); one of 1024: 24 -> 7.2; 5 of 5004, 16 heads of 256 over 8, capped: 91 ->
 // 45; 16 heads over a latent of 576/512, 64 x 513 keys: 66 -> 22, 1 x 3002: 75 -> 13.
 // ---------------------------------------------------------------------------
 
@@ -403,10 +403,14 @@ struct DecodeArgs {
   unsigned* tickets;
 };
 
+// Keys and values are read once: as a stream (2) they leave the L2 to what is read again
+// (the sizes below: 64 x 2049 keys 109 -> 101 us, 5 x 5004 of 256 46.5 -> 45.5; latents
+// 16.4 -> 16.8, and stay as they were).
+template <bool STREAM>
 __device__ __forceinline__ void dt_to_lds(const char* src, char* dst) {
   __builtin_amdgcn_global_load_lds(
       (const __attribute__((address_space(1))) void*)src,
-      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+      (__attribute__((address_space(3))) void*)dst, 16, 0, STREAM ? 2 : 0);
 }
 
 // Place of a 16-byte piece within its row in LDS: keys are read a row a lane,
@@ -459,6 +463,100 @@ __device__ __forceinline__ bf16x8_t turned(const char* head, int d, const Decode
   return y;
 }
 
+// What a block has of its slice, [column of 16][4] a lane of wave `wid` for head l16, to
+// the output or to the partial results; the last block of a STEP merges them.  slices:
+// those that have keys.
+template <int DV, bool STEP, int N>
+__device__ __forceinline__ void finish_slice(const DecodeArgs& a, const f32x4 (&o)[N],
+                                             float m, float l, long row0, int G, int wid,
+                                             int l16, int lg, int slices) {
+  const long row = row0 + l16;
+  const int col = wid * N * 16 + lg * 4;
+  auto write = [&](long r, int c, const f32x4& v, float f) {
+    bf16 w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = f2bf(v[i] * f);
+    *reinterpret_cast<short4v*>(a.out + (r * DV + c) * 2) = *reinterpret_cast<short4v*>(w);
+  };
+  if (slices == 1 && a.out) {
+    if (l16 >= G) return;
+    const float f = 1.0f / l;
+#pragma unroll
+    for (int d = 0; d < N; ++d) write(row, col + d * 16, o[d], f);
+    return;
+  }
+  const long part = row * a.nsplit + blockIdx.y;
+  if constexpr (!STEP) {
+    if (l16 >= G) return;
+#pragma unroll
+    for (int d = 0; d < N; ++d)
+      *reinterpret_cast<f32x4*>(a.part_o + part * DV + col + d * 16) = o[d];
+    if (wid == 0 && lg == 0) {
+      a.part_ml[part * 2] = m;
+      a.part_ml[part * 2 + 1] = l;
+    }
+  } else {
+    if (l16 < G) {
+#pragma unroll
+      for (int d = 0; d < N; ++d) leave(a.part_o + part * DV + col + d * 16, o[d]);
+      if (wid == 0 && lg == 0) {
+        typedef float f32x2 __attribute__((ext_vector_type(2)));
+        __hip_atomic_store(reinterpret_cast<u64*>(a.part_ml) + part,
+                           __builtin_bit_cast(u64, f32x2{m, l}), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    __shared__ unsigned before;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+      before = __hip_atomic_fetch_add(a.tickets + blockIdx.x, 1u, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (before + 1 != (unsigned)slices) return;
+    if (threadIdx.x == 0)
+      __hip_atomic_store(a.tickets + blockIdx.x, 0u, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    for (int i = threadIdx.x; i < G * (DV / 4); i += blockDim.x) {
+      const int g = i / (DV / 4), c = i % (DV / 4) * 4;
+      const long p0 = (row0 + g) * a.nsplit;
+      float top = -1e30f, all = 0.0f;
+      f32x4 sum = {0, 0, 0, 0};
+      for (int n0 = 0; n0 < slices; n0 += 16) {  // many at once, with their weights
+        u64x2 v[16];
+        f32x2 ml[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const long n = p0 + min(n0 + j, slices - 1);
+          ml[j] = __builtin_bit_cast(f32x2, found(a.part_ml + n * 2));
+          const float* at = a.part_o + n * DV + c;
+          v[j] = u64x2{found(at), found(at + 2)};
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float most = top;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) most = fmaxf(most, ml[j][0]);
+        const float keep = __builtin_amdgcn_exp2f(top - most);
+        top = most;
+        all *= keep;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[r] *= keep;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          if (n0 + j >= slices) continue;
+          const f32x4 f = __builtin_bit_cast(f32x4, v[j]);
+          const float by = __builtin_amdgcn_exp2f(ml[j][0] - top);
+          all += ml[j][1] * by;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sum[r] += f[r] * by;
+        }
+      }
+      write(row0 + g, c, sum, 1.0f / all);
+    }
+  }
+}
+
 // STEP: queries and the token's key are turned here, its key and value go to the cache
 // and into the last tile, and the last block of a head merges the slices.  The chain
 // through memory to that block takes what the merging kernel took (5 us), the rotations
@@ -502,13 +600,13 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
 #pragma unroll
     for (int i = 0; i < KB / 4096; ++i) {
       const int part = i * 4 + wid, s = part * 64 + lane, row = s / KP;
-      dt_to_lds(ks + min(row, last) * (DK * 2) +
+      dt_to_lds<!INROW>(ks + min(row, last) * (DK * 2) +
                     dt_place<KP, true>(row, s % KP) * 16, dst + part * 1024);
     }
 #pragma unroll
     for (int i = 0; i < VB / 4096; ++i) {
       const int part = i * 4 + wid, s = part * 64 + lane, row = s / VP;
-      dt_to_lds(vs + min(row, last) * (DV * 2) +
+      dt_to_lds<!INROW>(vs + min(row, last) * (DV * 2) +
                     dt_place<VP, false>(row, s % VP) * 16,
                 dst + KB + part * 1024);
     }
@@ -658,93 +756,224 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
 
   l += __shfl_xor(l, 16, WAVE);
   l += __shfl_xor(l, 32, WAVE);
-  const long row = row0 + l16;
-  const int col = wid * ND * 16 + lg * 4;
-  auto write = [&](long r, int c, const f32x4& v, float f) {
-    bf16 w[4];
+  finish_slice<DV, STEP>(a, o, m, l, row0, G, wid, l16, lg,
+                         STEP ? max(1, (S - lo + per - 1) / max(per, 1)) : a.nsplit);
+}
+
+// Heads of 64 and 128.  A wave has tiles of 32 keys of its own, which go to its own LDS,
+// NB of them by turns, and keeps outputs of all columns: scores come out of the first
+// product as the second one takes them, so that waves meet at the end of a slice only, and
+// each makes its own keys' weights.  In the kernel above a tile's scores pass two barriers
+// and all waves make all weights, a chain of 2 us beside loads of 3.  64 sequences of 2049
+// keys, 32 heads of 128 over 8: 101 us there, 92 here (5.8 TB/s); one of 1024: 9.6, 9.8.
+#define DW_WAVES 2
+template <int D, int NB, bool STEP>
+__global__ __launch_bounds__(DW_WAVES* WAVE) void attn_decode_wave_kernel(
+    const DecodeArgs a) {
+  constexpr int KT = 32, P = D / 8, NK = D / 32, ND = D / 16, BYTES = KT * D * 2;
+  constexpr int LOADS = 2 * BYTES / 1024;
+  // LDS whose size the compiler knows it guards: a read would wait for all loads to LDS
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+
+  const int S = a.s_ptr ? (int)min((long)*a.s_ptr + 1, a.cap) : a.S;
+  const int b = blockIdx.x / a.Hkv, hk = blockIdx.x % a.Hkv;
+  const int G = a.Hq / a.Hkv;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int l16 = lane & 15, lg = lane >> 4;
+  constexpr int SPAN = DW_WAVES * KT;
+  const int lo = a.window > 0 && S > a.window ? S - a.window : 0;
+  const int per = ((S - lo + a.nsplit - 1) / a.nsplit + SPAN - 1) / SPAN * SPAN;
+  const int from = min(S, lo + per * (int)blockIdx.y);
+  const int to = min(S, from + per);
+  if (STEP && from >= to && from > lo) return;  // nothing of the keys, nor of the count
+
+  char* own = smem + wid * NB * 2 * BYTES;
+  const char* kbase = a.k + (long)blockIdx.x * a.cap * (D * 2);
+  const char* vbase = a.v + (long)blockIdx.x * a.cap * (D * 2);
+  // rows behind the slice repeat its last one; their weights are zero
+  auto stage = [&](int t, int buf) {
+    char* dst = own + buf * (2 * BYTES);
+    const char* ks = kbase + (long)t * (D * 2);
+    const char* vs = vbase + (long)t * (D * 2);
+    const int last = to - 1 - t;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = f2bf(v[i] * f);
-    *reinterpret_cast<short4v*>(a.out + (r * DV + c) * 2) = *reinterpret_cast<short4v*>(w);
+    for (int i = 0; i < BYTES / 1024; ++i) {
+      const int at = i * WAVE + lane, row = at / P;
+      dt_to_lds<true>(ks + min(row, last) * (D * 2) + dt_place<P, true>(row, at % P) * 16,
+                dst + i * 1024);
+    }
+#pragma unroll
+    for (int i = 0; i < BYTES / 1024; ++i) {
+      const int at = i * WAVE + lane, row = at / P;
+      dt_to_lds<true>(vs + min(row, last) * (D * 2) + dt_place<P, false>(row, at % P) * 16,
+                dst + BYTES + i * 1024);
+    }
   };
-  // slices that have keys
-  const int slices = STEP ? max(1, (S - lo + per - 1) / max(per, 1)) : a.nsplit;
-  if (slices == 1 && a.out) {
-    if (l16 >= G) return;
-    const float f = 1.0f / l;
+  const int first = from + wid * KT, tiles = max(0, (to - first + SPAN - 1) / SPAN);
+  auto tile = [&](int i) { return first + i * SPAN; };
 #pragma unroll
-    for (int d = 0; d < ND; ++d) write(row, col + d * 16, o[d], f);
-    return;
-  }
-  const long part = row * a.nsplit + blockIdx.y;
-  if constexpr (!STEP) {
-    if (l16 >= G) return;
+  for (int i = 0; i < NB; ++i)
+    if (i < tiles) stage(tile(i), i);
+
+  const long row0 = (long)b * a.Hq + hk * G;  // first query head
+  bf16x8_t qf[NK];
+  {
+    const char* head = STEP ? a.q + ((long)b * a.qs + (hk * G + min(l16, G - 1)) * D) * 2
+                            : a.q + (row0 + min(l16, G - 1)) * (D * 2);
 #pragma unroll
-    for (int d = 0; d < ND; ++d)
-      *reinterpret_cast<f32x4*>(a.part_o + part * DV + col + d * 16) = o[d];
-    if (wid == 0 && lg == 0) {
-      a.part_ml[part * 2] = m;
-      a.part_ml[part * 2 + 1] = l;
-    }
-  } else {
-    if (l16 < G) {
-#pragma unroll
-      for (int d = 0; d < ND; ++d) leave(a.part_o + part * DV + col + d * 16, o[d]);
-      if (wid == 0 && lg == 0) {
-        typedef float f32x2 __attribute__((ext_vector_type(2)));
-        __hip_atomic_store(reinterpret_cast<u64*>(a.part_ml) + part,
-                           __builtin_bit_cast(u64, f32x2{m, l}), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-    __shared__ unsigned before;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0)
-      before = __hip_atomic_fetch_add(a.tickets + blockIdx.x, 1u, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (before + 1 != (unsigned)slices) return;
-    if (threadIdx.x == 0)
-      __hip_atomic_store(a.tickets + blockIdx.x, 0u, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    for (int i = threadIdx.x; i < G * (DV / 4); i += AD_BLOCK) {
-      const int g = i / (DV / 4), c = i % (DV / 4) * 4;
-      const long p0 = (row0 + g) * a.nsplit;
-      float top = -1e30f, all = 0.0f;
-      f32x4 sum = {0, 0, 0, 0};
-      for (int n0 = 0; n0 < slices; n0 += 16) {  // many at once, with their weights
-        u64x2 v[16];
-        f32x2 ml[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const long n = p0 + min(n0 + j, slices - 1);
-          ml[j] = __builtin_bit_cast(f32x2, found(a.part_ml + n * 2));
-          const float* at = a.part_o + n * DV + c;
-          v[j] = u64x2{found(at), found(at + 2)};
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        float most = top;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) most = fmaxf(most, ml[j][0]);
-        const float keep = __builtin_amdgcn_exp2f(top - most);
-        top = most;
-        all *= keep;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sum[r] *= keep;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          if (n0 + j >= slices) continue;
-          const f32x4 f = __builtin_bit_cast(f32x4, v[j]);
-          const float by = __builtin_amdgcn_exp2f(ml[j][0] - top);
-          all += ml[j][1] * by;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) sum[r] += f[r] * by;
-        }
-      }
-      write(row0 + g, c, sum, 1.0f / all);
+    for (int i = 0; i < NK; ++i) {
+      if constexpr (STEP) qf[i] = turned<D>(head, i * 32 + lg * 8, a);
+      else qf[i] = *reinterpret_cast<const bf16x8_t*>(head + i * 64 + lg * 16);
     }
   }
+  // the token itself, at S - 1; it has no place where the cache is full
+  const int tail = (to - 1 - from) / KT;  // the slice's last tile
+  const bool newest = STEP && from < to && to == S && tail % DW_WAVES == wid &&
+                      (!a.s_ptr || *a.s_ptr < a.cap);
+  const int piece = lane % P;  // of its rows
+  bf16x8_t fresh_k, fresh_v;
+  if (newest) {
+    const long at = (long)blockIdx.x * a.cap + S - 1;
+    fresh_v = *reinterpret_cast<const bf16x8_t*>(
+        a.vnew + ((long)b * a.vs + hk * D + piece * 8) * 2);
+    fresh_k = turned<D>(a.knew + ((long)b * a.ks + hk * D) * 2, piece * 8, a);
+    if (lane < P) {
+      *reinterpret_cast<bf16x8_t*>(const_cast<char*>(a.k) + (at * D + piece * 8) * 2) =
+          fresh_k;
+      *reinterpret_cast<bf16x8_t*>(const_cast<char*>(a.v) + (at * D + piece * 8) * 2) =
+          fresh_v;
+    }
+  }
+  float m = -1e30f, l = 0.0f;  // reference of the exponents (base 2), sum
+  f32x4 o[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) o[d] = f32x4{0, 0, 0, 0};
+  // waited for here: a wait in the loop would be one for all tiles under way
+#pragma unroll
+  for (int i = 0; i < NK; ++i) asm volatile("" : "+v"(qf[i]));
+  if (newest) asm volatile("" : "+v"(fresh_k), "+v"(fresh_v));
+
+  int buf = 0;
+  for (int i = 0; i < tiles; ++i, buf = buf + 1 == NB ? 0 : buf + 1) {
+    const int t = tile(i);
+    // tiles behind this one stay on their way
+    if (i + NB - 1 < tiles)
+      asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NB - 1) * LOADS) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    char* kt = own + buf * (2 * BYTES);
+    char* vt = kt + BYTES;
+    if (newest && t + SPAN >= to) {
+      // what came from the token's place in the cache is not there yet, in its row and
+      // in those behind, which repeat it
+      const int row = S - 1 - t;
+      if (lane < P)
+        *reinterpret_cast<bf16x8_t*>(kt + row * P * 16 +
+                                     dt_place<P, true>(row, piece) * 16) = fresh_k;
+      for (int r = row + lane / P; r < KT; r += WAVE / P)
+        *reinterpret_cast<bf16x8_t*>(vt + r * P * 16 +
+                                     dt_place<P, false>(r, piece) * 16) = fresh_v;
+    }
+    f32x4 s[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+    for (int i = 0; i < NK; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const bf16x8_t f = *reinterpret_cast<const bf16x8_t*>(
+            kt + (h * 16 + l16) * P * 16 + dt_place<P, true>(l16, i * 4 + lg) * 16);
+        s[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f, qf[i], s[h], 0, 0, 0);
+      }
+    float p[8], top = -INFINITY;
+    auto key_of = [&](int i) { return i / 4 * 16 + lg * 4 + (i & 3); };
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] = s[i / 4][i & 3];
+    if (a.score.out > 0.0f) {
+      soft_capped(a.score, p);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) p[i] *= a.score.lin;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (t + key_of(i) >= to) p[i] = -INFINITY;
+      top = fmaxf(top, p[i]);
+    }
+    top = column_max(top);
+    const float m_new = fmaxf(m, top);
+    if (__any(m_new > m)) {
+      const float f = __builtin_amdgcn_exp2f(m - m_new);
+      m = m_new;
+      l *= f;
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[d][r] *= f;
+    }
+    u32x4 w[3];  // pairs: the upper halves of what is left of each weight
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+      float f[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        f[h] = __builtin_amdgcn_exp2f(p[j + h] - m);
+        l += f[h];
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const unsigned a = __float_as_uint(f[0]), b = __float_as_uint(f[1]);
+        w[i][j / 2] = __builtin_amdgcn_perm(b, a, 0x07060302);
+        f[0] -= __uint_as_float(a & 0xFFFF0000u);
+        f[1] -= __uint_as_float(b & 0xFFFF0000u);
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      const int row = lg * 4 + (l16 >> 2);  // of each half of 16 keys
+      const char* src = vt + row * P * 16 +
+                        dt_place<P, false>(row, d * 2 + (l16 >> 1 & 1)) * 16 + (l16 & 1) * 8;
+      const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (__attribute__((address_space(3))) s16x4*)src);
+      const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (__attribute__((address_space(3))) s16x4*)(src + 16 * P * 16));
+      const bf16x8_t v = __builtin_bit_cast(
+          bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            v, __builtin_bit_cast(bf16x8_t, w[i]), o[d], 0, 0, 0);
+    }
+    // all of the tile is read
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (i + NB < tiles) stage(tile(i + NB), buf);
+  }
+  l += __shfl_xor(l, 16, WAVE);
+  l += __shfl_xor(l, 32, WAVE);
+
+  // waves' outputs: each finishes half of the columns
+  constexpr int N = ND / DW_WAVES;
+  static_assert(DW_WAVES == 2 && NB * 4 * BYTES >= DW_WAVES * (N * 4 + 2) * WAVE * 4, "room");
+  f32x4* ro = reinterpret_cast<f32x4*>(smem);                    // [waves][N][lanes]
+  float* rm = reinterpret_cast<float*>(ro + DW_WAVES * N * WAVE);  // [waves][2][lanes]
+  __syncthreads();
+#pragma unroll
+  for (int d = 0; d < N; ++d) ro[(wid * N + d) * WAVE + lane] = wid ? o[d] : o[N + d];
+  rm[(wid * 2) * WAVE + lane] = m;
+  rm[(wid * 2 + 1) * WAVE + lane] = l;
+  __syncthreads();
+  const float om = rm[(wid ^ 1) * 2 * WAVE + lane], ol = rm[((wid ^ 1) * 2 + 1) * WAVE + lane];
+  const float most = fmaxf(m, om);
+  const float mine = __builtin_amdgcn_exp2f(m - most), its = __builtin_amdgcn_exp2f(om - most);
+  f32x4 mo[N];
+#pragma unroll
+  for (int d = 0; d < N; ++d) {
+    const f32x4 v = ro[((wid ^ 1) * N + d) * WAVE + lane];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      mo[d][r] = (wid ? o[N + d][r] : o[d][r]) * mine + v[r] * its;
+  }
+  finish_slice<D, STEP>(a, mo, most, l * mine + ol * its, row0, G, wid, l16, lg,
+                        STEP ? max(1, (S - lo + per - 1) / max(per, 1)) : a.nsplit);
 }
 
 // One block per query head: weighs the slices (an empty one has sum zero) and
@@ -795,13 +1024,26 @@ extern "C" int attn_decode_tile(int G, int Dk, int Dv, bool inrow) {
 template <int DK, int DV, int KT, bool INROW>
 static void attn_decode_tile_go(const DecodeArgs& a, int B, hipStream_t stream) {
   const dim3 grid((unsigned)(B * a.Hkv), (unsigned)a.nsplit), block(AD_BLOCK);
-  if constexpr (DK == DV && !INROW) {
-    if (a.tickets) {
+  if constexpr (DK <= 128) {
+    // a wave's tiles: 32 KB
+    constexpr int NB = 256 / DK, smem = DW_WAVES * NB * 2 * 32 * DK * 2;
+    const dim3 two(DW_WAVES * WAVE);
+    auto go = [&](auto kernel) {
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+      kernel<<<grid, two, smem, stream>>>(a);
+    };
+    if (a.tickets) go(&attn_decode_wave_kernel<DK, NB, true>);
+    else go(&attn_decode_wave_kernel<DK, NB, false>);
+  } else if constexpr (DK == DV && !INROW) {
+    if (a.tickets)
       attn_decode_tile_kernel<DK, DV, KT, INROW, true><<<grid, block, 0, stream>>>(a);
-      return;
-    }
+    else
+      attn_decode_tile_kernel<DK, DV, KT, INROW, false><<<grid, block, 0, stream>>>(a);
+  } else {
+    attn_decode_tile_kernel<DK, DV, KT, INROW, false><<<grid, block, 0, stream>>>(a);
   }
-  attn_decode_tile_kernel<DK, DV, KT, INROW, false><<<grid, block, 0, stream>>>(a);
+  if (a.tickets) return;
   if (a.nsplit > 1 && a.out)
     attn_decode_merge_kernel<<<dim3((unsigned)(B * a.Hq)), dim3(128), 0,
                                stream>>>(a.part_o, a.part_ml, (short*)a.out,
