@@ -404,8 +404,8 @@ struct DecodeArgs {
 };
 
 // Keys and values are read once: as a stream (2) they leave the L2 to what is read again
-// (the sizes below: 64 x 2049 keys 109 -> 101 us, 5 x 5004 of 256 46.5 -> 45.5; latents
-// 16.4 -> 16.8, and stay as they were).
+// (64 x 2049 keys 109 -> 101 us, 5 x 5004 of 256 46.5 -> 45.5; latents 16.4 -> 16.8, and
+// stay as they were).
 template <bool STREAM>
 __device__ __forceinline__ void dt_to_lds(const char* src, char* dst) {
   __builtin_amdgcn_global_load_lds(
@@ -557,13 +557,7 @@ __device__ __forceinline__ void finish_slice(const DecodeArgs& a, const f32x4 (&
   }
 }
 
-// STEP: queries and the token's key are turned here, its key and value go to the cache
-// and into the last tile, and the last block of a head merges the slices.  The chain
-// through memory to that block takes what the merging kernel took (5 us), the rotations
-// 2 to 3 instead of 4.6 in a kernel of their own: one sequence of 1024 keys, 32 heads of
-// 128 over 8, 14.1 -> 9.6 us for the three; 5 of 5004, 16 of 256 over 8, 51 -> 50; 64
-// of 2049 as before (one slice, 109).
-template <int DK, int DV, int KT, bool INROW, bool STEP>
+template <int DK, int DV, int KT, bool INROW>
 __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
     const DecodeArgs a) {
   constexpr int KP = DK / 8, VP = INROW ? KP : DV / 8;  // pieces of a row
@@ -572,7 +566,6 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
   constexpr int HALVES = 64 / KT;
   static_assert(KT == 64 || KT == 32, "four waves make the scores of a tile");
   static_assert(NK % HALVES == 0 && KB % 4096 == 0 && VB % 4096 == 0, "sizes");
-  static_assert(!STEP || (DK == DV && !INROW && (DK & (DK - 1)) == 0), "step");
   __shared__ __attribute__((aligned(16))) char smem[2 * (KB + VB)];
   __shared__ float sc[2][HALVES][KT][16];
 
@@ -587,7 +580,6 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
   const int per = ((S - lo + a.nsplit - 1) / a.nsplit + KT - 1) / KT * KT;
   const int from = min(S, lo + per * (int)blockIdx.y);
   const int to = min(S, from + per);
-  if (STEP && from >= to && from > lo) return;  // nothing of the keys, nor of the count
 
   const char* kbase = a.k + (long)blockIdx.x * a.cap * (DK * 2);
   const char* vbase = a.v + (long)blockIdx.x * a.cap * (DV * 2);
@@ -616,34 +608,12 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
   const long row0 = (long)b * a.Hq + hk * G;  // first query head
   const int kb = KT == 64 ? wid : wid & 1, half = KT == 64 ? 0 : wid >> 1;
   bf16x8_t qf[NK / HALVES];
-  if constexpr (STEP) {
-    const char* head = a.q + ((long)b * a.qs + (hk * G + min(l16, G - 1)) * DK) * 2;
-#pragma unroll
-    for (int i = 0; i < NK / HALVES; ++i)
-      qf[i] = turned<DK>(head, (half * (NK / HALVES) + i) * 32 + lg * 8, a);
-  } else {
+  {
     const char* src = a.q + (row0 + min(l16, G - 1)) * (DK * 2) +
                       half * (NK / HALVES) * 64 + lg * 16;
 #pragma unroll
     for (int i = 0; i < NK / HALVES; ++i)
       qf[i] = *reinterpret_cast<const bf16x8_t*>(src + i * 64);
-  }
-  // the token itself, at S - 1; it has no place where the cache is full
-  const bool newest = STEP && from < to && to == S && (!a.s_ptr || *a.s_ptr < a.cap);
-  constexpr int PIECES = DK / 8;
-  const int own = threadIdx.x % PIECES;  // piece of its rows
-  bf16x8_t fresh_k, fresh_v;
-  if (newest) {
-    const long at = (long)blockIdx.x * a.cap + S - 1;
-    fresh_v = *reinterpret_cast<const bf16x8_t*>(
-        a.vnew + ((long)b * a.vs + hk * DV + own * 8) * 2);
-    if (threadIdx.x < PIECES) {
-      fresh_k = turned<DK>(a.knew + ((long)b * a.ks + hk * DK) * 2, own * 8, a);
-      *reinterpret_cast<bf16x8_t*>(const_cast<char*>(a.k) + (at * DK + own * 8) * 2) =
-          fresh_k;
-      *reinterpret_cast<bf16x8_t*>(const_cast<char*>(a.v) + (at * DV + own * 8) * 2) =
-          fresh_v;
-    }
   }
   float m = -1e30f, l = 0.0f;  // reference of the exponents (base 2), sum
   f32x4 o[ND];
@@ -657,19 +627,6 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
     if (t + KT < to) stage(t + KT, buf ^ 1);
     const char* kt = smem + buf * (KB + VB);
     const char* vt = kt + KB;
-    if (newest && t + KT >= to) {
-      // what came from the token's place in the cache is not there yet, in its row and
-      // in those behind, which repeat it
-      const int row = S - 1 - t;
-      if (threadIdx.x < PIECES)
-        *reinterpret_cast<bf16x8_t*>(const_cast<char*>(kt) + row * KP * 16 +
-                                     dt_place<KP, true>(row, own) * 16) = fresh_k;
-      for (int r = row + threadIdx.x / PIECES; r < KT; r += AD_BLOCK / PIECES)
-        *reinterpret_cast<bf16x8_t*>(const_cast<char*>(vt) + r * VP * 16 +
-                                     dt_place<VP, INROW>(r, own) * 16) = fresh_v;
-      __syncthreads();
-    }
-
     f32x4 s4 = {0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < NK / HALVES; ++i) {
@@ -756,16 +713,22 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
 
   l += __shfl_xor(l, 16, WAVE);
   l += __shfl_xor(l, 32, WAVE);
-  finish_slice<DV, STEP>(a, o, m, l, row0, G, wid, l16, lg,
-                         STEP ? max(1, (S - lo + per - 1) / max(per, 1)) : a.nsplit);
+  finish_slice<DV, false>(a, o, m, l, row0, G, wid, l16, lg, a.nsplit);
 }
 
-// Heads of 64 and 128.  A wave has tiles of 32 keys of its own, which go to its own LDS,
+// Heads of 64, 128 and 256.  A wave has tiles of 32 keys of its own, which go to its own LDS,
 // NB of them by turns, and keeps outputs of all columns: scores come out of the first
 // product as the second one takes them, so that waves meet at the end of a slice only, and
 // each makes its own keys' weights.  In the kernel above a tile's scores pass two barriers
 // and all waves make all weights, a chain of 2 us beside loads of 3.  64 sequences of 2049
-// keys, 32 heads of 128 over 8: 101 us there, 92 here (5.8 TB/s); one of 1024: 9.6, 9.8.
+// keys, 32 heads of 128 over 8: 101 us there, 92 here (5.8 TB/s); one of 1024: 9.6, 9.8; 5 of
+// 5004, 16 of 256 over 8: 45.5, 43.5 (a CU has two waves of those; refills of a tile's
+// keys ahead of its values gain nothing).
+// STEP: queries and the token's key are turned here, its key and value go to the cache
+// and into the last tile, and the last block of a head merges the slices.  The chain
+// through memory to that block takes what the merging kernel took (5 us), the rotations
+// 2 to 3 instead of 4.6 in a kernel of their own: one sequence of 1024 keys, 32 heads of
+// 128 over 8, 14.1 -> 9.6 us for the three.
 #define DW_WAVES 2
 template <int D, int NB, bool STEP>
 __global__ __launch_bounds__(DW_WAVES* WAVE) void attn_decode_wave_kernel(
@@ -1011,7 +974,7 @@ __global__ __launch_bounds__(128) void attn_decode_merge_kernel(
 // head sizes (keys, values), keys of a tile, values within the keys' rows
 #define DT_SIZES(DO)                                                         \
   DO(64, 64, 64, false) DO(128, 128, 64, false) DO(192, 128, 32, false)      \
-  DO(256, 256, 32, false) DO(576, 512, 32, true)
+  DO(256, 256, 64, false) DO(576, 512, 32, true)
 
 extern "C" int attn_decode_tile(int G, int Dk, int Dv, bool inrow) {
   if (G > 16) return 0;
@@ -1024,9 +987,9 @@ extern "C" int attn_decode_tile(int G, int Dk, int Dv, bool inrow) {
 template <int DK, int DV, int KT, bool INROW>
 static void attn_decode_tile_go(const DecodeArgs& a, int B, hipStream_t stream) {
   const dim3 grid((unsigned)(B * a.Hkv), (unsigned)a.nsplit), block(AD_BLOCK);
-  if constexpr (DK <= 128) {
-    // a wave's tiles: 32 KB
-    constexpr int NB = 256 / DK, smem = DW_WAVES * NB * 2 * 32 * DK * 2;
+  if constexpr (DK == DV) {
+    // a wave's tiles: 32 KB, of heads of 256 twice that
+    constexpr int NB = DK < 256 ? 256 / DK : 2, smem = DW_WAVES * NB * 2 * 32 * DK * 2;
     const dim3 two(DW_WAVES * WAVE);
     auto go = [&](auto kernel) {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -1035,13 +998,8 @@ static void attn_decode_tile_go(const DecodeArgs& a, int B, hipStream_t stream) 
     };
     if (a.tickets) go(&attn_decode_wave_kernel<DK, NB, true>);
     else go(&attn_decode_wave_kernel<DK, NB, false>);
-  } else if constexpr (DK == DV && !INROW) {
-    if (a.tickets)
-      attn_decode_tile_kernel<DK, DV, KT, INROW, true><<<grid, block, 0, stream>>>(a);
-    else
-      attn_decode_tile_kernel<DK, DV, KT, INROW, false><<<grid, block, 0, stream>>>(a);
   } else {
-    attn_decode_tile_kernel<DK, DV, KT, INROW, false><<<grid, block, 0, stream>>>(a);
+    attn_decode_tile_kernel<DK, DV, KT, INROW><<<grid, block, 0, stream>>>(a);
   }
   if (a.tickets) return;
   if (a.nsplit > 1 && a.out)

@@ -436,10 +436,10 @@ void mla_append_kv(torch::Tensor kvh, torch::Tensor kpe, torch::Tensor kcache,
 // all at work at once, and no slice under one tile.  256 blocks leave half of the
 // loads in flight unused (5 sequences of 5004 keys, 8 heads of 256: 68 us, 45 with
 // 512), 1024 come in two rounds and double what the merge reads (48 us; 64 cached
-// latents of 2048 tokens: 49 us, 40 with 512).
-static int decode_slices(long pairs, long span, int tile) {
+// latents of 2048 tokens: 49 us, 40 with 512).  Of heads of 256 a CU has one block.
+static int decode_slices(long pairs, long span, int tile, int blocks = 512) {
   return (int)std::max<long>(
-      1, std::min<long>({64, 512 / std::max<long>(pairs, 1),
+      1, std::min<long>({64, blocks / std::max<long>(pairs, 1),
                          (span + tile - 1) / tile}));
 }
 
@@ -483,7 +483,8 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                        ? attn_decode_tile(Hq / Hkv, Dk, Dv, inrow)
                        : 0;
   if (tile) {
-    const int nsplit = decode_slices((long)B * Hkv, s_ptr ? kScap : (long)S, tile);
+    const int nsplit = decode_slices((long)B * Hkv, s_ptr ? kScap : (long)S, tile,
+                                     Dk == 256 ? 256 : 512);
     torch::Tensor po, pml;
     if (nsplit > 1) {
       po = torch::empty({(long)B * Hq * nsplit * Dv}, fopts);
@@ -567,7 +568,8 @@ c10::optional<torch::Tensor> attn_step(
     TORCH_CHECK(pos0 >= 0 && pos0 < cap, "no room in the cache");
   }
   const int tile = attn_decode_tile((int)(Hq / Hkv), (int)D, (int)D, false);
-  const int nsplit = decode_slices(B * Hkv, s_ptr ? cap : pos0 + 1, tile);
+  const int nsplit = decode_slices(B * Hkv, s_ptr ? cap : pos0 + 1, tile,
+                                   D == 256 ? 256 : 512);
   auto out = torch::empty({B, 1, Hq * D}, q.options());
   torch::Tensor part;
   if (nsplit > 1)
