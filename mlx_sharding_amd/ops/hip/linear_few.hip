@@ -283,15 +283,19 @@ static void linear_few_go(LinearFewArgs a, int split, hipStream_t stream) {
 // is made in every block: one of x, 128256 rows of 4096 202 us so, 181 with four, of
 // 32000 rows of 3584 51 and 44).  A unit needs
 // both its halves; four from 16384 rows on (28672 rows, 16 of x, norm: 50 us, 53
-// with two; 12800, one of x: 14.0 with two, 15.8).  One tile takes two steps at a time:
-// 4096 rows of 4096 8.3 us, of 14336 22.2, with four 9.2 and 23.3.
+// with two; 12800, one of x: 14.0 with two, 15.8), but two for short contractions into
+// less than 24576, where blocks of four come in little more than one round (one of x, K
+// 2048: 16384 rows 14.8 us, 14.1 with two, 21888 24.1, 20.6, 28672 24.1, 24.6).  One
+// tile takes two steps at a time: 4096 rows of 4096 8.3 us, of 14336 22.2, with four 9.2
+// and 23.3.
 static void linear_few_tiles(const LinearFewArgs& a, int act, int split,
                              hipStream_t stream) {
+  const bool four = a.O >= 8192 && !(a.K <= 2048 && a.O < 12288);
   if (act == LF_SILU) {
-    if (a.O >= 8192) linear_few_go<4, LF_SILU, 4, 2>(a, 1, stream);
+    if (four) linear_few_go<4, LF_SILU, 4, 2>(a, 1, stream);
     else linear_few_go<2, LF_SILU, 8, 4>(a, 1, stream);
   } else if (act == LF_GELU) {
-    if (a.O >= 8192) linear_few_go<4, LF_GELU, 4, 2>(a, 1, stream);
+    if (four) linear_few_go<4, LF_GELU, 4, 2>(a, 1, stream);
     else linear_few_go<2, LF_GELU, 8, 4>(a, 1, stream);
   } else if (a.O <= 4096) {
     linear_few_go<1, LF_PLAIN, 8, 2>(a, split, stream);
