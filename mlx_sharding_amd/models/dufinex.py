@@ -115,9 +115,7 @@ class DufinexStageModel(RaggedStageModel):
             layer_outputs: Optional[list] = None) -> torch.Tensor:
         W = self.config.hidden_size
         dtype = next(self.parameters()).dtype
-        x = self.residual(x)
-        if self.shard.is_first:
-            x.mul_(float(self.config["embedding"]["scale"]))
+        x = self.residual(x, float(self.config["embedding"]["scale"]))
         items = self.layer_items()
         first = self.shard.start_layer
 

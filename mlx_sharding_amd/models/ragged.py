@@ -14,12 +14,11 @@ from typing import Dict, List, Optional, Tuple
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.paged import PagedState, RaggedBatch, RaggedCache, RaggedLayerCache
-from ..ops.ragged import Rotary
+from ..ops.ragged import Rotary, token_rows
 from .base import Linear, RMSNorm, StageModel, owned_layer_indices
 
 
@@ -159,11 +158,11 @@ class RaggedStageModel(StageModel):
             got = self._tables[rotary] = rotary.tables(rows, device)
         return got
 
-    def residual(self, x: torch.Tensor) -> torch.Tensor:
-        """What the first owned layer adds to: embedded token ids, or a copy
-        of the residual stream that the previous stage handed on."""
+    def residual(self, x: torch.Tensor, scale: float = 1.0) -> torch.Tensor:
+        """What the first owned layer adds to: embedded token ids times ``scale``,
+        or a copy of the residual stream that the previous stage handed on."""
         if self.shard.is_first:
-            return F.embedding(x, self.embed.weight).float()
+            return token_rows(x, self.embed.weight, scale)
         return x[:, : self.config.hidden_size].float().contiguous().clone()
 
     def logits(self, h: torch.Tensor) -> torch.Tensor:

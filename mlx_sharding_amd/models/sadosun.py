@@ -130,7 +130,7 @@ class SadosunStageModel(RaggedStageModel):
         dtype = next(self.parameters()).dtype
         if self.shard.is_first:
             side = F.embedding(x, self.side.embed.weight)
-            x = self.residual(x).mul_(float(self.config["embedding"]["scale"]))
+            x = self.residual(x, float(self.config["embedding"]["scale"]))
         else:
             side = x[:, W:].to(dtype)
             x = self.residual(x)

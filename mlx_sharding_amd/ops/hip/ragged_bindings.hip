@@ -19,6 +19,8 @@ struct AddNormArgs {
 };
 
 extern "C" {
+void launch_token_rows(const long*, const void*, float*, long, long, int, float,
+                       hipStream_t);
 void launch_clamped_glu(const void*, const void*, const void*, const void*,
                         void*, long, int, long, long, float, float, bool, bool,
                         hipStream_t);
@@ -813,6 +815,26 @@ Tensor cap_logits(Tensor z, double scale, double limit) {
   return o;
 }
 
+// tokens [...] of a bf16 table [vocab, W], times scale, in fp32
+Tensor token_rows(Tensor tokens, Tensor table, double scale) {
+  TORCH_CHECK(tokens.is_cuda() && tokens.scalar_type() == torch::kInt64 &&
+              tokens.is_contiguous(), "tokens int64");
+  TORCH_CHECK(table.device() == tokens.device() &&
+              table.scalar_type() == torch::kBFloat16 && table.dim() == 2 &&
+              table.is_contiguous() && table.size(0) >= 1 && table.size(1) >= 8 &&
+              table.size(1) % 8 == 0, "table");
+  aligned16(table, "table");
+  const long W = table.size(1);
+  TORCH_CHECK(tokens.numel() * (W / 8) < (1L << 32), "sizes");
+  auto sizes = tokens.sizes().vec();
+  sizes.push_back(W);
+  auto out = torch::empty(sizes, table.options().dtype(torch::kFloat32));
+  if (tokens.numel())
+    launch_token_rows(tokens.data_ptr<int64_t>(), table.data_ptr(), out.data_ptr<float>(),
+                      tokens.numel(), table.size(0), (int)W, (float)scale, stream());
+  return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -824,6 +846,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("clamped_glu", &clamped_glu, py::arg("gate"), py::arg("up"),
         py::arg("limit"), py::arg("alpha"), py::arg("gate_bias") = py::none(),
         py::arg("up_bias") = py::none());
+  m.def("token_rows", &token_rows);
   m.def("add_norm", &add_norm, py::arg("x"), py::arg("y"), py::arg("w_post"),
         py::arg("w_next"), py::arg("f32"), py::arg("eps"), py::arg("offset"),
         py::arg("mult"), py::arg("where"), py::arg("wide"),

@@ -55,6 +55,19 @@ def _ext(op: str):
     return ext
 
 
+def token_rows(tokens, table, scale: float = 1.0):
+    """Rows of a table for tokens, in fp32 and times ``scale``."""
+    from . import plain
+    ext = hip_ragged() if tokens.is_cuda else None
+    if (ext is not None and tokens.dtype == torch.int64 and tokens.is_contiguous()
+            and table.device == tokens.device and table.dtype == torch.bfloat16
+            and table.is_contiguous() and table.shape[1] % 8 == 0
+            and table.data_ptr() % 16 == 0 and plain(tokens) and plain(table)):
+        return ext.token_rows(tokens, table, scale)
+    rows = F.embedding(tokens, table).float()
+    return rows if scale == 1.0 else rows.mul_(scale)
+
+
 def _pad(n: int, to: int) -> int:
     return (n + to - 1) // to * to
 

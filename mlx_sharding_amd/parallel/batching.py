@@ -94,9 +94,12 @@ class BatchEngine:
                                 for r, h in zip(rids, held)))
         ids = [t for j in batch.order for t in portions[j].tokens]
         start = {batch.order[e]: batch.host[e][0] for e in range(len(portions))}
-        ids += [start[j] + int(w) for j, p in enumerate(portions) for w in p.want]
+        wanted = [start[j] + int(w) for j, p in enumerate(portions) for w in p.want]
+        ids += wanted
         x, rows = upload(np.array(ids, dtype=np.int64), self.device).split(
             [batch.n_tokens, len(ids) - batch.n_tokens])
+        if wanted == list(range(batch.n_tokens)):
+            rows = None  # all of them, as they are
         logits = self.model.run(x, batch, state, rows=rows)
         for p, h in zip(portions, held):
             h.length += len(p.tokens)
