@@ -23,28 +23,45 @@
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// Two lines of 64 bytes, which a block asks for at once: numbers of a third line, or of the
+// second when the first had come, took every launch 0.4 us.
 struct LinearFewArgs {
   const __bf16 *x, *w, *bias, *res, *norm;
   __bf16* y;
-  int M, O, K;             // O: columns of y
+  short M;
+  // parts > 1: blocks share a tile's contraction, `share` steps (few) or stages
+  // (some) each.  part [tiles of y, parts, tiles of x, WAVE, 4], count: one number per
+  // tile of y and x, zero before.
+  unsigned char parts;
+  unsigned char fours;     // bias and residual are read by fours
+  int O, K;                // O: columns of y
+  int share;
   long ldx, ldw, ldr, ldy;
-  float eps, offset;       // norm weights are norm + offset
-  // gridDim.y > 1: blocks share a tile's contraction, `share` steps (few) or stages
-  // (some) each.  part [tiles of y, gridDim.y,
-  // tiles of x, WAVE, 4], count: one number per tile of y and x, zero before.
-  float* part;
-  unsigned* count;
-  unsigned* zero;          // n_zero numbers that this launch clears for a later one
-  int n_zero, share;
+  union {
+    struct { float eps, offset; };  // norm weights are norm + offset
+    float* part;                    // without a norm
+  };
+  unsigned turn;           // 2^32 / chunks of a share, rounded up, for first_of
+  int n_zero;              // numbers at zero that this launch clears for a later one
+  unsigned *count, *zero;
 };
+static_assert(sizeof(LinearFewArgs) == 128, "two lines");
+
+// all of a, now
+__device__ __forceinline__ void arrive(const LinearFewArgs& a) {
+  asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.bias), "s"(a.res), "s"(a.norm), "s"(a.O),
+               "s"(a.K), "s"(a.share), "s"(a.ldx), "s"(a.ldw), "s"(a.turn), "s"(a.zero));
+}
 
 // Where a block begins in the n chunks of a contraction; it goes round from there.
 // Rows of W and of x lie powers of two apart as a rule, and blocks in step at one column
 // ask few of the memory's channels: 16384 rows of 2048, 12 of x, 16.4 us from column 0 on,
 // 14.1 so (the blocks of an XCD, which are every eighth, three chunks apart; one apart
 // 14.2, seven 14.5); 28672 of 4096 with norm and unit 45.6, 43.5; 6144 of 4096 14.7, 13.2.
-__device__ __forceinline__ int first_of(int n) {
-  return (blockIdx.x >> 3) * 3 % (unsigned)max(n, 1);
+// `turn` divides by the chunks of a whole share: the last may have less.
+__device__ __forceinline__ int first_of(const LinearFewArgs& a, int whole, int n) {
+  const unsigned at = (blockIdx.x >> 3) * 3;
+  return max(min((int)(at - __umulhi(at, a.turn) * whole), n - 1), 0);
 }
 
 // The sums of a tile that blocks share: leaves this one's, and true in the one that
@@ -54,7 +71,7 @@ __device__ __forceinline__ bool sums_of_all(const LinearFewArgs& a, long tile,
                                             int lane, f32x4& v) {
   typedef unsigned long long u64;
   typedef u64 u64x2 __attribute__((ext_vector_type(2)));
-  u64* to = reinterpret_cast<u64*>(a.part) + (tile * gridDim.y * WAVE + lane) * 2;
+  u64* to = reinterpret_cast<u64*>(a.part) + (tile * a.parts * WAVE + lane) * 2;
   const u64x2 own = __builtin_bit_cast(u64x2, v);
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -66,11 +83,11 @@ __device__ __forceinline__ bool sums_of_all(const LinearFewArgs& a, long tile,
     before = __hip_atomic_fetch_add(a.count + tile, 1u, __ATOMIC_RELAXED,
                                     __HIP_MEMORY_SCOPE_AGENT);
   before = __builtin_amdgcn_readfirstlane(before);
-  if (before + 1 != gridDim.y) return false;
+  if (before + 1 != a.parts) return false;
   asm volatile("" ::: "memory");
   v = f32x4{0, 0, 0, 0};
 #pragma unroll 4
-  for (unsigned s = 0; s < gridDim.y; ++s) {
+  for (unsigned s = 0; s < a.parts; ++s) {
     u64x2 p;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -85,10 +102,32 @@ __device__ __forceinline__ bool sums_of_all(const LinearFewArgs& a, long tile,
 
 enum { LF_PLAIN = 0, LF_SILU = 1, LF_GELU = 2 };
 
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+
+// What is added to four columns of y, if it may be read by fours.  Asked for before the
+// contraction: behind it, the residual's were four reads one after the other (us without
+// and with a residual; one of x, 2048 rows of 2048 5.4 and 5.6, so 5.1 both; 12 of x, 4096
+// of 4096 9.4 and 9.9, so 9.2 both; 64 of x 13.8 and 14.4, so 13.5 and 13.9).
+template <int ACT>
+struct Ends {
+  bf16x4_t res, bias[ACT ? 2 : 1];
+
+  __device__ __forceinline__ void read(const LinearFewArgs& a, int row, int col) {
+    col = min(col, a.O - 4);
+    if (a.res)
+      res = *reinterpret_cast<const bf16x4_t*>(a.res + min(row, a.M - 1) * a.ldr + col);
+    if (a.bias) {
+#pragma unroll
+      for (int h = 0; h < (ACT ? 2 : 1); ++h)
+        bias[h] = *reinterpret_cast<const bf16x4_t*>(a.bias + h * a.O + col);
+    }
+  }
+};
+
 // sums of four columns of y from `col` on, and of an up projection's, to memory
 template <int ACT>
-__device__ __forceinline__ void finish_columns(const LinearFewArgs& a, int row,
-                                               int col, const f32x4* v) {
+__device__ __forceinline__ void finish_columns(const LinearFewArgs& a, int row, int col,
+                                               const f32x4* v, const Ends<ACT>& e) {
   float o[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -97,8 +136,8 @@ __device__ __forceinline__ void finish_columns(const LinearFewArgs& a, int row,
     if (ACT) {
       float up = v[1][j];
       if (a.bias) {
-        f += (float)a.bias[at];
-        up += (float)a.bias[a.O + at];
+        f += (float)(a.fours ? e.bias[0][j] : a.bias[at]);
+        up += (float)(a.fours ? e.bias[ACT ? 1 : 0][j] : a.bias[a.O + at]);
       }
       if (ACT == LF_SILU) {
         f = f / (1.0f + __expf(-f)) * up;
@@ -107,14 +146,13 @@ __device__ __forceinline__ void finish_columns(const LinearFewArgs& a, int row,
         f = 0.5f * f * (1.0f + tanhf(z)) * up;
       }
     } else if (a.bias) {
-      f += (float)a.bias[at];
+      f += (float)(a.fours ? e.bias[0][j] : a.bias[at]);
     }
-    if (a.res) f += (float)a.res[(long)row * a.ldr + at];
+    if (a.res) f += (float)(a.fours ? e.res[j] : a.res[(long)row * a.ldr + at]);
     o[j] = f;
   }
   __bf16* y = a.y + (long)row * a.ldy + col;
   if (col + 3 < a.O && a.ldy % 4 == 0) {
-    typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
     *reinterpret_cast<bf16x4_t*>(y) =
         bf16x4_t{(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
   } else {
@@ -132,6 +170,7 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
   __shared__ __attribute__((aligned(16))) f32x4 red[NW][RT][WAVE];
   __shared__ float squares[NORM ? NW : 1][WAVE];
 
+  arrive(a);
   const int lane = threadIdx.x & (WAVE - 1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l16 = lane & 15, lg = lane >> 4;
@@ -165,7 +204,7 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
 
   // this block's share of the contraction
   const int s0 = blockIdx.y * a.share, steps = min(a.share, a.K / 32 - s0);
-  const int chunks = steps / U, first = first_of(chunks);
+  const int chunks = steps / U, first = first_of(a, a.share / U, chunks);
   // operands of one chunk; the next one's are asked for before this one is used,
   // rows of x among them, as loads come back in order
   struct Chunk {
@@ -199,13 +238,31 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
                                                          0, 0, 0);
     }
   };
+  static_assert(YT <= NW, "a tile of y for a wave");
+  Ends<ACT> ends;
   Chunk one, two;
   if (wid < chunks) fetch(one, wid);
-  for (int c = wid; c < chunks; c += 2 * NW) {
-    if (c + NW < chunks) fetch(two, c + NW);
+  if (a.fours && wid < YT) ends.read(a, l16, row0 + wid * 16 + lg * 4);
+  // fetches under a condition would have their users wait for all that is under way (one
+  // of x, 4096 rows of 14336 24.3 us so, 23.7 as it is; 32000 of 2048 with norm 27.0, 26.0)
+  int c = wid;
+  for (; c + 2 * NW < chunks; c += 2 * NW) {
+    fetch(two, c + NW);
+    __builtin_amdgcn_sched_barrier(0);
     use(one);
-    if (c + 2 * NW < chunks) fetch(one, c + 2 * NW);
-    if (c + NW < chunks) use(two);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(one, c + 2 * NW);
+    __builtin_amdgcn_sched_barrier(0);
+    use(two);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (c + NW < chunks) {
+    fetch(two, c + NW);
+    __builtin_amdgcn_sched_barrier(0);
+    use(one);
+    use(two);
+  } else if (c < chunks) {
+    use(one);
   }
   // steps that make no whole chunk
   for (int s = s0 + chunks * U + wid; s < s0 + steps; s += NW) {
@@ -226,7 +283,8 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
   if (a.zero && blockIdx.x == 0)
     for (int i = threadIdx.x; i < a.n_zero; i += NW * WAVE) a.zero[i] = 0;
   // a wave per tile of y: four columns of a row a lane
-  for (int r = wid; r < YT; r += NW) {
+  if (wid < YT) {
+    const int r = wid;
     f32x4 v[ACT ? 2 : 1];
 #pragma unroll
     for (int h = 0; h < (ACT ? 2 : 1); ++h) {
@@ -250,25 +308,30 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[h][j] *= f;
     }
-    if (!ACT && !NORM && gridDim.y > 1 &&
+    if (!ACT && !NORM && a.parts > 1 &&
         !sums_of_all(a, (long)blockIdx.x * YT + r, lane, v[0]))
-      continue;
-    if (l16 < a.M) finish_columns<ACT>(a, l16, row0 + r * 16 + lg * 4, v);
+      return;
+    if (l16 < a.M) finish_columns<ACT>(a, l16, row0 + r * 16 + lg * 4, v, ends);
   }
 }
 
 // Blocks that share a tile's contraction, as many as have something of it.
-static dim3 shared_grid(LinearFewArgs& a, int cols, int steps, int split) {
+// per: steps or stages of a chunk
+static dim3 shared_grid(LinearFewArgs& a, int cols, int steps, int per, int split) {
   a.share = (steps + split - 1) / split;
-  return dim3((unsigned)((a.O + cols - 1) / cols),
-              (unsigned)((steps + a.share - 1) / a.share));
+  const int parts = (steps + a.share - 1) / a.share;
+  a.parts = (unsigned char)parts;
+  const int chunks = a.share / per;
+  a.turn = chunks > 1 ? (unsigned)(((1ull << 32) + chunks - 1) / chunks) : 0;
+  return dim3((unsigned)((a.O + cols - 1) / cols), (unsigned)parts);
 }
 
 template <int RT, int ACT, int NW, int U>
 static void linear_few_go(LinearFewArgs a, int split, hipStream_t stream) {
   constexpr int cols = 16 * (ACT ? RT / 2 : RT);
-  const dim3 grid = shared_grid(a, cols, a.K / 32, split), block(NW * WAVE);
   // the norm's weights and sums need registers: shorter chunks
+  const dim3 grid = shared_grid(a, cols, a.K / 32, a.norm ? 2 : U, split);
+  const dim3 block(NW * WAVE);
   if (a.norm) {
     linear_few_kernel<RT, ACT, true, NW, 2><<<grid, block, 0, stream>>>(a);
   } else {
@@ -361,7 +424,7 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
   // this block's share of the contraction
   const int s0 = blockIdx.y * a.share;
   const int stages = min(a.share, (a.K + KS * 32 - 1) / (KS * 32) - s0);
-  const int first = first_of(stages);
+  const int first = first_of(a, a.share, stages);
   auto turned = [&](int t) {
     t = min(t, stages - 1) + first;
     return s0 + (t >= stages ? t - stages : t);
@@ -417,6 +480,14 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
   };
 #pragma unroll
   for (int t = 0; t < RING - 1; ++t) issue(t, t);
+  // younger than what the first stages wait for: they wait for no less
+  constexpr int TILES = (YT * TT + LS_WAVES - 1) / LS_WAVES;  // of y and x, of a wave
+  Ends<ACT> ends[TILES];
+#pragma unroll
+  for (int q = 0; q < TILES; ++q) {
+    const int n = min(wid + q * LS_WAVES, YT * TT - 1);
+    if (a.fours) ends[q].read(a, n % TT * 16 + l16, row0 + n / TT * 16 + lg * 4);
+  }
   int t0 = 0;
   for (; t0 + RING <= stages; t0 += RING) {
 #pragma unroll
@@ -453,8 +524,10 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
 
   if (a.zero && blockIdx.x == 0)
     for (int i = threadIdx.x; i < a.n_zero; i += LS_WAVES * WAVE) a.zero[i] = 0;
-  for (int n = wid; n < YT * TT; n += LS_WAVES) {
-    const int r = n / TT, i = n % TT;
+#pragma unroll
+  for (int q = 0; q < TILES; ++q) {
+    const int n = wid + q * LS_WAVES, r = n / TT, i = n % TT;
+    if (n >= YT * TT) break;
     f32x4 v[ACT ? 2 : 1];
 #pragma unroll
     for (int h = 0; h < (ACT ? 2 : 1); ++h) {
@@ -478,11 +551,11 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[h][j] *= f;
     }
-    if (!ACT && !NORM && gridDim.y > 1 &&
+    if (!ACT && !NORM && a.parts > 1 &&
         !sums_of_all(a, ((long)blockIdx.x * YT + r) * TT + i, lane, v[0]))
       continue;
     if (i * 16 + l16 < a.M)
-      finish_columns<ACT>(a, i * 16 + l16, row0 + r * 16 + lg * 4, v);
+      finish_columns<ACT>(a, i * 16 + l16, row0 + r * 16 + lg * 4, v, ends[q]);
   }
 }
 
@@ -497,7 +570,7 @@ static void linear_some_go(LinearFewArgs a, int split, hipStream_t stream) {
     (void)hipFuncSetAttribute(
         reinterpret_cast<const void*>(&linear_some_kernel<RT, TT, KS, ACT, NORM>),
         hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-  const dim3 grid = shared_grid(a, cols, (a.K + KS * 32 - 1) / (KS * 32), split);
+  const dim3 grid = shared_grid(a, cols, (a.K + KS * 32 - 1) / (KS * 32), 1, split);
   linear_some_kernel<RT, TT, KS, ACT, NORM>
       <<<grid, dim3(LS_WAVES * WAVE), smem, stream>>>(a);
 }
@@ -546,7 +619,8 @@ static void linear_some(const LinearFewArgs& a, int act, int split, hipStream_t 
 // Whether rows of x go through LDS: above 16, and above 8 where a block would read them
 // for many columns or from many blocks (12 of x; registers, LDS: 4096 rows of 4096 9.5,
 // 9.2 us; of 14336 26, 23.8; 2048 of 8192 15.7, 12.5; 8192 of 3584 15, 13.0; 2048 of
-// 2048 6.2, 6.4; 3648 of 2048 with norm 7.3, 8.3).  With norms or units few rows, too,
+// 2048 6.2, 6.4; 8192 of 512 4.6, 5.2; 6144 of 1536 7.1, 7.3; 3648 of 2048 with norm 7.3,
+// 8.3).  With norms or units few rows, too,
 // where a block has four tiles of W's rows (one of x; 16032 of 4096 with norm 30.8, 25.2
 // us; 12800 of 2048 15.9, 13.4; units of 12288 of 4096 27.8, 23.8).  Not where there are
 // blocks for all CUs and the contraction is short (12 of x; units of 16384 of 2048 14.6,
@@ -558,7 +632,7 @@ static bool few_through_lds(int M, int O, int K, int act, bool norm) {
   if (M > 16) return true;
   if (rows >= 16384 && K <= 2048) return false;
   if (rows > 24576 && (!act || M <= 8)) return false;
-  if (M > 8) return rows > 4096 || K > 2048;
+  if (M > 8) return rows > 4096 ? K >= 2048 : K > 2048;
   return (act || norm) && rows > 8192;
 }
 
@@ -593,10 +667,16 @@ extern "C" void launch_linear_few(const void* x, const void* w, const void* bias
                                   long ldr, long ldy, float eps, float offset,
                                   int act, unsigned* count, float* part,
                                   unsigned* zero, int n_zero, hipStream_t stream) {
-  const LinearFewArgs a{(const __bf16*)x, (const __bf16*)w, (const __bf16*)bias,
-                        (const __bf16*)res, (const __bf16*)norm, (__bf16*)y,
-                        M, O, K, ldx, ldw, ldr, ldy, eps, offset, part, count, zero,
-                        n_zero, 0};
+  LinearFewArgs a{};
+  a.x = (const __bf16*)x, a.w = (const __bf16*)w, a.bias = (const __bf16*)bias;
+  a.res = (const __bf16*)res, a.norm = (const __bf16*)norm, a.y = (__bf16*)y;
+  a.M = (short)M, a.O = O, a.K = K;
+  a.ldx = ldx, a.ldw = ldw, a.ldr = ldr, a.ldy = ldy;
+  if (norm) a.eps = eps, a.offset = offset;
+  else a.part = part;
+  a.count = count, a.zero = zero, a.n_zero = n_zero;
+  a.fours = (bias || res) && O % 4 == 0 && (long)bias % 8 == 0 && (long)res % 8 == 0 &&
+            (!res || ldr % 4 == 0);
   const int split = count ? few_split(M, O, K, act, norm != nullptr) : 1;
   if (few_through_lds(M, O, K, act, norm != nullptr)) {
     linear_some(a, act, split, stream);

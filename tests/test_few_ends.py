@@ -1,0 +1,32 @@
+"""What few rows' products add to their columns, read by fours or alone."""
+
+import pytest
+import torch
+
+from mlx_sharding_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("act", [None, "silu"])
+@pytest.mark.parametrize("M,O,K", [(1, 4, 32), (3, 20, 96), (16, 68, 64), (5, 8196, 160),
+                                   (17, 4, 32), (33, 4100, 96), (64, 36, 2080),
+                                   (2, 70, 64), (40, 18, 64)])
+@pytest.mark.parametrize("shift,pad", [(0, 0), (1, 0), (0, 3), (4, 8)])
+def test_ends(M, O, K, act, shift, pad):
+    g = torch.Generator("cuda").manual_seed(O + M)
+
+    def rand(*n):
+        return torch.randn(*n, generator=g, device="cuda").bfloat16()
+
+    rows = 2 * O if act else O
+    x, w = rand(M, K), rand(rows, K) / K ** 0.5
+    bias = rand(rows + 8)[shift: shift + rows]
+    res = rand(M * (O + pad) + 8)[shift: shift + M * (O + pad)].view(M, O + pad)[:, :O]
+    z = x.double() @ w.double().T + bias.double()
+    if act:
+        z = torch.nn.functional.silu(z[:, :O]) * z[:, O:]
+    want = z + res.double()
+    got = ops._linear_few(x, w, bias, res, None, act)
+    # half a place of bf16, and sums of K products in fp32
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=1e-4)
