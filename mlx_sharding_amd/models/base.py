@@ -113,8 +113,9 @@ def feed(into, out, x: torch.Tensor, act: str, norm: Optional[nn.Module] = None,
     """The gated unit of ``into``'s halves through ``out``, as ``project`` of each; one
     call for few rows."""
     if into.bias is None and out.bias is None and x.is_cuda:
-        w_in = dense_weight(into, x.shape[-1])
-        w_out = dense_weight(out, sum(into.splits) // 2)
+        w_in = into.weight if into.quant is None else dense_weight(into, x.shape[-1])
+        w_out = (out.weight if out.quant is None
+                 else dense_weight(out, sum(into.splits) // 2))
         if w_in is not None and w_out is not None:
             y = ops.feed_few(x, w_in, w_out, act, norm, residual)
             if y is not None:
@@ -285,8 +286,10 @@ class StageModel(nn.Module):
         # without embeddings the first parameter is a packed uint32
         # weight, and a uint32 KV cache silently truncates every K/V
         # value to zero (caught as PP-parity divergence)
-        p = next(self.parameters())
-        fp = next((q for q in self.parameters() if q.is_floating_point()), p)
+        every = self.parameters()
+        p = next(every)
+        fp = p if p.is_floating_point() else next(
+            (q for q in every if q.is_floating_point()), p)
         from ..ops.kvcache import make_cache
         return make_cache(self.cache_specs(),
                           dtype=dtype or fp.dtype,
