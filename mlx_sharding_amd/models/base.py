@@ -167,12 +167,11 @@ def head(norm: nn.Module, x: torch.Tensor, out: Optional[nn.Module] = None,
     for few rows.  For 33 to 64 of them and many weights the library's product behind a
     norm of its own is the faster one (64 rows, here and there: 16032 x 4096 30, 35 us;
     32000 x 2048 34.5, 37.8; 21720 x 3584 49, 41; 128256 x 4096 236, 221)."""
-    V, K = table.shape if out is None else (out.out_features, out.in_features)
-    if (ops.few_tokens(x) and (x.numel() <= 32 * K or V * K <= 1 << 26)
-            and as_built(norm)):
-        if out is None:
-            return ops.project(x, table, norm=norm)
-        if as_built(out):
+    if ops.few_tokens(x) and as_built(norm) and (out is None or as_built(out)):
+        V, K = table.shape if out is None else (out.out_features, out.in_features)
+        if x.numel() <= 32 * K or V * K <= 1 << 26:
+            if out is None:
+                return ops.project(x, table, norm=norm)
             return project(out, x, norm=norm)
     x = norm(x)
     return x @ table.t() if out is None else out(x)

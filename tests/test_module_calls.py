@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from mlx_sharding_amd.config import ModelConfig
-from mlx_sharding_amd.models import deepseek_v2, gemma2, llama
+from mlx_sharding_amd.models import deepseek_v2, gemma2, get_model_class, llama
 from mlx_sharding_amd.models.base import as_built
 from mlx_sharding_amd.models.fuse import fuse_model
 from mlx_sharding_amd.ops.kvcache import KVCache
@@ -143,3 +143,26 @@ def test_as_built():
         assert as_built(norm, proj)
     proj.forward = lambda x: x
     assert not as_built(norm, proj)
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("kind", ["llama", "experts"])
+def test_replaced_head_runs(kind, device):
+    """A head of another class, which need not say what it takes and gives."""
+    raw = ({"model_type": "llama", **BASE} if kind == "llama" else
+           {"model_type": "deepseek_v2", **LATENT, "n_routed_experts": 8})
+    config = ModelConfig.from_dict({**raw, "num_hidden_layers": 1, "vocab_size": 64})
+    with torch.device(device):
+        model = get_model_class(config.model_type)(config, config.shard(0, 1))
+    torch.manual_seed(0)
+    for name, p in model.named_parameters():
+        p.data.normal_(1.0 if "norm" in name else 0.0, 0.05)
+    tokens = torch.arange(5, device=device)[None]
+    want = model(tokens).float()
+    head, model.lm_head = model.lm_head, torch.nn.Identity()
+    got = model(tokens)
+    assert got.shape == (1, 5, 256)
+    got = torch.nn.functional.linear(got, head.weight).float()
+    # the normed row is rounded to bf16 on both sides, or its factor is applied behind
+    assert (got - want).norm() < 8e-3 * want.norm()
