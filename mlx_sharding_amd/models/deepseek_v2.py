@@ -486,9 +486,9 @@ class DeepseekV2MoE(nn.Module):
     def _beside(self, y):
         """The shared experts' matrices, where they go with the routed ones."""
         m = self.shared_experts
-        if (m is None or m._fused_gu is None or not as_built(m, m.down_proj)
-                or m._fused_gu.bias is not None or m.down_proj.bias is not None
-                or not ops.few_tokens(y)):
+        if (m is None or not as_built(m) or not as_built(*m.read())
+                or m._fused_gu is None or m._fused_gu.bias is not None
+                or m.down_proj.bias is not None or not ops.few_tokens(y)):
             return None
         both = (dense_weight(m._fused_gu, y.shape[1]),
                 dense_weight(m.down_proj, m.down_proj.in_features))

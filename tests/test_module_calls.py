@@ -166,3 +166,30 @@ def test_replaced_head_runs(kind, device):
     got = torch.nn.functional.linear(got, head.weight).float()
     # the normed row is rounded to bf16 on both sides, or its factor is applied behind
     assert (got - want).norm() < 8e-3 * want.norm()
+
+
+class Halved(torch.nn.Module):
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, x):
+        return self.inner(x) * 0.5
+
+
+@torch.no_grad()
+def test_replaced_shared_experts_are_not_read():
+    layer, _, _ = a_layer("experts", True, "cpu")
+    layer.mlp.shared_experts = Halved(layer.mlp.shared_experts)
+    assert layer.mlp._beside(torch.zeros(1, 256, dtype=torch.bfloat16)) is None
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+def test_replaced_shared_experts_run():
+    layer, cache, rope = a_layer("experts", True)
+    layer.mlp.shared_experts = Halved(layer.mlp.shared_experts)
+    same, theirs, _ = a_layer("experts", True)
+    same.mlp.shared_experts.down_proj.weight.mul_(0.5)
+    for y, expect in zip(steps(layer, cache, rope), steps(same, theirs, rope)):
+        assert (y.double() - expect.double()).norm() < 0.02 * expect.double().norm()
