@@ -42,7 +42,7 @@ def upload(values: np.ndarray, device) -> torch.Tensor:
     if device.type != "cuda":
         return torch.from_numpy(values).to(device)
     held = torch.empty(values.shape, dtype=torch.from_numpy(values).dtype,
-                       pin_memory=True)
+                       device="cpu", pin_memory=True)
     held.numpy()[...] = values
     return held.to(device, non_blocking=True)
 

@@ -4,7 +4,9 @@ import numpy as np
 import pytest
 import torch
 
+import tuvutar_cases as cases
 from mlx_sharding_amd.ops.paged import RaggedBatch, PagedState, RowSpec, upload
+from mlx_sharding_amd.parallel.batching import BatchEngine, Portion
 
 
 @pytest.mark.parametrize("n", [0, 1, 7, 4096])
@@ -23,6 +25,28 @@ def test_upload_behind_work(n):
         x = x @ x / 64.0
     out = [upload(np.full(n, i, dtype=np.int32), "cuda") for i in range(200)]
     assert all(t.tolist() == [i] * n for i, t in enumerate(out))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("default", ["cpu", "meta", "cuda"])
+def test_upload_with_a_default_device(default):
+    with torch.device(default):
+        t = upload(np.arange(5, dtype=np.int32), "cuda")
+    assert t.device.type == "cuda" and t.tolist() == [0, 1, 2, 3, 4]
+
+
+@pytest.mark.gpu
+def test_batches_with_a_default_device():
+    cfg = cases.config(32, 40, [cases.delta(2, 1, 16, 16, 4, ff=48)])
+    model = cases.build(cfg, cases.weights(cfg), "cuda")
+    steps = [[3, 1, 4, 1, 5], [9], [2]]
+    want, got = BatchEngine(model, 128, 2), BatchEngine(model, 128, 2)
+    for tokens in steps:
+        portion = Portion("a", tokens, [len(tokens) - 1])
+        a = want.step([portion])
+        with torch.device("cuda"):
+            b = got.step([portion])
+        assert torch.equal(a, b)
 
 
 def _places(device):
