@@ -477,7 +477,8 @@ class GatedMLP(nn.Module):
         self.fused = FusedColumns([self.gate, self.up])
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        if self.fused is not None and ops.few_tokens(h) and as_built(self.down):
+        if (self.fused is not None and ops.few_tokens(h) and as_built(self.down)
+                and self.act is self.ACTS[self.kind]):
             return feed(self.fused, self.down, h, self.kind)
         g, u = self.fused(h) if self.fused is not None else (self.gate(h), self.up(h))
         return self.down(self.act(g, u))

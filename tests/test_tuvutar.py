@@ -93,6 +93,23 @@ def test_gated_mlp(device, dtype, ff):
     assert cases.error(m(h.to(device)), want) < (2e-6 if dtype == F32 else 2e-2)
 
 
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("n", [7, 70])
+def test_gated_mlp_with_another_unit(device, n):
+    """An ``act`` that was set on the module, for few tokens as for many."""
+    from mlx_sharding_amd.models.mixers import GatedMLP
+    torch.manual_seed(0)
+    m = GatedMLP(64, 64, "silu")
+    for p in m.parameters():
+        p.data.normal_(0.0, 0.1)
+    m.to(device).prepare()
+    m.act = lambda gate, up: gate.relu() * up
+    h = torch.randn(n, 64).bfloat16().to(device)
+    g, u = (h.double() @ w.weight.double().T for w in (m.gate, m.up))
+    want = (g.relu() * u) @ m.down.weight.double().T
+    assert cases.error(m(h), want) < 2e-2
+
+
 class Mixer:
     """One mixer of a layer with its storage: feed portions, compare."""
 
