@@ -70,7 +70,7 @@ class LlamaAttention(nn.Module):
         offset = 0
         gp = None
         out = None
-        if cache is not None and T == 1:
+        if T == 1 and type(cache) is KVCache:  # others append by methods of their own
             out = cache.attend_step(q, k, v, cos, sin, self.scale)
         if out is not None:
             pass

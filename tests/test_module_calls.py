@@ -193,3 +193,43 @@ def test_replaced_shared_experts_run():
     same.mlp.shared_experts.down_proj.weight.mul_(0.5)
     for y, expect in zip(steps(layer, cache, rope), steps(same, theirs, rope)):
         assert (y.double() - expect.double()).norm() < 0.02 * expect.double().norm()
+
+
+class Rows:
+    """A cache of a program's own: what a layer needs of one on the CPU."""
+    graph_pos = None
+
+    def __init__(self):
+        self.offset, self.k, self.v = 0, [], []
+
+    def update(self, k, v):
+        self.offset += k.shape[2]
+        self.k.append(k)
+        self.v.append(v)
+        return torch.cat(self.k, 2), torch.cat(self.v, 2)
+
+
+class Noted(KVCache):
+    def append_rope_qkv(self, q, *rest):
+        self.seen = getattr(self, "seen", 0) + q.shape[1]
+        return super().append_rope_qkv(q, *rest)
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("kind", ["llama", "gemma2"])
+def test_other_caches_on_the_cpu(kind):
+    want = steps(*a_layer(kind, False, "cpu"), device="cpu")
+    layer, _, rope = a_layer(kind, False, "cpu")
+    for y, expect in zip(steps(layer, Rows(), rope, "cpu"), want):
+        assert torch.equal(y, expect)
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+@pytest.mark.parametrize("kind", ["llama", "gemma2"])
+def test_caches_with_methods_of_their_own(kind):
+    layer, _, rope = a_layer(kind, True)
+    cache = Noted(2, 64, 64, device="cuda")
+    for y, expect in zip(steps(layer, cache, rope), steps(*a_layer(kind, True))):
+        assert (y.double() - expect.double()).norm() < 0.02 * expect.double().norm()
+    assert cache.seen == cache.offset == 150
