@@ -228,7 +228,8 @@ class StageModel(nn.Module):
         else:
             pos = first.graph_pos if first is not None else None
             if (pos is not None and x.shape[1] == 1 and type(embed) is nn.Embedding
-                    and as_built(embed) and embed.max_norm is None):
+                    and as_built(embed) and embed.max_norm is None
+                    and getattr(self.rope_for, "__func__", None) is StageModel.rope_for):
                 found = ops.step_begin(x, embed.weight, scale, pos,
                                        *self._rope_tables(x.device, first.capacity))
                 if found is not None:

@@ -233,3 +233,36 @@ def test_caches_with_methods_of_their_own(kind):
     for y, expect in zip(steps(layer, cache, rope), steps(*a_layer(kind, True))):
         assert (y.double() - expect.double()).norm() < 0.02 * expect.double().norm()
     assert cache.seen == cache.offset == 150
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("where", ["class", "instance"])
+def test_rotations_of_a_models_own(where, device, monkeypatch):
+    """A captured step's rotations are those that the model's rope_for gives."""
+    def own(self, cache0, T, device):
+        cos, sin, offset = llama.LlamaStageModel.rope_for(self, cache0, T, device)
+        return cos + 1.0, sin, offset
+
+    class Other(llama.LlamaStageModel):
+        rope_for = own
+
+    config = ModelConfig.from_dict({"model_type": "llama", **BASE,
+                                    "num_hidden_layers": 1, "vocab_size": 64})
+    cls = Other if where == "class" else llama.LlamaStageModel
+    with torch.device(device):
+        model = cls(config, config.shard(0, 1))
+    if where == "instance":
+        model.rope_for = own.__get__(model)
+    if device == "cpu":      # as the kernel would, were it asked
+        monkeypatch.setattr(llama.ops, "step_begin",
+                            lambda x, table, scale, pos, cos, sin:
+                            (table[x], cos[pos], sin[pos]))
+    cache = model.make_cache()
+    cache[0].ensure_capacity(16, 1)
+    cache[0].graph_pos = torch.tensor([5], dtype=torch.int32, device=device)
+    x = torch.tensor([[3]], device=device)
+    h, cos, sin = model.begin(x, cache, model.model.embed_tokens)
+    want = model.rope_for(cache[0], 1, torch.device(device))
+    assert torch.equal(cos, want[0]) and torch.equal(sin, want[1])
+    assert torch.equal(h, model.model.embed_tokens(x))
