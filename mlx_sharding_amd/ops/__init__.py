@@ -725,6 +725,7 @@ def expert_rows(y, choice, weight, gate, up, down, bits: int, group_size: int,
 def expert_shared_ok(n_tokens: int, H: int, w_in, w_out) -> bool:
     """Whether expert_rows takes a shared feed-forward of these matrices along."""
     return (n_tokens <= 8 and w_in is not None and w_out is not None
+            and not os.environ.get("MLXS_AMD_DENSE_GEMV")  # names another kernel
             and w_out.shape[-1] % 64 == 0 and max(H, w_out.shape[-1]) <= 4096
             and tuple(w_in.shape) == (2 * w_out.shape[-1], H) and w_out.shape[0] == H
             and all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous()

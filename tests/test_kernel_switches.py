@@ -48,6 +48,21 @@ def test_dense_gemv(kind, seen, monkeypatch):
 
 
 @torch.no_grad()
+def test_dense_gemv_of_shared_experts(seen, monkeypatch):
+    layer, _, _ = a_layer("experts", True)
+    x = torch.randn(1, 1, 256, device="cuda").bfloat16()
+    norm = layer.post_attention_layernorm
+    expect = layer.mlp.decode(x, None, norm).double()
+    assert "moe_rows" in seen and "dense_gemv" not in seen
+    seen.clear()
+    monkeypatch.setenv("MLXS_AMD_DENSE_GEMV", "1")
+    y = layer.mlp.decode(x, None, norm).double()
+    assert seen.count("dense_gemv") == 2
+    # units and their product are rounded to bf16 on both sides
+    assert (y - expect).norm() < 8e-3 * expect.norm()
+
+
+@torch.no_grad()
 @pytest.mark.parametrize("bits", [0, 4])
 def test_resident_experts(bits, seen, monkeypatch):
     """Routed experts of packed weights on their bf16 copies; bf16 ones have none."""
