@@ -482,7 +482,7 @@ def moe_gate(router_logits, top_k: int, n_group: int = 1, topk_group: int = 1,
     up to 64 experts in one group, else torch's."""
     if (use_native(router_logits) and n_group <= 1 and _plain(router_logits)
             and router_logits.dtype == torch.bfloat16 and router_logits.is_contiguous()
-            and router_logits.shape[0] and top_k <= router_logits.shape[1] <= 64):
+            and router_logits.shape[0] and 0 < top_k <= router_logits.shape[1] <= 64):
         return tuple(hip_ext().moe_choose(router_logits, top_k, routed_scaling_factor,
                                           norm_topk_prob))
     return ref.moe_gate(router_logits, top_k, n_group, topk_group,

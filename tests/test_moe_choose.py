@@ -32,6 +32,11 @@ def test_choice_of_ties_and_no_numbers():
     assert idx.tolist() == [[0, 1, 2]] * 3     # in their order, each once
 
 
+def test_no_choice():
+    w, idx = ops.moe_gate(torch.zeros(3, 9, dtype=torch.bfloat16, device="cuda"), 0)
+    assert w.shape == idx.shape == (3, 0) and idx.dtype == torch.int64
+
+
 @pytest.mark.parametrize("top", [1, 2, 3, 4, 6, 7, 9])
 @pytest.mark.parametrize("H", [4, 1028, 2048])
 def test_sum(top, H):
