@@ -96,7 +96,8 @@ class BatchEngine:
         start = {batch.order[e]: batch.host[e][0] for e in range(len(portions))}
         wanted = [start[j] + int(w) for j, p in enumerate(portions) for w in p.want]
         ids += wanted
-        x, rows = upload(np.array(ids, dtype=np.int64), self.device).split(
+        # whatever has a whole number: tokens may be scalars on a device
+        x, rows = upload(np.fromiter(ids, np.int64, len(ids)), self.device).split(
             [batch.n_tokens, len(ids) - batch.n_tokens])
         if wanted == list(range(batch.n_tokens)):
             rows = None  # all of them, as they are

@@ -49,6 +49,32 @@ def test_batches_with_a_default_device():
         assert torch.equal(a, b)
 
 
+class OnDevice:
+    """A token as a scalar on a GPU shows itself to numpy."""
+
+    def __init__(self, value):
+        self.value = value
+
+    def __array__(self, *args, **kwargs):
+        raise TypeError("not on the host")
+
+    def __int__(self):
+        return self.value
+
+    __index__ = __int__
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_tokens_that_are_scalars(device):
+    cfg = cases.config(32, 40, [cases.delta(2, 1, 16, 16, 4, ff=48)])
+    engine = BatchEngine(cases.build(cfg, cases.weights(cfg), device), 128, 2)
+    scalar = OnDevice if device == "cpu" else lambda t: torch.tensor(t, device=device)
+    tokens = [3, 1, 4]
+    want = engine.step([Portion("a", tokens, [2])])
+    got = engine.step([Portion("b", [scalar(t) for t in tokens], [2])])
+    assert torch.equal(got, want)
+
+
 def _places(device):
     state = PagedState([RowSpec(8)], 512, 3, torch.float32, torch.device(device))
     for r, n in enumerate((5, 64, 130)):
