@@ -32,7 +32,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------------------
 // Experts of the tokens, a wave each.  Bound by its instructions, five for each pair of
 // experts.  For 32768 tokens of 64 experts softmax, selection, sorting, scaling and
-// conversions of their own took 160 us (the selection alone 119); 25 here.
+// conversions of their own took 160 us (the selection alone 119); 23 here.
 // ---------------------------------------------------------------------------
 
 __global__ __launch_bounds__(256) void moe_choose_kernel(

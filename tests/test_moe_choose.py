@@ -32,6 +32,21 @@ def test_choice_of_ties_and_no_numbers():
     assert idx.tolist() == [[0, 1, 2]] * 3     # in their order, each once
 
 
+@pytest.mark.parametrize("normalize", [False, True])
+@pytest.mark.parametrize("spread", [1.0, 8.0])
+def test_weights_keep_their_bits(spread, normalize):
+    g = torch.Generator("cuda").manual_seed(1)
+    logits = (torch.randn(4096, 64, generator=g, device="cuda") * spread).bfloat16()
+    w = ops.moe_gate(logits, 6, norm_topk_prob=normalize)[0].double()
+    want = torch.softmax(logits.double(), -1).topk(6, -1).values
+    if normalize:
+        want = want / want.sum(-1, keepdim=True)
+    # in units of 2^-24, each a rounding: the exponential two, its sum over 64 lanes six,
+    # the quotient two; the second sum and quotient as many less the exponential
+    off = (w.sort(-1, descending=True).values - want).abs() / want
+    assert float(off.max()) < (18 if normalize else 10) * 2 ** -24
+
+
 def test_no_choice():
     w, idx = ops.moe_gate(torch.zeros(3, 9, dtype=torch.bfloat16, device="cuda"), 0)
     assert w.shape == idx.shape == (3, 0) and idx.dtype == torch.int64
