@@ -58,7 +58,7 @@ class ExpertShape:
         return TILE_SHORT if few else TILE_LONG
 
     def tiles(self, tokens: int) -> int:
-        """Pairs of a tile of the persistent kernel (moe_tiles.hip), 0: the others'.
+        """Pairs of a tile of the persistent kernel (moe_tiles_kernel.h), 0: the others'.
         Few pairs an expert are one tile of 16 for most, which reads weights as fast;
         with few experts of few units there is not a tile for every second CU.  Measured
         (us for both products, router and placement; as before, with 128, with 256):
@@ -115,7 +115,7 @@ def route(h, router, correction, sh: ExpertShape, routing: Routing = Routing()):
 
 
 def _tiled(h, up, down) -> bool:
-    """Whether moe_tiles.hip takes these operands."""
+    """Whether ragged_experts_tiles.hip takes these operands."""
     K, (_, O, F) = up.shape[2], down.shape
     return (h.dtype == torch.bfloat16 and O % 64 == 0 and min(K, F, O) >= 128
             and up.shape[1] == 2 * F and max(K, O) * F < 2 ** 31

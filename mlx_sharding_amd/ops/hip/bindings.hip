@@ -821,8 +821,6 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   return out.transpose(1, 2);
 }
 
-// Routed experts of a prompt: silu(x gate^T) * (x up^T), down of that, for the pairs
-// of choice [N, top] (int64).  Returns (rows [N * top, H], place of each pair).
 // Softmax of rows of logits [N, E]: (weights fp32, experts) of the `top` largest.
 std::vector<torch::Tensor> moe_choose(torch::Tensor logits, int64_t top, double scaling,
                                       bool normalize) {
@@ -839,6 +837,8 @@ std::vector<torch::Tensor> moe_choose(torch::Tensor logits, int64_t top, double 
   return {weight, choice};
 }
 
+// Routed experts of a prompt: silu(x gate^T) * (x up^T), down of that, for the pairs
+// of choice [N, top] (int64).  Returns (rows [N * top, H], place of each pair).
 std::vector<torch::Tensor> moe_tiles(torch::Tensor x, torch::Tensor choice,
                                      torch::Tensor gate, torch::Tensor up,
                                      torch::Tensor down, int64_t tile) {
@@ -877,11 +877,11 @@ std::vector<torch::Tensor> moe_tiles(torch::Tensor x, torch::Tensor choice,
   MoeTilesArgs a{(const char*)x.data_ptr(), (const char*)gate.data_ptr(),
                  (const char*)up.data_ptr(), (__bf16*)h.data_ptr(), tokens, tiles,
                  n_tiles, x.stride(0) * 2, (int)I, (int)H, 0, I * H * 2};
-  launch_moe_tiles(&a, (int)tile, MT_SILU, cur_stream());
+  launch_moe_tiles(&a, (int)tile, true, cur_stream());
   MoeTilesArgs b{(const char*)h.data_ptr(), (const char*)down.data_ptr(), nullptr,
                  (__bf16*)y.data_ptr(), nullptr, tiles, n_tiles, I * 2, (int)H,
                  (int)I, 0, I * H * 2};
-  launch_moe_tiles(&b, (int)tile, MT_SUMS, cur_stream());
+  launch_moe_tiles(&b, (int)tile, false, cur_stream());
   return {y, where};
 }
 

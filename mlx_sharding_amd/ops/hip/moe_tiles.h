@@ -1,4 +1,4 @@
-// Arguments of the routed experts' kernels of a prompt (moe_tiles.hip).
+// Arguments of the routed experts' kernels of a prompt.
 #pragma once
 
 #include "hip_common.h"
@@ -37,6 +37,8 @@ struct MoeTilesArgs {
 extern "C" {
 void launch_moe_choose(const void*, long*, float*, int, int, int, int, float, hipStream_t);
 void launch_moe_place(const MoePlaceArgs*, hipStream_t);
-// pairs of a tile: 256 or 128
-void launch_moe_tiles(MoeTilesArgs*, int tile, MoeUnit, hipStream_t);
+// pairs of a tile: 256 or 128; gated: silu (moe_tiles.hip) or clamped units
+// (ragged_experts_tiles.hip), else sums
+void launch_moe_tiles(MoeTilesArgs*, int tile, bool gated, hipStream_t);
+void launch_clamped_tiles(MoeTilesArgs*, int tile, bool gated, hipStream_t);
 }

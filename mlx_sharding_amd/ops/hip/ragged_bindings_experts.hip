@@ -147,7 +147,7 @@ Tensor expert_gemm(Tensor x, c10::optional<Tensor> tokens, Tensor tiles,
   return out;
 }
 
-// Both products of clamped units, by moe_tiles.hip: rows of x, which tokens of the pairs
+// Both products of clamped units (ragged_experts_tiles.hip): rows of x, which tokens of the pairs
 // are, times up [experts, 2 F, K] and the pairs' scale, and those times down [experts, O,
 // F] -> [pairs, O].  tiles of 128 or 256 pairs, of which `used` are there.
 Tensor expert_tiles(Tensor x, Tensor tokens, Tensor tiles, Tensor used, Tensor up,
@@ -175,11 +175,11 @@ Tensor expert_tiles(Tensor x, Tensor tokens, Tensor tiles, Tensor used, Tensor u
                  ints(tokens, pairs, "tokens"), ints(tiles, 0, "tiles"),
                  ints(used, 1, "used"), stride * 2, (int)F, (int)K, 0, 2 * F * K * 2,
                  scale.data_ptr<float>(), (float)limit, (float)alpha};
-  launch_moe_tiles(&a, (int)tile, MT_CLAMPED, stream());
+  launch_clamped_tiles(&a, (int)tile, true, stream());
   MoeTilesArgs b{(const char*)h.data_ptr(), (const char*)down.data_ptr(), nullptr,
                  (__bf16*)y.data_ptr(), nullptr, a.tiles, a.n_tiles, F * 2, (int)O,
                  (int)F, 0, O * F * 2};
-  launch_moe_tiles(&b, (int)tile, MT_SUMS, stream());
+  launch_clamped_tiles(&b, (int)tile, false, stream());
   return y;
 }
 
