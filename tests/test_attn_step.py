@@ -1,4 +1,5 @@
-"""A token's rotations, cache rows and attention in one kernel, beside the separate ones."""
+"""A token's rotations, cache rows and attention in one kernel, beside the separate ones
+and against 64 bits."""
 
 import math
 
@@ -38,6 +39,21 @@ def _token(B, Hq, Hkv, D, gen):
             torch.cos(angle), torch.sin(angle))
 
 
+def _exact(q, cos, sin, keys, values, cap, window):
+    """Attention in 64 bits of a query, turned and rounded, to keys [B, Hkv, S, D]."""
+    B, _, Hq, D = q.shape
+    a, b = q.double().chunk(2, -1)
+    c, s = cos.double(), sin.double()
+    q = torch.cat([a * c - b * s, b * c + a * s], -1).bfloat16().double()
+    if window:
+        keys, values = keys[:, :, -window:], values[:, :, -window:]
+    k, v = (t.double().repeat_interleave(Hq // t.shape[1], 1) for t in (keys, values))
+    z = (k @ q.transpose(1, 2).transpose(2, 3)).squeeze(-1) * 0.1
+    if cap:
+        z = cap * torch.tanh(z / cap)
+    return (torch.softmax(z, -1)[:, :, None] @ v).reshape(B, 1, -1)
+
+
 # no key before, the token first, last and in the middle of a tile, one slice and 64,
 # slices without keys (captured ones are made for the whole room)
 @pytest.mark.parametrize("captured", [False, True])
@@ -65,6 +81,11 @@ def test_same_as_separate_kernels(B, Hq, Hkv, D, cached, window, cap, captured):
         want = want.transpose(1, 2).reshape(B, 1, -1)
         assert got.shape == want.shape
         assert float((got.float() - want.float()).norm() / want.float().norm()) < 2e-3
+        exact = _exact(q, cos, sin, *(t[:, :, : cached + step + 1] for t in (one._k, one._v)),
+                       cap, window)
+        # results are rounded to 8 bits, half a step of 2^-8 at most; few of the query's
+        # values the other way
+        assert float((got.double() - exact).norm() / exact.norm()) < 2e-3
         assert not one._tickets.any()
         if captured:
             for c in (one, two):

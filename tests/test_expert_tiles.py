@@ -1,4 +1,4 @@
-"""Clamped experts of many tokens on the persistent tiles, beside the CPU's."""
+"""Clamped experts of many tokens on the persistent tiles, against 64-bit products."""
 
 import pytest
 import torch
@@ -21,29 +21,55 @@ def _operands(N, sh, seed=0):
     return new(N, sh.widthp).bfloat16(), router, up, down
 
 
+def _exact(h, idx, weight, up, down, sh):
+    """(outputs of the chosen experts in 64 bits, how far bf16 units and results may be
+    off) for pairs [N, top]; those of identity experts are zero."""
+    out = torch.zeros(*idx.shape, sh.width, dtype=torch.float64, device=h.device)
+    bound = torch.zeros_like(out)
+    for e in range(sh.experts):
+        t, j = (idx == e).nonzero(as_tuple=True)
+        p = (h[t].double() @ up[e].double().T) * weight[t, j, None].double()
+        g, u = p[:, : sh.ffp].clamp(max=GLU.limit), p[:, sh.ffp:].clamp(-GLU.limit, GLU.limit)
+        unit = g * torch.sigmoid(GLU.alpha * g) * (u + 1)
+        w = down[e].double()
+        out[t, j] = unit @ w.T
+        # half a step of 2^-8 each; sums, exponentials and quotients in 32 bits
+        bound[t, j] = 2.0 ** -8 * (out[t, j].abs() + unit.abs() @ w.abs().T) + 1e-5
+    return out, bound
+
+
 # a mean of 16 pairs and of one more, 127 and 128: the borders of the kernels; experts
-# without pairs; contractions of two and more than four stages; output tiles' remainders
-@pytest.mark.parametrize("N,width,ff,E,top", [
-    (128, 128, 2048, 8, 1), (129, 128, 2048, 8, 1), (1016, 128, 2048, 8, 1),
-    (1024, 128, 2048, 8, 1), (300, 320, 192, 90, 6), (2100, 192, 320, 64, 4)])
-def test_beside_cpu(N, width, ff, E, top):
-    sh = experts.ExpertShape(width, ff, E, 0, top)
-    assert sh.tiles(N) == (0 if N == 128 else 128 if N * top < 128 * E else 256)
-    h, router, up, down = _operands(N, sh)
+# without pairs; contractions of two and more than four stages; output tiles' remainders;
+# experts that hand a row on, whose pairs have no places
+@pytest.mark.parametrize("routing", [ON_INPUT, experts.Routing("sigmoid", False, True)])
+@pytest.mark.parametrize("N,width,ff,E,identity,top", [
+    (128, 128, 2048, 8, 0, 1), (129, 128, 2048, 8, 0, 1), (1016, 128, 2048, 8, 0, 1),
+    (1024, 128, 2048, 8, 0, 1), (300, 320, 192, 90, 0, 6), (2100, 192, 320, 64, 0, 4),
+    (400, 128, 1024, 16, 5, 3), (900, 192, 2048, 8, 1, 2)])
+def test_against_64_bits(N, width, ff, E, identity, top, routing):
+    sh = experts.ExpertShape(width, ff, E, identity, top)
+    mean = N * top / sh.total
+    assert sh.tiles(N) == (0 if mean <= 16 else 128 if mean < 128 else 256)
+    h, router, up, down = (t.cuda() for t in _operands(N, sh))
     if E == 90:
         h[:] = h[:1]            # all tokens choose alike
-    want, at, _ = experts.expert_rows(h, router, None, up, down, sh, ON_INPUT, GLU)
-    got, where, weight = experts.expert_rows(h.cuda(), router.cuda(), None, up.cuda(),
-                                             down.cuda(), sh, ON_INPUT, GLU)
-    assert weight is None
-    # a token's experts as a set: pairs of rows in the order of choice
-    a = want[at.long()].double()
-    b = got[where.long()].double().cpu()
-    # two experts whose scores are nearly tied may change places: compare the sums
-    a, b = a.sum(1), b.sum(1)
-    off = (a - b).norm(dim=1) / a.norm(dim=1)
-    # units and results rounded to bf16
-    assert float(off.median()) < 4e-3 and float((off > 2e-2).double().mean()) < 0.01
+    idx, weight = hip_ragged().expert_route(
+        h, router, None, sh.total, sh.experts, top, routing.score == "sigmoid",
+        routing.normalize)[:2]
+    # the choice: no other expert's logit is larger, but by the error of a sum of 32 bits
+    z = h.double() @ experts.unpack(router, sh.total, sh.widthp).double().T
+    assert bool((idx.sort(-1).values.diff(dim=-1) > 0).all())
+    left = z.scatter(-1, idx.long(), float("-inf")).max(-1).values
+    assert bool((left <= z.gather(-1, idx.long()).min(-1).values + 1e-4).all())
+    # the rest has that choice on both sides
+    got, where, rest = experts.expert_rows(h, router, None, up, down, sh, routing, GLU)
+    assert rest is None and bool(((where < 0) == (idx >= E)).all())
+    own = where[where >= 0].sort().values
+    assert torch.equal(own, torch.arange(len(own), device="cuda", dtype=torch.int32))
+    want, bound = _exact(h, idx, weight, up, down, sh)
+    there = where >= 0
+    rows = got[where[there].long()].double()
+    assert bool(((rows - want[there]).abs() <= bound[there]).all())
 
 
 def test_refusals():

@@ -53,9 +53,9 @@ def test_step_end(rows, n):
 
 # normed rows and results rounded to bf16: below 4e-3 of the result's 2-norm
 @pytest.mark.parametrize("rows", [1, 32, 33, 64, 65])
-@pytest.mark.parametrize("V", [1000, 16400])   # less and more than 2^25 weights
-def test_head(rows, V):
-    K = 2048
+@pytest.mark.parametrize("V", [1000, 32768, 32784])   # up to 2^26 weights, and more
+def test_head(rows, V, monkeypatch):
+    K, fused = 2048, []
     g = torch.Generator("cuda").manual_seed(V)
     new = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
     norm, out = RMSNorm(K, 1e-5, 1.0).cuda(), Linear(K, V).cuda()
@@ -65,6 +65,11 @@ def test_head(rows, V):
     h = x.double()
     h = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + 1e-5)
     want = (h * (norm.weight.double() + 1)) @ out.weight.double().t()
+    project = ops.project
+    monkeypatch.setattr(ops, "project", lambda *a, **k: (fused.append(k["norm"]),
+                                                         project(*a, **k))[1])
     for got in (head(norm, x, out), head(norm, x, table=out.weight)):
         assert got.shape == (rows, 1, V)
         assert float((got.double() - want).norm() / want.norm()) < 4e-3
+    # the norm goes with the product, or before the library's
+    assert fused == [norm] * (2 if rows <= 32 or (rows <= 64 and V <= 32768) else 0)
