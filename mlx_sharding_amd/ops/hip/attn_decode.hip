@@ -364,8 +364,8 @@ extern "C" bool attn_decode_supported_shape(int G, int Dv) {
 // of its keys.  Tiles of keys and values go to LDS without passing registers, the
 // next one while this one is worked on; what it reads from memory is all that
 // bounds it, and two blocks a CU keep 64 KB and more in flight.  S^T = K Q^T on
-// 16x16x32 products: a wave takes 16 keys of a tile of 32 and half of the
-// contraction, leaves its scores in LDS, and after a barrier every wave has the
+// 16x16x32 products: a wave takes 16 keys (with tiles of 32 keys also half of the
+// contraction), leaves its scores in LDS, and after a barrier every wave has the
 // weights of the whole tile in the layout of the next product's operand and makes
 // a quarter of the output's columns, O^T = V^T P^T.  So waves share no outputs.
 // V^T is read by ds_read_b64_tr_b16 out of rows as they lie in memory; values that
@@ -375,10 +375,9 @@ extern "C" bool attn_decode_supported_shape(int G, int Dv) {
 // parts, which keep 16 bits, and 3 less than with parts that are rounded, not cut off).
 // Slices come from the length on the device, so they are even under capture.
 // Measured (before: dot products and sums on the vector units, up to 8 slices of
-// the capacity): 16 heads over a latent of 576/512, 64 x 513 keys: 66 -> 22 us,
-// 1 x 3002: 75 -> 13.  Heads of 64, 128 and 256, which have the kernel behind this one
-// now: 64 sequences of 2049 keys, 32 heads of 128 over 8: 179 -> 98; one of 1024:
-// 24 -> 7.2; 5 of 5004, 16 heads of 256 over 8, capped: 91 -> 45.
+// the capacity): 64 sequences of 2049 keys, 32 heads of 128 over 8: 179 -> 98 us
+// (now in the kernel for heads of 64 and 128); one of 1024: 24 -> 7.2; 5 of 5004, 16 heads of 256 over 8, capped: 91 ->
+// 45; 16 heads over a latent of 576/512, 64 x 513 keys: 66 -> 22, 1 x 3002: 75 -> 13.
 // ---------------------------------------------------------------------------
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -558,16 +557,17 @@ __device__ __forceinline__ void finish_slice(const DecodeArgs& a, const f32x4 (&
   }
 }
 
-template <int DK, int DV, bool INROW>
+template <int DK, int DV, int KT, bool INROW>
 __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
     const DecodeArgs a) {
-  constexpr int KT = 32;  // keys of a tile
   constexpr int KP = DK / 8, VP = INROW ? KP : DV / 8;  // pieces of a row
   constexpr int NK = DK / 32, ND = DV / 64;
   constexpr int KB = KT * DK * 2, VB = INROW ? 0 : KT * DV * 2;
-  static_assert(NK % 2 == 0 && KB % 4096 == 0 && VB % 4096 == 0, "sizes");
+  constexpr int HALVES = 64 / KT;
+  static_assert(KT == 64 || KT == 32, "four waves make the scores of a tile");
+  static_assert(NK % HALVES == 0 && KB % 4096 == 0 && VB % 4096 == 0, "sizes");
   __shared__ __attribute__((aligned(16))) char smem[2 * (KB + VB)];
-  __shared__ float sc[2][2][KT][16];
+  __shared__ float sc[2][HALVES][KT][16];
 
   const int S = a.s_ptr ? (int)min((long)*a.s_ptr + 1, a.cap) : a.S;
   const int b = blockIdx.x / a.Hkv, hk = blockIdx.x % a.Hkv;
@@ -606,13 +606,13 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
   if (from < to) stage(from, 0);
 
   const long row0 = (long)b * a.Hq + hk * G;  // first query head
-  const int kb = wid & 1, half = wid >> 1;
-  bf16x8_t qf[NK / 2];
+  const int kb = KT == 64 ? wid : wid & 1, half = KT == 64 ? 0 : wid >> 1;
+  bf16x8_t qf[NK / HALVES];
   {
     const char* src = a.q + (row0 + min(l16, G - 1)) * (DK * 2) +
-                      half * (NK / 2) * 64 + lg * 16;
+                      half * (NK / HALVES) * 64 + lg * 16;
 #pragma unroll
-    for (int i = 0; i < NK / 2; ++i)
+    for (int i = 0; i < NK / HALVES; ++i)
       qf[i] = *reinterpret_cast<const bf16x8_t*>(src + i * 64);
   }
   float m = -1e30f, l = 0.0f;  // reference of the exponents (base 2), sum
@@ -629,8 +629,8 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
     const char* vt = kt + KB;
     f32x4 s4 = {0, 0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < NK / 2; ++i) {
-      const int piece = (half * (NK / 2) + i) * 4 + lg;
+    for (int i = 0; i < NK / HALVES; ++i) {
+      const int piece = (half * (NK / HALVES) + i) * 4 + lg;
       const bf16x8_t f = *reinterpret_cast<const bf16x8_t*>(
           kt + (kb * 16 + l16) * KP * 16 + dt_place<KP, true>(l16, piece) * 16);
       s4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f, qf[i], s4, 0, 0, 0);
@@ -639,18 +639,21 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
     for (int r = 0; r < 4; ++r) sc[buf][half][kb * 16 + lg * 4 + r][l16] = s4[r];
     __syncthreads();
 
-    float p[8], top = -INFINITY;
+    float p[KT / 4], top = -INFINITY;  // 8 of every 32 keys
     auto key_of = [&](int i) { return i / 4 * 16 + lg * 4 + (i & 3); };
 #pragma unroll
-    for (int i = 0; i < 8; ++i) p[i] = sc[buf][0][key_of(i)][l16] + sc[buf][1][key_of(i)][l16];
+    for (int i = 0; i < KT / 4; ++i) {
+      p[i] = sc[buf][0][key_of(i)][l16];
+      if (HALVES == 2) p[i] += sc[buf][HALVES - 1][key_of(i)][l16];
+    }
     if (a.score.out > 0.0f) {
       soft_capped(a.score, p);
     } else {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) p[i] *= a.score.lin;
+      for (int i = 0; i < KT / 4; ++i) p[i] *= a.score.lin;
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < KT / 4; ++i) {
       if (t + key_of(i) >= to) p[i] = -INFINITY;
       top = fmaxf(top, p[i]);
     }
@@ -665,43 +668,47 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[d][r] *= f;
     }
-    bf16x8_t v[ND];
-    u32x4 w[3];  // pairs: the upper halves of what is left of each weight
 #pragma unroll
-    for (int j = 0; j < 8; j += 2) {
-      float f[2];
+    for (int x = 0; x < KT / 32; ++x) {
+      bf16x8_t v[ND];
+      u32x4 w[3];  // pairs: the upper halves of what is left of each weight
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        f[h] = __builtin_amdgcn_exp2f(p[j + h] - m);
-        l += f[h];
+      for (int j = 0; j < 8; j += 2) {
+        float f[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          f[h] = __builtin_amdgcn_exp2f(p[x * 8 + j + h] - m);
+          l += f[h];
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const unsigned a = __float_as_uint(f[0]), b = __float_as_uint(f[1]);
+          w[i][j / 2] = __builtin_amdgcn_perm(b, a, 0x07060302);
+          f[0] -= __uint_as_float(a & 0xFFFF0000u);
+          f[1] -= __uint_as_float(b & 0xFFFF0000u);
+        }
       }
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const unsigned a = __float_as_uint(f[0]), b = __float_as_uint(f[1]);
-        w[i][j / 2] = __builtin_amdgcn_perm(b, a, 0x07060302);
-        f[0] -= __uint_as_float(a & 0xFFFF0000u);
-        f[1] -= __uint_as_float(b & 0xFFFF0000u);
+      for (int d = 0; d < ND; ++d) {
+        const int row = lg * 4 + (l16 >> 2);  // of this half of 16 keys
+        const int piece = (wid * ND + d) * 2 + (l16 >> 1 & 1);
+        const char* src = vt + (x * 32 + row) * VP * 16 +
+                          dt_place<VP, INROW>(row, piece) * 16 + (l16 & 1) * 8;
+        const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(INROW ? src - KB : src));
+        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(
+                (INROW ? src - KB : src) + 16 * VP * 16));
+        v[d] = __builtin_bit_cast(
+            bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
       }
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              v[d], __builtin_bit_cast(bf16x8_t, w[i]), o[d], 0, 0, 0);
     }
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-      const int row = lg * 4 + (l16 >> 2);  // of each half of 16 keys
-      const int piece = (wid * ND + d) * 2 + (l16 >> 1 & 1);
-      const char* src = (INROW ? kt : vt) + row * VP * 16 +
-                        dt_place<VP, INROW>(row, piece) * 16 + (l16 & 1) * 8;
-      const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) s16x4*)src);
-      const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) s16x4*)(src + 16 * VP * 16));
-      v[d] = __builtin_bit_cast(
-          bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int d = 0; d < ND; ++d)
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            v[d], __builtin_bit_cast(bf16x8_t, w[i]), o[d], 0, 0, 0);
   }
 
   l += __shfl_xor(l, 16, WAVE);
@@ -964,7 +971,7 @@ __global__ __launch_bounds__(128) void attn_decode_merge_kernel(
   }
 }
 
-// head sizes (keys, values), keys that a block takes at once, values within the keys' rows
+// head sizes (keys, values), keys of a tile, values within the keys' rows
 #define DT_SIZES(DO)                                                         \
   DO(64, 64, 64, false) DO(128, 128, 64, false) DO(192, 128, 32, false)      \
   DO(256, 256, 64, false) DO(576, 512, 32, true)
@@ -977,7 +984,7 @@ extern "C" int attn_decode_tile(int G, int Dk, int Dv, bool inrow) {
   return 0;
 }
 
-template <int DK, int DV, bool INROW>
+template <int DK, int DV, int KT, bool INROW>
 static void attn_decode_tile_go(const DecodeArgs& a, int B, hipStream_t stream) {
   const dim3 grid((unsigned)(B * a.Hkv), (unsigned)a.nsplit), block(AD_BLOCK);
   if constexpr (DK == DV) {
@@ -992,7 +999,7 @@ static void attn_decode_tile_go(const DecodeArgs& a, int B, hipStream_t stream) 
     if (a.tickets) go(&attn_decode_wave_kernel<DK, NB, true>);
     else go(&attn_decode_wave_kernel<DK, NB, false>);
   } else {
-    attn_decode_tile_kernel<DK, DV, INROW><<<grid, block, 0, stream>>>(a);
+    attn_decode_tile_kernel<DK, DV, KT, INROW><<<grid, block, 0, stream>>>(a);
   }
   if (a.tickets) return;
   if (a.nsplit > 1 && a.out)
@@ -1005,7 +1012,7 @@ static void attn_decode_tile_size(const DecodeArgs& a, int B, int Dk, int Dv, bo
                                   hipStream_t stream) {
 #define DT_GO(K, V, T, R)                         \
   if (Dk == K && Dv == V && inrow == R)           \
-    attn_decode_tile_go<K, V, R>(a, B, stream);
+    attn_decode_tile_go<K, V, T, R>(a, B, stream);
   DT_SIZES(DT_GO)
 #undef DT_GO
 }
