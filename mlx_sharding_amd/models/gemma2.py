@@ -64,7 +64,7 @@ class Gemma2Attention(nn.Module):
         out = None
         if T == 1 and type(cache) is KVCache:  # others append by methods of their own
             out = cache.attend_step(q, k, v, cos, sin, self.scale, self.softcap,
-                                    self.sliding_window)
+                                    self.sliding_window, faster=True)
         if out is not None:
             return self.o_proj(out)
         if cache is not None and ops.use_native(x):

@@ -71,7 +71,7 @@ class LlamaAttention(nn.Module):
         gp = None
         out = None
         if T == 1 and type(cache) is KVCache:  # others append by methods of their own
-            out = cache.attend_step(q, k, v, cos, sin, self.scale)
+            out = cache.attend_step(q, k, v, cos, sin, self.scale, faster=True)
         if out is not None:
             pass
         elif cache is not None and ops.use_native(x):

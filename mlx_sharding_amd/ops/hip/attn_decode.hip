@@ -22,6 +22,8 @@
 #include "hip_common.h"
 #include "soft_cap.h"
 
+#include <type_traits>
+
 #define AD_BLOCK 256
 
 // DVT = v-columns per thread (ceil(Dv / AD_BLOCK)): 1 for Dv <= 256,
@@ -376,7 +378,7 @@ extern "C" bool attn_decode_supported_shape(int G, int Dv) {
 // Slices come from the length on the device, so they are even under capture.
 // Measured (before: dot products and sums on the vector units, up to 8 slices of
 // the capacity): 64 sequences of 2049 keys, 32 heads of 128 over 8: 179 -> 98 us
-// (now in the kernel for heads of 64 and 128); one of 1024: 24 -> 7.2; 5 of 5004, 16 heads of 256 over 8, capped: 91 ->
+// (5.5 TB/s); one of 1024: 24 -> 7.2; 5 of 5004, 16 heads of 256 over 8, capped: 91 ->
 // 45; 16 heads over a latent of 576/512, 64 x 513 keys: 66 -> 22, 1 x 3002: 75 -> 13.
 // ---------------------------------------------------------------------------
 
@@ -404,8 +406,9 @@ struct DecodeArgs {
 };
 
 // Keys and values are read once: as a stream (2) they leave the L2 to what is read again
-// (64 x 2049 keys 109 -> 101 us, 5 x 5004 of 256 46.5 -> 45.5; latents 16.4 -> 16.8, and
-// stay as they were).
+// (64 x 2049 keys 109 -> 101 us, 5 x 5004 of 256 46.5 -> 45.5).  Not by the tiles of a
+// block, which few of them come to and to which they may come out of the L2 (latents 16.4
+// -> 16.8 as a stream, 512 keys of heads of 64 5.6 -> 5.8).
 template <bool STREAM>
 __device__ __forceinline__ void dt_to_lds(const char* src, char* dst) {
   __builtin_amdgcn_global_load_lds(
@@ -518,42 +521,68 @@ __device__ __forceinline__ void finish_slice(const DecodeArgs& a, const f32x4 (&
       __hip_atomic_store(a.tickets + blockIdx.x, 0u, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
     typedef float f32x2 __attribute__((ext_vector_type(2)));
-    for (int i = threadIdx.x; i < G * (DV / 4); i += blockDim.x) {
-      const int g = i / (DV / 4), c = i % (DV / 4) * 4;
-      const long p0 = (row0 + g) * a.nsplit;
-      float top = -1e30f, all = 0.0f;
-      f32x4 sum = {0, 0, 0, 0};
-      for (int n0 = 0; n0 < slices; n0 += 16) {  // many at once, with their weights
-        u64x2 v[16];
-        f32x2 ml[16];
+    const int items = G * (DV / 4);  // four columns of a head
+    // a thread asks for 16 partial results at once, with their weights: those of so many
+    // slices and of as many items as that leaves
+    auto merge = [&](auto at_once) {
+      constexpr int PER = decltype(at_once)::value, AT = 16 / PER;
+      for (int i0 = threadIdx.x; i0 < items; i0 += blockDim.x * AT) {
+        float top[AT], all[AT];
+        f32x4 sum[AT];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const long n = p0 + min(n0 + j, slices - 1);
-          ml[j] = __builtin_bit_cast(f32x2, found(a.part_ml + n * 2));
-          const float* at = a.part_o + n * DV + c;
-          v[j] = u64x2{found(at), found(at + 2)};
+        for (int t = 0; t < AT; ++t) {
+          top[t] = -1e30f;
+          all[t] = 0.0f;
+          sum[t] = f32x4{0, 0, 0, 0};
         }
-        __builtin_amdgcn_sched_barrier(0);
-        float most = top;
+        for (int n0 = 0; n0 < slices; n0 += PER) {
+          u64x2 v[AT][PER];
+          f32x2 ml[AT][PER];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) most = fmaxf(most, ml[j][0]);
-        const float keep = __builtin_amdgcn_exp2f(top - most);
-        top = most;
-        all *= keep;
+          for (int t = 0; t < AT; ++t) {
+            const int i = min(i0 + t * (int)blockDim.x, items - 1);
+            const long p0 = (row0 + i / (DV / 4)) * a.nsplit;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sum[r] *= keep;
+            for (int j = 0; j < PER; ++j) {
+              const long n = p0 + min(n0 + j, slices - 1);
+              ml[t][j] = __builtin_bit_cast(f32x2, found(a.part_ml + n * 2));
+              const float* at = a.part_o + n * DV + i % (DV / 4) * 4;
+              v[t][j] = u64x2{found(at), found(at + 2)};
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          if (n0 + j >= slices) continue;
-          const f32x4 f = __builtin_bit_cast(f32x4, v[j]);
-          const float by = __builtin_amdgcn_exp2f(ml[j][0] - top);
-          all += ml[j][1] * by;
+          for (int t = 0; t < AT; ++t) {
+            float most = top[t];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) sum[r] += f[r] * by;
+            for (int j = 0; j < PER; ++j) most = fmaxf(most, ml[t][j][0]);
+            const float keep = __builtin_amdgcn_exp2f(top[t] - most);
+            top[t] = most;
+            all[t] *= keep;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[t][r] *= keep;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+              if (n0 + j >= slices) continue;
+              const f32x4 f = __builtin_bit_cast(f32x4, v[t][j]);
+              const float by = __builtin_amdgcn_exp2f(ml[t][j][0] - most);
+              all[t] += ml[t][j][1] * by;
+#pragma unroll
+              for (int r = 0; r < 4; ++r) sum[t][r] += f[r] * by;
+            }
+          }
+        }
+#pragma unroll
+        for (int t = 0; t < AT; ++t) {
+          const int i = i0 + t * (int)blockDim.x;
+          if (i < items)
+            write(row0 + i / (DV / 4), i % (DV / 4) * 4, sum[t], 1.0f / all[t]);
         }
       }
-      write(row0 + g, c, sum, 1.0f / all);
-    }
+    };
+    if (slices > 8) merge(std::integral_constant<int, 16>());
+    else if (slices > 4) merge(std::integral_constant<int, 8>());
+    else merge(std::integral_constant<int, 4>());
   }
 }
 
@@ -592,13 +621,13 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
 #pragma unroll
     for (int i = 0; i < KB / 4096; ++i) {
       const int part = i * 4 + wid, s = part * 64 + lane, row = s / KP;
-      dt_to_lds<!INROW>(ks + min(row, last) * (DK * 2) +
+      dt_to_lds<false>(ks + min(row, last) * (DK * 2) +
                     dt_place<KP, true>(row, s % KP) * 16, dst + part * 1024);
     }
 #pragma unroll
     for (int i = 0; i < VB / 4096; ++i) {
       const int part = i * 4 + wid, s = part * 64 + lane, row = s / VP;
-      dt_to_lds<!INROW>(vs + min(row, last) * (DV * 2) +
+      dt_to_lds<false>(vs + min(row, last) * (DV * 2) +
                     dt_place<VP, false>(row, s % VP) * 16,
                 dst + KB + part * 1024);
     }
@@ -716,7 +745,8 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
   finish_slice<DV, false>(a, o, m, l, row0, G, wid, l16, lg, a.nsplit);
 }
 
-// Heads of 64, 128 and 256.  A wave has tiles of 32 keys of its own, which go to its own LDS,
+// Whole steps of heads of 64, 128 and 256, and attention alone where there is much of it
+// (attn_decode_wave).  A wave has tiles of 32 keys of its own, which go to its own LDS,
 // NB of them by turns, and keeps outputs of all columns: scores come out of the first
 // product as the second one takes them, so that waves meet at the end of a slice only, and
 // each makes its own keys' weights.  In the kernel above a tile's scores pass two barriers
@@ -726,9 +756,9 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
 // keys ahead of its values gain nothing).
 // STEP: queries and the token's key are turned here, its key and value go to the cache
 // and into the last tile, and the last block of a head merges the slices.  The chain
-// through memory to that block takes what the merging kernel took (5 us), the rotations
-// 2 to 3 instead of 4.6 in a kernel of their own: one sequence of 1024 keys, 32 heads of
-// 128 over 8, 14.1 -> 9.6 us for the three.
+// through memory to that block takes 3 us and 1.3 for what a thread asks for at once, the
+// merging kernel 4.5; the rotations 2 to 3 instead of 4.6 in a kernel of their own: one
+// sequence of 1024 keys, 32 heads of 128 over 8, 14.1 -> 9.6 us for the three.
 #define DW_WAVES 2
 template <int D, int NB, bool STEP>
 __global__ __launch_bounds__(DW_WAVES* WAVE) void attn_decode_wave_kernel(
@@ -974,7 +1004,7 @@ __global__ __launch_bounds__(128) void attn_decode_merge_kernel(
 // head sizes (keys, values), keys of a tile, values within the keys' rows
 #define DT_SIZES(DO)                                                         \
   DO(64, 64, 64, false) DO(128, 128, 64, false) DO(192, 128, 32, false)      \
-  DO(256, 256, 64, false) DO(576, 512, 32, true)
+  DO(256, 256, 32, false) DO(576, 512, 32, true)
 
 extern "C" int attn_decode_tile(int G, int Dk, int Dv, bool inrow) {
   if (G > 16) return 0;
@@ -984,24 +1014,36 @@ extern "C" int attn_decode_tile(int G, int Dk, int Dv, bool inrow) {
   return 0;
 }
 
+// Whether attention alone has tiles of a wave.  The kernel's two waves a block are longer at
+// one tile of keys, and read faster where a CU has many.  Time of a wave's tiles over a
+// block's, by tiles of 64 keys of all pairs: heads of 64, below 64 of them 1.05, 128 to
+// 255 .99, above 512 .95 and less; of 128, below 32 1.09, 256 to 511 1.00, above 512 .96, above
+// 2048 .85; of 256 1.1 and more for most.
+extern "C" bool attn_decode_wave(int D, long pairs, long span) {
+  const long tiles = pairs * ((span + 63) / 64);
+  return D == 64 ? tiles >= 128 : D == 128 && tiles >= 512;
+}
+
+// wave: tiles of a wave, also for a call that is not a whole step
 template <int DK, int DV, int KT, bool INROW>
-static void attn_decode_tile_go(const DecodeArgs& a, int B, hipStream_t stream) {
+static void attn_decode_tile_go(const DecodeArgs& a, int B, bool wave, hipStream_t stream) {
   const dim3 grid((unsigned)(B * a.Hkv), (unsigned)a.nsplit), block(AD_BLOCK);
   if constexpr (DK == DV) {
     // a wave's tiles: 32 KB, of heads of 256 twice that
     constexpr int NB = DK < 256 ? 256 / DK : 2, smem = DW_WAVES * NB * 2 * 32 * DK * 2;
-    const dim3 two(DW_WAVES * WAVE);
     auto go = [&](auto kernel) {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-      kernel<<<grid, two, smem, stream>>>(a);
+      kernel<<<grid, dim3(DW_WAVES * WAVE), smem, stream>>>(a);
     };
-    if (a.tickets) go(&attn_decode_wave_kernel<DK, NB, true>);
-    else go(&attn_decode_wave_kernel<DK, NB, false>);
-  } else {
-    attn_decode_tile_kernel<DK, DV, KT, INROW><<<grid, block, 0, stream>>>(a);
+    if (a.tickets) return go(&attn_decode_wave_kernel<DK, NB, true>);
+    if constexpr (DK < 256) {
+      if (wave) go(&attn_decode_wave_kernel<DK, NB, false>);
+    } else {
+      wave = false;
+    }
   }
-  if (a.tickets) return;
+  if (!wave) attn_decode_tile_kernel<DK, DV, KT, INROW><<<grid, block, 0, stream>>>(a);
   if (a.nsplit > 1 && a.out)
     attn_decode_merge_kernel<<<dim3((unsigned)(B * a.Hq)), dim3(128), 0,
                                stream>>>(a.part_o, a.part_ml, (short*)a.out,
@@ -1009,10 +1051,10 @@ static void attn_decode_tile_go(const DecodeArgs& a, int B, hipStream_t stream) 
 }
 
 static void attn_decode_tile_size(const DecodeArgs& a, int B, int Dk, int Dv, bool inrow,
-                                  hipStream_t stream) {
+                                  bool wave, hipStream_t stream) {
 #define DT_GO(K, V, T, R)                         \
   if (Dk == K && Dv == V && inrow == R)           \
-    attn_decode_tile_go<K, V, T, R>(a, B, stream);
+    attn_decode_tile_go<K, V, T, R>(a, B, wave, stream);
   DT_SIZES(DT_GO)
 #undef DT_GO
 }
@@ -1021,12 +1063,12 @@ static void attn_decode_tile_size(const DecodeArgs& a, int B, int Dk, int Dv, bo
 extern "C" void launch_attn_decode_tile(
     const void* q, const void* k, const void* v, void* out, float* part_o,
     float* part_ml, int nsplit, const int* s_ptr, int B, int Hq, int Hkv, int S,
-    long Scap, int Dk, int Dv, bool inrow, float scale, float softcap,
+    long Scap, int Dk, int Dv, bool inrow, bool wave, float scale, float softcap,
     int window, hipStream_t stream) {
   const DecodeArgs a{(const char*)q, (const char*)k, (const char*)v, (char*)out,
                      part_o, part_ml, s_ptr, Hq, Hkv, S, nsplit, window, Scap,
                      soft_cap(scale, softcap)};
-  attn_decode_tile_size(a, B, Dk, Dv, inrow, stream);
+  attn_decode_tile_size(a, B, Dk, Dv, inrow, wave, stream);
 }
 
 // A step of one token per sequence: rows of q, k and v with strides of qs, ks and vs
@@ -1044,5 +1086,5 @@ extern "C" void launch_attn_step(const void* q, const void* k, const void* v, lo
                      part_o, part_ml, s_ptr, Hq, Hkv, S, nsplit, window, Scap,
                      soft_cap(scale, softcap), (const char*)k, (const char*)v, qs, ks, vs,
                      cos, sin, tickets};
-  attn_decode_tile_size(a, B, D, D, false, stream);
+  attn_decode_tile_size(a, B, D, D, false, true, stream);
 }

@@ -46,8 +46,9 @@ bool attn_decode_supported_shape(int, int);
 int attn_decode_tile(int, int, int, bool);
 void launch_attn_decode_tile(const void*, const void*, const void*, void*,
                              float*, float*, int, const int*, int, int, int,
-                             int, long, int, int, bool, float, float, int,
+                             int, long, int, int, bool, bool, float, float, int,
                              hipStream_t);
+bool attn_decode_wave(int, long, long);
 void launch_attn_step(const void*, const void*, const void*, long, long, long,
                       const float*, const float*, void*, void*, void*, float*, float*,
                       unsigned*, int, const int*, int, int, int, int, long, int, float,
@@ -436,7 +437,7 @@ void mla_append_kv(torch::Tensor kvh, torch::Tensor kpe, torch::Tensor kcache,
 // all at work at once, and no slice under one tile.  256 blocks leave half of the
 // loads in flight unused (5 sequences of 5004 keys, 8 heads of 256: 68 us, 45 with
 // 512), 1024 come in two rounds and double what the merge reads (48 us; 64 cached
-// latents of 2048 tokens: 49 us, 40 with 512).  Of heads of 256 a CU has one block.
+// latents of 2048 tokens: 49 us, 40 with 512).  Whole steps of heads of 256 have one a CU.
 static int decode_slices(long pairs, long span, int tile, int blocks = 512) {
   return (int)std::max<long>(
       1, std::min<long>({64, blocks / std::max<long>(pairs, 1),
@@ -483,8 +484,11 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                        ? attn_decode_tile(Hq / Hkv, Dk, Dv, inrow)
                        : 0;
   if (tile) {
-    const int nsplit = decode_slices((long)B * Hkv, s_ptr ? kScap : (long)S, tile,
-                                     Dk == 256 ? 256 : 512);
+    const long keys = s_ptr ? kScap : (long)S;
+    const bool wave = Dk == Dv && attn_decode_wave(Dk, (long)B * Hkv,
+                                                   window > 0 ? std::min(keys, (long)window)
+                                                              : keys);
+    const int nsplit = decode_slices((long)B * Hkv, keys, tile);
     torch::Tensor po, pml;
     if (nsplit > 1) {
       po = torch::empty({(long)B * Hq * nsplit * Dv}, fopts);
@@ -494,7 +498,7 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
         qc.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
         nsplit > 1 ? po.data_ptr<float>() : nullptr,
         nsplit > 1 ? pml.data_ptr<float>() : nullptr, nsplit, s_ptr, B, Hq, Hkv,
-        S, kScap, Dk, Dv, inrow, (float)scale, (float)softcap, (int)window,
+        S, kScap, Dk, Dv, inrow, wave, (float)scale, (float)softcap, (int)window,
         cur_stream());
     return out;
   }
@@ -530,7 +534,7 @@ c10::optional<torch::Tensor> attn_step(
     torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor cos,
     torch::Tensor sin, torch::Tensor kcache, torch::Tensor vcache,
     c10::optional<torch::Tensor> pos, int64_t pos0, torch::Tensor tickets, double scale,
-    double softcap, int64_t window) {
+    double softcap, int64_t window, bool faster) {
   if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || kcache.dim() != 4 ||
       q.size(1) != 1)
     return c10::nullopt;
@@ -567,9 +571,26 @@ c10::optional<torch::Tensor> attn_step(
   } else {
     TORCH_CHECK(pos0 >= 0 && pos0 < cap, "no room in the cache");
   }
-  const int tile = attn_decode_tile((int)(Hq / Hkv), (int)D, (int)D, false);
-  const int nsplit = decode_slices(B * Hkv, s_ptr ? cap : pos0 + 1, tile,
-                                   D == 256 ? 256 : 512);
+  // The last block of a head's merges its slices, 16 partial results a thread at once, a
+  // chain of 1.3 us (heads of 256: 2.4), where the kernel of its own takes 4.5 us for any
+  // number of them.  So slices are as many as two chains have, one of heads of 256, and
+  // where that would be less than half of them (of heads of 256: less than all) the
+  // separate kernels are faster; of heads of 256, of which a CU has one block, also for few
+  // pairs and for more than there are CUs.  Sequences x heads over heads of a size, keys:
+  // us of the separate kernels, of this one with all slices, with as many as here: 1 x 8
+  // over 8 of 128, 3339: 12.1, 15.9, 12.6; 1 x 32 over 8 of 128, 1970: 11.9, 12.2, 11.9;
+  // 1 x 128 over 8 of 128, 757: 10.8, 13.5, 11.2; 5 x 16 over 1 of 256, 226: 11.8, 22.0;
+  // 35 x 32 over 8 of 256, 89: 15.1, 21.8.  Of 1200 random sizes in captured steps 720
+  // come here and take .73 of the separate kernels' time, 63 of them 3 to 16% more.  An
+  // eager call takes the host 8 us and 15.8 for the separate ones, and so few keys of
+  // heads of 256 (24: 7.1 us here, 5.8 there) come here, too.
+  const bool wide = D == 256;
+  const long pairs = B * Hkv, chains = (Hq / Hkv * D + 511) / 512;
+  const int most = std::max<int>(1, (wide ? 16 : 32) / chains);
+  const int slices = decode_slices(pairs, s_ptr ? cap : pos0 + 1, 64, wide ? 256 : 512);
+  if (faster && (wide ? slices > most || pairs < 8 || pairs > 256 : slices > 2 * most))
+    return c10::nullopt;
+  const int nsplit = std::min(slices, most);
   auto out = torch::empty({B, 1, Hq * D}, q.options());
   torch::Tensor part;
   if (nsplit > 1)
@@ -667,7 +688,7 @@ torch::Tensor mla_attend(torch::Tensor q, torch::Tensor cache, torch::Tensor w,
   launch_attn_decode_tile(q.data_ptr(), cache.data_ptr(), cache.data_ptr(), nullptr,
                           po.data_ptr<float>(), pml.data_ptr<float>(), n, s_ptr,
                           (int)N, (int)heads, 1, (int)S, cache.size(2), (int)D,
-                          (int)rank, true, (float)scale, 0.0f, 0, cur_stream());
+                          (int)rank, true, false, (float)scale, 0.0f, 0, cur_stream());
   auto out = torch::empty({N, heads * vdim}, q.options());
   const MlaFinishArgs a{po.data_ptr<float>(), pml.data_ptr<float>(),
                         (const __bf16*)w.data_ptr(), (__bf16*)out.data_ptr(), (int)N,

@@ -110,9 +110,11 @@ class KVCache:
 
     def attend_step(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                     cos: torch.Tensor, sin: torch.Tensor, scale: float,
-                    softcap: float = 0.0, window: int = 0) -> Optional[torch.Tensor]:
+                    softcap: float = 0.0, window: int = 0,
+                    faster: bool = False) -> Optional[torch.Tensor]:
         """append_rope_qkv of one token per sequence and its attention in one kernel:
-        [B, 1, heads * D]; None (and nothing appended) where that does not take it."""
+        [B, 1, heads * D]; None (and nothing appended) where that does not take it, or,
+        asked for what is ``faster``, where the separate kernels are."""
         from .. import ops as _ops
         if not (self.dtype == torch.bfloat16 and k.shape[1] == 1
                 and self.k_head_dim == self.v_head_dim == k.shape[3]
@@ -124,7 +126,7 @@ class KVCache:
                 return None  # the zeros would be written by replays only
             self._make_tickets()
         out = _ops.hip_ext().attn_step(q, k, v, cos, sin, self._k, self._v, pos, at,
-                                       self._tickets, scale, softcap, window)
+                                       self._tickets, scale, softcap, window, faster)
         if out is not None:
             self.wrote(1)
         return out

@@ -143,3 +143,50 @@ def test_replays():
             c._v[:, :, p - 6: p] = -0.5
         torch.cuda.synchronize()
     assert not one._tickets.any()
+
+
+# partial results merged 4, 8 and 16 slices at once: fewer items than threads, a
+# remainder, eight a thread; slices of a batch and one more
+@pytest.mark.parametrize("B,Hq,Hkv,D,keys", [
+    (1, 3, 1, 64, 200), (1, 3, 1, 64, 300), (1, 6, 2, 64, 1100), (1, 14, 2, 128, 250),
+    (1, 14, 2, 128, 500), (2, 16, 1, 128, 257), (1, 32, 2, 128, 1500), (1, 16, 1, 256, 65),
+    (1, 7, 1, 256, 300), (9, 16, 8, 256, 700)])
+def test_merges(B, Hq, Hkv, D, keys):
+    g = torch.Generator("cuda").manual_seed(keys)
+    one, _ = _caches(B, Hkv, D, keys - 1, keys, False, g)
+    (q, k, v), cos, sin = _token(B, Hq, Hkv, D, g)
+    got = one.attend_step(q, k, v, cos, sin, 0.1)
+    exact = _exact(q, cos, sin, one.k, one.v, 0.0, 0)
+    assert float((got.double() - exact).norm() / exact.norm()) < 2e-3  # as above
+    assert not one._tickets.any()
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,keys,taken", [
+    (1, 4, 1, 128, 8000, True), (1, 8, 1, 128, 2048, True), (1, 8, 1, 128, 2049, False),
+    (1, 16, 1, 128, 1024, True), (1, 16, 1, 128, 1025, False), (1, 8, 8, 256, 1024, True),
+    (1, 8, 8, 256, 1025, False), (1, 4, 4, 256, 100, False), (32, 8, 8, 256, 40, True),
+    (33, 8, 8, 256, 40, False)])
+def test_where_it_is_faster(B, Hq, Hkv, D, keys, taken):
+    g = torch.Generator("cuda").manual_seed(keys)
+    one, _ = _caches(B, Hkv, D, keys - 1, keys, False, g)
+    (q, k, v), cos, sin = _token(B, Hq, Hkv, D, g)
+    got = one.attend_step(q, k, v, cos, sin, 0.1, faster=True)
+    assert (got is not None) == taken and one.offset == (keys if taken else keys - 1)
+    assert one.attend_step(q, k, v, cos, sin, 0.1) is not None
+
+
+# a wave's own tiles from 128 tiles of 64 keys of heads of 64 on, 512 of 128; before, and
+# for heads of 256, tiles of a block
+@pytest.mark.parametrize("B,Hq,Hkv,D,keys", [
+    (4, 16, 4, 64, 448), (4, 16, 4, 64, 449), (16, 32, 8, 128, 192), (16, 32, 8, 128, 193),
+    (64, 16, 8, 128, 64), (16, 8, 4, 256, 511)])
+@pytest.mark.parametrize("window", [0, 100])
+def test_attention_alone(B, Hq, Hkv, D, keys, window):
+    g = torch.Generator("cuda").manual_seed(keys)
+    new = lambda h, s: torch.randn(B, h, s, D, generator=g, device="cuda").bfloat16()  # noqa: E731
+    q, k, v = new(Hq, 1), new(Hkv, keys), new(Hkv, keys)
+    got = ops.attention(q, k, v, 0.1, sliding_window=window)
+    one, zero = torch.ones(1, D // 2, device="cuda"), torch.zeros(1, D // 2, device="cuda")
+    exact = _exact(q.transpose(1, 2), one, zero, k, v, 0.0, window)
+    got = got.transpose(1, 2).reshape(B, 1, -1)
+    assert float((got.double() - exact).norm() / exact.norm()) < 2e-3  # as above
