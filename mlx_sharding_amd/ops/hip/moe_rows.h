@@ -18,7 +18,9 @@ struct MoeRowsArgs {
   const __bf16 *dx, *dw;
   __bf16* dy;
   int dense, N, DO, DK;
+  unsigned by_blocks, by_rows;  // reciprocals that launch_moe_rows fills in
 };
+static_assert(sizeof(MoeRowsArgs) <= 128, "two lines");
 
 struct MoeRouteArgs {
   const __bf16 *x, *residual, *norm, *gate;  // rows [N, H], [H], [E, H]

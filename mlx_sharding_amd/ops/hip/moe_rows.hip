@@ -108,7 +108,11 @@ struct Packed {
         const bool up = BITS == 4 && (j & 1);
         const unsigned word = BITS == 4 ? u[i] >> (8 * (j / 2))
                                         : u[2 * i + j / 2] >> (8 * (j & 1));
-        const unsigned v = masked(word, up ? LOW << 4 : LOW, up ? 0x54005400u : 0x64006400u);
+        // (of 8 bits the compiler's two are the faster ones: one token, 8 experts of 512 x
+        // 1024 5.9 us, 5.6 so)
+        const unsigned v =
+            BITS == 8 ? (word & LOW) | 0x64006400u
+                      : masked(word, up ? LOW << 4 : LOW, up ? 0x54005400u : 0x64006400u);
         const _Float16 c = (_Float16)((up ? -64.0f : -1024.0f) - MID);
         const f16x2 f =
             (__builtin_bit_cast(f16x2, v) + f16x2{c, c}) * s2 + b2;
@@ -134,13 +138,15 @@ __device__ __forceinline__ void dense_tiles(const MoeRowsArgs& a, f32x4* red) {
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l16 = lane & 15, lg = lane >> 4;
   auto load = [](const __bf16* p) { return *reinterpret_cast<const bf16x8_t*>(p); };
-  const __bf16* xp = a.dx + (long)min(l16, a.N - 1) * a.DK + lg * 8;
+  // places within x and w in 32 bits (sizes are up to 4096): pointers were one register
+  // too many
+  const unsigned xp = min(l16, a.N - 1) * a.DK + lg * 8;
   const int t = blockIdx.x;
-  const __bf16* wp[MATS];
+  unsigned wp[MATS];
   f32x4 acc[MATS];
 #pragma unroll
   for (int m = 0; m < MATS; ++m) {
-    wp[m] = a.dw + ((long)m * a.DO + t * 16 + l16) * a.DK + lg * 8;
+    wp[m] = (unsigned)(m * a.DO + t * 16 + l16) * a.DK + lg * 8;
     acc[m] = f32x4{0, 0, 0, 0};
   }
   // three ahead: what a wave has of 2048 columns is four
@@ -153,9 +159,9 @@ __device__ __forceinline__ void dense_tiles(const MoeRowsArgs& a, f32x4* red) {
 #pragma unroll
     for (int m = 0; m < MATS; ++m)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) f.w[m][i] = load(wp[m] + k + i * 32);
+      for (int i = 0; i < 2; ++i) f.w[m][i] = load(a.dw + (wp[m] + k + i * 32));
 #pragma unroll
-    for (int i = 0; i < 2; ++i) f.x[i] = load(xp + k + i * 32);
+    for (int i = 0; i < 2; ++i) f.x[i] = load(a.dx + (xp + k + i * 32));
   };
   constexpr int STEP = MR_WAVES * 64;
 #pragma unroll
@@ -200,21 +206,32 @@ __device__ __forceinline__ void dense_tiles(const MoeRowsArgs& a, f32x4* red) {
 // Work is counted in tiles: 16 rows of an expert's matrices by up to 16 of its pairs.
 // Every block counts the pairs of all experts and takes an even share of all tiles, one
 // after the other.  With a block per expert and range of rows the longest one has the
-// expert with most pairs (64 experts of 1408 x 2048 at 4 bits, 64 tokens: an expert has 12
-// of them 91 us so, 90 shared; 52 179, 70; 128 tokens, 22 126, 112; one token 18.3, 20.2,
-// which is the counting).  Choices stay in LDS for the search of an expert's pairs, which
-// goes through them one load after the other otherwise (64 tokens, both products: 97 us
-// from memory, 92 so).
-template <int BITS, int GS, int UPW, bool UP>
+// expert with most pairs (both products of 64 experts of 1408 x 2048 at 4 bits: 64 tokens
+// 94.9 us so, 86.9 shared; 128 130.7, 95.9; one, whose choices are counted first, 19.8,
+// 17.5).  Choices stay in LDS for the search of an expert's pairs, which goes through
+// them one load after the other otherwise (64 tokens, both products: 97 us from memory,
+// 92 so).  Up to 64 pairs are a lane each of one wave, which finds those of an expert by
+// ballots (one token 19.4 us by counts in LDS, 17.5 so; 32 pairs of 64 experts of 256 x
+// 512 10.9 and, with shares that end with a group, 8.7; a block per expert 8.1).  What
+// that is slower than a block per expert, up to 1 us for both products of small experts,
+// is the counting.
+template <int BITS, int UPW, bool UP>
+constexpr bool two_a_cu() {
+  return UPW <= (BITS == 16 && UP ? 1 : 2);
+}
+
+// FEW: up to 64 pairs
+template <int BITS, int GS, int UPW, bool UP, bool FEW>
 __global__ __launch_bounds__(
-    MR_BLOCK, UPW <= (BITS == 16 && UP ? 1 : 2) ? 4 : 2) void moe_rows_kernel(
+    MR_BLOCK, (two_a_cu<BITS, UPW, UP>() ? 4 : 2)) void moe_rows_kernel(
     const MoeRowsArgs a) {
   typedef Operand<BITS> Op;
   typedef typename Op::V V;
   constexpr int MATS = UP ? 2 : 1;
   __shared__ int count[64], ends[64];
+  __shared__ unsigned long long members[FEW ? 64 : 1];  // of the pairs, those of an expert
   __shared__ short list[16];
-  __shared__ unsigned char chosen[MR_PAIRS];  // experts, 255: none
+  __shared__ unsigned char chosen[FEW ? 1 : MR_PAIRS];  // experts, 255: none
   __shared__ __attribute__((aligned(16))) f32x4 red[2][MR_WAVES][MATS][WAVE];
 
   if ((int)blockIdx.x < a.dense) {
@@ -225,28 +242,67 @@ __global__ __launch_bounds__(
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l16 = lane & 15, lg = lane >> 4;
   const int rows = a.O / 16;
-  if (threadIdx.x < 64) count[threadIdx.x] = 0;
-  __syncthreads();
-  for (int i = threadIdx.x; i < a.pairs; i += MR_BLOCK) {
-    const unsigned e = a.choice[i];
-    chosen[i] = (unsigned char)min(e, 255u);
-    if (e < (unsigned)a.experts) atomicAdd(&count[e], 1);
-  }
-  __syncthreads();
-  if (wid == 0) {
-    int n = (count[lane] + 15) / 16;  // groups of pairs up to this expert
+  // of the lanes up to this one the sum of (n + 15) / 16, which is below 2^PLANES: groups
+  // of pairs up to a lane's expert
+  auto groups_up_to = [&](int n) {
+    constexpr int PLANES = FEW ? 3 : 7;
+    const unsigned long long upto = ~0ull >> (WAVE - 1 - lane);
+    const int g = (n + 15) / 16;
+    int sum = 0;
 #pragma unroll
-    for (int off = 1; off < WAVE; off <<= 1) {
-      const int o = __shfl_up(n, off, WAVE);
-      if (lane >= off) n += o;
+    for (int b = 0; b < PLANES; ++b) sum += __popcll(__ballot(g >> b & 1) & upto) << b;
+    return sum;
+  };
+  // An entry per expert; FEW: per pair, of which the first of its expert counts, and what
+  // it holds comes by ballots of one wave.
+  if constexpr (FEW) {
+    if (wid == 0) {
+      const unsigned e = lane < a.pairs ? a.choice[lane] : 255u;
+      unsigned long long same = __ballot(e < (unsigned)a.experts);
+#pragma unroll
+      for (int b = 0; b < 6; ++b) {
+        const bool bit = e >> b & 1;
+        const unsigned long long with = __ballot(bit);
+        same &= bit ? with : ~with;
+      }
+      const bool leads = e < (unsigned)a.experts && __ffsll(same) - 1 == lane;
+      ends[lane] = groups_up_to(leads ? __popcll(same) : 0);
+      count[lane] = e;
+      members[lane] = same;
     }
-    ends[lane] = n;
+  } else {
+    if (threadIdx.x < 64) count[threadIdx.x] = 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < a.pairs; i += MR_BLOCK) {
+      const unsigned e = a.choice[i];
+      chosen[i] = (unsigned char)min(e, 255u);
+      if (e < (unsigned)a.experts) atomicAdd(&count[e], 1);
+    }
+    __syncthreads();
+    if (wid == 0) ends[lane] = groups_up_to(count[lane]);
   }
   __syncthreads();
-  const unsigned all = ends[63] * rows, blocks = gridDim.x - a.dense;
-  const unsigned b = blockIdx.x - a.dense;
-  int at = b * all / blocks;
-  const int stop = (b + 1) * all / blocks;
+  const unsigned groups = __builtin_amdgcn_readfirstlane(ends[WAVE - 1]), all = groups * rows;
+  // This block's share of them.  `per` is the largest share that there has to be: with as
+  // many rows to every block of a group, and fewer to its last one, where that takes no more
+  // blocks, so that no block begins twice; else all / blocks or one more, from 0 to `all`
+  // over all blocks.  Divisions are multiplications by reciprocals: exact ones, but that of
+  // the last way.
+  auto over = [](unsigned x, unsigned n) {  // below 2^16
+    return (unsigned)(((float)x + 0.5f) * __builtin_amdgcn_rcpf((float)n));
+  };
+  const unsigned b = blockIdx.x - a.dense, blocks = gridDim.x - a.dense;
+  const unsigned per = max(1u, __umulhi(all + blocks - 1, a.by_blocks));
+  const unsigned parts = over(rows + per - 1, per);
+  int at, stop;
+  if (groups * parts <= blocks) {
+    const unsigned group = over(b, parts);
+    at = min(group, groups) * rows + (b - group * parts) * per;
+    stop = group < groups ? min((group + 1) * rows, at + per) : at;
+  } else {
+    at = __umulhi(b * all, a.by_blocks);
+    stop = __umulhi((b + 1) * all, a.by_blocks);
+  }
 
   const int units = a.K / MR_UNIT;
   const int k0 = wid * MR_UNIT + lg * 32;
@@ -257,12 +313,14 @@ __global__ __launch_bounds__(
   int buf = 0;
   while (at < stop) {
     // one group of one expert's pairs, rows t0 to t1
-    const int group = at / rows, t0 = at - group * rows;
+    const int group = __umulhi(at, a.by_rows), t0 = at - group * rows;
     const int t1 = min(rows, t0 + stop - at);
     at += t1 - t0;
-    const int e = __popcll(__ballot(ends[lane] <= group));
-    const int first = (group - (e ? ends[e - 1] : 0)) * 16;
-    const int n = min(16, count[e] - first);
+    const int place = __popcll(__ballot(ends[lane] <= group));
+    auto same = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    const int first = (group - (place ? same(ends[place - 1]) : 0)) * 16;
+    const int e = FEW ? same(count[place]) : place;
+    const int n = min(16, same(FEW ? __popcll(members[place]) : count[place]) - first);
 
     // this lane's place in its first unit of the first rows
     const long begin = ((long)e * rows + t0) * step +
@@ -281,18 +339,30 @@ __global__ __launch_bounds__(
 #pragma unroll
       for (int m = 0; m < MATS; ++m) fetch(next[m][u], m, u, 0);
     }
-    if (wid == 0) {
-      int found = -first;
-      for (int i = 0; i < a.pairs && found < 16; i += WAVE) {
-        const bool mine = i + lane < a.pairs && chosen[i + lane] == e;
-        const unsigned long long which = __ballot(mine);
-        const int place = found + __popcll(which & ((1ull << lane) - 1));
-        if (mine && place >= 0 && place < 16) list[place] = (short)(i + lane);
-        found += __popcll(which);
+    int pair;
+    if constexpr (FEW) {
+      // the n pairs from `first` on go to the lowest lanes, the others anywhere else
+      const unsigned long long which = members[place];
+      const int to = __popcll(which & ((1ull << lane) - 1)) - first;
+      const bool listed = (which >> lane & 1) && to >= 0 && to < 16;
+      pair = __builtin_amdgcn_ds_permute((listed ? to : 16 + lane % 48) * 4, lane);
+      pair = __shfl(pair, min(l16, n - 1), WAVE);
+    } else {
+      if (wid == 0) {
+        int found = -first;
+        for (int i = 0; i < a.pairs && found < 16; i += WAVE) {
+          const bool mine = i + lane < a.pairs && chosen[i + lane] == e;
+          const unsigned long long with = __ballot(mine);
+          const int place = found + __popcll(with & ((1ull << lane) - 1));
+          if (mine && place >= 0 && place < 16) list[place] = (short)(i + lane);
+          found += __popcll(with);
+        }
       }
+      __syncthreads();
+      pair = list[min(l16, n - 1)];
     }
-    __syncthreads();
-    const int pair = list[min(l16, n - 1)];
+    // asked for here: behind the products it was waited for
+    const float weight = UP ? 0.0f : a.weight[pair];
     V x[UPW][4];
 #pragma unroll
     for (int u = 0; u < UPW; ++u) {
@@ -356,9 +426,8 @@ __global__ __launch_bounds__(
         }
         *reinterpret_cast<H4*>((typename Op::E*)a.y + to) = h;
       } else {
-        const float w = a.weight[pair];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[0][j] *= w;
+        for (int j = 0; j < 4; ++j) v[0][j] *= weight;
         *reinterpret_cast<f32x4*>((float*)a.y + to) = v[0];
       }
     }
@@ -426,23 +495,44 @@ extern "C" void launch_moe_pack(const void* w, const void* scale,
   }
 }
 
-template <int BITS, int GS, bool UP>
-static void moe_rows_go(const MoeRowsArgs& a, hipStream_t stream) {
+// 2^32 / n, rounded up, for n above 1
+static unsigned reciprocal(unsigned n) {
+  return (unsigned)(((1ull << 32) + n - 1) / n);
+}
+
+template <int BITS, int GS, bool UP, bool FEW>
+static void moe_rows_run(MoeRowsArgs a, hipStream_t stream) {
   // Two blocks a CU, all at work at once (64 tokens, 64 experts, 4 bits: 89 us; 116 with
-  // one, 103 with four), or a tile each where there are fewer.
-  const dim3 grid((unsigned)(
-      a.dense + min(512 - a.dense, a.O / 16 * min(a.experts, a.pairs))));
-  const dim3 block(MR_BLOCK);
+  // one, 103 with four), or a tile each where there are fewer.  One where a CU holds one:
+  // a block without a tile, of which there may be many, is then in the way of one that has
+  // some (6 tokens of 16 experts of 1024 x 3072 in bf16, first product: 384 blocks 30.1
+  // us, 256 18.8).
+  auto go = [&](auto kernel, int resident) {
+    const int tiles = a.O / 16 * min(a.experts, a.pairs);
+    const int room = max(resident - a.dense, resident / 2);
+    const unsigned blocks = min(room, tiles);
+    a.by_blocks = reciprocal(blocks);
+    a.by_rows = reciprocal(a.O / 16);
+    kernel<<<dim3(a.dense + blocks), dim3(MR_BLOCK), 0, stream>>>(a);
+  };
+#define MR_GO(U) go(&moe_rows_kernel<BITS, GS, U, UP, FEW>, two_a_cu<BITS, U, UP>() ? 512 : 256)
   const int upw = (a.K / MR_UNIT + MR_WAVES - 1) / MR_WAVES;
   if (upw <= 1) {
-    moe_rows_kernel<BITS, GS, 1, UP><<<grid, block, 0, stream>>>(a);
+    MR_GO(1);
   } else if (upw <= 2) {
-    moe_rows_kernel<BITS, GS, 2, UP><<<grid, block, 0, stream>>>(a);
+    MR_GO(2);
   } else if (upw <= 3) {
-    moe_rows_kernel<BITS, GS, 3, UP><<<grid, block, 0, stream>>>(a);
+    MR_GO(3);
   } else if constexpr (BITS < 16) {
-    moe_rows_kernel<BITS, GS, 5, UP><<<grid, block, 0, stream>>>(a);
+    MR_GO(5);
   }
+#undef MR_GO
+}
+
+template <int BITS, int GS, bool UP>
+static void moe_rows_go(const MoeRowsArgs& a, hipStream_t stream) {
+  if (a.pairs <= WAVE) moe_rows_run<BITS, GS, UP, true>(a, stream);
+  else moe_rows_run<BITS, GS, UP, false>(a, stream);
 }
 
 // the longest contraction

@@ -50,9 +50,11 @@ def test_shares(N, E, top, I, H, bits, uneven):
 
 
 @pytest.mark.parametrize("N", [1, 7, 8])
-@pytest.mark.parametrize("S,bits", [(64, 4), (576, 16), (4096, 4)])
-def test_shared_beside(N, S, bits):
-    E, top, I, H = 16, 3, 128, 512
+@pytest.mark.parametrize("S,bits,H", [
+    (64, 4, 512), (576, 16, 512), (4096, 4, 512),
+    (4096, 4, 4096)])    # 256 blocks beside, of kernels of which a CU has one block
+def test_shared_beside(N, S, bits, H):
+    E, top, I = 16, 3, 128
     gen = torch.Generator("cuda").manual_seed(N + S)
     randn = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
     g, u = stack(E, I, H, bits, 64, gen)[0], stack(E, I, H, bits, 64, gen)[0]
@@ -80,3 +82,28 @@ def test_shared_apart():
     assert not ops.expert_shared_ok(1, 512, w(2 * 4160, 512), w(512, 4160))
     assert not ops.expert_shared_ok(1, 512, w(256, 512), None)
     assert not ops.expert_shared_ok(1, 512, w(256, 520)[:, :512], w(512, 128))
+
+
+# up to 64 pairs by ballots, more by counts: both sides of the line, groups of one expert
+# that fill up, shares that end with a group (rows a multiple of them) and that do not,
+# blocks with nothing to do
+@pytest.mark.parametrize("N,E,top,I,H,bits", [
+    (64, 3, 1, 128, 384, 4), (65, 3, 1, 128, 384, 4), (32, 64, 2, 384, 640, 8),
+    (33, 64, 2, 384, 640, 8), (16, 64, 4, 1408, 512, 4), (10, 64, 6, 128, 3072, 16),
+    (3, 64, 1, 128, 5120, 4)])
+@pytest.mark.parametrize("spread", [1, 5, 64])
+def test_groups(N, E, top, I, H, bits, spread):
+    gen = torch.Generator("cuda").manual_seed(N + I)
+    (g, gd), (u, ud) = stack(E, I, H, bits, 64, gen), stack(E, I, H, bits, 64, gen)
+    d, dd = stack(E, H, I, bits, 64, gen)
+    y = torch.randn(N, H, generator=gen, device="cuda").bfloat16()
+    # pairs at the last few experts
+    few = max(top, min(E, spread))
+    choice = E - 1 - torch.stack([torch.randperm(few, generator=gen, device="cuda")[:top]
+                                  for _ in range(N)])
+    choice = choice.int().contiguous()
+    weight = torch.rand(N, top, generator=gen, device="cuda")
+    got = ops.expert_rows(y, choice, weight, g, u, d, bits, 64).double()
+    want = _exact(y, choice, weight, gd, ud, dd)
+    # as above
+    assert float((got - want).norm() / want.norm()) < (4e-3 if bits == 16 else 1e-3)
