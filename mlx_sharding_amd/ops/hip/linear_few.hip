@@ -54,12 +54,16 @@ __device__ __forceinline__ void arrive(const LinearFewArgs& a) {
 }
 
 // Where a block begins in the n chunks of a contraction; it goes round from there.
-// Rows of W and of x lie powers of two apart as a rule, and blocks in step at one column
-// ask few of the memory's channels: 16384 rows of 2048, 12 of x, 16.4 us from column 0 on,
-// 14.1 so (the blocks of an XCD, which are every eighth, three chunks apart; one apart
-// 14.2, seven 14.5); 28672 of 4096 with norm and unit 45.6, 43.5; 6144 of 4096 14.7, 13.2.
-// `turn` divides by the chunks of a whole share: the last may have less.
+// Of rows of W that lie a multiple of 2048 apart, blocks in step at one column ask few of the
+// memory's channels: 16384 rows of 2048, 12 of x, 16.4 us from column 0 on, 14.1 so (the
+// blocks of an XCD, which are every eighth, three chunks apart; one apart 14.2, seven 14.5);
+// 28672 of 4096 with norm and unit 45.6, 43.5; 6144 of 4096 14.7, 13.2; 64 of x, four tiles
+// .87 of the time.  Rows that lie otherwise need none, and going round costs them up to 10%
+// (turn 0: 8 of x, 16064 units of 5376 64.0 us from column 0 on, 70.2 else; one of x, 7008
+// rows of 16192 42.6, 46.8).  `turn` divides by the chunks of a whole share: the last may
+// have less.
 __device__ __forceinline__ int first_of(const LinearFewArgs& a, int whole, int n) {
+  if (!a.turn) return 0;
   const unsigned at = (blockIdx.x >> 3) * 3;
   return max(min((int)(at - __umulhi(at, a.turn) * whole), n - 1), 0);
 }
@@ -163,8 +167,9 @@ __device__ __forceinline__ void finish_columns(const LinearFewArgs& a, int row, 
 }
 
 // RT tiles of 16 rows of W; with a gated unit half of them are the gate's, the
-// others the up projection's
-template <int RT, int ACT, bool NORM, int NW, int U>
+// others the up projection's.  SHARED: blocks have a share of a contraction each (in every
+// kernel they cost 1% of the time: 9 of x, 4608 rows of 512 3.91 us so, 3.83 as it is)
+template <int RT, int ACT, bool NORM, int NW, int U, bool SHARED>
 __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
     const LinearFewArgs a) {
   __shared__ __attribute__((aligned(16))) f32x4 red[NW][RT][WAVE];
@@ -203,7 +208,8 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
   };
 
   // this block's share of the contraction
-  const int s0 = blockIdx.y * a.share, steps = min(a.share, a.K / 32 - s0);
+  const int s0 = SHARED ? blockIdx.y * a.share : 0;
+  const int steps = SHARED ? min(a.share, a.K / 32 - s0) : a.K / 32;
   const int chunks = steps / U, first = first_of(a, a.share / U, chunks);
   // operands of one chunk; the next one's are asked for before this one is used,
   // rows of x among them, as loads come back in order
@@ -308,9 +314,7 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[h][j] *= f;
     }
-    if (!ACT && !NORM && a.parts > 1 &&
-        !sums_of_all(a, (long)blockIdx.x * YT + r, lane, v[0]))
-      return;
+    if (SHARED && !sums_of_all(a, (long)blockIdx.x * YT + r, lane, v[0])) return;
     if (l16 < a.M) finish_columns<ACT>(a, l16, row0 + r * 16 + lg * 4, v, ends);
   }
 }
@@ -322,7 +326,8 @@ static dim3 shared_grid(LinearFewArgs& a, int cols, int steps, int per, int spli
   const int parts = (steps + a.share - 1) / a.share;
   a.parts = (unsigned char)parts;
   const int chunks = a.share / per;
-  a.turn = chunks > 1 ? (unsigned)(((1ull << 32) + chunks - 1) / chunks) : 0;
+  a.turn = chunks > 1 && a.ldw % 2048 == 0
+               ? (unsigned)(((1ull << 32) + chunks - 1) / chunks) : 0;
   return dim3((unsigned)((a.O + cols - 1) / cols), (unsigned)parts);
 }
 
@@ -332,10 +337,16 @@ static void linear_few_go(LinearFewArgs a, int split, hipStream_t stream) {
   // the norm's weights and sums need registers: shorter chunks
   const dim3 grid = shared_grid(a, cols, a.K / 32, a.norm ? 2 : U, split);
   const dim3 block(NW * WAVE);
+  if constexpr (RT == 1 && U == 2) {
+    if (a.parts > 1) {
+      linear_few_kernel<RT, ACT, false, NW, U, true><<<grid, block, 0, stream>>>(a);
+      return;
+    }
+  }
   if (a.norm) {
-    linear_few_kernel<RT, ACT, true, NW, 2><<<grid, block, 0, stream>>>(a);
+    linear_few_kernel<RT, ACT, true, NW, 2, false><<<grid, block, 0, stream>>>(a);
   } else {
-    linear_few_kernel<RT, ACT, false, NW, U><<<grid, block, 0, stream>>>(a);
+    linear_few_kernel<RT, ACT, false, NW, U, false><<<grid, block, 0, stream>>>(a);
   }
 }
 
@@ -383,8 +394,14 @@ static void linear_few_tiles(const LinearFewArgs& a, int act, int split,
 // bytes: 10.6 us for 64 x 2048 x 2048, 70 for 64 x 4096 x 28672.
 #define LS_WAVES 8
 
+// What blocks have of a contraction: all of it, from the first column on or from a column
+// of their own (first_of), or a share.  Up to 4096 rows of W first columns of their own gain
+// nothing, and what they and shares take cost short kernels up to 8% (17 of x, 1024 rows of
+// 2048 4.85 us without, 5.1 with; units of 896 of 4416 14.5, 15.7).
+enum { LS_WHOLE = 0, LS_TURNED = 1, LS_SHARED = 2 };
+
 // RT, TT: tiles of 16 rows of W and of x
-template <int RT, int TT, int KS, int ACT, bool NORM>
+template <int RT, int TT, int KS, int ACT, bool NORM, int WAY>
 __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
     const LinearFewArgs a) {
   constexpr int YT = ACT ? RT / 2 : RT;
@@ -421,17 +438,20 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
     }
   }
   bf16x8_t g[NORM ? RING : 1];
-  // this block's share of the contraction
-  const int s0 = blockIdx.y * a.share;
-  const int stages = min(a.share, (a.K + KS * 32 - 1) / (KS * 32) - s0);
-  const int first = first_of(a, a.share, stages);
-  auto turned = [&](int t) {
-    t = min(t, stages - 1) + first;
-    return s0 + (t >= stages ? t - stages : t);
+  constexpr int W = KS * 32;  // columns of a stage
+  const int s0 = WAY == LS_SHARED ? blockIdx.y * a.share : 0;
+  const int all = (a.K + W - 1) / W - s0;
+  const int stages = WAY == LS_SHARED ? min(a.share, all) : all;
+  // the first column of a stage, counted from those that the loop is at
+  const int end = (s0 + stages) * W, span = stages * W;
+  int base = (s0 + (WAY == LS_WHOLE ? 0 : first_of(a, a.share, stages))) * W;
+  auto column = [&](int t) {
+    const int k = base + t * W;
+    return WAY != LS_WHOLE && k >= end ? k - span : k;
   };
   // columns behind the last one repeat others of its row; nobody takes them
   auto issue = [&](int t, int slot) {
-    const int k0 = turned(t) * (KS * 32);
+    const int k0 = column(t);
 #pragma unroll
     for (int i = 0; i < PARTS; ++i)
       __builtin_amdgcn_global_load_lds(
@@ -451,8 +471,8 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
 #pragma unroll
     for (int r = 0; r < RT; ++r) acc[r][i] = f32x4{0, 0, 0, 0};
   }
-  auto use = [&](int t, int s) {
-    if ((turned(t) * KS + step) * 32 >= a.K) return;
+  auto use = [&](int s) {
+    if (column(s) + step * 32 >= a.K) return;
     const char* at = smem + s * STAGE + l16 * RP * 16 + place(l16, step * 4 + lg) * 16;
     bf16x8_t w[RT], v[TW];
 #pragma unroll
@@ -497,9 +517,10 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
       __builtin_amdgcn_s_waitcnt((BEHIND & 15) | (BEHIND >> 4) << 14 | 0xf70);
       asm volatile("s_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-      issue(t0 + s + RING - 1, (s + RING - 1) % RING);
-      use(t0 + s, s);
+      issue(s + RING - 1, (s + RING - 1) % RING);
+      use(s);
     }
+    base += RING * W;
   }
   // the remainder is on its way
   __builtin_amdgcn_sched_barrier(0);
@@ -508,7 +529,7 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int s = 0; s < RING - 1; ++s)
-    if (t0 + s < stages) use(t0 + s, s);
+    if (t0 + s < stages) use(s);
   __syncthreads();
   f32x4* red = reinterpret_cast<f32x4*>(smem);  // [steps][RT][TT][lanes]
 #pragma unroll
@@ -551,7 +572,7 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[h][j] *= f;
     }
-    if (!ACT && !NORM && a.parts > 1 &&
+    if (WAY == LS_SHARED &&
         !sums_of_all(a, ((long)blockIdx.x * YT + r) * TT + i, lane, v[0]))
       continue;
     if (i * 16 + l16 < a.M)
@@ -566,13 +587,21 @@ static void linear_some_go(LinearFewArgs a, int split, hipStream_t stream) {
   constexpr int stage = (RT + TT) * KS * 1024;
   constexpr int ring = (4 * stage > 140 * 1024 ? 3 : 4) * stage;
   constexpr int smem = ring > KS * RT * TT * 1024 ? ring : KS * RT * TT * 1024;
-  if (smem > 56 * 1024)  // with the sums of squares above the default limit
-    (void)hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&linear_some_kernel<RT, TT, KS, ACT, NORM>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   const dim3 grid = shared_grid(a, cols, (a.K + KS * 32 - 1) / (KS * 32), 1, split);
-  linear_some_kernel<RT, TT, KS, ACT, NORM>
-      <<<grid, dim3(LS_WAVES * WAVE), smem, stream>>>(a);
+  auto go = [&](auto kernel) {
+    if (smem > 56 * 1024)  // with the sums of squares above the default limit
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    kernel<<<grid, dim3(LS_WAVES * WAVE), smem, stream>>>(a);
+  };
+  if constexpr (RT > 1 && !ACT && !NORM) {
+    if (a.parts > 1) return go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_SHARED>);
+  }
+  if constexpr (RT > 1) {
+    if (a.turn && !(RT == 2 && ACT && a.O <= 2048))
+      return go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_TURNED>);
+  }
+  go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_WHOLE>);
 }
 
 template <int RT, int ACT>

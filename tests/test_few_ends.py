@@ -30,3 +30,21 @@ def test_ends(M, O, K, act, shift, pad):
     got = ops._linear_few(x, w, bias, res, None, act)
     # half a place of bf16, and sums of K products in fp32
     torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=1e-4)
+
+
+# rows of W that lie a multiple of 2048 apart: blocks begin at columns of their own and go
+# round, through registers and LDS, with fewer chunks than blocks and an incomplete last one
+@pytest.mark.parametrize("M", [3, 12, 40])
+@pytest.mark.parametrize("O,K", [(48, 2048), (4500, 96), (4500, 2016), (9000, 160), (9000, 2048)])
+@pytest.mark.parametrize("act", [None, "silu"])
+def test_rows_apart(M, O, K, act):
+    g = torch.Generator("cuda").manual_seed(O + M)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(2 * O if act else O, 2048, generator=g, device="cuda") / K ** 0.5
+         ).bfloat16()[:, :K]
+    z = x.double() @ w.double().T
+    if act:
+        z = torch.nn.functional.silu(z[:, :O]) * z[:, O:]
+    got = ops._linear_few(x, w, None, None, None, act)
+    # half a place of bf16, and sums of K products in fp32
+    torch.testing.assert_close(got.double(), z, rtol=2 ** -8, atol=1e-4)
