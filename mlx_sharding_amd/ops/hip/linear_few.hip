@@ -350,39 +350,54 @@ static void linear_few_go(LinearFewArgs a, int split, hipStream_t stream) {
   }
 }
 
-// Tiles of W's rows per block: one up to 4096 rows, which are 256 blocks; two up
-// to 8192 (6144 rows, 16 of x: 13.7 us, 17.0 with one); beyond that four, where
-// rows of x are read once for 64 of W (28672 rows, 16 of x: 48 us, 51 with two, 56
-// with one), but one for few rows of x without a norm (one: 38 us, 45 with four; the norm
-// is made in every block: one of x, 128256 rows of 4096 202 us so, 181 with four, of
-// 32000 rows of 3584 51 and 44).  A unit needs
-// both its halves; four from 16384 rows on (28672 rows, 16 of x, norm: 50 us, 53
-// with two; 12800, one of x: 14.0 with two, 15.8), but two for short contractions into
-// less than 24576, where blocks of four come in little more than one round (one of x, K
-// 2048: 16384 rows 14.8 us, 14.1 with two, 21888 24.1, 20.6, 28672 24.1, 24.6).  One
-// tile takes two steps at a time: 4096 rows of 4096 8.3 us, of 14336 22.2, with four 9.2
-// and 23.3.
+// Tiles of W's rows per block.  A CU reads about 38 bytes a nanosecond, W and, from L2, x,
+// so it is those with which the busiest CU reads the fewest rows of both: its blocks, one
+// after the other, times what a block reads.  Over 2800 random sizes these are within .4%
+// of the fastest (us with one, two, four: 28672 rows of 4096, one of x 38, 42, 45; 16 of x
+// 56, 51, 48; 8192 of 3584, 12 of x 15.8, 15.0, 18.2; 11312 of 1472, one of x 8.0, 8.6,
+// 9.4).  Through registers a block's norm or unit costs about four rows more, and 16 where
+// rows are short; four tiles else three, as they have fewer loads under way (units of one of
+// x, 26528 of 512 with two 15.9, four 13.1; 7 of x, norm, 23552 rows of 576 9.9, 8.8; 4 of
+// x, 26272 rows of 3840 with one 39.1, four 42.5).  through: rows of x by LDS, up to 8 as 8
+// (which has four tiles wherever so few are).
+static int few_tiles(int M, int O, int K, int act, bool norm, bool through) {
+  const bool more = act || norm;
+  const int rows = through ? max(M, 8) : M + (!more ? 0 : K <= 1024 ? 16 : 4);
+  int best = 0;
+  long least = 0;
+  for (int tiles = 4; tiles >= (act ? 2 : 1); tiles /= 2) {
+    const int cols = 16 * tiles / (act ? 2 : 1), blocks = (O + cols - 1) / cols;
+    const int fewer = tiles == 4 && !more && !through ? 3 : 0;
+    const long reads = (long)((blocks + 255) / 256) * (16 * tiles + rows + fewer);
+    if (!best || reads < least) best = tiles, least = reads;
+  }
+  return best;
+}
+
+// One tile takes two steps at a time (4096 rows of 4096 8.3 us, of 14336 22.2, with four 9.2
+// and 23.3; 23744 rows of 544 7.5, 9.1), but four in long rows of more than one round
+// (28672 of 4096 41, 38).
 static void linear_few_tiles(const LinearFewArgs& a, int act, int split,
                              hipStream_t stream) {
-  const bool four = a.O >= 8192 && !(a.K <= 2048 && a.O < 12288);
+  const int tiles = few_tiles(a.M, a.O, a.K, act, a.norm != nullptr, false);
   if (act == LF_SILU) {
-    if (four) linear_few_go<4, LF_SILU, 4, 2>(a, 1, stream);
+    if (tiles == 4) linear_few_go<4, LF_SILU, 4, 2>(a, 1, stream);
     else linear_few_go<2, LF_SILU, 8, 4>(a, 1, stream);
   } else if (act == LF_GELU) {
-    if (four) linear_few_go<4, LF_GELU, 4, 2>(a, 1, stream);
+    if (tiles == 4) linear_few_go<4, LF_GELU, 4, 2>(a, 1, stream);
     else linear_few_go<2, LF_GELU, 8, 4>(a, 1, stream);
-  } else if (a.O <= 4096) {
-    linear_few_go<1, LF_PLAIN, 8, 2>(a, split, stream);
-  } else if (a.O > 8192 && a.M <= 4 && !a.norm) {
-    linear_few_go<1, LF_PLAIN, 8, 4>(a, 1, stream);
-  } else if (a.O <= 8192) {
-    linear_few_go<2, LF_PLAIN, 8, 4>(a, 1, stream);
-  } else {
+  } else if (tiles == 4) {
     linear_few_go<4, LF_PLAIN, 4, 2>(a, 1, stream);
+  } else if (tiles == 2) {
+    linear_few_go<2, LF_PLAIN, 8, 4>(a, 1, stream);
+  } else if (a.O > 4096 && a.K >= 4096) {
+    linear_few_go<1, LF_PLAIN, 8, 4>(a, 1, stream);
+  } else {
+    linear_few_go<1, LF_PLAIN, 8, 2>(a, split, stream);
   }
 }
 
-// The same for 17 to 64 rows of x.  Read by each wave from L2 as above, rows of x
+// The same for more rows of x (few_through_lds).  Read by each wave from L2 as above, they
 // would be the larger part of what is read, and 64 bytes of each of 16 rows take a
 // load four times as long as whole lines; here x and W come to LDS in whole lines, KS
 // steps of 32 columns at a time, into a ring of stages.  A wave takes one of the steps,
@@ -621,62 +636,52 @@ static void linear_some_tiles(const LinearFewArgs& a, int split, hipStream_t str
   }
 }
 
-// Tiles of W's rows per block: one up to 4096 rows, which are 256 blocks, two up to
-// 8192, then four (64 of x; one, two, four: 4096 rows of 4096 13.7, 17.0, 21.7 us;
-// 5632 of 2048 15.0, 10.8, 13.6; 11264 of 2048 23.3, 19.8, 15.4).  Blocks that share
-// tiles have two, or four above 2816 rows.
+// Blocks that share a contraction have two tiles up to 2048 rows and four above (few_split).
 static void linear_some(const LinearFewArgs& a, int act, int split, hipStream_t stream) {
-  const bool many = (act ? 2 : 1) * a.O > 8192;
+  const int tiles = split > 1 ? (a.O <= 2048 ? 2 : 4)
+                              : few_tiles(a.M, a.O, a.K, act, a.norm != nullptr, true);
   if (act == LF_SILU) {
-    if (many) linear_some_tiles<4, LF_SILU>(a, 1, stream);
+    if (tiles == 4) linear_some_tiles<4, LF_SILU>(a, 1, stream);
     else linear_some_tiles<2, LF_SILU>(a, 1, stream);
   } else if (act == LF_GELU) {
-    if (many) linear_some_tiles<4, LF_GELU>(a, 1, stream);
+    if (tiles == 4) linear_some_tiles<4, LF_GELU>(a, 1, stream);
     else linear_some_tiles<2, LF_GELU>(a, 1, stream);
-  } else if (split > 1) {
-    if (a.O <= 2816) linear_some_tiles<2, LF_PLAIN>(a, split, stream);
-    else linear_some_tiles<4, LF_PLAIN>(a, split, stream);
-  } else if (a.O <= 4096) {
+  } else if (tiles == 1) {
     linear_some_tiles<1, LF_PLAIN>(a, 1, stream);
-  } else if (many) {
-    linear_some_tiles<4, LF_PLAIN>(a, 1, stream);
+  } else if (tiles == 2) {
+    linear_some_tiles<2, LF_PLAIN>(a, split, stream);
   } else {
-    linear_some_tiles<2, LF_PLAIN>(a, 1, stream);
+    linear_some_tiles<4, LF_PLAIN>(a, split, stream);
   }
 }
 
-// Whether rows of x go through LDS: above 16, and above 8 where a block would read them
-// for many columns or from many blocks (12 of x; registers, LDS: 4096 rows of 4096 9.5,
-// 9.2 us; of 14336 26, 23.8; 2048 of 8192 15.7, 12.5; 8192 of 3584 15, 13.0; 2048 of
-// 2048 6.2, 6.4; 8192 of 512 4.6, 5.2; 6144 of 1536 7.1, 7.3; 3648 of 2048 with norm 7.3,
-// 8.3).  With norms or units few rows, too,
-// where a block has four tiles of W's rows (one of x; 16032 of 4096 with norm 30.8, 25.2
-// us; 12800 of 2048 15.9, 13.4; units of 12288 of 4096 27.8, 23.8).  Not where there are
-// blocks for all CUs and the contraction is short (12 of x; units of 16384 of 2048 14.6,
-// 16.6, of 21888 24.1, 25.3; 32000 of 2048 25.0, 27.2), nor where blocks come in many
-// rounds (12 of x; 128256 of 4096 with norm 182, 192; 18000 of 4096 43, 40; one of x,
-// units of 37888 of 3584 59, 61).
+// Whether rows of x go through LDS: above 16, and fewer where rows are long, as a block's
+// chain through registers is the longer one (time by LDS over that by registers, 9 to 16
+// of x: rows of 4096 and more .70 to 1.0, but 1.07 for 9 of x into up to 4096 with norm; of
+// 2048 to 4096 without a norm .78 to 1.0 and up to 1.05, with one about .95 for 8192 to 24576
+// rows of W and 1.0 to 1.15 for others; up to 8 of x, with a norm: 8192 to 12288 rows of W of
+// 4096 and more .87 to 1.03, others 1.0 to 1.35).
 static bool few_through_lds(int M, int O, int K, int act, bool norm) {
   const int rows = (act ? 2 : 1) * O;
   if (M > 16) return true;
-  if (rows >= 16384 && K <= 2048) return false;
-  if (rows > 24576 && (!act || M <= 8)) return false;
-  if (M > 8) return rows > 4096 ? K >= 2048 : K > 2048;
-  return (act || norm) && rows > 8192;
+  if (M > 8 && K >= 4096) return M > 11 || act || !norm || rows > 4096;
+  if (M > 8) return K >= 2048 && (!norm || (rows > 8192 && rows <= 24576));
+  return norm && K >= 4096 && rows > 8192 && rows <= 12288;
 }
 
-// Blocks that share a tile's contraction where the caller has room for their sums.  x is
-// read once per block, four times W with 16 rows of W and 64 of x: long rows then have
-// blocks of more rows and a part of the columns each (us, alone and shared; 64 of x: 4096
-// rows of 14336 39.6, 29.0; 3584 of 14336 39, 28.3; 2048 of 8192 20.7, 13.4, of 5632 17.6,
-// 11.5, of 2816 10.5, 8.9; 12 of x, 2048 of 8192 12.5, 10.5; 32 of x, 4096 of 14336 29.7,
-// 25.2, but 12 of these 23.8, 24.7).  Up to 2816 rows of W leave CUs idle without (one
-// of x, 2048 of 8192: 11.6, 9.7).
+// Blocks that share a tile's contraction where the caller has room for their sums, as many
+// as come in one round: x is read once per block, four times W with 16 rows of W and 64 of
+// x, so that long rows have blocks of more rows and a part of the columns each, and up to
+// 2048 rows of W leave CUs idle without (us, alone and shared: 64 of x, 2048 rows of 8192
+// 20.7, 13.4, 4096 of 14336 39.6, 29.0; one of x, 2048 of 8192 11.6, 9.7).  In two rounds
+// it loses (64 of x, 2816 rows of 4096 17.4, 19.9; one of x, 2816 of 8192 15.3, 18.3), with
+// short rows it costs what it gains (33 of x, 2048 rows of 2048 11.1, 11.7), and so it does
+// with four tiles for up to 16 of x (12 of x, 4096 rows of 14336 23.8, 24.7).
 static int few_split(int M, int O, int K, int act, bool norm) {
   if (act || norm) return 1;
-  if (!few_through_lds(M, O, K, act, norm)) return O <= 2816 && K >= 4096 ? 2 : 1;
-  if (O <= 2816) return K >= (M > 32 ? 2048 : 4096) ? 4 : 1;
-  return O <= 4608 && K >= 8192 && M > 16 ? 4 : 1;
+  if (!few_through_lds(M, O, K, act, norm)) return O <= 2048 && K >= 4096 ? 2 : 1;
+  if (O <= 2048) return K >= (M > 32 ? 2560 : 4096) ? 4 : 1;
+  return O <= 4096 && K >= 8192 && M > 16 ? 4 : 1;
 }
 
 // Room for a shared contraction: `numbers` to be cleared before, and sums behind them.

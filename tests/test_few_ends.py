@@ -1,5 +1,7 @@
 """What few rows' products add to their columns, read by fours or alone."""
 
+import types
+
 import pytest
 import torch
 
@@ -30,6 +32,34 @@ def test_ends(M, O, K, act, shift, pad):
     got = ops._linear_few(x, w, bias, res, None, act)
     # half a place of bf16, and sums of K products in fp32
     torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=1e-4)
+
+
+# where a round of 256 blocks ends, for each number of tiles, and where rows of x change
+# between registers and LDS
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("act", [None, "silu"])
+@pytest.mark.parametrize("M,K", [(1, 64), (8, 4096), (9, 2048), (16, 2016), (17, 96), (64, 64)])
+@pytest.mark.parametrize("rows", [4096, 4112, 8192, 8224, 12304, 16416, 24608])
+def test_rounds(M, K, rows, act, norm):
+    g = torch.Generator("cuda").manual_seed(rows + M)
+
+    def rand(*n):
+        return torch.randn(*n, generator=g, device="cuda").bfloat16()
+
+    x, w = rand(M, K), rand(rows, K) / K ** 0.5
+    n = types.SimpleNamespace(weight=rand(K), eps=1e-5, weight_offset=0.0) if norm else None
+    h = x.double()
+    if norm:
+        h = h * (h.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * n.weight.double()
+    z = h @ w.double().T
+    # 32-bit sums, and rows rounded to bf16 behind the norm
+    off = (h.abs() @ w.double().abs().T) * (K * 2.0 ** -24 + (2.0 ** -8 if norm else 0.0))
+    if act:  # silu grows by at most 1.13 of its argument
+        gate, up, og, ou = *z.chunk(2, -1), *off.chunk(2, -1)
+        unit = torch.nn.functional.silu(gate)
+        z, off = unit * up, 1.13 * og * (up.abs() + ou) + unit.abs() * ou + 1e-6
+    got = ops._linear_few(x, w, None, None, n, act)
+    assert bool(((got.double() - z).abs() <= 2.0 ** -8 * z.abs() + off + 1e-6).all())
 
 
 # rows of W that lie a multiple of 2048 apart: blocks begin at columns of their own and go
