@@ -94,14 +94,6 @@ static torch::Tensor linear_few_run(const torch::Tensor& x, const torch::Tensor&
   return y;
 }
 
-static torch::Tensor linear_few(torch::Tensor x, torch::Tensor w,
-                                c10::optional<torch::Tensor> bias,
-                                c10::optional<torch::Tensor> residual,
-                                c10::optional<torch::Tensor> norm, double eps,
-                                double offset, int64_t act) {
-  return linear_few_run(x, w, bias, residual, norm, eps, offset, act, {}, {});
-}
-
 // An ordinary tensor that nothing differentiates, maps or traces.
 static bool linear_few_plain(const torch::Tensor& t) {
   static const c10::DispatchKeySet odd({
@@ -212,7 +204,7 @@ static torch::Tensor linear_few_shaped(const torch::Tensor& y, const torch::Tens
   return y.view(sizes);
 }
 
-// linear_few for x of any number of dimensions, or nothing where it does not run here.
+// linear_few_run for x of any number of dimensions, or nothing where it does not run here.
 // clear: int32 numbers that are zero afterwards.
 static c10::optional<torch::Tensor> linear_few_try(
     torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
