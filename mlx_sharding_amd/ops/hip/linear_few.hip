@@ -409,10 +409,11 @@ static void linear_few_tiles(const LinearFewArgs& a, int act, int split,
 // bytes: 10.6 us for 64 x 2048 x 2048, 70 for 64 x 4096 x 28672.
 #define LS_WAVES 8
 
-// What blocks have of a contraction: all of it, from the first column on or from a column
-// of their own (first_of), or a share.  Up to 4096 rows of W first columns of their own gain
-// nothing, and what they and shares take cost short kernels up to 8% (17 of x, 1024 rows of
-// 2048 4.85 us without, 5.1 with; units of 896 of 4416 14.5, 15.7).
+// What blocks have of a contraction: all of it, from the first column on or, where the memory
+// asks for it, from a column of their own (first_of), or a share.  Few blocks gain nothing by
+// a column of their own, and what it and shares take cost short kernels up to 8% (17 of x;
+// 512 rows of 4096 6.4 us without, 6.8 with, 1024 of 8192 12.7, 12.7, 2048 13.8, 13.25, 4096
+// 17.5, 15.4; units of 2048 of 4096 with norm 14.0, 14.3, of 3072 of 8192 26.8, 25.9).
 enum { LS_WHOLE = 0, LS_TURNED = 1, LS_SHARED = 2 };
 
 // RT, TT: tiles of 16 rows of W and of x
@@ -457,14 +458,18 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
   const int s0 = WAY == LS_SHARED ? blockIdx.y * a.share : 0;
   const int all = (a.K + W - 1) / W - s0;
   const int stages = WAY == LS_SHARED ? min(a.share, all) : all;
-  // the first column of a stage, counted from those that the loop is at
+  // the first column of a stage, counted from those that the loop is at.  Stages behind the
+  // last one repeat it, and columns behind the last one others of its row; nobody takes
+  // them (64 of x, 28672 rows of 4096 with norm 53.6 us, 54.4 where they are the first again)
   const int end = (s0 + stages) * W, span = stages * W;
   int base = (s0 + (WAY == LS_WHOLE ? 0 : first_of(a, a.share, stages))) * W;
+  const int last = base + span - W;
   auto column = [&](int t) {
-    const int k = base + t * W;
-    return WAY != LS_WHOLE && k >= end ? k - span : k;
+    int k = base + t * W;
+    if (WAY == LS_WHOLE) return k;
+    k = min(k, last);
+    return k >= end ? k - span : k;
   };
-  // columns behind the last one repeat others of its row; nobody takes them
   auto issue = [&](int t, int slot) {
     const int k0 = column(t);
 #pragma unroll
@@ -612,11 +617,10 @@ static void linear_some_go(LinearFewArgs a, int split, hipStream_t stream) {
   if constexpr (RT > 1 && !ACT && !NORM) {
     if (a.parts > 1) return go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_SHARED>);
   }
-  if constexpr (RT > 1) {
-    if (a.turn && !(RT == 2 && ACT && a.O <= 2048))
-      return go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_TURNED>);
-  }
-  go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_WHOLE>);
+  if (a.turn && grid.x >= (ACT || NORM ? 192 : 128))
+    go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_TURNED>);
+  else
+    go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_WHOLE>);
 }
 
 template <int RT, int ACT>
