@@ -660,17 +660,18 @@ static void linear_some(const LinearFewArgs& a, int act, int split, hipStream_t 
 }
 
 // Whether rows of x go through LDS: above 16, and fewer where rows are long, as a block's
-// chain through registers is the longer one (time by LDS over that by registers, 9 to 16
-// of x: rows of 4096 and more .70 to 1.0, but 1.07 for 9 of x into up to 4096 with norm; of
-// 2048 to 4096 without a norm .78 to 1.0 and up to 1.05, with one about .95 for 8192 to 24576
-// rows of W and 1.0 to 1.15 for others; up to 8 of x, with a norm: 8192 to 12288 rows of W of
-// 4096 and more .87 to 1.03, others 1.0 to 1.35).
+// chain through registers is the longer one.  Time by LDS over that by registers: 9 to 16 of
+// x, rows of 2304 to 4096 .63 to 1.04, of 2048 .84 to 1.02 for 8192 to 12288 rows of W (16 of
+// x without a norm .95 to .97 from 4096 on) and up to 1.24 for others; into up to 4096 with
+// norm, 9 of x 1.08 to 1.17, 12 1.02 to 1.11, 16 of 4096 .97 to 1.0 and of 8192 .9; up to 8
+// of x, with a norm, 8192 to 12288 rows of W of 4096 and more .87 to 1.03, others 1.0 to 1.35.
 static bool few_through_lds(int M, int O, int K, int act, bool norm) {
   const int rows = (act ? 2 : 1) * O;
+  const bool some = rows > (M > 12 && !norm ? 4096 : 8192) && rows <= 12288;
   if (M > 16) return true;
-  if (M > 8 && K >= 4096) return M > 11 || act || !norm || rows > 4096;
-  if (M > 8) return K >= 2048 && (!norm || (rows > 8192 && rows <= 24576));
-  return norm && K >= 4096 && rows > 8192 && rows <= 12288;
+  if (M <= 8) return norm && K >= 4096 && some;
+  if (norm && !act && rows <= 4096) return M > 12 && K >= 4096;
+  return K > 2048 || (K == 2048 && some);
 }
 
 // Blocks that share a tile's contraction where the caller has room for their sums, as many
