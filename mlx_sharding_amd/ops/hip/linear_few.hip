@@ -350,7 +350,7 @@ static void linear_few_go(LinearFewArgs a, int split, hipStream_t stream) {
   }
 }
 
-// Tiles of W's rows per block.  A CU reads about 38 bytes a nanosecond, W and, from L2, x,
+// Tiles of W's rows per block.  A CU reads about 30 bytes a nanosecond, W and, from L2, x,
 // so it is those with which the busiest CU reads the fewest rows of both: its blocks, one
 // after the other, times what a block reads.  Over 2800 random sizes these are within .4%
 // of the fastest (us with one, two, four: 28672 rows of 4096, one of x 38, 42, 45; 16 of x
