@@ -486,7 +486,8 @@ class DeepseekV2MoE(nn.Module):
     def _beside(self, y):
         """The shared experts' matrices, where they go with the routed ones."""
         m = self.shared_experts
-        if (m is None or not as_built(m) or not as_built(*m.read())
+        if (m is None or y.shape[0] > ops.SHARED_TOKENS
+                or not as_built(m) or not as_built(*m.read())
                 or m._fused_gu is None or m._fused_gu.bias is not None
                 or m.down_proj.bias is not None or not ops.few_tokens(y)):
             return None

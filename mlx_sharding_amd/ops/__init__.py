@@ -722,9 +722,12 @@ def expert_rows(y, choice, weight, gate, up, down, bits: int, group_size: int,
     return rows if shared is None else (rows, other)
 
 
+SHARED_TOKENS = 8  # that a shared feed-forward goes along with in expert_rows
+
+
 def expert_shared_ok(n_tokens: int, H: int, w_in, w_out) -> bool:
     """Whether expert_rows takes a shared feed-forward of these matrices along."""
-    return (n_tokens <= 8 and w_in is not None and w_out is not None
+    return (n_tokens <= SHARED_TOKENS and w_in is not None and w_out is not None
             and not os.environ.get("MLXS_AMD_DENSE_GEMV")  # names another kernel
             and w_out.shape[-1] % 64 == 0 and max(H, w_out.shape[-1]) <= 4096
             and tuple(w_in.shape) == (2 * w_out.shape[-1], H) and w_out.shape[0] == H
