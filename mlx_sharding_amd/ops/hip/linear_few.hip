@@ -54,14 +54,14 @@ __device__ __forceinline__ void arrive(const LinearFewArgs& a) {
 }
 
 // Where a block begins in the n chunks of a contraction; it goes round from there.
-// Of rows of W that lie a multiple of 2048 apart, blocks in step at one column ask few of the
-// memory's channels: 16384 rows of 2048, 12 of x, 16.4 us from column 0 on, 14.1 so (the
-// blocks of an XCD, which are every eighth, three chunks apart; one apart 14.2, seven 14.5);
-// 28672 of 4096 with norm and unit 45.6, 43.5; 6144 of 4096 14.7, 13.2; 64 of x, four tiles
-// .87 of the time.  Rows that lie otherwise need none, and going round costs them up to 10%
-// (turn 0: 8 of x, 16064 units of 5376 64.0 us from column 0 on, 70.2 else; one of x, 7008
-// rows of 16192 42.6, 46.8).  `turn` divides by the chunks of a whole share: the last may
-// have less.
+// Where rows of W lie in step (in_step), blocks at one column ask few of the memory's
+// channels: 16384 rows of 2048, 12 of x, 16.4 us from column 0 on, 14.1 so (the blocks of an
+// XCD, which are every eighth, three chunks apart; one apart 14.2, seven 14.5); 28672 of 4096
+// with norm and unit 45.6, 43.5; 6144 of 4096 14.7, 13.2; 14080 of 5504, 8 of x, 39.3, 32.5;
+// 64 of x, four tiles, rows of 4096 .87 of the time.  Others need none, and going round costs
+// them up to 10% (turn 0: 8 of x, 16064 units of 5376 64.0 us from column 0 on, 70.2 else; one
+// of x, 7008 rows of 16192 42.6, 46.8).  `turn` divides by the chunks of a whole share: the
+// last may have less.
 __device__ __forceinline__ int first_of(const LinearFewArgs& a, int whole, int n) {
   if (!a.turn) return 0;
   const unsigned at = (blockIdx.x >> 3) * 3;
@@ -319,6 +319,16 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
   }
 }
 
+// Whether rows that lie ld apart meet the same few of the memory's channels: up to five of
+// them are a multiple of 16 KB, or miss it by less than a channel's 256 bytes.
+static bool in_step(long ld) {
+  for (int n = 1; n <= 5; ++n) {
+    const int off = (int)(n * ld * 2 % 16384);
+    if (min(off, 16384 - off) <= 256) return true;
+  }
+  return false;
+}
+
 // Blocks that share a tile's contraction, as many as have something of it.
 // per: steps or stages of a chunk
 static dim3 shared_grid(LinearFewArgs& a, int cols, int steps, int per, int split) {
@@ -326,7 +336,7 @@ static dim3 shared_grid(LinearFewArgs& a, int cols, int steps, int per, int spli
   const int parts = (steps + a.share - 1) / a.share;
   a.parts = (unsigned char)parts;
   const int chunks = a.share / per;
-  a.turn = chunks > 1 && a.ldw % 2048 == 0
+  a.turn = chunks > 1 && in_step(a.ldw)
                ? (unsigned)(((1ull << 32) + chunks - 1) / chunks) : 0;
   return dim3((unsigned)((a.O + cols - 1) / cols), (unsigned)parts);
 }
@@ -414,6 +424,7 @@ static void linear_few_tiles(const LinearFewArgs& a, int act, int split,
 // a column of their own, and what it and shares take cost short kernels up to 8% (17 of x;
 // 512 rows of 4096 6.4 us without, 6.8 with, 1024 of 8192 12.7, 12.7, 2048 13.8, 13.25, 4096
 // 17.5, 15.4; units of 2048 of 4096 with norm 14.0, 14.3, of 3072 of 8192 26.8, 25.9).
+// Four tiles a block are for rows enough.
 enum { LS_WHOLE = 0, LS_TURNED = 1, LS_SHARED = 2 };
 
 // RT, TT: tiles of 16 rows of W and of x
@@ -617,7 +628,7 @@ static void linear_some_go(LinearFewArgs a, int split, hipStream_t stream) {
   if constexpr (RT > 1 && !ACT && !NORM) {
     if (a.parts > 1) return go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_SHARED>);
   }
-  if (a.turn && grid.x >= (ACT || NORM ? 192 : 128))
+  if (a.turn && (RT == 4 || grid.x >= (ACT || NORM ? 192 : 128)))
     go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_TURNED>);
   else
     go(&linear_some_kernel<RT, TT, KS, ACT, NORM, LS_WHOLE>);
