@@ -365,14 +365,14 @@ static void linear_few_go(LinearFewArgs a, int split, hipStream_t stream) {
 // after the other, times what a block reads.  Over 2800 random sizes these are within .4%
 // of the fastest (us with one, two, four: 28672 rows of 4096, one of x 38, 42, 45; 16 of x
 // 56, 51, 48; 8192 of 3584, 12 of x 15.8, 15.0, 18.2; 11312 of 1472, one of x 8.0, 8.6,
-// 9.4).  Through registers a block's norm or unit costs about four rows more, and 16 where
+// 9.4).  Through registers a block's norm or unit costs about four rows more, and 24 where
 // rows are short; four tiles else three, as they have fewer loads under way (units of one of
 // x, 26528 of 512 with two 15.9, four 13.1; 7 of x, norm, 23552 rows of 576 9.9, 8.8; 4 of
 // x, 26272 rows of 3840 with one 39.1, four 42.5).  through: rows of x by LDS, up to 8 as 8
 // (which has four tiles wherever so few are).
 static int few_tiles(int M, int O, int K, int act, bool norm, bool through) {
   const bool more = act || norm;
-  const int rows = through ? max(M, 8) : M + (!more ? 0 : K <= 1024 ? 16 : 4);
+  const int rows = through ? max(M, 8) : M + (!more ? 0 : K <= 1024 ? 24 : 4);
   int best = 0;
   long least = 0;
   for (int tiles = 4; tiles >= (act ? 2 : 1); tiles /= 2) {
@@ -675,12 +675,13 @@ static void linear_some(const LinearFewArgs& a, int act, int split, hipStream_t 
 // x, rows of 2304 to 4096 .63 to 1.04, of 2048 .84 to 1.02 for 8192 to 12288 rows of W (16 of
 // x without a norm .95 to .97 from 4096 on) and up to 1.24 for others; into up to 4096 with
 // norm, 9 of x 1.08 to 1.17, 12 1.02 to 1.11, 16 of 4096 .97 to 1.0 and of 8192 .9; up to 8
-// of x, with a norm, 8192 to 12288 rows of W of 4096 and more .87 to 1.03, others 1.0 to 1.35.
+// of x, with a norm or unit, 8192 to 12288 rows of W of 2304 and more .87 to 1.03, others 1.0
+// to 1.35.
 static bool few_through_lds(int M, int O, int K, int act, bool norm) {
   const int rows = (act ? 2 : 1) * O;
   const bool some = rows > (M > 12 && !norm ? 4096 : 8192) && rows <= 12288;
   if (M > 16) return true;
-  if (M <= 8) return norm && K >= 4096 && some;
+  if (M <= 8) return (act || norm) && K > 2048 && some;
   if (norm && !act && rows <= 4096) return M > 12 && K >= 4096;
   return K > 2048 || (K == 2048 && some);
 }
@@ -691,13 +692,14 @@ static bool few_through_lds(int M, int O, int K, int act, bool norm) {
 // 2048 rows of W leave CUs idle without (us, alone and shared: 64 of x, 2048 rows of 8192
 // 20.7, 13.4, 4096 of 14336 39.6, 29.0; one of x, 2048 of 8192 11.6, 9.7).  In two rounds
 // it loses (64 of x, 2816 rows of 4096 17.4, 19.9; one of x, 2816 of 8192 15.3, 18.3), with
-// short rows it costs what it gains (33 of x, 2048 rows of 2048 11.1, 11.7), and so it does
-// with four tiles for up to 16 of x (12 of x, 4096 rows of 14336 23.8, 24.7).
+// short rows it costs what it gains (33 of x, 2048 rows of 2048 11.1, 11.7).  With four tiles
+// up to 16 of x gain from rows of 12288 into up to 3584 on (12 of x, into 2816 23.8, 21.0,
+// into 3584 26.1, 24.3; into 4096 27.7, 28.3; 10240 into 2816 20.6, 20.9).
 static int few_split(int M, int O, int K, int act, bool norm) {
   if (act || norm) return 1;
   if (!few_through_lds(M, O, K, act, norm)) return O <= 2048 && K >= 4096 ? 2 : 1;
   if (O <= 2048) return K >= (M > 32 ? 2560 : 4096) ? 4 : 1;
-  return O <= 4096 && K >= 8192 && M > 16 ? 4 : 1;
+  return K >= 8192 && (M > 16 ? O <= 4096 : K >= 12288 && O <= 3584) ? 4 : 1;
 }
 
 // Room for a shared contraction: `numbers` to be cleared before, and sums behind them.

@@ -45,8 +45,8 @@ TOL = 4e-3
     (64, 32, 16, "silu"),             # the smallest contraction: not shared
     (256, 4128, 100, "silu"),         # columns that make no whole tile, a last short step
     (2048, 5632, 2048, "silu"),       # shared by two or four
-    (512, 8224, 2816, "gelu_tanh"),   # the last size of two tiles a block
-    (512, 8192, 2848, "gelu_tanh"),   # the first of four
+    (512, 8224, 2816, "gelu_tanh"),   # shared by blocks of four tiles, above 16 rows
+    (512, 8192, 2848, "gelu_tanh"),
     (512, 7264, 4608, "silu"),        # below 8192 columns: not shared
 ])
 def test_feed_few(M, K, ff, O, act):
@@ -59,6 +59,18 @@ def test_feed_few(M, K, ff, O, act):
         # sums have one order whichever block comes last
         for _ in range(3):
             assert torch.equal(ops.feed_few(*case[:3], act, *case[3:]), got)
+
+
+@pytest.mark.parametrize("M,ff,O", [
+    (16, 4096, 2048), (1, 4096, 2048), (64, 2560, 2048), (64, 2528, 2048),
+    (16, 4096, 2064), (9, 12288, 2064), (16, 12288, 3584), (16, 12256, 3584),
+    (16, 12288, 3600), (17, 8192, 4096), (17, 8192, 4112)])
+def test_where_shares_begin(M, ff, O):
+    """The last sizes that blocks share, and the first that they do not."""
+    case = _case(M, 64, ff, O, False, True)
+    want, got = _exact(*case, "silu"), ops.feed_few(*case[:3], "silu", *case[3:])
+    assert float((got.double() - want).norm() / want.norm()) < TOL
+    assert torch.equal(ops.feed_few(*case[:3], "silu", *case[3:]), got)
 
 
 def test_feed_few_captured():
