@@ -576,7 +576,9 @@ c10::optional<torch::Tensor> attn_step(
   // number of them.  So slices are as many as two chains have, one of heads of 256, and
   // where that would be less than half of them (of heads of 256: less than all) the
   // separate kernels are faster; of heads of 256, of which a CU has one block, also for few
-  // pairs and for more than there are CUs.  Sequences x heads over heads of a size, keys:
+  // pairs with more than one slice and for more than there are CUs.  Keys are those that a
+  // window leaves (1 x 56 over 8 of 128, 4279 behind a window of 1024: 12.7 us of the
+  // separate kernels, 10.7 here).  Sequences x heads over heads of a size, keys:
   // us of the separate kernels, of this one with all slices, with as many as here: 1 x 8
   // over 8 of 128, 3339: 12.1, 15.9, 12.6; 1 x 32 over 8 of 128, 1970: 11.9, 12.2, 11.9;
   // 1 x 128 over 8 of 128, 757: 10.8, 13.5, 11.2; 5 x 16 over 1 of 256, 226: 11.8, 22.0;
@@ -587,8 +589,11 @@ c10::optional<torch::Tensor> attn_step(
   const bool wide = D == 256;
   const long pairs = B * Hkv, chains = (Hq / Hkv * D + 511) / 512;
   const int most = std::max<int>(1, (wide ? 16 : 32) / chains);
-  const int slices = decode_slices(pairs, s_ptr ? cap : pos0 + 1, 64, wide ? 256 : 512);
-  if (faster && (wide ? slices > most || pairs < 8 || pairs > 256 : slices > 2 * most))
+  const long held = s_ptr ? cap : pos0 + 1;
+  const int slices = decode_slices(pairs, window > 0 ? std::min(held, (long)window) : held,
+                                   64, wide ? 256 : 512);
+  if (faster && (wide ? slices > most || (pairs < 8 && slices > 1) || pairs > 256
+                      : slices > 2 * most))
     return c10::nullopt;
   const int nsplit = std::min(slices, most);
   auto out = torch::empty({B, 1, Hq * D}, q.options());

@@ -175,6 +175,20 @@ def test_where_it_is_faster(B, Hq, Hkv, D, keys, taken):
     assert one.attend_step(q, k, v, cos, sin, 0.1) is not None
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,D,keys,window,taken", [
+    (1, 8, 1, 128, 4000, 2048, True), (1, 8, 1, 128, 4000, 2049, False),
+    (1, 4, 4, 256, 64, 0, True), (1, 4, 4, 256, 65, 0, False), (1, 4, 4, 256, 200, 64, True)])
+def test_where_a_window_or_one_slice_is_faster(B, Hq, Hkv, D, keys, window, taken):
+    g = torch.Generator("cuda").manual_seed(keys)
+    one, _ = _caches(B, Hkv, D, keys - 1, keys, False, g)
+    (q, k, v), cos, sin = _token(B, Hq, Hkv, D, g)
+    got = one.attend_step(q, k, v, cos, sin, 0.1, window=window, faster=True)
+    assert (got is not None) == taken
+    if taken:
+        exact = _exact(q, cos, sin, one.k, one.v, 0.0, window)
+        assert float((got.double() - exact).norm() / exact.norm()) < 2e-3  # as above
+
+
 # a wave's own tiles from 128 tiles of 64 keys of heads of 64 on, 512 of 128; before, and
 # for heads of 256, tiles of a block
 @pytest.mark.parametrize("B,Hq,Hkv,D,keys", [
