@@ -1,18 +1,23 @@
 // Products of routed experts over tiles of one expert's (token, expert) pairs.
 //
-// What bounds them: the matrix cores.  A block of four waves makes 256 pairs
-// by 256 rows of weights, a wave 128 x 128, whose sums fill the accumulation
-// registers: a step of 32 columns then takes 1024 cycles of every core and half as
-// many of LDS.  Four stages of LDS are a ring: while one is worked on, the next is
-// complete and two are on their way, straight from memory.  Operands of a half step
-// are read and loads are asked for between the products of the half step before; one
-// barrier a step.  A block walks over its tiles without a gap: behind a tile's last
-// stage the ring goes on with the next one's, and results are stored meanwhile.
-// Pieces of 16 bytes within a row of 64 are swapped by the row, so that rows that a
-// read meets lie in different banks.
-// Measured: 32768 tokens, top 6 of 64 experts, 2048 -> 1408: 1.94 ms (1167 TFLOP/s),
-// 1408 -> 2048: 1.15 (984); with a block per tile 2.07 and 1.29, loads in one run
-// behind the barrier 2.31 and 1.39.
+// What bounds them: the matrix cores, and the power that they draw (clocks of 1.7 to 1.8
+// GHz).  A block of four waves makes 256 pairs by 256 rows of weights, a wave 128 x 128,
+// whose sums fill the accumulation registers: a stage of 64 columns then takes 2048 cycles
+// of every core and half as many of LDS.  Rows of 64 columns are whole lines of 128 bytes
+// (of 32 columns twice as many requests), and pieces of 16 bytes within a row are swapped
+// by the row, so that rows that a read meets lie in different banks.  LDS holds two
+// stages; a wave works on one by quarters, and each half of its operands is replaced by
+// loads of the stage after the next as soon as all waves have read it.  More than three
+// instructions between two products hold up the second, and so do loads that come in one
+// run: loads and LDS reads stand alone between products, eight apart, with addresses that
+// need one scalar sum.  A block walks over its tiles without a gap: behind a tile's last
+// stage come the next one's, and results are stored meanwhile.
+// Products of 16 x 16 x 32 move half as many sums per operation as those of 32 x 32 x 16:
+// at one share of busy cores clocks are 7% higher.
+// Measured: 32768 tokens, top 6 of 64 experts, 2048 -> 1408: 2.02 -> 1.80 ms (1260
+// TFLOP/s), 1408 -> 2048: 1.20 -> 1.03 (1100), before with a ring of four stages of 32
+// columns; one wait for a stage's loads, all in its middle: 1.92 and 1.11.  Without loads
+// the cores are 78% busy, without loads and reads 83, as it is 74.
 // Clamped units read their pairs' weights out of LDS at the end of an item, where a load
 // from memory would wait for the stages under way.
 #pragma once
@@ -20,25 +25,29 @@
 #include "moe_tiles.h"
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// s_waitcnt for at most n loads and stores and r LDS reads under way
+constexpr int vm_wait(int n, int r) { return (n & 15) | 0x70 | r << 8 | (n >> 4) << 14; }
 
 #define MT_GROUP 4  // tiles whose blocks run together, with the same weights
 // MT: pairs of a tile
 template <int MT, MoeUnit UNIT>
 __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a) {
+#ifdef __HIP_DEVICE_COMPILE__  // buffer resources are no type of the host's
   constexpr bool GLU = UNIT != MT_SUMS;
-  constexpr int NP = MT / 64;          // 32-pair tiles of a wave
-  constexpr int L = 4 + NP;            // loads per wave and stage
-  constexpr int ST = (256 + MT) * 64;  // bytes of a stage
-  constexpr int NC = GLU ? 128 : 256;  // outputs of a block
+  constexpr int NX = MT / 32;           // 16-pair tiles of a wave, rows of x it brings in 8
+  constexpr int L = 8 + NX, LH = L / 2;  // loads per wave and stage, and half a stage
+  constexpr int ST = (256 + MT) * 128;  // bytes of a stage
+  constexpr int NC = GLU ? 128 : 256;   // outputs of a block
+  constexpr int STORES = NX * NC / 64;  // a wave's, of an item
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int l32 = lane & 31, hi = lane >> 5;
   const int wm = wid >> 1, wn = wid & 1;
-  const int nk = a.K / 32;
+  const int stages = a.K / 64;
 
   // an XCD has consecutive tiles, its blocks walk them in groups
   const int total = *a.n_tiles;
@@ -57,156 +66,201 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a)
       if (xcd * per + ti < total) return {xcd * per + ti, rest / group * NC};
     }
   };
-  // a tile's entry is asked for an item ahead, by vector loads: one that is waited
-  // for where it is needed would wait for all that was stored before it
-  int nought = 0;
-  asm volatile("" : "+v"(nought));
-  struct Entry { int e, p0, np; };
-  auto entry = [&](int tile) -> Entry {
-    const int* t = a.tiles + max(tile, 0) * 3 + nought;
-    return {t[0], t[1], t[2]};
+  // a tile's entry is read by scalar loads: what vector loads bring to registers would
+  // be waited for with all stages under way (tokens and weights go to LDS)
+  auto item = [&](const Place& at) -> Item {
+    const auto* t = (const __attribute__((address_space(4))) int*)a.tiles + max(at.tile, 0) * 3;
+    return {t[0], t[1], t[2], at.n0};
   };
-  auto item = [&](const Entry& x, int n0) -> Item {
-    return {__builtin_amdgcn_readfirstlane(x.e), __builtin_amdgcn_readfirstlane(x.p0),
-            __builtin_amdgcn_readfirstlane(x.np), n0};
+  // A wave's rows of a stage: of the weights, of which a load brings rows WR behind those
+  // of the load before (behind the last rows the last ones again: O is a multiple of 64),
+  // the first and the last load's; of x, each lane's.  Of a gated unit, waves 0 and 1
+  // bring gate rows, 2 and 3 up rows (16 by turns).
+  constexpr unsigned WR = GLU ? 16 : 32;
+  const unsigned wide = (unsigned)a.K * 2;
+  struct Rows { const char *w, *x; unsigned w_off, w_at[8], off[NX]; };
+  auto pair_of = [&](const Item& it, int i) {
+    return min((i * 4 + wid) * 8 + (lane >> 3), it.np - 1);
   };
-  auto place = [](int row, int piece) { return piece ^ ((row >> 2) & 3); };
-  // A wave's rows of a stage: bases that it shares, 32-bit offsets from there.  Of a
-  // gated unit, waves 0 and 1 bring gate rows, 2 and 3 up rows (32 by turns).
-  struct Rows { const char *w, *x; unsigned off[L]; };
-  auto tokens = [&](const Item& it, int (&t)[NP]) {
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int p = min((i * 4 + wid) * 16 + (lane >> 2), it.np - 1);
-      t[i] = GLU ? a.tokens[it.p0 + p] : p;
-    }
-  };
-  auto rows_of = [&](const Item& it, const int (&t)[NP], Rows& s) {
+  // t: rows of x
+  auto rows_of = [&](const Item& it, const int (&t)[NX], Rows& s) {
+    const unsigned at = ((lane & 7) ^ (lane >> 3)) * 16;
     s.w = (GLU && wid >> 1 ? a.w2 : a.w) + it.e * a.wstride;
     s.x = a.x + (GLU ? 0 : it.p0 * a.xstride);
+    s.w_off = (it.n0 + (GLU ? wid & 1 : wid) * 8 + (lane >> 3)) * wide + at;
 #pragma unroll
-    for (int i = 0; i < L; ++i) {
-      const int r = (i % 4 * 4 + wid) * 16 + (lane >> 2);
-      const int piece = place(r, lane & 3);
-      if (i < 4) {
-        const int o = it.n0 + (GLU ? (r >> 7) * 64 + (r >> 6 & 1) * 32 + (r & 31) : r);
-        s.off[i] = (unsigned)min(o, a.O - 1) * (unsigned)(a.K * 2) + piece * 16;
-      } else {
-        s.off[i] = (unsigned)t[i - 4] * (unsigned)a.xstride + piece * 16;
-      }
-    }
+    for (int i = 0; i < 8; ++i) s.w_at[i] = min(i * WR, a.O - WR - it.n0) * wide;
+#pragma unroll
+    for (int i = 0; i < NX; ++i) s.off[i] = (unsigned)t[i] * (unsigned)a.xstride + at;
   };
-  auto load = [&](const Rows& s, int k, int g, int i) {
-    const int part = i < 4 ? i * 4 + wid : 16 + (i - 4) * 4 + wid;
-    const char* base = (i < 4 ? s.w : s.x) + k * 64;
-    __builtin_amdgcn_global_load_lds(
-        (const __attribute__((address_space(1))) void*)(base + s.off[i]),
-        (__attribute__((address_space(3))) void*)(smem + (g & 3) * ST + part * 1024), 16, 0, 0);
+  // the i-th of the loads of a stage, to the place of stage g
+  auto load = [&](const Rows& s, __amdgpu_buffer_rsrc_t w, __amdgpu_buffer_rsrc_t x, int g,
+                  int i) {
+    auto* to = (__attribute__((address_space(3))) void*)(smem + (g & 1) * ST +
+                                                         (i * 4 + wid) * 1024);
+    if (i < 8) __builtin_amdgcn_raw_ptr_buffer_load_lds(w, to, 16, s.w_off, s.w_at[i], 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(x, to, 16, s.off[i - 8], 0, 0, 0);
   };
+  // the k-th stage
+  auto columns = [](const char* p, int k) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(p + k * 128), 0, -1, 0x00027000);
+  };
+  // numbers that belong to an item's pairs, into LDS
+  auto numbers = [&](const void* of, const Item& it, char* to) {
+    if (wid * 64 < MT)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(
+              (const int*)of + it.p0 + min(wid * 64 + lane, it.np - 1)),
+          (__attribute__((address_space(3))) void*)(to + wid * 256), 4, 0, 0);
+  };
+  // read here: the compiler would wait for all loads to LDS
+  auto number = [](const char* at) {
+    int v;
+    asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(v)
+                 : "v"((const __attribute__((address_space(3))) char*)at) : "memory");
+    return v;
+  };
+  char* const next_tokens = smem + 2 * ST;
   Place at = advance();
   if (at.tile < 0) return;
-  Item it = item(entry(at.tile), at.n0);
+  Item it = item(at);
   at = advance();
-  Entry ahead = entry(at.tile);
-  int tok[NP];
   Rows rows;
-  tokens(it, tok);
-  rows_of(it, tok, rows);
-
-  f32x16 acc[4][NP];
-  struct Frags { bf16x8_t w[4], x[NP]; };
-  int wo[2], xo[2];
+  {
+    int tok[NX];
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const int pl = place(l32, 2 * s + hi) * 16;
-    wo[s] = (wn * 128 + l32) * 64 + pl;
-    xo[s] = (256 + wm * (MT / 2) + l32) * 64 + pl;
-  }
-  auto rd = [](const char* p) { return *reinterpret_cast<const bf16x8_t*>(p); };
-  // products of `f`; between them operands of the next half step and loads
-  auto half = [&](const Frags& f, Frags& n, int g, int s, auto&& fetch) {
-    const char* b = smem + (g & 3) * ST;
-    auto wr = [&](int i) { n.w[i] = rd(b + wo[s] + i * 2048); };
-    auto xr = [&](int i) { if (i < NP) n.x[i] = rd(b + xo[s] + i * 2048); };
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-      for (int j = 0; j < NP; ++j) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[i], f.x[j], acc[i][j], 0, 0, 0);
-        if (j == 0) {
-          __builtin_amdgcn_sched_barrier(0);
-          if (i == 0) { wr(0); xr(0); xr(1); }
-          if (i == 1) { wr(1); xr(2); xr(3); }
-          if (i == 2) { wr(2); wr(3); }
-          fetch(i);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < NX; ++i) {
+      tok[i] = pair_of(it, i);
+      if (GLU) tok[i] = a.tokens[it.p0 + tok[i]];
     }
+    rows_of(it, tok, rows);
+  }
+
+  // A stage is worked on by quarters: halves of a wave's rows of weights by halves of its
+  // rows of x.  Operands of a half are w[half][tile][columns / 32], x likewise.
+  constexpr int HX = NX / 2;
+  f32x4 acc[8][NX];
+  bf16x8_t w[2][4][2], x[2][HX][2];
+  const int l16 = lane & 15;
+  const int wo = (wn * 128 + l16) * 128, xo = (256 + wm * (MT / 2) + l16) * 128;
+  const int at16[2] = {((lane >> 4) ^ (l16 & 7)) * 16, ((lane >> 4 | 4) ^ (l16 & 7)) * 16};
+  auto rd = [](const char* p) { return *reinterpret_cast<const bf16x8_t*>(p); };
+  // the r-th operand of a half
+  auto read_w = [&](int g, int h, int r) {
+    w[h][r >> 1][r & 1] =
+        rd(smem + (g & 1) * ST + at16[r & 1] + wo + (h * 4 + (r >> 1)) * 2048);
+  };
+  auto read_x = [&](int g, int h, int r) {
+    x[h][r >> 1][r & 1] =
+        rd(smem + (g & 1) * ST + at16[r & 1] + xo + (h * HX + (r >> 1)) * 2048);
+  };
+  // the c-th load of a half: a wave's share of w[h] and x[h] of all waves
+  auto load_half = [&](const Rows& s, __amdgpu_buffer_rsrc_t sw, __amdgpu_buffer_rsrc_t sx,
+                       int g, int h, int c) {
+    constexpr int Q = NX / 4;
+    if (c < 4) load(s, sw, sx, g, (c >> 1) * 4 + h * 2 + (c & 1));
+    else load(s, sw, sx, g, 8 + (c - 4) / Q * 2 * Q + h * Q + (c - 4) % Q);
   };
 #pragma unroll
-  for (int g = 0; g < 3; ++g)
+  for (int g = 0; g < 2; ++g)
 #pragma unroll
-    for (int i = 0; i < (g < 2 ? L : L / 2); ++i) load(rows, g, g, i);
+    for (int c = 0; c < L; ++c)
+      load_half(rows, columns(rows.w, g), columns(rows.x, g), g, c / LH, c % LH);
   __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(L + L / 2) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(L) : "memory");
   __builtin_amdgcn_sched_barrier(0);
-  Frags f0, f1;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) f0.w[i] = rd(smem + wo[0] + i * 2048);
+  for (int r = 0; r < 8; ++r) read_w(0, 0, r);
 #pragma unroll
-  for (int i = 0; i < NP; ++i) f0.x[i] = rd(smem + xo[0] + i * 2048);
+  for (int r = 0; r < NX; ++r) read_x(0, 0, r);
 
   int g = 0;  // stages so far
   int flip = 0;
+  int lax = 0;  // meetings behind all of an item's stores
   for (bool more = true; more;) {
     more = at.tile >= 0;
-    const Item nx = more ? item(ahead, at.n0) : it;
+    const Item nx = more ? item(at) : it;
     if (more) at = advance();
-    ahead = entry(at.tile);
-    tokens(nx, tok);
+    // read two stages before this item's end, when the second stage has waited for them
+    if constexpr (GLU) numbers(a.tokens, nx, next_tokens);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < NP; ++j)
+      for (int j = 0; j < NX; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+        for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0f;
     // weights of this item's pairs go to LDS, and are there some steps later; those of
     // the item before may still be read
     if constexpr (UNIT == MT_CLAMPED) {
       flip ^= 1;
-      if (wid * 64 < MT)
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) void*)(
-                a.scale + it.p0 + min(wid * 64 + lane, it.np - 1)),
-            (__attribute__((address_space(3))) void*)(
-                smem + 4 * ST + (flip * MT + wid * 64) * 4), 4, 0, 0);
+      numbers(a.scale, it, next_tokens + (1 + flip) * MT * 4);
     }
-    auto step = [&](auto&& fetch) {
-      half(f0, f1, g, 1, [&](int i) {
-        if (L / 2 + i < L) fetch(2, L / 2 + i);
-      });
-      __builtin_amdgcn_s_waitcnt(0x70 | L);
-      asm volatile("s_barrier" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      half(f1, f0, g + 1, 0, [&](int i) {
-        if (i < L / 2) fetch(3, i);
-      });
+    // A stage's products; between them, one at a time and evenly, operands of the quarter
+    // behind, and loads of the stage after the next.  Loads replace a half when all waves
+    // have read it (they meet twice a stage, in the middle of a quarter, where nobody
+    // waits for an operand), and are read three quarters of a stage later at least.
+    auto between = [&](int m, __amdgpu_buffer_rsrc_t sw, __amdgpu_buffer_rsrc_t sx) {
+      constexpr int Q = 4 * NX, EACH = NX / 4;  // products of a quarter, from read to read
+      const int r = m % Q / EACH;
+      const bool now = m % EACH == 0;
+      if (m < Q && now && r < NX) read_x(g, 1, r);
+      if (m / Q == 1 && now && r < 8) read_w(g, 1, r);
+      if (m / Q == 2 && now && r < 8) read_w(g + 1, 0, r);
+      if (m / Q == 3) {  // behind the last product of the one that it replaces
+        const int n = m - 3 * Q;
+        if (n % 8 == 7 || (n % 8 == 0 && n)) read_x(g + 1, 0, n / 4 - 1);
+        if (n == Q - 1) read_x(g + 1, 0, NX - 1);
+      }
+#pragma unroll
+      for (int c = 0; c < LH; ++c) {
+        if (m == Q / 2 + 1 + c * (2 * Q / LH)) load_half(rows, sw, sx, g, 0, c);
+        if (m == 5 * Q / 2 + 1 + c * (3 * Q / 2 / LH)) load_half(rows, sw, sx, g, 1, c);
+      }
+      if (m == Q / 2 - 1 || m == 5 * Q / 2 - 1) {
+        // an item's stores came behind these loads and need not be done
+        constexpr int READS = NX < 8 ? NX : 8;
+        __builtin_amdgcn_s_waitcnt(vm_wait(LH + STORES, READS));
+        if (__builtin_expect(lax <= 0, 1)) __builtin_amdgcn_s_waitcnt(vm_wait(LH, READS));
+        asm volatile("s_barrier" ::: "memory");
+        --lax;
+      }
     };
-    int k = 0;
-    do {  // 4 stages at least
-      step([&](int d, int i) { load(rows, k + d, g + d, i); });
-      ++k, ++g;
-    } while (k < nk - 3);
-    // behind the last stage of this item come the next one's
-    Rows next;
-    rows_of(nx, tok, next);
-    for (; k < nk; ++k, ++g)
-      step([&](int d, int i) {
-        const bool same = k + d < nk;
-        load(same ? rows : next, same ? k + d : k + d - nk, g + d, i);
-      });
+    auto stage = [&](int k) {
+      const auto sw = columns(rows.w, k), sx = columns(rows.x, k);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int hw = q >> 1, hx = (q ^ q >> 1) & 1;
+#pragma unroll
+        for (int j = 0; j < HX; ++j)
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              f32x4& to = acc[hw * 4 + t][hx * HX + j];
+              to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[hw][t][c], x[hx][j][c], to, 0, 0, 0);
+              __builtin_amdgcn_sched_barrier(0);
+              between(((q * HX + j) * 2 + c) * 4 + t, sw, sx);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+      }
+      ++g;
+    };
+    if (GLU && stages < 4) asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    int k = 2;
+    for (int left = stages - 2, part = 0; part < 2; left = 2, ++part) {
+      if (part) {  // behind the last stage of this item come the next one's
+        k = 0;
+        int tok[NX];
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {
+          tok[i] = pair_of(nx, i);
+          if (GLU) tok[i] = number(next_tokens + tok[i] * 4);
+        }
+        rows_of(nx, tok, rows);
+      }
+      for (; left > 0; --left, ++k) stage(k);
+    }
     __builtin_amdgcn_sched_barrier(0);
     // sums are taken out of the accumulation registers one by one: read by the
     // compiler, all are copied at once, more than there are registers for.  It does
@@ -217,7 +271,8 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a)
       asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(acc[i][j][r]));
       return v;
     };
-    // lane: pair l32, outputs (r & 3) + 8 (r >> 2) + 4 hi of 32
+    // lane: pair l16, outputs 4 (lane / 16) .. + 3 of 16; of two such runs, lanes get 8
+    // outputs side by side
     auto store = [&](__bf16* row, int o, const float (&lo)[4], const float (&up)[4]) {
       u32x2 x, y;
 #pragma unroll
@@ -225,60 +280,53 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const MoeTilesArgs a)
         x[h] = __builtin_bit_cast(unsigned, bf16x2_t{(__bf16)lo[2 * h], (__bf16)lo[2 * h + 1]});
         y[h] = __builtin_bit_cast(unsigned, bf16x2_t{(__bf16)up[2 * h], (__bf16)up[2 * h + 1]});
       }
-      const auto s0 = __builtin_amdgcn_permlane32_swap(x[0], y[0], false, false);
-      const auto s1 = __builtin_amdgcn_permlane32_swap(x[1], y[1], false, false);
-      o += hi * 8;
+      const auto s0 = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
+      const auto s1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
+      o += (lane >> 4 & 1) * 16 + (lane >> 5) * 8;
       if (o < a.O) *reinterpret_cast<u32x4*>(row + o) = u32x4{s0[0], s1[0], s0[1], s1[1]};
     };
 #pragma unroll
-    for (int j = 0; j < NP; ++j) {
-      const int p = wm * (MT / 2) + j * 32 + l32;
+    for (int j = 0; j < NX; ++j) {
+      const int p = wm * (MT / 2) + j * 16 + l16;
       // all lanes take part in the exchange
       __bf16* row = a.y + (long)(it.p0 + min(p, it.np - 1)) * a.O;
-      // read here: the compiler would wait for all loads to LDS
       float by = 1.0f;
-      if constexpr (UNIT == MT_CLAMPED) {
-        const auto* at = (__attribute__((address_space(3))) char*)(
-            smem + 4 * ST + (flip * MT + p) * 4);
-        asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
-                     : "=&v"(by) : "v"(at) : "memory");
+      if constexpr (UNIT == MT_CLAMPED)
+        by = __builtin_bit_cast(float, number(next_tokens + ((1 + flip) * MT + p) * 4));
+#pragma unroll
+      for (int i = 0; i < 8; i += GLU ? 4 : 2) {
+        float v[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if (GLU) {
+              float z = sum(i + 2 * h, j, r), u = sum(i + 2 * h + 1, j, r);
+              if constexpr (UNIT == MT_CLAMPED) {
+                z = fminf(z * by, a.limit);
+                u = fminf(fmaxf(u * by, -a.limit), a.limit) + 1.0f;
+                v[h][r] = z * __builtin_amdgcn_rcpf(1.0f + __expf(-a.alpha * z)) * u;
+              } else {
+                v[h][r] = z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)) * u;
+              }
+            } else v[h][r] = sum(i + h, j, r);
+          }
+        // rows behind the last pair repeat it
+        store(row, it.n0 + wn * (NC / 2) + i * (GLU ? 8 : 16), v[0], v[1]);
+        __builtin_amdgcn_sched_barrier(0);
       }
-#pragma unroll
-      for (int i = 0; i < (GLU ? 2 : 4); ++i)
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          float v[2][4];
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int c = (2 * q + h) * 4 + r;
-              if (GLU) {
-                float z = sum(2 * i, j, c), u = sum(2 * i + 1, j, c);
-                if constexpr (UNIT == MT_CLAMPED) {
-                  z = fminf(z * by, a.limit);
-                  u = fminf(fmaxf(u * by, -a.limit), a.limit) + 1.0f;
-                  v[h][r] = z * __builtin_amdgcn_rcpf(1.0f + __expf(-a.alpha * z)) * u;
-                } else {
-                  v[h][r] = z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)) * u;
-                }
-              } else v[h][r] = sum(i, j, c);
-            }
-          const int o = it.n0 + wn * (NC / 2) + i * 32 + q * 16;
-          // rows behind the last pair repeat it
-          store(row, o, v[0], v[1]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
     }
+    lax = it.n0 + NC <= a.O ? 2 : 0;  // else some were left out
     it = nx;
-    rows = next;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
 }
 
 template <int MT, MoeUnit UNIT>
 static void moe_tiles_go(MoeTilesArgs& a, hipStream_t stream) {
-  const int smem = 4 * (256 + MT) * 64 + (UNIT == MT_CLAMPED ? 2 * MT * 4 : 0);
+  const int smem = 2 * (256 + MT) * 128 +
+                   MT * 4 * (UNIT == MT_SUMS ? 0 : UNIT == MT_SILU ? 1 : 3);
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_tiles_kernel<MT, UNIT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   const int across = UNIT != MT_SUMS ? 128 : 256;

@@ -23,12 +23,13 @@ def routes(kind, N, E, top, gen):
 
 # one stage more than the ring has, remainders of the tiles of 256 and 128 rows of
 # weights, tiles of one pair, as many pairs as a tile has and one more, many tiles a
-# block; more than one placing block
+# block, with two, three and more stages of 64 columns; more than one placing block
 @pytest.mark.parametrize("tile", [128, 256])
 @pytest.mark.parametrize("N,E,top,H,I,kind", [
     (1, 3, 1, 128, 128, "any"), (257, 3, 1, 192, 320, "one"), (256, 2, 1, 128, 192, "one"),
     (43, 8, 6, 128, 192, "any"), (700, 7, 3, 320, 128, "few"), (1500, 160, 6, 256, 448, "any"),
-    (5000, 4, 2, 512, 704, "any")])
+    (5000, 4, 2, 512, 704, "any"), (3000, 160, 6, 1024, 128, "any"),
+    (2000, 160, 6, 1088, 192, "any"), (1500, 160, 6, 128, 1024, "any")])
 def test_against_64_bits(N, E, top, H, I, kind, tile):
     gen = torch.Generator("cuda").manual_seed(N + H)
     bf = lambda *s: torch.randn(*s, generator=gen, device="cuda").bfloat16()  # noqa: E731
