@@ -53,8 +53,8 @@ def as_built(*modules) -> bool:
 class Linear(nn.Module):
     """Dense or MLX-affine-quantized linear, chosen per checkpoint key.
 
-    Dense path → ops.linear: linear_few.hip for up to 64 rows, else the
-    library.  Quantized path → the w4a16/w8a16 dequant-GEMM op.  Parameter names (weight/scales/biases)
+    Dense path → ops.linear: linear_few.hip for up to 64 rows, else
+    linear_tiles.hip or the library.  Quantized path → the w4a16/w8a16 dequant-GEMM op.  Parameter names (weight/scales/biases)
     match the MLX checkpoint layout so pre-quantized checkpoints load
     directly (/root/reference/shard/utils.py:54-65 predicate: a
     `.scales` key exists for the module).
@@ -129,11 +129,12 @@ def project(m, x: torch.Tensor, *, norm: Optional[nn.Module] = None,
             clear: Optional[torch.Tensor] = None) -> torch.Tensor:
     """ops.project with the weights of a Linear or FusedColumns, packed ones
     through their bf16 copy."""
-    w, q = dense_weight(m, x.shape[-1]), m.quant
+    q = m.quant
+    w = dense_weight(m, x.shape[-1]) if q is None or ops.use_native(x) else None
     if w is not None:
         return ops.project(x, w, m.bias, norm=norm, act=act, residual=residual,
                            clear=clear)
-    # no room for the copy
+    # no room for the copy, or no kernels
     if clear is not None:
         clear.zero_()
     if norm is not None:

@@ -111,10 +111,8 @@ class Gemma2MLP(nn.Module):
         if norm is not None:
             x = norm(x)
         if self._fused_gu is not None:
-            g, u = self._fused_gu(x)
-        else:
-            g, u = self.gate_proj(x), self.up_proj(x)
-        return self.down_proj(ops.geglu(g, u))
+            return self.down_proj(project(self._fused_gu, x, act="gelu_tanh"))
+        return self.down_proj(ops.geglu(self.gate_proj(x), self.up_proj(x)))
 
 
 class Gemma2DecoderLayer(nn.Module):

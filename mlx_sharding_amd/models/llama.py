@@ -125,10 +125,8 @@ class LlamaMLP(nn.Module):
         if residual is not None:
             return residual + self(x)
         if self._fused_gu is not None:
-            g, u = self._fused_gu(x)
-        else:
-            g, u = self.gate_proj(x), self.up_proj(x)
-        return self.down_proj(ops.swiglu(g, u))
+            return self.down_proj(project(self._fused_gu, x, act="silu"))
+        return self.down_proj(ops.swiglu(self.gate_proj(x), self.up_proj(x)))
 
 
 class LlamaDecoderLayer(nn.Module):

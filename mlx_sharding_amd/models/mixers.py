@@ -23,7 +23,7 @@ from ..ops.paged import (HistorySpec, LayerSpec, LayerStore, RaggedBatch,
 from ..ops.ragged import (ClampedGLU, DeltaShape, GroupedShape, LatentShape,
                           Rotary, Turns)
 from ..ops.recurrent import ScanShape
-from .base import Linear, RMSNorm, as_built, feed
+from .base import Linear, RMSNorm, as_built, feed, project
 
 
 def _param(*shape, dtype) -> nn.Parameter:
@@ -477,9 +477,10 @@ class GatedMLP(nn.Module):
         self.fused = FusedColumns([self.gate, self.up])
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        if (self.fused is not None and ops.few_tokens(h) and as_built(self.down)
-                and self.act is self.ACTS[self.kind]):
-            return feed(self.fused, self.down, h, self.kind)
+        if self.fused is not None and self.act is self.ACTS[self.kind]:
+            if ops.few_tokens(h) and as_built(self.down):
+                return feed(self.fused, self.down, h, self.kind)
+            return self.down(project(self.fused, h, act=self.kind))
         g, u = self.fused(h) if self.fused is not None else (self.gate(h), self.up(h))
         return self.down(self.act(g, u))
 

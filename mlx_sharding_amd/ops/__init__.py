@@ -314,7 +314,8 @@ def _few_for(x, *weights):
 
 
 def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None, clear=None):
-    """project on linear_few.hip, or None where that does not take it."""
+    """project on linear_few.hip (of more rows a product or a unit on linear_tiles.hip),
+    or None where that does not take it."""
     ext = _few_for(x, weight)
     if ext is None:
         return None
@@ -341,8 +342,8 @@ def feed_few(x, w_in, w_out, act, norm=None, residual=None):
 def project(x, weight, bias=None, *, norm=None, act=None, residual=None, clear=None):
     """x W^T + bias, of x's rows as ``norm`` (an RMSNorm) makes them; ``act``:
     the gated unit act(gate) * up of the result's halves; plus ``residual``;
-    ``clear``: numbers (int32) that are zero afterwards.  One kernel for few rows, else
-    one for each of these."""
+    ``clear``: numbers (int32) that are zero afterwards.  One kernel for few rows, and for
+    many the product with its unit where that is faster, else one for each of these."""
     if x.is_cuda:
         y = _linear_few(x, weight, bias, residual, norm, act, clear)
         if y is not None:
@@ -370,7 +371,8 @@ def few_tokens(x: torch.Tensor) -> bool:
 
 
 def linear(x, weight, bias=None):
-    """Dense linear; up to 64 rows run on linear_few.hip where it takes them.  The MFMA
+    """Dense linear; up to 64 rows run on linear_few.hip where it takes them, more on
+    linear_tiles.hip where that is faster than the library.  The MFMA
     decode GEMV (MLXS_AMD_DENSE_GEMV=1) was a NEGATIVE result at batch-64 decode shapes:
     hipBLASLt's small-GEMM kernels run ~13 us in-graph and the split-K fp32-atomic
     traffic (M*O*4*nk bytes) rivals the weight bytes on small-O projections

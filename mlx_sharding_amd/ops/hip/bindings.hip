@@ -1457,6 +1457,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_rows_longest", [](int64_t bits) { return moe_rows_longest((int)bits); });
   m.def("moe_combine", &moe_combine);
   m.def("moe_tiles", &moe_tiles);
+  m.def("linear_tiles", &linear_tiles);
+  m.def("linear_tiles_plan", &linear_tiles_planned);
   m.def("mfma_probe", &mfma_probe);
   m.def("w4a16_gemv", &w4a16_gemv);
   m.def("w4f16_gemv", &w4f16_gemv);

@@ -1,5 +1,5 @@
-// y = x W^T for up to 64 rows, with what goes with it (linear_few.hip); part of
-// both extensions.
+// y = x W^T for up to 64 rows, with what goes with it (linear_few.hip), and for more
+// where linear_tiles.hip is the better one; part of both extensions.
 #pragma once
 
 #include <torch/extension.h>
@@ -11,6 +11,8 @@
 
 #include <cstdlib>
 #include <cstring>
+
+#include "linear_tiles.h"
 
 extern "C" void launch_linear_few(const void*, const void*, const void*,
                                   const void*, const void*, void*, int, int, int,
@@ -204,12 +206,73 @@ static torch::Tensor linear_few_shaped(const torch::Tensor& y, const torch::Tens
   return y.view(sizes);
 }
 
-// linear_few_run for x of any number of dimensions, or nothing where it does not run here.
+// Products of more rows (linear_tiles.hip): x [M, K], w [O, K] (act: [2 O, K]).
+static torch::Tensor linear_tiles(const torch::Tensor& x, const torch::Tensor& w,
+                                  const c10::optional<torch::Tensor>& bias, int64_t act,
+                                  int64_t tile, int64_t shares) {
+  TORCH_CHECK(linear_few_input(x) && linear_few_weight(w, x) && x.dim() == 2 &&
+                  x.size(1) == w.size(1) && act >= 0 && act <= 2 &&
+                  linear_few_along(x, w.size(0), w.size(0), bias, {}, {}),
+              "linear_tiles takes bf16 rows that begin at multiples of 16 bytes");
+  const long M = x.size(0), K = x.size(1), O = w.size(0) / (act ? 2 : 1);
+  TORCH_CHECK(M >= 1 && M < 1L << 30 && K % 64 == 0 && O % 64 == 0 && O >= 64 && K < 1L << 22 &&
+                  O < 1L << 30 && (!act || (w.size(0) == 2 * O && !bias)) && x.stride(0) >= K &&
+                  w.stride(0) >= K && x.stride(0) < 1L << 22 && w.stride(0) < 1L << 22 &&
+                  (tile == 128 || tile == 256) && shares >= 1 && (shares == 1 || !act) &&
+                  K / 64 / shares >= 3 && shares * M < 1L << 30,
+              "sizes that there is no kernel for");
+  c10::OptionalDeviceGuard guard;  // and the device's current stream
+  if (x.get_device() != c10::hip::current_device()) guard.reset_device(x.device());
+  auto y = torch::empty({M, O}, x.options());
+  torch::Tensor parts;
+  if (bias || shares > 1)
+    parts = torch::empty({shares, M, O}, x.options().dtype(torch::kFloat32));
+  LinearTilesArgs a{x.data_ptr(), w.data_ptr(), bias ? bias->data_ptr() : nullptr, y.data_ptr(),
+                    parts.defined() ? parts.data_ptr<float>() : nullptr, (int)M, (int)O, (int)K,
+                    (int)act, (int)shares, x.stride(0) * 2, w.stride(0) * 2};
+  launch_linear_tiles(&a, (int)tile, c10::hip::getCurrentHIPStream().stream());
+  return y;
+}
+
+// (tile, shares) of a product of M rows, tile 0 where it is the library's
+static std::pair<int64_t, int64_t> linear_tiles_planned(int64_t M, int64_t O, int64_t K,
+                                                        int64_t act, bool bias) {
+  int shares = 1;
+  const int tile = linear_tiles_plan(M, O, K, (int)act, bias, &shares);
+  return {tile, shares};
+}
+
+// The product of more than 64 rows, or nothing where it does not run here.
+static c10::optional<torch::Tensor> linear_many_try(const torch::Tensor& x,
+                                                    const torch::Tensor& w,
+                                                    const c10::optional<torch::Tensor>& bias,
+                                                    int64_t act) {
+  if (w.dim() != 2 || x.dim() < 1 || w.size(1) < 1 || x.size(-1) != w.size(1) ||
+      (act && w.size(0) % 2))
+    return {};
+  const long K = w.size(1), M = x.numel() / K, O = w.size(0) / (act ? 2 : 1);
+  if (M <= 64 || M >= 1L << 24) return {};
+  const auto [tile, shares] = linear_tiles_planned(M, O, K, act, bias.has_value());
+  if (!tile || !linear_few_input(x) || !linear_few_weight(w, x) || linear_few_other(K) ||
+      w.stride(0) < K || w.stride(0) >= 1L << 22 ||
+      !linear_few_along(x, w.size(0), w.size(0), bias, {}, {}))
+    return {};
+  const auto rows = linear_few_rows(x);
+  if (rows.stride(0) < K || rows.stride(0) >= 1L << 22) return {};
+  return linear_few_shaped(linear_tiles(rows, w, bias, act, tile, shares), x);
+}
+
+// linear_few_run for x of any number of dimensions (a product of more rows, on its own:
+// linear_tiles), or nothing where it does not run here.
 // clear: int32 numbers that are zero afterwards.
 static c10::optional<torch::Tensor> linear_few_try(
     torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
     c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> norm,
     double eps, double offset, int64_t act, c10::optional<torch::Tensor> clear) {
+  if (x.dim() && x.numel() > 64 * x.size(-1)) {
+    if (residual.has_value() || norm.has_value() || clear.has_value()) return {};
+    return linear_many_try(x, w, bias, act);
+  }
   if (!linear_few_takes(x, w, !residual.has_value() && !norm.has_value() && !act) ||
       !linear_few_along(x, w.size(0) / (act ? 2 : 1), w.size(0), bias, residual, norm))
     return {};

@@ -15,9 +15,10 @@ struct MoePlaceArgs {
   int pairs, top, experts, blocks, tile;
 };
 
-// What is made of the sums: themselves, silu(those with w) * those with w2, or
-// g sigmoid(alpha g) (u + 1) of both times scale[p], g at most `limit`, u within +-limit.
-enum MoeUnit { MT_SUMS = 0, MT_SILU = 1, MT_CLAMPED = 2 };
+// What is made of the sums: themselves, silu(those with w) * those with w2 (or gelu), or
+// g sigmoid(alpha g) (u + 1) of both times scale[p], g at most `limit`, u within +-limit;
+// or themselves in 32 bits.
+enum MoeUnit { MT_SUMS = 0, MT_SILU = 1, MT_CLAMPED = 2, MT_GELU = 3, MT_PARTS = 4 };
 
 // y[p, o] of x[token of p] . w[expert of p, o] (and w2).  K and O are multiples of 64, K
 // at least 128; rows of w begin at 16 bytes; offsets within x (tokens given) and within
@@ -32,6 +33,10 @@ struct MoeTilesArgs {
   long wstride;            // bytes from one expert's matrix to the next
   const float* scale;      // clamped: [pairs]
   float limit, alpha;
+  unsigned ldw;            // bytes from one row of w to the next
+  // dense: rows of x; parts of the contraction, and their sums [shares, rows, O]
+  int rows, shares;
+  float* parts;
 };
 
 extern "C" {

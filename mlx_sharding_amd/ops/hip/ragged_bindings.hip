@@ -843,6 +843,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("residual"), py::arg("norm"), py::arg("eps"), py::arg("offset"),
         py::arg("act"), py::arg("clear") = py::none());
   m.def("feed_few_try", &feed_few_try);
+  m.def("linear_tiles", &linear_tiles);
+  m.def("linear_tiles_plan", &linear_tiles_planned);
   m.def("clamped_glu", &clamped_glu, py::arg("gate"), py::arg("up"),
         py::arg("limit"), py::arg("alpha"), py::arg("gate_bias") = py::none(),
         py::arg("up_bias") = py::none());
