@@ -459,7 +459,7 @@ void delta_long(Tensor y, Tensor conv_w, Tensor A_log, Tensor dt,
     TORCH_CHECK(((uintptr_t)t->data_ptr()) % 8 == 0, "unaligned operand");
   const long nc = chunks.size(0);
   // depths 16 * 2^k take the walk with a fixed depth
-  long Dp = 16;
+  long Dp = 32;
   while (Dp < D) Dp *= 2;
   if (Dp > 128) Dp = (D + 15) / 16 * 16;
   const long Vp = (V + 15) / 16 * 16;

@@ -17,8 +17,9 @@
 //    outputs O = diag(exp G) Q S0 + A U, and the next state
 //    exp(G_last) S0 + K^T diag(exp(G_last - G)) U.  One kernel makes
 //    (I + L)^-1 diag(beta) and A of all chunks at once, a second walks the
-//    chunks of a (request, head, 16 or 32 value columns).  All products run on the
-//    fp32 matrix cores.
+//    chunks of a (request, head, 16 or 32 value columns).  Products run on the fp32
+//    matrix cores, those of the walk (depths of 32, 64 and 128) as six products of
+//    bf16 parts that keep all bits.
 //  * decays per channel: exp(G) is a vector then, and L and A sum
 //    k_i[d] k_j[d] exp(G_i[d] - G_j[d]) over channels.  Between the tokens of two
 //    neighbouring blocks, with the second block's begin as reference, that is a
@@ -1136,31 +1137,75 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(
   }
 }
 
-// The same walk with the state depth fixed at 16 * ND, CT column tiles a block, and
-// eight waves: four for the state (K S, then U, then the next S), four for the
-// outputs (Q S, A U), a SIMD has one of each.  Chunks follow one another, so what
-// counts is the way from one state to the next: three products with a barrier
-// behind each.  The matrix cores are at work for most of it, as the output waves
-// fill what the state waves leave.
-//   * K lies in LDS, once for its rows (K S) and its columns (the next S), and is
-//     loaded there a chunk ahead without registers; 16-byte pieces of a row are
-//     swapped by the row, so that neither way of reading meets banks twice.  All
-//     other operands are asked for a chunk ahead, too.
-//   * S, U and what leads to U lie transposed in LDS, [column][row]: one 16-byte
-//     access has what four products take or make.
-//   * column blocks of one (request, head) read the same operands and run on one
-//     XCD; two column tiles a block halve what comes out of its L2, where there are
-//     blocks enough.
-// CH: decays per channel; then K for the state (kt) is another array.
+// The same walk with the state depth fixed at 32 * KD, CT column tiles a block, and
+// eight waves: four for the state (K S, then U, then the next S), four for the outputs
+// (Q S, A U); a SIMD has one of each, and both split K of the next chunk.  Chunks follow
+// one another, so what counts is the way from one state to the next: three products with
+// a barrier behind each.
+//   * Every operand is a sum of three bf16 parts that keep all of its 24 bits, and a
+//     product is that of six pairs of parts, the smallest of which lies 2^-16 below the
+//     largest; what is left out lies below fp32's own rounding.  The matrix cores take
+//     16 times as many bf16 products as fp32 ones, 2.7 times as many of six.  Sums of the
+//     largest pair and of the others are kept apart until the end.
+//   * Parts of K lie in LDS, once for its rows (K S) and for its columns (the next S,
+//     read transposed), split there a chunk ahead; pieces of a row are swapped by the
+//     row, so that neither way of reading meets banks twice.
+//   * S, U and what leads to U lie transposed in LDS, [column][row], parts apart.
+//   * column blocks of one (request, head) read the same operands and run on one XCD;
+//     two column tiles a block halve what comes out of its L2, where there are blocks
+//     enough.
+// CH: decays per channel; K for the state (kt) is another array, split in the chunk
+// that it is for.
 // Rows past the end of a chunk repeat its last one: their beta is 0, so they write
 // nothing, and their outputs are not stored.
-// Bound by fp32 matrix products: 128 of a SIMD per chunk and tile, 1.7 us, of 3.4
-// (5.8 for two tiles); the rest is latency at the three barriers, and loads, which
-// take a third more of the first phase when they are all asked for at its start.
-// Depth 128, 16 heads, one block per column tile and four waves before: 2 x 4001
-// tokens 343 -> 229 us, 1 x 8192 641 -> 398, 8 x 1024 354 -> 184, 11 requests of 17
-// to 1160 212 -> 143; decays per channel, 2 x 4001 350 -> 285, 6 of 30 to 900 117 -> 92.
-template <typename T, int ND, int CT, bool CH>
+// Bound by what the two waves of a SIMD issue: of 8400 cycles a chunk (two tiles, depth
+// 128) 2900 are products, 3900 splits and what goes with them; with half of the products
+// it takes 12% less, with splits left out 23%.  All of K by the output waves: 9700.
+// Depth 128, 32 heads: 2 x 4001 tokens 390 -> 288 us with fp32 products before, 11
+// requests of 17 to 1160 233 -> 171; decays per channel, 16 heads, 13 of 9 to 900
+// 122 -> 99.  Errors of a layer against 64 bits .94 to .99 of those before.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// eight numbers in three bf16 parts each, rounded: the third is exact
+struct Parts8 {
+  bf16x8 p[3];
+};
+// The next bf16 part of two numbers, cut off; else rounded.  Of a product one side is cut
+// off and the other rounded: what is left out then has no sign of its own.
+__device__ __forceinline__ unsigned cut_pair(float& x, float& y, bool more) {
+  const unsigned a = __float_as_uint(x), b = __float_as_uint(y);
+  if (more) {
+    x -= __uint_as_float(a & 0xFFFF0000u);
+    y -= __uint_as_float(b & 0xFFFF0000u);
+  }
+  return __builtin_amdgcn_perm(b, a, 0x07060302);
+}
+__device__ __forceinline__ unsigned round_pair(float& x, float& y, bool more) {
+  const unsigned p = __builtin_bit_cast(unsigned, bf16x2{(__bf16)x, (__bf16)y});
+  if (more) {
+    x -= __uint_as_float(p << 16);
+    y -= __uint_as_float(p & 0xFFFF0000u);
+  }
+  return p;
+}
+template <bool CUT, int N, typename V>
+__device__ __forceinline__ void split3(float (&v)[N], V (&to)[3]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    unsigned pairs[N / 2];
+#pragma unroll
+    for (int j = 0; j < N; j += 2)
+      pairs[j / 2] = CUT ? cut_pair(v[j], v[j + 1], i < 2) : round_pair(v[j], v[j + 1], i < 2);
+    to[i] = __builtin_bit_cast(V, pairs);
+  }
+}
+__device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, Parts8& to) {
+  float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  split3<true>(v, to.p);
+}
+
+template <typename T, int KD, int CT, bool CH>
 __global__ __launch_bounds__(512, 2) void delta_walk_fixed_kernel(
     const float* __restrict__ qn, const float* __restrict__ kn,
     const float* __restrict__ ktn, const T* __restrict__ vn, const float* __restrict__ tm,
@@ -1169,11 +1214,11 @@ __global__ __launch_bounds__(512, 2) void delta_walk_fixed_kernel(
     const int* __restrict__ chunks, const int* __restrict__ chunk_cu,
     const int* __restrict__ pos0, const int* __restrict__ slots, int n_short,
     int tok_base, int n_long, int KH, int H, int D, int V, int Vp) {
-  constexpr int Dp = ND * 16;
-  constexpr int NT = (ND + 3) / 4;       // state row tiles per wave
-  constexpr int KP = Dp / 4;             // 16-byte pieces of a row of K
-  constexpr int KW = DR_CHUNK * Dp;      // one chunk of K
-  constexpr int SS = Dp + 4, US = DR_CHUNK + 4;
+  constexpr int Dp = KD * 32, ND = Dp / 16;
+  constexpr int NT = (ND + 3) / 4;         // state row tiles per wave
+  constexpr int KB = DR_CHUNK * Dp * 2;    // bytes of one part of a chunk of K
+  constexpr int SB = CT * 16 * Dp * 2;     // ... of the state
+  constexpr int UB = CT * 16 * DR_CHUNK * 2;  // ... of U
   const int cols = Vp / (16 * CT), pairs = H * n_long;
   int pair = blockIdx.x / cols, vt = blockIdx.x % cols;
   if (pairs % 8 == 0) {  // blocks go round the XCDs
@@ -1190,29 +1235,42 @@ __global__ __launch_bounds__(512, 2) void delta_walk_fixed_kernel(
   const int lr = lane & 15, g4 = lane >> 4;
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  float* kl = reinterpret_cast<float*>(smem);    // [2][64][Dp] K
-  float* kc = kl + 2 * KW;                       // [64][Dp] kt (CH)
-  float* st = kl + (CH ? 3 : 2) * KW;            // [CT][16][SS] state
-  float* xt = st + CT * 16 * SS;                 // [CT][16][US] V - exp(G) K S
-  float* ut = xt + CT * 16 * US;                 // [CT][16][US] U
-  float* wt = ut + CT * 16 * US;                 // ... exp(G_last - G) U
+  char* const kl = smem;              // [2][3][64][Dp] K by turns; CH: K, kt
+  char* const st = kl + 6 * KB;       // [3][CT * 16][Dp] state
+  char* const xt = st + 3 * SB;       // [3][CT * 16][64] V - exp(G) K S
+  char* const ut = xt + 3 * UB;       // U
+  char* const wt = ut + 3 * UB;       // exp(G_last - G) U (CH: U), tokens as K is read
 
-  // place of a piece in a row's LDS
-  auto place = [](int row, int piece) { return piece ^ (row & (KP < 16 ? KP - 1 : 15)); };
-  // one of PARTS pieces that this wave brings of a chunk of K.  Offsets in a chunk are
-  // 32 bits wide.
-  constexpr int PARTS = (KW / 256 + 7) / 8;
-  const unsigned krow = KH * Dp * 4;
-  auto stage = [&](const float* src, float* dst, int i0, int len, int i) {
-    const char* from = reinterpret_cast<const char*>(src + ((long)i0 * KH + kh) * Dp);
-    const int part = i * 8 + wid;
-    if (KW / 256 % 8 && part >= KW / 256) return;
-    const int at = part * 64 + lane, row = at / KP;
-    __builtin_amdgcn_global_load_lds(
-        (const __attribute__((address_space(1))) void*)(
-            from + (unsigned)min(row, len - 1) * krow +
-            (unsigned)place(row, at % KP) * 16),
-        (__attribute__((address_space(3))) void*)(dst + part * 256), 16, 0, 0);
+  // byte of an element in rows of Dp, by pieces of 32 bytes, and in rows of 64 tokens, by
+  // pieces of 16
+  auto deep = [](int row, int d) {
+    return row * Dp * 2 + (((d >> 4) ^ (row & (ND < 8 ? ND - 1 : 7))) << 5) + (d & 15) * 2;
+  };
+  auto wide = [](int col, int i) {
+    return col * 128 + (((i >> 3) ^ (col & 7)) << 4) + (i & 7) * 2;
+  };
+  auto get8 = [](const char* p, int part, Parts8& to) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) to.p[i] = *reinterpret_cast<const bf16x8*>(p + i * part);
+  };
+  auto put4 = [](auto cut, const f32x4& x, char* p, int part) {
+    float v[4] = {x[0], x[1], x[2], x[3]};
+    bf16x4 to[3];
+    split3<decltype(cut)::value>(v, to);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x4*>(p + i * part) = to[i];
+  };
+  // a product of CT tiles; small: sums of all pairs of parts but the largest
+  auto product = [](const Parts8& a, const Parts8 (&b)[CT], f32x4 (&sum)[CT],
+                    f32x4 (&small)[CT]) {
+    constexpr int I[6] = {0, 2, 1, 0, 0, 1}, J[6] = {2, 0, 1, 0, 1, 0};
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+        f32x4& to = q == 3 ? sum[t] : small[t];
+        to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[I[q]], b[t].p[J[q]], to, 0, 0, 0);
+      }
   };
 
   // the two kinds of waves have loops of their own, with the same barriers
@@ -1232,292 +1290,334 @@ __global__ __launch_bounds__(512, 2) void delta_walk_fixed_kernel(
         for (int r = 0; r < 4; ++r)
           own[n][t][r] = keeps && !fresh && d0 + r < D && v < V
                              ? sg[(long)(d0 + r) * V + v] : 0.0f;
-        if (keeps && d0 < Dp) store4(st + (t * 16 + lr) * SS + d0, own[n][t]);
+        if (keeps && d0 < Dp) put4(std::false_type{}, own[n][t], st + deep(t * 16 + lr, d0), SB);
       }
     }
 
-    const long rstride = (long)KH * Dp;
     const int row = w * 16 + lr;              // A-operand row
     const int row_c = w * 16 + g4 * 4;        // first C row
-
-    const unsigned vrow = H * Vp;
+    const unsigned vrow = H * Vp, krow = KH * Dp;  // from row to row
     // 0, unknown to the compiler: scalar loads come in any order, and a wait for LDS
     // would be one for all of them
     unsigned nought = 0;
     asm volatile("" : "+v"(nought));
-    // what comes a chunk ahead: T or A, rows of Q (output waves), V and decays
+    // what comes a chunk ahead: T or A, rows of Q and K (output waves), V and decays
     struct Ahead {
-      f32x4 m[4], q[ND], gr, gl, gd[NT];
+      f32x4 m[4], gr, gl, gd[NT], q[2 * KD], k[KD], kt[CH ? KD : 1];
       T v[CT][4];
       float all;
     };
-    // in pieces, to go between the products: asked for at once they stand in the way
-    constexpr int PIECES = PARTS + 5 + (keeps ? CT : ND);
-    auto fetch = [&](Ahead& f, float* kd, int c, int i0, int len, int i) {
-      const long ch = (long)c * H + h;
-      const float* gc = ge + ch * (CH ? Dp : 128);
-      if (i < PARTS) {
-        stage(kn, kd, i0, len, i);
-      } else if (i < PARTS + 4) {
-        const int j = i - PARTS;
-        const float* mp = (keeps ? tm : am) + ch * 4096;
-        if (j <= w) f.m[j] = load4(mp + (unsigned)(row * 64 + g4 * 4 + j * 16));
-      } else if (i == PARTS + 4) {
-        if (!CH) f.gr = load4(gc + (unsigned)row_c);
-        if constexpr (keeps) {
-          if (!CH) {
-            f.gl = load4(gc + (unsigned)(64 + row_c));
-            f.all = gc[63 + nought];
-          } else {
+    // what is above is asked for before what follows is begun
+    auto issued = [] { __builtin_amdgcn_sched_barrier(0); };
+    // a lane's pieces of 4 columns of this wave's 8 rows of K: a load takes whole lines
+    constexpr int PR = Dp / 4;                // pieces of a row
+    auto k_row = [&](int s) { return wid * 8 + s * (64 / PR) + lane / PR; };
+    auto fetch_k = [&](const float* src, f32x4* to, int i0, int len) {
+      const float* from = src + ((long)i0 * KH + kh) * Dp + lane % PR * 4;
 #pragma unroll
-            for (int n = 0; n < NT; ++n) {
-              const int d0 = w * 16 + n * 64;
-              if (d0 < Dp) f.gd[n] = load4(gc + (unsigned)(d0 + g4 * 4));
-            }
-          }
-        }
-      } else if constexpr (keeps) {
-        const int t = i - PARTS - 5;
-        const T* vp = vn + ((long)i0 * H + h) * Vp + v0;
+      for (int s = 0; s < KD; ++s)
+        to[s] = load4(from + (unsigned)min(k_row(s), len - 1) * krow);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto put_k = [&](const f32x4* k, char* to) {
+      float v[4 * KD];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          f.v[t][r] = vp[(unsigned)min(row_c + r, len - 1) * vrow + (unsigned)(t * 16 + lr)];
-      } else {
-        const int d = i - PARTS - 5;
-        const float* qp = qn + ((long)i0 * KH + kh) * Dp;
-        f.q[d] = load4(qp + (unsigned)min(row, len - 1) * (krow / 4) +
-                       (unsigned)(d * 16 + g4 * 4));
+      for (int i = 0; i < 4 * KD; ++i) v[i] = k[i / 4][i % 4];
+      // part by part: a wave alone would wait for each of its steps
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        unsigned pairs[2 * KD];
+#pragma unroll
+        for (int j = 0; j < 2 * KD; ++j) pairs[j] = cut_pair(v[2 * j], v[2 * j + 1], i < 2);
+        issued();
+#pragma unroll
+        for (int s = 0; s < KD; ++s)
+          *reinterpret_cast<uint2*>(to + i * KB + deep(k_row(s), lane % PR * 4)) =
+              uint2{pairs[2 * s], pairs[2 * s + 1]};
       }
     };
-    // a barrier for what waves wrote into LDS; loads on their way there for the next
-    // chunk, which __syncthreads would wait for, go on
-    auto sync_lds = [] {
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // What comes a chunk ahead is asked for piece by piece, between products: a wave that
+    // asks for all at once waits for the loads before it (4400 cycles of 11700 a chunk).
+    auto fetch_m = [&](Ahead& f, int c) {
+      const long ch = (long)c * H + h;
+      const float* mp = (keeps ? tm : am) + ch * 4096 + row * 64 + g4 * 8;
+      f.m[0] = load4(mp);
+      f.m[1] = load4(mp + 4);
+      if (w >= 2) {
+        f.m[2] = load4(mp + 32);
+        f.m[3] = load4(mp + 36);
+      }
       __builtin_amdgcn_sched_barrier(0);
     };
-    // loads above stay above: what follows finds its operands under way
-    auto issued = [] { __builtin_amdgcn_sched_barrier(0); };
+    auto fetch_g = [&](Ahead& f, int c) {
+      const float* gc = ge + ((long)c * H + h) * (CH ? Dp : 128);
+      if (!CH) f.gr = load4(gc + row_c);
+      if constexpr (keeps) {
+        if constexpr (!CH) {
+          f.gl = load4(gc + 64 + row_c);
+          f.all = gc[63 + nought];
+        } else {
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            const int d0 = w * 16 + n * 64;
+            if (d0 < Dp) f.gd[n] = load4(gc + d0 + g4 * 4);
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto fetch_v = [&](Ahead& f, int i0, int len, int t) {
+      const T* vp = vn + ((long)i0 * H + h) * Vp + v0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        f.v[t][r] = vp[(unsigned)min(row_c + r, len - 1) * vrow + (unsigned)(t * 16 + lr)];
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto fetch_q = [&](Ahead& f, int i0, int len, int d) {
+      const float* qp = qn + ((long)i0 * KH + kh) * Dp + (unsigned)min(row, len - 1) * krow +
+                        g4 * 8;
+      f.q[2 * d] = load4(qp + d * 32);
+      f.q[2 * d + 1] = load4(qp + d * 32 + 4);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // a barrier for what waves wrote into LDS; loads to registers go on
+    auto sync_lds = [] {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
 
     const int c_end = chunk_cu[e + 1];
     int c = chunk_cu[e];
     int i0 = chunks[2 * c] - tok_base, len = chunks[2 * c + 1];
     int cn = min(c + 1, c_end - 1);  // the last one is fetched twice
     int j0 = chunks[2 * cn] - tok_base, jl = chunks[2 * cn + 1];
-    Ahead now = {}, next = {};
-    float vf[CT][4];
-    auto arrived = [&] {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      now = next;
-      // made here, so that no later use waits for the loads behind these
-      auto here = [](auto& x) { asm volatile("" : "+v"(x)); };
+    Ahead now = {};
+    fetch_m(now, c);
+    fetch_g(now, c);
+    if constexpr (keeps) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) here(now.m[j]);
-      if (!CH) here(now.gr);
-      if constexpr (keeps) {
-        if (!CH) here(now.gl);
-        if (!CH) here(now.all);
+      for (int t = 0; t < CT; ++t) fetch_v(now, i0, len, t);
+    } else {
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
-          if (CH) here(now.gd[n]);
-#pragma unroll
-        for (int t = 0; t < CT; ++t)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            vf[t][r] = (float)now.v[t][r];
-            here(vf[t][r]);
-          }
-      } else {
-#pragma unroll
-        for (int d = 0; d < ND; ++d) here(now.q[d]);
-      }
-    };
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) fetch(next, kl, c, i0, len, i);
-    auto stage_kt = [&](int i0, int len) {
-#pragma unroll
-      for (int i = 0; i < PARTS; ++i) stage(ktn, kc, i0, len, i);
-    };
-    if (CH) stage_kt(i0, len);
-    arrived();
+      for (int d = 0; d < KD; ++d) fetch_q(now, i0, len, d);
+    }
+    fetch_k(kn, now.k, i0, len);
+    if constexpr (CH) fetch_k(ktn, now.kt, i0, len);
+    put_k(now.k, kl);
     __syncthreads();
 
     for (int buf = 0; c < c_end; ++c, buf ^= 1) {
       const int ahead = min(cn + 1, c_end - 1);
       const int* then = chunks + 2 * (ahead + nought);  // at any multiple of 4 bytes
       const int then_row = then[0], then_len = then[1];
-      const float* k = kl + buf * KW;
+      Ahead next = {};
+      const char* k = kl + (CH ? 0 : buf * 3 * KB);
+      const char* kt = kl + (CH ? 3 : buf * 3) * KB;
 
-      f32x4 acc[CT];
+      f32x4 acc[CT], low[CT];
 #pragma unroll
-      for (int t = 0; t < CT; ++t) acc[t] = zero;
-      // rows of K or Q times the state for pieces FROM to TO of the depth, GR of
-      // them under way while others are in the matrix cores
-      auto rows_of = [&](auto from, auto to) {
-        constexpr int F = decltype(from)::value, E = decltype(to)::value;
-        constexpr int GR = CT == 1 ? 4 : 2;
-        f32x4 a[E - F], b[E - F][CT];
-        auto read = [&](int d) {
-          if constexpr (keeps)
-            a[d - F] = load4(k + row * Dp + place(row, d * 4 + g4) * 4);
+      for (int t = 0; t < CT; ++t) acc[t] = low[t] = zero;
+      // Rows of K or Q times the state, 32 of the depth at a time.  Reads stand well ahead
+      // of the products, and splitting between them.
+      Parts8 ra[keeps ? 2 : 1], rb[2][CT];
+      auto read = [&](int d) {
+        if constexpr (keeps) get8(k + deep(row, d * 32 + g4 * 8), KB, ra[d & 1]);
 #pragma unroll
-          for (int t = 0; t < CT; ++t)
-            b[d - F][t] = load4(st + (t * 16 + lr) * SS + d * 16 + g4 * 4);
-        };
-#pragma unroll
-        for (int d = F; d < E && d < F + GR; ++d) read(d);
+        for (int t = 0; t < CT; ++t)
+          get8(st + deep(t * 16 + lr, d * 32 + g4 * 8), SB, rb[d & 1][t]);
         issued();
-#pragma unroll
-        for (int d0 = F; d0 < E; d0 += GR) {
-#pragma unroll
-          for (int d = d0 + GR; d < d0 + 2 * GR && d < E; ++d) read(d);
-          issued();
-#pragma unroll
-          for (int d = d0; d < d0 + GR && d < E; ++d) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-              for (int t = 0; t < CT; ++t)
-                acc[t] = mma4(keeps ? a[d - F][s] : now.q[d][s], b[d - F][t][s], acc[t]);
-            issued();
-            constexpr int per = (PIECES + ND - 1) / ND;
-#pragma unroll
-            for (int i = d * per; i < (d + 1) * per && i < PIECES; ++i)
-              fetch(next, kl + (buf ^ 1) * KW, cn, j0, jl, i);
-            issued();
-          }
+      };
+      auto rows_of = [&](int d) {
+        if constexpr (keeps) {
+          product(ra[d & 1], rb[d & 1], acc, low);
+        } else {
+          split8(now.q[2 * d], now.q[2 * d + 1], ra[0]);
+          product(ra[0], rb[d & 1], acc, low);
         }
-      };
-      // the matrix of this wave times columns of `x`
-      auto lower = [&](const float* x, f32x4 (&to)[CT]) {
-        f32x4 b[4][CT];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int t = 0; t < CT; ++t)
-            b[j][t] = load4(x + (t * 16 + lr) * US + j * 16 + g4 * 4);
         issued();
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (j <= w) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-              for (int t = 0; t < CT; ++t) to[t] = mma4(now.m[j][s], b[j][t][s], to[t]);
-          }
       };
-      using std::integral_constant;
+      // the matrix of this wave, whose tiles above the diagonal are not there
+      Parts8 m[2];
+      auto matrix = [&] {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const bool there = j * 2 + (g4 >> 1) <= w;
+          split8(there ? now.m[2 * j] : zero, there ? now.m[2 * j + 1] : zero, m[j]);
+        }
+        issued();
+      };
+      // ... times columns of `x`
+      Parts8 lb[2][CT];
+      auto read_lower = [&](const char* x) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int t = 0; t < CT; ++t) get8(x + wide(t * 16 + lr, j * 32 + g4 * 8), UB, lb[j][t]);
+        issued();
+      };
+      auto lower = [&](f32x4 (&to)[CT], f32x4 (&small)[CT]) {
+        product(m[0], lb[0], to, small);
+        if (w >= 2) product(m[1], lb[1], to, small);
+      };
+      constexpr int HALF = (KD + 1) / 2;  // of the output waves' steps, in the first phase
       if constexpr (keeps) {
-        rows_of(integral_constant<int, 0>{}, integral_constant<int, ND>{});
+        read(0);
+        if (KD > 1) read(1);
+        float vf[CT][4];
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) vf[t][r] = (float)now.v[t][r];
+        matrix();
+#pragma unroll
+        for (int d = 0; d < KD; ++d) {
+          rows_of(d);
+          if (d + 2 < KD) read(d + 2);
+        }
+        fetch_g(next, cn);
+        fetch_k(kn, next.k, j0, jl);
+        if constexpr (CH) put_k(now.kt, kl + 3 * KB);
 #pragma unroll
         for (int t = 0; t < CT; ++t) {
           f32x4 x;
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            x[r] = vf[t][r] - (CH ? acc[t][r] : now.gr[r] * acc[t][r]);
-          store4(xt + (t * 16 + lr) * US + row_c, x);
+          for (int r = 0; r < 4; ++r) {
+            const float s = acc[t][r] + low[t][r];
+            x[r] = vf[t][r] - (CH ? s : now.gr[r] * s);
+          }
+          put4(std::false_type{}, x, xt + wide(t * 16 + lr, row_c), UB);
         }
       } else {
-        rows_of(integral_constant<int, 0>{}, integral_constant<int, (ND + 1) / 2>{});
+#pragma unroll
+        for (int d = 0; d < HALF; ++d) read(d);
+        if constexpr (CH) put_k(now.kt, kl + 3 * KB);
+        fetch_g(next, cn);
+        fetch_k(kn, next.k, j0, jl);
+#pragma unroll
+        for (int d = 0; d < HALF; ++d) rows_of(d);
       }
       sync_lds();
 
-      float ka[NT][4][4];  // columns of kt
-      if constexpr (keeps) {
-        f32x4 u[CT];
+      // columns of kt: four tokens of one column out of rows, a lane's of 32 are
+      // 4 g4 .. + 3 and 16 more
+      Parts8 ka[NT][2];
+      auto columns = [&] {
+        const char* from = kt;
 #pragma unroll
-        for (int t = 0; t < CT; ++t) u[t] = zero;
-        if (!CH) {
+        for (int n = 0; n < NT; ++n) {
+          const int d0 = min(w * 16 + n * 64, Dp - 16);
 #pragma unroll
-          for (int n = 0; n < NT; ++n)
+          for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int i = 0; i < 3; ++i) {
+              s16x4 v[2];
 #pragma unroll
-              for (int s = 0; s < 4; ++s) {
-                const int i = j * 16 + g4 * 4 + s, d = min(w * 16 + n * 64, Dp - 16) + lr;
-                ka[n][j][s] = k[i * Dp + place(i, d >> 2) * 4 + (lr & 3)];
+              for (int q = 0; q < 2; ++q) {
+                const int token = j * 32 + q * 16 + g4 * 4 + (lr >> 2);
+                v[q] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) s16x4*)(
+                        from + i * KB + deep(token, d0 + (lr & 3) * 4)));
               }
+              ka[n][j].p[i] = __builtin_bit_cast(
+                  bf16x8, __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7));
+            }
         }
-        lower(xt, u);
+      };
+      // place of four tokens of a row as columns() has them
+      const int turned = (w >> 1) * 32 + g4 * 8 + (w & 1) * 4;
+      if constexpr (keeps) {
+        f32x4 u[CT], small[CT];
+#pragma unroll
+        for (int t = 0; t < CT; ++t) u[t] = small[t] = zero;
+        read_lower(xt);
+        if (!CH) columns();
+        issued();
+        lower(u, small);
+        fetch_m(next, cn);
+        if constexpr (CH) fetch_k(ktn, next.kt, j0, jl);
 #pragma unroll
         for (int t = 0; t < CT; ++t) {
-          store4(ut + (t * 16 + lr) * US + row_c, u[t]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) u[t][r] += small[t][r];
+          put4(std::false_type{}, u[t], ut + wide(t * 16 + lr, row_c), UB);
           if (!CH) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) u[t][r] *= now.gl[r];
-            store4(wt + (t * 16 + lr) * US + row_c, u[t]);
           }
+          put4(std::false_type{}, u[t], wt + wide(t * 16 + lr, turned), UB);
         }
       } else {
-        if constexpr (ND > 1)
-          rows_of(integral_constant<int, (ND + 1) / 2>{}, integral_constant<int, ND>{});
-        if (!CH) {
 #pragma unroll
-          for (int t = 0; t < CT; ++t)
+        for (int d = HALF; d < KD; ++d) read(d);
+        matrix();
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[t][r] *= now.gr[r];
-        }
+        for (int d = HALF; d < KD; ++d) rows_of(d);
+        if constexpr (CH) fetch_k(ktn, next.kt, j0, jl);
+#pragma unroll
+        for (int d = 0; d < HALF; ++d) fetch_q(next, j0, jl, d);
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            acc[t][r] += low[t][r];
+            low[t][r] = 0.0f;
+            if (!CH) acc[t][r] *= now.gr[r];
+          }
       }
-      if (CH) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // kt of this chunk
       sync_lds();
 
       if constexpr (keeps) {
-        const float* uw = CH ? ut : wt;
-        f32x4 b[4][CT];
+        if (CH) columns();
+        Parts8 b[2][CT];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int t = 0; t < CT; ++t)
-            b[j][t] = load4(uw + (t * 16 + lr) * US + j * 16 + g4 * 4);
-        if (CH) {
-#pragma unroll
-          for (int n = 0; n < NT; ++n)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-              for (int s = 0; s < 4; ++s) {
-                const int i = j * 16 + g4 * 4 + s, d = min(w * 16 + n * 64, Dp - 16) + lr;
-                ka[n][j][s] = kc[i * Dp + place(i, d >> 2) * 4 + (lr & 3)];
-              }
-        }
+          for (int t = 0; t < CT; ++t) get8(wt + wide(t * 16 + lr, j * 32 + g4 * 8), UB, b[j][t]);
         issued();
+        f32x4 small[NT][CT];
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
-          for (int t = 0; t < CT; ++t)
+          for (int t = 0; t < CT; ++t) {
+            small[n][t] = zero;
 #pragma unroll
             for (int r = 0; r < 4; ++r) own[n][t][r] *= CH ? now.gd[n][r] : now.all;
+          }
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int s = 0; s < 4; ++s)
+          for (int n = 0; n < NT; ++n) product(ka[n][j], b[j], own[n], small[n]);
 #pragma unroll
-            for (int n = 0; n < NT; ++n)
-#pragma unroll
-              for (int t = 0; t < CT; ++t)
-                own[n][t] = mma4(ka[n][j][s], b[j][t][s], own[n][t]);
+        for (int t = 0; t < CT; ++t) fetch_v(next, j0, jl, t);
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
           const int d0 = w * 16 + n * 64;
           if (d0 >= Dp) continue;
 #pragma unroll
-          for (int t = 0; t < CT; ++t)
-            store4(st + (t * 16 + lr) * SS + d0 + g4 * 4, own[n][t]);
+          for (int t = 0; t < CT; ++t) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) own[n][t][r] += small[n][t][r];
+            put4(std::false_type{}, own[n][t], st + deep(t * 16 + lr, d0 + g4 * 4), SB);
+          }
         }
+        put_k(next.k, kl + (CH ? 0 : (buf ^ 1) * 3 * KB));
       } else {
-        lower(ut, acc);
+        read_lower(ut);
+        put_k(next.k, kl + (CH ? 0 : (buf ^ 1) * 3 * KB));
+        issued();
+        lower(acc, low);
+        fetch_m(next, cn);
+#pragma unroll
+        for (int d = HALF; d < KD; ++d) fetch_q(next, j0, jl, d);
         float* op = o + ((long)i0 * H + h) * Vp + v0;
 #pragma unroll
         for (int t = 0; t < CT; ++t)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            if (row_c + r < len) op[(unsigned)(row_c + r) * vrow + t * 16 + lr] = acc[t][r];
+            if (row_c + r < len)
+              op[(unsigned)(row_c + r) * vrow + t * 16 + lr] = acc[t][r] + low[t][r];
       }
-      arrived();
-      __syncthreads();
-      // all have read this chunk's kt
-      if (CH && c + 1 < c_end) stage_kt(j0, jl);
+      sync_lds();
+      now = next;
       i0 = j0;
       len = jl;
       cn = ahead;
@@ -1619,35 +1719,33 @@ struct DeltaLongArgs {
   float eps;
 };
 
-template <typename T, int ND, int CT, bool CH>
+template <typename T, int KD, int CT, bool CH>
 static void delta_walk_tiles(const DeltaLongArgs& a, const DeltaDims& dm,
                              const float* q, const float* k, const float* kt,
                              int KH, hipStream_t stream) {
-  const size_t smem =
-      ((CH ? 3 : 2) * DR_CHUNK * ND * 16 +
-       CT * 16 * (ND * 16 + 4 + 3 * (DR_CHUNK + 4))) * sizeof(float);
+  // three parts of two bytes: K twice, the state, and X, U and W
+  const int smem = 6 * (2 * DR_CHUNK * KD * 32 + CT * 16 * (KD * 32 + 3 * DR_CHUNK));
   if (smem > 65536)
     (void)hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&delta_walk_fixed_kernel<T, ND, CT, CH>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+        reinterpret_cast<const void*>(&delta_walk_fixed_kernel<T, KD, CT, CH>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   const dim3 grid((unsigned)(a.Vp / (16 * CT) * dm.H * a.n_long));
-  delta_walk_fixed_kernel<T, ND, CT, CH><<<grid, dim3(512), smem, stream>>>(
+  delta_walk_fixed_kernel<T, KD, CT, CH><<<grid, dim3(512), smem, stream>>>(
       q, k, kt, (const T*)a.vn, a.tm, a.am, a.ge, a.state, a.o, a.chunks,
       a.chunk_cu, a.pos0, a.slots, a.n_short, a.tok_base, a.n_long, KH, dm.H, dm.D,
       dm.V, a.Vp);
 }
 
-template <typename T, int ND, bool CH>
+template <typename T, int KD, bool CH>
 static void delta_walk_go(const DeltaLongArgs& a, const DeltaDims& dm,
                           const float* q, const float* k, const float* kt, int KH,
                           hipStream_t stream) {
-  // A CU has one block, so with more than 256 column tiles two of them a block: 32
-  // chunks of 4 requests, 16 heads, 231 us with one, 186 with two; at 256 (2 requests
-  // of 63 chunks) 228 and 344.
+  // A CU has one block, so with more than 256 column tiles two of them a block (a chunk of
+  // two takes 1.3 times as long as of one).
   if (a.Vp % 32 == 0 && (long)a.Vp / 16 * dm.H * a.n_long > 256) {
-    delta_walk_tiles<T, ND, 2, CH>(a, dm, q, k, kt, KH, stream);
+    delta_walk_tiles<T, KD, 2, CH>(a, dm, q, k, kt, KH, stream);
   } else {
-    delta_walk_tiles<T, ND, 1, CH>(a, dm, q, k, kt, KH, stream);
+    delta_walk_tiles<T, KD, 1, CH>(a, dm, q, k, kt, KH, stream);
   }
 }
 
@@ -1658,10 +1756,9 @@ static void delta_walk_t(const DeltaLongArgs& a, const DeltaDims& dm,
                          dim3 grid, hipStream_t stream) {
   const dim3 block(256);
 #define DW_GO(N) delta_walk_go<T, N, CH>(a, dm, q, k, kt, KH, stream)
-  if (a.Dp == 16) DW_GO(1);
-  else if (a.Dp == 32) DW_GO(2);
-  else if (a.Dp == 64) DW_GO(4);
-  else if (a.Dp == 128) DW_GO(8);
+  if (a.Dp == 32) DW_GO(1);
+  else if (a.Dp == 64) DW_GO(2);
+  else if (a.Dp == 128) DW_GO(4);
   else {
     const size_t smem = ((size_t)a.Dp + 3 * 64) * 17 * sizeof(float);
     delta_walk_kernel<T, CH><<<grid, block, smem, stream>>>(
