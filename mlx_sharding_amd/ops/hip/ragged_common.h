@@ -38,10 +38,6 @@ struct Frag<__bf16> {
     bf16x4 b = *reinterpret_cast<const bf16x4*>(p1);
     v = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
   }
-  __device__ __forceinline__ void load_strided(const __bf16* p, int stride) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = p[j * stride];
-  }
 };
 
 template <>
@@ -54,13 +50,6 @@ struct Frag<float> {
   __device__ __forceinline__ void load44(const float* p0, const float* p1) {
     a = *reinterpret_cast<const f32x4*>(p0);
     b = *reinterpret_cast<const f32x4*>(p1);
-  }
-  __device__ __forceinline__ void load_strided(const float* p, int stride) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      a[j] = p[j * stride];
-      b[j] = p[(j + 4) * stride];
-    }
   }
 };
 

@@ -14,6 +14,29 @@
 #define LA_KT 32  // keys per tile, absorbed
 #define LA_MAXSPLIT WAVE
 
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// Column lr of 32 rows of 16 columns, rows lg*4 + 0..3 and 16 + lg*4 + 0..3.
+__device__ __forceinline__ void load_columns(Frag<__bf16>& f, const __bf16* p,
+                                             int stride, int lr, int lg) {
+  const __bf16* src = p + (lg * 4 + (lr >> 2)) * stride + (lr & 3) * 4;
+  const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s16x4*)src);
+  const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s16x4*)(src + 16 * stride));
+  f.v = __builtin_bit_cast(
+      bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+__device__ __forceinline__ void load_columns(Frag<float>& f, const float* p,
+                                             int stride, int lr, int lg) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    f.a[j] = p[(lg * 4 + j) * stride + lr];
+    f.b[j] = p[(16 + lg * 4 + j) * stride + lr];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Absorbed.  A query row is one (token, head) pair of one request; a block
 // serves 16 rows of one request over one slice of its keys.  The key tile is
@@ -21,6 +44,12 @@
 // (values).  Scores are computed transposed (keys x rows), so a lane holds
 // one query row and the softmax needs two shuffles.
 //   grid (short requests, splits, row tiles)
+// A slice is a few tiles, so latency bounds it: a thread asks for its whole
+// share of a tile at once, into registers, and for the next tile before it
+// works on this one.  Columns of the values come from transposing LDS reads,
+// whose order of the keys is that of the scores' accumulators.  12 requests of
+// up to 1300 keys, 16 heads, rank 512 + 64: 12.9 us (28.9 us with pieces asked
+// for one after the other and columns read value by value).
 // ND: 16-wide latent column tiles per wave; rankp == 64 * ND.
 // ---------------------------------------------------------------------------
 
@@ -53,7 +82,6 @@ __global__ __launch_bounds__(LA_BLOCK) void latent_attn_short_kernel(
 
   const int W = rankp + rotp;
   const int WS = W + 8;
-  const int nvec = W / 8;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   T* qs = reinterpret_cast<T*>(smem);    // [16][WS]
   T* ks = qs + 16 * WS;                  // [LA_KT][WS]
@@ -64,15 +92,71 @@ __global__ __launch_bounds__(LA_BLOCK) void latent_attn_short_kernel(
   const int wid = tid / WAVE;
   const int lr = lane & 15, lg = lane >> 4;
 
-  for (int i = tid; i < 16 * nvec; i += LA_BLOCK) {
-    const int r = i / nvec, c = (i - r * nvec) * 8;
-    const int row = min(r0 + r, rows - 1);
+  // pieces of 8 values: of the latent part ND a thread and tile, of the
+  // rotated part one (those past the first 64 columns are copied directly)
+  typedef T T8 __attribute__((ext_vector_type(8)));
+  constexpr int LV = 8 * ND;
+  constexpr int NQ = (16 * LV + LA_BLOCK - 1) / LA_BLOCK;
+  const int rv = rotp / 8;
+  T8 tile_l[ND], tile_r, query_l[NQ];
+  const int rot_r = tid / rv, rot_c = rankp + (tid - rot_r * rv) * 8;
+
+  const auto rows_of = [&](int t) {
+    const long page = pages[(long)e * P + t / RG_PAGE];
+    return pool + (page * RG_PAGE + t % RG_PAGE) * (long)W;
+  };
+  const auto fetch = [&](int t) {
+    const T* src = rows_of(t);  // all of the 32 rows lie in one page
+#pragma unroll
+    for (int j = 0; j < ND; ++j) {
+      const int i = tid + j * LA_BLOCK;
+      tile_l[j] = *reinterpret_cast<const T8*>(src + (long)(i / LV) * W +
+                                               i % LV * 8);
+    }
+    if (rot_r < LA_KT)
+      tile_r = *reinterpret_cast<const T8*>(src + (long)rot_r * W + rot_c);
+  };
+  // rows past the request's keys are zeros, whatever the page holds there
+  const auto put = [&](int t) {
+    const int valid = S - t;
+#pragma unroll
+    for (int j = 0; j < ND; ++j) {
+      const int i = tid + j * LA_BLOCK, r = i / LV;
+      *reinterpret_cast<T8*>(ks + r * WS + i % LV * 8) =
+          r < valid ? tile_l[j] : T8(0);
+    }
+    if (rot_r < LA_KT)
+      *reinterpret_cast<T8*>(ks + rot_r * WS + rot_c) =
+          rot_r < valid ? tile_r : T8(0);
+    for (int i = tid + LA_BLOCK; i < LA_KT * rv; i += LA_BLOCK) {
+      const int r = i / rv, c = rankp + (i - r * rv) * 8;
+      if (r < valid)
+        copy8(ks + r * WS + c, rows_of(t) + (long)r * W + c);
+      else
+        zero8(ks + r * WS + c);
+    }
+  };
+
+  const auto query_at = [&](int r) { return min(r0 + r, rows - 1); };
+#pragma unroll
+  for (int j = 0; j < NQ; ++j) {
+    const int i = tid + j * LA_BLOCK, row = query_at(min(i / LV, 15));
     const int tok = row / H, h = row - tok * H;
-    const T* src = c < rankp
-                       ? q_abs + ((long)h * Nt + t0 + tok) * rankp + c
-                       : q + (long)(t0 + tok) * qstride + (long)h * dq + qoff +
-                             (c - rankp);
-    copy8(qs + r * WS + c, src);
+    query_l[j] = *reinterpret_cast<const T8*>(
+        q_abs + ((long)h * Nt + t0 + tok) * rankp + i % LV * 8);
+  }
+  if (lo < hi) fetch(lo);
+  for (int i = tid; i < 16 * rv; i += LA_BLOCK) {
+    const int r = i / rv, c = (i - r * rv) * 8, row = query_at(r);
+    const int tok = row / H, h = row - tok * H;
+    copy8(qs + r * WS + rankp + c,
+          q + (long)(t0 + tok) * qstride + (long)h * dq + qoff + c);
+  }
+#pragma unroll
+  for (int j = 0; j < NQ; ++j) {
+    const int i = tid + j * LA_BLOCK;
+    if (i < 16 * LV)
+      *reinterpret_cast<T8*>(qs + i / LV * WS + i % LV * 8) = query_l[j];
   }
 
   const int my_row = min(r0 + lr, rows - 1);
@@ -92,18 +176,8 @@ __global__ __launch_bounds__(LA_BLOCK) void latent_attn_short_kernel(
 
   for (int t = lo; t < hi; t += LA_KT) {
     __syncthreads();
-    {
-      const long page = pages[(long)e * P + t / RG_PAGE];
-      const T* src = pool + (page * RG_PAGE + t % RG_PAGE) * (long)W;
-      const int valid = min(LA_KT, S - t);
-      for (int i = tid; i < LA_KT * nvec; i += LA_BLOCK) {
-        const int r = i / nvec, c = (i - r * nvec) * 8;
-        if (r < valid)
-          copy8(ks + r * WS + c, src + (long)r * W + c);
-        else
-          zero8(ks + r * WS + c);
-      }
-    }
+    put(t);
+    if (t + LA_KT < hi) fetch(t + LA_KT);
     __syncthreads();
     {
       f32x4 c4 = {0, 0, 0, 0};
@@ -124,7 +198,7 @@ __global__ __launch_bounds__(LA_BLOCK) void latent_attn_short_kernel(
     float mx = -1e30f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int k = lg * 8 + j;
+      const int k = (j >> 2) * 16 + lg * 4 + (j & 3);
       const float s =
           (sp[k * 17 + lr] + sp[(LA_KT + k) * 17 + lr]) * scale;
       p[j] = (t + k < limit) ? s : -1e30f;
@@ -146,11 +220,10 @@ __global__ __launch_bounds__(LA_BLOCK) void latent_attn_short_kernel(
     l_run = l_run * alpha + sum;
     Frag<T> ph, pl;
     split_weights(p, ph, pl);
-    const T* va = ks + (lg * 8) * WS + wid * ND * 16 + lr;
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
       Frag<T> a;
-      a.load_strided(va + d * 16, WS);
+      load_columns(a, ks + (wid * ND + d) * 16, WS, lr, lg);
       f32x4 c4 = acc[d];
 #pragma unroll
       for (int j = 0; j < 4; ++j) c4[j] *= alpha;
