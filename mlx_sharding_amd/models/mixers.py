@@ -108,6 +108,13 @@ class NormedLinear(Linear):
         self.norm = RMSNorm(normed, eps, dtype=dtype)
 
 
+# Tokens up to which the heads' products of absorbed attention take the kernel for
+# few rows.  16 heads, 128 and 512 wide, into the latent space and out of it: 12 rows
+# 2.4 and 2.8 us (library with its copies 7.6 and 13.5), 256 rows 7.8 and 7.4 (10.2
+# and 17.7), 512 rows 13.4 and 16.4 (12.1 and 13.4).
+FEW_TOKENS = 256
+
+
 class LatentAttention(nn.Module):
     """Causal softmax attention over a cached low-rank latent.
 
@@ -165,6 +172,9 @@ class LatentAttention(nn.Module):
         # absorbed form: [H, dimp, rankp] into the query, [H, rankp, vdp] out
         self.w_absorb = self.w_uk.view(H, sh.dimp, sh.rankp)
         self.w_emit = self.w_uv.view(H, sh.vdp, sh.rankp).transpose(1, 2).contiguous()
+        # and the same with the contraction along the rows, for few tokens
+        self.w_absorb_few = self.w_absorb.transpose(1, 2).contiguous()
+        self.w_emit_few = self.w_uv.view(H, sh.vdp, sh.rankp)
         wo = F.pad(wo.view(width, H, sh.vdim), (0, sh.vdp - sh.vdim))
         self.w_o = wo.reshape(width, H * sh.vdp).contiguous()
         self.ready = True
@@ -190,12 +200,17 @@ class LatentAttention(nn.Module):
         parts = []
         if n:
             qn = q[:n].unflatten(1, (H, sh.dq))[..., : sh.dimp]
-            q_abs = torch.bmm(qn.transpose(0, 1).contiguous(), self.w_absorb)
+            few = q.is_cuda and n <= FEW_TOKENS
+            q_abs = ragged.latent_heads(qn, self.w_absorb_few, True) if few else \
+                torch.bmm(qn.transpose(0, 1).contiguous(), self.w_absorb)
             o = ragged.latent_attention_absorbed(q, q_abs, store, sh,
                                                  self.scale, batch, n_req,
                                                  max_len)
-            o = torch.bmm(o, self.w_emit)               # [H, n, vdp]
-            parts.append(o.transpose(0, 1).reshape(n, H * sh.vdp))
+            if few:
+                o = ragged.latent_heads(o.transpose(0, 1), self.w_emit_few, False)
+            else:
+                o = torch.bmm(o, self.w_emit).transpose(0, 1)  # [n, H, vdp]
+            parts.append(o.reshape(n, H * sh.vdp))
         if n < batch.n_tokens:
             parts.append(ragged.latent_attention_expanded(
                 q, store, self.w_uk, self.w_uv, sh, self.scale, batch))

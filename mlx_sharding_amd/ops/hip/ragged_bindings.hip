@@ -39,6 +39,8 @@ void launch_latent_attn_short(const void*, const void*, const void*, void*,
                               float*, float*, const int*, const int*,
                               const int*, int, int, int, long, int, int, int,
                               int, float, int, int, int, bool, hipStream_t);
+void launch_latent_heads(const void*, const void*, void*, int, int, int, int,
+                         long, long, long, long, bool, hipStream_t);
 void launch_latent_attn_long_bf16(const LatentLongArgs*, int, int,
                                   hipStream_t);
 void launch_latent_attn_long_f32(const LatentLongArgs*, int, int, hipStream_t);
@@ -295,6 +297,26 @@ Tensor latent_attn_short(Tensor q_abs, Tensor q, Tensor pool, Tensor cu,
       ints(pos0, n_req, "pos0"), ints(pages, 0, "pages"), (int)pages.size(1),
       (int)H, (int)Nt, qs, (int)dq, (int)qoff, (int)rankp, (int)rotp,
       (float)scale, (int)n_req, (int)nsplit, (int)tiles, f32, stream());
+  return out;
+}
+
+// x [n, H, K] (or a view of it), w [H, O, K] -> [n, H, O], heads_first: [H, n, O]
+Tensor latent_heads(Tensor x, Tensor w, bool heads_first) {
+  const bool f32 = is_f32(x, "x");
+  check_like(w, x, "w");
+  TORCH_CHECK(x.dim() == 3 && w.dim() == 3 && w.is_contiguous());
+  const long n = x.size(0), H = x.size(1), K = x.size(2), O = w.size(1);
+  TORCH_CHECK(w.size(0) == H && w.size(2) == K && K % 32 == 0 && O % 16 == 0 &&
+              K > 0 && H <= 65535 && n <= 65535 * 16);
+  TORCH_CHECK(x.stride(2) == 1 && x.stride(0) % 8 == 0 && x.stride(1) % 8 == 0);
+  aligned16(x, "x");
+  aligned16(w, "w");
+  auto out = torch::empty({heads_first ? H : n, heads_first ? n : H, O}, x.options());
+  if (n == 0 || H == 0 || O == 0) return out;
+  launch_latent_heads(x.data_ptr(), w.data_ptr(), out.data_ptr(), (int)n, (int)H,
+                      (int)O, (int)K, x.stride(0), x.stride(1),
+                      heads_first ? O : H * O, heads_first ? n * O : O, f32,
+                      stream());
   return out;
 }
 
@@ -856,6 +878,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("latent_append", &latent_append);
   m.def("latent_gather", &latent_gather);
   m.def("latent_attn_short", &latent_attn_short);
+  m.def("latent_heads", &latent_heads);
   m.def("latent_attn_long", &latent_attn_long);
   m.def("delta_short", &delta_short);
   m.def("delta_long", &delta_long);

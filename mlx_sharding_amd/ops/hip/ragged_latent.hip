@@ -337,3 +337,76 @@ extern "C" void launch_latent_attn_short(
                                 pages, P, H, Nt, qstride, dq, qoff, rankp,
                                 rotp, scale, n_req, nsplit, row_tiles, stream);
 }
+
+// ---------------------------------------------------------------------------
+// Products of every head with its own weights, few rows: queries into the
+// latent space (contraction dimp) and its values out of it (contraction rankp).
+//   out[h][t] = w[h] x[h][t]        w [H, O, K]
+// A block makes 16 outputs of MT tiles of 16 rows, its four waves a quarter of
+// the contraction each; every load is issued before the first product, so a
+// call costs about one trip to memory.  The library gives 16 blocks to 12 rows
+// of 16 heads and wants its rows gathered first.
+//   grid (O / 16, H, row blocks)
+// ---------------------------------------------------------------------------
+template <typename T, int MT>
+__global__ __launch_bounds__(LA_BLOCK) void latent_heads_kernel(
+    const T* __restrict__ x, const T* __restrict__ w, T* __restrict__ out,
+    int n, int O, int K, long xt, long xh, long ot, long oh) {
+  __shared__ f32x4 part[4][MT][WAVE];
+  const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int o0 = blockIdx.x * 16, h = blockIdx.y, r0 = blockIdx.z * 16 * MT;
+  const int steps = K / 32, lo = wid * steps / 4, hi = (wid + 1) * steps / 4;
+  const T* wp = w + ((long)h * O + o0 + lr) * K + lg * 8;
+  const T* xp[MT];
+  f32x4 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    xp[i] = x + min(r0 + i * 16 + lr, n - 1) * xt + h * xh + lg * 8;
+    acc[i] = f32x4{0, 0, 0, 0};
+  }
+#pragma unroll 4
+  for (int k = lo; k < hi; ++k) {
+    Frag<T> a, b;
+    a.load(wp + k * 32);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      b.load(xp[i] + k * 32);
+      acc[i] = mma(a, b, acc[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i) part[wid][i][lane] = acc[i];
+  __syncthreads();
+  for (int i = wid; i < MT; i += 4) {
+    const int row = r0 + i * 16 + lr;
+    const f32x4 sum = (part[0][i][lane] + part[1][i][lane]) +
+                      (part[2][i][lane] + part[3][i][lane]);
+    if (row < n) store4(out + row * ot + h * oh + o0 + lg * 4, sum);
+  }
+}
+
+template <typename T>
+static void latent_heads_t(const void* x, const void* w, void* out, int n,
+                           int H, int O, int K, long xt, long xh, long ot,
+                           long oh, hipStream_t stream) {
+  const int mt = n <= 16 ? 1 : n <= 32 ? 2 : 4;
+  dim3 grid((unsigned)(O / 16), (unsigned)H, (unsigned)((n + 16 * mt - 1) / (16 * mt)));
+#define LH_GO(MT)                                                          \
+  latent_heads_kernel<T, MT><<<grid, dim3(LA_BLOCK), 0, stream>>>(         \
+      (const T*)x, (const T*)w, (T*)out, n, O, K, xt, xh, ot, oh)
+  if (mt == 1) LH_GO(1);
+  else if (mt == 2) LH_GO(2);
+  else LH_GO(4);
+#undef LH_GO
+}
+
+extern "C" void launch_latent_heads(const void* x, const void* w, void* out,
+                                    int n, int H, int O, int K, long xt,
+                                    long xh, long ot, long oh, bool f32,
+                                    hipStream_t stream) {
+  if (f32)
+    latent_heads_t<float>(x, w, out, n, H, O, K, xt, xh, ot, oh, stream);
+  else
+    latent_heads_t<__bf16>(x, w, out, n, H, O, K, xt, xh, ot, oh, stream);
+}

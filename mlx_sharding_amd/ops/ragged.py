@@ -243,6 +243,13 @@ def latent_append(dkv, norm_w, eps: float, store: LayerStore, q, sh: LatentShape
     store.rows[pages * PAGE + pos % PAGE] = row
 
 
+def latent_heads(x, w, heads_first: bool):
+    """Every head's product with its own weights on the GPU: x [n, heads, k]
+    (or [heads, n, k] transposed), w [heads, out, k]; returns [n, heads, out],
+    or [heads, n, out]."""
+    return _ext("latent_heads").latent_heads(x, w, heads_first)
+
+
 def latent_attention_absorbed(q, q_abs, store: LayerStore, sh: LatentShape,
                               scale: float, batch: RaggedBatch, n_req: int,
                               max_len: int):

@@ -48,3 +48,27 @@ def test_against_64_bits(heads, rank, rot, dtype):
     # sums of up to 2501 products of weights that add up to 1
     bound = 2.0 ** -8 * 1.05 if dtype == torch.bfloat16 else 2.0 ** -18
     assert (got - want).abs().max() <= bound * want.abs().max()
+
+
+# one row, a tile of 16 with one less and one more, every count of tiles a block;
+# contractions of one step, fewer than the waves, uneven among them; both layouts
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 64, 131, 256])
+@pytest.mark.parametrize("wide, out, dtype", [
+    (32, 16, torch.bfloat16), (96, 80, torch.bfloat16), (512, 128, torch.bfloat16),
+    (160, 64, torch.float32),
+])
+def test_products_of_heads(n, wide, out, dtype):
+    torch.manual_seed(n)
+    x = torch.randn(n, 3, wide + 8, device="cuda").to(dtype)[..., :wide]
+    w = torch.randn(3, out, wide, device="cuda").to(dtype)
+    want = torch.einsum("nhk,hok->nho", x.cpu().double(), w.cpu().double())
+    size = torch.einsum("nhk,hok->nho", x.cpu().double().abs(), w.cpu().double().abs())
+    # the result's rounding (bf16 keeps 8 bits: half a last place is up to 2^-8 of the
+    # value), and 32-bit sums of ``wide`` products
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    bound = unit * want.abs() + wide * 2.0 ** -24 * size
+    got = ragged.latent_heads(x, w, False).cpu().double()
+    assert ((got - want).abs() <= bound).all()
+    assert torch.equal(ragged.latent_heads(
+        x.transpose(0, 1).contiguous().transpose(0, 1), w, True).cpu().double(),
+        got.transpose(0, 1))
