@@ -686,7 +686,15 @@ torch::Tensor mla_attend(torch::Tensor q, torch::Tensor cache, torch::Tensor w,
   } else {
     TORCH_CHECK(S >= 1 && S <= cache.size(2), "rows of the cache");
   }
-  const int n = decode_slices(N, s_ptr ? cache.size(2) : S, tile);
+  const long span = s_ptr ? cache.size(2) : S;
+  // A slice more is a partial result more that every block of mla_finish reads of each of
+  // its up to 16 tokens, and fewer tiles one after the other: 8 sqrt(tiles / tokens) of
+  // them are near the least of both (with both kernels, by slices: 16 sequences of 577
+  // keys 19: 22.8 us, 10: 18.1, 7: 16.5, 4: 18.3; 8 of 1000 32: 18.6, 16: 15.4, 8: 15.7;
+  // 4 of 2000 63: 18.6, 32: 15.4, 16: 15.7; one of 3001 47: 12.7, 32: 13.2, 16: 17.5).
+  const long tiles = (span + tile - 1) / tile;
+  const int n = std::min(decode_slices(N, span, tile),
+                         std::max(1, (int)(8.0 * std::sqrt((double)tiles / std::min(N, 16L)))));
   auto fopts = q.options().dtype(torch::kFloat32);
   auto po = torch::empty({N * heads * n, rank}, fopts);
   auto pml = torch::empty({N * heads * n, 2}, fopts);
@@ -696,8 +704,9 @@ torch::Tensor mla_attend(torch::Tensor q, torch::Tensor cache, torch::Tensor w,
                           (int)rank, true, false, (float)scale, 0.0f, 0, cur_stream());
   auto out = torch::empty({N, heads * vdim}, q.options());
   const MlaFinishArgs a{po.data_ptr<float>(), pml.data_ptr<float>(),
-                        (const __bf16*)w.data_ptr(), (__bf16*)out.data_ptr(), (int)N,
-                        (int)heads, (int)rank, (int)vdim, n};
+                        (const __bf16*)w.data_ptr(), (__bf16*)out.data_ptr(), s_ptr,
+                        (int)N, (int)heads, (int)rank, (int)vdim, n, tile,
+                        (int)(s_ptr ? cache.size(2) : S)};
   launch_mla_finish(&a, cur_stream());
   return out;
 }

@@ -15,12 +15,13 @@ struct MlaPrepareArgs {
   float eps, offset;
 };
 
-// up to 64 slices; rank a multiple of 32, vdim of 16
+// up to 64 slices of whole tiles of keys; rank a multiple of 32, vdim of 16
 struct MlaFinishArgs {
   const float *part_o, *part_ml;  // of attn_decode.hip, rank columns
   const __bf16* w;                // [heads, vdim, rank]
   __bf16* out;                    // [N, heads, vdim]
-  int N, heads, rank, vdim, slices;
+  const int* pos;                 // of the last key, or null: `keys` of them
+  int N, heads, rank, vdim, slices, tile, keys;
 };
 
 // Rows of a prompt.  rank and rope are multiples of 8, all rows begin at 16 bytes.

@@ -5,7 +5,7 @@ from types import SimpleNamespace
 import pytest
 import torch
 
-from mlx_sharding_amd.ops import ragged
+from mlx_sharding_amd.ops import hip_ext, ragged
 from mlx_sharding_amd.ops.paged import PagedState, RaggedBatch, RowSpec
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +72,27 @@ def test_products_of_heads(n, wide, out, dtype):
     assert torch.equal(ragged.latent_heads(
         x.transpose(0, 1).contiguous().transpose(0, 1), w, True).cpu().double(),
         got.transpose(0, 1))
+
+
+# room for many more keys than there are, as in a captured step; slices shared by groups
+# of threads, by halves of them and not at all; fewer slices than groups
+@pytest.mark.parametrize("N", [1, 2, 3, 17])
+@pytest.mark.parametrize("S, room", [(1, 4096), (33, 1024), (65, 65), (700, 1024),
+                                     (2049, 4096)])
+def test_slices_of_cached_latents(N, S, room):
+    H, rank, rope, vdim, scale = 16, 512, 64, 128, 0.05
+    torch.manual_seed(N + S)
+    q = torch.randn(N, H, 1, rank + rope, device="cuda").bfloat16()
+    cache = torch.full((N, 1, room, rank + rope), float("nan"), device="cuda").bfloat16()
+    cache[:, :, :S] = torch.randn(N, 1, S, rank + rope, device="cuda").bfloat16()
+    w = (torch.randn(H, vdim, rank, device="cuda") * 0.05).bfloat16()
+    pos = torch.tensor([S - 1], dtype=torch.int32, device="cuda")
+    got = hip_ext().mla_attend(q, cache, w, scale, pos, 1).double().view(N, H, vdim)
+    keys = cache[:, 0, :S].double()
+    p = torch.softmax(torch.einsum("nhd,nsd->nhs", q[:, :, 0].double(), keys) * scale, -1)
+    latent = torch.einsum("nhs,nsr->nhr", p, keys[..., :rank])
+    want = torch.einsum("nhr,hvr->nhv", latent, w.double())
+    size = torch.einsum("nhr,hvr->nhv", latent.abs(), w.double().abs())
+    # the latent's rounding to bf16, the result's, and 32-bit scores and sums
+    bound = 2.0 ** -8 * (size + want.abs()) + 2.0 ** -16 * size
+    assert ((got - want).abs() <= bound).all()
