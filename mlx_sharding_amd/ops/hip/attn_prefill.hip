@@ -16,15 +16,20 @@
 // lies in LDS as it lies in memory.
 //
 // What bounds it: the matrix cores and the exponentials and maxima between them,
-// which alternate in one wave; two waves a SIMD fill each other's gaps.  Keys and
-// values of a tile go to LDS without passing registers, the next tile while this
-// one is worked on.  16-byte pieces of a row are swapped by the row's low bits
+// which alternate in one wave; two waves a SIMD fill each other's gaps, the one that
+// multiplies first (s_setprio: 8192 tokens as below 534 -> 525 us, of 256 behind 4096
+// 208 -> 190).  Tiles of 64 keys have the exponentials among the second products, which a
+// wave alone on its SIMD needs (2048 tokens: 55 us with the priority raised between, 50.5
+// so, 52.2 before); tiles of 32 of 256 columns have no registers for that (215 us, 190).
+// Keys and values of a tile go to LDS without passing registers, the next tile while
+// this one is worked on (that the compiler has the reads of values wait for it costs
+// nothing: without 559.8 us, 559.7).  16-byte pieces of a row are swapped by the row's low bits
 // (on their way from memory, the place in LDS is fixed), without which the rows
 // that a read meets share their banks.
 // Measured (before: 16 queries a wave, scores through LDS, V transposed element by
-// element): 8192 tokens, 32 heads of 128 over 8: 5310 -> 601 us (914 TFLOP/s);
-// 4096 tokens, 16 heads of 256 over 8, capped: 1600 -> 240 us (572), 1905 behind 4096
-// with a window of 4096: 210 us (400 and 450 while places in LDS had a register each
+// element): 8192 tokens, 32 heads of 128 over 8: 5310 -> 525 us (1047 TFLOP/s);
+// 4096 tokens, 16 heads of 256 over 8, capped: 1600 -> 210 us (654), 1905 behind 4096
+// with a window of 4096: 190 us (400 and 450 while places in LDS had a register each
 // and were spilled: each reload waited for the next tile's loads; 13 and 15 us more with
 // all of a query in registers); 64 prompts of 512, 16 heads of 192/128: 1216 -> 176 us
 // (490); 57 tokens: 8.4 -> 7.6 us.
@@ -251,15 +256,16 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
   for (int d = 0; d < (ND < 4 ? ND : 4); ++d)
     vplace[d] = vkey * VP * 16 + (i16 & 1) * 8 +
                 value_place<VP>(vkey, d * 4 + (lane >> 4 & 1) * 2 + (i16 >> 1 & 1)) * 16;
-  int buf = 0;
-  for (int t = from; t < end; t += KT, buf ^= 1) {
+  auto work = [&](int t, auto which) {
+    constexpr int buf = decltype(which)::value;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (t + KT < end) stage(t + KT, buf ^ 1);
-    if (t > any_hi || t + KT <= any_lo) continue;
+    if (t > any_hi || t + KT <= any_lo) return;
     const char* kt = smem + buf * (KB + VB);
     const char* vt = kt + KB;
 
+    __builtin_amdgcn_s_setprio(1);
     f32x16 s[NB];
 #pragma unroll
     for (int n = 0; n < NB; ++n)
@@ -275,6 +281,17 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
                                                      ql + (i - NK + QL) * 1024);
         s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, q, s[n], 0, 0, 0);
       }
+    // three of the tile's reads before the first product, then one a product: what the
+    // compiler arranges waits for every second read
+    constexpr int READS = NK * NB, AHEAD = READS < 3 ? READS : 3;
+    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+    for (int i = 0; i < READS - AHEAD; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+    __builtin_amdgcn_s_setprio(0);
     if (CAP) {
 #pragma unroll
       for (int n = 0; n < NB; ++n) {
@@ -322,6 +339,7 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
         sum += s[n][r];
       }
     l += sum;
+    if (KT == 32) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int x = 0; x < KT / 16; ++x) {
       bf16x8_t p, rest;
@@ -346,6 +364,11 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
               __builtin_bit_cast(bf16x8_t, v), rest, o[d], 0, 0, 0);
       }
     }
+  };
+  // two tiles a turn: where a tile lies is known
+  for (int t = from; t < end; t += 2 * KT) {
+    work(t, std::integral_constant<int, 0>());
+    if (t + KT < end) work(t + KT, std::integral_constant<int, 1>());
   }
 
   l += __shfl_xor(l, 32, WAVE);
