@@ -28,11 +28,13 @@
 // that a read meets share their banks.
 // Measured (before: 16 queries a wave, scores through LDS, V transposed element by
 // element): 8192 tokens, 32 heads of 128 over 8: 5310 -> 525 us (1047 TFLOP/s);
-// 4096 tokens, 16 heads of 256 over 8, capped: 1600 -> 210 us (654), 1905 behind 4096
-// with a window of 4096: 190 us (400 and 450 while places in LDS had a register each
+// 4096 tokens, 16 heads of 256 over 8, capped: 1600 -> 173 us (794), 1905 behind 4096
+// with a window of 4096: 161 us (400 and 450 while places in LDS had a register each
 // and were spilled: each reload waited for the next tile's loads; 13 and 15 us more with
 // all of a query in registers); 64 prompts of 512, 16 heads of 192/128: 1216 -> 176 us
 // (490); 57 tokens: 8.4 -> 7.6 us.
+
+#include <algorithm>
 
 #include "hip_common.h"
 #include "soft_cap.h"
@@ -99,13 +101,18 @@ __device__ __forceinline__ int value_place(int row, int piece) {
   return piece;
 }
 
+// keys of a tile
+constexpr int ap_keys(int DK, int DV) { return DK + DV > 320 ? 32 : 64; }
+
 // NOPE: columns of a key that lie with the values, 0: rows of keys and of values.
 // RAGGED: portions of a batch; weights enter the second product in two bf16 parts, as
 // they do in that cache's other kernels.
-template <int DK, int DV, bool CAP, int NOPE = 0, bool RAGGED = false>
-__global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
+// TEAMS: of four waves each, with tiles of their own, that share the keys of the same
+// queries by turns and add up through LDS.
+template <int DK, int DV, bool CAP, int TEAMS, int NOPE = 0, bool RAGGED = false>
+__global__ __launch_bounds__(AP_BLOCK* TEAMS, 2) void attn_prefill_kernel(
     const PrefillArgs a) {
-  constexpr int KT = DK + DV > 320 ? 32 : 64;  // keys of a tile
+  constexpr int KT = ap_keys(DK, DV);
   constexpr int KP = DK / 8, VP = DV / 8;      // pieces of a row
   constexpr int NK = DK / 16, NB = KT / 32, ND = (DV + 31) / 32;
   constexpr int KB = KT * DK * 2, VB = KT * DV * 2;
@@ -113,9 +120,8 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
   // registers to read keys and values ahead of their products.
   constexpr int QL = DK == 256 ? 4 : 0;
   // a lane of the columns behind DV = 16 reads past its row
-  __shared__ __attribute__((aligned(16))) char smem[2 * (KB + VB) +
-                                                    AP_WAVES * QL * 1024 +
-                                                    (DV < 32 ? 64 : 0)];
+  constexpr int OWN = 2 * (KB + VB) + AP_WAVES * QL * 1024 + (DV < 32 ? 64 : 0);
+  __shared__ __attribute__((aligned(16))) char smem_all[TEAMS * OWN];
 
   // Blocks go round the XCDs.  Each XCD takes whole heads, `group` of them at a
   // time, and their longest tiles first: heads that share keys share an L2.
@@ -143,7 +149,9 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
     k0 = a.cuk[e - a.n_short];
   }
   const int lane = threadIdx.x & (WAVE - 1);
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int team = wave / AP_WAVES, wid = wave % AP_WAVES;
+  char* smem = smem_all + team * OWN;
   const int l32 = lane & 31, hi = lane >> 5;
   const char *kbase, *vbase, *pbase = nullptr;
   if (RAGGED) {
@@ -191,6 +199,9 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
   const int end = min(S, offset + min(q0 + AP_WAVES * 32, T));
   int from = 0;
   if (a.window > 0) from = max(0, offset + q0 - a.window + 1) & ~(KT - 1);
+  constexpr int TURN = TEAMS * KT;
+  const int turns = (max(end - from, 0) + TURN - 1) / TURN;
+  from += team * KT;
   if (from < end) stage(from, 0);
 
   const int w0 = q0 + wid * 32;  // this wave's first query
@@ -260,7 +271,7 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
     constexpr int buf = decltype(which)::value;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (t + KT < end) stage(t + KT, buf ^ 1);
+    if (t + TURN < end) stage(t + TURN, buf ^ 1);
     if (t > any_hi || t + KT <= any_lo) return;
     const char* kt = smem + buf * (KB + VB);
     const char* vt = kt + KB;
@@ -365,12 +376,37 @@ __global__ __launch_bounds__(AP_BLOCK, 2) void attn_prefill_kernel(
       }
     }
   };
-  // two tiles a turn: where a tile lies is known
-  for (int t = from; t < end; t += 2 * KT) {
-    work(t, std::integral_constant<int, 0>());
-    if (t + KT < end) work(t + KT, std::integral_constant<int, 1>());
+  // two of its tiles at a time: where a tile lies is known
+  for (int i = 0; i < turns; i += 2) {
+    work(from + i * TURN, std::integral_constant<int, 0>());
+    if (i + 1 < turns) work(from + (i + 1) * TURN, std::integral_constant<int, 1>());
   }
 
+  if constexpr (TEAMS == 2) {
+    constexpr int EACH = ND * 16 + 2;
+    static_assert(AP_WAVES * EACH * WAVE * 4 <= TEAMS * OWN, "sums fit");
+    float* of = reinterpret_cast<float*>(smem_all) + wid * EACH * WAVE + lane;
+    __syncthreads();  // all of the tiles are read
+    if (team == 1) {
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) of[(d * 16 + r) * WAVE] = o[d][r];
+      of[ND * 16 * WAVE] = m;
+      of[(ND * 16 + 1) * WAVE] = l;
+    }
+    __syncthreads();
+    if (team == 1) return;
+    const float m2 = of[ND * 16 * WAVE], l2 = of[(ND * 16 + 1) * WAVE];
+    const float top = fmaxf(m, m2);
+    const float f1 = __builtin_amdgcn_exp2f(m - top), f2 = __builtin_amdgcn_exp2f(m2 - top);
+    l = l * f1 + l2 * f2;
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        o[d][r] = o[d][r] * f1 + of[(d * 16 + r) * WAVE] * f2;
+  }
   l += __shfl_xor(l, 32, WAVE);
   if (w0 + l32 >= T) return;
   const float f = 1.0f / l;
@@ -402,14 +438,41 @@ extern "C" bool attn_prefill_supported(int Dk, int Dv) {
   return false;
 }
 
+// A block of one team leaves a SIMD one wave while it has a CU to itself: where there are
+// no more blocks than CUs, and at the end of a causal prompt of two blocks a CU, which
+// the longest blocks are alone with.  Two teams fill it and halve the chain of tiles;
+// adding them up costs 1 to 2 us, so the chain has to be long, and blocks of like length
+// gain nothing.  One team, two, us: 16 heads of 256, capped: 1905 tokens behind 4096 264,
+// 206 (with a window of 4096 197, 161), 384 24.5, 23.9, 256 18.8, 19.9, 64 8.0, 10.5; 4096
+// (512 blocks) 212, 173, with a window of 1024 95, 110; 32 of 128: 1024 24.0, 22.1, 640
+// 16.5, 16.2, 512 14.0, 14.4, 64 behind 4032 75, 57; 1500 (384 blocks) 35.9, 31.9, 2048
+// (512) 51.3, 48, 3000 (768) 90, 103; 2 x 1024 (512) 30.2, 32.4; 4 x 768 22.2, 24.3.
+static bool two_teams(const PrefillArgs& a, unsigned blocks, int keys) {
+  const bool whole = a.window <= 0 || a.window >= a.S;
+  const int longest =
+      ((whole ? a.S : (int)std::min<long>(a.S, (long)a.window + AP_WAVES * 32 - 1)) + keys - 1) / keys;
+  if (blocks <= 256) return longest >= 10;
+  return blocks <= 512 && longest >= 24 && whole && a.offset == 0;
+}
+
+template <int DK, int DV, bool CAP, int NOPE = 0, bool RAGGED = false>
+static void attn_prefill_run(const PrefillArgs& a, hipStream_t stream) {
+  const unsigned blocks = (unsigned)a.heads * a.tiles;
+  if constexpr (!RAGGED) {
+    if (two_teams(a, blocks, ap_keys(DK, DV))) {
+      attn_prefill_kernel<DK, DV, CAP, 2, NOPE>
+          <<<dim3(blocks), dim3(2 * AP_BLOCK), 0, stream>>>(a);
+      return;
+    }
+  }
+  attn_prefill_kernel<DK, DV, CAP, 1, NOPE, RAGGED>
+      <<<dim3(blocks), dim3(AP_BLOCK), 0, stream>>>(a);
+}
+
 template <int DK, int DV>
 static void attn_prefill_go(const PrefillArgs& a, bool cap, hipStream_t stream) {
-  const dim3 grid((unsigned)a.heads * a.tiles), block(AP_BLOCK);
-  if (cap) {
-    attn_prefill_kernel<DK, DV, true><<<grid, block, 0, stream>>>(a);
-  } else {
-    attn_prefill_kernel<DK, DV, false><<<grid, block, 0, stream>>>(a);
-  }
+  if (cap) attn_prefill_run<DK, DV, true>(a, stream);
+  else attn_prefill_run<DK, DV, false>(a, stream);
 }
 
 // the arguments that follow from sizes and options
@@ -470,8 +533,7 @@ extern "C" void launch_mla_prompt(const void* q, const void* kv, const void* cac
   a.cos = cos;
   a.sin = sin;
   prefill_setup(a, B, scale, 0.0f, 0, causal_offset);
-  attn_prefill_kernel<192, 128, false, 128>
-      <<<dim3((unsigned)a.heads * a.tiles), dim3(AP_BLOCK), 0, stream>>>(a);
+  attn_prefill_run<192, 128, false, 128>(a, stream);
 }
 
 // The same for portions of a batch: q rows [dq = 192], turned; k [keys, H * 128], v
@@ -497,8 +559,7 @@ extern "C" void launch_latent_prompt(const void* q, const void* k, const void* v
   a.tok_base = tok_base;
   prefill_setup(a, 1, scale, 0.0f, 0, 0);
   a.tiles = n_tiles;
-  attn_prefill_kernel<192, 128, false, 128, true>
-      <<<dim3((unsigned)a.heads * a.tiles), dim3(AP_BLOCK), 0, stream>>>(a);
+  attn_prefill_run<192, 128, false, 128, true>(a, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -302,3 +302,34 @@ def test_latent_prompt(B, T, at, H):
     # 2^-8 times |q k| near 1, few of them; weights are rounded to bf16
     bound = 2.0 ** -8 * expect.abs() + 2.0 ** -7 * size + 1e-5
     assert bool(((out.transpose(1, 2) - expect).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("Dk,Dv", [(32, 16), (64, 64), (128, 128), (192, 128), (256, 256)])
+def test_prefill_two_teams(Dk, Dv):
+    """Long keys of few blocks, whose tiles two teams take by turns: odd and even
+    numbers of tiles, a team without a tile for a wave's queries, windows that begin
+    inside either team's first tile, more blocks than CUs; scores that grow with the
+    key and with its distance, so that either team's reference is far above."""
+    torch.manual_seed(Dk + Dv)
+    for B, Hq, Hkv, T, offset, cap, window, scale, slope in (
+            (1, 8, 4, 641, 0, 0.0, 0, 0.1, 0), (1, 2, 1, 1, 704, 0.0, 0, 0.1, 0),
+            (1, 4, 2, 130, 900, 20.0, 0, 0.1, 0), (2, 3, 1, 200, 1000, 0.0, 700, 0.1, 0),
+            (1, 2, 2, 64, 2000, 0.0, 737, -0.1, 0), (1, 24, 8, 1600, 0, 0.0, 0, 0.1, 0),
+            (1, 2, 2, 150, 600, 0.0, 0, 1.0, 4), (1, 2, 2, 150, 600, 0.0, 0, 1.0, -4)):
+        S = T + offset
+        q = torch.randn(B, Hq, T, Dk, device="cuda").bfloat16()
+        k, v = cached(B, Hkv, S, Dk, 37), cached(B, Hkv, S, Dv, 37)
+        if slope:
+            q[..., 0] = 1.0
+            k[..., 0] = torch.arange(S, device="cuda") / 4 * slope
+        out = ext().attn_prefill(q, k, v, scale, cap, window, offset).double()
+        expect, size = attention(q, k, v, scale, cap, window, offset)
+        # as above; scores of up to 800 are off by 2^-24 of themselves each way
+        bound = 2.0 ** -8 * (size + expect.abs()) + 2.0 ** -12 * size + 1e-6
+        assert (out.shape == expect.shape
+                and bool(((out - expect).abs() <= bound).all())), (T, offset, window, slope)
+
+
+@pytest.mark.parametrize("B,T,at,H", [(1, 700, 0, 2), (2, 129, 640, 3)])
+def test_latent_prompt_two_teams(B, T, at, H):
+    test_latent_prompt(B, T, at, H)
