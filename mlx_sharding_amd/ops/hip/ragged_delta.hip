@@ -649,7 +649,8 @@ __global__ __launch_bounds__(DC_BLOCK) void delta_conv_state_kernel(
 //   am [chunks, H, 64, 64]  A (lower tiles only)
 //   ge [chunks, H, 2, 64]   exp(G), exp(G_last - G)
 // Bound by latency, and by what is written.  Operands are on their way a step ahead, and
-// the value heads of a q/k head run on one XCD: 126 chunks of 32 heads 138 -> 110 us.
+// the value heads of a q/k head run on one XCD: 126 chunks of 32 heads 138 -> 110 us;
+// two of them in a block: 118 -> 84.
 // ---------------------------------------------------------------------------
 
 #define DR_LS 68
@@ -713,17 +714,24 @@ __device__ __forceinline__ void invert_tiles(float* ls, const float* by, float* 
   }
 }
 
+// Value heads of a q/k head that a block makes one after the other, from the same
+// products, which are half of a head's work (fp32 matrix cores).  Blocks of one head,
+// of two, us: 32 heads over 16, 126 chunks 118, 84, 63 59.8, 47.6, 32 38.1, 25.4, 16 19.2,
+// 18.4, 10 (320 blocks) 18.2, 17.3, 5 14.1, 18.1: those leave CUs idle.
+#define DC_HEADS 2
+
 __global__ __launch_bounds__(256) void delta_chunk_kernel(
     const float* __restrict__ qn, const float* __restrict__ kn,
     const float* __restrict__ lg, const float* __restrict__ bt,
     float* __restrict__ tm, float* __restrict__ am, float* __restrict__ ge,
-    const int* __restrict__ chunks, int n_chunks, int tok_base, int KH, int H, int Dp) {
+    const int* __restrict__ chunks, int n_chunks, int tok_base, int KH, int H, int Dp,
+    int per) {
   // blocks go round the XCDs: eight pairs of a chunk and a q/k head, then their next
-  // value head, which reads the same rows from the L2 they came to
-  const int r = H / KH, round = blockIdx.x / (8 * r), at = blockIdx.x - round * 8 * r;
-  const int pair = round * 8 + at % 8;
+  // `per` value heads, which read the same rows from the L2 they came to
+  const int r = H / KH, g = r / per, round = blockIdx.x / (8 * g);
+  const int at = blockIdx.x - round * 8 * g, pair = round * 8 + at % 8;
   if (pair >= n_chunks * KH) return;
-  const int c = pair / KH, kh = pair - c * KH, h = kh * r + at / 8;
+  const int c = pair / KH, kh = pair - c * KH, h0 = kh * r + at / 8 * per;
   const int i0 = chunks[2 * c] - tok_base;
   const int len = chunks[2 * c + 1];
   const int tid = threadIdx.x;
@@ -731,12 +739,13 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(
   const int wid = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int lr = lane & 15, g4 = lane >> 4;
 
-  __shared__ double gs[DR_CHUNK];
-  __shared__ float bs[DR_CHUNK];
+  __shared__ double gs[DC_HEADS][DR_CHUNK];
+  __shared__ float bs[DC_HEADS][DR_CHUNK];
   __shared__ __attribute__((aligned(16))) float ls[DR_CHUNK * DR_LS];
 
-  const long ch = (long)c * H + h;
-  if (wid == 0) {
+  if (wid < per) {
+    const int h = h0 + wid;
+    const long ch = (long)c * H + h;
     // running sum of log decays; differences of it must stay exact to fp32,
     // also behind strong decays, hence double
     const bool in = lane < len;
@@ -747,8 +756,8 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(
       if (lane >= off) g += o;
     }
     const double last = __shfl(g, WAVE - 1, WAVE);
-    gs[lane] = g;
-    bs[lane] = in ? bt[(long)(i0 + lane) * H + h] : 0.0f;
+    gs[wid][lane] = g;
+    bs[wid][lane] = in ? bt[(long)(i0 + lane) * H + h] : 0.0f;
     ge[ch * 128 + lane] = expf((float)g);
     ge[ch * 128 + 64 + lane] = expf((float)(last - g));
   }
@@ -795,20 +804,24 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(
     if (d + 16 < Dp) use(two);
   }
   __syncthreads();
+  for (int n = 0; n < per; ++n) {
+    const long ch = (long)c * H + h0 + n;
+    if (n) __syncthreads();  // the last head's matrix is read
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (j > wid) continue;
-    const int col = j * 16 + lr;
+    for (int j = 0; j < 4; ++j) {
+      if (j > wid) continue;
+      const int col = j * 16 + lr;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = wid * 16 + g4 * 4 + r;
-      const float dec = col <= row ? expf((float)(gs[row] - gs[col])) : 0.0f;
-      ls[row * DR_LS + col] = col < row ? bs[row] * dec * kk[j][r] : 0.0f;
-      am[ch * 4096 + row * 64 + col] = dec * qk[j][r];
+      for (int r = 0; r < 4; ++r) {
+        const int row = wid * 16 + g4 * 4 + r;
+        const float dec = col <= row ? expf((float)(gs[n][row] - gs[n][col])) : 0.0f;
+        ls[row * DR_LS + col] = col < row ? bs[n][row] * dec * kk[j][r] : 0.0f;
+        am[ch * 4096 + row * 64 + col] = dec * qk[j][r];
+      }
     }
+    __syncthreads();
+    invert_tiles(ls, bs[n], tm + ch * 4096, wid, lane);
   }
-  __syncthreads();
-  invert_tiles(ls, bs, tm + ch * 4096, wid, lane);
 }
 
 // The same for decays per channel, and what the walk multiplies the state with:
@@ -1818,10 +1831,13 @@ static void delta_long_t(const DeltaLongArgs& a, const DeltaDims& dm,
 #undef DCH_GO
     delta_walk_t<T, true>(a, dm, a.qg, a.kg, a.kl, dm.H, g4, stream);
   } else {
-    const dim3 g((unsigned)(((long)a.n_chunks * dm.KH + 7) / 8 * 8 * (dm.H / dm.KH)));
+    const long pairs = (long)a.n_chunks * dm.KH;
+    const int r = dm.H / dm.KH;
+    const int per = r % DC_HEADS == 0 && pairs * r >= 256 ? DC_HEADS : 1;
+    const dim3 g((unsigned)((pairs + 7) / 8 * 8 * (r / per)));
     delta_chunk_kernel<<<g, block, 0, stream>>>(
         a.qn, a.kn, a.lg, a.bt, a.tm, a.am, a.ge, a.chunks, a.n_chunks, a.tok_base,
-        dm.KH, dm.H, a.Dp);
+        dm.KH, dm.H, a.Dp, per);
     delta_walk_t<T, false>(a, dm, a.qn, a.kn, a.kn, dm.KH, g4, stream);
   }
   dim3 g5((unsigned)((a.n_tok * dm.H + 4 * DG_ROWS - 1) / (4 * DG_ROWS)));

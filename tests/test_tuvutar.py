@@ -476,3 +476,13 @@ def test_bf16_matches_cpu_path_on_kernel_shapes():
     want = c.run(h.bfloat16().float(), [700])
     for sizes in ([700], [500, 1], [300, 128, 16]):
         assert cases.error(g.run(h, sizes), want) < 3e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv_heads,tokens", [(24, 4, 690), (32, 16, 520), (9, 3, 1900)])
+def test_delta_chunks_of_many_heads(heads, kv_heads, tokens):
+    """Blocks that make two value heads of a q/k head, the last round of them not full,
+    and an odd number of heads that they cannot share."""
+    m = Mixer(cases.delta(heads, kv_heads, 16, 16, 3), 64, F32, "cuda")
+    h = torch.randn(tokens, 64, generator=torch.Generator().manual_seed(3))
+    assert cases.error(m.run(h, [tokens]), m.want(h)) < 2e-5
