@@ -7,11 +7,12 @@ Policy (deliberate, per the MI355X-native design):
     native path.  Set ``MLXS_AMD_FORCE_TORCH=1`` only for debugging.
   * On CPU tensors the torch reference implementations run (the
     reference's CPU plumbing config needs no GPU code).
-  * Plain dense GEMMs of more than 64 rows (qkv/o projections, dense MLP
+  * Plain dense GEMMs of more than 64 rows (qkv/o projections, most dense MLP
     matmuls) go through torch.matmul → hipBLASLt/rocBLAS, which is the
     intended library path.  Everything else is ours: products of up to 64
     rows, with the norm, unit and residual around them (linear_few.hip),
-    norms, rope, attention, w4a16, routed experts.
+    gated units and long contractions into few columns of more rows
+    (linear_tiles.hip), norms, rope, attention, w4a16, routed experts.
 """
 
 from __future__ import annotations
