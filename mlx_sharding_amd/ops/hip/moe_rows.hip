@@ -28,8 +28,8 @@
 // them to s q + b; values of a word are laid out in pairs for it.  The vector units are
 // at work for half of the time at 4 bits; with every second value left where it is, as
 // part of 64 + q, and both masks in one instruction a word of eight takes 13 of them
-// instead of 19 (64 tokens, both products: 92 -> 87 us).  Loads further ahead gain nothing
-// (two tiles 103 us), and cost tokens of which a block has one tile.
+// instead of 19 (64 tokens, both products: 92 -> 87 us).  A wave has one tile's loads under
+// way beside the one it works on, and waits for its oldest only (both products 84 -> 71 us).
 // Measured, norm, router, choice, experts and sum of 64 experts of 1408 x 2048 (6 a
 // token) beside the kernels before (norm and residual apart): 1 token at 4 bits
 // 33 us, 48 and norms; 64 tokens 105, 166 (experts alone 3.5 TB/s); 8 bits 147,
@@ -332,105 +332,119 @@ __global__ __launch_bounds__(
       const char* p = wp[m] + t * step + (long)u * far;  // between a wave's units
       r.load(p, p + scales);
     };
-    Packed<BITS> next[MATS][UPW];
+    // C units of this wave.  Their number is known: where loads are left out between
+    // others, the compiler has more waited for than is used (both products of 64 tokens at
+    // 4 bits, 64 experts: 84.5 us, 71.5 so; 1 token 16.9, 15.5; 64 at 8 bits 127, 119, in
+    // bf16 227, 221; only one unit a wave in bf16 is slower, 28.3 us, 29.2).
+    auto work = [&](auto mine, auto has) {
+      constexpr int C = decltype(mine)::value;
+      Packed<BITS> next[MATS][C];
 #pragma unroll
-    for (int u = 0; u < UPW; ++u) {
-      if (wid + u * MR_WAVES >= units) continue;
+      for (int u = 0; u < C; ++u) {
+        if (!has(u)) continue;
 #pragma unroll
-      for (int m = 0; m < MATS; ++m) fetch(next[m][u], m, u, 0);
-    }
-    int pair;
-    if constexpr (FEW) {
-      // the n pairs from `first` on go to the lowest lanes, the others anywhere else
-      const unsigned long long which = members[place];
-      const int to = __popcll(which & ((1ull << lane) - 1)) - first;
-      const bool listed = (which >> lane & 1) && to >= 0 && to < 16;
-      pair = __builtin_amdgcn_ds_permute((listed ? to : 16 + lane % 48) * 4, lane);
-      pair = __shfl(pair, min(l16, n - 1), WAVE);
-    } else {
-      if (wid == 0) {
-        int found = -first;
-        for (int i = 0; i < a.pairs && found < 16; i += WAVE) {
-          const bool mine = i + lane < a.pairs && chosen[i + lane] == e;
-          const unsigned long long with = __ballot(mine);
-          const int place = found + __popcll(with & ((1ull << lane) - 1));
-          if (mine && place >= 0 && place < 16) list[place] = (short)(i + lane);
-          found += __popcll(with);
+        for (int m = 0; m < MATS; ++m) fetch(next[m][u], m, u, 0);
+      }
+      int pair;
+      if constexpr (FEW) {
+        // the n pairs from `first` on go to the lowest lanes, the others anywhere else
+        const unsigned long long which = members[place];
+        const int to = __popcll(which & ((1ull << lane) - 1)) - first;
+        const bool listed = (which >> lane & 1) && to >= 0 && to < 16;
+        pair = __builtin_amdgcn_ds_permute((listed ? to : 16 + lane % 48) * 4, lane);
+        pair = __shfl(pair, min(l16, n - 1), WAVE);
+      } else {
+        if (wid == 0) {
+          int found = -first;
+          for (int i = 0; i < a.pairs && found < 16; i += WAVE) {
+            const bool mine = i + lane < a.pairs && chosen[i + lane] == e;
+            const unsigned long long with = __ballot(mine);
+            const int place = found + __popcll(with & ((1ull << lane) - 1));
+            if (mine && place >= 0 && place < 16) list[place] = (short)(i + lane);
+            found += __popcll(with);
+          }
+        }
+        __syncthreads();
+        pair = list[min(l16, n - 1)];
+      }
+      // asked for here: behind the products it was waited for
+      const float weight = UP ? 0.0f : a.weight[pair];
+      V x[C][4];
+#pragma unroll
+      for (int u = 0; u < C; ++u) {
+        if (!has(u)) continue;
+        const short* src = (const short*)a.x +
+                           (long)(UP ? pair / a.top : pair) * a.K + k0 +
+                           u * MR_WAVES * MR_UNIT;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (UP && BITS != 16) {
+            const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(src + i * 8);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[u][i][j] = (_Float16)(float)v[j];
+          } else {
+            x[u][i] = *reinterpret_cast<const V*>(src + i * 8);
+          }
         }
       }
-      __syncthreads();
-      pair = list[min(l16, n - 1)];
-    }
-    // asked for here: behind the products it was waited for
-    const float weight = UP ? 0.0f : a.weight[pair];
-    V x[UPW][4];
+      for (int t = t0; t < t1; ++t, buf ^= 1) {
+        f32x4 acc[MATS];
 #pragma unroll
-    for (int u = 0; u < UPW; ++u) {
-      if (wid + u * MR_WAVES >= units) continue;
-      const short* src = (const short*)a.x +
-                         (long)(UP ? pair / a.top : pair) * a.K + k0 +
-                         u * MR_WAVES * MR_UNIT;
+        for (int m = 0; m < MATS; ++m) acc[m] = f32x4{0, 0, 0, 0};
+        const int ahead = min(t + 1, t1 - 1) - t0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if constexpr (UP && BITS != 16) {
-          const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(src + i * 8);
+        for (int u = 0; u < C; ++u) {
+          if (!has(u)) continue;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) x[u][i][j] = (_Float16)(float)v[j];
-        } else {
-          x[u][i] = *reinterpret_cast<const V*>(src + i * 8);
+          for (int m = 0; m < MATS; ++m) {
+            // The next words come into the registers that are free after these products: a
+            // copy of a load that is under way would wait for it.
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              acc[m] = Op::mma(next[m][u].operand(i), x[u][i], acc[m]);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(next[m][u], m, u, ahead);
+          }
         }
-      }
-    }
-    for (int t = t0; t < t1; ++t, buf ^= 1) {
-      f32x4 acc[MATS];
 #pragma unroll
-      for (int m = 0; m < MATS; ++m) acc[m] = f32x4{0, 0, 0, 0};
-      const int ahead = min(t + 1, t1 - 1) - t0;
-#pragma unroll
-      for (int u = 0; u < UPW; ++u) {
-        if (wid + u * MR_WAVES >= units) continue;
+        for (int m = 0; m < MATS; ++m) red[buf][wid][m][lane] = acc[m];
+        __syncthreads();
+        // one wave finishes these rows, the others go on
+        if (wid != t % MR_WAVES) continue;
+        f32x4 v[MATS];
 #pragma unroll
         for (int m = 0; m < MATS; ++m) {
-          const Packed<BITS> r = next[m][u];
-          fetch(next[m][u], m, u, ahead);
+          v[m] = red[buf][0][m][lane];
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            acc[m] = Op::mma(r.operand(i), x[u][i], acc[m]);
+          for (int w = 1; w < MR_WAVES; ++w) {
+            const f32x4 p = red[buf][w][m][lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[m][j] += p[j];
+          }
+        }
+        if (l16 >= n) continue;
+        const long to = (long)pair * a.O + t * 16 + lg * 4;
+        if constexpr (UP) {
+          typedef typename Op::H H4;
+          H4 h;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float g = v[0][j];
+            h[j] = (typename Op::E)(g / (1.0f + __expf(-g)) * v[MATS - 1][j]);
+          }
+          *reinterpret_cast<H4*>((typename Op::E*)a.y + to) = h;
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[0][j] *= weight;
+          *reinterpret_cast<f32x4*>((float*)a.y + to) = v[0];
         }
       }
-#pragma unroll
-      for (int m = 0; m < MATS; ++m) red[buf][wid][m][lane] = acc[m];
-      __syncthreads();
-      // one wave finishes these rows, the others go on
-      if (wid != t % MR_WAVES) continue;
-      f32x4 v[MATS];
-#pragma unroll
-      for (int m = 0; m < MATS; ++m) {
-        v[m] = red[buf][0][m][lane];
-#pragma unroll
-        for (int w = 1; w < MR_WAVES; ++w) {
-          const f32x4 p = red[buf][w][m][lane];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[m][j] += p[j];
-        }
-      }
-      if (l16 >= n) continue;
-      const long to = (long)pair * a.O + t * 16 + lg * 4;
-      if constexpr (UP) {
-        typedef typename Op::H H4;
-        H4 h;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float g = v[0][j];
-          h[j] = (typename Op::E)(g / (1.0f + __expf(-g)) * v[MATS - 1][j]);
-        }
-        *reinterpret_cast<H4*>((typename Op::E*)a.y + to) = h;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[0][j] *= weight;
-        *reinterpret_cast<f32x4*>((float*)a.y + to) = v[0];
-      }
-    }
+    };
+    auto there = [&](int u) { return wid + u * MR_WAVES < units; };
+    auto always = [](int) { return true; };
+    if constexpr (UPW == 1) work(std::integral_constant<int, UPW>(), there);
+    else if (there(UPW - 1)) work(std::integral_constant<int, UPW>(), always);
+    else work(std::integral_constant<int, UPW - 1>(), always);
   }
 }
 
