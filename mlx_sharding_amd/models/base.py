@@ -56,8 +56,9 @@ class Linear(nn.Module):
     Dense path → ops.linear: linear_few.hip for up to 64 rows, else
     linear_tiles.hip or the library.  Quantized path → the w4a16/w8a16
     dequant-GEMM op.  Parameter names (weight/scales/biases) match the MLX
-    checkpoint layout so pre-quantized checkpoints load directly (/root/reference/shard/utils.py:54-65 predicate: a
-    `.scales` key exists for the module).
+    checkpoint layout so pre-quantized checkpoints load directly
+    (/root/reference/shard/utils.py:54-65 predicate: a `.scales` key exists
+    for the module).
     """
 
     def __init__(self, in_features: int, out_features: int,
