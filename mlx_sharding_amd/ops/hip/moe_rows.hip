@@ -440,6 +440,8 @@ __global__ __launch_bounds__(
         }
       }
     };
+    // UPW is units / MR_WAVES, rounded up (the launch has an instance for each), so a wave
+    // has UPW of them or one less, and without a second one maybe none.
     auto there = [&](int u) { return wid + u * MR_WAVES < units; };
     auto always = [](int) { return true; };
     if constexpr (UPW == 1) work(std::integral_constant<int, UPW>(), there);
@@ -538,7 +540,8 @@ static void moe_rows_run(MoeRowsArgs a, hipStream_t stream) {
   } else if (upw <= 3) {
     MR_GO(3);
   } else if constexpr (BITS < 16) {
-    MR_GO(5);
+    if (upw <= 4) MR_GO(4);
+    else MR_GO(5);
   }
 #undef MR_GO
 }

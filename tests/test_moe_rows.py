@@ -91,6 +91,19 @@ def test_experts(N, E, top, I, H, bits, gs):
     assert bool(((alone - total).abs() <= bound).all())
 
 
+# Units of 128 of the contraction, of which eight waves have as many or one less each: 25 to
+# 40, one wave's last one missing, most waves' and none; in either product.  Up to 64 pairs
+# and more.
+@pytest.mark.parametrize("N,E,top", [(5, 3, 2), (70, 2, 1)])
+@pytest.mark.parametrize("units,bits,gs", [
+    (25, 4, 64), (28, 4, 32), (31, 4, 128), (25, 8, 128), (28, 8, 64), (31, 8, 32),
+    (32, 4, 64), (33, 8, 64), (36, 4, 128), (39, 8, 32), (9, 4, 64), (15, 8, 64),
+    (17, 4, 32), (20, 8, 128), (23, 4, 64), (15, 16, 128), (17, 16, 128), (20, 16, 128)])
+def test_units_that_some_waves_lack(N, E, top, units, bits, gs):
+    test_experts(N, E, top, 384, units * 128, bits, gs)
+    test_experts(N, E, top, units * 128, 384, bits, gs)
+
+
 def test_ties_and_rows_that_are_no_numbers():
     """Equal scores: the first experts.  NaN: some experts, each once."""
     H, E, top = 256, 12, 4
