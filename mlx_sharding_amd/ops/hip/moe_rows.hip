@@ -312,6 +312,13 @@ __global__ __launch_bounds__(
                      (l16 * (MR_UNIT / GS) + lg * 32 / GS) * 4;
   int buf = 0;
   while (at < stop) {
+    // What follows from a lane's number is made anew for each group of more than 64 pairs in
+    // bf16 with one unit a wave: kept, it is more than there are registers for, and reloads
+    // wait for the words that are under way (64 tokens, top 6 of 64 experts of 1024 x 1024:
+    // 93.0 us, 84.2 so; with loads that products wait for 87.4).
+    int self = lane;
+    if constexpr (BITS == 16 && UPW == 1 && !FEW) asm volatile("" : "+v"(self));
+    const int l16 = self & 15, lg = self >> 4;
     // one group of one expert's pairs, rows t0 to t1
     const int group = __umulhi(at, a.by_rows), t0 = at - group * rows;
     const int t1 = min(rows, t0 + stop - at);
@@ -335,7 +342,7 @@ __global__ __launch_bounds__(
     // C units of this wave.  Their number is known: where loads are left out between
     // others, the compiler has more waited for than is used (both products of 64 tokens at
     // 4 bits, 64 experts: 84.5 us, 71.5 so; 1 token 16.9, 15.5; 64 at 8 bits 127, 119, in
-    // bf16 227, 221; only one unit a wave in bf16 is slower, 28.3 us, 29.2).
+    // bf16 227, 221).
     auto work = [&](auto mine, auto has) {
       constexpr int C = decltype(mine)::value;
       Packed<BITS> next[MATS][C];
@@ -349,18 +356,18 @@ __global__ __launch_bounds__(
       if constexpr (FEW) {
         // the n pairs from `first` on go to the lowest lanes, the others anywhere else
         const unsigned long long which = members[place];
-        const int to = __popcll(which & ((1ull << lane) - 1)) - first;
-        const bool listed = (which >> lane & 1) && to >= 0 && to < 16;
-        pair = __builtin_amdgcn_ds_permute((listed ? to : 16 + lane % 48) * 4, lane);
+        const int to = __popcll(which & ((1ull << self) - 1)) - first;
+        const bool listed = (which >> self & 1) && to >= 0 && to < 16;
+        pair = __builtin_amdgcn_ds_permute((listed ? to : 16 + self % 48) * 4, lane);
         pair = __shfl(pair, min(l16, n - 1), WAVE);
       } else {
         if (wid == 0) {
           int found = -first;
           for (int i = 0; i < a.pairs && found < 16; i += WAVE) {
-            const bool mine = i + lane < a.pairs && chosen[i + lane] == e;
+            const bool mine = i + self < a.pairs && chosen[i + self] == e;
             const unsigned long long with = __ballot(mine);
-            const int place = found + __popcll(with & ((1ull << lane) - 1));
-            if (mine && place >= 0 && place < 16) list[place] = (short)(i + lane);
+            const int place = found + __popcll(with & ((1ull << self) - 1));
+            if (mine && place >= 0 && place < 16) list[place] = (short)(i + self);
             found += __popcll(with);
           }
         }
@@ -407,17 +414,17 @@ __global__ __launch_bounds__(
           }
         }
 #pragma unroll
-        for (int m = 0; m < MATS; ++m) red[buf][wid][m][lane] = acc[m];
+        for (int m = 0; m < MATS; ++m) red[buf][wid][m][self] = acc[m];
         __syncthreads();
         // one wave finishes these rows, the others go on
         if (wid != t % MR_WAVES) continue;
         f32x4 v[MATS];
 #pragma unroll
         for (int m = 0; m < MATS; ++m) {
-          v[m] = red[buf][0][m][lane];
+          v[m] = red[buf][0][m][self];
 #pragma unroll
           for (int w = 1; w < MR_WAVES; ++w) {
-            const f32x4 p = red[buf][w][m][lane];
+            const f32x4 p = red[buf][w][m][self];
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[m][j] += p[j];
           }
