@@ -93,13 +93,14 @@ __global__ __launch_bounds__(LA_BLOCK) void latent_attn_short_kernel(
   const int lr = lane & 15, lg = lane >> 4;
 
   // pieces of 8 values: of the latent part ND a thread and tile, of the
-  // rotated part one (those past the first 64 columns are copied directly)
+  // rotated part one (those past the first 64 columns are copied directly), or
+  // none where nothing is rotated
   typedef T T8 __attribute__((ext_vector_type(8)));
   constexpr int LV = 8 * ND;
   constexpr int NQ = (16 * LV + LA_BLOCK - 1) / LA_BLOCK;
   const int rv = rotp / 8;
   T8 tile_l[ND], tile_r, query_l[NQ];
-  const int rot_r = tid / rv, rot_c = rankp + (tid - rot_r * rv) * 8;
+  const int rot_r = rv ? tid / rv : LA_KT, rot_c = rankp + (tid - rot_r * rv) * 8;
 
   const auto rows_of = [&](int t) {
     const long page = pages[(long)e * P + t / RG_PAGE];

@@ -13,10 +13,11 @@ pytestmark = pytest.mark.gpu
 
 # one key, a tile of 32 keys and a page of 64 less one, whole and more; slices of
 # several tiles; tiles of 16 rows with remainders; rotated parts of one piece a
-# thread, less and more; what lies behind a request's keys is not a number
+# thread, less, more and none; what lies behind a request's keys is not a number
 @pytest.mark.parametrize("heads, rank, rot, dtype", [
     (16, 512, 64, torch.bfloat16), (3, 64, 32, torch.bfloat16),
     (5, 1024, 96, torch.bfloat16), (4, 128, 160, torch.float32),
+    (6, 512, 0, torch.bfloat16), (3, 64, 0, torch.float32),
 ])
 def test_against_64_bits(heads, rank, rot, dtype):
     dev = torch.device("cuda")
