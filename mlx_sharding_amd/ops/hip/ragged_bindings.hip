@@ -307,12 +307,13 @@ Tensor latent_heads(Tensor x, Tensor w, bool heads_first) {
   TORCH_CHECK(x.dim() == 3 && w.dim() == 3 && w.is_contiguous());
   const long n = x.size(0), H = x.size(1), K = x.size(2), O = w.size(1);
   TORCH_CHECK(w.size(0) == H && w.size(2) == K && K % 32 == 0 && O % 16 == 0 &&
-              K > 0 && H <= 65535 && n <= 65535 * 16);
+              H <= 65535 && n <= 65535 * 16);
   TORCH_CHECK(x.stride(2) == 1 && x.stride(0) % 8 == 0 && x.stride(1) % 8 == 0);
   aligned16(x, "x");
   aligned16(w, "w");
   auto out = torch::empty({heads_first ? H : n, heads_first ? n : H, O}, x.options());
   if (n == 0 || H == 0 || O == 0) return out;
+  if (K == 0) return out.zero_();  // heads of a rotated part alone
   launch_latent_heads(x.data_ptr(), w.data_ptr(), out.data_ptr(), (int)n, (int)H,
                       (int)O, (int)K, x.stride(0), x.stride(1),
                       heads_first ? O : H * O, heads_first ? n * O : O, f32,

@@ -52,11 +52,11 @@ def test_against_64_bits(heads, rank, rot, dtype):
 
 
 # one row, a tile of 16 with one less and one more, every count of tiles a block;
-# contractions of one step, fewer than the waves, uneven among them; both layouts
+# contractions of one step, fewer than the waves, uneven among them, none; both layouts
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 64, 131, 256])
 @pytest.mark.parametrize("wide, out, dtype", [
     (32, 16, torch.bfloat16), (96, 80, torch.bfloat16), (512, 128, torch.bfloat16),
-    (160, 64, torch.float32),
+    (160, 64, torch.float32), (0, 64, torch.bfloat16),
 ])
 def test_products_of_heads(n, wide, out, dtype):
     torch.manual_seed(n)
