@@ -127,7 +127,7 @@ __global__ __launch_bounds__(512) void mla_finish_kernel(const MlaFinishArgs a) 
   // the count (an empty one has weight zero).
   int used = n;
   if (n > 8) {
-    const int keys = a.pos ? min(*a.pos + 1, a.keys) : a.keys;
+    const int keys = max(1, a.pos ? min(*a.pos + 1, a.keys) : a.keys);
     const int per = ((keys + n - 1) / n + a.tile - 1) / a.tile * a.tile;
     used = min(n, (keys + per - 1) / per);
   }

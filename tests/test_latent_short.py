@@ -97,3 +97,13 @@ def test_slices_of_cached_latents(N, S, room):
     # the latent's rounding to bf16, the result's, and 32-bit scores and sums
     bound = 2.0 ** -8 * (size + want.abs()) + 2.0 ** -16 * size
     assert ((got - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("room", [65, 4096])
+def test_a_place_before_the_first_key(room):
+    """No keys, few slices and many: no numbers."""
+    q = torch.randn(2, 16, 1, 576, device="cuda").bfloat16()
+    cache = torch.randn(2, 1, room, 576, device="cuda").bfloat16()
+    w = torch.randn(16, 128, 512, device="cuda").bfloat16()
+    pos = torch.tensor([-1], dtype=torch.int32, device="cuda")
+    assert hip_ext().mla_attend(q, cache, w, 0.05, pos, 1).isnan().all()
