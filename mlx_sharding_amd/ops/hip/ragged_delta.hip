@@ -18,8 +18,8 @@
 //    exp(G_last) S0 + K^T diag(exp(G_last - G)) U.  One kernel makes
 //    (I + L)^-1 diag(beta) and A of all chunks at once, a second walks the
 //    chunks of a (request, head, 16 or 32 value columns).  Products run on the fp32
-//    matrix cores, those of the walk (depths of 32, 64 and 128) as six products of
-//    bf16 parts that keep all bits.
+//    matrix cores, those of the walk (depths of 32, 64 and 128) as eight products of
+//    bf16 parts, no further off than fp32's.
 //  * decays per channel: exp(G) is a vector then, and L and A sum
 //    k_i[d] k_j[d] exp(G_i[d] - G_j[d]) over channels.  Between the tokens of two
 //    neighbouring blocks, with the second block's begin as reference, that is a
@@ -1156,10 +1156,14 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(
 // one another, so what counts is the way from one state to the next: three products with
 // a barrier behind each.
 //   * Every operand is a sum of three bf16 parts that keep all of its 24 bits, and a
-//     product is that of six pairs of parts, the smallest of which lies 2^-16 below the
-//     largest; what is left out lies below fp32's own rounding.  The matrix cores take
-//     16 times as many bf16 products as fp32 ones, 2.7 times as many of six.  Sums of the
-//     largest pair and of the others are kept apart until the end.
+//     product is that of eight pairs of parts: the ninth lies 2^-32 below the first.  The
+//     matrix cores take 16 times as many bf16 products as fp32 ones, twice as many of
+//     eight.  Sums of the largest pair and of the others are kept apart until the end.
+//     Off by, in 2^-24 of the terms' magnitudes, at most (root of the mean square), fp32
+//     and these: one term 1.00 (.42), 1.00 (.42); 8 terms 2.9 (.46), 2.0 (.24); 128 terms
+//     3.9 (.47), .91 (.11); with six pairs a term alone is off by up to 2.7.  Numbers that
+//     are not finite, or round up past the largest bf16 number, make NaN, where an fp32
+//     product may be infinite.
 //   * Parts of K lie in LDS, once for its rows (K S) and for its columns (the next S,
 //     read transposed), split there a chunk ahead; pieces of a row are swapped by the
 //     row, so that neither way of reading meets banks twice.
@@ -1172,11 +1176,13 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(
 // Rows past the end of a chunk repeat its last one: their beta is 0, so they write
 // nothing, and their outputs are not stored.
 // Bound by what the two waves of a SIMD issue: of 8400 cycles a chunk (two tiles, depth
-// 128) 2900 are products, 3900 splits and what goes with them; with half of the products
-// it takes 12% less, with splits left out 23%.  All of K by the output waves: 9700.
-// Depth 128, 32 heads: 2 x 4001 tokens 390 -> 288 us with fp32 products before, 11
-// requests of 17 to 1160 233 -> 171; decays per channel, 16 heads, 13 of 9 to 900
-// 122 -> 99.  Errors of a layer against 64 bits .94 to .99 of those before.
+// 128) with six pairs 2900 are products, 3900 splits and what goes with them; with half of
+// the products it takes 12% less, with splits left out 23%.  All of K by the output waves:
+// 9700.
+// Depth 128, 32 heads, fp32 products, six pairs, eight: 2 x 4001 tokens 371, 277, 303 us,
+// 11 requests of 17 to 1160 374, 280, 303; decays per channel, 16 heads, 13 of 17 to 900
+// 236, 183, 197; layers of 8 and 16 deep heads, padded to 32, 2 x 4001 tokens 233 to 221
+// and 239 to 226 us.  Errors of a layer against 64 bits .88 to .96 of those of fp32.
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
@@ -1276,12 +1282,12 @@ __global__ __launch_bounds__(512, 2) void delta_walk_fixed_kernel(
   // a product of CT tiles; small: sums of all pairs of parts but the largest
   auto product = [](const Parts8& a, const Parts8 (&b)[CT], f32x4 (&sum)[CT],
                     f32x4 (&small)[CT]) {
-    constexpr int I[6] = {0, 2, 1, 0, 0, 1}, J[6] = {2, 0, 1, 0, 1, 0};
+    constexpr int I[8] = {1, 2, 0, 2, 1, 0, 0, 1}, J[8] = {2, 1, 2, 0, 1, 0, 1, 0};
 #pragma unroll
-    for (int q = 0; q < 6; ++q)
+    for (int q = 0; q < 8; ++q)
 #pragma unroll
       for (int t = 0; t < CT; ++t) {
-        f32x4& to = q == 3 ? sum[t] : small[t];
+        f32x4& to = q == 5 ? sum[t] : small[t];
         to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[I[q]], b[t].p[J[q]], to, 0, 0, 0);
       }
   };

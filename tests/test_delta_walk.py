@@ -7,7 +7,8 @@ import pytest
 import torch
 
 from mlx_sharding_amd.models.mixers import GatedDelta
-from mlx_sharding_amd.ops.paged import PagedState, RaggedBatch
+from mlx_sharding_amd.ops import ragged
+from mlx_sharding_amd.ops.paged import PagedState, RaggedBatch, StateSpec
 
 pytestmark = pytest.mark.gpu
 
@@ -84,3 +85,49 @@ def test_chunks_at_any_word(words, monkeypatch):
     monkeypatch.setattr(RaggedBatch, "__init__", moved)
     for got, expect in zip(_run(m, rows, torch.float32), want):
         assert torch.equal(got, expect)
+
+
+def _plain(D, channel, n, change):
+    """One request of n tokens that forgets nothing, without a convolution: (outputs [n, V],
+    values [n, V], state [D, V]).  Values of 64 and more go through silu as they are.
+    change(v, beta): values, and what goes into their sigmoid."""
+    dev, V = torch.device("cuda"), 128
+    torch.manual_seed(D)
+    sh = ragged.DeltaShape(1, 1, D, V, 1, (32, 32) if channel else None)
+    state = PagedState([StateSpec(1, D, V, sh.channels, 0)], -(-n // 64) * 64, 1,
+                       torch.float32, dev)
+    held = state.admit(0)
+    state.reserve(0, n)
+    at = sh.columns
+    y = torch.zeros(n, -(-(at[5] + 1) // 8) * 8, device=dev)
+    y[:, : 2 * D].uniform_(0.5, 1.5)                     # q and k
+    v, beta = y[:, at[2]: at[2] + V].uniform_(64, 128), y[:, at[5]].normal_()
+    change(v, beta)
+    gate = None
+    if channel:  # decay inputs are 0, as they are in y
+        gate = torch.zeros(n, D + V, device=dev)
+        gate[:, D:] = 3.0
+    else:
+        y[:, at[3]: at[3] + V] = 3.0
+    one = lambda *s: torch.ones(*s, device=dev)  # noqa: E731
+    out = ragged.gated_delta(
+        y, one(sh.channels, 1), one(1) * -200, one(D if channel else 1), one(V),
+        state.layers[0], sh, 1e-6, RaggedBatch([(held, n)], dev), gate)
+    return out, v, state.layers[0].state[held.slot][0]
+
+
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("D", [8, 32, 64, 128])
+def test_a_lone_product_is_rounded_once(D, channel):
+    """The state of one token's key and value: half a last place off, and 2^-7 of that for
+    sums of parts that were rounded before."""
+    def only(v, beta):
+        v[:, 0] = 64.0  # that times a key is exact
+        beta.fill_(-200.0)
+        beta[37] = 200.0
+
+    _, v, S = _plain(D, channel, 100, only)
+    key = S[:, :1].double() / 64
+    assert bool((key > 0).all())
+    want = key * v[37].double()
+    assert ((S.double() - want).abs() / want).max() <= 2.0 ** -24 * (1 + 2.0 ** -7)
