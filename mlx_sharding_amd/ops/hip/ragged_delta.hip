@@ -1464,13 +1464,15 @@ __global__ __launch_bounds__(512, 2) void delta_walk_fixed_kernel(
         }
         issued();
       };
-      // ... times columns of `x`
+      // ... times columns of `x`; beside tiles that are not there, zeros, lie tokens of this
+      // wave's own tile: what is no number in a later one stays there
       Parts8 lb[2][CT];
       auto read_lower = [&](const char* x) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int t = 0; t < CT; ++t) get8(x + wide(t * 16 + lr, j * 32 + g4 * 8), UB, lb[j][t]);
+          for (int t = 0; t < CT; ++t)
+            get8(x + wide(t * 16 + lr, min(j * 32 + g4 * 8, w * 16 + 8)), UB, lb[j][t]);
         issued();
       };
       auto lower = [&](f32x4 (&to)[CT], f32x4 (&small)[CT]) {

@@ -131,3 +131,17 @@ def test_a_lone_product_is_rounded_once(D, channel):
     assert bool((key > 0).all())
     want = key * v[37].double()
     assert ((S.double() - want).abs() / want).max() <= 2.0 ** -24 * (1 + 2.0 ** -7)
+
+
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("token", [16, 20, 52, 127])
+def test_what_is_no_number_stays_with_its_neighbours(token, channel):
+    """Tokens before those 16 that a value without a number lies in do not see it."""
+    def spoil(v, beta):
+        v[token, 5] = float("nan")
+
+    want = _plain(64, channel, 150, lambda v, beta: None)[0]
+    got = _plain(64, channel, 150, spoil)[0]
+    before = token // 16 * 16
+    assert torch.equal(got[:before], want[:before])
+    assert bool(got[token].isnan().any())
