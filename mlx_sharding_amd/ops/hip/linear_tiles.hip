@@ -13,19 +13,24 @@
 // widths and 65 to 8192 rows 1.16 times faster on average where chosen, 1.02 at least (us,
 // there and here: 1905 rows of 4096 into 2 x 14336 385, 361; 6000 of 3584 1083, 928; 1000
 // of 2048 into 2 x 8192 65, 53; 8192 of 2048 467, 411; but 600 of 4096 140, 160).
-//   Long contractions into few columns leave the library with few tiles (16 widths, 1.34
-// times faster on average, 10 of 136 sizes slower, by up to 11%): 80 rows of 14336 into
-// 3584 42 and 31, 512 88 and 69, 1000 of 18944 185 and 117, 330 of 8192 into 2048 31 and
-// 28; below 8192 it is the better one (281 of 5632 into 2048 24, 25), and from some 1300
-// rows on, where columns are a multiple of 1024 (3684 of 14336 into 4096 315, 331).
-// Where they are not its kernels fall to half of their rate at some row counts (into 3584:
-// 1905 rows 333 and 168, 3684 465 and 307; 1700 158 and 171).
+//   Long contractions into few columns leave the library with few tiles: it takes those of
+// 256 x 256, one after the other over the contraction, so the rule counts them.  Library's
+// time over that here, 65 to 8192 rows, 12 widths from 1024, 11 contractions: chosen ones
+// 1.48 times on average, 55 of 1983 slower (by 3 to 16%); above 16384 columns 1.98 (9 of
+// 789), 13824 to 16384 1.26 (21 of 697), 11008 and 12288 1.18 (14 of 371).  With 81 to 128
+// tiles, 11008 and 12288: 1.09 (16 of 78), 13824 and 14336: 1.17 (6 of 86), above 16384
+// 1.49 (9 of 147).  With 129 to 256 the library's kernel may be a good one or take twice as
+// long (14336 into 3584: 3684 rows 466 and 272, 4096 rows 273 and 299; 1.03, 271 of 390).
+// From 8192 on only into a fifth as many columns: 1.07 (11 of 126; 65 rows of 8192 into
+// 1024 1.23), above 40 tiles .94.  Rows of whole 32 KB meet few of the memory's channels,
+// which shares in tiles of 128 rows show: 65 rows of 16384 into 8192 63 and 107.
 extern "C" int linear_tiles_plan(long M, long O, long K, int act, bool bias, int* shares) {
   *shares = 1;
   if (M <= 64 || K < 192 || K % 64 || O < 64 || O % 64 || (act && bias)) return 0;
-  const bool plain = K >= 8192 && K >= 2 * O && O >= 1024 &&
-                     (M <= 1280 || (K >= 14336 && O % 1024));
-  if (!act && !plain) return 0;
+  const long across = ((M + 255) / 256) * ((O + 255) / 256);
+  const bool plain = K < 10240 ? K >= 8192 && K >= 5 * O && across <= 40
+                               : K >= (K % 16384 ? 2 : 3) * O && across <= (K < 13312 ? 80 : 128);
+  if (!act && (!plain || O < 1024)) return 0;
   const long stages = K / 64;
   const int most = act ? 1 : 16;
   double least = 0;

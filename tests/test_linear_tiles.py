@@ -103,6 +103,18 @@ def test_forms_that_the_rule_takes(M, O, K, act):
             assert bool(((got.reshape(M, -1).double() - want).abs() <= off).all())
 
 
+@pytest.mark.parametrize("M,O,K,taken", [
+    (65, 1024, 8128, False), (65, 1024, 8192, True), (65, 960, 8192, False),
+    (65, 1600, 8192, True), (65, 1664, 8192, False), (2560, 1024, 8192, True),
+    (2561, 1024, 8192, False), (65, 1984, 10176, True), (65, 2048, 10176, False),
+    (65, 5120, 10240, True), (65, 5184, 10240, False), (5120, 1024, 12288, True),
+    (5121, 1024, 12288, False), (2048, 4096, 14336, True), (2049, 4096, 14336, False),
+    (1905, 3584, 14336, True), (65, 5440, 16384, True), (65, 5504, 16384, False),
+    (64, 3584, 14336, False)])
+def test_borders_of_the_rule_for_long_contractions(M, O, K, taken):
+    assert bool(ext().linear_tiles_plan(M, O, K, 0, False)[0]) == taken
+
+
 def test_what_is_watched_keeps_torch():
     x, w, _ = operands(300, 1024, 8192)
     assert ops._linear_few(x, w) is not None
