@@ -689,12 +689,14 @@ torch::Tensor mla_attend(torch::Tensor q, torch::Tensor cache, torch::Tensor w,
   const long span = s_ptr ? cache.size(2) : S;
   // A slice more is a partial result more that every block of mla_finish reads of each of
   // its up to 16 tokens, and fewer tiles one after the other: 8 sqrt(tiles / tokens) of
-  // them are near the least of both (with both kernels, by slices: 16 sequences of 577
-  // keys 19: 22.8 us, 10: 18.1, 7: 16.5, 4: 18.3; 8 of 1000 32: 18.6, 16: 15.4, 8: 15.7;
-  // 4 of 2000 63: 18.6, 32: 15.4, 16: 15.7; one of 3001 47: 12.7, 32: 13.2, 16: 17.5).
+  // them are near the least of both, and so are all of up to five tiles (both kernels, by
+  // slices: 16 sequences of 577 keys 16: 17.1 us, 10: 17.3, 8: 16.0, 4: 18.0; of 130 keys 5:
+  // 13.1, 4: 13.9; 4 of 2000 56: 15.2, 32: 15.2, 16: 15.6; one of 3001 64: 12.7, 32: 13.2,
+  // 16: 17.3).  Over 166 sizes 2% behind the best of 20 counts on average, 5 where there
+  // are as many as CUs hold.
   const long tiles = (span + tile - 1) / tile;
   const int n = std::min(decode_slices(N, span, tile),
-                         std::max(1, (int)(8.0 * std::sqrt((double)tiles / std::min(N, 16L)))));
+                         std::max(5, (int)(8.0 * std::sqrt((double)tiles / std::min(N, 16L)))));
   auto fopts = q.options().dtype(torch::kFloat32);
   auto po = torch::empty({N * heads * n, rank}, fopts);
   auto pml = torch::empty({N * heads * n, 2}, fopts);

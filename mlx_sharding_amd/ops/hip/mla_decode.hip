@@ -110,8 +110,9 @@ __global__ __launch_bounds__(MD_BLOCK) void mla_prepare_kernel(
 // Bound by the trips to memory that follow one another, and by what a CU reads: the
 // slices' maxima, the first partial results and the first rows of the matrix are under
 // way together, slices that hold no keys are left out, and where the tokens leave threads
-// over, groups of them share a token's slices.  With the attention before it, one token
-// of 3001 keys 14.4 -> 12.7 us, of 577 11.4 -> 10.5, 128 tokens of 577 34.6 -> 31.4.
+// over, groups of them share a token's slices.  64 slices of 5 tokens 12.5 -> 11.5 us, 32 of
+// 16 as fast (13.8), 17 (32 before) 14.3 -> 8.6; with the attention before it one token of
+// 3001 keys 14.4 -> 12.7, of 577 11.4 -> 10.8, 128 tokens of 577 34.6 -> 31.4.
 __global__ __launch_bounds__(512) void mla_finish_kernel(const MlaFinishArgs a) {
   // a token's latent [16][rank + 8] in bf16: the odd stride keeps the 16 rows that
   // a read meets in different banks
@@ -209,20 +210,39 @@ __global__ __launch_bounds__(512) void mla_finish_kernel(const MlaFinishArgs a) 
     for (int j = 0; j < 4; ++j) r[j] = (__bf16)o[j];
     *reinterpret_cast<bf16x4_t*>(lat + x.t * stride + x.d) = r;
   };
+  // Of an item the slices from s on, eight more on their way.  Sums of whole eights have
+  // no conditions, which their loads would wait for one by one.
+  auto eight = [&](f32x4& o, const f32x4 (&v)[8], const Item& x, int s) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float f = weight[x.t][s + j];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[k] += v[j][k] * f;
+    }
+  };
+  auto total = [&](f32x4 (&v)[8], const Item& x, int s, int end) {
+    f32x4 u[8], o = {0, 0, 0, 0};
+    for (; s + 16 <= end; s += 16) {
+      load(u, x, s + 8, end);
+      eight(o, v, x, s);
+      if (s + 16 < end) load(v, x, s + 16, end);
+      eight(o, u, x, s + 8);
+    }
+    if (s + 8 < end) load(u, x, s + 8, end);
+    if (s + 8 <= end) eight(o, v, x, s);
+    else add(o, v, x, s, end);
+    if (s + 8 < end) add(o, u, x, s + 8, end);
+    return o;
+  };
+  f32x4 v[8];
   if (groups > 1) {
     const int g = over(threadIdx.x, items), share = (used + groups - 1) / groups;
     const Item x = item_of(g < groups ? (int)threadIdx.x - g * items : 0);
-    const int end = g < groups ? min(used, (g + 1) * share) : 0;
-    int s = g * share;
-    f32x4 v[8], o = {0, 0, 0, 0};
+    const int end = g < groups ? min(used, (g + 1) * share) : 0, s = g * share;
     load(v, x, min(s, used - 1), max(end, 1));
     if (first < last) fetch(rows(first), 0);
     weigh();
-    while (s < end) {
-      add(o, v, x, s, end);
-      s += 8;
-      if (s < end) load(v, x, s, end);
-    }
+    f32x4 o = total(v, x, s, end);
     sums[threadIdx.x] = o;
     __syncthreads();
     if (g == 0) {
@@ -235,18 +255,11 @@ __global__ __launch_bounds__(512) void mla_finish_kernel(const MlaFinishArgs a) 
     }
   } else {
     Item x = item_of(min((int)threadIdx.x, items - 1));
-    f32x4 v[8];
     load(v, x, 0, used);
     if (first < last) fetch(rows(first), 0);
     weigh();
     for (int i = threadIdx.x; i < items;) {
-      f32x4 o = {0, 0, 0, 0};
-      for (int s = 0; s < used;) {
-        add(o, v, x, s, used);
-        s += 8;
-        if (s < used) load(v, x, s, used);
-      }
-      keep(x, o);
+      keep(x, total(v, x, 0, used));
       i += 512;
       if (i < items) {
         x = item_of(i);
