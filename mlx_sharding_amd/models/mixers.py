@@ -108,11 +108,16 @@ class NormedLinear(Linear):
         self.norm = RMSNorm(normed, eps, dtype=dtype)
 
 
-# Tokens up to which the heads' products of absorbed attention take the kernel for
-# few rows.  16 heads, 128 and 512 wide, into the latent space and out of it: 12 rows
-# 2.4 and 2.8 us (library with its copies 7.6 and 13.5), 256 rows 7.8 and 7.4 (10.2
-# and 17.7), 512 rows 13.4 and 16.4 (12.1 and 13.4).
+# Tokens, and products of them, up to which the heads' products of absorbed attention take
+# the kernel for few rows, whose blocks of 16 outputs read the rows again and again.  16
+# heads, 128 and 512 wide, into the latent space and out of it: 12 rows 2.4 and 2.8 us
+# (library with its copies 7.6 and 13.5), 256 rows 7.8 and 7.4 (10.2 and 17.7), 512 rows
+# 13.4 and 16.4 (12.1 and 13.4).  1 to 128 heads, 32 to 192 and 64 to 1024 wide, library's
+# time over the kernel's: up to these products 1.08 to 5.2 in bf16, .95 to 12 in 32 bits
+# (6 of 282 below .97); above them down to .32 (64 heads of 128 and 512, 64 rows 1.20, 128
+# rows .92, 256 .68).
 FEW_TOKENS = 256
+FEW_PRODUCTS = {torch.bfloat16: 750_000_000, torch.float32: 450_000_000}
 
 
 class LatentAttention(nn.Module):
@@ -179,6 +184,12 @@ class LatentAttention(nn.Module):
         self.w_o = wo.reshape(width, H * sh.vdp).contiguous()
         self.ready = True
 
+    def few(self, n: int) -> bool:
+        """Whether the heads' products of n tokens take the kernel for few rows."""
+        sh = self.shape
+        return (n <= FEW_TOKENS and n * sh.heads * sh.rankp * (sh.dimp + sh.vdp)
+                <= FEW_PRODUCTS.get(self.w_uk.dtype, 0))
+
     def forward(self, h: torch.Tensor, batch: RaggedBatch, store: LayerStore,
                 tables) -> torch.Tensor:
         """store: the layer's own, or that of the layer it reads."""
@@ -200,7 +211,7 @@ class LatentAttention(nn.Module):
         parts = []
         if n:
             qn = q[:n].unflatten(1, (H, sh.dq))[..., : sh.dimp]
-            few = q.is_cuda and n <= FEW_TOKENS
+            few = q.is_cuda and self.few(n)
             q_abs = ragged.latent_heads(qn, self.w_absorb_few, True) if few else \
                 torch.bmm(qn.transpose(0, 1).contiguous(), self.w_absorb)
             o = ragged.latent_attention_absorbed(q, q_abs, store, sh,

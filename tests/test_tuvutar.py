@@ -162,6 +162,14 @@ LATENTS = {
 }
 
 
+@pytest.mark.parametrize("heads,dtype,last", [
+    (16, BF16, 256), (64, BF16, 89), (128, BF16, 44), (16, F32, 143), (64, F32, 35)])
+def test_tokens_that_the_kernel_for_few_rows_takes(heads, dtype, last):
+    mix = Mixer(cases.latent(heads, 128, 64, 128, 512), 32, dtype, "cpu").mix
+    mix.prepare()
+    assert mix.few(last) and not mix.few(last + 1)
+
+
 @pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("kind", LATENTS)
