@@ -446,23 +446,26 @@ extern "C" bool attn_prefill_supported(int Dk, int Dv) {
 // the longest blocks are alone with.  Two teams fill it and halve the chain of tiles;
 // adding them up costs 1 to 2 us, so the chain has to be long, and blocks of like length
 // gain nothing.  One team, two, us: 16 heads of 256, capped: 1905 tokens behind 4096 264,
-// 206 (with a window of 4096 197, 161), 384 24.5, 23.9, 256 18.8, 19.9, 64 8.0, 10.5; 4096
-// (512 blocks) 212, 173, with a window of 1024 95, 110; 32 of 128: 1024 24.0, 22.1, 640
-// 16.5, 16.2, 512 14.0, 14.4, 64 behind 4032 75, 57; 1500 (384 blocks) 35.9, 31.9, 2048
-// (512) 51.3, 48, 3000 (768) 90, 103; 2 x 1024 (512) 30.2, 32.4; 4 x 768 22.2, 24.3.
-static bool two_teams(const PrefillArgs& a, unsigned blocks, int keys) {
+// 206 (with a window of 4096 197, 161), 384 24.7, 24.5, 320 19.7, 20.6, 64 8.0, 10.5; 4096
+// (512 blocks) 212, 173, with a window of 1024 95, 110; not capped 512 27.1, 26.8, 448 22.3,
+// 22.6; 32 of 128: 1024 24.0, 22.1, 640 16.5, 16.2, 200 behind 400 16.3, 16.7, 64 behind
+// 4032 75, 57; 1300 (352 blocks) 31.2, 28.1, 2048 (512) 51.3, 48, 3000 (768) 90, 103;
+// 2 x 1024 (512) 30.2, 32.4; 4 x 768 22.2, 24.3; 8 x 900, 8 heads of 256 (512) 49, 56.
+// Of 2142 sizes of 64 to 256 columns with up to 512 blocks 1300 have two, one of them 3%
+// slower so, and the rule is 1.0% behind the better one of both on average.
+static bool two_teams(const PrefillArgs& a, unsigned blocks, bool wide) {
   const bool whole = a.window <= 0 || a.window >= a.S;
-  const int longest =
-      ((whole ? a.S : (int)std::min<long>(a.S, (long)a.window + AP_WAVES * 32 - 1)) + keys - 1) / keys;
-  if (blocks <= 256) return longest >= 10;
-  return blocks <= 512 && longest >= 24 && whole && a.offset == 0;
+  const long longest =
+      whole ? a.S : std::min<long>(a.S, (long)a.window + AP_WAVES * 32 - 1);  // keys
+  if (blocks <= 256) return longest >= (!wide ? 608 : a.cap.out > 0.0f ? 384 : 512);
+  return blocks <= 512 && longest >= 1280 && whole && a.offset == 0;
 }
 
 template <int DK, int DV, bool CAP, int NOPE = 0, bool RAGGED = false>
 static void attn_prefill_run(const PrefillArgs& a, hipStream_t stream) {
   const unsigned blocks = (unsigned)a.heads * a.tiles;
   if constexpr (!RAGGED) {
-    if (two_teams(a, blocks, ap_keys(DK, DV))) {
+    if (two_teams(a, blocks, ap_keys(DK, DV) == 32)) {
       attn_prefill_kernel<DK, DV, CAP, 2, NOPE>
           <<<dim3(blocks), dim3(2 * AP_BLOCK), 0, stream>>>(a);
       return;
