@@ -177,7 +177,8 @@ class LatentAttention(nn.Module):
         # absorbed form: [H, dimp, rankp] into the query, [H, rankp, vdp] out
         self.w_absorb = self.w_uk.view(H, sh.dimp, sh.rankp)
         self.w_emit = self.w_uv.view(H, sh.vdp, sh.rankp).transpose(1, 2).contiguous()
-        # and the same with the contraction along the rows, for few tokens
+        # and the same with the contraction along the rows, for few tokens (one is a copy
+        # more: 2 MB a layer of 16 heads of 128 and 512)
         self.w_absorb_few = self.w_absorb.transpose(1, 2).contiguous()
         self.w_emit_few = self.w_uv.view(H, sh.vdp, sh.rankp)
         wo = F.pad(wo.view(width, H, sh.vdim), (0, sh.vdp - sh.vdim))

@@ -9,8 +9,9 @@
 // the best tile and shares of those tried are .5% faster on average), and of the sums'
 // second kernel.
 //   Gated units save a pass over both halves, so they are here unless the tiles fill their
-// last round badly, beside a library at .95 to 1.5 PFLOP/s by its contraction: over 13
-// widths and 65 to 8192 rows 1.16 times faster on average where chosen, 1.02 at least (us,
+// last round badly, beside a library at .95 to 1.5 PFLOP/s by its contraction: over 12
+// widths, 11 contractions of 512 to 8192 and 65 to 8192 rows 1.32 times faster on average
+// where chosen (from 2.0 at 512 columns to 1.04 at 8192), 1 of 1409 sizes slower by 3% (us,
 // there and here: 1905 rows of 4096 into 2 x 14336 385, 361; 6000 of 3584 1083, 928; 1000
 // of 2048 into 2 x 8192 65, 53; 8192 of 2048 467, 411; but 600 of 4096 140, 160).
 //   Long contractions into few columns leave the library with few tiles: it takes those of

@@ -649,8 +649,8 @@ __global__ __launch_bounds__(DC_BLOCK) void delta_conv_state_kernel(
 //   am [chunks, H, 64, 64]  A (lower tiles only)
 //   ge [chunks, H, 2, 64]   exp(G), exp(G_last - G)
 // Bound by latency, and by what is written.  Operands are on their way a step ahead, and
-// the value heads of a q/k head run on one XCD: 126 chunks of 32 heads 138 -> 110 us;
-// two of them in a block: 118 -> 84.
+// the value heads of a q/k head run on one XCD: 126 chunks of 32 heads 138 -> 110 us; with
+// two of them in a block 118 -> 84 (another card, on which that kernel took 118).
 // ---------------------------------------------------------------------------
 
 #define DR_LS 68
