@@ -166,9 +166,9 @@ read_in_place(nn.Embedding)
 def head(norm: nn.Module, x: torch.Tensor, out: Optional[nn.Module] = None,
          table: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``out``, or the product with an embedding's rows, of x's normed rows; one kernel
-    for few rows.  For 33 to 64 of them and many weights the library's product behind a
-    norm of its own is the faster one (64 rows, here and there: 16032 x 4096 30, 35 us;
-    32000 x 2048 34.5, 37.8; 21720 x 3584 49, 41; 128256 x 4096 236, 221)."""
+    for few rows.  For 33 to 64 of them and many weights the norm has a kernel of its own
+    (2 us of 40 and more; 64 rows, the product alone and the library's: 21720 x 3584 33.8,
+    38.6 us; 32000 x 3584 46.0, 44.3; 128256 x 4096 192, 213)."""
     if ops.few_tokens(x) and as_built(norm) and (out is None or as_built(out)):
         V, K = table.shape if out is None else (out.out_features, out.in_features)
         if x.numel() <= 32 * K or V * K <= 1 << 26:
@@ -176,7 +176,7 @@ def head(norm: nn.Module, x: torch.Tensor, out: Optional[nn.Module] = None,
                 return ops.project(x, table, norm=norm)
             return project(out, x, norm=norm)
     x = norm(x)
-    return x @ table.t() if out is None else out(x)
+    return ops.linear(x, table) if out is None else out(x)
 
 
 class StageModel(nn.Module):

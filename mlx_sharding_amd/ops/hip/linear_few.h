@@ -149,22 +149,18 @@ static bool linear_few_weight(const torch::Tensor& w, const torch::Tensor& x) {
 
 // Whether a product of this size runs here.  A contraction above 8192 for 8 rows, or
 // into 4096: 8 rows of 14336 into 4096 take 24.6 us here and 26.6 in the library, 32
-// rows 30.4 and 30.5, 64 rows 40.1 and 38.9.  alone: with nothing taken along; then the
-// library is the better one for many rows of large weights (64 rows of 4096 into 28672:
-// 54 us here, 51 there).
-static bool linear_few_sizes(long rows, long O, long K, bool alone) {
+// rows 30.4 and 30.5, 64 rows 40.1 and 38.9.
+static bool linear_few_sizes(long rows, long O, long K) {
   return O >= 1 && K >= 32 && K % 32 == 0 && rows >= 1 && rows <= 64 &&
-         !(K > 8192 && rows > 8 && O > 4096) &&
-         !(alone && rows > 32 && O * K > 1 << 25) && !linear_few_other(K);
+         !(K > 8192 && rows > 8 && O > 4096) && !linear_few_other(K);
 }
 
 // Whether x w^T runs here.
-static bool linear_few_takes(const torch::Tensor& x, const torch::Tensor& w,
-                             bool alone) {
+static bool linear_few_takes(const torch::Tensor& x, const torch::Tensor& w) {
   if (!linear_few_input(x) || !linear_few_weight(w, x) || w.size(1) < 1 ||
       x.size(-1) != w.size(1))
     return false;
-  return linear_few_sizes(x.numel() / w.size(1), w.size(0), w.size(1), alone);
+  return linear_few_sizes(x.numel() / w.size(1), w.size(0), w.size(1));
 }
 
 // Whether a product here takes along what it is given: a bias per row of w and norm
@@ -273,7 +269,7 @@ static c10::optional<torch::Tensor> linear_few_try(
     if (residual.has_value() || norm.has_value() || clear.has_value()) return {};
     return linear_many_try(x, w, bias, act);
   }
-  if (!linear_few_takes(x, w, !residual.has_value() && !norm.has_value() && !act) ||
+  if (!linear_few_takes(x, w) ||
       !linear_few_along(x, w.size(0) / (act ? 2 : 1), w.size(0), bias, residual, norm))
     return {};
   const auto rows = linear_few_rows(x);
@@ -299,15 +295,13 @@ static c10::optional<torch::Tensor> feed_few_try(
     c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> norm, double eps,
     double offset, int64_t act) {
   TORCH_CHECK(act == 1 || act == 2, "unknown unit");
-  if (!linear_few_takes(x, w_in, false) || !linear_few_weight(w_out, x) ||
+  if (!linear_few_takes(x, w_in) || !linear_few_weight(w_out, x) ||
       w_in.size(0) != 2 * w_out.size(1))
     return {};
   const int M = x.numel() / x.size(-1), O = w_out.size(0), I = w_out.size(1);
   // long contractions into many columns have a kernel of their own (gemm_kseg.hip)
   if (I >= 16384 && O >= 8192 && !residual.has_value()) return {};
-  int shared = 0;
-  if (O >= 1 && I >= 32) linear_few_room(M, O, I, &shared);
-  if (!linear_few_sizes(M, O, I, !shared && !residual.has_value()) ||
+  if (!linear_few_sizes(M, O, I) ||
       !linear_few_along(x, I, 2 * I, {}, {}, norm) ||
       !linear_few_along(x, O, O, {}, residual, {}))
     return {};

@@ -19,152 +19,7 @@
 // these: 48, 59; 1 x 14336 x 4096: 22.5, 26; 8 of these: 24.6, 26.6; 16: 29, 26.
 // With norm and unit, 1 x 4096 x 28672: 46, beside 72 for three kernels.
 
-#include "hip_common.h"
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// Two lines of 64 bytes, which a block asks for at once: numbers of a third line, or of the
-// second when the first had come, took every launch 0.4 us.
-struct LinearFewArgs {
-  const __bf16 *x, *w, *bias, *res, *norm;
-  __bf16* y;
-  short M;
-  // parts > 1: blocks share a tile's contraction, `share` steps (few) or stages
-  // (some) each.  part [tiles of y, parts, tiles of x, WAVE, 4], count: one number per
-  // tile of y and x, zero before.
-  unsigned char parts;
-  unsigned char fours;     // bias and residual are read by fours
-  int O, K;                // O: columns of y
-  int share;
-  long ldx, ldw, ldr, ldy;
-  union {
-    struct { float eps, offset; };  // norm weights are norm + offset
-    float* part;                    // without a norm
-  };
-  unsigned turn;           // 2^32 / chunks of a share, rounded up, for first_of
-  int n_zero;              // numbers at zero that this launch clears for a later one
-  unsigned *count, *zero;
-};
-static_assert(sizeof(LinearFewArgs) == 128, "two lines");
-
-// all of a, now
-__device__ __forceinline__ void arrive(const LinearFewArgs& a) {
-  asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.bias), "s"(a.res), "s"(a.norm), "s"(a.O),
-               "s"(a.K), "s"(a.share), "s"(a.ldx), "s"(a.ldw), "s"(a.turn), "s"(a.zero));
-}
-
-// Where a block begins in the n chunks of a contraction; it goes round from there.
-// Where rows of W lie in step (in_step), blocks at one column ask few of the memory's
-// channels: 16384 rows of 2048, 12 of x, 16.4 us from column 0 on, 14.1 so (the blocks of an
-// XCD, which are every eighth, three chunks apart; one apart 14.2, seven 14.5); 28672 of 4096
-// with norm and unit 45.6, 43.5; 6144 of 4096 14.7, 13.2; 14080 of 5504, 8 of x, 39.3, 32.5;
-// 64 of x, four tiles, rows of 4096 .87 of the time.  Others need none, and going round costs
-// them up to 10% (turn 0: 8 of x, 16064 units of 5376 64.0 us from column 0 on, 70.2 else; one
-// of x, 7008 rows of 16192 42.6, 46.8).  `turn` divides by the chunks of a whole share: the
-// last may have less.
-__device__ __forceinline__ int first_of(const LinearFewArgs& a, int whole, int n) {
-  if (!a.turn) return 0;
-  const unsigned at = (blockIdx.x >> 3) * 3;
-  return max(min((int)(at - __umulhi(at, a.turn) * whole), n - 1), 0);
-}
-
-// The sums of a tile that blocks share: leaves this one's, and true in the one that
-// comes last, which then has all, added in the blocks' order.  Sums pass the L2s, which
-// XCDs have of their own, by accesses of the device's scope.
-__device__ __forceinline__ bool sums_of_all(const LinearFewArgs& a, long tile,
-                                            int lane, f32x4& v) {
-  typedef unsigned long long u64;
-  typedef u64 u64x2 __attribute__((ext_vector_type(2)));
-  u64* to = reinterpret_cast<u64*>(a.part) + (tile * a.parts * WAVE + lane) * 2;
-  const u64x2 own = __builtin_bit_cast(u64x2, v);
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    __hip_atomic_store(to + blockIdx.y * (WAVE * 2) + i, own[i], __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  unsigned before = 0;
-  if (lane == 0)
-    before = __hip_atomic_fetch_add(a.count + tile, 1u, __ATOMIC_RELAXED,
-                                    __HIP_MEMORY_SCOPE_AGENT);
-  before = __builtin_amdgcn_readfirstlane(before);
-  if (before + 1 != a.parts) return false;
-  asm volatile("" ::: "memory");
-  v = f32x4{0, 0, 0, 0};
-#pragma unroll 4
-  for (unsigned s = 0; s < a.parts; ++s) {
-    u64x2 p;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      p[i] = __hip_atomic_load(to + s * (WAVE * 2) + i, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-    const f32x4 f = __builtin_bit_cast(f32x4, p);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] += f[j];
-  }
-  return true;
-}
-
-enum { LF_PLAIN = 0, LF_SILU = 1, LF_GELU = 2 };
-
-typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-
-// What is added to four columns of y, if it may be read by fours.  Asked for before the
-// contraction: behind it, the residual's were four reads one after the other (us without
-// and with a residual; one of x, 2048 rows of 2048 5.4 and 5.6, so 5.1 both; 12 of x, 4096
-// of 4096 9.4 and 9.9, so 9.2 both; 64 of x 13.8 and 14.4, so 13.5 and 13.9).
-template <int ACT>
-struct Ends {
-  bf16x4_t res, bias[ACT ? 2 : 1];
-
-  __device__ __forceinline__ void read(const LinearFewArgs& a, int row, int col) {
-    col = min(col, a.O - 4);
-    if (a.res)
-      res = *reinterpret_cast<const bf16x4_t*>(a.res + min(row, a.M - 1) * a.ldr + col);
-    if (a.bias) {
-#pragma unroll
-      for (int h = 0; h < (ACT ? 2 : 1); ++h)
-        bias[h] = *reinterpret_cast<const bf16x4_t*>(a.bias + h * a.O + col);
-    }
-  }
-};
-
-// sums of four columns of y from `col` on, and of an up projection's, to memory
-template <int ACT>
-__device__ __forceinline__ void finish_columns(const LinearFewArgs& a, int row, int col,
-                                               const f32x4* v, const Ends<ACT>& e) {
-  float o[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int at = min(col + j, a.O - 1);
-    float f = v[0][j];
-    if (ACT) {
-      float up = v[1][j];
-      if (a.bias) {
-        f += (float)(a.fours ? e.bias[0][j] : a.bias[at]);
-        up += (float)(a.fours ? e.bias[ACT ? 1 : 0][j] : a.bias[a.O + at]);
-      }
-      if (ACT == LF_SILU) {
-        f = f / (1.0f + __expf(-f)) * up;
-      } else {
-        const float z = 0.7978845608028654f * (f + 0.044715f * f * f * f);
-        f = 0.5f * f * (1.0f + tanhf(z)) * up;
-      }
-    } else if (a.bias) {
-      f += (float)(a.fours ? e.bias[0][j] : a.bias[at]);
-    }
-    if (a.res) f += (float)(a.fours ? e.res[j] : a.res[(long)row * a.ldr + at]);
-    o[j] = f;
-  }
-  __bf16* y = a.y + (long)row * a.ldy + col;
-  if (col + 3 < a.O && a.ldy % 4 == 0) {
-    *reinterpret_cast<bf16x4_t*>(y) =
-        bf16x4_t{(__bf16)o[0], (__bf16)o[1], (__bf16)o[2], (__bf16)o[3]};
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (col + j < a.O) y[j] = (__bf16)o[j];
-  }
-}
+#include "linear_few_kernel.h"
 
 // RT tiles of 16 rows of W; with a gated unit half of them are the gate's, the
 // others the up projection's.  SHARED: blocks have a share of a contraction each (in every
@@ -210,7 +65,7 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
   // this block's share of the contraction
   const int s0 = SHARED ? blockIdx.y * a.share : 0;
   const int steps = SHARED ? min(a.share, a.K / 32 - s0) : a.K / 32;
-  const int chunks = steps / U, first = first_of(a, a.share / U, chunks);
+  const int chunks = steps / U, first = first_of(a, a.share / U, chunks, blockIdx.x);
   // operands of one chunk; the next one's are asked for before this one is used,
   // rows of x among them, as loads come back in order
   struct Chunk {
@@ -317,16 +172,6 @@ __global__ __launch_bounds__(NW * WAVE) void linear_few_kernel(
     if (SHARED && !sums_of_all(a, (long)blockIdx.x * YT + r, lane, v[0])) return;
     if (l16 < a.M) finish_columns<ACT>(a, l16, row0 + r * 16 + lg * 4, v, ends);
   }
-}
-
-// Whether rows that lie ld apart meet the same few of the memory's channels: up to five of
-// them are a multiple of 16 KB, or miss it by less than a channel's 256 bytes.
-static bool in_step(long ld) {
-  for (int n = 1; n <= 5; ++n) {
-    const int off = (int)(n * ld * 2 % 16384);
-    if (min(off, 16384 - off) <= 256) return true;
-  }
-  return false;
 }
 
 // Blocks that share a tile's contraction, as many as have something of it.
@@ -473,7 +318,7 @@ __global__ __launch_bounds__(LS_WAVES * WAVE) void linear_some_kernel(
   // last one repeat it, and columns behind the last one others of its row; nobody takes
   // them (64 of x, 28672 rows of 4096 with norm 53.6 us, 54.4 where they are the first again)
   const int end = (s0 + stages) * W, span = stages * W;
-  int base = (s0 + (WAY == LS_WHOLE ? 0 : first_of(a, a.share, stages))) * W;
+  int base = (s0 + (WAY == LS_WHOLE ? 0 : first_of(a, a.share, stages, blockIdx.x))) * W;
   const int last = base + span - W;
   auto column = [&](int t) {
     int k = base + t * W;
@@ -691,14 +536,16 @@ static bool few_through_lds(int M, int O, int K, int act, bool norm) {
 // x, so that long rows have blocks of more rows and a part of the columns each, and up to
 // 2048 rows of W leave CUs idle without (us, alone and shared: 64 of x, 2048 rows of 8192
 // 20.7, 13.4, 4096 of 14336 39.6, 29.0; one of x, 2048 of 8192 11.6, 9.7).  In two rounds
-// it loses (64 of x, 2816 rows of 4096 17.4, 19.9; one of x, 2816 of 8192 15.3, 18.3), with
-// short rows it costs what it gains (33 of x, 2048 rows of 2048 11.1, 11.7).  With four tiles
+// it loses (64 of x, 2816 rows of 4096 17.4, 19.9; one of x, 2816 of 8192 15.3, 18.3), and
+// short rows of more than 16 of x are linear_own_kernel's (shared and there: 64 of x, 1536 rows
+// of 2816 7.4, 5.8, 1616 of 4288 10.2, 9.5, 1504 of 5632 10.9, 11.3, 2048 of 8704 16.7, 19.1;
+// 20 of x, 1536 of 5120 8.7, 7.9, 29 of x, 2048 of 9216 12.7, 15.3).  With four tiles
 // up to 16 of x gain from rows of 12288 into up to 3584 on (12 of x, into 2816 23.8, 21.0,
 // into 3584 26.1, 24.3; into 4096 27.7, 28.3; 10240 into 2816 20.6, 20.9).
 static int few_split(int M, int O, int K, int act, bool norm) {
   if (act || norm) return 1;
   if (!few_through_lds(M, O, K, act, norm)) return O <= 2048 && K >= 4096 ? 2 : 1;
-  if (O <= 2048) return K >= (M > 32 ? 2560 : 4096) ? 4 : 1;
+  if (O <= 2048) return K >= (M > 32 ? 5632 : M > 16 ? 7168 : 4096) ? 4 : 1;
   return K >= 8192 && (M > 16 ? O <= 4096 : K >= 12288 && O <= 3584) ? 4 : 1;
 }
 
@@ -730,6 +577,7 @@ extern "C" void launch_linear_few(const void* x, const void* w, const void* bias
   a.fours = (bias || res) && O % 4 == 0 && (long)bias % 8 == 0 && (long)res % 8 == 0 &&
             (!res || ldr % 4 == 0);
   const int split = count ? few_split(M, O, K, act, norm != nullptr) : 1;
+  if (split == 1 && linear_own_go(a, act, stream)) return;
   if (few_through_lds(M, O, K, act, norm != nullptr)) {
     linear_some(a, act, split, stream);
   } else {

@@ -1,0 +1,534 @@
+// y = x W^T for 17 to 64 rows of x, whole contractions (what goes along: linear_few.hip).
+//
+// A CU reads rows through LDS at 100 bytes a nanosecond and more as long as a load takes
+// whole lines (128 bytes of 8 rows; 64 bytes of 16 rows, as operands straight to registers
+// are: 35), so that products of up to 30 MB are not bound by what a block reads of x, but by
+// the chain of its stages: the waves of linear_some_kernel meet at each one, 0.6 us of which
+// are 0.35 of reads from LDS and products and, with a norm, 0.85 (64 rows of 2048 into 3648).
+// Two kernels without it:
+//
+//   linear_own_kernel   each wave has a ring of its own in LDS and takes chunks of 64 columns
+//                       by turns, so that no wave waits for another before the sums; for up
+//                       to four tiles of W's rows
+//   linear_ring_kernel  five to eight tiles, which is more than such rings have room for:
+//                       waves meet, half of them load W, half x, in rings of lengths that
+//                       suit each
+//
+// Both take any number of tiles, so that blocks are one round of the chip where few_tiles'
+// two and four leave a second one half empty, and rows of x may be split between blocks
+// that lie eight apart, on one XCD, whose L2 then has W's rows for both.
+#include "linear_few_kernel.h"
+
+namespace {
+
+constexpr int OWN_WAVES = 8;
+
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// Waits until at most the loads of the `younger` last chunks, PER each, are under way; J: of
+// how many that may be at most.
+template <int J, int PER>
+__device__ __forceinline__ void wait_chunks(int younger) {
+  if constexpr (J == 0) {
+    wait_loads<0>();
+  } else {
+    if (younger >= J) wait_loads<J * PER>();
+    else wait_chunks<J - 1, PER>(younger);
+  }
+}
+
+// 16 bytes a lane from memory to LDS (at + 16 * lane).  The compiler does not know of the
+// load, which would have it wait for all before reads of LDS; no register is written.
+__device__ __forceinline__ void to_lds(const char* from, unsigned at) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(from)
+               : "memory", "m0");
+}
+__device__ __forceinline__ unsigned lds_at(const char* smem) {
+  return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) char*)smem;
+}
+
+// The row of W of row `row` of a block's tiles.  A tile of a gated unit has eight columns:
+// rows 4g and 4g + 1 are the gate's of columns 2g and 2g + 1, the two others the up
+// projection's, so that a lane has both sums of a column.
+template <bool GATED>
+__device__ __forceinline__ const __bf16* row_of(const LinearFewArgs& a, int col0, int row) {
+  if (!GATED) return a.w + (long)min(col0 + row, a.O - 1) * a.ldw;
+  const int t = row >> 4, q = row & 15;
+  const int col = min(col0 + t * 8 + (q >> 2) * 2 + (q & 1), a.O - 1);
+  return a.w + (long)((q & 2 ? a.O : 0) + col) * a.ldw;
+}
+
+// a tile's sums to memory (gated: act(gate) * up of two columns); parts: the unit
+template <bool GATED>
+__device__ __forceinline__ void finish_tile(const LinearFewArgs& a, int row, int col0, int lg,
+                                            const f32x4& v, const Ends<0>& e) {
+  if (!GATED) {
+    finish_columns<LF_PLAIN>(a, row, col0 + lg * 4, &v, e);
+    return;
+  }
+  const int col = col0 + lg * 2;
+  float o[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int at = min(col + j, a.O - 1);
+    float f = v[j], up = v[j + 2];
+    if (a.bias) f += (float)a.bias[at], up += (float)a.bias[a.O + at];
+    if (a.parts == LF_SILU) {
+      f = f / (1.0f + __expf(-f)) * up;
+    } else {
+      const float z = 0.7978845608028654f * (f + 0.044715f * f * f * f);
+      f = 0.5f * f * (1.0f + tanhf(z)) * up;
+    }
+    if (a.res) f += (float)a.res[(long)row * a.ldr + at];
+    o[j] = f;
+  }
+  __bf16* y = a.y + (long)row * a.ldy + col;
+  if (col + 1 < a.O && a.ldy % 2 == 0) {
+    *reinterpret_cast<bf16x2_t*>(y) = bf16x2_t{(__bf16)o[0], (__bf16)o[1]};
+  } else {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (col + j < a.O) y[j] = (__bf16)o[j];
+  }
+}
+
+// What a wave's rows of x become with the norm's weights, and their squares.
+__device__ __forceinline__ bf16x8_t times(bf16x8_t v, bf16x8_t g, float offset, float& sq) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float f = (float)v[j];
+    sq = fmaf(f, f, sq);
+    v[j] = (__bf16)(f * ((float)g[j] + offset));
+  }
+  return v;
+}
+
+// The sums of all shares of a tile of `steps` of the contraction, times the norm's factor.
+template <int TT, int SHARES, int TW, bool NORM>
+__device__ __forceinline__ f32x4 sum_of(const LinearFewArgs& a, const f32x4* red,
+                                        const float (*squares)[TW][WAVE], int tiles, int n,
+                                        int lane) {
+  const int i = n % TT;
+  f32x4 v{0, 0, 0, 0};
+#pragma unroll
+  for (int p = 0; p < SHARES; ++p) {
+    const f32x4 f = red[(p * tiles + n) * WAVE + lane];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] += f[j];
+  }
+  if (NORM) {
+    float s = 0.0f;
+#pragma unroll
+    for (int p = 0; p < SHARES; ++p) s += squares[i / TW * SHARES + p][i % TW][lane];
+    s += __shfl_xor(s, 16, WAVE);
+    s += __shfl_xor(s, 32, WAVE);
+    const float f = rsqrtf(s / a.K + a.eps);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] *= f;
+  }
+  return v;
+}
+
+// RT, TT: tiles of 16 rows of W and of x; SL: chunks of a wave under way.  The norm's weights
+// lie in LDS, all of them.
+template <int RT, int TT, int SL, bool GATED, bool NORM>
+__global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_own_kernel(const LinearFewArgs a) {
+  constexpr int LOADS = (RT + TT) * 2, CHUNK = LOADS * 1024;
+  constexpr int COLS = (GATED ? 8 : 16) * RT;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ float squares[NORM ? OWN_WAVES : 1][TT][WAVE];
+
+  arrive(a);
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int l16 = lane & 15, lg = lane >> 4;
+  // groups of x's rows: blocks eight apart
+  const int groups = (a.M + 16 * TT - 1) / (16 * TT);
+  int bx = blockIdx.x, x0 = 0;
+  if (groups > 1) {
+    const int pack = bx >> 3;
+    x0 = pack % groups * (16 * TT);
+    bx = pack / groups * 8 + (bx & 7);
+    if (bx * COLS >= a.O) return;
+  }
+  const int col0 = bx * COLS;
+
+  // A load is 8 rows of 128 bytes.  Pieces of a row are swapped by the row, so that those
+  // that a read meets lie in different banks.
+  const char* from[LOADS];
+  int col[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) col[i] = ((lane & 7) ^ ((i * 8 + (lane >> 3)) & 7)) * 8;
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = i * 8 + (lane >> 3);
+    from[i] = (const char*)(i < RT * 2
+                                ? row_of<GATED>(a, col0, row)
+                                : a.x + (long)min(x0 + row - RT * 16, a.M - 1) * a.ldx);
+  }
+  const int chunks = (a.K + 63) / 64;
+  const int first = first_of(a, a.share, chunks, bx);
+  const int mine = wid < chunks ? (chunks - 1 - wid) / OWN_WAVES + 1 : 0;
+  auto chunk = [&](int n) {
+    const int c = wid + n * OWN_WAVES + first;
+    return c >= chunks ? c - chunks : c;
+  };
+  const int ring = wid * SL * CHUNK;
+  const unsigned lds = lds_at(smem);
+  auto issue = [&](int n, int slot) {
+    const int k0 = chunk(n) * 64;
+    unsigned k[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) k[i] = (unsigned)min(k0 + col[i], a.K - 8) * 2;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      to_lds(from[i] + k[i & 1], lds + ring + slot * CHUNK + i * 1024);
+  };
+  constexpr int G = OWN_WAVES * SL * CHUNK;  // where the norm's weights lie
+  if (NORM) {
+    for (int i = wid; i * 512 < a.K; i += OWN_WAVES)
+      to_lds((const char*)(a.norm + min(i * 512 + lane * 8, a.K - 8)), lds + G + i * 1024);
+  }
+#pragma unroll
+  for (int s = 0; s < SL; ++s)
+    if (s < mine) issue(s, s);
+
+  f32x4 acc[RT][TT];
+  float sq[TT];
+#pragma unroll
+  for (int i = 0; i < TT; ++i) {
+    sq[i] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[r][i] = f32x4{0, 0, 0, 0};
+  }
+  if (NORM) {
+    wait_chunks<SL, LOADS>(mine);
+    asm volatile("s_barrier" ::: "memory");
+  }
+  constexpr int TILES = (RT * TT + OWN_WAVES - 1) / OWN_WAVES;  // of y, of a wave
+  Ends<0> ends[TILES];
+  if (!GATED && a.fours) {
+#pragma unroll
+    for (int q = 0; q < TILES; ++q) {
+      const int n = min(wid + q * OWN_WAVES, RT * TT - 1);
+      ends[q].read(a, x0 + n % TT * 16 + l16, col0 + n / TT * 16 + lg * 4);
+    }
+  }
+  int slot = 0;
+  for (int n = 0; n < mine; ++n) {
+    wait_chunks<SL - 1, LOADS>(mine - 1 - n);
+    const int k0 = chunk(n) * 64;
+    const char* at = smem + ring + slot * CHUNK + l16 * 128;
+    bf16x8_t w[RT][2], v[TT][2], g[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int piece = ((u * 4 + lg) ^ (l16 & 7)) * 16;
+#pragma unroll
+      for (int i = 0; i < TT; ++i)
+        v[i][u] = *reinterpret_cast<const bf16x8_t*>(at + (RT + i) * 2048 + piece);
+      if (NORM)
+        g[u] = *reinterpret_cast<const bf16x8_t*>(smem + G + (k0 + u * 32 + lg * 8) * 2);
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+        w[r][u] = *reinterpret_cast<const bf16x8_t*>(at + r * 2048 + piece);
+    }
+    // all read: the chunk's place is free
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (n + SL < mine) issue(n + SL, slot);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (u && k0 + 32 >= a.K) break;  // K is a multiple of 32
+#pragma unroll
+      for (int i = 0; i < TT; ++i) {
+        const bf16x8_t x = NORM ? times(v[i][u], g[u], a.offset, sq[i]) : v[i][u];
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+          acc[r][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[r][u], x, acc[r][i], 0, 0, 0);
+      }
+    }
+    if (++slot == SL) slot = 0;
+  }
+  __syncthreads();
+  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [waves][RT][TT][lanes]
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int i = 0; i < TT; ++i) red[((wid * RT + r) * TT + i) * WAVE + lane] = acc[r][i];
+  if (NORM) {
+#pragma unroll
+    for (int i = 0; i < TT; ++i) squares[wid][i][lane] = sq[i];
+  }
+  __syncthreads();
+
+  if (a.zero && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < a.n_zero; i += OWN_WAVES * WAVE) a.zero[i] = 0;
+#pragma unroll
+  for (int q = 0; q < TILES; ++q) {
+    const int n = wid + q * OWN_WAVES;
+    if (n >= RT * TT) break;
+    const f32x4 v = sum_of<TT, OWN_WAVES, TT, NORM>(a, red, squares, RT * TT, n, lane);
+    const int row = x0 + n % TT * 16 + l16;
+    if (row < a.M)
+      finish_tile<GATED>(a, row, col0 + n / TT * (GATED ? 8 : 16), lg, v, ends[q]);
+  }
+}
+
+// RT, TT as above (one group of x's rows); RW, RX: stages of 128 columns of W and of x in
+// LDS, a row of the norm's weights behind x's.
+template <int RT, int TT, int RW, int RX, bool GATED, bool NORM>
+__global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_ring_kernel(const LinearFewArgs a) {
+  constexpr int KS = 4, TW = TT * KS / OWN_WAVES;  // steps of a stage, tiles of x of a wave
+  constexpr int COLS = (GATED ? 8 : 16) * RT;
+  constexpr int SW = RT * 4096, SX = TT * 4096 + (NORM ? 1024 : 0), XS = RW * SW;
+  constexpr int MOST = RT > TT ? RT : TT;  // loads of a wave and stage: RT or TT
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ float squares[NORM ? OWN_WAVES : 1][TW][WAVE];
+
+  arrive(a);
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int step = wid % KS, tile0 = wid / KS * TW, part = wid & 3;
+  const int col0 = blockIdx.x * COLS;
+  const bool loads_w = wid < 4;
+
+  // a load is 4 rows of 256 bytes, pieces swapped by the row
+  const char* from[MOST];
+  int col[MOST];
+#pragma unroll
+  for (int i = 0; i < MOST; ++i) {
+    const int row = (i * 4 + part) * 4 + (lane >> 4);
+    col[i] = ((lane & 15) ^ (row & 15)) * 8;
+    from[i] = (const char*)(loads_w ? row_of<GATED>(a, col0, row)
+                                    : a.x + (long)min(row, a.M - 1) * a.ldx);
+  }
+  constexpr int W = KS * 32;  // columns of a stage
+  const int stages = (a.K + W - 1) / W;
+  const int first = first_of(a, a.share, stages, blockIdx.x);
+  auto column = [&](int t) {
+    const int c = t + first;
+    return (c >= stages ? c - stages : c) * W;
+  };
+  const unsigned lds = lds_at(smem);
+  auto issue_w = [&](int t, int slot) {
+    const int k0 = column(t);
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+      to_lds(from[i] + (unsigned)min(k0 + col[i], a.K - 8) * 2,
+             lds + slot * SW + (i * 4 + part) * 1024);
+  };
+  auto issue_x = [&](int t, int slot) {
+    const int k0 = column(t);
+#pragma unroll
+    for (int i = 0; i < TT; ++i)
+      to_lds(from[i] + (unsigned)min(k0 + col[i], a.K - 8) * 2,
+             lds + XS + slot * SX + (i * 4 + part) * 1024);
+    if (NORM)  // the same from each of the four waves
+      to_lds((const char*)(a.norm + min(k0 + (lane & 15) * 8, a.K - 8)),
+             lds + XS + slot * SX + TT * 4096);
+  };
+  f32x4 acc[RT][TW];
+  float sq[TW];
+#pragma unroll
+  for (int i = 0; i < TW; ++i) {
+    sq[i] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[r][i] = f32x4{0, 0, 0, 0};
+  }
+  const int piece = l16 * 256 + ((step * 4 + lg) ^ l16) * 16;
+  if (loads_w) {
+#pragma unroll
+    for (int t = 0; t < RW - 1; ++t)
+      if (t < stages) issue_w(t, t);
+  } else {
+#pragma unroll
+    for (int t = 0; t < RX - 1; ++t)
+      if (t < stages) issue_x(t, t);
+  }
+  constexpr int TILES = (RT * TT + OWN_WAVES - 1) / OWN_WAVES;  // of y, of a wave
+  Ends<0> ends[TILES];
+  if (!GATED && a.fours) {
+#pragma unroll
+    for (int q = 0; q < TILES; ++q) {
+      const int n = min(wid + q * OWN_WAVES, RT * TT - 1);
+      ends[q].read(a, n % TT * 16 + l16, col0 + n / TT * 16 + lg * 4);
+    }
+  }
+  int sw = 0, sx = 0;
+  for (int t = 0; t < stages; ++t) {
+    if (loads_w) wait_chunks<RW - 2, RT>(stages - 1 - t);
+    else wait_chunks<RX - 2, TT + (NORM ? 1 : 0)>(stages - 1 - t);
+    asm volatile("s_barrier" ::: "memory");
+    // into the place of the stage before, which all have read
+    if (loads_w) {
+      if (t + RW - 1 < stages) issue_w(t + RW - 1, sw ? sw - 1 : RW - 1);
+    } else if (t + RX - 1 < stages) {
+      issue_x(t + RX - 1, sx ? sx - 1 : RX - 1);
+    }
+    if (column(t) + step * 32 < a.K) {
+      const char* wb = smem + sw * SW + piece;
+      const char* xb = smem + XS + sx * SX + piece;
+      bf16x8_t w[RT], v[TW], g;
+#pragma unroll
+      for (int i = 0; i < TW; ++i)
+        v[i] = *reinterpret_cast<const bf16x8_t*>(xb + (tile0 + i) * 4096);
+      if (NORM)
+        g = *reinterpret_cast<const bf16x8_t*>(smem + XS + sx * SX + TT * 4096 +
+                                               (step * 4 + lg) * 16);
+#pragma unroll
+      for (int r = 0; r < RT; ++r) w[r] = *reinterpret_cast<const bf16x8_t*>(wb + r * 4096);
+#pragma unroll
+      for (int i = 0; i < TW; ++i) {
+        const bf16x8_t x = NORM ? times(v[i], g, a.offset, sq[i]) : v[i];
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+          acc[r][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[r], x, acc[r][i], 0, 0, 0);
+      }
+    }
+    if (++sw == RW) sw = 0;
+    if (++sx == RX) sx = 0;
+  }
+  __syncthreads();
+  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [steps][RT][TT][lanes]
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+      red[((step * RT + r) * TT + tile0 + i) * WAVE + lane] = acc[r][i];
+  if (NORM) {
+#pragma unroll
+    for (int i = 0; i < TW; ++i) squares[wid][i][lane] = sq[i];
+  }
+  __syncthreads();
+
+  if (a.zero && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < a.n_zero; i += OWN_WAVES * WAVE) a.zero[i] = 0;
+#pragma unroll
+  for (int q = 0; q < TILES; ++q) {
+    const int n = wid + q * OWN_WAVES;
+    if (n >= RT * TT) break;
+    const f32x4 v = sum_of<TT, KS, TW, NORM>(a, red, squares, RT * TT, n, lane);
+    const int row = n % TT * 16 + l16;
+    if (row < a.M)
+      finish_tile<GATED>(a, row, col0 + n / TT * (GATED ? 8 : 16), lg, v, ends[q]);
+  }
+}
+
+// columns: of a chunk or stage
+void turned(LinearFewArgs& a, int act, int columns) {
+  a.parts = (unsigned char)act;
+  a.share = (a.K + columns - 1) / columns;
+  a.turn = a.share > 1 && in_step(a.ldw)
+               ? (unsigned)(((1ull << 32) + a.share - 1) / a.share) : 0;
+}
+
+template <typename Kernel>
+void launch(Kernel kernel, const LinearFewArgs& a, int blocks, int smem, hipStream_t stream) {
+  if (smem > 48 * 1024)  // with the sums of squares above the default limit
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  kernel<<<blocks, OWN_WAVES * WAVE, smem, stream>>>(a);
+}
+
+template <int RT, int TT>
+void own(LinearFewArgs a, int act, hipStream_t stream) {
+  const int cols = (act ? 8 : 16) * RT, groups = (a.M + 16 * TT - 1) / (16 * TT);
+  int blocks = (a.O + cols - 1) / cols;
+  if (groups > 1) blocks = (blocks + 7) / 8 * 8 * groups;
+  turned(a, act, 64);
+  // two chunks of a wave where there is room; a norm's instructions cover for one (64 rows
+  // of 2048 into 3648: 8.8 us with one, 9.5 with two)
+  constexpr int room = RT + TT <= 4 ? 2 : 1;
+  auto go = [&](auto kernel, int slots) {
+    const int ring = OWN_WAVES * slots * (RT + TT) * 2048 + (a.norm ? (a.K + 511) / 512 * 1024 : 0);
+    const int sums = OWN_WAVES * RT * TT * 1024;
+    launch(kernel, a, blocks, ring > sums ? ring : sums, stream);
+  };
+  if (a.norm) {
+    if (act) go(&linear_own_kernel<RT, TT, 1, true, true>, 1);
+    else go(&linear_own_kernel<RT, TT, 1, false, true>, 1);
+  } else {
+    if (act) go(&linear_own_kernel<RT, TT, room, true, false>, room);
+    else go(&linear_own_kernel<RT, TT, room, false, false>, room);
+  }
+}
+
+template <int RT, int TT>
+void ring(LinearFewArgs a, int act, hipStream_t stream) {
+  constexpr int RW = TT == 2 ? (RT >= 7 ? 4 : 5) : (RT >= 7 ? 3 : 4), RX = TT == 2 && RT < 8 ? 4 : 3;
+  const int cols = (act ? 8 : 16) * RT, blocks = (a.O + cols - 1) / cols;
+  turned(a, act, 128);
+  auto go = [&](auto kernel) {
+    const int rings = RW * RT * 4096 + RX * (TT * 4096 + (a.norm ? 1024 : 0));
+    const int sums = RT * TT * 4096;
+    launch(kernel, a, blocks, rings > sums ? rings : sums, stream);
+  };
+  if (a.norm) {
+    if (act) go(&linear_ring_kernel<RT, TT, RW, RX, true, true>);
+    else go(&linear_ring_kernel<RT, TT, RW, RX, false, true>);
+  } else {
+    if (act) go(&linear_ring_kernel<RT, TT, RW, RX, true, false>);
+    else go(&linear_ring_kernel<RT, TT, RW, RX, false, false>);
+  }
+}
+
+// Tiles of W's rows and of x's.  What the busiest CU reads decides: its blocks, one after the
+// other, times what a block reads; where two read as much, fewer rows of x a block.  Over 600
+// random sizes (17 to 64 rows, with and without norm and unit) the kernels so chosen take .81
+// of linear_some_kernel's time and .4% more than the fastest of 14 (us, there and here; 64 of
+// x: units of 14336 of 4096 with norm, seven tiles 60.2, 44.2; of 10944 of 2048, six 31.0,
+// 22.3; 6144 of 4096 with norm, three of 32 rows of x 21.5, 17.0; 3648 of 2048 with norm, two
+// of 32 11.4, 8.8; 2048 of 2048, one of 32 6.6, 5.6; 32 of x, one of 16 5.4, 4.8).
+// linear_some_kernel keeps what it does as well or better: four tiles for all rows of x
+// without a norm (16176 rows of 2048 16.3, 17.3; units of 7408 of 1024 10.1, 11.3), and norms
+// of more weights than LDS has room for beside the rings.
+struct OwnTiles {
+  int rt, tt;  // rt 0: linear_some_kernel's
+};
+OwnTiles own_tiles(int M, int O, int K, int act, bool norm) {
+  if (M <= 16 || (norm && K > 8192)) return {0, 0};
+  const int tiles = (O + (act ? 7 : 15)) / (act ? 8 : 16);
+  OwnTiles best{0, 0};
+  int least = 0;
+  auto offer = [&](int rt, int tt) {
+    const int blocks = (tiles + rt - 1) / rt * ((M + 16 * tt - 1) / (16 * tt));
+    const int reads = (blocks + 255) / 256 * (rt + tt);
+    if (!best.rt || reads < least || (reads == least && tt < best.tt))
+      best = {rt, tt}, least = reads;
+  };
+  const int whole = M <= 32 ? 2 : 4;
+  for (int rt = 1; rt <= 8; ++rt) {
+    offer(rt, whole);
+    if (rt <= 4) offer(rt, whole / 2);
+  }
+  if (!norm && best.rt == 4 && best.tt == whole) return {0, 0};
+  return best;
+}
+
+}  // namespace
+
+bool linear_own_go(LinearFewArgs a, int act, hipStream_t stream) {
+  const OwnTiles t = own_tiles(a.M, a.O, a.K, act, a.norm != nullptr);
+  switch (t.rt * 8 + t.tt) {
+    case 1 * 8 + 1: own<1, 1>(a, act, stream); return true;
+    case 2 * 8 + 1: own<2, 1>(a, act, stream); return true;
+    case 3 * 8 + 1: own<3, 1>(a, act, stream); return true;
+    case 1 * 8 + 2: own<1, 2>(a, act, stream); return true;
+    case 2 * 8 + 2: own<2, 2>(a, act, stream); return true;
+    case 3 * 8 + 2: own<3, 2>(a, act, stream); return true;
+    case 4 * 8 + 2: own<4, 2>(a, act, stream); return true;
+    case 3 * 8 + 4: own<3, 4>(a, act, stream); return true;
+    case 4 * 8 + 4: own<4, 4>(a, act, stream); return true;
+    case 5 * 8 + 2: ring<5, 2>(a, act, stream); return true;
+    case 6 * 8 + 2: ring<6, 2>(a, act, stream); return true;
+    case 7 * 8 + 2: ring<7, 2>(a, act, stream); return true;
+    case 5 * 8 + 4: ring<5, 4>(a, act, stream); return true;
+    case 6 * 8 + 4: ring<6, 4>(a, act, stream); return true;
+    case 7 * 8 + 4: ring<7, 4>(a, act, stream); return true;
+    case 8 * 8 + 2: ring<8, 2>(a, act, stream); return true;
+    case 8 * 8 + 4: ring<8, 4>(a, act, stream); return true;
+  }
+  return false;
+}

@@ -23,7 +23,8 @@ NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 # extension -> its sources; MLXS_AMD_EXT=name[,name] builds only those
 # (bin/trace_run builds just what its model loads)
-SHARED = ("elementwise.hip", "linear_few.hip", "linear_tiles.hip")  # part of both
+SHARED = ("elementwise.hip", "linear_few.hip", "linear_own.hip",
+          "linear_tiles.hip")  # part of both
 SOURCES = {
     "_hip_ragged": lambda name: name.startswith("ragged_") or name in SHARED,
     "_hip_ops": lambda name: not name.startswith("ragged_"),

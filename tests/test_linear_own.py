@@ -1,0 +1,67 @@
+"""Products of 17 to 64 rows: every number of tiles, ragged ends of each size."""
+
+import types
+
+import pytest
+import torch
+
+from mlx_sharding_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def check(M, K, O, act, norm, bias, residual):
+    g = torch.Generator("cuda").manual_seed(O + M + K)
+
+    def rand(*n):
+        return torch.randn(*n, generator=g, device="cuda").bfloat16()
+
+    rows = 2 * O if act else O
+    x, w = rand(M, K), rand(rows, K) / K ** 0.5
+    n = types.SimpleNamespace(weight=rand(K), eps=1e-5, weight_offset=0.5) if norm else None
+    b = rand(rows) if bias else None
+    res = rand(M, O) if residual else None
+    h = x.double()
+    if norm:
+        h = (h * (h.square().mean(-1, keepdim=True) + 1e-5).rsqrt()
+             * (n.weight.double() + 0.5))
+    z = h @ w.double().T
+    # 32-bit sums, and rows rounded to bf16 behind the norm
+    off = (h.abs() @ w.double().abs().T) * (K * 2.0 ** -24 + (2.0 ** -8 if norm else 0.0))
+    if bias:
+        z = z + b.double()
+        off = off + z.abs() * 2.0 ** -23
+    if act:  # either unit grows by at most 1.13 of its argument
+        gate, up, og, ou = *z.chunk(2, -1), *off.chunk(2, -1)
+        unit = (torch.nn.functional.silu(gate) if act == "silu" else
+                torch.nn.functional.gelu(gate, approximate="tanh"))
+        z, off = unit * up, 1.13 * og * (up.abs() + ou) + unit.abs() * ou + 1e-6
+    if residual:
+        z = z + res.double()
+    got = ops._linear_few(x, w, b, res, n, act)
+    assert got is not None
+    # the result is rounded to bf16
+    assert ((got.double() - z).abs() <= off + z.abs() * 2.0 ** -8 + 1e-6).all()
+
+
+# tiles of 16 rows of W (8 columns of a unit) at both ends of the ranges that have one to eight
+# tiles a block
+@pytest.mark.parametrize("act", [None, "silu"])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("M,K", [(17, 160), (32, 64), (33, 96), (64, 1056)])
+@pytest.mark.parametrize("tiles", [1, 128, 129, 256, 257, 384, 385, 512, 513, 768, 769, 1024,
+                                   1025, 1280, 1281, 1536, 1537, 1792, 1793, 2048,
+                                   2049])
+def test_tiles(M, K, tiles, norm, act):
+    check(M, K, tiles * (8 if act else 16) - 4, act, norm, not norm, norm == bool(act))
+
+
+# sums of three columns at the end, odd ones, one; contractions of one step and of parts of a
+# chunk, a stage and a round of the waves
+@pytest.mark.parametrize("act", [None, "silu", "gelu_tanh"])
+@pytest.mark.parametrize("M", [18, 31, 47, 63])
+@pytest.mark.parametrize("O,K", [(1, 32), (13, 992), (2049, 32), (4110, 544), (9001, 96),
+                                 (15001, 224), (300, 8192)])
+def test_ends(M, O, K, act):
+    check(M, K, O, act, True, False, False)
+    check(M, K, O, act, False, True, True)
