@@ -124,6 +124,18 @@ def feed(into, out, x: torch.Tensor, act: str, norm: Optional[nn.Module] = None,
     return project(out, project(into, x, norm=norm, act=act), residual=residual)
 
 
+def attend(qkv, out, x: torch.Tensor, norm: nn.Module, cos, sin, cache, heads: int,
+           scale: float, softcap: float = 0.0, window: int = 0,
+           residual: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """ops.attend_few with the weights of a FusedColumns and a Linear, or None."""
+    w_qkv, w_o = (m.weight if m.quant is None else dense_weight(m, n)
+                  for m, n in ((qkv, x.shape[-1]), (out, heads * cache.k_head_dim)))
+    if w_qkv is None or w_o is None:
+        return None
+    return ops.attend_few(x, w_qkv, qkv.bias, norm, cos, sin, cache, w_o, out.bias, residual,
+                          heads, scale, softcap, window)
+
+
 def project(m, x: torch.Tensor, *, norm: Optional[nn.Module] = None,
             act: Optional[str] = None,
             residual: Optional[torch.Tensor] = None,

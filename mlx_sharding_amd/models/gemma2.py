@@ -18,7 +18,7 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import (Linear, RMSNorm, StageModel, as_built, feed, head,
+from .base import (Linear, RMSNorm, StageModel, as_built, attend, feed, head,
                    owned_layer_indices, project, read_in_place)
 from .llama import _Inner
 
@@ -49,6 +49,11 @@ class Gemma2Attention(nn.Module):
         B, T, _ = x.shape
         if norm is not None and self._fused_qkv is None:
             x, norm = norm(x), None
+        if T > 1 and norm is not None and type(cache) is KVCache and as_built(self.o_proj):
+            out = attend(self._fused_qkv, self.o_proj, x, norm, cos, sin, cache, self.n_heads,
+                         self.scale, self.softcap, self.sliding_window)
+            if out is not None:
+                return out
         if norm is not None:
             q, k, v = project(self._fused_qkv, x, norm=norm).split(
                 self._fused_qkv.splits, -1)

@@ -16,7 +16,7 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import (Linear, RMSNorm, StageModel, as_built, feed, head,
+from .base import (Linear, RMSNorm, StageModel, as_built, attend, feed, head,
                    owned_layer_indices, project, read_in_place)
 
 
@@ -54,6 +54,11 @@ class LlamaAttention(nn.Module):
         """norm: for x's rows first; residual: added to what is returned.  For
         few tokens, where both go with the projections."""
         B, T, _ = x.shape
+        if T > 1 and norm is not None and self._fused_qkv is not None and type(cache) is KVCache:
+            out = attend(self._fused_qkv, self.o_proj, x, norm, cos, sin, cache, self.n_heads,
+                         self.scale, residual=residual)
+            if out is not None:
+                return out
         if self._fused_qkv is not None and norm is not None:
             q, k, v = project(self._fused_qkv, x, norm=norm).split(
                 self._fused_qkv.splits, -1)

@@ -340,6 +340,25 @@ def feed_few(x, w_in, w_out, act, norm=None, residual=None):
                             norm.weight_offset, _ACTS[act])
 
 
+def attend_few(x, w_qkv, b_qkv, norm, cos, sin, cache, w_o, b_o, residual, heads, scale,
+               softcap, window):
+    """Attention of few tokens, projections included (LlamaAttention), with a KVCache, in
+    one call: projections of x's rows as ``norm`` makes them, rotations, append, attention
+    and the output's projection, plus ``residual``.  None, and nothing appended, where one
+    of these does not run so."""
+    ext = _few_for(x, w_qkv, w_o) if x.is_cuda else None
+    if ext is None or ext is not _EXT or cache.graph_pos is not None:
+        return None
+    B, T, _ = x.shape
+    _, at = cache.claim(B, T)
+    out = ext.attend_few_try(x, w_qkv, b_qkv, norm.weight, norm.eps, norm.weight_offset,
+                             cos, sin, cache.keys_buffer(), cache.values_buffer(), at, w_o,
+                             b_o, residual, heads, scale, softcap, window)
+    if out is not None:
+        cache.wrote(T)
+    return out
+
+
 def project(x, weight, bias=None, *, norm=None, act=None, residual=None, clear=None):
     """x W^T + bias, of x's rows as ``norm`` (an RMSNorm) makes them; ``act``:
     the gated unit act(gate) * up of the result's halves; plus ``residual``;

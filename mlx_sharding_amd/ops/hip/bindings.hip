@@ -1416,10 +1416,63 @@ std::vector<torch::Tensor> moe_gate_subranges(torch::Tensor logits, int64_t K,
 
 }  // namespace
 
+// A layer's attention of few tokens that are no single ones, in one call: the products of
+// x's rows, as the norm makes them, with w_qkv (queries, keys, values of all heads), their
+// rotations, keys and values to the caches from place `at` on, attention, and w_o's product,
+// plus the residual.  Nothing, and nothing written, where one of these does not run here.
+// (Launched one by one from Python, six kernels of a layer took the host 70 us, these four
+// and a feed-forward 38.)
+c10::optional<torch::Tensor> attend_few_try(
+    torch::Tensor x, torch::Tensor w_qkv, c10::optional<torch::Tensor> b_qkv,
+    torch::Tensor norm, double eps, double offset, torch::Tensor cos, torch::Tensor sin,
+    torch::Tensor kcache, torch::Tensor vcache, int64_t at, torch::Tensor w_o,
+    c10::optional<torch::Tensor> b_o, c10::optional<torch::Tensor> residual, int64_t heads,
+    double scale, double softcap, int64_t window) {
+  if (x.dim() != 3 || kcache.dim() != 4 || !linear_few_takes(x, w_qkv) ||
+      !linear_few_weight(w_o, x))
+    return {};
+  const long B = x.size(0), T = x.size(1), M = B * T, Hkv = kcache.size(1),
+             cap = kcache.size(2), D = kcache.size(3), wide = (heads + 2 * Hkv) * D;
+  if (heads < 1 || Hkv < 1 || heads % Hkv || D < 32 || D % 32 || D > 256 ||
+      !attn_prefill_supported((int)D, (int)D) || w_qkv.size(0) != wide ||
+      w_o.size(1) != heads * D || !linear_few_sizes(M, w_o.size(0), heads * D) ||
+      !linear_few_along(x, wide, wide, b_qkv, {}, norm) ||
+      !linear_few_along(x, w_o.size(0), w_o.size(0), b_o, residual, {}) || at < 0 ||
+      at + T > cap)
+    return {};
+  for (const auto& t : {kcache, vcache})
+    if (t.device() != x.device() || t.scalar_type() != torch::kBFloat16 || t.dim() != 4 ||
+        t.size(0) != B || t.size(1) != Hkv || t.size(2) != cap || t.size(3) != D ||
+        !t.is_contiguous() || !linear_few_whole(t) || !linear_few_plain(t))
+      return {};
+  for (const auto& t : {cos, sin})
+    if (t.device() != x.device() || t.scalar_type() != torch::kFloat32 ||
+        !t.is_contiguous() || t.numel() != T * D / 2 || !linear_few_plain(t))
+      return {};
+  c10::OptionalDeviceGuard guard;  // and the device's current stream
+  if (x.get_device() != c10::hip::current_device()) guard.reset_device(x.device());
+  const auto y = linear_few_run(linear_few_rows(x), w_qkv, b_qkv, {}, norm, eps, offset, 0,
+                                {}, {});
+  const auto q = torch::empty({M, heads * D}, x.options());
+  const char* of = (const char*)y.data_ptr();
+  launch_rope_qkv(of, of + heads * D * 2, of + (heads + Hkv) * D * 2, cos.data_ptr<float>(),
+                  sin.data_ptr<float>(), q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(),
+                  nullptr, at, M, (int)T, (int)heads, (int)Hkv, (int)D, cap, wide, wide, wide,
+                  cur_stream());
+  const auto o = torch::empty({M, heads * D}, x.options());
+  launch_attn_prefill(q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), o.data_ptr(), (int)B,
+                      (int)heads, (int)Hkv, (int)T, (int)(at + T), T * heads * D, D, heads * D,
+                      cap, cap, (int)D, (int)D, (float)scale, (float)softcap, (int)window,
+                      (int)at, cur_stream());
+  if (residual.has_value()) residual = residual->reshape({M, -1});
+  return linear_few_shaped(linear_few_run(o, w_o, b_o, residual, {}, 0.0, 0.0, 0, {}, {}), x);
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "fused RMSNorm (gfx950)");
   m.def("norm_add", &norm_add);
   m.def("attn_step", &attn_step);
+  m.def("attend_few_try", &attend_few_try);
   m.def("step_begin", &step_begin);
   m.def("step_end", &step_end);
   m.def("rope_qkv", &rope_qkv, py::arg("q"), py::arg("k"), py::arg("v"),
