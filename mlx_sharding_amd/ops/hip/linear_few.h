@@ -75,7 +75,8 @@ static torch::Tensor linear_few_run(const torch::Tensor& x, const torch::Tensor&
   };
   const void* b = vec(bias, w.size(0));
   const void* n = vec(norm, K);
-  TORCH_CHECK(!n || whole(*norm), "norm weights begin at a multiple of 16 bytes");
+  TORCH_CHECK(!n || (whole(*norm) && K <= 32768),
+              "norm weights begin at a multiple of 16 bytes, up to 32768 of them");
   const void* r = nullptr;
   long ldr = 0;
   if (residual.has_value()) {
@@ -177,8 +178,10 @@ static bool linear_few_along(const torch::Tensor& x, long O, long biases,
   auto vec = [&](const c10::optional<torch::Tensor>& t, long n) {
     return !t.has_value() || (here(*t) && t->is_contiguous() && t->numel() == n);
   };
+  // (weights of a norm have to find room in LDS)
   if (!vec(bias, biases) || !vec(norm, x.size(-1)) ||
-      (norm.has_value() && reinterpret_cast<uintptr_t>(norm->data_ptr()) % 16))
+      (norm.has_value() &&
+       (reinterpret_cast<uintptr_t>(norm->data_ptr()) % 16 || x.size(-1) > 32768)))
     return false;
   if (!residual.has_value()) return true;
   return here(*residual) && residual->dim() == x.dim() && residual->size(-1) == O &&

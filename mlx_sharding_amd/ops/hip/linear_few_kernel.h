@@ -12,9 +12,9 @@ struct LinearFewArgs {
   const __bf16 *x, *w, *bias, *res, *norm;
   __bf16* y;
   short M;
-  // parts > 1: blocks share a tile's contraction, `share` steps (few) or stages
-  // (some) each.  part [tiles of y, parts, tiles of x, WAVE, 4], count: one number per
-  // tile of y and x, zero before.
+  // parts > 1: blocks share a tile's contraction, `share` stages each.  part [tiles of y,
+  // parts, tiles of x, WAVE, 4], count: one number per tile of y and x, zero before.
+  // (linear_own.hip: the unit, and the chunks or stages of the whole contraction)
   unsigned char parts;
   unsigned char fours;     // bias and residual are read by fours
   int O, K;                // O: columns of y
@@ -160,6 +160,8 @@ static bool in_step(long ld) {
   return false;
 }
 
-// Products of 17 to 64 rows on the kernels of linear_own.hip, or false where they are
+// Products of whole contractions on the kernels of linear_own.hip, or false where they are
 // linear_few.hip's.
 bool linear_own_go(LinearFewArgs a, int act, hipStream_t stream);
+// A contraction that `split` blocks share, for up to 16 rows of x.
+void linear_own_shared(LinearFewArgs a, int split, hipStream_t stream);

@@ -1,4 +1,4 @@
-// y = x W^T for 17 to 64 rows of x, whole contractions (what goes along: linear_few.hip).
+// y = x W^T for up to 64 rows of x, whole contractions (what goes along: linear_few.hip).
 //
 // A CU reads rows through LDS at 100 bytes a nanosecond and more as long as a load takes
 // whole lines (128 bytes of 8 rows; 64 bytes of 16 rows, as operands straight to registers
@@ -9,19 +9,20 @@
 //
 //   linear_own_kernel   each wave has a ring of its own in LDS and takes chunks of 64 columns
 //                       by turns, so that no wave waits for another before the sums; for up
-//                       to four tiles of W's rows
+//                       to four tiles of W's rows, and eight where rows of x are few
 //   linear_ring_kernel  five to eight tiles, which is more than such rings have room for:
 //                       waves meet, half of them load W, half x, in rings of lengths that
 //                       suit each
 //
-// Both take any number of tiles, so that blocks are one round of the chip where few_tiles'
-// two and four leave a second one half empty, and rows of x may be split between blocks
-// that lie eight apart, on one XCD, whose L2 then has W's rows for both.
+// Both take any number of tiles, so that blocks are one round of the chip where two and four
+// would leave a second one half empty, and rows of x may be split between blocks that lie
+// eight apart, on one XCD, whose L2 then has W's rows for both.
 #include "linear_few_kernel.h"
 
 namespace {
 
 constexpr int OWN_WAVES = 8;
+constexpr int OWN_LDS = 150 * 1024;  // that rings may take, beside squares
 
 template <int N>
 __device__ __forceinline__ void wait_loads() {
@@ -132,8 +133,8 @@ __device__ __forceinline__ f32x4 sum_of(const LinearFewArgs& a, const f32x4* red
 }
 
 // RT, TT: tiles of 16 rows of W and of x; SL: chunks of a wave under way.  The norm's weights
-// lie in LDS, all of them.
-template <int RT, int TT, int SL, bool GATED, bool NORM>
+// lie in LDS, all of them.  SHARED: blocks have a share of a contraction each.
+template <int RT, int TT, int SL, bool GATED, bool NORM, bool SHARED>
 __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_own_kernel(const LinearFewArgs a) {
   constexpr int LOADS = (RT + TT) * 2, CHUNK = LOADS * 1024;
   constexpr int COLS = (GATED ? 8 : 16) * RT;
@@ -168,12 +169,13 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_own_kernel(const Line
                                 ? row_of<GATED>(a, col0, row)
                                 : a.x + (long)min(x0 + row - RT * 16, a.M - 1) * a.ldx);
   }
-  const int chunks = (a.K + 63) / 64;
+  const int c0 = SHARED ? blockIdx.y * a.share : 0;
+  const int all = (a.K + 63) / 64 - c0, chunks = SHARED ? min(a.share, all) : all;
   const int first = first_of(a, a.share, chunks, bx);
   const int mine = wid < chunks ? (chunks - 1 - wid) / OWN_WAVES + 1 : 0;
   auto chunk = [&](int n) {
     const int c = wid + n * OWN_WAVES + first;
-    return c >= chunks ? c - chunks : c;
+    return c0 + (c >= chunks ? c - chunks : c);
   };
   const int ring = wid * SL * CHUNK;
   const unsigned lds = lds_at(smem);
@@ -268,7 +270,8 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_own_kernel(const Line
   for (int q = 0; q < TILES; ++q) {
     const int n = wid + q * OWN_WAVES;
     if (n >= RT * TT) break;
-    const f32x4 v = sum_of<TT, OWN_WAVES, TT, NORM>(a, red, squares, RT * TT, n, lane);
+    f32x4 v = sum_of<TT, OWN_WAVES, TT, NORM>(a, red, squares, RT * TT, n, lane);
+    if (SHARED && !sums_of_all(a, (long)bx * RT * TT + n, lane, v)) continue;
     const int row = x0 + n % TT * 16 + l16;
     if (row < a.M)
       finish_tile<GATED>(a, row, col0 + n / TT * (GATED ? 8 : 16), lg, v, ends[q]);
@@ -432,26 +435,38 @@ void launch(Kernel kernel, const LinearFewArgs& a, int blocks, int smem, hipStre
   kernel<<<blocks, OWN_WAVES * WAVE, smem, stream>>>(a);
 }
 
+// LDS of a block; slots: chunks of a wave
+int own_room(int rt, int tt, int slots, int K, bool norm) {
+  const int ring = OWN_WAVES * slots * (rt + tt) * 2048 + (norm ? (K + 511) / 512 * 1024 : 0);
+  const int sums = OWN_WAVES * rt * tt * 1024;
+  return ring > sums ? ring : sums;
+}
+
 template <int RT, int TT>
 void own(LinearFewArgs a, int act, hipStream_t stream) {
   const int cols = (act ? 8 : 16) * RT, groups = (a.M + 16 * TT - 1) / (16 * TT);
   int blocks = (a.O + cols - 1) / cols;
   if (groups > 1) blocks = (blocks + 7) / 8 * 8 * groups;
   turned(a, act, 64);
-  // two chunks of a wave where there is room; a norm's instructions cover for one (64 rows
-  // of 2048 into 3648: 8.8 us with one, 9.5 with two)
-  constexpr int room = RT + TT <= 4 ? 2 : 1;
+  // Two chunks of a wave where blocks are small; a norm's instructions cover for one (64 rows
+  // of 2048 into 3648: 8.8 us with one, 9.5 with two) but in long rows of few (1 to 16 rows
+  // of 2048 to 4096 .98, of more than 6144 .90).
+  constexpr int most = RT == 1 || (RT == 2 && TT == 2) ? 2 : 1;
   auto go = [&](auto kernel, int slots) {
-    const int ring = OWN_WAVES * slots * (RT + TT) * 2048 + (a.norm ? (a.K + 511) / 512 * 1024 : 0);
-    const int sums = OWN_WAVES * RT * TT * 1024;
-    launch(kernel, a, blocks, ring > sums ? ring : sums, stream);
+    launch(kernel, a, blocks, own_room(RT, TT, slots, a.K, a.norm != nullptr), stream);
   };
   if (a.norm) {
-    if (act) go(&linear_own_kernel<RT, TT, 1, true, true>, 1);
-    else go(&linear_own_kernel<RT, TT, 1, false, true>, 1);
+    if constexpr (RT == 1 && TT == 1) {
+      if (a.K >= 2048 && own_room(RT, TT, most, a.K, true) <= OWN_LDS) {
+        if (act) return go(&linear_own_kernel<RT, TT, most, true, true, false>, most);
+        return go(&linear_own_kernel<RT, TT, most, false, true, false>, most);
+      }
+    }
+    if (act) go(&linear_own_kernel<RT, TT, 1, true, true, false>, 1);
+    else go(&linear_own_kernel<RT, TT, 1, false, true, false>, 1);
   } else {
-    if (act) go(&linear_own_kernel<RT, TT, room, true, false>, room);
-    else go(&linear_own_kernel<RT, TT, room, false, false>, room);
+    if (act) go(&linear_own_kernel<RT, TT, most, true, false, false>, most);
+    else go(&linear_own_kernel<RT, TT, most, false, false, false>, most);
   }
 }
 
@@ -475,39 +490,59 @@ void ring(LinearFewArgs a, int act, hipStream_t stream) {
 }
 
 // Tiles of W's rows and of x's.  What the busiest CU reads decides: its blocks, one after the
-// other, times what a block reads; where two read as much, fewer rows of x a block.  Over 600
-// random sizes (17 to 64 rows, with and without norm and unit) the kernels so chosen take .81
-// of linear_some_kernel's time and .4% more than the fastest of 14 (us, there and here; 64 of
-// x: units of 14336 of 4096 with norm, seven tiles 60.2, 44.2; of 10944 of 2048, six 31.0,
-// 22.3; 6144 of 4096 with norm, three of 32 rows of x 21.5, 17.0; 3648 of 2048 with norm, two
-// of 32 11.4, 8.8; 2048 of 2048, one of 32 6.6, 5.6; 32 of x, one of 16 5.4, 4.8).
-// linear_some_kernel keeps what it does as well or better: four tiles for all rows of x
-// without a norm (16176 rows of 2048 16.3, 17.3; units of 7408 of 1024 10.1, 11.3), and norms
-// of more weights than LDS has room for beside the rings.
+// other, times what a block reads, up to 16 rows of x as half a tile, as most of their loads
+// find lines in L1, and where more than four tiles leave a CU one block, half a tile more.
+// Where two read as much, fewer rows of x or tiles a block.  Over 650 random sizes of 17 to 64
+// rows, with and without norm and unit, the kernels so chosen take .81 of the time of stages
+// that waves meet at and .4% more than the fastest of 14 (us; 64 of x: units of 14336 of 4096
+// with norm, seven tiles 60.2, 44.2; of 10944 of 2048, six 31.0, 22.3; 6144 of 4096 with norm,
+// three of 32 rows of x 21.5, 17.0; 3648 of 2048 with norm, two of 32 11.4, 8.8; 2048 of 2048,
+// one of 32 6.6, 5.6; 32 of x, one of 16 5.4, 4.8).  Over 350 of 1 to 16 rows they take .85 of
+// the time of operands straight to registers and 1% more than the fastest (one of x: units of
+// 14336 of 4096 with norm 43.3, 40.2, 6144 of 4096 13.2, 11.5, 2048 of 2048 4.7, 4.0; 5 of x,
+// 3584 of 14336 22.6, 20.2; 12 of x, 12352 of 2048 12.3, 11.4; 16 of x, 4096 of 2048 7.3, 6.1).
+// linear_some_kernel keeps what it does as well or better: four tiles for 17 and more rows of x
+// in one block, without a norm (16176 rows of 2048 16.3, 17.3; units of 7408 of 1024 10.1,
+// 11.3).
 struct OwnTiles {
   int rt, tt;  // rt 0: linear_some_kernel's
 };
 OwnTiles own_tiles(int M, int O, int K, int act, bool norm) {
-  if (M <= 16 || (norm && K > 8192)) return {0, 0};
   const int tiles = (O + (act ? 7 : 15)) / (act ? 8 : 16);
   OwnTiles best{0, 0};
-  int least = 0;
+  long least = 0;
   auto offer = [&](int rt, int tt) {
-    const int blocks = (tiles + rt - 1) / rt * ((M + 16 * tt - 1) / (16 * tt));
-    const int reads = (blocks + 255) / 256 * (rt + tt);
+    if ((rt <= 4 || tt == 1) && own_room(rt, tt, 1, K, norm) > OWN_LDS) return;
+    const long blocks = (long)(tiles + rt - 1) / rt * ((M + 16 * tt - 1) / (16 * tt));
+    const int halves = M > 16 ? 2 * (rt + tt) : 2 * rt + 1 + (rt > 4);
+    const long reads = (blocks + 255) / 256 * halves;
     if (!best.rt || reads < least || (reads == least && tt < best.tt))
       best = {rt, tt}, least = reads;
   };
-  const int whole = M <= 32 ? 2 : 4;
+  const int whole = M <= 16 ? 1 : M <= 32 ? 2 : 4;
   for (int rt = 1; rt <= 8; ++rt) {
     offer(rt, whole);
-    if (rt <= 4) offer(rt, whole / 2);
+    if (rt <= 4 && whole > 1) offer(rt, whole / 2);
   }
-  if (!norm && best.rt == 4 && best.tt == whole) return {0, 0};
+  if (!norm && best.rt == 4 && best.tt == whole && whole > 1) return {0, 0};
   return best;
 }
 
 }  // namespace
+
+// Blocks of a tile of up to 16 rows of x share its contraction.
+void linear_own_shared(LinearFewArgs a, int split, hipStream_t stream) {
+  turned(a, LF_PLAIN, 64);
+  const int chunks = a.share;
+  a.share = (chunks + split - 1) / split;
+  a.parts = (unsigned char)((chunks + a.share - 1) / a.share);
+  if (a.turn) a.turn = a.share > 1 ? (unsigned)(((1ull << 32) + a.share - 1) / a.share) : 0;
+  const int smem = own_room(1, 1, 2, a.K, false);
+  const auto kernel = &linear_own_kernel<1, 1, 2, false, false, true>;
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  kernel<<<dim3((unsigned)((a.O + 15) / 16), a.parts), OWN_WAVES * WAVE, smem, stream>>>(a);
+}
 
 bool linear_own_go(LinearFewArgs a, int act, hipStream_t stream) {
   const OwnTiles t = own_tiles(a.M, a.O, a.K, act, a.norm != nullptr);
@@ -515,6 +550,11 @@ bool linear_own_go(LinearFewArgs a, int act, hipStream_t stream) {
     case 1 * 8 + 1: own<1, 1>(a, act, stream); return true;
     case 2 * 8 + 1: own<2, 1>(a, act, stream); return true;
     case 3 * 8 + 1: own<3, 1>(a, act, stream); return true;
+    case 4 * 8 + 1: own<4, 1>(a, act, stream); return true;
+    case 5 * 8 + 1: own<5, 1>(a, act, stream); return true;
+    case 6 * 8 + 1: own<6, 1>(a, act, stream); return true;
+    case 7 * 8 + 1: own<7, 1>(a, act, stream); return true;
+    case 8 * 8 + 1: own<8, 1>(a, act, stream); return true;
     case 1 * 8 + 2: own<1, 2>(a, act, stream); return true;
     case 2 * 8 + 2: own<2, 2>(a, act, stream); return true;
     case 3 * 8 + 2: own<3, 2>(a, act, stream); return true;

@@ -1,4 +1,4 @@
-"""Products of 17 to 64 rows: every number of tiles, ragged ends of each size."""
+"""Products of up to 64 rows: every number of tiles, ragged ends of each size."""
 
 import types
 
@@ -48,7 +48,7 @@ def check(M, K, O, act, norm, bias, residual):
 # tiles a block
 @pytest.mark.parametrize("act", [None, "silu"])
 @pytest.mark.parametrize("norm", [False, True])
-@pytest.mark.parametrize("M,K", [(17, 160), (32, 64), (33, 96), (64, 1056)])
+@pytest.mark.parametrize("M,K", [(1, 96), (16, 1120), (17, 160), (32, 64), (33, 96), (64, 1056)])
 @pytest.mark.parametrize("tiles", [1, 128, 129, 256, 257, 384, 385, 512, 513, 768, 769, 1024,
                                    1025, 1280, 1281, 1536, 1537, 1792, 1793, 2048,
                                    2049])
@@ -59,9 +59,29 @@ def test_tiles(M, K, tiles, norm, act):
 # sums of three columns at the end, odd ones, one; contractions of one step and of parts of a
 # chunk, a stage and a round of the waves
 @pytest.mark.parametrize("act", [None, "silu", "gelu_tanh"])
-@pytest.mark.parametrize("M", [18, 31, 47, 63])
+@pytest.mark.parametrize("M", [2, 15, 18, 31, 47, 63])
 @pytest.mark.parametrize("O,K", [(1, 32), (13, 992), (2049, 32), (4110, 544), (9001, 96),
                                  (15001, 224), (300, 8192)])
 def test_ends(M, O, K, act):
     check(M, K, O, act, True, False, False)
     check(M, K, O, act, False, True, True)
+
+
+# contractions that two and four blocks share, from the shortest on, with ends of tiles, chunks
+# and shares
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("I,O", [(5632, 2048), (5664, 1040), (5696, 1024), (6176, 3), (16384, 900)])
+def test_shared(M, I, O):
+    g = torch.Generator("cuda").manual_seed(I + O)
+
+    def rand(*n):
+        return torch.randn(*n, generator=g, device="cuda").bfloat16()
+
+    x, w_in, w_out = rand(M, 64), rand(2 * I, 64) / 8, rand(O, I) / I ** 0.5
+    res = rand(M, O)
+    for _ in range(3):  # numbers are cleared each time
+        got = ops.feed_few(x, w_in, w_out, "silu", None, res)
+        units = ops._linear_few(x, w_in, None, None, None, "silu")
+        want = units.double() @ w_out.double().T + res.double()
+        off = (units.double().abs() @ w_out.double().abs().T) * (I * 2.0 ** -24)
+        assert ((got.double() - want).abs() <= off + want.abs() * 2.0 ** -8 + 1e-6).all()
