@@ -315,8 +315,8 @@ def _few_for(x, *weights):
 
 
 def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None, clear=None):
-    """project on linear_few.hip (of more rows a product or a unit on linear_tiles.hip),
-    or None where that does not take it."""
+    """project on linear_few.hip and linear_own.hip (of more rows a product or a unit on
+    linear_own.hip or linear_tiles.hip), or None where they do not take it."""
     ext = _few_for(x, weight)
     if ext is None:
         return None
@@ -391,8 +391,8 @@ def few_tokens(x: torch.Tensor) -> bool:
 
 
 def linear(x, weight, bias=None):
-    """Dense linear; up to 64 rows run on linear_few.hip where it takes them, more on
-    linear_tiles.hip where that is faster than the library.  The MFMA
+    """Dense linear; up to 64 rows run on linear_few.hip and linear_own.hip where they take
+    them, more on linear_own.hip or linear_tiles.hip where that is faster than the library.  The MFMA
     decode GEMV (MLXS_AMD_DENSE_GEMV=1) was a NEGATIVE result at batch-64 decode shapes:
     hipBLASLt's small-GEMM kernels run ~13 us in-graph and the split-K fp32-atomic
     traffic (M*O*4*nk bytes) rivals the weight bytes on small-O projections

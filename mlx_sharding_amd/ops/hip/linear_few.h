@@ -1,5 +1,5 @@
-// y = x W^T for up to 64 rows, with what goes with it (linear_few.hip), and for more
-// where linear_tiles.hip is the better one; part of both extensions.
+// y = x W^T for up to 64 rows, with what goes with it (linear_few.hip, linear_own.hip), and
+// for more where linear_own.hip or linear_tiles.hip is the better one; part of both extensions.
 #pragma once
 
 #include <torch/extension.h>
@@ -19,6 +19,7 @@ extern "C" void launch_linear_few(const void*, const void*, const void*,
                                   long, long, long, long, float, float, int,
                                   unsigned*, float*, unsigned*, int, hipStream_t);
 extern "C" long linear_few_room(int, int, int, int*);
+extern "C" int linear_own_many(long, long, long, int);
 
 // Room for a product whose contraction blocks share; whatever runs before it clears the
 // numbers.
@@ -61,8 +62,10 @@ static torch::Tensor linear_few_run(const torch::Tensor& x, const torch::Tensor&
   TORCH_CHECK(act >= 0 && act <= 2, "unknown unit");
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "shapes");
   const int M = x.size(0), K = x.size(1), O = w.size(0) / (act ? 2 : 1);
-  TORCH_CHECK(M >= 1 && M <= 64 && K >= 32 && K % 32 == 0 && O >= 1,
-              "1 to 64 rows of a multiple of 32");
+  TORCH_CHECK(M >= 1 && K >= 32 && K % 32 == 0 && O >= 1 &&
+                  (M <= 64 || (!norm && !residual && !room.n && !clear.n &&
+                               linear_own_many(M, O, K, (int)act))),
+              "1 to 64 rows of a multiple of 32, or more that there is a kernel for");
   TORCH_CHECK(!act || w.size(0) % 2 == 0, "a gated unit has two halves");
   for (const auto& t : {x, w})
     TORCH_CHECK(t.stride(1) == 1 && t.stride(0) % 8 == 0 && whole(t),
@@ -251,11 +254,16 @@ static c10::optional<torch::Tensor> linear_many_try(const torch::Tensor& x,
     return {};
   const long K = w.size(1), M = x.numel() / K, O = w.size(0) / (act ? 2 : 1);
   if (M <= 64 || M >= 1L << 24) return {};
-  const auto [tile, shares] = linear_tiles_planned(M, O, K, act, bias.has_value());
-  if (!tile || !linear_few_input(x) || !linear_few_weight(w, x) || linear_few_other(K) ||
-      w.stride(0) < K || w.stride(0) >= 1L << 22 ||
-      !linear_few_along(x, w.size(0), w.size(0), bias, {}, {}))
+  const bool own = linear_own_many(M, O, K, (int)act);
+  const auto [tile, shares] = own ? std::pair<int64_t, int64_t>{0, 1}
+                                  : linear_tiles_planned(M, O, K, act, bias.has_value());
+  if ((!own && !tile) || !linear_few_input(x) || !linear_few_weight(w, x) ||
+      linear_few_other(K) || !linear_few_along(x, w.size(0), w.size(0), bias, {}, {}))
     return {};
+  if (own)
+    return linear_few_shaped(
+        linear_few_run(linear_few_rows(x), w, bias, {}, {}, 0.0, 0.0, act, {}, {}), x);
+  if (w.stride(0) < K || w.stride(0) >= 1L << 22) return {};
   const auto rows = linear_few_rows(x);
   if (rows.stride(0) < K || rows.stride(0) >= 1L << 22) return {};
   return linear_few_shaped(linear_tiles(rows, w, bias, act, tile, shares), x);

@@ -61,6 +61,18 @@ __device__ __forceinline__ const __bf16* row_of(const LinearFewArgs& a, int col0
   return a.w + (long)((q & 2 ? a.O : 0) + col) * a.ldw;
 }
 
+// A block's place among those of W's rows, and its first row of x, of which it has `rows`:
+// blocks of the same rows of W are eight apart.
+struct BlockPlace {
+  int bx, x0;
+};
+__device__ __forceinline__ BlockPlace place_of(const LinearFewArgs& a, int rows) {
+  const int groups = (a.M + rows - 1) / rows;
+  if (groups == 1) return {(int)blockIdx.x, 0};
+  const int pack = blockIdx.x >> 3;
+  return {pack / groups * 8 + (int)(blockIdx.x & 7), pack % groups * rows};
+}
+
 // a tile's sums to memory (gated: act(gate) * up of two columns); parts: the unit
 template <bool GATED>
 __device__ __forceinline__ void finish_tile(const LinearFewArgs& a, int row, int col0, int lg,
@@ -145,16 +157,9 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_own_kernel(const Line
   const int lane = threadIdx.x & (WAVE - 1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l16 = lane & 15, lg = lane >> 4;
-  // groups of x's rows: blocks eight apart
-  const int groups = (a.M + 16 * TT - 1) / (16 * TT);
-  int bx = blockIdx.x, x0 = 0;
-  if (groups > 1) {
-    const int pack = bx >> 3;
-    x0 = pack % groups * (16 * TT);
-    bx = pack / groups * 8 + (bx & 7);
-    if (bx * COLS >= a.O) return;
-  }
-  const int col0 = bx * COLS;
+  const BlockPlace place = place_of(a, 16 * TT);
+  const int bx = place.bx, x0 = place.x0, col0 = bx * COLS;
+  if (col0 >= a.O) return;
 
   // A load is 8 rows of 128 bytes.  Pieces of a row are swapped by the row, so that those
   // that a read meets lie in different banks.
@@ -294,7 +299,9 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_ring_kernel(const Lin
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l16 = lane & 15, lg = lane >> 4;
   const int step = wid % KS, tile0 = wid / KS * TW, part = wid & 3;
-  const int col0 = blockIdx.x * COLS;
+  const BlockPlace at = place_of(a, 16 * TT);
+  const int x0 = at.x0, col0 = at.bx * COLS;
+  if (col0 >= a.O) return;
   const bool loads_w = wid < 4;
 
   // a load is 4 rows of 256 bytes, pieces swapped by the row
@@ -305,11 +312,11 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_ring_kernel(const Lin
     const int row = (i * 4 + part) * 4 + (lane >> 4);
     col[i] = ((lane & 15) ^ (row & 15)) * 8;
     from[i] = (const char*)(loads_w ? row_of<GATED>(a, col0, row)
-                                    : a.x + (long)min(row, a.M - 1) * a.ldx);
+                                    : a.x + (long)min(x0 + row, a.M - 1) * a.ldx);
   }
   constexpr int W = KS * 32;  // columns of a stage
   const int stages = (a.K + W - 1) / W;
-  const int first = first_of(a, a.share, stages, blockIdx.x);
+  const int first = first_of(a, a.share, stages, at.bx);
   auto column = [&](int t) {
     const int c = t + first;
     return (c >= stages ? c - stages : c) * W;
@@ -356,7 +363,7 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_ring_kernel(const Lin
 #pragma unroll
     for (int q = 0; q < TILES; ++q) {
       const int n = min(wid + q * OWN_WAVES, RT * TT - 1);
-      ends[q].read(a, n % TT * 16 + l16, col0 + n / TT * 16 + lg * 4);
+      ends[q].read(a, x0 + n % TT * 16 + l16, col0 + n / TT * 16 + lg * 4);
     }
   }
   int sw = 0, sx = 0;
@@ -413,7 +420,7 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_ring_kernel(const Lin
     const int n = wid + q * OWN_WAVES;
     if (n >= RT * TT) break;
     const f32x4 v = sum_of<TT, KS, TW, NORM>(a, red, squares, RT * TT, n, lane);
-    const int row = n % TT * 16 + l16;
+    const int row = x0 + n % TT * 16 + l16;
     if (row < a.M)
       finish_tile<GATED>(a, row, col0 + n / TT * (GATED ? 8 : 16), lg, v, ends[q]);
   }
@@ -473,7 +480,9 @@ void own(LinearFewArgs a, int act, hipStream_t stream) {
 template <int RT, int TT>
 void ring(LinearFewArgs a, int act, hipStream_t stream) {
   constexpr int RW = TT == 2 ? (RT >= 7 ? 4 : 5) : (RT >= 7 ? 3 : 4), RX = TT == 2 && RT < 8 ? 4 : 3;
-  const int cols = (act ? 8 : 16) * RT, blocks = (a.O + cols - 1) / cols;
+  const int cols = (act ? 8 : 16) * RT, groups = (a.M + 16 * TT - 1) / (16 * TT);
+  int blocks = (a.O + cols - 1) / cols;
+  if (groups > 1) blocks = (blocks + 7) / 8 * 8 * groups;
   turned(a, act, 128);
   auto go = [&](auto kernel) {
     const int rings = RW * RT * 4096 + RX * (TT * 4096 + (a.norm ? 1024 : 0));
@@ -528,7 +537,34 @@ OwnTiles own_tiles(int M, int O, int K, int act, bool norm) {
   return best;
 }
 
+// The same for 65 and more rows of x, where one round of blocks has them all: few tiles of 32
+// rows or more of 64, whichever read less, and rt 0 where the kernels of more rows are the better
+// ones.  Those wait for whole tiles of 128 rows of x and more, often on a part of the CUs; but
+// what a block reads here grows with its tiles and the groups that read W, and from six tiles,
+// from 384 rows or above contractions of 8192 they catch up (178 rows of 8192 into 7792, six
+// tiles, 82.2 us here, 52.2; 299 of 14336 into 1984 50.8, 38.3).  Over 233 random sizes that are
+// taken the time is .71 of theirs (us, before and now: 211 rows of 512 into 512 6.3, 3.0; 90 of
+// 2048 into 1024 8.4, 4.6; 70 of 4096 into 3584 14.1, 10.3; 193 of 2048 into 4544 19.8, 13.1;
+// units of 4096 of 74 of 5120 32.7, 28.9).  Contractions below 512 are not measured, and stay.
+OwnTiles own_tiles_many(int M, int O, int K, int act) {
+  const int tiles = (O + (act ? 7 : 15)) / (act ? 8 : 16);
+  OwnTiles best{0, 0};
+  if (M > 384 || K < 512 || K > 8192) return best;
+  for (const int tt : {2, 4}) {
+    const int groups = (M + 16 * tt - 1) / (16 * tt), most = tt == 2 ? 3 : M <= 128 ? 8 : 5;
+    const int rt = (tiles + 256 / groups - 1) / (256 / groups);
+    if (rt <= most && (!best.rt || rt + tt < best.rt + best.tt)) best = {rt, tt};
+  }
+  return best;
+}
+
 }  // namespace
+
+// Whether the product of more than 64 rows, on its own, is one of these.
+extern "C" int linear_own_many(long M, long O, long K, int act) {
+  return M > 64 && M <= 384 && O >= 1 && O < 1 << 17 && K <= 8192 && K % 32 == 0 &&
+         own_tiles_many((int)M, (int)O, (int)K, act).rt > 0;
+}
 
 // Blocks of a tile of up to 16 rows of x share its contraction.
 void linear_own_shared(LinearFewArgs a, int split, hipStream_t stream) {
@@ -545,7 +581,8 @@ void linear_own_shared(LinearFewArgs a, int split, hipStream_t stream) {
 }
 
 bool linear_own_go(LinearFewArgs a, int act, hipStream_t stream) {
-  const OwnTiles t = own_tiles(a.M, a.O, a.K, act, a.norm != nullptr);
+  const OwnTiles t = a.M > 64 ? own_tiles_many(a.M, a.O, a.K, act)
+                              : own_tiles(a.M, a.O, a.K, act, a.norm != nullptr);
   switch (t.rt * 8 + t.tt) {
     case 1 * 8 + 1: own<1, 1>(a, act, stream); return true;
     case 2 * 8 + 1: own<2, 1>(a, act, stream); return true;
@@ -559,6 +596,8 @@ bool linear_own_go(LinearFewArgs a, int act, hipStream_t stream) {
     case 2 * 8 + 2: own<2, 2>(a, act, stream); return true;
     case 3 * 8 + 2: own<3, 2>(a, act, stream); return true;
     case 4 * 8 + 2: own<4, 2>(a, act, stream); return true;
+    case 1 * 8 + 4: own<1, 4>(a, act, stream); return true;
+    case 2 * 8 + 4: own<2, 4>(a, act, stream); return true;
     case 3 * 8 + 4: own<3, 4>(a, act, stream); return true;
     case 4 * 8 + 4: own<4, 4>(a, act, stream); return true;
     case 5 * 8 + 2: ring<5, 2>(a, act, stream); return true;

@@ -1,4 +1,4 @@
-"""Products of up to 64 rows: every number of tiles, ragged ends of each size."""
+"""Products of few rows: every number of tiles, ragged ends of each size."""
 
 import types
 
@@ -65,6 +65,21 @@ def test_tiles(M, K, tiles, norm, act):
 def test_ends(M, O, K, act):
     check(M, K, O, act, True, False, False)
     check(M, K, O, act, False, True, True)
+
+
+# 65 and more rows: groups of 32 and 64, with as many tiles as fit a round of 256 blocks, and one
+# more; the longest contraction, and the shortest
+@pytest.mark.parametrize("act", [None, "silu", "gelu_tanh"])
+@pytest.mark.parametrize("M,K", [(65, 512), (96, 1056), (97, 544), (128, 8192), (129, 608), (192, 992),
+                                 (384, 576)])
+@pytest.mark.parametrize("of,rt", [(32, 1), (32, 2), (32, 3), (64, 1), (64, 2), (64, 3), (64, 4),
+                                   (64, 5), (64, 6), (64, 8)])
+def test_more_rows(M, K, of, rt, act):
+    if rt > 5 and M > 128:
+        return
+    tiles = rt * (256 // (-(-M // of)))
+    for t in (tiles - rt + 1, tiles):
+        check(M, K, t * (8 if act else 16) - 3, act, False, rt % 2 == 0, False)
 
 
 # contractions that two and four blocks share, from the shortest on, with ends of tiles, chunks
