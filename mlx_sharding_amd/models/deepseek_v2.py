@@ -483,31 +483,38 @@ class DeepseekV2MoE(nn.Module):
                                        m.down_proj.weight, self.top_k,
                                        *self._packing()))
 
-    def _beside(self, y):
+    def _beside(self, y, fits):
         """The shared experts' matrices, where they go with the routed ones."""
         m = self.shared_experts
-        if (m is None or y.shape[0] > ops.SHARED_TOKENS
-                or not as_built(m) or not as_built(*m.read())
+        if (m is None or not as_built(m) or not as_built(*m.read())
                 or m._fused_gu is None or m._fused_gu.bias is not None
                 or m.down_proj.bias is not None or not ops.few_tokens(y)):
             return None
         both = (dense_weight(m._fused_gu, y.shape[1]),
                 dense_weight(m.down_proj, m.down_proj.in_features))
-        return both if ops.expert_shared_ok(*y.shape, *both) else None
+        return both if fits(*y.shape, *both) else None
 
     def decode(self, x, residual, norm, tickets=None):
         """The residual x (+ residual) after this feed-forward of it, normed:
         three kernels for the routed and the shared experts, with norm, router and
         choice in a fourth.  tickets: a zero (int32) per token."""
         shape, H = x.shape, x.shape[-1]
-        y, h, choice, weight = ops.expert_route(
-            x.reshape(-1, H), None if residual is None else residual.reshape(-1, H),
+        flat = x.reshape(-1, H)
+        around = None
+        if tickets is not None and residual is None:
+            around = self._beside(flat, ops.expert_begin_ok)
+        y, h, choice, weight, *units = ops.expert_route(
+            flat, None if residual is None else residual.reshape(-1, H),
             norm, self.gate.weight, self.top_k, self.routed_scaling_factor,
-            self.norm_topk_prob, tickets)
+            self.norm_topk_prob, tickets, around and around[0])
         m = self.switch_mlp
         stacks = [[p.weight] if m.quant is None else [p.weight, p.scales, p.biases]
                   for p in (m.gate_proj, m.up_proj, m.down_proj)]
-        packed, beside = self._packing(), self._beside(y)
+        packed = self._packing()
+        if around is not None:
+            rows = ops.expert_rows(y, choice, weight, *stacks, *packed)
+            return ops.expert_finish(*units, around[1], rows, h).view(shape)
+        beside = self._beside(y, ops.expert_shared_ok)
         if beside is not None:
             rows, shared = ops.expert_rows(y, choice, weight, *stacks, *packed, beside)
         else:

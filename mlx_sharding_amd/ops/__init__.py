@@ -717,13 +717,14 @@ def expert_rows_ok(x, gate_w, up, down, top: int, bits: int, group_size: int
 
 
 def expert_route(x, residual, norm, gate_w, top: int, scaling: float,
-                 normalize: bool, tickets=None):
+                 normalize: bool, tickets=None, w_in=None):
     """(rows of x + residual as ``norm`` makes them, x + residual, experts and
     weights of every token), one kernel; rows [N, H].  tickets: N zeros (int32), with
-    which a token has several blocks; they are used up."""
+    which a token has several blocks; they are used up.  w_in [2 S, H] of a shared
+    feed-forward (expert_begin_ok): its units [N, S], too, in the same kernel."""
     return _require_ext("moe_route").moe_route(
         _whole(x), None if residual is None else _whole(residual), norm.weight,
-        norm.eps, norm.weight_offset, gate_w, top, scaling, normalize, tickets)
+        norm.eps, norm.weight_offset, gate_w, top, scaling, normalize, tickets, w_in)
 
 
 def _whole(t: torch.Tensor) -> torch.Tensor:
@@ -755,6 +756,22 @@ def expert_shared_ok(n_tokens: int, H: int, w_in, w_out) -> bool:
             and tuple(w_in.shape) == (2 * w_out.shape[-1], H) and w_out.shape[0] == H
             and all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous()
                     and t.data_ptr() % 16 == 0 for t in (w_in, w_out)))
+
+
+def expert_begin_ok(n_tokens: int, H: int, w_in, w_out) -> bool:
+    """Whether expert_route and expert_finish take halves of a shared feed-forward of
+    these matrices along."""
+    return (n_tokens <= 64 and H <= 4096 and w_in is not None and w_out is not None
+            and not os.environ.get("MLXS_AMD_DENSE_GEMV")  # names another kernel
+            and w_out.shape[-1] % 64 == 0 and w_out.shape[-1] <= 8192
+            and tuple(w_in.shape) == (2 * w_out.shape[-1], H) and w_out.shape[0] == H
+            and all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in (w_in, w_out)))
+
+
+def expert_finish(units, w_out, rows, h):
+    """h + a token's rows + units w_out^T, bf16 [N, H], one kernel."""
+    return _require_ext("moe_finish").moe_finish(units, w_out, rows, h)
 
 
 def _expert_stack(m, bits: int, group_size: int) -> torch.Tensor:

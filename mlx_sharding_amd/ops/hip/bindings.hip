@@ -1141,13 +1141,16 @@ static void check_rows(const torch::Tensor& t, const char* name, long n, long w)
 }
 
 // x [N, H] (+ residual) -> normed rows, x + residual (or x), experts and weights
-// of every token [N, top].  tickets [N]: zeros that the blocks of a token count with
+// of every token [N, top].  tickets [N]: zeros that the blocks of a token count with.
+// w_in [2 S, H]: a shared feed-forward, whose units [N, S] of the normed rows come behind
+// (with tickets, without a residual, up to 64 rows of 4096)
 std::vector<torch::Tensor> moe_route(torch::Tensor x,
                                      c10::optional<torch::Tensor> residual,
                                      torch::Tensor norm, double eps,
                                      double offset, torch::Tensor gate,
                                      int64_t top, double scaling, bool normalize,
-                                     c10::optional<torch::Tensor> tickets) {
+                                     c10::optional<torch::Tensor> tickets,
+                                     c10::optional<torch::Tensor> w_in) {
   TORCH_CHECK(x.dim() == 2 && gate.dim() == 2 && norm.dim() == 1, "shapes");
   const long N = x.size(0), H = x.size(1), E = gate.size(0);
   TORCH_CHECK(N >= 1 && H % 128 == 0 && H <= 8192,
@@ -1177,8 +1180,18 @@ std::vector<torch::Tensor> moe_route(torch::Tensor x,
       (float)offset, (float)scaling, normalize,
       tickets.has_value() ? logits.data_ptr<float>() : nullptr,
       tickets.has_value() ? reinterpret_cast<unsigned*>(tickets->data_ptr<int>()) : nullptr};
-  launch_moe_route(&a, (int)N, cur_stream());
-  return {y, h, choice, weight};
+  if (!w_in.has_value()) {
+    launch_moe_route(&a, (int)N, cur_stream());
+    return {y, h, choice, weight};
+  }
+  TORCH_CHECK(tickets.has_value() && !residual.has_value() && N <= 64 && H <= 4096,
+              "rows that a shared feed-forward goes with");
+  const long S = w_in->size(0) / 2;
+  TORCH_CHECK(S >= 1 && S < 1L << 24, "units");
+  check_rows(*w_in, "w_in", 2 * S, H);
+  auto units = torch::empty({N, S}, x.options());
+  launch_moe_begin(&a, (int)N, w_in->data_ptr(), units.data_ptr(), (int)S, cur_stream());
+  return {y, h, choice, weight, units};
 }
 
 // Packed words [E, O, K * bits / 32] with scales and offsets [E, O, K / gs] in the
@@ -1296,6 +1309,26 @@ std::vector<torch::Tensor> moe_rows(torch::Tensor x, torch::Tensor choice,
   }
   launch_moe_rows(&b, (int)bits, (int)gs, false, cur_stream());
   return {y, ys};
+}
+
+// units [N, S] w_out [H, S]^T, a token's pairs [N * top, H] and the rows h, added up in 32 bits
+torch::Tensor moe_finish(torch::Tensor units, torch::Tensor w_out, torch::Tensor rows,
+                         torch::Tensor h) {
+  TORCH_CHECK(units.dim() == 2 && w_out.dim() == 2 && rows.dim() == 2, "shapes");
+  const long N = units.size(0), S = units.size(1), H = w_out.size(0);
+  TORCH_CHECK(N >= 1 && N <= 64 && S >= 32 && S % 32 == 0 && S <= 65536 && H >= 16 &&
+                  H % 16 == 0 && H < 1L << 24, "sizes of the shared feed-forward");
+  check_rows(units, "units", N, S);
+  check_rows(w_out, "w_out", H, S);
+  check_rows(h, "h", N, H);
+  TORCH_CHECK(rows.is_cuda() && rows.device() == units.device() &&
+                  rows.scalar_type() == torch::kFloat32 && rows.is_contiguous() &&
+                  rows.size(1) == H && rows.size(0) >= N && rows.size(0) % N == 0, "rows");
+  auto out = torch::empty({N, H}, units.options());
+  launch_moe_finish(units.data_ptr(), w_out.data_ptr(), rows.data_ptr<float>(), h.data_ptr(),
+                    out.data_ptr(), (int)N, (int)H, (int)S, (int)(rows.size(0) / N),
+                    cur_stream());
+  return out;
 }
 
 // A token's pairs, and the rows h and shared where given, added up in 32 bits
@@ -1515,11 +1548,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   });
   m.def("moe_route", &moe_route, py::arg("x"), py::arg("residual"), py::arg("norm"),
         py::arg("eps"), py::arg("offset"), py::arg("gate"), py::arg("top"),
-        py::arg("scaling"), py::arg("normalize"), py::arg("tickets") = py::none());
+        py::arg("scaling"), py::arg("normalize"), py::arg("tickets") = py::none(),
+        py::arg("w_in") = py::none());
   m.def("moe_pack", &moe_pack);
   m.def("moe_rows", &moe_rows);
   m.def("moe_rows_longest", [](int64_t bits) { return moe_rows_longest((int)bits); });
   m.def("moe_combine", &moe_combine);
+  m.def("moe_finish", &moe_finish);
   m.def("moe_tiles", &moe_tiles);
   m.def("linear_tiles", &linear_tiles);
   m.def("linear_tiles_plan", &linear_tiles_planned);

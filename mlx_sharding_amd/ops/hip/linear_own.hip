@@ -17,270 +17,13 @@
 // Both take any number of tiles, so that blocks are one round of the chip where two and four
 // would leave a second one half empty, and rows of x may be split between blocks that lie
 // eight apart, on one XCD, whose L2 then has W's rows for both.
-#include "linear_few_kernel.h"
+#include "linear_own_kernel.h"
 
 namespace {
 
-constexpr int OWN_WAVES = 8;
-constexpr int OWN_LDS = 150 * 1024;  // that rings may take, beside squares
-
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// Waits until at most the loads of the `younger` last chunks, PER each, are under way; J: of
-// how many that may be at most.
-template <int J, int PER>
-__device__ __forceinline__ void wait_chunks(int younger) {
-  if constexpr (J == 0) {
-    wait_loads<0>();
-  } else {
-    if (younger >= J) wait_loads<J * PER>();
-    else wait_chunks<J - 1, PER>(younger);
-  }
-}
-
-// 16 bytes a lane from memory to LDS (at + 16 * lane).  The compiler does not know of the
-// load, which would have it wait for all before reads of LDS; no register is written.
-__device__ __forceinline__ void to_lds(const char* from, unsigned at) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(from)
-               : "memory", "m0");
-}
-__device__ __forceinline__ unsigned lds_at(const char* smem) {
-  return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) char*)smem;
-}
-
-// The row of W of row `row` of a block's tiles.  A tile of a gated unit has eight columns:
-// rows 4g and 4g + 1 are the gate's of columns 2g and 2g + 1, the two others the up
-// projection's, so that a lane has both sums of a column.
-template <bool GATED>
-__device__ __forceinline__ const __bf16* row_of(const LinearFewArgs& a, int col0, int row) {
-  if (!GATED) return a.w + (long)min(col0 + row, a.O - 1) * a.ldw;
-  const int t = row >> 4, q = row & 15;
-  const int col = min(col0 + t * 8 + (q >> 2) * 2 + (q & 1), a.O - 1);
-  return a.w + (long)((q & 2 ? a.O : 0) + col) * a.ldw;
-}
-
-// A block's place among those of W's rows, and its first row of x, of which it has `rows`:
-// blocks of the same rows of W are eight apart.
-struct BlockPlace {
-  int bx, x0;
-};
-__device__ __forceinline__ BlockPlace place_of(const LinearFewArgs& a, int rows) {
-  const int groups = (a.M + rows - 1) / rows;
-  if (groups == 1) return {(int)blockIdx.x, 0};
-  const int pack = blockIdx.x >> 3;
-  return {pack / groups * 8 + (int)(blockIdx.x & 7), pack % groups * rows};
-}
-
-// a tile's sums to memory (gated: act(gate) * up of two columns); parts: the unit
-template <bool GATED>
-__device__ __forceinline__ void finish_tile(const LinearFewArgs& a, int row, int col0, int lg,
-                                            const f32x4& v, const Ends<0>& e) {
-  if (!GATED) {
-    finish_columns<LF_PLAIN>(a, row, col0 + lg * 4, &v, e);
-    return;
-  }
-  const int col = col0 + lg * 2;
-  float o[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int at = min(col + j, a.O - 1);
-    float f = v[j], up = v[j + 2];
-    if (a.bias) f += (float)a.bias[at], up += (float)a.bias[a.O + at];
-    if (a.parts == LF_SILU) {
-      f = f / (1.0f + __expf(-f)) * up;
-    } else {
-      const float z = 0.7978845608028654f * (f + 0.044715f * f * f * f);
-      f = 0.5f * f * (1.0f + tanhf(z)) * up;
-    }
-    if (a.res) f += (float)a.res[(long)row * a.ldr + at];
-    o[j] = f;
-  }
-  __bf16* y = a.y + (long)row * a.ldy + col;
-  if (col + 1 < a.O && a.ldy % 2 == 0) {
-    *reinterpret_cast<bf16x2_t*>(y) = bf16x2_t{(__bf16)o[0], (__bf16)o[1]};
-  } else {
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      if (col + j < a.O) y[j] = (__bf16)o[j];
-  }
-}
-
-// What a wave's rows of x become with the norm's weights, and their squares.
-__device__ __forceinline__ bf16x8_t times(bf16x8_t v, bf16x8_t g, float offset, float& sq) {
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const float f = (float)v[j];
-    sq = fmaf(f, f, sq);
-    v[j] = (__bf16)(f * ((float)g[j] + offset));
-  }
-  return v;
-}
-
-// The sums of all shares of a tile of `steps` of the contraction, times the norm's factor.
-template <int TT, int SHARES, int TW, bool NORM>
-__device__ __forceinline__ f32x4 sum_of(const LinearFewArgs& a, const f32x4* red,
-                                        const float (*squares)[TW][WAVE], int tiles, int n,
-                                        int lane) {
-  const int i = n % TT;
-  f32x4 v{0, 0, 0, 0};
-#pragma unroll
-  for (int p = 0; p < SHARES; ++p) {
-    const f32x4 f = red[(p * tiles + n) * WAVE + lane];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] += f[j];
-  }
-  if (NORM) {
-    float s = 0.0f;
-#pragma unroll
-    for (int p = 0; p < SHARES; ++p) s += squares[i / TW * SHARES + p][i % TW][lane];
-    s += __shfl_xor(s, 16, WAVE);
-    s += __shfl_xor(s, 32, WAVE);
-    const float f = rsqrtf(s / a.K + a.eps);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] *= f;
-  }
-  return v;
-}
-
-// RT, TT: tiles of 16 rows of W and of x; SL: chunks of a wave under way.  The norm's weights
-// lie in LDS, all of them.  SHARED: blocks have a share of a contraction each.
-template <int RT, int TT, int SL, bool GATED, bool NORM, bool SHARED>
+template <int RT, int TT, int SL, bool GATED, bool NORM, bool SHARED, bool PAIRS = false>
 __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_own_kernel(const LinearFewArgs a) {
-  constexpr int LOADS = (RT + TT) * 2, CHUNK = LOADS * 1024;
-  constexpr int COLS = (GATED ? 8 : 16) * RT;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  __shared__ float squares[NORM ? OWN_WAVES : 1][TT][WAVE];
-
-  arrive(a);
-  const int lane = threadIdx.x & (WAVE - 1);
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int l16 = lane & 15, lg = lane >> 4;
-  const BlockPlace place = place_of(a, 16 * TT);
-  const int bx = place.bx, x0 = place.x0, col0 = bx * COLS;
-  if (col0 >= a.O) return;
-
-  // A load is 8 rows of 128 bytes.  Pieces of a row are swapped by the row, so that those
-  // that a read meets lie in different banks.
-  const char* from[LOADS];
-  int col[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) col[i] = ((lane & 7) ^ ((i * 8 + (lane >> 3)) & 7)) * 8;
-#pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
-    const int row = i * 8 + (lane >> 3);
-    from[i] = (const char*)(i < RT * 2
-                                ? row_of<GATED>(a, col0, row)
-                                : a.x + (long)min(x0 + row - RT * 16, a.M - 1) * a.ldx);
-  }
-  const int c0 = SHARED ? blockIdx.y * a.share : 0;
-  const int all = (a.K + 63) / 64 - c0, chunks = SHARED ? min(a.share, all) : all;
-  const int first = first_of(a, a.share, chunks, bx);
-  const int mine = wid < chunks ? (chunks - 1 - wid) / OWN_WAVES + 1 : 0;
-  auto chunk = [&](int n) {
-    const int c = wid + n * OWN_WAVES + first;
-    return c0 + (c >= chunks ? c - chunks : c);
-  };
-  const int ring = wid * SL * CHUNK;
-  const unsigned lds = lds_at(smem);
-  auto issue = [&](int n, int slot) {
-    const int k0 = chunk(n) * 64;
-    unsigned k[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) k[i] = (unsigned)min(k0 + col[i], a.K - 8) * 2;
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i)
-      to_lds(from[i] + k[i & 1], lds + ring + slot * CHUNK + i * 1024);
-  };
-  constexpr int G = OWN_WAVES * SL * CHUNK;  // where the norm's weights lie
-  if (NORM) {
-    for (int i = wid; i * 512 < a.K; i += OWN_WAVES)
-      to_lds((const char*)(a.norm + min(i * 512 + lane * 8, a.K - 8)), lds + G + i * 1024);
-  }
-#pragma unroll
-  for (int s = 0; s < SL; ++s)
-    if (s < mine) issue(s, s);
-
-  f32x4 acc[RT][TT];
-  float sq[TT];
-#pragma unroll
-  for (int i = 0; i < TT; ++i) {
-    sq[i] = 0.0f;
-#pragma unroll
-    for (int r = 0; r < RT; ++r) acc[r][i] = f32x4{0, 0, 0, 0};
-  }
-  if (NORM) {
-    wait_chunks<SL, LOADS>(mine);
-    asm volatile("s_barrier" ::: "memory");
-  }
-  constexpr int TILES = (RT * TT + OWN_WAVES - 1) / OWN_WAVES;  // of y, of a wave
-  Ends<0> ends[TILES];
-  if (!GATED && a.fours) {
-#pragma unroll
-    for (int q = 0; q < TILES; ++q) {
-      const int n = min(wid + q * OWN_WAVES, RT * TT - 1);
-      ends[q].read(a, x0 + n % TT * 16 + l16, col0 + n / TT * 16 + lg * 4);
-    }
-  }
-  int slot = 0;
-  for (int n = 0; n < mine; ++n) {
-    wait_chunks<SL - 1, LOADS>(mine - 1 - n);
-    const int k0 = chunk(n) * 64;
-    const char* at = smem + ring + slot * CHUNK + l16 * 128;
-    bf16x8_t w[RT][2], v[TT][2], g[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int piece = ((u * 4 + lg) ^ (l16 & 7)) * 16;
-#pragma unroll
-      for (int i = 0; i < TT; ++i)
-        v[i][u] = *reinterpret_cast<const bf16x8_t*>(at + (RT + i) * 2048 + piece);
-      if (NORM)
-        g[u] = *reinterpret_cast<const bf16x8_t*>(smem + G + (k0 + u * 32 + lg * 8) * 2);
-#pragma unroll
-      for (int r = 0; r < RT; ++r)
-        w[r][u] = *reinterpret_cast<const bf16x8_t*>(at + r * 2048 + piece);
-    }
-    // all read: the chunk's place is free
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (n + SL < mine) issue(n + SL, slot);
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (u && k0 + 32 >= a.K) break;  // K is a multiple of 32
-#pragma unroll
-      for (int i = 0; i < TT; ++i) {
-        const bf16x8_t x = NORM ? times(v[i][u], g[u], a.offset, sq[i]) : v[i][u];
-#pragma unroll
-        for (int r = 0; r < RT; ++r)
-          acc[r][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[r][u], x, acc[r][i], 0, 0, 0);
-      }
-    }
-    if (++slot == SL) slot = 0;
-  }
-  __syncthreads();
-  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [waves][RT][TT][lanes]
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int i = 0; i < TT; ++i) red[((wid * RT + r) * TT + i) * WAVE + lane] = acc[r][i];
-  if (NORM) {
-#pragma unroll
-    for (int i = 0; i < TT; ++i) squares[wid][i][lane] = sq[i];
-  }
-  __syncthreads();
-
-  if (a.zero && blockIdx.x == 0)
-    for (int i = threadIdx.x; i < a.n_zero; i += OWN_WAVES * WAVE) a.zero[i] = 0;
-#pragma unroll
-  for (int q = 0; q < TILES; ++q) {
-    const int n = wid + q * OWN_WAVES;
-    if (n >= RT * TT) break;
-    f32x4 v = sum_of<TT, OWN_WAVES, TT, NORM>(a, red, squares, RT * TT, n, lane);
-    if (SHARED && !sums_of_all(a, (long)bx * RT * TT + n, lane, v)) continue;
-    const int row = x0 + n % TT * 16 + l16;
-    if (row < a.M)
-      finish_tile<GATED>(a, row, col0 + n / TT * (GATED ? 8 : 16), lg, v, ends[q]);
-  }
+  own_block<RT, TT, SL, GATED, NORM, SHARED, PAIRS>(a, blockIdx.x);
 }
 
 // RT, TT as above (one group of x's rows); RW, RX: stages of 128 columns of W and of x in
@@ -299,7 +42,7 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_ring_kernel(const Lin
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int l16 = lane & 15, lg = lane >> 4;
   const int step = wid % KS, tile0 = wid / KS * TW, part = wid & 3;
-  const BlockPlace at = place_of(a, 16 * TT);
+  const BlockPlace at = place_of(a, 16 * TT, blockIdx.x);
   const int x0 = at.x0, col0 = at.bx * COLS;
   if (col0 >= a.O) return;
   const bool loads_w = wid < 4;
@@ -426,27 +169,12 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_ring_kernel(const Lin
   }
 }
 
-// columns: of a chunk or stage
-void turned(LinearFewArgs& a, int act, int columns) {
-  a.parts = (unsigned char)act;
-  a.share = (a.K + columns - 1) / columns;
-  a.turn = a.share > 1 && in_step(a.ldw)
-               ? (unsigned)(((1ull << 32) + a.share - 1) / a.share) : 0;
-}
-
 template <typename Kernel>
 void launch(Kernel kernel, const LinearFewArgs& a, int blocks, int smem, hipStream_t stream) {
   if (smem > 48 * 1024)  // with the sums of squares above the default limit
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   kernel<<<blocks, OWN_WAVES * WAVE, smem, stream>>>(a);
-}
-
-// LDS of a block; slots: chunks of a wave
-int own_room(int rt, int tt, int slots, int K, bool norm) {
-  const int ring = OWN_WAVES * slots * (rt + tt) * 2048 + (norm ? (K + 511) / 512 * 1024 : 0);
-  const int sums = OWN_WAVES * rt * tt * 1024;
-  return ring > sums ? ring : sums;
 }
 
 template <int RT, int TT>

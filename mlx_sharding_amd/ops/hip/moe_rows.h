@@ -43,6 +43,10 @@ void launch_moe_pack(const void*, const void*, const void*, void*, int, int, int
                      int, hipStream_t);
 void launch_moe_rows(const MoeRowsArgs*, int, int, bool, hipStream_t);
 int moe_rows_longest(int);
+// moe_shared.hip
+void launch_moe_begin(const MoeRouteArgs*, int, const void*, void*, int, hipStream_t);
+void launch_moe_finish(const void*, const void*, const float*, const void*, void*, int, int,
+                       int, int, hipStream_t);
 void launch_moe_route(const MoeRouteArgs*, int, hipStream_t);
 void launch_moe_combine(const float*, const void*, const void*, void*, int, int,
                         int, hipStream_t);
