@@ -16,7 +16,7 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import (Linear, RMSNorm, StageModel, as_built, attend, feed, head,
+from .base import (Linear, RMSNorm, StageModel, as_built, attend, dense_weight, feed, head,
                    owned_layer_indices, project, read_in_place)
 
 
@@ -76,7 +76,10 @@ class LlamaAttention(nn.Module):
         gp = None
         out = None
         if T == 1 and type(cache) is KVCache:  # others append by methods of their own
-            out = cache.attend_step(q, k, v, cos, sin, self.scale, faster=True)
+            ahead = None  # a hint, for the few sequences that it is for
+            if B <= 16 and as_built(self.o_proj):
+                ahead = dense_weight(self.o_proj, self.n_heads * self.head_dim)
+            out = cache.attend_step(q, k, v, cos, sin, self.scale, faster=True, ahead=ahead)
         if out is not None:
             pass
         elif cache is not None and ops.use_native(x):

@@ -20,6 +20,7 @@
 // indexed (guide §5.4 rule 20).
 
 #include "hip_common.h"
+#include "warm.h"
 #include "soft_cap.h"
 
 #include <type_traits>
@@ -403,6 +404,7 @@ struct DecodeArgs {
   long qs, ks, vs;
   const float *cos, *sin;  // [DK / 2]
   unsigned* tickets;
+  Warm warm;               // for blocks from slice nsplit on
 };
 
 // Keys and values are read once: as a stream (2) they leave the L2 to what is read again
@@ -759,7 +761,13 @@ __global__ __launch_bounds__(AD_BLOCK, 2) void attn_decode_tile_kernel(
 // through memory to that block takes 3 us and 1.3 for what a thread asks for at once, the
 // merging kernel 4.5; the rotations 2 to 3 instead of 4.6 in a kernel of their own: one
 // sequence of 1024 keys, 32 heads of 128 over 8, 14.1 -> 9.6 us for the three.
+// Most of such a step is that chain, with the memory idle: beside few pairs and keys, blocks
+// of their own fetch the output projection's weights (warm.h).  A step of that sequence, four
+// layers with projections, 408 -> 399 us (attention 9 -> 11, projection 8 -> 5.9), of one of
+// 300, heads of 64, 132 -> 128.6; 8 of 1000 over 4 heads of 64 144.5 -> 145, so not for those.
 #define DW_WAVES 2
+#define DW_WARM_PAIRS 16
+#define DW_WARM_KEYS (8L << 20)  // bytes of keys and values
 template <int D, int NB, bool STEP>
 __global__ __launch_bounds__(DW_WAVES* WAVE) void attn_decode_wave_kernel(
     const DecodeArgs a) {
@@ -776,6 +784,14 @@ __global__ __launch_bounds__(DW_WAVES* WAVE) void attn_decode_wave_kernel(
   const int l16 = lane & 15, lg = lane >> 4;
   constexpr int SPAN = DW_WAVES * KT;
   const int lo = a.window > 0 && S > a.window ? S - a.window : 0;
+  if (STEP && (int)blockIdx.y >= a.nsplit) {
+    if ((long)gridDim.x * (S - lo) * (D * 4) > DW_WARM_KEYS) return;  // keys have the memory busy
+    const unsigned at =
+        (unsigned)(unsigned long long)(const __attribute__((address_space(3))) char*)smem;
+    warm_rows(a.warm, blockIdx.y * gridDim.x + blockIdx.x, a.nsplit * gridDim.x,
+              gridDim.y * gridDim.x, wid, DW_WAVES, at + wid * 1024);
+    return;
+  }
   const int per = ((S - lo + a.nsplit - 1) / a.nsplit + SPAN - 1) / SPAN * SPAN;
   const int from = min(S, lo + per * (int)blockIdx.y);
   const int to = min(S, from + per);
@@ -1031,10 +1047,13 @@ static void attn_decode_tile_go(const DecodeArgs& a, int B, bool wave, hipStream
   if constexpr (DK == DV) {
     // a wave's tiles: 32 KB, of heads of 256 twice that
     constexpr int NB = DK < 256 ? 256 / DK : 2, smem = DW_WAVES * NB * 2 * 32 * DK * 2;
+    // blocks that fetch weights: one a CU, which has room for two (of heads of 256 for one)
+    const bool warm = a.warm.w && DK < 256 && grid.x <= DW_WARM_PAIRS && grid.x * grid.y <= 256;
+    const dim3 more(grid.x, grid.y + (warm ? (255 + grid.x) / grid.x : 0));
     auto go = [&](auto kernel) {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-      kernel<<<grid, dim3(DW_WAVES * WAVE), smem, stream>>>(a);
+      kernel<<<a.tickets ? more : grid, dim3(DW_WAVES * WAVE), smem, stream>>>(a);
     };
     if (a.tickets) return go(&attn_decode_wave_kernel<DK, NB, true>);
     if constexpr (DK < 256) {
@@ -1081,10 +1100,10 @@ extern "C" void launch_attn_step(const void* q, const void* k, const void* v, lo
                                  float* part_ml, unsigned* tickets, int nsplit,
                                  const int* s_ptr, int B, int Hq, int Hkv, int S,
                                  long Scap, int D, float scale, float softcap, int window,
-                                 hipStream_t stream) {
+                                 const Warm* warm, hipStream_t stream) {
   const DecodeArgs a{(const char*)q, (const char*)kcache, (const char*)vcache, (char*)out,
                      part_o, part_ml, s_ptr, Hq, Hkv, S, nsplit, window, Scap,
                      soft_cap(scale, softcap), (const char*)k, (const char*)v, qs, ks, vs,
-                     cos, sin, tickets};
+                     cos, sin, tickets, *warm};
   attn_decode_tile_size(a, B, D, D, false, true, stream);
 }

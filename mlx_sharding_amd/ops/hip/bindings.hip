@@ -9,6 +9,7 @@
 #include "linear_few.h"
 #include "mla_decode.h"
 #include "moe_rows.h"
+#include "warm.h"
 #include "moe_tiles.h"
 
 extern "C" {
@@ -52,7 +53,7 @@ bool attn_decode_wave(int, long, long);
 void launch_attn_step(const void*, const void*, const void*, long, long, long,
                       const float*, const float*, void*, void*, void*, float*, float*,
                       unsigned*, int, const int*, int, int, int, int, long, int, float,
-                      float, int, hipStream_t);
+                      float, int, const Warm*, hipStream_t);
 void launch_attn_prefill(const void*, const void*, const void*, void*, int,
                          int, int, int, int, long, long, long, long, long, int,
                          int, float, float, int, int, hipStream_t);
@@ -526,15 +527,30 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
   return out;
 }
 
+// What may be fetched of the weights `ahead` [O, K] of a product of M rows behind a kernel on
+// like's device: a hint, nothing where it is of another kind.
+static Warm warm_of(const c10::optional<torch::Tensor>& ahead, const torch::Tensor& like,
+                    long M, long K) {
+  Warm warm{};
+  if (ahead.has_value() && ahead->device() == like.device() &&
+      ahead->scalar_type() == torch::kBFloat16 && ahead->dim() == 2 && ahead->size(1) == K &&
+      ahead->stride(1) == 1 && ahead->stride(0) % 8 == 0 &&
+      reinterpret_cast<uintptr_t>(ahead->data_ptr()) % 16 == 0 &&
+      !linear_own_warm(M, ahead->size(0), K, ahead->stride(0), ahead->data_ptr(), &warm))
+    warm = Warm{};
+  return warm;
+}
+
 // Attention of one token per sequence from its projections on: q [B, 1, Hq, D], k and v
 // [B, 1, Hkv, D] before rotations, whose row goes to the caches at pos (on the device) or
 // pos0; tickets [B * Hkv] of zeros, which they are again afterwards.  [B, 1, Hq * D], or
-// nothing where these are operands of the separate kernels.
+// nothing where these are operands of the separate kernels.  ahead: weights [O, Hq * D] of
+// the product behind it, which may be fetched meanwhile.
 c10::optional<torch::Tensor> attn_step(
     torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor cos,
     torch::Tensor sin, torch::Tensor kcache, torch::Tensor vcache,
     c10::optional<torch::Tensor> pos, int64_t pos0, torch::Tensor tickets, double scale,
-    double softcap, int64_t window, bool faster) {
+    double softcap, int64_t window, bool faster, c10::optional<torch::Tensor> ahead) {
   if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || kcache.dim() != 4 ||
       q.size(1) != 1)
     return c10::nullopt;
@@ -601,13 +617,14 @@ c10::optional<torch::Tensor> attn_step(
   if (nsplit > 1)
     part = torch::empty({B * Hq * nsplit * (D + 2)}, q.options().dtype(torch::kFloat32));
   float* po = nsplit > 1 ? part.data_ptr<float>() : nullptr;
+  const Warm warm = warm_of(ahead, q, B, Hq * D);
   launch_attn_step(q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0),
                    v.stride(0), cos.data_ptr<float>(), sin.data_ptr<float>(),
                    kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(), po,
                    po ? po + B * Hq * nsplit * D : nullptr,
                    reinterpret_cast<unsigned*>(tickets.data_ptr<int>()), nsplit, s_ptr,
                    (int)B, (int)Hq, (int)Hkv, (int)pos0 + 1, cap, (int)D, (float)scale,
-                   (float)softcap, (int)window, cur_stream());
+                   (float)softcap, (int)window, &warm, cur_stream());
   return out;
 }
 

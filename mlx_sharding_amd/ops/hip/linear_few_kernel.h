@@ -3,6 +3,7 @@
 #pragma once
 
 #include "hip_common.h"
+#include "warm.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -47,9 +48,7 @@ __device__ __forceinline__ void arrive(const LinearFewArgs& a) {
 // last may have less.
 __device__ __forceinline__ int first_of(const LinearFewArgs& a, int whole, int n,
                                         unsigned block) {
-  if (!a.turn) return 0;
-  const unsigned at = (block >> 3) * 3;
-  return max(min((int)(at - __umulhi(at, a.turn) * whole), n - 1), 0);
+  return first_chunk(a.turn, whole, n, block);
 }
 
 // The sums of a tile that blocks share: leaves this one's, and true in the one that

@@ -339,3 +339,22 @@ bool linear_own_go(LinearFewArgs a, int act, hipStream_t stream) {
   }
   return false;
 }
+
+// Up to 28 MB in all: the L2s have 32 (a step of one sequence, 32 heads of 128 over 8, 4096 by
+// 4096 behind them: 8 MB 402 us, 16 401, 24 to 40 398, none 406).
+extern "C" bool linear_own_warm(long M, long O, long K, long ld, const void* w, Warm* out) {
+  if (M < 1 || M > 16 || O < 1 || O >= 1L << 24 || K < 512 || K >= 1L << 22 || K % 32 ||
+      ld < K || ld >= 1L << 22)
+    return false;
+  LinearFewArgs a{};
+  a.M = (short)M, a.O = (int)O, a.K = (int)K, a.ldw = ld;
+  turned(a, LF_PLAIN, 64);
+  const int rt = own_tiles(a.M, a.O, a.K, LF_PLAIN, false).rt;
+  if (!rt) return false;
+  const int blocks = (a.O + 16 * rt - 1) / (16 * rt);
+  const long most = (28L << 20) / ((long)blocks * rt * 16 * 128);
+  if (most < 1) return false;
+  *out = Warm{(const char*)w, ld * 2, rt * 16, a.O, a.K, (int)min((long)a.share, most), blocks,
+              a.turn};
+  return true;
+}

@@ -110,11 +110,12 @@ class KVCache:
 
     def attend_step(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                     cos: torch.Tensor, sin: torch.Tensor, scale: float,
-                    softcap: float = 0.0, window: int = 0,
-                    faster: bool = False) -> Optional[torch.Tensor]:
+                    softcap: float = 0.0, window: int = 0, faster: bool = False,
+                    ahead: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
         """append_rope_qkv of one token per sequence and its attention in one kernel:
         [B, 1, heads * D]; None (and nothing appended) where that does not take it, or,
-        asked for what is ``faster``, where the separate kernels are."""
+        asked for what is ``faster``, where the separate kernels are.  ahead: weights of
+        the product behind it, which are fetched meanwhile."""
         from .. import ops as _ops
         if not (self.dtype == torch.bfloat16 and k.shape[1] == 1
                 and self.k_head_dim == self.v_head_dim == k.shape[3]
@@ -126,7 +127,8 @@ class KVCache:
                 return None  # the zeros would be written by replays only
             self._make_tickets()
         out = _ops.hip_ext().attn_step(q, k, v, cos, sin, self._k, self._v, pos, at,
-                                       self._tickets, scale, softcap, window, faster)
+                                       self._tickets, scale, softcap, window, faster,
+                                       ahead)
         if out is not None:
             self.wrote(1)
         return out
