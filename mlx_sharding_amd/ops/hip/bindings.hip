@@ -9,6 +9,7 @@
 #include "linear_few.h"
 #include "mla_decode.h"
 #include "moe_rows.h"
+#include "linear_turned.h"
 #include "warm.h"
 #include "moe_tiles.h"
 
@@ -1470,8 +1471,8 @@ std::vector<torch::Tensor> moe_gate_subranges(torch::Tensor logits, int64_t K,
 // x's rows, as the norm makes them, with w_qkv (queries, keys, values of all heads), their
 // rotations, keys and values to the caches from place `at` on, attention, and w_o's product,
 // plus the residual.  Nothing, and nothing written, where one of these does not run here.
-// (Launched one by one from Python, six kernels of a layer took the host 70 us, these four
-// and a feed-forward 38.)
+// (Launched one by one from Python, six kernels of a layer took the host 70 us, four in this
+// call and a feed-forward 38; three are left.)
 c10::optional<torch::Tensor> attend_few_try(
     torch::Tensor x, torch::Tensor w_qkv, c10::optional<torch::Tensor> b_qkv,
     torch::Tensor norm, double eps, double offset, torch::Tensor cos, torch::Tensor sin,
@@ -1486,6 +1487,7 @@ c10::optional<torch::Tensor> attend_few_try(
   if (heads < 1 || Hkv < 1 || heads % Hkv || D < 32 || D % 32 || D > 256 ||
       !attn_prefill_supported((int)D, (int)D) || w_qkv.size(0) != wide ||
       w_o.size(1) != heads * D || !linear_few_sizes(M, w_o.size(0), heads * D) ||
+      !linear_turned_takes(M, heads + 2 * Hkv, D, x.size(2)) ||
       !linear_few_along(x, wide, wide, b_qkv, {}, norm) ||
       !linear_few_along(x, w_o.size(0), w_o.size(0), b_o, residual, {}) || at < 0 ||
       at + T > cap)
@@ -1501,14 +1503,14 @@ c10::optional<torch::Tensor> attend_few_try(
       return {};
   c10::OptionalDeviceGuard guard;  // and the device's current stream
   if (x.get_device() != c10::hip::current_device()) guard.reset_device(x.device());
-  const auto y = linear_few_run(linear_few_rows(x), w_qkv, b_qkv, {}, norm, eps, offset, 0,
-                                {}, {});
   const auto q = torch::empty({M, heads * D}, x.options());
-  const char* of = (const char*)y.data_ptr();
-  launch_rope_qkv(of, of + heads * D * 2, of + (heads + Hkv) * D * 2, cos.data_ptr<float>(),
-                  sin.data_ptr<float>(), q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(),
-                  nullptr, at, M, (int)T, (int)heads, (int)Hkv, (int)D, cap, wide, wide, wide,
-                  cur_stream());
+  const auto rows = linear_few_rows(x);
+  const TurnedArgs t{cos.data_ptr<float>(), sin.data_ptr<float>(), (__bf16*)kcache.data_ptr(),
+                     (__bf16*)vcache.data_ptr(), cap, at, (int)T, (int)heads, (int)Hkv};
+  launch_linear_turned(rows.data_ptr(), w_qkv.data_ptr(),
+                       b_qkv.has_value() ? b_qkv->data_ptr() : nullptr, norm.data_ptr(),
+                       q.data_ptr(), (int)M, (int)w_qkv.size(1), (int)D, rows.stride(0),
+                       w_qkv.stride(0), (float)eps, (float)offset, &t, cur_stream());
   const auto o = torch::empty({M, heads * D}, x.options());
   launch_attn_prefill(q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), o.data_ptr(), (int)B,
                       (int)heads, (int)Hkv, (int)T, (int)(at + T), T * heads * D, D, heads * D,

@@ -2,6 +2,8 @@
 // that are made of it.
 #pragma once
 
+#include <type_traits>
+
 #include "linear_few_kernel.h"
 
 namespace {
@@ -35,14 +37,18 @@ __device__ __forceinline__ unsigned lds_at(const char* smem) {
   return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) char*)smem;
 }
 
-// The row of W of row `row` of a block's tiles.  A tile of a gated unit has eight columns:
-// rows 4g and 4g + 1 are the gate's of columns 2g and 2g + 1, the two others the up
-// projection's, so that a lane has both sums of a column.
-template <bool GATED>
+// How a tile's sixteen rows lie in W.  GATED: a tile has eight columns, rows 4g and 4g + 1 are
+// the gate's of columns 2g and 2g + 1, the two others the up projection's, O rows behind them, so
+// that a lane has both sums of a column.  TURNED: the same with the two dimensions that a rotation
+// takes, n_zero apart (half a head, a power of two); O counts them as one.
+enum { APART = 0, GATED_ROWS = 1, TURNED_ROWS = 2 };
+template <int ROWS>
 __device__ __forceinline__ const __bf16* row_of(const LinearFewArgs& a, int col0, int row) {
-  if (!GATED) return a.w + (long)min(col0 + row, a.O - 1) * a.ldw;
+  if (ROWS == APART) return a.w + (long)min(col0 + row, a.O - 1) * a.ldw;
   const int t = row >> 4, q = row & 15;
   const int col = min(col0 + t * 8 + (q >> 2) * 2 + (q & 1), a.O - 1);
+  if (ROWS == TURNED_ROWS)
+    return a.w + (long)(2 * col - (col & (a.n_zero - 1)) + (q & 2 ? a.n_zero : 0)) * a.ldw;
   return a.w + (long)((q & 2 ? a.O : 0) + col) * a.ldw;
 }
 
@@ -59,7 +65,7 @@ __device__ __forceinline__ BlockPlace place_of(const LinearFewArgs& a, int rows,
 }
 
 // a tile's sums to memory (gated: act(gate) * up of two columns); parts: the unit
-template <bool GATED>
+template <int GATED>
 __device__ __forceinline__ void finish_tile(const LinearFewArgs& a, int row, int col0, int lg,
                                             const f32x4& v, const Ends<0>& e) {
   if (!GATED) {
@@ -156,8 +162,9 @@ struct PairRows {
 // RT, TT: tiles of 16 rows of W and of x; SL: chunks of a wave under way.  The norm's weights
 // lie in LDS, all of them.  SHARED: blocks have a share of a contraction each.  PAIRS: to a
 // row of y, n_zero rows of `part` are added, which lie side by side (no norm, no share).
-template <int RT, int TT, int SL, bool GATED, bool NORM, bool SHARED, bool PAIRS>
-__device__ __forceinline__ void own_block(const LinearFewArgs& a, int block) {
+// finish: what becomes of a tile's sums (finish_tile).
+template <int RT, int TT, int SL, int GATED, bool NORM, bool SHARED, bool PAIRS, typename F>
+__device__ __forceinline__ void own_block(const LinearFewArgs& a, int block, F finish) {
   constexpr int LOADS = (RT + TT) * 2, CHUNK = LOADS * 1024;
   constexpr int COLS = (GATED ? 8 : 16) * RT;
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -298,8 +305,15 @@ __device__ __forceinline__ void own_block(const LinearFewArgs& a, int block) {
     const int row = x0 + n % TT * 16 + l16;
     if (PAIRS) pairs[q].add(v, a.n_zero);
     if (row < a.M)
-      finish_tile<GATED>(a, row, col0 + n / TT * (GATED ? 8 : 16), lg, v, ends[q]);
+      finish(row, col0 + n / TT * (GATED ? 8 : 16), lg, v, ends[q]);
   }
+}
+template <int RT, int TT, int SL, bool GATED, bool NORM, bool SHARED, bool PAIRS>
+__device__ __forceinline__ void own_block(const LinearFewArgs& a, int block) {
+  own_block<RT, TT, SL, GATED, NORM, SHARED, PAIRS>(
+      a, block, [&](int row, int col, int lg, const f32x4& v, const Ends<0>& e) {
+        finish_tile<GATED>(a, row, col, lg, v, e);
+      });
 }
 
 // columns: of a chunk or stage
@@ -315,6 +329,42 @@ inline int own_room(int rt, int tt, int slots, int K, bool norm) {
   const int ring = OWN_WAVES * slots * (rt + tt) * 2048 + (norm ? (K + 511) / 512 * 1024 : 0);
   const int sums = OWN_WAVES * rt * tt * 1024;
   return ring > sums ? ring : sums;
+}
+
+// Tiles of W's rows and of x's for M rows and `tiles`, beside `others` blocks, in kernels
+// that take no more than four of W's: as for other products (linear_own.hip).
+struct Tiles {
+  int rt, tt, blocks;
+};
+inline Tiles tiles_beside(int M, int tiles, int others, int K, bool norm) {
+  Tiles best{0, 0, 0};
+  long least = 0;
+  const int whole = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  for (int rt = 1; rt <= 4; ++rt)
+    for (int tt = whole; tt && tt * 2 >= whole; tt /= 2) {
+      if (own_room(rt, tt, 1, K, norm) > OWN_LDS) continue;
+      const int groups = (M + 16 * tt - 1) / (16 * tt);
+      int blocks = (tiles + rt - 1) / rt;
+      if (groups > 1) blocks = (blocks + 7) / 8 * 8 * groups;
+      const long reads = (long)((blocks + others + 255) / 256) *
+                         (M > 16 ? 2 * (rt + tt) : 2 * rt + 1);
+      if (!best.rt || reads < least || (reads == least && tt < best.tt))
+        best = {rt, tt, blocks}, least = reads;
+    }
+  return best;
+}
+
+// f with the constants rt and tt
+template <typename F>
+void with_tiles(const Tiles& t, F f) {
+  switch (t.rt * 8 + t.tt) {
+#define CASE(R, T) \
+  case R * 8 + T: f(std::integral_constant<int, R>(), std::integral_constant<int, T>()); break;
+    CASE(1, 1) CASE(2, 1) CASE(3, 1) CASE(4, 1)
+    CASE(1, 2) CASE(2, 2) CASE(3, 2) CASE(4, 2)
+    CASE(1, 4) CASE(2, 4) CASE(3, 4) CASE(4, 4)
+#undef CASE
+  }
 }
 
 }  // namespace

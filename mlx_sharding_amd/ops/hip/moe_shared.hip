@@ -140,48 +140,12 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void moe_finish_kernel(const Line
   own_block<RT, TT, RT == 1 ? 2 : 1, false, false, false, true>(a, blockIdx.x);
 }
 
-// Tiles of W's rows and of x's for M rows and `tiles`, beside `others` blocks: as for other
-// products (linear_own.hip), of up to four of W's rows.
-struct Tiles {
-  int rt, tt, blocks;
-};
-Tiles tiles_beside(int M, int tiles, int others, int K, bool norm) {
-  Tiles best{0, 0, 0};
-  long least = 0;
-  const int whole = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-  for (int rt = 1; rt <= 4; ++rt)
-    for (int tt = whole; tt && tt * 2 >= whole; tt /= 2) {
-      if (own_room(rt, tt, 1, K, norm) > OWN_LDS) continue;
-      const int groups = (M + 16 * tt - 1) / (16 * tt);
-      int blocks = (tiles + rt - 1) / rt;
-      if (groups > 1) blocks = (blocks + 7) / 8 * 8 * groups;
-      const long reads = (long)((blocks + others + 255) / 256) *
-                         (M > 16 ? 2 * (rt + tt) : 2 * rt + 1);
-      if (!best.rt || reads < least || (reads == least && tt < best.tt))
-        best = {rt, tt, blocks}, least = reads;
-    }
-  return best;
-}
-
 template <typename Kernel, typename Args>
 void go(Kernel kernel, const Args& a, int blocks, int smem, hipStream_t stream) {
   if (smem > 48 * 1024)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   kernel<<<blocks, OWN_WAVES * WAVE, smem, stream>>>(a);
-}
-
-// f with the constants rt and tt
-template <typename F>
-void with_tiles(const Tiles& t, F f) {
-  switch (t.rt * 8 + t.tt) {
-#define CASE(R, T) \
-  case R * 8 + T: f(std::integral_constant<int, R>(), std::integral_constant<int, T>()); break;
-    CASE(1, 1) CASE(2, 1) CASE(3, 1) CASE(4, 1)
-    CASE(1, 2) CASE(2, 2) CASE(3, 2) CASE(4, 2)
-    CASE(1, 4) CASE(2, 4) CASE(3, 4) CASE(4, 4)
-#undef CASE
-  }
 }
 
 }  // namespace
