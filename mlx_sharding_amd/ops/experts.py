@@ -138,12 +138,9 @@ def expert_rows(h, router, correction, up, down, sh: ExpertShape,
         tiled = sh.tiles(N) if (routing.on_input and glu is not None
                                 and _tiled(h, up, down)) else 0
         tile = tiled or sh.tile(N)
-        idx, weight, rank, hist = ext.expert_route(
+        weight, where, tokens, tiles, used, scale = ext.expert_place(
             h, router, correction, sh.total, sh.experts, sh.top,
-            routing.score == "sigmoid", routing.normalize)
-        scale = weight if routing.on_input else None
-        where, tokens, tiles, used, scale = ext.expert_plan(idx, rank, hist, scale,
-                                                            sh.experts, tile)
+            routing.score == "sigmoid", routing.normalize, routing.on_input, tile)
         if tiled:
             return ext.expert_tiles(h, tokens, tiles, used, up, down, scale, tile,
                                     glu.limit, glu.alpha), where, None

@@ -4,7 +4,7 @@
 #include "ragged_experts.h"
 
 extern "C" {
-void launch_expert_route(const RouteArgs*, bool, hipStream_t);
+void launch_expert_route(const RouteArgs*, const PlanArgs*, bool, hipStream_t);
 void launch_expert_plan(const PlanArgs*, hipStream_t);
 void launch_expert_gemm(const ExpertGemmArgs*, int, bool, hipStream_t);
 void launch_expert_combine(const CombineArgs*, bool, hipStream_t);
@@ -19,12 +19,12 @@ Tensor int_rows(const Tensor& like, std::vector<int64_t> sizes) {
 
 // h [N, K], w [total / 16, K / 32, 64, 8], correction [total] or none
 // -> chosen [N, top], weights [N, top], ranks [N, top], histograms
-std::tuple<Tensor, Tensor, Tensor, Tensor> expert_route(
-    Tensor h, Tensor w, c10::optional<Tensor> correction, int64_t total,
-    int64_t experts, int64_t top, bool sigmoid, bool normalize) {
-  const bool f32 = is_f32(h, "h");
+using Routes = std::tuple<Tensor, Tensor, Tensor, Tensor>;
+Routes route_args(RouteArgs& a, const Tensor& h, const Tensor& w,
+                  const c10::optional<Tensor>& correction, int64_t total, int64_t experts,
+                  int64_t top, bool sigmoid, bool normalize) {
+  is_f32(h, "h");
   check_like(w, h, "router");
-  RouteArgs a = {};
   a.sigmoid = sigmoid;
   a.normalize = normalize;
   a.hstride = rows2(h, "h");
@@ -56,16 +56,22 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> expert_route(
   a.weight = weight.data_ptr<float>();
   a.rank = rank.data_ptr<int>();
   a.hist = hist.data_ptr<int>();
-  if (a.n) launch_expert_route(&a, f32, stream());
   return {idx, weight, rank, hist};
+}
+
+Routes expert_route(Tensor h, Tensor w, c10::optional<Tensor> correction, int64_t total,
+                    int64_t experts, int64_t top, bool sigmoid, bool normalize) {
+  RouteArgs a = {};
+  const auto routes = route_args(a, h, w, correction, total, experts, top, sigmoid, normalize);
+  if (a.n) launch_expert_route(&a, nullptr, is_f32(h, "h"), stream());
+  return routes;
 }
 
 // -> rows of the pairs [N, top], tokens of the rows [N * top], tiles [*, 3], how many
 // of them there are, and the rows' weights [N * top] if weight is given
-std::tuple<Tensor, Tensor, Tensor, Tensor, c10::optional<Tensor>> expert_plan(
-    Tensor idx, Tensor rank, Tensor hist, c10::optional<Tensor> weight,
-    int64_t experts, int64_t tile) {
-  PlanArgs a = {};
+using Plan = std::tuple<Tensor, Tensor, Tensor, Tensor, c10::optional<Tensor>>;
+Plan plan_args(PlanArgs& a, const Tensor& idx, const Tensor& rank, const Tensor& hist,
+               const c10::optional<Tensor>& weight, int64_t experts, int64_t tile) {
   TORCH_CHECK(idx.dim() == 2 && hist.dim() == 2);
   a.n = idx.size(0);
   a.top = (int)idx.size(1);
@@ -97,8 +103,33 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, c10::optional<Tensor>> expert_plan(
     a.weight = weight->data_ptr<float>();
     a.scale = scale->data_ptr<float>();
   }
-  if (a.n) launch_expert_plan(&a, stream());
   return {where, tokens, tiles, used, scale};
+}
+
+Plan expert_plan(Tensor idx, Tensor rank, Tensor hist, c10::optional<Tensor> weight,
+                 int64_t experts, int64_t tile) {
+  PlanArgs a = {};
+  const auto plan = plan_args(a, idx, rank, hist, weight, experts, tile);
+  if (a.n) launch_expert_plan(&a, stream());
+  return plan;
+}
+
+// Both: weights [N, top], and expert_plan's (with weights where they go on the input)
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, c10::optional<Tensor>> expert_place(
+    Tensor h, Tensor w, c10::optional<Tensor> correction, int64_t total, int64_t experts,
+    int64_t top, bool sigmoid, bool normalize, bool on_input, int64_t tile) {
+  RouteArgs r = {};
+  const auto [idx, weight, rank, hist] =
+      route_args(r, h, w, correction, total, experts, top, sigmoid, normalize);
+  PlanArgs p = {};
+  c10::optional<Tensor> along;
+  if (on_input) along = weight;
+  const auto [where, tokens, tiles, used, scale] =
+      plan_args(p, idx, rank, hist, along, experts, tile);
+  const bool one = r.n <= EX_TOK && total <= 64;
+  if (r.n) launch_expert_route(&r, one ? &p : nullptr, is_f32(h, "h"), stream());
+  if (r.n && !one) launch_expert_plan(&p, stream());
+  return {weight, where, tokens, tiles, used, scale};
 }
 
 // x rows (of `tokens`, or the pairs' own) times w [experts, O, K] and the rows'
@@ -246,6 +277,7 @@ Tensor token_gate(Tensor x, Tensor w, Tensor e) {
 void bind_experts(pybind11::module_& m) {
   m.def("expert_route", &expert_route);
   m.def("expert_plan", &expert_plan);
+  m.def("expert_place", &expert_place);
   m.def("expert_gemm", &expert_gemm);
   m.def("expert_tiles", &expert_tiles);
   m.def("expert_combine", &expert_combine);

@@ -17,7 +17,8 @@
 // LDS.  Then a wave per token makes scores and picks.  Up to 64 experts are a lane each,
 // and both halves of the waves take parts of their contraction: one block of 16 tokens is
 // a chain of latencies (16 x 64 x 2048, 6 of them: 17.1 us, with all waves 16.3, picked
-// in registers, too, 12.7).
+// in registers, too, 12.7).  Where that is all, it places the pairs as well (plan.n above 0),
+// which takes a kernel of its own 5.3 us (13.2 without, 13.3 with it).
 // ---------------------------------------------------------------------------
 
 #define RT_BLOCK 1024
@@ -27,7 +28,7 @@
 
 template <typename T>
 __global__ __launch_bounds__(RT_BLOCK) void expert_route_kernel(
-    const RouteArgs a) {
+    const RouteArgs a, const PlanArgs plan) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int totalp = (a.total + 63) / 64 * 64;
   float* part = reinterpret_cast<float*>(smem);        // [parts][16][RT_LS]
@@ -97,6 +98,8 @@ __global__ __launch_bounds__(RT_BLOCK) void expert_route_kernel(
   }
   __syncthreads();
 
+  int held = 0, held_at = 0;  // of few experts: a lane's choice, and its rank
+  float held_weight = 0.0f;
   for (int t = wid; t < n; t += RT_WAVES) {
     const float* z = logits + t * totalp;
     if (few) {
@@ -130,9 +133,12 @@ __global__ __launch_bounds__(RT_BLOCK) void expert_route_kernel(
       }
       if (lane < a.top) {
         const long p = (t0 + t) * a.top + lane;
-        a.idx[p] = my_e;
-        a.weight[p] = a.normalize ? mine * (1.0f / (picked + 1e-20f)) : mine;
-        a.rank[p] = my_e < a.experts ? atomicAdd(&counts[my_e], 1) : 0;
+        held = my_e;
+        held_weight = a.normalize ? mine * (1.0f / (picked + 1e-20f)) : mine;
+        held_at = my_e < a.experts ? atomicAdd(&counts[my_e], 1) : 0;
+        a.idx[p] = held;
+        a.weight[p] = held_weight;
+        a.rank[p] = held_at;
       }
       continue;
     }
@@ -199,9 +205,49 @@ __global__ __launch_bounds__(RT_BLOCK) void expert_route_kernel(
   __syncthreads();
   for (int e = tid; e < a.experts; e += RT_BLOCK)
     a.hist[(long)blockIdx.x * a.experts + e] = counts[e];
+  if (!plan.n) return;
+
+  // expert_plan_kernel's work, an expert a lane of every wave, a token a wave
+  const int pairs = lane < a.experts ? counts[lane] : 0;
+  const int cuts = (pairs + plan.tile - 1) / plan.tile;
+  int sp = pairs, st = cuts;
+#pragma unroll
+  for (int o = 1; o < WAVE; o <<= 1) {
+    const int u = __shfl_up(sp, o, WAVE), v = __shfl_up(st, o, WAVE);
+    if (lane >= o) {
+      sp += u;
+      st += v;
+    }
+  }
+  const int used = __shfl(st, WAVE - 1, WAVE);
+  if (wid < n) {
+    const int begin = __shfl(sp - pairs, held & (WAVE - 1), WAVE);
+    if (lane < a.top) {
+      const int q = wid * a.top + lane;
+      const bool placed = held < a.experts;
+      plan.where[q] = placed ? begin + held_at : -1;
+      if (placed) {
+        plan.tokens[begin + held_at] = wid;
+        if (plan.scale) plan.scale[begin + held_at] = held_weight;
+      }
+    }
+  }
+  if (wid) return;
+  if (lane == 0) *plan.used = used;
+  for (int i = 0; i < cuts; ++i) {
+    int* t = plan.tiles + (long)(st - cuts + i) * 3;
+    t[0] = lane;
+    t[1] = sp - pairs + i * plan.tile;
+    t[2] = min(plan.tile, pairs - i * plan.tile);
+  }
+  for (int i = used + lane; i < plan.n_tiles; i += WAVE) {
+    int* t = plan.tiles + (long)i * 3;
+    t[0] = t[1] = t[2] = 0;
+  }
 }
 
-extern "C" void launch_expert_route(const RouteArgs* a, bool f32,
+// plan: places up to 16 tokens' pairs of up to 64 experts, too (null: none)
+extern "C" void launch_expert_route(const RouteArgs* a, const PlanArgs* plan, bool f32,
                                     hipStream_t stream) {
   const int totalp = (a->total + 63) / 64 * 64;
   const int parts = RT_PARTS * EX_TOK * RT_LS, picks = RT_WAVES * totalp;
@@ -213,7 +259,8 @@ extern "C" void launch_expert_route(const RouteArgs* a, bool f32,
     (void)hipFuncSetAttribute(                                              \
         reinterpret_cast<const void*>(&expert_route_kernel<T>),             \
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);             \
-    expert_route_kernel<T><<<grid, dim3(RT_BLOCK), smem, stream>>>(*a);     \
+    expert_route_kernel<T><<<grid, dim3(RT_BLOCK), smem, stream>>>(         \
+        *a, plan ? *plan : PlanArgs{});                                     \
   } while (0)
   if (f32) EX_GO(float);
   else EX_GO(__bf16);
