@@ -513,9 +513,9 @@ class GatedMLP(nn.Module):
 
 
 class BiasedMLP(nn.Module):
-    """W_down glu(W_gate h + b, W_up h + b) + b.  The products are plain ones;
-    the unit adds its biases itself, and the last one is left to what comes
-    next."""
+    """W_down glu(W_gate h + b, W_up h + b) + b.  Few rows take the unit and its
+    biases along in the first product, else they are a kernel behind it; the last
+    bias is left to what comes next."""
 
     def __init__(self, width: int, ff: int, glu: ClampedGLU,
                  dtype: torch.dtype = torch.bfloat16):
@@ -533,18 +533,27 @@ class BiasedMLP(nn.Module):
         self.half = -(-ff // 8) * 8
         w = self.gate.weight.data
         self.w_in = w.new_zeros(2 * self.half, w.shape[1])
+        self.b_in = w.new_zeros(2 * self.half)
         for at, m in ((0, self.gate), (self.half, self.up)):
-            part = self.w_in[at: at + ff]
-            part.copy_(m.weight.data)
-            m.weight.data = part
+            for own, both in ((m.weight, self.w_in), (m.bias, self.b_in)):
+                part = both[at: at + ff]
+                part.copy_(own.data)
+                own.data = part
 
     def rows(self, h: torch.Tensor):
         """(output without the last bias, that bias)."""
         if self.w_in is None:
             self.prepare()
-        y, ff = ops.linear(h, self.w_in), self.gate.out_features
-        u = self.glu(y[:, :ff], y[:, self.half: self.half + ff],
-                     self.gate.bias, self.up.bias)
+        ff = self.gate.out_features
+        u = None
+        if type(self.glu) is ClampedGLU:
+            u = ops.clamped_few(h, self.w_in, self.b_in, self.glu.limit, self.glu.alpha)
+        if u is not None:
+            u = u[:, :ff]
+        else:
+            y = ops.linear(h, self.w_in)
+            u = self.glu(y[:, :ff], y[:, self.half: self.half + ff],
+                         self.gate.bias, self.up.bias)
         return ops.linear(u, self.down.weight), self.down.bias
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:

@@ -327,6 +327,13 @@ def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None, clear=
                               norm.weight_offset, _ACTS[act], clear)
 
 
+def clamped_few(x, weight, bias, limit: float, alpha: float):
+    """The clamped unit (ragged.ClampedGLU) of the halves of x W^T + bias, of few rows, or
+    None where linear_own.hip does not take it."""
+    ext = _few_for(x, weight) if x.is_cuda else None
+    return None if ext is None else ext.linear_clamped_try(x, weight, bias, limit, alpha)
+
+
 def feed_few(x, w_in, w_out, act, norm=None, residual=None):
     """A feed-forward of few rows in one call: w_out of the gated unit of w_in's halves,
     of x's rows as ``norm`` makes them, plus ``residual``; None where linear_few.hip does

@@ -1556,6 +1556,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_few_try", &linear_few_try, py::arg("x"), py::arg("w"), py::arg("bias"),
         py::arg("residual"), py::arg("norm"), py::arg("eps"), py::arg("offset"),
         py::arg("act"), py::arg("clear") = py::none());
+  m.def("linear_clamped_try", &linear_clamped_try);
   m.def("feed_few_try", &feed_few_try);
   m.def("mla_rows", &mla_rows);
   m.def("mla_prompt", &mla_prompt);

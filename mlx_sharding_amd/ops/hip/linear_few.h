@@ -41,7 +41,8 @@ struct LinearFewRoom {
 };
 
 // x [M, K], w [O, K] (act: [2 O, K]); bias per row of w, residual [M, O], norm
-// weights [K] for the rows of x; act 0: none, 1: silu, 2: gelu_tanh.  room: for a shared
+// weights [K] for the rows of x; act 0: none, 1: silu, 2: gelu_tanh, 3: clamped, by eps and
+// offset (LF_CLAMPED), without a norm.  room: for a shared
 // contraction; clear: the numbers of another one's that runs behind this.
 static torch::Tensor linear_few_run(const torch::Tensor& x, const torch::Tensor& w,
                                     const c10::optional<torch::Tensor>& bias,
@@ -59,7 +60,7 @@ static torch::Tensor linear_few_run(const torch::Tensor& x, const torch::Tensor&
   };
   bf16(x);
   bf16(w);
-  TORCH_CHECK(act >= 0 && act <= 2, "unknown unit");
+  TORCH_CHECK(act >= 0 && act <= (norm || room.n ? 2 : 3), "unknown unit");
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "shapes");
   const int M = x.size(0), K = x.size(1), O = w.size(0) / (act ? 2 : 1);
   TORCH_CHECK(M >= 1 && K >= 32 && K % 32 == 0 && O >= 1 &&
@@ -296,6 +297,23 @@ static c10::optional<torch::Tensor> linear_few_try(
   }
   return linear_few_shaped(
       linear_few_run(rows, w, bias, residual, norm, eps, offset, act, {}, cleared), x);
+}
+
+// The clamped unit of x w^T + bias, of up to 64 rows and of more that linear_own.hip takes, or
+// nothing where that does not run here.
+static c10::optional<torch::Tensor> linear_clamped_try(const torch::Tensor& x,
+                                                       const torch::Tensor& w,
+                                                       const c10::optional<torch::Tensor>& bias,
+                                                       double limit, double alpha) {
+  if (!linear_few_input(x) || !linear_few_weight(w, x) || w.size(1) < 1 || w.size(0) % 2 ||
+      x.size(-1) != w.size(1))
+    return {};
+  const long K = w.size(1), M = x.numel() / K, O = w.size(0) / 2;
+  if (linear_few_other(K) || !linear_few_along(x, O, w.size(0), bias, {}, {}) ||
+      !(M > 64 ? linear_own_many(M, O, K, 3) : linear_few_sizes(M, O, K)))
+    return {};
+  return linear_few_shaped(
+      linear_few_run(linear_few_rows(x), w, bias, {}, {}, limit, alpha, 3, {}, {}), x);
 }
 
 // A feed-forward: w_out of the gated unit of w_in's halves (act 1 or 2), of x's rows as

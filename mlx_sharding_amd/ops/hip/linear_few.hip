@@ -260,7 +260,7 @@ extern "C" void launch_linear_few(const void* x, const void* w, const void* bias
   a.res = (const __bf16*)res, a.norm = (const __bf16*)norm, a.y = (__bf16*)y;
   a.M = (short)M, a.O = O, a.K = K;
   a.ldx = ldx, a.ldw = ldw, a.ldr = ldr, a.ldy = ldy;
-  if (norm) a.eps = eps, a.offset = offset;
+  if (norm || act == LF_CLAMPED) a.eps = eps, a.offset = offset;
   else a.part = part;
   a.count = count, a.zero = zero, a.n_zero = n_zero;
   a.fours = (bias || res) && O % 4 == 0 && (long)bias % 8 == 0 && (long)res % 8 == 0 &&

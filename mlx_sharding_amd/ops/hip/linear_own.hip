@@ -309,8 +309,9 @@ void linear_own_shared(LinearFewArgs a, int split, hipStream_t stream) {
 }
 
 bool linear_own_go(LinearFewArgs a, int act, hipStream_t stream) {
-  const OwnTiles t = a.M > 64 ? own_tiles_many(a.M, a.O, a.K, act)
-                              : own_tiles(a.M, a.O, a.K, act, a.norm != nullptr);
+  OwnTiles t = a.M > 64 ? own_tiles_many(a.M, a.O, a.K, act)
+                        : own_tiles(a.M, a.O, a.K, act, a.norm != nullptr);
+  if (!t.rt && act == LF_CLAMPED) t = {4, a.M <= 32 ? 2 : 4};  // which has no other kernel
   switch (t.rt * 8 + t.tt) {
     case 1 * 8 + 1: own<1, 1>(a, act, stream); return true;
     case 2 * 8 + 1: own<2, 1>(a, act, stream); return true;

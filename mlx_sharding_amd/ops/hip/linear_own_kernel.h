@@ -81,6 +81,9 @@ __device__ __forceinline__ void finish_tile(const LinearFewArgs& a, int row, int
     if (a.bias) f += (float)a.bias[at], up += (float)a.bias[a.O + at];
     if (a.parts == LF_SILU) {
       f = f / (1.0f + __expf(-f)) * up;
+    } else if (a.parts == LF_CLAMPED) {
+      f = fminf(f, a.eps);
+      f = f / (1.0f + __expf(-a.offset * f)) * (fminf(fmaxf(up, -a.eps), a.eps) + 1.0f);
     } else {
       const float z = 0.7978845608028654f * (f + 0.044715f * f * f * f);
       f = 0.5f * f * (1.0f + tanhf(z)) * up;
