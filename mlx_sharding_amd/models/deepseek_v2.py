@@ -483,8 +483,9 @@ class DeepseekV2MoE(nn.Module):
                                        m.down_proj.weight, self.top_k,
                                        *self._packing()))
 
-    def _beside(self, y, fits):
-        """The shared experts' matrices, where they go with the routed ones."""
+    def _beside(self, y, fits=None):
+        """The shared experts' matrices, where they go with the routed ones (``fits``:
+        with other kernels of theirs)."""
         m = self.shared_experts
         if (m is None or not as_built(m) or not as_built(*m.read())
                 or m._fused_gu is None or m._fused_gu.bias is not None
@@ -492,7 +493,7 @@ class DeepseekV2MoE(nn.Module):
             return None
         both = (dense_weight(m._fused_gu, y.shape[1]),
                 dense_weight(m.down_proj, m.down_proj.in_features))
-        return both if fits(*y.shape, *both) else None
+        return both if (fits or ops.expert_shared_ok)(*y.shape, *both) else None
 
     def decode(self, x, residual, norm, tickets=None):
         """The residual x (+ residual) after this feed-forward of it, normed:
@@ -514,7 +515,7 @@ class DeepseekV2MoE(nn.Module):
         if around is not None:
             rows = ops.expert_rows(y, choice, weight, *stacks, *packed)
             return ops.expert_finish(*units, around[1], rows, h).view(shape)
-        beside = self._beside(y, ops.expert_shared_ok)
+        beside = self._beside(y)
         if beside is not None:
             rows, shared = ops.expert_rows(y, choice, weight, *stacks, *packed, beside)
         else:
