@@ -152,11 +152,24 @@ class LlamaDecoderLayer(nn.Module):
                 and as_built(*attn.read(), *mlp.read())):
             h = attn(x, cos, sin, cache, norm, x)
             return mlp(h, self.post_attention_layernorm, h)
-        attn = attn(norm(x), cos, sin, cache)
-        # fused: h = x + attn; y = rms_norm(h) in one kernel
-        pn = self.post_attention_layernorm
-        y, h = ops.rms_norm_residual(attn, x, pn.weight, pn.eps,
-                                     pn.weight_offset)
+        pn, H = self.post_attention_layernorm, x.shape[-1]
+        more = ops.more_tokens(x)  # of which each half of the layer may be as few
+        if (more and x.shape[1] > 1 and type(cache) is KVCache and as_built(attn, norm)
+                and as_built(*attn.read()) and attn._fused_qkv is not None
+                and ops.one_round(x, (sum(attn._fused_qkv.splits), H, None),
+                                  (H, attn.n_heads * attn.head_dim, None))):
+            h, y = attn(x, cos, sin, cache, norm, x), None
+        else:
+            # fused: h = x + attn; y = rms_norm(h) in one kernel
+            y, h = ops.rms_norm_residual(attn(norm(x), cos, sin, cache), x, pn.weight,
+                                         pn.eps, pn.weight_offset)
+        if (y is None and as_built(mlp, pn) and as_built(*mlp.read())
+                and mlp._fused_gu is not None
+                and ops.one_round(h, (sum(mlp._fused_gu.splits) // 2, H, "silu"),
+                                  (H, sum(mlp._fused_gu.splits) // 2, None))):
+            return mlp(h, pn, h)
+        if y is None:
+            y = pn(h)
         return h + mlp(y)
 
 

@@ -259,6 +259,7 @@ def _dq_cache_ok(nbytes: int) -> bool:
 
 
 _FEW_ROWS = 64  # tokens of a batch that linear_few takes
+_MORE_ROWS = 384  # that linear_own.hip has products of
 _ACTS = {None: 0, "silu": 1, "gelu_tanh": 2}
 
 
@@ -395,6 +396,20 @@ def few_tokens(x: torch.Tensor) -> bool:
     (``project``)."""
     return (x.dtype == torch.bfloat16 and 0 < x.numel() <= _FEW_ROWS * x.shape[-1]
             and use_native(x) and _plain(x))
+
+
+def more_tokens(x: torch.Tensor) -> bool:
+    """Whether products of x's rows may be ones of ``one_round``."""
+    return (x.dtype == torch.bfloat16
+            and _FEW_ROWS * x.shape[-1] < x.numel() <= _MORE_ROWS * x.shape[-1]
+            and use_native(x) and _plain(x))
+
+
+def one_round(x: torch.Tensor, *products) -> bool:
+    """Whether products of more tokens (more_tokens), of (columns, contraction, ``act``),
+    come in one round of blocks each and take what lies between them along."""
+    takes, rows = hip_ext().linear_own_many, x.numel() // x.shape[-1]
+    return all(takes(rows, o, k, _ACTS[act]) for o, k, act in products)
 
 
 def linear(x, weight, bias=None):

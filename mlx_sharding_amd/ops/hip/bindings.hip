@@ -1479,14 +1479,16 @@ c10::optional<torch::Tensor> attend_few_try(
     torch::Tensor kcache, torch::Tensor vcache, int64_t at, torch::Tensor w_o,
     c10::optional<torch::Tensor> b_o, c10::optional<torch::Tensor> residual, int64_t heads,
     double scale, double softcap, int64_t window) {
-  if (x.dim() != 3 || kcache.dim() != 4 || !linear_few_takes(x, w_qkv) ||
-      !linear_few_weight(w_o, x))
+  if (x.dim() != 3 || kcache.dim() != 4 || !linear_few_input(x) ||
+      !linear_few_weight(w_qkv, x) || !linear_few_weight(w_o, x) || w_qkv.size(1) < 1 ||
+      x.size(2) != w_qkv.size(1) ||
+      !linear_few_more(x.numel() / x.size(2), w_qkv.size(0), x.size(2), 0))
     return {};
   const long B = x.size(0), T = x.size(1), M = B * T, Hkv = kcache.size(1),
              cap = kcache.size(2), D = kcache.size(3), wide = (heads + 2 * Hkv) * D;
   if (heads < 1 || Hkv < 1 || heads % Hkv || D < 32 || D % 32 || D > 256 ||
       !attn_prefill_supported((int)D, (int)D) || w_qkv.size(0) != wide ||
-      w_o.size(1) != heads * D || !linear_few_sizes(M, w_o.size(0), heads * D) ||
+      w_o.size(1) != heads * D || !linear_few_more(M, w_o.size(0), heads * D, 0) ||
       !linear_turned_takes(M, heads + 2 * Hkv, D, x.size(2)) ||
       !linear_few_along(x, wide, wide, b_qkv, {}, norm) ||
       !linear_few_along(x, w_o.size(0), w_o.size(0), b_o, residual, {}) || at < 0 ||
@@ -1525,6 +1527,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("norm_add", &norm_add);
   m.def("attn_step", &attn_step);
   m.def("attend_few_try", &attend_few_try);
+  m.def("linear_own_many", [](int64_t M, int64_t O, int64_t K, int64_t act) {
+    return (bool)linear_own_many(M, O, K, (int)act);
+  });
   m.def("step_begin", &step_begin);
   m.def("step_end", &step_end);
   m.def("rope_qkv", &rope_qkv, py::arg("q"), py::arg("k"), py::arg("v"),

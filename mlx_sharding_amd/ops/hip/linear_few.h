@@ -64,8 +64,7 @@ static torch::Tensor linear_few_run(const torch::Tensor& x, const torch::Tensor&
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "shapes");
   const int M = x.size(0), K = x.size(1), O = w.size(0) / (act ? 2 : 1);
   TORCH_CHECK(M >= 1 && K >= 32 && K % 32 == 0 && O >= 1 &&
-                  (M <= 64 || (!norm && !residual && !room.n && !clear.n &&
-                               linear_own_many(M, O, K, (int)act))),
+                  (M <= 64 || (!room.n && linear_own_many(M, O, K, (int)act))),
               "1 to 64 rows of a multiple of 32, or more that there is a kernel for");
   TORCH_CHECK(!act || w.size(0) % 2 == 0, "a gated unit has two halves");
   for (const auto& t : {x, w})
@@ -158,6 +157,13 @@ static bool linear_few_weight(const torch::Tensor& w, const torch::Tensor& x) {
 static bool linear_few_sizes(long rows, long O, long K) {
   return O >= 1 && K >= 32 && K % 32 == 0 && rows >= 1 && rows <= 64 &&
          !(K > 8192 && rows > 8 && O > 4096) && !linear_few_other(K);
+}
+
+// The same with more rows, where one round of blocks has them all (linear_own.hip).
+// O: columns of the result, of two halves of w's rows with a unit.
+static bool linear_few_more(long rows, long O, long K, int act) {
+  if (rows <= 64) return linear_few_sizes(rows, act ? 2 * O : O, K);
+  return !linear_few_other(K) && linear_own_many(rows, O, K, act);
 }
 
 // Whether x w^T runs here.
@@ -324,19 +330,20 @@ static c10::optional<torch::Tensor> feed_few_try(
     c10::optional<torch::Tensor> residual, c10::optional<torch::Tensor> norm, double eps,
     double offset, int64_t act) {
   TORCH_CHECK(act == 1 || act == 2, "unknown unit");
-  if (!linear_few_takes(x, w_in) || !linear_few_weight(w_out, x) ||
-      w_in.size(0) != 2 * w_out.size(1))
+  if (!linear_few_input(x) || !linear_few_weight(w_in, x) || !linear_few_weight(w_out, x) ||
+      w_in.size(1) < 1 || x.size(-1) != w_in.size(1) || w_in.size(0) != 2 * w_out.size(1) ||
+      !linear_few_more(x.numel() / w_in.size(1), w_out.size(1), w_in.size(1), (int)act))
     return {};
   const int M = x.numel() / x.size(-1), O = w_out.size(0), I = w_out.size(1);
   // long contractions into many columns have a kernel of their own (gemm_kseg.hip)
   if (I >= 16384 && O >= 8192 && !residual.has_value()) return {};
-  if (!linear_few_sizes(M, O, I) ||
+  if (!linear_few_more(M, O, I, 0) ||
       !linear_few_along(x, I, 2 * I, {}, {}, norm) ||
       !linear_few_along(x, O, O, {}, residual, {}))
     return {};
   const auto rows = linear_few_rows(x);
   if (residual.has_value() && x.dim() != 2) residual = residual->reshape({M, -1});
-  const LinearFewRoom room(M, O, I, rows);
+  const auto room = M <= 64 ? LinearFewRoom(M, O, I, rows) : LinearFewRoom();
   const auto units =
       linear_few_run(rows, w_in, {}, {}, norm, eps, offset, act, {}, room);
   return linear_few_shaped(

@@ -1,5 +1,5 @@
 // q, k and v of few tokens: their product with the rows' norm, the rotations of queries and keys,
-// and keys and values to the cache, up to 64 rows in one kernel.
+// and keys and values to the cache, up to 384 rows in one kernel.
 //
 // A tile of linear_own_kernel has the two dimensions that a rotation takes in one lane (row_of),
 // which turns them as rounded, so that the results are those of the product and rope_qkv_kernel.
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_turned_kernel(const T
 }  // namespace
 
 extern "C" bool linear_turned_takes(long M, long heads, long D, long K) {
-  return M >= 1 && M <= 64 && K >= 32 && K % 32 == 0 && K <= 32768 && D >= 32 && D <= 256 &&
+  return M >= 1 && M <= 384 && K >= 32 && K % 32 == 0 && K <= 32768 && D >= 32 && D <= 256 &&
          (D & (D - 1)) == 0 && heads * D < 1L << 24 &&
          tiles_beside((int)M, (int)(heads * D / 16), 0, (int)K, true).rt > 0;
 }
