@@ -152,8 +152,8 @@ static bool linear_few_weight(const torch::Tensor& w, const torch::Tensor& x) {
 }
 
 // Whether a product of this size runs here.  A contraction above 8192 for 8 rows, or
-// into 4096: 8 rows of 14336 into 4096 take 24.6 us here and 26.6 in the library, 32
-// rows 30.4 and 30.5, 64 rows 40.1 and 38.9.
+// into 4096: 8 rows of 14336 into 4096 take 23.0 us here and 24.9 in the library, 32
+// rows 32.7 and 32.4, 64 rows 38.2 and 40.2.
 static bool linear_few_sizes(long rows, long O, long K) {
   return O >= 1 && K >= 32 && K % 32 == 0 && rows >= 1 && rows <= 64 &&
          !(K > 8192 && rows > 8 && O > 4096) && !linear_few_other(K);
