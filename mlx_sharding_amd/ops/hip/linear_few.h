@@ -151,12 +151,14 @@ static bool linear_few_weight(const torch::Tensor& w, const torch::Tensor& x) {
          w.stride(0) % 8 == 0 && linear_few_whole(w);
 }
 
-// Whether a product of this size runs here.  A contraction above 8192 for 8 rows, or
-// into 4096: 8 rows of 14336 into 4096 take 23.0 us here and 24.9 in the library, 32
-// rows 32.7 and 32.4, 64 rows 38.2 and 40.2.
+// Whether a product of this size runs here.  Contractions of 16384 and more into many columns
+// have a kernel of their own (gemm_kseg.hip) or are the library's.  Over 90 random sizes of 9 to
+// 64 rows of 8704 to 16352 into 4112 to 20000 the time here is .89 of the library's, at most
+// 1.05 (16 rows of 13824 into 5120 32.7 us there; 8 rows of 14336 into 4096 23.0 us here and
+// 24.9, 64 rows 38.2 and 40.2).
 static bool linear_few_sizes(long rows, long O, long K) {
   return O >= 1 && K >= 32 && K % 32 == 0 && rows >= 1 && rows <= 64 &&
-         !(K > 8192 && rows > 8 && O > 4096) && !linear_few_other(K);
+         !(K >= 16384 && rows > 8 && O > 4096) && !linear_few_other(K);
 }
 
 // The same with more rows, where one round of blocks has them all (linear_own.hip).

@@ -67,6 +67,15 @@ def test_ends(M, O, K, act):
     check(M, K, O, act, False, True, True)
 
 
+# long contractions into many columns
+@pytest.mark.parametrize("act", [None, "silu"])
+@pytest.mark.parametrize("M,K,O", [(9, 8224, 4097), (17, 9216, 8200), (64, 8224, 4112),
+                                   (33, 16352, 5000), (64, 13824, 9001)])
+def test_long(M, K, O, act):
+    check(M, K, O, act, False, True, True)
+    check(M, K, O, act, True, False, False)
+
+
 # 65 and more rows: groups of 32 and 64, with as many tiles as fit a round of 256 blocks, and one
 # more; the longest contraction, and the shortest
 @pytest.mark.parametrize("act", [None, "silu", "gelu_tanh"])
