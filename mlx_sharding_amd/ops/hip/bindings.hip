@@ -533,7 +533,7 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k, torch::Tensor v,
 static Warm warm_of(const c10::optional<torch::Tensor>& ahead, const torch::Tensor& like,
                     long M, long K) {
   Warm warm{};
-  if (ahead.has_value() && ahead->device() == like.device() &&
+  if (ahead.has_value() && linear_few_plain(*ahead) && ahead->device() == like.device() &&
       ahead->scalar_type() == torch::kBFloat16 && ahead->dim() == 2 && ahead->size(1) == K &&
       ahead->stride(1) == 1 && ahead->stride(0) % 8 == 0 &&
       reinterpret_cast<uintptr_t>(ahead->data_ptr()) % 16 == 0 &&
@@ -1202,7 +1202,8 @@ std::vector<torch::Tensor> moe_route(torch::Tensor x,
     launch_moe_route(&a, (int)N, cur_stream());
     return {y, h, choice, weight};
   }
-  TORCH_CHECK(tickets.has_value() && !residual.has_value() && N <= 64 && H <= 4096,
+  TORCH_CHECK(tickets.has_value() && !residual.has_value() && N <= 64 && H <= 4096 &&
+                  w_in->device() == x.device(),
               "rows that a shared feed-forward goes with");
   const long S = w_in->size(0) / 2;
   TORCH_CHECK(S >= 1 && S < 1L << 24, "units");
@@ -1339,6 +1340,7 @@ torch::Tensor moe_finish(torch::Tensor units, torch::Tensor w_out, torch::Tensor
   check_rows(units, "units", N, S);
   check_rows(w_out, "w_out", H, S);
   check_rows(h, "h", N, H);
+  TORCH_CHECK(w_out.device() == units.device() && h.device() == units.device(), "one device");
   TORCH_CHECK(rows.is_cuda() && rows.device() == units.device() &&
                   rows.scalar_type() == torch::kFloat32 && rows.is_contiguous() &&
                   rows.size(1) == H && rows.size(0) >= N && rows.size(0) % N == 0, "rows");

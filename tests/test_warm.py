@@ -42,8 +42,20 @@ def test_other_weights():
     g = torch.Generator("cuda").manual_seed(1)
     one, two = _caches(1, 8, 128, 50, 100, False, g)
     w = torch.randn(512, 4096, device="cuda").bfloat16()
-    for ahead in (w.float(), w.cpu(), w[:, :4000], w.t().contiguous().t(), w[0], w[:0],
+    for ahead in (w.float(), w.cpu(), w[:, :4000], torch.nn.Parameter(w), w.t().contiguous().t(), w[0], w[:0],
                   torch.empty(512 * 4096 + 1, device="cuda").bfloat16()[1:].view(512, 4096)):
         (q, k, v), cos, sin = _token(1, 32, 8, 128, g)
         assert torch.equal(one.attend_step(q, k, v, cos, sin, 0.1, ahead=ahead),
                            two.attend_step(q, k, v, cos, sin, 0.1))
+
+
+def test_mapped_weights():
+    """Weights that are mapped, of which there is no one address."""
+    g = torch.Generator("cuda").manual_seed(2)
+    one, two = _caches(1, 8, 128, 50, 100, False, g)
+    (q, k, v), cos, sin = _token(1, 32, 8, 128, g)
+    want = two.attend_step(q, k, v, cos, sin, 0.1)
+    several = torch.randn(2, 512, 4096, device="cuda").bfloat16()
+    got = torch.vmap(lambda w: one.attend_step(q, k, v, cos, sin, 0.1, ahead=w) @ w.t())(
+        several[:1])
+    assert torch.equal(got[0], want @ several[0].t())
