@@ -21,14 +21,14 @@
 
 namespace {
 
-template <int RT, int TT, int SL, bool GATED, bool NORM, bool SHARED, bool PAIRS = false>
+template <int RT, int TT, int SL, int GATED, bool NORM, bool SHARED, bool PAIRS = false>
 __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_own_kernel(const LinearFewArgs a) {
   own_block<RT, TT, SL, GATED, NORM, SHARED, PAIRS>(a, blockIdx.x);
 }
 
 // RT, TT as above (one group of x's rows); RW, RX: stages of 128 columns of W and of x in
 // LDS, a row of the norm's weights behind x's.
-template <int RT, int TT, int RW, int RX, bool GATED, bool NORM>
+template <int RT, int TT, int RW, int RX, int GATED, bool NORM>
 __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_ring_kernel(const LinearFewArgs a) {
   constexpr int KS = 4, TW = TT * KS / OWN_WAVES;  // steps of a stage, tiles of x of a wave
   constexpr int COLS = (GATED ? 8 : 16) * RT;
@@ -200,7 +200,8 @@ void own(LinearFewArgs a, int act, hipStream_t stream) {
     if (act) go(&linear_own_kernel<RT, TT, 1, true, true, false>, 1);
     else go(&linear_own_kernel<RT, TT, 1, false, true, false>, 1);
   } else {
-    if (act) go(&linear_own_kernel<RT, TT, most, true, false, false>, most);
+    if (act == LF_CLAMPED) go(&linear_own_kernel<RT, TT, most, CLAMPED_ROWS, false, false>, most);
+    else if (act) go(&linear_own_kernel<RT, TT, most, true, false, false>, most);
     else go(&linear_own_kernel<RT, TT, most, false, false, false>, most);
   }
 }
@@ -221,7 +222,8 @@ void ring(LinearFewArgs a, int act, hipStream_t stream) {
     if (act) go(&linear_ring_kernel<RT, TT, RW, RX, true, true>);
     else go(&linear_ring_kernel<RT, TT, RW, RX, false, true>);
   } else {
-    if (act) go(&linear_ring_kernel<RT, TT, RW, RX, true, false>);
+    if (act == LF_CLAMPED) go(&linear_ring_kernel<RT, TT, RW, RX, CLAMPED_ROWS, false>);
+    else if (act) go(&linear_ring_kernel<RT, TT, RW, RX, true, false>);
     else go(&linear_ring_kernel<RT, TT, RW, RX, false, false>);
   }
 }
