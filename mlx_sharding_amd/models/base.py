@@ -109,14 +109,19 @@ def dense_weight(m, in_features: int) -> Optional[torch.Tensor]:
                                q.group_size, q.bits)
 
 
+def weight_for(m, x: torch.Tensor, in_features: int) -> Optional[torch.Tensor]:
+    """dense_weight as ``project`` of rows like x reads it: packed words have a copy only
+    on the GPU, and only where torch's own operators are not asked for."""
+    return dense_weight(m, in_features) if m.quant is None or ops.use_native(x) else None
+
+
 def feed(into, out, x: torch.Tensor, act: str, norm: Optional[nn.Module] = None,
          residual: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The gated unit of ``into``'s halves through ``out``, as ``project`` of each; one
     call for few rows."""
     if into.bias is None and out.bias is None and x.is_cuda:
-        w_in = into.weight if into.quant is None else dense_weight(into, x.shape[-1])
-        w_out = (out.weight if out.quant is None
-                 else dense_weight(out, sum(into.splits) // 2))
+        w_in = weight_for(into, x, x.shape[-1])
+        w_out = weight_for(out, x, sum(into.splits) // 2)
         if w_in is not None and w_out is not None:
             y = ops.feed_few(x, w_in, w_out, act, norm, residual)
             if y is not None:
@@ -128,8 +133,8 @@ def attend(qkv, out, x: torch.Tensor, norm: nn.Module, cos, sin, cache, heads: i
            scale: float, softcap: float = 0.0, window: int = 0,
            residual: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """ops.attend_few with the weights of a FusedColumns and a Linear, or None."""
-    w_qkv, w_o = (m.weight if m.quant is None else dense_weight(m, n)
-                  for m, n in ((qkv, x.shape[-1]), (out, heads * cache.k_head_dim)))
+    w_qkv = weight_for(qkv, x, x.shape[-1])
+    w_o = weight_for(out, x, heads * cache.k_head_dim)
     if w_qkv is None or w_o is None:
         return None
     return ops.attend_few(x, w_qkv, qkv.bias, norm, cos, sin, cache, w_o, out.bias, residual,
@@ -142,8 +147,7 @@ def project(m, x: torch.Tensor, *, norm: Optional[nn.Module] = None,
             clear: Optional[torch.Tensor] = None) -> torch.Tensor:
     """ops.project with the weights of a Linear or FusedColumns, packed ones
     through their bf16 copy."""
-    q = m.quant
-    w = dense_weight(m, x.shape[-1]) if q is None or ops.use_native(x) else None
+    q, w = m.quant, weight_for(m, x, x.shape[-1])
     if w is not None:
         return ops.project(x, w, m.bias, norm=norm, act=act, residual=residual,
                            clear=clear)

@@ -16,8 +16,8 @@ import torch.nn as nn
 from .. import ops
 from ..config import ModelConfig, ShardSpec
 from ..ops.kvcache import KVCache
-from .base import (Linear, RMSNorm, StageModel, as_built, attend, dense_weight, feed, head,
-                   owned_layer_indices, project, read_in_place)
+from .base import (Linear, RMSNorm, StageModel, as_built, attend, feed, head,
+                   owned_layer_indices, project, read_in_place, weight_for)
 
 
 @read_in_place
@@ -78,7 +78,7 @@ class LlamaAttention(nn.Module):
         if T == 1 and type(cache) is KVCache:  # others append by methods of their own
             ahead = None  # a hint, for the few sequences that it is for
             if B <= 16 and as_built(self.o_proj):
-                ahead = dense_weight(self.o_proj, self.n_heads * self.head_dim)
+                ahead = weight_for(self.o_proj, x, self.n_heads * self.head_dim)
             out = cache.attend_step(q, k, v, cos, sin, self.scale, faster=True, ahead=ahead)
         if out is not None:
             pass

@@ -1067,6 +1067,11 @@ torch::Tensor w4a16_gemv(torch::Tensor x, torch::Tensor wq,
 torch::Tensor dequant(torch::Tensor wq, torch::Tensor scales,
                       torch::Tensor biases, int64_t H, int64_t gs,
                       int64_t bits) {
+  check_bf16(scales, "scales");
+  check_bf16(biases, "biases");
+  TORCH_CHECK(wq.is_cuda() && wq.element_size() == 4 && wq.device() == scales.device() &&
+                  biases.device() == scales.device(),
+              "dequant takes words of 32 bits, scales and biases on one GPU");
   const long O = wq.size(0);
   auto out = torch::empty({O, H}, scales.options());
   launch_dequant(wq.contiguous().data_ptr(), scales.contiguous().data_ptr(),
