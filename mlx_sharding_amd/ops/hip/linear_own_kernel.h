@@ -27,12 +27,6 @@ __device__ __forceinline__ void wait_chunks(int younger) {
   }
 }
 
-// 16 bytes a lane from memory to LDS (at + 16 * lane).  The compiler does not know of the
-// load, which would have it wait for all before reads of LDS; no register is written.
-__device__ __forceinline__ void to_lds(const char* from, unsigned at) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(from)
-               : "memory", "m0");
-}
 __device__ __forceinline__ unsigned lds_at(const char* smem) {
   return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) char*)smem;
 }

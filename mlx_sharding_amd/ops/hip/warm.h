@@ -6,6 +6,16 @@
 
 #include "hip_common.h"
 
+// 16 bytes a lane from memory to LDS (at + 16 * lane).  The compiler does not know of the
+// load, which would have it wait for all before reads of LDS; no register is written.  Nor does
+// it look into the text: a load to LDS may not read M0 in the cycle behind the scalar unit's
+// write of it, so that one idle instruction lies between.
+__device__ __forceinline__ void to_lds(const char* from, unsigned at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at),
+               "v"(from)
+               : "memory", "m0");
+}
+
 struct Warm {
   const char* w;  // null: none
   long ld;        // bytes from row to row
@@ -38,8 +48,7 @@ __device__ __forceinline__ void warm_rows(const Warm& a, int block, int base, in
       c = c >= all ? c - all : c;
       const int row = min(b * a.rows + i % (a.rows / 8) * 8 + (lane >> 3), a.O - 1);
       const char* from = a.w + (long)row * a.ld + min(c * 64 + (lane & 7) * 8, a.K - 8) * 2;
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(from)
-                   : "memory", "m0");
+      to_lds(from, lds);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
