@@ -113,7 +113,7 @@ __global__ __launch_bounds__(OWN_WAVES * WAVE) void linear_ring_kernel(const Lin
   for (int t = 0; t < stages; ++t) {
     if (loads_w) wait_chunks<RW - 2, RT>(stages - 1 - t);
     else wait_chunks<RX - 2, TT + (NORM ? 1 : 0)>(stages - 1 - t);
-    asm volatile("s_barrier" ::: "memory");
+    meet();
     // into the place of the stage before, which all have read
     if (loads_w) {
       if (t + RW - 1 < stages) issue_w(t + RW - 1, sw ? sw - 1 : RW - 1);

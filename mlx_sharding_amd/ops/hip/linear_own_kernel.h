@@ -27,6 +27,12 @@ __device__ __forceinline__ void wait_chunks(int younger) {
   }
 }
 
+// A barrier for loads to LDS on either side of it: this wave's reads of LDS have returned, so that
+// other waves may load into their places.
+__device__ __forceinline__ void meet() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 __device__ __forceinline__ unsigned lds_at(const char* smem) {
   return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) char*)smem;
 }
@@ -228,7 +234,7 @@ __device__ __forceinline__ void own_block(const LinearFewArgs& a, int block, F f
   }
   if (NORM) {
     wait_chunks<SL, LOADS>(mine);
-    asm volatile("s_barrier" ::: "memory");
+    meet();
   }
   constexpr int TILES = (RT * TT + OWN_WAVES - 1) / OWN_WAVES;  // of y, of a wave
   Ends<0> ends[TILES];

@@ -26,3 +26,15 @@ def test_a_load_to_lds_waits_for_its_place(path):
                 # where the place is written elsewhere, nobody knows how far before
                 wrote = [k for k in range(i) if re.match(r"s_\w+ m0\b", piece[k])]
                 assert wrote and i - wrote[-1] >= 2, (path.name, piece)
+
+
+@pytest.mark.parametrize("path", SOURCES, ids=lambda p: p.name)
+def test_a_barrier_says_what_lies_before_it(path):
+    """Behind a barrier in assembly others load into places that this wave has read: its reads
+    have returned, in the same piece, or by a wait or a fence that the compiler keeps beside it."""
+    text = path.read_text()
+    for at in re.finditer(r"asm volatile\(\s*\"[^\"]*s_barrier", text):
+        before = text[:at.start()].splitlines()[-2:]
+        assert ("s_waitcnt" in at.group() or any("amdgcn_s_waitcnt" in line
+                                                 or "amdgcn_sched_barrier" in line
+                                                 for line in before)), path.name
