@@ -533,12 +533,10 @@ class BiasedMLP(nn.Module):
         self.half = -(-ff // 8) * 8
         w = self.gate.weight.data
         self.w_in = w.new_zeros(2 * self.half, w.shape[1])
-        self.b_in = w.new_zeros(2 * self.half)
         for at, m in ((0, self.gate), (self.half, self.up)):
-            for own, both in ((m.weight, self.w_in), (m.bias, self.b_in)):
-                part = both[at: at + ff]
-                part.copy_(own.data)
-                own.data = part
+            part = self.w_in[at: at + ff]
+            part.copy_(m.weight.data)
+            m.weight.data = part
 
     def rows(self, h: torch.Tensor):
         """(output without the last bias, that bias)."""
@@ -547,7 +545,8 @@ class BiasedMLP(nn.Module):
         ff = self.gate.out_features
         u = None
         if type(self.glu) is ClampedGLU:
-            u = ops.clamped_few(h, self.w_in, self.b_in, self.glu.limit, self.glu.alpha)
+            u = ops.clamped_few(h, self.w_in, (self.gate.bias, self.up.bias),
+                                self.glu.limit, self.glu.alpha)
         if u is not None:
             u = u[:, :ff]
         else:

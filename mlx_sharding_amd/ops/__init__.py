@@ -330,9 +330,16 @@ def _linear_few(x, weight, bias=None, residual=None, norm=None, act=None, clear=
 
 def clamped_few(x, weight, bias, limit: float, alpha: float):
     """The clamped unit (ragged.ClampedGLU) of the halves of x W^T + bias, of few rows, or
-    None where linear_own.hip does not take it."""
-    ext = _few_for(x, weight) if x.is_cuda else None
-    return None if ext is None else ext.linear_clamped_try(x, weight, bias, limit, alpha)
+    None where linear_own.hip does not take it.  A bias may be a pair, of the first columns of
+    each half."""
+    if bias is None:
+        bias = None, None
+    elif type(bias) is not tuple:
+        bias = bias.chunk(2) if bias.shape == weight.shape[:1] else ()
+    if len(bias) != 2:
+        return None
+    ext = _few_for(x, weight, *(b for b in bias if b is not None)) if x.is_cuda else None
+    return None if ext is None else ext.linear_clamped_try(x, weight, *bias, limit, alpha)
 
 
 def feed_few(x, w_in, w_out, act, norm=None, residual=None):

@@ -42,14 +42,16 @@ struct LinearFewRoom {
 
 // x [M, K], w [O, K] (act: [2 O, K]); bias per row of w, residual [M, O], norm
 // weights [K] for the rows of x; act 0: none, 1: silu, 2: gelu_tanh, 3: clamped, by eps and
-// offset (LF_CLAMPED), without a norm.  room: for a shared
-// contraction; clear: the numbers of another one's that runs behind this.
+// offset (LF_CLAMPED), without a norm, its bias the gate's and `up` the up projection's, of the
+// first columns each (the others have none).  room: for a shared contraction; clear: the numbers
+// of another one's that runs behind this.
 static torch::Tensor linear_few_run(const torch::Tensor& x, const torch::Tensor& w,
                                     const c10::optional<torch::Tensor>& bias,
                                     const c10::optional<torch::Tensor>& residual,
                                     const c10::optional<torch::Tensor>& norm, double eps,
                                     double offset, int64_t act, const LinearFewRoom& room,
-                                    const LinearFewRoom& clear) {
+                                    const LinearFewRoom& clear,
+                                   const c10::optional<torch::Tensor>& up = {}) {
   auto bf16 = [&](const torch::Tensor& t) {
     TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 &&
                     t.device() == x.device(),
@@ -76,7 +78,11 @@ static torch::Tensor linear_few_run(const torch::Tensor& x, const torch::Tensor&
     TORCH_CHECK(t->is_contiguous() && t->numel() == n, "size of a vector");
     return t->data_ptr();
   };
-  const void* b = vec(bias, w.size(0));
+  const long biased = act == 3 && bias ? bias->numel() : w.size(0);
+  TORCH_CHECK(act != 3 || (bias.has_value() == up.has_value() && !residual && !clear.n &&
+                           (!bias || (biased >= 1 && biased <= O))),
+              "both halves of a clamped unit have a bias, or none");
+  const void* b = vec(bias, biased);
   const void* n = vec(norm, K);
   TORCH_CHECK(!n || (whole(*norm) && K <= 32768),
               "norm weights begin at a multiple of 16 bytes, up to 32768 of them");
@@ -90,12 +96,14 @@ static torch::Tensor linear_few_run(const torch::Tensor& x, const torch::Tensor&
     r = residual->data_ptr();
     ldr = residual->stride(0);
   }
+  if (act == 3) r = vec(up, biased);  // (LF_CLAMPED)
   c10::OptionalDeviceGuard guard;  // and the device's current stream
   if (x.get_device() != c10::hip::current_device()) guard.reset_device(x.device());
   auto y = torch::empty({M, O}, x.options());
   launch_linear_few(x.data_ptr(), w.data_ptr(), b, r, n, y.data_ptr(), M, O, K,
                     x.stride(0), w.stride(0), ldr, O, (float)eps, (float)offset,
-                    (int)act, room.numbers, room.sums, clear.numbers, clear.n,
+                    (int)act, room.numbers, room.sums, clear.numbers,
+                    act == 3 ? (int)biased : clear.n,
                     c10::hip::getCurrentHIPStream().stream());
   return y;
 }
@@ -307,21 +315,24 @@ static c10::optional<torch::Tensor> linear_few_try(
       linear_few_run(rows, w, bias, residual, norm, eps, offset, act, {}, cleared), x);
 }
 
-// The clamped unit of x w^T + bias, of up to 64 rows and of more that linear_own.hip takes, or
-// nothing where that does not run here.
+// The clamped unit of x w^T, with a bias for the first columns of each half, of up to 64 rows and
+// of more that linear_own.hip takes, or nothing where that does not run here.
 static c10::optional<torch::Tensor> linear_clamped_try(const torch::Tensor& x,
                                                        const torch::Tensor& w,
-                                                       const c10::optional<torch::Tensor>& bias,
+                                                       const c10::optional<torch::Tensor>& gate,
+                                                       const c10::optional<torch::Tensor>& up,
                                                        double limit, double alpha) {
   if (!linear_few_input(x) || !linear_few_weight(w, x) || w.size(1) < 1 || w.size(0) % 2 ||
       x.size(-1) != w.size(1))
     return {};
   const long K = w.size(1), M = x.numel() / K, O = w.size(0) / 2;
-  if (linear_few_other(K) || !linear_few_along(x, O, w.size(0), bias, {}, {}) ||
+  const long n = gate.has_value() ? gate->numel() : O;
+  if (linear_few_other(K) || gate.has_value() != up.has_value() || n < 1 || n > O ||
+      !linear_few_along(x, O, n, gate, {}, {}) || !linear_few_along(x, O, n, up, {}, {}) ||
       !(M > 64 ? linear_own_many(M, O, K, 3) : linear_few_sizes(M, O, K)))
     return {};
   return linear_few_shaped(
-      linear_few_run(linear_few_rows(x), w, bias, {}, {}, limit, alpha, 3, {}, {}), x);
+      linear_few_run(linear_few_rows(x), w, gate, {}, {}, limit, alpha, 3, {}, {}, up), x);
 }
 
 // A feed-forward: w_out of the gated unit of w_in's halves (act 1 or 2), of x's rows as

@@ -88,7 +88,8 @@ __device__ __forceinline__ bool sums_of_all(const LinearFewArgs& a, long tile,
 }
 
 // LF_CLAMPED: g = min(gate, eps), u = up within eps, g sigmoid(offset g) (u + 1), on the kernels
-// of linear_own.hip, without a norm
+// of linear_own.hip, without a norm or a residual; of the first n_zero columns, bias is added to
+// the gate and res, a vector like it, to the up projection
 enum { LF_PLAIN = 0, LF_SILU = 1, LF_GELU = 2, LF_CLAMPED = 3 };
 
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));

@@ -80,7 +80,11 @@ __device__ __forceinline__ void finish_tile(const LinearFewArgs& a, int row, int
   for (int j = 0; j < 2; ++j) {
     const int at = min(col + j, a.O - 1);
     float f = v[j], up = v[j + 2];
-    if (a.bias) f += (float)a.bias[at], up += (float)a.bias[a.O + at];
+    if (GATED == CLAMPED_ROWS) {
+      if (a.bias && at < a.n_zero) f += (float)a.bias[at], up += (float)a.res[at];
+    } else if (a.bias) {
+      f += (float)a.bias[at], up += (float)a.bias[a.O + at];
+    }
     if (GATED == CLAMPED_ROWS) {
       f = fminf(f, a.eps);
       f = f / (1.0f + __expf(-a.offset * f)) * (fminf(fmaxf(up, -a.eps), a.eps) + 1.0f);
@@ -90,7 +94,7 @@ __device__ __forceinline__ void finish_tile(const LinearFewArgs& a, int row, int
       const float z = 0.7978845608028654f * (f + 0.044715f * f * f * f);
       f = 0.5f * f * (1.0f + tanhf(z)) * up;
     }
-    if (a.res) f += (float)a.res[(long)row * a.ldr + at];
+    if (GATED != CLAMPED_ROWS && a.res) f += (float)a.res[(long)row * a.ldr + at];
     o[j] = f;
   }
   __bf16* y = a.y + (long)row * a.ldy + col;
