@@ -54,7 +54,8 @@ class LlamaAttention(nn.Module):
         """norm: for x's rows first; residual: added to what is returned.  For
         few tokens, where both go with the projections."""
         B, T, _ = x.shape
-        if T > 1 and norm is not None and self._fused_qkv is not None and type(cache) is KVCache:
+        if (T > 1 and norm is not None and self._fused_qkv is not None
+                and type(cache) is KVCache and as_built(self.o_proj)):
             out = attend(self._fused_qkv, self.o_proj, x, norm, cos, sin, cache, self.n_heads,
                          self.scale, residual=residual)
             if out is not None:

@@ -168,6 +168,31 @@ def test_replaced_head_runs(kind, device):
     assert (got - want).norm() < 8e-3 * want.norm()
 
 
+@torch.no_grad()
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("kind", ["llama", "gemma2"])
+@pytest.mark.parametrize("T", [1, 9, 100])
+def test_attention_alone_calls_its_output(kind, T, device):
+    """An attention that is given the norm of its rows, with a hook on its output's
+    projection, and with a module of another class there."""
+    layer, cache, rope = a_layer(kind, True, device)
+    attn, norm = layer.self_attn, layer.input_layernorm
+    torch.manual_seed(T)
+    x = torch.randn(1, T, 256, device=device).bfloat16()
+    angle = torch.rand(T, rope // 2, device=device)
+
+    def call():
+        return attn(x, torch.cos(angle), torch.sin(angle), KVCache(2, 64, 64, device=device), norm)
+
+    want = call().double()
+    handle = attn.o_proj.register_forward_hook(lambda m, args, y: y * 2)
+    hooked = call().double()
+    handle.remove()
+    attn.o_proj = Halved(attn.o_proj)
+    for got in (hooked / 2, call().double() * 2):
+        assert (got - want).norm() < 0.02 * want.norm()
+
+
 class Halved(torch.nn.Module):
     def __init__(self, inner):
         super().__init__()
