@@ -9,14 +9,14 @@
 //
 //   linear_own_kernel   each wave has a ring of its own in LDS and takes chunks of 64 columns
 //                       by turns, so that no wave waits for another before the sums; for up
-//                       to four tiles of W's rows, and eight where rows of x are few
+//                       to four tiles of W's rows, and five and seven of up to 16 rows of x
 //   linear_ring_kernel  five to eight tiles, which is more than such rings have room for:
 //                       waves meet, half of them load W, half x, in rings of lengths that
 //                       suit each
 //
-// Both take any number of tiles, so that blocks are one round of the chip where two and four
-// would leave a second one half empty, and rows of x may be split between blocks that lie
-// eight apart, on one XCD, whose L2 then has W's rows for both.
+// Tiles are as many as make blocks one round of the chip where two and four would leave a second
+// one half empty, and rows of x may be split between blocks that lie eight apart, on one XCD,
+// whose L2 then has W's rows for both.
 #include "linear_own_kernel.h"
 
 namespace {
@@ -187,6 +187,7 @@ void own(LinearFewArgs a, int act, hipStream_t stream) {
   // of 2048 into 3648: 8.8 us with one, 9.5 with two) but in long rows of few (1 to 16 rows
   // of 2048 to 4096 .98, of more than 6144 .90).
   constexpr int most = RT == 1 || (RT == 2 && TT == 2) ? 2 : 1;
+  static_assert(own_room(RT, TT, most, 0, false) <= OWN_LDS, "room of the chunks that it has");
   auto go = [&](auto kernel, int slots) {
     launch(kernel, a, blocks, own_room(RT, TT, slots, a.K, a.norm != nullptr), stream);
   };
@@ -251,6 +252,9 @@ OwnTiles own_tiles(int M, int O, int K, int act, bool norm) {
   OwnTiles best{0, 0};
   long least = 0;
   auto offer = [&](int rt, int tt) {
+    // Three and four tiles read in two rounds no more than these in one, and one of W beside
+    // 64 rows of x no less than three beside 32: they would never be the first with the least.
+    if ((tt == 1 && (rt == 6 || rt == 8)) || (rt == 1 && tt == 4)) return;
     if ((rt <= 4 || tt == 1) && own_room(rt, tt, 1, K, norm) > OWN_LDS) return;
     const long blocks = (long)(tiles + rt - 1) / rt * ((M + 16 * tt - 1) / (16 * tt));
     const int halves = M > 16 ? 2 * (rt + tt) : 2 * rt + 1 + (rt > 4);
@@ -320,14 +324,11 @@ bool linear_own_go(LinearFewArgs a, int act, hipStream_t stream) {
     case 3 * 8 + 1: own<3, 1>(a, act, stream); return true;
     case 4 * 8 + 1: own<4, 1>(a, act, stream); return true;
     case 5 * 8 + 1: own<5, 1>(a, act, stream); return true;
-    case 6 * 8 + 1: own<6, 1>(a, act, stream); return true;
     case 7 * 8 + 1: own<7, 1>(a, act, stream); return true;
-    case 8 * 8 + 1: own<8, 1>(a, act, stream); return true;
     case 1 * 8 + 2: own<1, 2>(a, act, stream); return true;
     case 2 * 8 + 2: own<2, 2>(a, act, stream); return true;
     case 3 * 8 + 2: own<3, 2>(a, act, stream); return true;
     case 4 * 8 + 2: own<4, 2>(a, act, stream); return true;
-    case 1 * 8 + 4: own<1, 4>(a, act, stream); return true;
     case 2 * 8 + 4: own<2, 4>(a, act, stream); return true;
     case 3 * 8 + 4: own<3, 4>(a, act, stream); return true;
     case 4 * 8 + 4: own<4, 4>(a, act, stream); return true;

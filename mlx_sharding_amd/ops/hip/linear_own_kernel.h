@@ -334,7 +334,7 @@ inline void turned(LinearFewArgs& a, int act, int columns) {
 }
 
 // LDS of a block; slots: chunks of a wave
-inline int own_room(int rt, int tt, int slots, int K, bool norm) {
+constexpr int own_room(int rt, int tt, int slots, int K, bool norm) {
   const int ring = OWN_WAVES * slots * (rt + tt) * 2048 + (norm ? (K + 511) / 512 * 1024 : 0);
   const int sums = OWN_WAVES * rt * tt * 1024;
   return ring > sums ? ring : sums;
@@ -351,7 +351,8 @@ inline Tiles tiles_beside(int M, int tiles, int others, int K, bool norm) {
   const int whole = M <= 16 ? 1 : M <= 32 ? 2 : 4;
   for (int rt = 1; rt <= 4; ++rt)
     for (int tt = whole; tt && tt * 2 >= whole; tt /= 2) {
-      if (own_room(rt, tt, 1, K, norm) > OWN_LDS) continue;
+      // (one tile of W and 64 rows of x: as in linear_own.hip)
+      if ((rt == 1 && tt == 4) || own_room(rt, tt, 1, K, norm) > OWN_LDS) continue;
       const int groups = (M + 16 * tt - 1) / (16 * tt);
       int blocks = (tiles + rt - 1) / rt;
       if (groups > 1) blocks = (blocks + 7) / 8 * 8 * groups;
@@ -371,7 +372,7 @@ void with_tiles(const Tiles& t, F f) {
   case R * 8 + T: f(std::integral_constant<int, R>(), std::integral_constant<int, T>()); break;
     CASE(1, 1) CASE(2, 1) CASE(3, 1) CASE(4, 1)
     CASE(1, 2) CASE(2, 2) CASE(3, 2) CASE(4, 2)
-    CASE(1, 4) CASE(2, 4) CASE(3, 4) CASE(4, 4)
+    CASE(2, 4) CASE(3, 4) CASE(4, 4)
 #undef CASE
   }
 }

@@ -1,4 +1,4 @@
-"""Products of few rows: every number of tiles, ragged ends of each size."""
+"""Products of few rows: every number of tiles a block that their sizes lead to, ragged ends."""
 
 import types
 
