@@ -7,9 +7,18 @@ import torch
 import torch.nn.functional as F
 
 from mlx_sharding_amd import ops
+from mlx_sharding_amd.models.fuse import fuse_model
 from test_moe_rows import decoder_layer
 
 pytestmark = pytest.mark.gpu
+
+
+def fused_layer(bits):
+    """One whose shared experts have their two first matrices side by side."""
+    layer = decoder_layer(bits)
+    fuse_model(layer)
+    assert layer.mlp.shared_experts._fused_gu is not None
+    return layer
 
 
 # one block of tokens and two, groups of 16, 32 and 64 rows and one more; parts of 16 experts;
@@ -80,12 +89,13 @@ def test_apart():
 @pytest.mark.parametrize("B", [1, 8, 64, 65])
 def test_layer(bits, B, monkeypatch):
     """A layer's step beside the one without them."""
-    layer = decoder_layer(bits)
+    layer = fused_layer(bits)
     x = torch.randn(B, 1, 512, device="cuda").bfloat16()
     tickets = torch.zeros(B, dtype=torch.int32, device="cuda")
-    norm = layer.post_attention_layernorm
+    norm, finish, calls = layer.post_attention_layernorm, ops.expert_finish, []
+    monkeypatch.setattr(ops, "expert_finish", lambda *a: calls.append(1) or finish(*a))
     got = layer.mlp.decode(x, None, norm, tickets.clone()).double()
-    assert bool((tickets == 0).all())
+    assert bool(calls) == (B <= 64) and bool((tickets == 0).all())
     monkeypatch.setattr(ops, "expert_begin_ok", lambda *a: False)
     want = layer.mlp.decode(x, None, norm, tickets.clone()).double()
     # sums in other orders: a choice between experts that are nearly tied may differ
@@ -95,7 +105,7 @@ def test_layer(bits, B, monkeypatch):
 
 def test_captured():
     """Replays of a captured step, with the step itself between them."""
-    layer = decoder_layer(4)
+    layer = fused_layer(4)
     x = torch.randn(20, 1, 512, device="cuda").bfloat16()
     norm = layer.post_attention_layernorm
     tickets = torch.zeros(20, dtype=torch.int32, device="cuda")
