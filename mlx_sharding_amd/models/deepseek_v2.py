@@ -502,8 +502,10 @@ class DeepseekV2MoE(nn.Module):
         shape, H = x.shape, x.shape[-1]
         flat = x.reshape(-1, H)
         around = None
+        packed = self._packing()
         if tickets is not None and residual is None:
-            around = self._beside(flat, ops.expert_begin_ok)
+            around = self._beside(flat, lambda *a: ops.expert_begin_ok(*a) and
+                                  ops.expert_begin_pays(*a, packed[0] < 16))
         y, h, choice, weight, *units = ops.expert_route(
             flat, None if residual is None else residual.reshape(-1, H),
             norm, self.gate.weight, self.top_k, self.routed_scaling_factor,
@@ -511,7 +513,6 @@ class DeepseekV2MoE(nn.Module):
         m = self.switch_mlp
         stacks = [[p.weight] if m.quant is None else [p.weight, p.scales, p.biases]
                   for p in (m.gate_proj, m.up_proj, m.down_proj)]
-        packed = self._packing()
         if around is not None:
             rows = ops.expert_rows(y, choice, weight, *stacks, *packed)
             return ops.expert_finish(*units, around[1], rows, h).view(shape)

@@ -85,6 +85,18 @@ def test_apart():
                              n and torch.zeros(n, dtype=torch.int32, device="cuda"), w(128, 128))
 
 
+@pytest.mark.parametrize("bits,B,taken", [(0, 1, False), (4, 8, False), (4, 9, True),
+                                          (0, 64, True), (0, 65, False)])
+def test_small_layers_of_few_tokens_have_their_own(bits, B, taken, monkeypatch):
+    layer, calls = fused_layer(bits), []
+    finish = ops.expert_finish
+    monkeypatch.setattr(ops, "expert_finish", lambda *a: calls.append(1) or finish(*a))
+    layer.mlp.decode(torch.randn(B, 1, 512, device="cuda").bfloat16(), None,
+                     layer.post_attention_layernorm,
+                     torch.zeros(B, dtype=torch.int32, device="cuda"))
+    assert bool(calls) == taken
+
+
 @pytest.mark.parametrize("bits", [0, 4])
 @pytest.mark.parametrize("B", [1, 8, 64, 65])
 def test_layer(bits, B, monkeypatch):
@@ -93,6 +105,7 @@ def test_layer(bits, B, monkeypatch):
     x = torch.randn(B, 1, 512, device="cuda").bfloat16()
     tickets = torch.zeros(B, dtype=torch.int32, device="cuda")
     norm, finish, calls = layer.post_attention_layernorm, ops.expert_finish, []
+    monkeypatch.setattr(ops, "expert_begin_pays", lambda *a: True)
     monkeypatch.setattr(ops, "expert_finish", lambda *a: calls.append(1) or finish(*a))
     got = layer.mlp.decode(x, None, norm, tickets.clone()).double()
     assert bool(calls) == (B <= 64) and bool((tickets == 0).all())
@@ -127,3 +140,13 @@ def test_captured():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, step())
+
+
+def test_what_pays():
+    """Ends of the rule, which looks at sizes alone."""
+    w = lambda S: types.SimpleNamespace(shape=(0, S))  # noqa: E731
+    for n, H, S, packed, pays in (
+            (8, 2048, 64, True, True), (8, 2048, 2047, False, False), (8, 2048, 2048, False, True),
+            (8, 2047, 64, True, False), (8, 1024, 4096, True, True), (8, 1024, 4095, True, False),
+            (1, 128, 4097, False, True), (9, 128, 64, False, True)):
+        assert ops.expert_begin_pays(n, H, None, w(S), packed) == pays
