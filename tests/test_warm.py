@@ -14,7 +14,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,Hq,Hkv,D,cached,O", [
     (1, 32, 8, 128, 700, 4096), (1, 32, 4, 64, 5, 2048), (1, 9, 9, 64, 100, 1), (3, 14, 2, 128, 64, 40),
     (16, 8, 1, 64, 900, 1000), (2, 28, 4, 128, 3000, 20000), (17, 16, 1, 64, 40, 512),
-    (1, 16, 8, 256, 90, 640)])
+    (1, 16, 8, 256, 90, 640),
+    # the fewest weights that are fetched, and one row less
+    (1, 9, 9, 64, 100, 1366), (1, 9, 9, 64, 100, 1365), (3, 14, 2, 128, 64, 1001),
+    (16, 8, 1, 64, 900, 3001)])
 def test_same(B, Hq, Hkv, D, cached, O, captured):
     g = torch.Generator("cuda").manual_seed(cached)
     one, two = _caches(B, Hkv, D, cached, cached + 40, captured, g)
