@@ -6,7 +6,8 @@
 //   moe_down     the pairs' outputs, weighted, in 32 bits
 //   moe_combine  a token's pairs, shared experts and residual added up
 //
-// (up to 64 tokens with a shared feed-forward have moe_shared.hip's for the first and last)
+// (9 to 64 tokens with a shared feed-forward, and fewer with a large one, have moe_shared.hip's
+// for the first and last)
 //
 // No sort: a block counts every expert's pairs, which tells its share of the work, and
 // looks through the choices (at most 1024) for those of an expert.  Rows of pairs lie at
